@@ -106,7 +106,7 @@ typedef struct QaConv2Params {
     int8_t* x;
     int8_t* B;
     int8_t* C;
-    int8_t* conv_state;                  /* update only */
+    int8_t* conv_state;                  /* update: shifted in place; forward: receives the last conv_state_len inputs, or null */
     const float* x_out_scales;           /* [1] or [n_groups, nhead_groups, ndim_groups] */
     const float* B_out_scales;           /* [1] or [n_groups] */
     const float* C_out_scales;
@@ -115,7 +115,7 @@ typedef struct QaConv2Params {
     float scale_x, scale_B, scale_C;     /* input scales of the three parts */
     float scale_wx, scale_wB, scale_wC;  /* weight scales */
     float scale_bx, scale_bB, scale_bC;  /* bias scales */
-    float reserved0;
+    float x_out_scale;                   /* internal: the one output scale when x_out_scales is null (Mamba1 conv) */
 } QaConv2Params;
 
 int qa_quamba2_conv1d_fwd(const QaConv2Params* p, void* stream);
@@ -245,6 +245,15 @@ typedef struct QaSScanParams {
      * the number of 64-channel workgroups per batch entry that take four lanes per channel.  A mapping the
      * shape does not admit returns QA_ERR_SHAPE or QA_ERR_UNSUPPORTED.  Results agree to fp32 rounding. */
     int32_t mapping;
+    /* token_major = 1: u, delta and z have channels contiguous (u_d_stride == delta_d_stride == z_d_stride == 1, steps
+     * u_l_stride ... apart) and B, C states contiguous (B_dstate_stride == C_dstate_stride == 1, steps B_l_stride ...
+     * apart), as the row-major projections leave them; all of them 4-byte aligned with strides of whole words.
+     * dstate 16, one group, dim a multiple of 4, none of the carry fields above, mapping 0.  `workspace` (or null):
+     * scratch for scanning few sequences as segments side by side.  segments, segment_len: set by the library. */
+    int32_t token_major, segments, segment_len, reserved0;
+    int64_t u_l_stride, delta_l_stride, z_l_stride, B_l_stride, C_l_stride;
+    void* workspace;
+    int64_t workspace_bytes;
 } QaSScanParams;
 
 /* marker bit 30, lanes in bits 20..27, the second argument in bits 0..19; a value without the marker is refused */
@@ -404,7 +413,7 @@ typedef struct QaSsdParams {
     int32_t D_has_hdim;          /* D is (nheads, headdim) instead of (nheads) */
     int32_t nhead_groups, ndim_groups;  /* 0 = per-tensor x scale */
     int32_t final_state_is_fp32; /* 1: fp32 final states, 0: int8 with state scale */
-    int32_t reserved0;
+    int32_t dt_row_stride;       /* elements between the steps of dt; 0: nheads (contiguous) */
     float dt_min, dt_max;        /* clamp after softplus */
     const int8_t* x;             /* (batch, seqlen, nheads, headdim) contiguous */
     const void* dt;              /* int8 or fp32 (batch, seqlen, nheads) contiguous */
@@ -455,6 +464,89 @@ int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream);
  * into a HIP graph.  The size check comes before any runtime call. */
 #define QA_SSD_STATIC_SCRATCH_BYTES (64ll << 20)
 int qa_ssd_chunk_scan_fwd_noalloc(const QaSsdParams* p, void* stream);
+
+/* ------------------------------------------------------------------------------------------
+ * The assembled mixers: every kernel of one layer call enqueued by one library call, with the intermediates in one
+ * caller-supplied workspace.  forward: a prompt from zero states (quamba/qMambaLayer.py:895-943, qMamba2.py:905-985);
+ * step: one token per sequence, both states advanced in place (qMambaLayer.py:945-1010, qMamba2.py:987-1068).
+ * Activations stay row-major (token, channel) from in_proj to out_proj.
+ * ---------------------------------------------------------------------------------------- */
+/* a projection with one row of activations: the rule its module applies then */
+typedef enum QaRowRule { QA_ROW_SCALES = 0, QA_ROW_ALPHA = 1, QA_ROW_HALF_AWAY = 2 } QaRowRule;
+
+typedef struct QaLinearParams {
+    int32_t n, k;             /* rows of the weight (outputs and padding), inputs */
+    int32_t bits;             /* 8: int8 (n, k); 4: packed (n, k/2), see QaGemmW4A8Params */
+    int32_t row_rule;         /* QaRowRule, int8 weights only */
+    int32_t col_numel;        /* col_scale: 1 or n */
+    float alpha;              /* QA_ROW_ALPHA */
+    const void* weight;       /* contiguous rows, 16-byte aligned */
+    const void* s_group;      /* 4 bits: fp16 (k/128, n), or null (per channel) */
+    const float* col_scale;   /* per output column */
+    const float* row_scale;   /* one fp32 */
+} QaLinearParams;
+
+typedef struct QaMamba1Params {
+    int32_t batch, seqlen;
+    int32_t d_model, d_inner, d_state, d_conv, dt_rank;   /* d_state 16, d_conv 2..4 */
+    int32_t delta_softplus;
+    int32_t state_is_fp32, conv_state_len;
+    QaLinearParams in_proj, x_proj, dt_proj, out_proj;
+    const int8_t* conv_weight;         /* (d_inner, d_conv) contiguous */
+    const int8_t* conv_bias;           /* or null */
+    float conv_scale_x, conv_scale_w, conv_scale_b, conv_scale_out;
+    const int8_t* A_log;               /* (d_inner, d_state) contiguous */
+    const int8_t* D;                   /* or null */
+    const int8_t* dt_bias;             /* or null */
+    const float *A_scale, *D_scale, *dt_bias_scale, *u_scale, *dt_scale, *B_scale, *C_scale, *z_scale, *ssm_state_scale;
+    float had_scale;
+    int32_t reserved0;
+    const int8_t* hidden;              /* (batch, seqlen, d_model) contiguous */
+    void* out;                         /* fp16 (batch, seqlen, out_proj.n) */
+    int8_t* conv_state;                /* (batch, d_inner, conv_state_len); forward: or null */
+    int64_t conv_state_batch_stride, conv_state_c_stride, conv_state_l_stride;
+    void* ssm_state;                   /* (batch, d_inner, d_state) contiguous; forward: or null */
+    void* workspace;                   /* 256-byte aligned */
+    int64_t workspace_bytes;
+} QaMamba1Params;
+
+/* Bytes of workspace a forward (step 0) or step (1) call needs; 0: unsupported sizes. */
+int64_t qa_mamba1_workspace_bytes(const QaMamba1Params* p, int step);
+int qa_mamba1_forward(const QaMamba1Params* p, void* stream);
+int qa_mamba1_step(const QaMamba1Params* p, void* stream);
+
+typedef struct QaMamba2Params {
+    int32_t batch, seqlen;
+    int32_t d_model, d_inner, d_state, d_conv, headdim, ngroups, chunk_size;
+    int32_t delta_softplus, D_has_hdim;
+    int32_t state_is_fp32, conv_state_len;
+    int32_t conv_nhead_groups, conv_ndim_groups, nhead_groups, ndim_groups;
+    int32_t norm_group_size, norm_before_gate;
+    QaLinearParams in_proj, out_proj;
+    const int8_t* conv_weight;         /* (d_inner + 2 ngroups d_state, d_conv) contiguous */
+    const int8_t* conv_bias;           /* or null */
+    const float *x_out_scales, *B_out_scales, *C_out_scales;
+    const int32_t *conv_head_range, *conv_dim_range;
+    float scale_x, scale_B, scale_C, scale_wx, scale_wB, scale_wC, scale_bx, scale_bB, scale_bC;
+    float dt_min, dt_max, norm_eps, norm_z_scale, had_scale;
+    const int8_t* A_log;               /* (nheads) */
+    const int8_t* D;                   /* (nheads) or (nheads, headdim), or null */
+    const void* dt_bias;               /* fp16 (nheads), or null */
+    const float *A_log_scale, *D_scale, *dt_scale, *x_scales, *B_scale, *C_scale, *ssm_state_scale;
+    const int32_t *head_range, *dim_range;
+    const void* norm_weight;           /* fp16 (d_inner) */
+    const int8_t* hidden;              /* (batch, seqlen, d_model) contiguous */
+    void* out;                         /* fp16 (batch, seqlen, out_proj.n) */
+    int8_t* conv_state;                /* (batch, conv channels, conv_state_len); forward: or null */
+    int64_t conv_state_batch_stride, conv_state_c_stride, conv_state_l_stride;
+    void* ssm_state;                   /* (batch, nheads, headdim, d_state) contiguous; forward: or null */
+    void* workspace;                   /* 256-byte aligned */
+    int64_t workspace_bytes;
+} QaMamba2Params;
+
+int64_t qa_mamba2_workspace_bytes(const QaMamba2Params* p, int step);
+int qa_mamba2_forward(const QaMamba2Params* p, void* stream);
+int qa_mamba2_step(const QaMamba2Params* p, void* stream);
 
 #ifdef __cplusplus
 }

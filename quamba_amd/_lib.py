@@ -51,7 +51,7 @@ class QaConv2Params(C.Structure):
         ("scale_x", f32), ("scale_B", f32), ("scale_C", f32),
         ("scale_wx", f32), ("scale_wB", f32), ("scale_wC", f32),
         ("scale_bx", f32), ("scale_bB", f32), ("scale_bC", f32),
-        ("reserved0", f32),
+        ("x_out_scale", f32),
     ]
 
 
@@ -89,6 +89,9 @@ class QaSScanParams(C.Structure):
         ("scale_D", vp), ("scale_delta_bias", vp), ("scale_z", vp), ("scale_ssm_state", vp),
         ("out", vp), ("last_state_i8", vp), ("last_state_f32", vp),
         ("dt_sum_out", vp), ("carry_dt_sum", vp), ("carry_state", vp), ("carry_first", i32), ("mapping", i32),
+        ("token_major", i32), ("segments", i32), ("segment_len", i32), ("reserved0", i32),
+        ("u_l_stride", i64), ("delta_l_stride", i64), ("z_l_stride", i64), ("B_l_stride", i64), ("C_l_stride", i64),
+        ("workspace", vp), ("workspace_bytes", i64),
     ]
 
 
@@ -142,7 +145,7 @@ class QaSsdParams(C.Structure):
         ("batch", i32), ("seqlen", i32), ("nheads", i32), ("headdim", i32), ("dstate", i32),
         ("ngroups", i32), ("chunk_size", i32), ("dt_softplus", i32), ("dt_is_fp32", i32),
         ("D_has_hdim", i32), ("nhead_groups", i32), ("ndim_groups", i32),
-        ("final_state_is_fp32", i32), ("reserved0", i32),
+        ("final_state_is_fp32", i32), ("dt_row_stride", i32),
         ("dt_min", f32), ("dt_max", f32),
         ("x", vp), ("dt", vp), ("A_log", vp), ("B", vp), ("C", vp), ("D", vp), ("z", vp),
         ("dt_bias", vp),
@@ -151,6 +154,57 @@ class QaSsdParams(C.Structure):
         ("x_head_group_range", vp), ("x_dim_group_range", vp),
         ("out", vp), ("final_states", vp), ("workspace", vp), ("workspace_bytes", i64),
     ]
+
+
+class QaLinearParams(C.Structure):
+    _fields_ = [
+        ("n", i32), ("k", i32), ("bits", i32), ("row_rule", i32), ("col_numel", i32), ("alpha", f32),
+        ("weight", vp), ("s_group", vp), ("col_scale", vp), ("row_scale", vp),
+    ]
+
+
+QA_ROW_SCALES, QA_ROW_ALPHA, QA_ROW_HALF_AWAY = 0, 1, 2
+
+# what a call brings along, at the end of both layer blocks
+_CALL_FIELDS = [
+    ("hidden", vp), ("out", vp), ("conv_state", vp),
+    ("conv_state_batch_stride", i64), ("conv_state_c_stride", i64), ("conv_state_l_stride", i64),
+    ("ssm_state", vp), ("workspace", vp), ("workspace_bytes", i64),
+]
+
+
+class QaMamba1Params(C.Structure):
+    _fields_ = [
+        ("batch", i32), ("seqlen", i32),
+        ("d_model", i32), ("d_inner", i32), ("d_state", i32), ("d_conv", i32), ("dt_rank", i32),
+        ("delta_softplus", i32), ("state_is_fp32", i32), ("conv_state_len", i32),
+        ("in_proj", QaLinearParams), ("x_proj", QaLinearParams), ("dt_proj", QaLinearParams), ("out_proj", QaLinearParams),
+        ("conv_weight", vp), ("conv_bias", vp),
+        ("conv_scale_x", f32), ("conv_scale_w", f32), ("conv_scale_b", f32), ("conv_scale_out", f32),
+        ("A_log", vp), ("D", vp), ("dt_bias", vp),
+        ("A_scale", vp), ("D_scale", vp), ("dt_bias_scale", vp), ("u_scale", vp), ("dt_scale", vp), ("B_scale", vp),
+        ("C_scale", vp), ("z_scale", vp), ("ssm_state_scale", vp),
+        ("had_scale", f32), ("reserved0", i32),
+    ] + _CALL_FIELDS
+
+
+class QaMamba2Params(C.Structure):
+    _fields_ = [
+        ("batch", i32), ("seqlen", i32),
+        ("d_model", i32), ("d_inner", i32), ("d_state", i32), ("d_conv", i32), ("headdim", i32), ("ngroups", i32),
+        ("chunk_size", i32), ("delta_softplus", i32), ("D_has_hdim", i32), ("state_is_fp32", i32), ("conv_state_len", i32),
+        ("conv_nhead_groups", i32), ("conv_ndim_groups", i32), ("nhead_groups", i32), ("ndim_groups", i32),
+        ("norm_group_size", i32), ("norm_before_gate", i32),
+        ("in_proj", QaLinearParams), ("out_proj", QaLinearParams),
+        ("conv_weight", vp), ("conv_bias", vp), ("x_out_scales", vp), ("B_out_scales", vp), ("C_out_scales", vp),
+        ("conv_head_range", vp), ("conv_dim_range", vp),
+        ("scale_x", f32), ("scale_B", f32), ("scale_C", f32), ("scale_wx", f32), ("scale_wB", f32), ("scale_wC", f32),
+        ("scale_bx", f32), ("scale_bB", f32), ("scale_bC", f32),
+        ("dt_min", f32), ("dt_max", f32), ("norm_eps", f32), ("norm_z_scale", f32), ("had_scale", f32),
+        ("A_log", vp), ("D", vp), ("dt_bias", vp),
+        ("A_log_scale", vp), ("D_scale", vp), ("dt_scale", vp), ("x_scales", vp), ("B_scale", vp), ("C_scale", vp),
+        ("ssm_state_scale", vp), ("head_range", vp), ("dim_range", vp), ("norm_weight", vp),
+    ] + _CALL_FIELDS
 
 
 # name -> (restype, argtypes); every symbol declared in include/quamba_amd.h
@@ -174,6 +228,12 @@ SYMBOLS = {
     "qa_ssd_workspace_bytes": (C.c_int64, [C.POINTER(QaSsdParams)]),
     "qa_ssd_chunk_scan_fwd": (C.c_int, [C.POINTER(QaSsdParams), vp]),
     "qa_ssd_chunk_scan_fwd_noalloc": (C.c_int, [C.POINTER(QaSsdParams), vp]),
+    "qa_mamba1_workspace_bytes": (C.c_int64, [C.POINTER(QaMamba1Params), C.c_int]),
+    "qa_mamba1_forward": (C.c_int, [C.POINTER(QaMamba1Params), vp]),
+    "qa_mamba1_step": (C.c_int, [C.POINTER(QaMamba1Params), vp]),
+    "qa_mamba2_workspace_bytes": (C.c_int64, [C.POINTER(QaMamba2Params), C.c_int]),
+    "qa_mamba2_forward": (C.c_int, [C.POINTER(QaMamba2Params), vp]),
+    "qa_mamba2_step": (C.c_int, [C.POINTER(QaMamba2Params), vp]),
 }
 
 _lib = None

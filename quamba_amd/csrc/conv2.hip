@@ -16,6 +16,7 @@
 // with one byte permute, the taps are one packed int8 dot product per output (exact), the epilogue
 // is the cheap-with-exact-fallback route shared with the Mamba1 conv, one dword store per step.
 #include "conv_common.hpp"
+#include "mixer_common.hpp"
 
 namespace qa {
 namespace {
@@ -46,6 +47,7 @@ __device__ __forceinline__ Part part_of(const QaConv2Params& p, int ch) {
 
 // Output scale of channel `ch`; the range walk is the reference's (first range that contains the index).
 __device__ __forceinline__ float out_scale_of(const QaConv2Params& p, const Part& part, int ch) {
+    if (!p.x_out_scales) return p.x_out_scale;          // one host-side scale: the Mamba1 conv
     const bool grouped = p.x_head_group_range != nullptr && p.x_dim_group_range != nullptr;
     if (part.index != 0) {
         const float* s = part.index == 1 ? p.B_out_scales : p.C_out_scales;
@@ -163,6 +165,21 @@ __global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, in
             out_at += out_ls;
         }
     }
+    // the wave that reaches the end leaves the last inputs of its channels (still in the caches) in the conv state
+    if (p.conv_state && t_end == p.seqlen) {
+        int8_t* st = p.conv_state + b * p.conv_state_batch_stride + ch0 * p.conv_state_c_stride;
+        const bool words = p.conv_state_c_stride == 1 && (reinterpret_cast<uintptr_t>(st) & 3u) == 0 && p.conv_state_l_stride % 4 == 0;
+        for (int i = 0; i < p.conv_state_len; ++i) {
+            const int t = p.seqlen - p.conv_state_len + i;
+            const uint32_t v = t >= 0 ? *reinterpret_cast<const uint32_t*>(src + t * p.xBC_l_stride) : 0u;
+            if (words) {
+                *reinterpret_cast<uint32_t*>(st + i * p.conv_state_l_stride) = v;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) st[e * p.conv_state_c_stride + i * p.conv_state_l_stride] = static_cast<int8_t>(v >> (8 * e));
+            }
+        }
+    }
 }
 
 // Any alignment: one thread per output element, same arithmetic.
@@ -248,6 +265,30 @@ int validate(const QaConv2Params* p, bool update) {
 }  // namespace
 }  // namespace qa
 
+namespace qa {
+int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
+    // Steps per wave: 64, 128 or 256, whichever needs the fewest rounds of resident waves (seven per SIMD) times its
+    // own length plus a wave's set-up (taps, scales: about 24 steps' worth).  Batch 16 x 1024 steps x 10240 channels
+    // is 10240 waves of 64 steps on 7168 places - a second round at a third of the occupancy - or 5120 of 128.
+    int run = kRun;
+    {
+        const int64_t ch_blocks = (p.dim + 255) / 256, places = 7 * 4 * 256;
+        int64_t best = -1;
+        for (int r = 64; r <= 256; r *= 2) {
+            const int64_t waves = ch_blocks * (((p.seqlen + r - 1) / r + 3) / 4 * 4) * p.batch;
+            const int64_t cost = ((waves + places - 1) / places) * (r + 24);
+            if (best < 0 || cost < best) { best = cost; run = r; }
+        }
+    }
+    const int64_t run_blocks = (p.seqlen + 4 * run - 1) / (4 * run);
+    if (run_blocks > 65535) return QA_ERR_SHAPE;
+    dim3 grid((p.dim + 255) / 256, static_cast<unsigned>(run_blocks), p.batch);
+    if (p.silu_activation) hipLaunchKernelGGL(conv2_fwd_kernel<true>, grid, dim3(kThreads), 0, stream, p, run);
+    else hipLaunchKernelGGL(conv2_fwd_kernel<false>, grid, dim3(kThreads), 0, stream, p, run);
+    return check_launch();
+}
+}  // namespace qa
+
 extern "C" int qa_quamba2_conv1d_fwd(const QaConv2Params* p, void* stream_) {
     using namespace qa;
     const int st = validate(p, false);
@@ -262,27 +303,8 @@ extern "C" int qa_quamba2_conv1d_fwd(const QaConv2Params* p, void* stream_) {
                      aligned4(p->C) && mult4(p->xBC_batch_stride) && mult4(p->xBC_l_stride) &&
                      mult4(p->x_batch_stride) && mult4(p->x_l_stride) && mult4(p->B_batch_stride) &&
                      mult4(p->B_l_stride) && mult4(p->C_batch_stride) && mult4(p->C_l_stride);
-    if (vec) {
-        // Steps per wave: 64, 128 or 256, whichever needs the fewest rounds of resident waves (seven per SIMD) times its
-        // own length plus a wave's set-up (taps, scales: about 24 steps' worth).  Batch 16 x 1024 steps x 10240 channels
-        // is 10240 waves of 64 steps on 7168 places - a second round at a third of the occupancy - or 5120 of 128.
-        int run = kRun;
-        {
-            const int64_t ch_blocks = (p->dim + 255) / 256, places = 7 * 4 * 256;
-            int64_t best = -1;
-            for (int r = 64; r <= 256; r *= 2) {
-                const int64_t waves = ch_blocks * (((p->seqlen + r - 1) / r + 3) / 4 * 4) * p->batch;
-                const int64_t cost = ((waves + places - 1) / places) * (r + 24);
-                if (best < 0 || cost < best) { best = cost; run = r; }
-            }
-        }
-        const int64_t run_blocks = (p->seqlen + 4 * run - 1) / (4 * run);
-        if (run_blocks > 65535) return QA_ERR_SHAPE;
-        dim3 grid((p->dim + 255) / 256, static_cast<unsigned>(run_blocks), p->batch);
-        if (p->silu_activation) hipLaunchKernelGGL(conv2_fwd_kernel<true>, grid, dim3(kThreads), 0, stream, *p, run);
-        else hipLaunchKernelGGL(conv2_fwd_kernel<false>, grid, dim3(kThreads), 0, stream, *p, run);
-        return check_launch();
-    }
+    if (vec) return conv_channel_last_fwd(*p, stream);
+    if (p->conv_state) return QA_ERR_STRIDE;                      // (written by the kernel for aligned rows only)
     const int64_t blocks = (total + kThreads - 1) / kThreads;
     if (blocks > 0x7fffffffLL) return QA_ERR_SHAPE;
     hipLaunchKernelGGL(conv2_fwd_generic_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream, *p);

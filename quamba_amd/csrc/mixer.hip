@@ -1,0 +1,434 @@
+// The assembled mixers: one library call enqueues every kernel of a layer call.
+//
+// What a small call costs is the host: seven to nine launches, each behind its own argument checks, tensor
+// allocations and stream lookups in the caller's language (about 22 us each from Python against 3-5 us of kernel at
+// one token).  Here the intermediates are sections of one workspace and the launches follow each other at the
+// runtime's own pace.
+//
+// Layout: activations stay row-major (token, channel) from in_proj to out_proj.  The conv walks time with four
+// channels per lane, the scan stages token-major rows, x_proj and dt_proj are plain row-major products - so no second
+// copy of the conv's output, no transposition of B and C, no padding of the token count, and prompts of any length
+// run on the same kernels.
+#include "mixer_common.hpp"
+#include "ssd_common.hpp"
+
+#include <algorithm>
+
+namespace qa {
+namespace {
+
+constexpr int kExpandOnceRows = 1024;     // 4-bit weights are expanded once per call from this many rows on
+
+// Sections of the workspace, each 256-byte aligned.
+struct Carver {
+    uint8_t* base;
+    int64_t off = 0;
+    template <typename T>
+    T* take(int64_t bytes) {
+        T* r = base ? reinterpret_cast<T*>(base + off) : nullptr;
+        off = (off + bytes + 255) & ~int64_t(255);
+        return r;
+    }
+};
+
+struct Scratch {
+    void* p;
+    int64_t bytes;
+};
+
+int64_t expanded_bytes(const QaLinearParams& w, int64_t rows) {
+    return w.bits == 4 && rows >= kExpandOnceRows ? static_cast<int64_t>(w.n) * w.k : 0;
+}
+
+// d (rows, w.n) = the projection of a (rows, w.k).  channel_scale_last: the association of the transposed call
+// (to_seqlen_last), whose products and bits the row-major one reproduces.
+int project(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows, void* d, int out_type, bool channel_scale_last,
+            const Scratch& w8, void* stream) {
+    if (w.bits == 4) {
+        QaGemmW4A8Params p = {};
+        p.m = rows; p.n = w.n; p.k = w.k;
+        p.group_size = w.s_group ? 128 : -1;
+        p.out_type = out_type;
+        p.tok_scale_numel = 1;
+        p.lda = lda; p.ldd = w.n;
+        p.a = a; p.w_packed = static_cast<const uint8_t*>(w.weight); p.s_group = w.s_group;
+        p.s_channel = w.col_scale; p.s_token = w.row_scale; p.d = d;
+        if (expanded_bytes(w, rows)) { p.w8_workspace = w8.p; p.w8_workspace_bytes = w8.bytes; }
+        return qa_gemm_w4a8(&p, stream);
+    }
+    QaGemmW8A8Params p = {};
+    p.m = rows; p.n = w.n; p.k = w.k;
+    p.out_type = out_type;
+    p.lda = lda; p.ldw = w.k; p.ldd = w.n;
+    p.a = a; p.w = static_cast<const int8_t*>(w.weight); p.d = d;
+    p.a_scale = w.row_scale; p.w_scale = w.col_scale;
+    p.a_scale_numel = 1; p.w_scale_numel = w.col_numel;
+    if (channel_scale_last) {
+        p.scale_order = 1;
+    } else if (rows == 1 && w.row_rule == QA_ROW_ALPHA) {
+        p.use_alpha = 1;
+        p.alpha = w.alpha;
+    } else if (rows == 1 && w.row_rule == QA_ROW_HALF_AWAY) {
+        p.round_mode = QA_ROUND_HALF_AWAY;
+    }
+    return qa_gemm_w8a8(&p, stream);
+}
+
+bool linear_ok(const QaLinearParams& w) {
+    return (w.bits == 8 || w.bits == 4) && w.n > 0 && w.k > 0 && w.weight && w.col_scale && w.row_scale;
+}
+
+int hadamard(const void* y, int8_t* out, int rows, int dim, float scale, void* stream) {
+    QaHadamardParams h = {};
+    h.rows = rows; h.dim = dim; h.in_type = 0; h.scale = scale;
+    h.x_row_stride = dim; h.out_row_stride = dim;
+    h.x = y; h.out = out;
+    return qa_hadamard_quant(&h, stream);
+}
+
+#define QA_TRY(call)                       \
+    do {                                   \
+        const int st_ = (call);            \
+        if (st_ != QA_OK) return st_;      \
+    } while (0)
+
+// ---------------------------------------------------------------------------------------------
+// Mamba1
+// ---------------------------------------------------------------------------------------------
+struct Mamba1Buffers {
+    int8_t *xz, *x, *x_dbl, *dt, *yq;
+    __half* y;
+    Scratch w8, scan;
+    int64_t total;
+};
+
+QaSScanParams scan_sizes(const QaMamba1Params& p) {
+    QaSScanParams s = {};
+    s.batch = p.batch; s.dim = p.d_inner; s.seqlen = p.seqlen; s.dstate = p.d_state; s.n_groups = 1;
+    return s;
+}
+
+Mamba1Buffers carve(const QaMamba1Params& p, void* base) {
+    const int64_t t = static_cast<int64_t>(p.batch) * p.seqlen;
+    Carver c{static_cast<uint8_t*>(base)};
+    Mamba1Buffers b;
+    b.xz = c.take<int8_t>(t * p.in_proj.n);
+    b.x = c.take<int8_t>(t * p.d_inner);
+    b.x_dbl = c.take<int8_t>(t * p.x_proj.n);
+    b.dt = c.take<int8_t>(t * p.dt_proj.n);
+    b.yq = c.take<int8_t>(t * p.d_inner);
+    b.y = c.take<__half>(t * p.d_inner * 2);
+    b.w8.bytes = std::max(std::max(expanded_bytes(p.in_proj, t), expanded_bytes(p.x_proj, t)),
+                          std::max(expanded_bytes(p.dt_proj, t), expanded_bytes(p.out_proj, t)));
+    b.w8.p = c.take<uint8_t>(b.w8.bytes);
+    b.scan.bytes = sscan_token_major_workspace(scan_sizes(p));
+    b.scan.p = c.take<uint8_t>(b.scan.bytes);
+    b.total = c.off;
+    return b;
+}
+
+int validate(const QaMamba1Params* p) {
+    if (!p) return QA_ERR_NULL;
+    if (p->batch < 1 || p->seqlen < 1 || p->batch > 65535 || static_cast<int64_t>(p->batch) * p->seqlen > 0x7fffffff) return QA_ERR_SHAPE;
+    if (p->d_state != 16 || p->d_conv < 2 || p->d_conv > 4 || p->d_inner % 16 != 0 || p->dt_rank % 4 != 0) return QA_ERR_UNSUPPORTED;
+    for (const QaLinearParams* w : {&p->in_proj, &p->x_proj, &p->dt_proj, &p->out_proj})
+        if (!linear_ok(*w)) return QA_ERR_NULL;
+    if (p->in_proj.k != p->d_model || p->in_proj.n != 2 * p->d_inner || p->x_proj.k != p->d_inner ||
+        p->x_proj.n < p->dt_rank + 2 * p->d_state || p->x_proj.n % 4 != 0 || p->dt_proj.k != p->dt_rank ||
+        p->dt_proj.n != p->d_inner || p->out_proj.k != p->d_inner) return QA_ERR_SHAPE;
+    if (p->conv_state_len != p->d_conv && p->conv_state_len != p->d_conv - 1) return QA_ERR_SHAPE;
+    return QA_OK;
+}
+
+int ready(const QaMamba1Params* p, bool states) {
+    QA_TRY(validate(p));
+    if (!p->hidden || !p->out || !p->workspace || !p->conv_weight || !p->A_log) return QA_ERR_NULL;
+    if (states && (!p->conv_state || !p->ssm_state)) return QA_ERR_NULL;
+    if (p->workspace_bytes < carve(*p, nullptr).total || (reinterpret_cast<uintptr_t>(p->workspace) & 255u)) return QA_ERR_STRIDE;
+    return QA_OK;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Mamba2
+// ---------------------------------------------------------------------------------------------
+struct Mamba2Buffers {
+    int8_t *zxbcdt, *x, *B, *C, *yq;
+    __half *y, *yn;
+    Scratch w8, ssd;
+    int64_t total;
+};
+
+int heads_of(const QaMamba2Params& p) { return p.d_inner / p.headdim; }
+
+bool norm_fuses(const QaMamba2Params& p) {
+    const int d = p.d_inner, g = p.norm_group_size;
+    return (d == 2048 || d == 4096 || d == 8192) && (g == 512 || g == 1024 || g == 2048) && d % g == 0;
+}
+
+QaSsdParams ssd_sizes(const QaMamba2Params& p) {
+    QaSsdParams s = {};
+    s.batch = p.batch; s.seqlen = p.seqlen; s.nheads = heads_of(p); s.headdim = p.headdim; s.dstate = p.d_state;
+    s.ngroups = p.ngroups; s.chunk_size = p.chunk_size;
+    return s;
+}
+
+Mamba2Buffers carve(const QaMamba2Params& p, void* base, bool step) {
+    const int64_t t = static_cast<int64_t>(p.batch) * p.seqlen, bc = static_cast<int64_t>(p.ngroups) * p.d_state;
+    Carver c{static_cast<uint8_t*>(base)};
+    Mamba2Buffers b;
+    b.zxbcdt = c.take<int8_t>(t * p.in_proj.n);
+    b.x = c.take<int8_t>(t * p.d_inner);
+    b.B = c.take<int8_t>(t * bc);
+    b.C = c.take<int8_t>(t * bc);
+    b.yq = c.take<int8_t>(t * p.d_inner);
+    b.y = c.take<__half>(t * p.d_inner * 2);
+    b.yn = c.take<__half>(norm_fuses(p) ? 0 : t * p.d_inner * 2);
+    b.w8.bytes = std::max(expanded_bytes(p.in_proj, t), expanded_bytes(p.out_proj, t));
+    b.w8.p = c.take<uint8_t>(b.w8.bytes);
+    b.ssd.bytes = step ? 0 : ssd_workspace_layout(ssd_sizes(p)).total;
+    b.ssd.p = c.take<uint8_t>(b.ssd.bytes);
+    b.total = c.off;
+    return b;
+}
+
+int validate(const QaMamba2Params* p) {
+    if (!p) return QA_ERR_NULL;
+    if (p->batch < 1 || p->seqlen < 1 || p->batch > 65535 || static_cast<int64_t>(p->batch) * p->seqlen > 0x7fffffff) return QA_ERR_SHAPE;
+    if (p->headdim < 1 || p->d_inner % p->headdim != 0 || p->ngroups < 1 || heads_of(*p) % p->ngroups != 0) return QA_ERR_SHAPE;
+    if (p->d_conv < 2 || p->d_conv > 4 || p->d_inner % 16 != 0 || (p->ngroups * p->d_state) % 4 != 0) return QA_ERR_UNSUPPORTED;
+    for (const QaLinearParams* w : {&p->in_proj, &p->out_proj})
+        if (!linear_ok(*w)) return QA_ERR_NULL;
+    const int64_t used = 2LL * p->d_inner + 2LL * p->ngroups * p->d_state + heads_of(*p);
+    if (p->in_proj.k != p->d_model || p->in_proj.n < used || p->in_proj.n % 4 != 0 || p->out_proj.k != p->d_inner) return QA_ERR_SHAPE;
+    if (p->conv_state_len != p->d_conv && p->conv_state_len != p->d_conv - 1) return QA_ERR_SHAPE;
+    if (p->norm_group_size < 1 || p->d_inner % p->norm_group_size != 0) return QA_ERR_SHAPE;
+    return QA_OK;
+}
+
+int ready(const QaMamba2Params* p, bool step) {
+    QA_TRY(validate(p));
+    if (!p->hidden || !p->out || !p->workspace || !p->conv_weight || !p->A_log || !p->norm_weight) return QA_ERR_NULL;
+    if (!p->x_out_scales || !p->B_out_scales || !p->C_out_scales) return QA_ERR_NULL;
+    if (step && (!p->conv_state || !p->ssm_state)) return QA_ERR_NULL;
+    if (p->workspace_bytes < carve(*p, nullptr, step).total || (reinterpret_cast<uintptr_t>(p->workspace) & 255u)) return QA_ERR_STRIDE;
+    return QA_OK;
+}
+
+QaConv2Params conv2_of(const QaMamba2Params& p, const Mamba2Buffers& b) {
+    QaConv2Params c = {};
+    const int64_t bc = static_cast<int64_t>(p.ngroups) * p.d_state, len = p.seqlen;
+    c.batch = p.batch; c.dim = static_cast<int>(p.d_inner + 2 * bc); c.seqlen = p.seqlen; c.width = p.d_conv;
+    c.silu_activation = 1;
+    c.x_dim = p.d_inner; c.x_headdim = p.headdim; c.d_state = p.d_state; c.n_groups = p.ngroups;
+    c.nhead_groups = p.conv_nhead_groups; c.ndim_groups = p.conv_ndim_groups;
+    c.conv_state_len = p.conv_state_len;
+    c.xBC_batch_stride = len * p.in_proj.n; c.xBC_l_stride = p.in_proj.n; c.xBC_c_stride = 1;
+    c.x_batch_stride = len * p.d_inner; c.x_l_stride = p.d_inner; c.x_c_stride = 1;
+    c.B_batch_stride = len * bc; c.B_l_stride = bc; c.B_c_stride = 1;
+    c.C_batch_stride = len * bc; c.C_l_stride = bc; c.C_c_stride = 1;
+    c.weight_c_stride = p.d_conv; c.weight_width_stride = 1;
+    c.conv_state_batch_stride = p.conv_state_batch_stride; c.conv_state_c_stride = p.conv_state_c_stride; c.conv_state_l_stride = p.conv_state_l_stride;
+    c.xBC = b.zxbcdt + p.d_inner; c.weight = p.conv_weight; c.bias = p.conv_bias;
+    c.x = b.x; c.B = b.B; c.C = b.C; c.conv_state = p.conv_state;
+    c.x_out_scales = p.x_out_scales; c.B_out_scales = p.B_out_scales; c.C_out_scales = p.C_out_scales;
+    c.x_head_group_range = p.conv_head_range; c.x_dim_group_range = p.conv_dim_range;
+    c.scale_x = p.scale_x; c.scale_B = p.scale_B; c.scale_C = p.scale_C;
+    c.scale_wx = p.scale_wx; c.scale_wB = p.scale_wB; c.scale_wC = p.scale_wC;
+    c.scale_bx = p.scale_bx; c.scale_bB = p.scale_bB; c.scale_bC = p.scale_bC;
+    return c;
+}
+
+// gated norm, Hadamard rotation and quantisation, out_proj
+int mamba2_tail(const QaMamba2Params& p, const Mamba2Buffers& b, void* stream) {
+    const int rows = p.batch * p.seqlen;
+    QaNormGatedParams n = {};
+    n.rows = rows; n.dim = p.d_inner; n.group_size = p.norm_group_size;
+    n.norm_before_gate = p.norm_before_gate; n.out_mode = 0;
+    n.eps = p.norm_eps; n.z_scale = p.norm_z_scale;
+    n.x_row_stride = p.d_inner; n.z_row_stride = p.in_proj.n; n.out_row_stride = p.d_inner;
+    n.x = b.y; n.weight = p.norm_weight; n.qz = b.zxbcdt; n.out = b.yn;
+    if (norm_fuses(p)) {
+        QaHadamardParams h = {};
+        h.rows = rows; h.dim = p.d_inner; h.scale = p.had_scale; h.out_row_stride = p.d_inner; h.out = b.yq;
+        QA_TRY(qa_rmsnorm_gated_hadamard_quant(&n, &h, stream));
+    } else {
+        QA_TRY(qa_rmsnorm_gated(&n, stream));
+        QA_TRY(hadamard(b.yn, b.yq, rows, p.d_inner, p.had_scale, stream));
+    }
+    return project(p.out_proj, b.yq, p.d_inner, rows, p.out, QA_OUT_F16, false, b.w8, stream);
+}
+
+}  // namespace
+}  // namespace qa
+
+extern "C" int64_t qa_mamba1_workspace_bytes(const QaMamba1Params* p, int) {
+    using namespace qa;
+    return validate(p) == QA_OK ? carve(*p, nullptr).total : 0;
+}
+
+extern "C" int qa_mamba1_forward(const QaMamba1Params* p, void* stream) {
+    using namespace qa;
+    QA_TRY(ready(p, false));
+    const Mamba1Buffers b = carve(*p, p->workspace);
+    const int rows = p->batch * p->seqlen, d = p->d_inner;
+    const int64_t len = p->seqlen;
+    QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.xz, QA_OUT_I8, true, b.w8, stream));
+
+    QaConv2Params c = {};                    // every channel an x channel with one output scale
+    c.batch = p->batch; c.dim = d; c.seqlen = p->seqlen; c.width = p->d_conv;
+    c.silu_activation = 1;
+    c.x_dim = d; c.x_headdim = d; c.d_state = 1; c.n_groups = 1;
+    c.conv_state_len = p->conv_state_len;
+    c.xBC_batch_stride = len * 2 * d; c.xBC_l_stride = 2 * d; c.xBC_c_stride = 1;
+    c.x_batch_stride = len * d; c.x_l_stride = d; c.x_c_stride = 1;
+    c.weight_c_stride = p->d_conv; c.weight_width_stride = 1;
+    c.conv_state_batch_stride = p->conv_state_batch_stride; c.conv_state_c_stride = p->conv_state_c_stride; c.conv_state_l_stride = p->conv_state_l_stride;
+    c.xBC = b.xz; c.weight = p->conv_weight; c.bias = p->conv_bias; c.x = b.x; c.conv_state = p->conv_state;
+    c.scale_x = p->conv_scale_x; c.scale_wx = p->conv_scale_w; c.scale_bx = p->conv_scale_b; c.x_out_scale = p->conv_scale_out;
+    QA_TRY(conv_channel_last_fwd(c, static_cast<hipStream_t>(stream)));
+
+    QA_TRY(project(p->x_proj, b.x, d, rows, b.x_dbl, QA_OUT_I8, false, b.w8, stream));
+    QA_TRY(project(p->dt_proj, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, true, b.w8, stream));
+
+    QaSScanParams s = scan_sizes(*p);
+    const int64_t dbl = p->x_proj.n;
+    s.delta_softplus = p->delta_softplus;
+    s.token_major = 1;
+    s.u_batch_stride = len * d; s.u_l_stride = d; s.u_d_stride = 1;
+    s.delta_batch_stride = len * d; s.delta_l_stride = d; s.delta_d_stride = 1;
+    s.z_batch_stride = len * 2 * d; s.z_l_stride = 2 * d; s.z_d_stride = 1;
+    s.B_batch_stride = s.C_batch_stride = len * dbl;
+    s.B_l_stride = s.C_l_stride = dbl;
+    s.B_dstate_stride = s.C_dstate_stride = 1;
+    s.A_d_stride = p->d_state; s.A_dstate_stride = 1;
+    s.out_batch_stride = len * d; s.out_l_stride = d; s.out_d_stride = 1;
+    s.u = b.x; s.delta = b.dt; s.A_log = p->A_log; s.B = b.x_dbl + p->dt_rank; s.C = s.B + p->d_state;
+    s.D = p->D; s.delta_bias = p->dt_bias; s.z = b.xz + d;
+    s.scale_u = p->u_scale; s.scale_delta = p->dt_scale; s.scale_A = p->A_scale; s.scale_B = p->B_scale; s.scale_C = p->C_scale;
+    s.scale_D = p->D_scale; s.scale_delta_bias = p->dt_bias_scale; s.scale_z = p->z_scale; s.scale_ssm_state = p->ssm_state_scale;
+    s.out = b.y;
+    if (p->state_is_fp32) s.last_state_f32 = static_cast<float*>(p->ssm_state);
+    else s.last_state_i8 = static_cast<int8_t*>(p->ssm_state);
+    s.workspace = b.scan.p; s.workspace_bytes = b.scan.bytes;
+    QA_TRY(qa_sscan_fwd(&s, stream));
+
+    QA_TRY(hadamard(b.y, b.yq, rows, d, p->had_scale, stream));
+    return project(p->out_proj, b.yq, d, rows, p->out, QA_OUT_F16, false, b.w8, stream);
+}
+
+extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
+    using namespace qa;
+    QA_TRY(ready(p, true));
+    if (p->seqlen != 1) return QA_ERR_SHAPE;
+    const Mamba1Buffers b = carve(*p, p->workspace);
+    const int rows = p->batch, d = p->d_inner;
+    QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.xz, QA_OUT_I8, false, b.w8, stream));
+
+    QaConvParams c = {};
+    c.batch = rows; c.dim = d; c.seqlen = 1; c.width = p->d_conv;
+    c.silu_activation = 1;
+    c.x_batch_stride = 2 * d; c.x_c_stride = 1; c.x_l_stride = 1;
+    c.out_batch_stride = d; c.out_c_stride = 1; c.out_l_stride = 1;
+    c.weight_c_stride = p->d_conv; c.weight_width_stride = 1;
+    c.conv_state_batch_stride = p->conv_state_batch_stride; c.conv_state_c_stride = p->conv_state_c_stride; c.conv_state_l_stride = p->conv_state_l_stride;
+    c.conv_state_len = p->conv_state_len;
+    c.x = b.xz; c.weight = p->conv_weight; c.bias = p->conv_bias; c.out = b.x; c.conv_state = p->conv_state;
+    c.scale_x = p->conv_scale_x; c.scale_w = p->conv_scale_w; c.scale_b = p->conv_scale_b; c.scale_out = p->conv_scale_out;
+    QA_TRY(qa_causal_conv1d_update(&c, stream));
+
+    QA_TRY(project(p->x_proj, b.x, d, rows, b.x_dbl, QA_OUT_I8, false, b.w8, stream));
+    QA_TRY(project(p->dt_proj, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, false, b.w8, stream));
+
+    QaSsmUpdateParams u = {};
+    u.batch = rows; u.nheads = 1; u.dim = d; u.dstate = p->d_state; u.ngroups = 1;
+    u.dt_softplus = p->delta_softplus;
+    u.state_is_fp32 = p->state_is_fp32;
+    u.state_batch_stride = static_cast<int64_t>(d) * p->d_state; u.state_head_stride = u.state_batch_stride;
+    u.state_dim_stride = p->d_state; u.state_dstate_stride = 1;
+    u.x_batch_stride = u.x_head_stride = d; u.x_dim_stride = 1;
+    u.dt_batch_stride = u.dt_head_stride = d; u.dt_dim_stride = 1;
+    u.dt_bias_head_stride = d; u.dt_bias_dim_stride = 1;
+    u.A_head_stride = u.state_batch_stride; u.A_dim_stride = p->d_state; u.A_dstate_stride = 1;
+    u.B_batch_stride = u.B_group_stride = p->x_proj.n; u.B_dstate_stride = 1;
+    u.C_batch_stride = u.C_group_stride = p->x_proj.n; u.C_dstate_stride = 1;
+    u.D_head_stride = d; u.D_dim_stride = 1;
+    u.z_batch_stride = u.z_head_stride = 2 * d; u.z_dim_stride = 1;
+    u.out_batch_stride = u.out_head_stride = d; u.out_dim_stride = 1;
+    u.state = p->ssm_state; u.x = b.x; u.dt = b.dt; u.dt_bias = p->dt_bias; u.A_log = p->A_log;
+    u.B = b.x_dbl + p->dt_rank; u.C = u.B + p->d_state; u.D = p->D; u.z = b.xz + d;
+    u.x_scale = p->u_scale; u.dt_scale = p->dt_scale; u.dt_bias_scale = p->dt_bias_scale; u.A_log_scale = p->A_scale;
+    u.state_scale = p->ssm_state_scale; u.B_scale = p->B_scale; u.C_scale = p->C_scale; u.D_scale = p->D_scale; u.z_scale = p->z_scale;
+    u.out = b.y;
+    QA_TRY(qa_ssm_state_update(&u, stream));
+
+    QA_TRY(hadamard(b.y, b.yq, rows, d, p->had_scale, stream));
+    return project(p->out_proj, b.yq, d, rows, p->out, QA_OUT_F16, false, b.w8, stream);
+}
+
+extern "C" int64_t qa_mamba2_workspace_bytes(const QaMamba2Params* p, int step) {
+    using namespace qa;
+    return validate(p) == QA_OK ? carve(*p, nullptr, step != 0).total : 0;
+}
+
+extern "C" int qa_mamba2_forward(const QaMamba2Params* p, void* stream) {
+    using namespace qa;
+    QA_TRY(ready(p, false));
+    const Mamba2Buffers b = carve(*p, p->workspace, false);
+    const int rows = p->batch * p->seqlen;
+    QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.zxbcdt, QA_OUT_I8, false, b.w8, stream));
+    QA_TRY(conv_channel_last_fwd(conv2_of(*p, b), static_cast<hipStream_t>(stream)));
+
+    QaSsdParams s = ssd_sizes(*p);
+    s.dt_softplus = p->delta_softplus;
+    s.D_has_hdim = p->D_has_hdim;
+    s.nhead_groups = p->nhead_groups; s.ndim_groups = p->ndim_groups;
+    s.final_state_is_fp32 = p->state_is_fp32;
+    s.dt_row_stride = p->in_proj.n;
+    s.dt_min = p->dt_min; s.dt_max = p->dt_max;
+    s.x = b.x; s.B = b.B; s.C = b.C;
+    s.dt = b.zxbcdt + 2 * p->d_inner + 2 * p->ngroups * p->d_state;
+    s.A_log = p->A_log; s.D = p->D; s.dt_bias = p->dt_bias;
+    s.x_scale = p->x_scales; s.dt_scale = p->dt_scale; s.A_log_scale = p->A_log_scale; s.B_scale = p->B_scale; s.C_scale = p->C_scale;
+    s.D_scale = p->D_scale; s.state_scale = p->ssm_state_scale;
+    s.x_head_group_range = p->head_range; s.x_dim_group_range = p->dim_range;
+    s.out = b.y; s.final_states = p->ssm_state;
+    s.workspace = b.ssd.p; s.workspace_bytes = b.ssd.bytes;
+    QA_TRY(qa_ssd_chunk_scan_fwd(&s, stream));
+    return mamba2_tail(*p, b, stream);
+}
+
+extern "C" int qa_mamba2_step(const QaMamba2Params* p, void* stream) {
+    using namespace qa;
+    QA_TRY(ready(p, true));
+    if (p->seqlen != 1) return QA_ERR_SHAPE;
+    const Mamba2Buffers b = carve(*p, p->workspace, true);
+    const int rows = p->batch, heads = heads_of(*p);
+    QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.zxbcdt, QA_OUT_I8, false, b.w8, stream));
+    const QaConv2Params c = conv2_of(*p, b);
+    QA_TRY(qa_quamba2_conv1d_update(&c, stream));
+
+    QaSsmUpdateParams u = {};
+    const int64_t bc = static_cast<int64_t>(p->ngroups) * p->d_state;
+    u.batch = rows; u.nheads = heads; u.dim = p->headdim; u.dstate = p->d_state; u.ngroups = p->ngroups;
+    u.dt_softplus = p->delta_softplus;
+    u.state_is_fp32 = p->state_is_fp32;
+    u.dt_bias_is_fp16 = 1;
+    u.nhead_groups = p->nhead_groups; u.ndim_groups = p->ndim_groups;
+    u.state_dstate_stride = 1; u.state_dim_stride = p->d_state;
+    u.state_head_stride = static_cast<int64_t>(p->headdim) * p->d_state; u.state_batch_stride = u.state_head_stride * heads;
+    u.x_batch_stride = p->d_inner; u.x_head_stride = p->headdim; u.x_dim_stride = 1;
+    u.dt_batch_stride = p->in_proj.n; u.dt_head_stride = 1;
+    u.dt_bias_head_stride = 1;
+    u.A_head_stride = 1;
+    u.B_batch_stride = u.C_batch_stride = bc; u.B_group_stride = u.C_group_stride = p->d_state; u.B_dstate_stride = u.C_dstate_stride = 1;
+    u.D_head_stride = p->D_has_hdim ? p->headdim : 1; u.D_dim_stride = p->D_has_hdim ? 1 : 0;
+    u.out_batch_stride = p->d_inner; u.out_head_stride = p->headdim; u.out_dim_stride = 1;
+    u.state = p->ssm_state; u.x = b.x; u.dt = b.zxbcdt + 2 * p->d_inner + 2 * bc; u.dt_bias = p->dt_bias; u.A_log = p->A_log;
+    u.B = b.B; u.C = b.C; u.D = p->D;
+    u.x_scale = p->x_scales; u.dt_scale = p->dt_scale; u.A_log_scale = p->A_log_scale; u.state_scale = p->ssm_state_scale;
+    u.B_scale = p->B_scale; u.C_scale = p->C_scale; u.D_scale = p->D_scale;
+    u.x_head_group_range = p->head_range; u.x_dim_group_range = p->dim_range;
+    u.out = b.y;
+    QA_TRY(qa_ssm_state_update(&u, stream));
+    return mamba2_tail(*p, b, stream);
+}

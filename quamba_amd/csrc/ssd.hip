@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void ssd_cumsum_kernel(QaSsdParams p, float* d
         const int t = c * Q + lane * E + e;
         float v = 0.0f;
         if (t < p.seqlen) {
-            const int64_t di = (static_cast<int64_t>(b) * p.seqlen + t) * p.nheads + h;
+            const int64_t di = (static_cast<int64_t>(b) * p.seqlen + t) * ssd_dt_stride(p) + h;
             if (p.dt_is_fp32) {
                 v = static_cast<const float*>(p.dt)[di];
             } else {

@@ -11,6 +11,9 @@ constexpr float kSsdLog2e = 1.44269504088896341f;
 
 __device__ __forceinline__ float ssd_exp(float x) { return __builtin_amdgcn_exp2f(x * kSsdLog2e); }
 
+// elements between the steps of dt
+__device__ __forceinline__ int ssd_dt_stride(const QaSsdParams& p) { return p.dt_row_stride ? p.dt_row_stride : p.nheads; }
+
 struct SsdWorkspace {            // sections of the workspace (byte offsets), see qa_ssd_workspace_bytes
     int64_t dt, dA, prev, xs, srow, total;
 };

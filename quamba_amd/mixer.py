@@ -6,9 +6,9 @@ in_proj (seqlen-last int8) -> x | z halves -> causal conv -> x_proj -> dt | B | 
 form with the rolling conv state and the recurrent state updated in place.  This is the caller the
 operators are built for; it owns no arithmetic of its own.
 
-Two things the reference does with a copy are done in place here because the kernels take strides:
-the conv and the scan read the x and z halves of in_proj's buffer directly, and B / C are passed to the
-scan as transposed views only when that is free (they are tiny; a contiguous copy is made otherwise).
+A call goes to the library as a whole (qa_mamba1_forward / _step, qa_mamba2_forward / _step: every kernel of the layer
+enqueued by one call, activations row-major from in_proj to out_proj).  The same chain over the modules, one by one,
+serves what that call does not cover: replaced or hooked sub-modules, unusual sizes, strided states.
 """
 import copy
 import math
@@ -17,6 +17,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _layer_call, _lib
+from ._layer_call import _need, _ptr, linear_block
 from .conv import QCausalConv1D
 from .hadamard import QHadamard
 from .linear import (W4A8B8O8Linear, W4A8B8O8LinearParallel, W4A8B16O16Linear, W8A8B8O8Linear, W8A8B8O8LinearParallel,
@@ -82,7 +84,41 @@ class W8A8QMamba(nn.Module):
         """The form the linear classes of this precision take an activation scale in (a float here)."""
         return float(torch.as_tensor(act_scales[key]).item())
 
-    @torch.no_grad()
+    def _native_modules(self):
+        """The sub-modules in the order of the library call, or None when one of them is not the stock class."""
+        m = self._modules
+        mods = (m["in_proj"], m["conv1d"], m["x_proj"], m["dt_proj"], m["selective_scan"], m["had"], m["out_proj"])
+        want = (self._in_proj_cls, QCausalConv1D, self._x_proj_cls, W8A8B8O8Linear, QSScan, QHadamard, self._out_proj_cls)
+        for md, cls in zip(mods, want):
+            if type(md) is not cls:
+                return None
+        return mods
+
+    def _scalars(self):
+        m = self._modules
+        c, s, h = m["conv1d"], m["selective_scan"], m["had"]
+        return (c.input_scale, c.weight_scale, c.bias_scale, c.output_scale, id(c.bias), s.delta_softplus, h.x_H_scale, h.had_scale,
+                getattr(m["in_proj"], "alpha", 0.0), getattr(m["x_proj"], "alpha", 0.0), m["dt_proj"].alpha,
+                getattr(m["out_proj"], "alpha", 0.0))
+
+    def _native_block(self, dev):
+        p, D, N = _lib.QaMamba1Params(), self.d_inner, self.d_state
+        c, s = self.conv1d, self.selective_scan
+        p.d_model, p.d_inner, p.d_state, p.d_conv, p.dt_rank = self.d_model, D, N, self.d_conv, self.dt_rank
+        p.conv_state_len = self.d_conv
+        p.delta_softplus = int(bool(s.delta_softplus))
+        for name in ("in_proj", "x_proj", "dt_proj", "out_proj"):
+            setattr(p, name, linear_block(getattr(self, name), dev))
+        p.conv_weight, p.conv_bias = _ptr(c.weight, torch.int8, D * self.d_conv, dev), _ptr(c.bias, torch.int8, D, dev)
+        p.conv_scale_x, p.conv_scale_w, p.conv_scale_b, p.conv_scale_out = c.input_scale, c.weight_scale, c.bias_scale, c.output_scale
+        p.A_log = _ptr(s.A_log, torch.int8, D * N, dev)
+        p.D, p.dt_bias = _ptr(s.D, torch.int8, D, dev), _ptr(s.dt_bias, torch.int8, D, dev)
+        for name in ("A_scale", "D_scale", "dt_bias_scale", "u_scale", "dt_scale", "B_scale", "C_scale", "z_scale", "ssm_state_scale"):
+            setattr(p, name, _ptr(getattr(s, name), torch.float32, 1, dev))
+        p.had_scale = self.had.had_scale / float(self.had.x_H_scale)
+        widths = (self.d_conv, self.d_conv - 1)                        # of the conv state, in forward and in step
+        return p, (D, (D, N), (widths, widths))
+
     def forward(self, hidden_states, inference_params=None, conv_state=None, ssm_state=None):
         """hidden_states int8 (B, L, d_model) -> fp16 (B, L, d_model).  With conv_state / ssm_state (or an
         inference_params cache) the states after the last token are stored into them."""
@@ -92,6 +128,14 @@ class W8A8QMamba(nn.Module):
             if inference_params.seqlen_offset > 0:
                 out, _, _ = self.step(hidden_states, conv_state, ssm_state)
                 return out
+        out = _layer_call.call(self, hidden_states, conv_state, ssm_state, False)
+        if out is not None:
+            return out.view(batch, seqlen, -1)
+        return self._forward_modules(hidden_states, conv_state, ssm_state)
+
+    @torch.no_grad()
+    def _forward_modules(self, hidden_states, conv_state, ssm_state):
+        batch, seqlen, _ = hidden_states.shape
         xz = self.in_proj.to_seqlen_last(hidden_states)                 # (B, 2D, L), strides (L, B*L, 1)
         x, z = xz.chunk(2, dim=1)                                       # views
         if conv_state is not None:
@@ -119,9 +163,15 @@ class W8A8QMamba(nn.Module):
             ssm_state.copy_(last_state)
         return self.out_proj(self.had(y))                               # (B, L, d_model) fp16
 
-    @torch.no_grad()
     def step(self, hidden_states, conv_state, ssm_state):
         assert hidden_states.shape[1] == 1, "Only support decoding with 1 token at a time for now"
+        out = _layer_call.call(self, hidden_states, conv_state, ssm_state, True)
+        if out is None:
+            out = self._step_modules(hidden_states, conv_state, ssm_state)
+        return out.unsqueeze(1), conv_state, ssm_state
+
+    @torch.no_grad()
+    def _step_modules(self, hidden_states, conv_state, ssm_state):
         xz = self.in_proj(hidden_states.squeeze(1))                     # (B, 2D)
         x, z = xz.chunk(2, dim=-1)
         x = self.conv1d.update(x, conv_state)
@@ -132,8 +182,7 @@ class W8A8QMamba(nn.Module):
             dt = dt.contiguous()
         dt = self.dt_proj(dt)
         y, ssm_state = self.selective_scan.update(ssm_state, x, dt, B, C, z=z)
-        out = self.out_proj(self.had(y))
-        return out.unsqueeze(1), conv_state, ssm_state
+        return self.out_proj(self.had(y))
 
     def allocate_inference_cache(self, batch_size, max_seqlen=None, dtype=None, **kwargs):
         device = self.out_proj.weight.device
@@ -209,10 +258,80 @@ class W4A8QMamba2(nn.Module):
     def _split(self, zxbcdt):
         return torch.split(zxbcdt, [self.d_ssm, self.d_ssm + 2 * self.ngroups * self.d_state, self.nheads], dim=-1)
 
-    @torch.no_grad()
+    def _native_modules(self):
+        """The sub-modules in the order of the library call, or None when one of them is not the stock class."""
+        from .chunk_scan import Quamba2ChunkScan
+        from .conv import Quamb2Conv1D
+        from .norm import QRMSNormGated
+        m = self._modules
+        mods = (m["in_proj"], m["conv1d"], m["qchunk_scan"], m["norm"], m["had"], m["out_proj"])
+        want = (self._in_proj_cls, Quamb2Conv1D, Quamba2ChunkScan, QRMSNormGated, QHadamard, self._out_proj_cls)
+        for md, cls in zip(mods, want):
+            if type(md) is not cls:
+                return None
+        return mods
+
+    def _scalars(self):
+        m = self._modules
+        c, s, n, h = m["conv1d"], m["qchunk_scan"], m["norm"], m["had"]
+        return (c.x_scale, c.B_scale, c.C_scale, c.wx_scale, c.wB_scale, c.wC_scale, c.bx_scale, c.bB_scale, c.bC_scale, id(c.bias),
+                id(c.x_head_group_range), id(c.x_dim_group_range), id(s.x_head_group_range), id(s.x_dim_group_range), s.chunk_size,
+                s.delta_softplus, s.dt_limit, s.D_has_hdim, n.eps, n.z_scale, n.group_size, n.norm_before_gate, n.use_float16_output,
+                h.x_H_scale, h.had_scale, getattr(m["out_proj"], "alpha", 0.0))
+
+    def _native_block(self, dev):
+        p, D, N, G, H = _lib.QaMamba2Params(), self.d_ssm, self.d_state, self.ngroups, self.nheads
+        c, s, n = self.conv1d, self.qchunk_scan, self.norm
+        _need(n.use_float16_output and n.bias is None and self.had.dim == D)
+        # the kernels' state counts: others run padded, module by module
+        _need(self.headdim % 64 != 0 or N in (64, 128) or N > 128 or s.chunk_size not in (64, 128, 256))
+        p.d_model, p.d_inner, p.d_state, p.d_conv, p.headdim, p.ngroups = self.d_model, D, N, self.d_conv, self.headdim, G
+        p.chunk_size, p.conv_state_len = s.chunk_size, self.d_conv
+        p.delta_softplus, p.D_has_hdim = int(bool(s.delta_softplus)), int(bool(s.D_has_hdim))
+        p.in_proj, p.out_proj = linear_block(self.in_proj, dev), linear_block(self.out_proj, dev)
+        conv_dim = D + 2 * G * N
+        p.conv_weight, p.conv_bias = _ptr(c.weight, torch.int8, conv_dim * self.d_conv, dev), _ptr(c.bias, torch.int8, conv_dim, dev)
+
+        def groups(hr, dr):
+            if hr is None:
+                return 0, 0, None, None
+            nh, nd = hr.shape[1], dr.shape[2]
+            return nh, nd, _ptr(hr, torch.int32, G * nh, dev), _ptr(dr, torch.int32, G * nh * nd, dev)
+
+        p.conv_nhead_groups, p.conv_ndim_groups, p.conv_head_range, p.conv_dim_range = groups(c.x_head_group_range, c.x_dim_group_range)
+        p.nhead_groups, p.ndim_groups, p.head_range, p.dim_range = groups(s.x_head_group_range, s.x_dim_group_range)
+        cg, sg = p.conv_nhead_groups * p.conv_ndim_groups, p.nhead_groups * p.ndim_groups
+        p.x_out_scales = _ptr(c.x_out_scales, torch.float32, G * cg if cg else 1, dev)
+        p.B_out_scales, p.C_out_scales = (_ptr(t, torch.float32, G if cg else 1, dev) for t in (c.B_out_scales, c.C_out_scales))
+        for name in ("x", "B", "C"):
+            setattr(p, "scale_" + name, getattr(c, name + "_scale"))
+            setattr(p, "scale_w" + name, getattr(c, "w" + name + "_scale"))
+            setattr(p, "scale_b" + name, getattr(c, "b" + name + "_scale") or 0.0)
+        p.dt_min, p.dt_max = float(s.dt_limit[0]), float(min(s.dt_limit[1], 3.0e38))
+        p.norm_eps, p.norm_z_scale, p.norm_before_gate = n.eps, float(n.z_scale), int(bool(n.norm_before_gate))
+        p.norm_group_size = D if n.group_size is None else n.group_size
+        p.norm_weight = _ptr(n.weight, torch.float16, D, dev)
+        p.had_scale = self.had.had_scale / float(self.had.x_H_scale)
+        p.A_log = _ptr(s.A_log, torch.int8, H, dev)
+        p.D = _ptr(s.D, torch.int8, D if s.D_has_hdim else H, dev)
+        p.dt_bias = _ptr(s.dt_bias, torch.float16, H, dev)
+        p.A_log_scale, p.dt_scale = _ptr(s.A_log_scale, torch.float32, 1, dev), _ptr(s.dt_scale, torch.float32, 1, dev)
+        p.D_scale = _ptr(s.D_scale, torch.float32, 1, dev) if s.D is not None else None
+        p.x_scales = _ptr(s.x_scales, torch.float32, G * sg if sg else 1, dev)
+        p.B_scale, p.C_scale = (_ptr(t, torch.float32, G if sg else 1, dev) for t in (s.B_scale, s.C_scale))
+        p.ssm_state_scale = _ptr(s.ssm_state_scale, torch.float32, G * sg * N if sg else 1, dev)
+        return p, (conv_dim, (H, self.headdim, N), ((self.d_conv,), (self.d_conv, self.d_conv - 1)))
+
     def forward(self, u, conv_state=None, ssm_state=None):
         """u int8 (B, L, d_model) -> fp16 (B, L, d_model); conv_state / ssm_state receive the states after
         the last token when given."""
+        out = _layer_call.call(self, u, conv_state, ssm_state, False)
+        if out is not None:
+            return out.view(u.shape[0], u.shape[1], -1)
+        return self._forward_modules(u, conv_state, ssm_state)
+
+    @torch.no_grad()
+    def _forward_modules(self, u, conv_state, ssm_state):
         batch, seqlen, _ = u.shape
         z, xBC, dt = self._split(self.in_proj(u))                   # views of (B, L, d_in_proj)
         if conv_state is not None:
@@ -236,14 +355,19 @@ class W4A8QMamba2(nn.Module):
             return self.norm.forward_hadamard(y, z, self.had)
         return self.had(self.norm(y, z))
 
-    @torch.no_grad()
     def step(self, hidden_states, conv_state, ssm_state):
         assert hidden_states.shape[1] == 1, "Only support decoding with 1 token at a time for now"
+        out = _layer_call.call(self, hidden_states, conv_state, ssm_state, True)
+        if out is None:
+            out = self._step_modules(hidden_states, conv_state, ssm_state)
+        return out.unsqueeze(1), conv_state, ssm_state
+
+    @torch.no_grad()
+    def _step_modules(self, hidden_states, conv_state, ssm_state):
         z, xBC, dt = self._split(self.in_proj(hidden_states.squeeze(1)))
         x, B, C = self.conv1d.update(xBC, conv_state)
         y = self.qchunk_scan.update(ssm_state, x, dt, B, C, z=None)
-        out = self.out_proj(self._norm_had(y.reshape(y.shape[0], self.d_ssm), z))
-        return out.unsqueeze(1), conv_state, ssm_state
+        return self.out_proj(self._norm_had(y.reshape(y.shape[0], self.d_ssm), z))
 
     def allocate_inference_cache(self, batch_size, max_seqlen=None, dtype=None, **kwargs):
         device = self.out_proj.weight.device

@@ -1,0 +1,78 @@
+"""The library call that enqueues a whole layer against the same layer run module by module: token counts around the
+edges of the scan's tiles and segments, both state types, states of three and four codes, one row (the single-row
+rules of the projections) and many; and what the call leaves to the modules."""
+import pytest
+import torch
+
+from quamba_amd import W4A8QMamba, W4A8QMamba2, W8A8QMamba, W8A8QMamba2, _layer_call
+from tests.test_mixer_variants_gpu import _mamba1, _mamba2, _ri
+
+pytestmark = pytest.mark.gpu
+MIXERS = [(W8A8QMamba, _mamba1), (W4A8QMamba, _mamba1), (W8A8QMamba2, _mamba2), (W4A8QMamba2, _mamba2)]
+
+
+def _states(m, dev, g, batch, dtype, width):
+    dim = m.conv1d.weight.shape[0]
+    conv = _ri(dev, g, batch, width, dim).transpose(1, 2) if hasattr(m, "qchunk_scan") else _ri(dev, g, batch, dim, width)
+    shape = (batch, m.nheads, m.headdim, m.d_state) if hasattr(m, "qchunk_scan") else (batch, m.d_inner, m.d_state)
+    ssm = _ri(dev, g, *shape) if dtype == torch.int8 else torch.randn(shape, device=dev, generator=g) * 0.1
+    return conv, ssm
+
+
+def _close(got, want, conv, ssm):
+    scale = float(want.float().abs().max()) + 1e-6
+    diff = (got.float() - want.float()).abs()
+    # fp16 scan outputs may differ in the last place, and int8 codes made of them by one step
+    assert float(diff.max()) <= 2e-2 * scale and float(diff.mean()) <= 1e-3 * scale
+    assert torch.equal(conv[0], conv[1])
+    a, b = ssm[0].float(), ssm[1].float()
+    if ssm[0].dtype == torch.int8:
+        assert float((a - b).abs().max()) <= 1 and float((a != b).float().mean()) <= 5e-3
+    else:
+        assert float((a - b).abs().max()) <= 1e-3 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("cls,build", MIXERS)
+@pytest.mark.parametrize("batch,seqlen,dtype,width", [(1, 1, torch.int8, 4), (1, 3, torch.float32, 3), (3, 33, torch.int8, 4),
+                                                      (2, 64, torch.float32, 4), (1, 257, torch.int8, 3), (2, 1029, torch.float32, 4)])
+def test_forward(dev, cls, build, batch, seqlen, dtype, width):
+    m, g = build(cls, dev, seed=seqlen)
+    width = 4 if hasattr(m, "qchunk_scan") else width            # (the second family's forward takes the whole window)
+    h = _ri(dev, g, batch, seqlen, 256)
+    conv, ssm = _states(m, dev, g, batch, dtype, width)
+    conv2, ssm2 = conv.clone(), ssm.clone()
+    out = _layer_call.call(m, h, conv, ssm, False)
+    assert out is not None, "the library call has to take this"
+    want = m._forward_modules(h, conv2, ssm2)
+    _close(out.view(batch, seqlen, -1), want, (conv, conv2), (ssm, ssm2))
+    assert torch.equal(m.forward(h), out.view(batch, seqlen, -1))          # without states
+
+
+@pytest.mark.parametrize("cls,build", MIXERS)
+@pytest.mark.parametrize("batch,dtype,width", [(1, torch.int8, 4), (1, torch.float32, 3), (7, torch.int8, 4), (33, torch.float32, 4), (70, torch.int8, 3)])
+def test_step(dev, cls, build, batch, dtype, width):
+    m, g = build(cls, dev, seed=batch)
+    h = _ri(dev, g, batch, 1, 256)
+    conv, ssm = _states(m, dev, g, batch, dtype, width)
+    conv2, ssm2 = conv.clone(), ssm.clone()
+    out = _layer_call.call(m, h, conv, ssm, True)
+    assert out is not None, "the library call has to take this"
+    want = m._step_modules(h, conv2, ssm2)
+    _close(out, want, (conv, conv2), (ssm, ssm2))
+
+
+@pytest.mark.parametrize("cls,build", MIXERS[:1] + MIXERS[3:])
+def test_changed_modules_are_seen(dev, cls, build):
+    m, g = build(cls, dev, seed=5)
+    h = _ri(dev, g, 2, 20, 256)
+    first = m.forward(h)
+    m.had.x_H_scale *= 2.0                                     # a scale, by value
+    second = m.forward(h)
+    assert not torch.equal(first, second) and torch.equal(second, m._forward_modules(h, None, None))
+    m.conv1d.weight = m.conv1d.weight.flip(0).contiguous()     # a buffer, by identity
+    third = m.forward(h)
+    assert not torch.equal(third, second) and torch.equal(third, m._forward_modules(h, None, None))
+    seen = []
+    hook = m.conv1d.register_forward_hook(lambda *a: seen.append(1))
+    assert torch.equal(m.forward(h), third) and seen           # hooked modules run one by one
+    hook.remove()
