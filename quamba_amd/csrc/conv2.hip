@@ -22,7 +22,6 @@ namespace qa {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kRun = 64;          // time steps per wave unless the launch picks more
 constexpr int kBatchLoads = 8;    // loads in flight per lane
 
 struct Part {
@@ -89,7 +88,7 @@ __device__ __forceinline__ int8_t* out_ptr(const QaConv2Params& p, const Part& p
     return p.C + b * p.C_batch_stride + local * p.C_c_stride;
 }
 
-// grid: x = blocks of 256 channels, y = blocks of 4 runs of kRun steps (one run per wave), z = batch
+// grid: x = blocks of 256 channels, y = blocks of 4 runs of `run` steps (one run per wave), z = batch
 template <bool SILU>
 __global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, int run) {
     const int lane = threadIdx.x & 63;
@@ -267,14 +266,15 @@ int validate(const QaConv2Params* p, bool update) {
 
 namespace qa {
 int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
-    // Steps per wave: 64, 128 or 256, whichever needs the fewest rounds of resident waves (seven per SIMD) times its
-    // own length plus a wave's set-up (taps, scales: about 24 steps' worth).  Batch 16 x 1024 steps x 10240 channels
-    // is 10240 waves of 64 steps on 7168 places - a second round at a third of the occupancy - or 5120 of 128.
-    int run = kRun;
+    // Steps per wave: 8 to 256, whichever needs the fewest rounds of resident waves (seven per SIMD) times its own length
+    // plus a wave's set-up (taps, scales: about 24 steps' worth).  Batch 16 x 1024 steps x 10240 channels is 10240 waves
+    // of 64 steps on 7168 places - a second round at a third of the occupancy - or 5120 of 128.  A short prompt
+    // (1 x 512 x 1536 channels: 48 waves of 64 steps, one after the other 19 us) takes short runs.
+    int run = kBatchLoads;
     {
         const int64_t ch_blocks = (p.dim + 255) / 256, places = 7 * 4 * 256;
         int64_t best = -1;
-        for (int r = 64; r <= 256; r *= 2) {
+        for (int r = kBatchLoads; r <= 256; r *= 2) {
             const int64_t waves = ch_blocks * (((p.seqlen + r - 1) / r + 3) / 4 * 4) * p.batch;
             const int64_t cost = ((waves + places - 1) / places) * (r + 24);
             if (best < 0 || cost < best) { best = cost; run = r; }
