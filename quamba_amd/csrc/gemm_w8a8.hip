@@ -7,6 +7,7 @@
 // csrc/linear/quant_linear_fwd_gemv_kernel.cuh:56-60 (roundf variant).
 // The tiling, LDS layout and epilogue are in gemm_core.hpp.
 #include "gemm_core.hpp"
+#include "gemv.hpp"
 
 // Built with -DQA_GEMM_CLK (bench.py --gemm-phase-clocks, never the product library) thread 0 of every workgroup of
 // the tiled kernel records the shader clock and the constant 100 MHz clock at four points - start, first fragments
@@ -333,6 +334,18 @@ extern "C" int qa_gemm_w8a8(const QaGemmW8A8Params* p, void* stream_) {
     if (static_cast<int64_t>(p->m) * p->lda >= 0x70000000LL || static_cast<int64_t>(p->n) * p->ldw >= 0x70000000LL) return QA_ERR_SHAPE;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const bool flex = p->use_alpha || p->round_mode != QA_ROUND_RNE;
+    if (p->m <= kGemvRows) {
+        GemvParams g = {};
+        g.m = p->m; g.n = p->n; g.k = p->k; g.bits = 8;
+        g.out_type = p->out_type;
+        g.rule = p->use_alpha ? kGemvAlpha : p->round_mode != QA_ROUND_RNE ? kGemvHalfAway : p->scale_order == 1 ? kGemvColOuter : kGemvRowOuter;
+        g.alpha = p->alpha;
+        g.half_away = p->round_mode != QA_ROUND_RNE;
+        g.row_numel = p->a_scale_numel; g.col_numel = p->w_scale_numel;
+        g.lda = p->lda; g.ldw = p->ldw; g.ldd = p->ldd;
+        g.a = p->a; g.w = p->w; g.row_scale = p->a_scale; g.col_scale = p->w_scale; g.d = p->d;
+        return gemv_launch(g, nullptr, stream);
+    }
     if (p->m <= 64) return flex ? dispatch_skinny<true>(*p, stream) : dispatch_skinny<false>(*p, stream);
     // the single-row rules (host alpha, round-half-away) only ever come with tiny M
     if (flex) return launch_gemm<2, 2, 2, 2, 2, true>(*p, stream);

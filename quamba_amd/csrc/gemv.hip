@@ -1,0 +1,300 @@
+// Up to eight activation rows against a weight matrix: a stream over the weights.
+//
+// A wave owns four rows of the weight and the whole of K: a lane takes 16 bytes of each row out of every 1024 (int8: 16
+// codes; 4 bits: 32 codes), so a load of the wave is 1 KB in one piece, and the loads of up to five such pieces of all
+// four rows go out before the first is used.  The matrix cores have nothing to give here - a tile of 32 activation rows
+// would be seven eighths or more empty - and their fragments would have to pass through LDS; the products are 4-way int8
+// dot products in the lane that loaded the codes, and LDS is not used at all.  The lanes' partial sums meet through lane
+// swaps (two stages, four values at a time) and row permutes.
+//
+// Bound by the memory round trips of a short kernel, not by bandwidth: 1 x 10240 x 2560 with 4-bit weights (13 MB)
+// 10.2 us as a 32-column matrix-core tile per workgroup.
+//
+// With a conv behind the product (GemvConv) the wave that holds a conv channel's new input also makes its conv step: the
+// operands of that step are requested with the weights, and a launch and a round trip through memory are saved.
+#include "conv2_common.hpp"
+#include "gemm_core.hpp"
+#include "gemv.hpp"
+#include "w4_expand.hpp"
+
+namespace qa {
+namespace {
+
+using gemm::v4u;
+using gemm::quant8;
+using gemm::one_f16_or_bf16;
+
+constexpr int kRows = 4;               // weight rows per wave
+
+// a, b: one value per lane each -> the lower half of the wave holds the sums of a over lane pairs (l, l + 32), the upper
+// half those of b
+__device__ __forceinline__ int fold32(int a, int b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(a), static_cast<unsigned>(b), false, false);
+    return static_cast<int>(r[0]) + static_cast<int>(r[1]);
+}
+// the same for the even and odd rows of sixteen lanes
+__device__ __forceinline__ int fold16(int a, int b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(a), static_cast<unsigned>(b), false, false);
+    return static_cast<int>(r[0]) + static_cast<int>(r[1]);
+}
+// sum over a row of sixteen lanes, in every lane of it
+__device__ __forceinline__ int row_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);       // lane ^ 1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);       // lane ^ 2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);      // mirrored in half a row
+    v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);      // mirrored in the row
+    return v;
+}
+
+typedef const __attribute__((address_space(4))) float* const_floats;
+typedef const __attribute__((address_space(4))) int32_t* const_ints;
+template <typename P, typename T>
+__device__ __forceinline__ P scalar_ptr(const T* p) { return reinterpret_cast<P>(reinterpret_cast<uintptr_t>(p)); }
+
+// out_scale_of (conv2_common.hpp) for the four channels ch .. ch + 3 of one head, the same in every lane: scalar loads,
+// which do not queue behind the weights, all of a level's at once.
+__device__ __forceinline__ void uniform_out_scales(const QaConv2Params& p, const Part& part, int ch, float (&s)[4]) {
+    if (!p.x_out_scales) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = p.x_out_scale;
+        return;
+    }
+    const bool grouped = p.x_head_group_range != nullptr && p.x_dim_group_range != nullptr;
+    const const_floats scales = scalar_ptr<const_floats>(part.index == 0 ? p.x_out_scales : part.index == 1 ? p.B_out_scales : p.C_out_scales);
+    int at[4];
+    if (part.index != 0 || !grouped) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) at[e] = grouped ? (ch + e - part.offset) / p.d_state : 0;
+    } else {
+        const int group_size = p.x_dim / p.n_groups, g = ch / group_size, head = (ch % group_size) / p.x_headdim, d = ch % p.x_headdim;
+        const const_ints hr = scalar_ptr<const_ints>(p.x_head_group_range) + g * p.nhead_groups;
+        int ends[kGemvConvGroups], hg = 0;
+#pragma unroll
+        for (int j = 0; j < kGemvConvGroups; ++j) ends[j] = hr[min(j, p.nhead_groups - 1)];
+#pragma unroll
+        for (int j = 0; j < kGemvConvGroups - 1; ++j) hg += j < p.nhead_groups - 1 && head >= ends[j] ? 1 : 0;
+        const int row = (g * p.nhead_groups + hg) * p.ndim_groups;
+        const const_ints dr = scalar_ptr<const_ints>(p.x_dim_group_range) + row;
+#pragma unroll
+        for (int j = 0; j < kGemvConvGroups; ++j) ends[j] = dr[min(j, p.ndim_groups - 1)];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            int dg = 0;
+#pragma unroll
+            for (int j = 0; j < kGemvConvGroups - 1; ++j) dg += j < p.ndim_groups - 1 && d + e >= ends[j] ? 1 : 0;
+            at[e] = row + dg;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = scales[at[e]];
+}
+
+// BATCH: pieces of K (1 KB of each weight row) whose loads are in flight together.  KS: waves of the workgroup that share
+// four rows, a contiguous part of K each.
+template <int BITS, int M, int KS, int BATCH, int OUT, bool CONV>
+__global__ __launch_bounds__(256) void gemv_kernel(GemvParams p, GemvConv f) {
+    constexpr int V = kRows * M, PER = V / 4;                    // values of the wave, and per lane after two folds
+    constexpr int kLaneCodes = BITS == 8 ? 16 : 32, kPieceCodes = 64 * kLaneCodes, AQ = kLaneCodes / 16;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), part_k = wave % KS;
+    const int n0 = (blockIdx.x * (static_cast<int>(blockDim.x) / (64 * KS)) + wave / KS) * kRows;
+    if (KS == 1 && n0 >= p.n) return;
+    // this wave's part of K
+    const int share = (p.k / kLaneCodes + KS - 1) / KS * kLaneCodes;
+    const int k_first = part_k * share, k_end = min(k_first + share, p.k);
+
+    const uint8_t* w_row[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) w_row[r] = static_cast<const uint8_t*>(p.w) + static_cast<int64_t>(min(n0 + r, p.n - 1)) * p.ldw;
+    const int pieces = (k_end - k_first + kPieceCodes - 1) / kPieceCodes;
+    v4u fw[BATCH][kRows], fa[BATCH][M][AQ];
+    uint2 fs[BATCH];
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) {
+            // (pieces and lanes past the end read the row's start; their activations are zeroed below)
+            const int k0 = k_first + (c0 + b) * kPieceCodes + lane * kLaneCodes, kk = k0 < k_end ? k0 : 0;
+#pragma unroll
+            for (int r = 0; r < kRows; ++r) fw[b][r] = *reinterpret_cast<const v4u*>(w_row[r] + kk * BITS / 8);
+            if constexpr (BITS == 4) fs[b] = *reinterpret_cast<const uint2*>(p.s_group + static_cast<int64_t>(kk / 128) * p.n + min(n0, p.n - 4));
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int8_t* a = p.a + min(m, p.m - 1) * p.lda + kk;
+#pragma unroll
+                for (int q = 0; q < AQ; ++q) fa[b][m][q] = *reinterpret_cast<const v4u*>(a + 16 * q);
+            }
+            if (c0 + b + 1 >= pieces) break;
+        }
+    };
+    load(0);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // the value this lane finishes: row `lane / 16` of four, `lane % 16` < PER
+    const int quarter = lane >> 4, slot = lane & 15;
+    const int value = (quarter >> 1) * (V / 2) + (quarter & 1) * PER + min(slot, PER - 1);
+    const int my_m = min(value / kRows, p.m - 1), my_n = min(n0 + value % kRows, p.n - 1);
+    const bool mine = slot < PER && value / kRows < p.m && n0 + value % kRows < p.n;
+    const float s_row = p.rule == kGemvAlpha ? p.alpha : p.row_scale[p.row_numel == 1 ? 0 : my_m];
+    const float s_col = p.rule == kGemvAlpha ? 1.0f : p.col_scale[p.col_numel == 1 ? 0 : my_n];
+
+    // operands of the conv step of this lane's column
+    bool conv_col = false;
+    int ch = 0;
+    int8_t* st = nullptr;
+    uint32_t taps = 0, held[3] = {};                             // the state's codes, as loaded
+    int bias_q = 0;
+    float c_out_scale = 1.0f;
+    Part part = {};
+    bool st_word = false;
+    // (the four columns of a wave are all conv channels, of one part and one head, or none is)
+    if (CONV && n0 >= f.ch0 && n0 < f.ch0 + f.conv.dim) {
+        const QaConv2Params& c = f.conv;
+        conv_col = true;
+        ch = my_n - f.ch0;
+        part = part_of(c, n0 - f.ch0);
+        taps = *reinterpret_cast<const uint32_t*>(c.weight + ch * 4);
+        bias_q = *(c.bias ? c.bias + ch : c.weight);
+        st = c.conv_state + my_m * c.conv_state_batch_stride + ch * c.conv_state_c_stride;
+        st_word = c.conv_state_len == 4 && c.conv_state_l_stride == 1 && (reinterpret_cast<uintptr_t>(c.conv_state) & 3u) == 0 &&
+                  c.conv_state_batch_stride % 4 == 0 && c.conv_state_c_stride % 4 == 0;
+        if (st_word) {
+            held[0] = *reinterpret_cast<const uint32_t*>(st);
+        } else {
+            const int drop = c.conv_state_len - 3;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) held[i] = static_cast<uint8_t>(st[(drop + i) * c.conv_state_l_stride]);
+        }
+        float scales[kRows];
+        uniform_out_scales(c, part, n0 - f.ch0, scales);
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) c_out_scale = value % kRows == r ? scales[r] : c_out_scale;
+    }
+
+    int acc[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[v] = 0;
+    for (int c0 = 0; c0 < pieces; c0 += BATCH) {
+        if (c0) load(c0);
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) {
+            if (c0 + b >= pieces) break;
+            const bool in = k_first + (c0 + b) * kPieceCodes + lane * kLaneCodes < k_end;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int q = 0; q < AQ; ++q) fa[b][m][q] = in ? fa[b][m][q] : v4u{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int r = 0; r < kRows; ++r) {
+                if constexpr (BITS == 8) {
+#pragma unroll
+                    for (int m = 0; m < M; ++m)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            acc[m * kRows + r] = __builtin_amdgcn_sdot4(static_cast<int>(fw[b][r][q]), static_cast<int>(fa[b][m][0][q]), acc[m * kRows + r], false);
+                } else {
+                    const uint32_t pair = r & 2 ? fs[b].y : fs[b].x;
+                    const uint32_t one = r & 1 ? pair >> 16 : pair & 0xffffu;
+                    const __half2 s2 = bits_h2(one | (one << 16));
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const uint2 e = expand_grouped(fw[b][r][q], s2);
+#pragma unroll
+                        for (int m = 0; m < M; ++m) {
+                            int& s = acc[m * kRows + r];
+                            s = __builtin_amdgcn_sdot4(static_cast<int>(e.x), static_cast<int>(fa[b][m][q / 2][2 * (q & 1)]), s, false);
+                            s = __builtin_amdgcn_sdot4(static_cast<int>(e.y), static_cast<int>(fa[b][m][q / 2][2 * (q & 1) + 1]), s, false);
+                        }
+                    }
+                }
+            }
+        }
+    }
+
+    int half[V / 2], sum = 0;
+#pragma unroll
+    for (int v = 0; v < V / 2; ++v) half[v] = fold32(acc[v], acc[v + V / 2]);
+#pragma unroll
+    for (int v = 0; v < PER; ++v) {
+        const int s = row_sum(fold16(half[v], half[v + PER]));
+        sum = slot == v ? s : sum;
+    }
+    if constexpr (KS > 1) {
+        __shared__ int parts[4][64];
+        if (part_k) parts[wave][lane] = sum;
+        __syncthreads();
+        if (part_k) return;
+#pragma unroll
+        for (int i = 1; i < KS; ++i) sum += parts[wave + i][lane];
+    }
+    if (!mine) return;
+    const float accf = static_cast<float>(sum);
+    float y = p.rule == kGemvHalfAway ? (s_col * s_row) * accf : p.rule == kGemvColOuter ? s_col * (s_row * accf)
+            : p.rule == kGemvAlpha ? s_row * accf : s_row * (s_col * accf);
+    asm volatile("" : "+v"(y));                                  // the fp32 product is rounded on its own
+    if constexpr (OUT == QA_OUT_I8) {
+        const int8_t q = static_cast<int8_t>(quant8(y, p.half_away ? QA_ROUND_HALF_AWAY : QA_ROUND_RNE));
+        if (CONV && conv_col) {
+            const QaConv2Params& c = f.conv;
+            const uint32_t kept = st_word ? held[0] >> 8 : held[0] | (held[1] << 8) | (held[2] << 16);
+            const uint32_t win = kept | (static_cast<uint32_t>(static_cast<uint8_t>(q)) << 24);
+            if (st_word) {
+                *reinterpret_cast<uint32_t*>(st) = win;
+            } else {
+                for (int i = 0; i < c.conv_state_len; ++i) st[i * c.conv_state_l_stride] = static_cast<int8_t>(win >> (8 * (i + 4 - c.conv_state_len)));
+            }
+            float v = c.bias ? part.s_bias * static_cast<float>(bias_q) : 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                v = __builtin_fmaf(part.s_in * static_cast<float>(static_cast<int8_t>(taps >> (8 * i))), static_cast<float>(static_cast<int8_t>(win >> (8 * i))), v);
+            int64_t ls, cs;
+            const ConvQuantRegs kq(c_out_scale);
+            out_ptr(c, part, my_m, ch, &ls, &cs)[0] = static_cast<int8_t>(conv_quant(v, c_out_scale, 1.0f / c_out_scale, c.silu_activation,
+                                                                                     conv_needs_exact_route(c_out_scale), kq));
+            return;
+        }
+        static_cast<int8_t*>(p.d)[my_m * p.ldd + my_n] = q;
+    } else {
+        static_cast<uint16_t*>(p.d)[my_m * p.ldd + my_n] = one_f16_or_bf16<OUT>(y);
+    }
+}
+
+template <int BITS, int M, int KS, int BATCH>
+int launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
+    const int64_t groups = (static_cast<int64_t>(p.n) + kRows - 1) / kRows;
+    const int per_block = KS > 1 || groups >= 1024 ? 4 : 1;      // waves; few waves: a workgroup each, spread over the part
+    const dim3 grid(static_cast<unsigned>((groups * KS + per_block - 1) / per_block)), block(64 * per_block);
+    const GemvConv none = {};
+    if (conv) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, true>), grid, block, 0, stream, p, *conv);
+    else if (p.out_type == QA_OUT_I8) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, false>), grid, block, 0, stream, p, none);
+    else if (p.out_type == QA_OUT_F16) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_F16, false>), grid, block, 0, stream, p, none);
+    else hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_BF16, false>), grid, block, 0, stream, p, none);
+    return check_launch();
+}
+
+// Waves per four rows.  A wave alone works through its rows' K at the pace of one wave's latencies, so K is split while the
+// rows alone leave the SIMDs short of waves (measured, us for 1 / 2 / 4 waves at one activation row: 4 bits 2560 x 5120 5.9 /
+// 5.8 / 4.9, 4096 x 8192 8.7 / 7.1 / 6.9, 10240 x 2560 7.4 / 6.5 / 9.1, 18560 x 4096 11.5 / 11.0 / 15.3; int8 192 x 5120
+// 2.7 / 2.8 / 2.6, 10240 x 2560 7.0 / 6.5 / 6.9); past about 5000 waves more of them only repeat the prologue.
+template <int BITS, int M, int B1, int B2, int B4>
+int pick(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
+    const int64_t groups = (static_cast<int64_t>(p.n) + kRows - 1) / kRows;
+    if (groups <= 1024 && p.k >= 1536) return launch<BITS, M, 4, B4>(p, conv, stream);
+    if (groups <= 2816 && p.k >= 2048) return launch<BITS, M, 2, B2>(p, conv, stream);
+    return launch<BITS, M, 1, B1>(p, conv, stream);
+}
+}  // namespace
+
+int gemv_launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
+    if (p.bits == 8) {
+        if (p.m == 1) return pick<8, 1, 4, 2, 2>(p, conv, stream);
+        if (p.m == 2) return pick<8, 2, 3, 2, 2>(p, conv, stream);
+        if (p.m <= 4) return pick<8, 4, 3, 2, 2>(p, conv, stream);
+        return pick<8, 8, 2, 2, 2>(p, conv, stream);
+    }
+    if (p.m == 1) return pick<4, 1, 2, 1, 1>(p, conv, stream);
+    if (p.m == 2) return pick<4, 2, 2, 1, 1>(p, conv, stream);
+    if (p.m <= 4) return pick<4, 4, 2, 1, 1>(p, conv, stream);
+    return pick<4, 8, 1, 1, 1>(p, conv, stream);
+}
+
+}  // namespace qa

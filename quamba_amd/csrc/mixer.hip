@@ -9,6 +9,7 @@
 // channels per lane, the scan stages token-major rows, x_proj and dt_proj are plain row-major products - so no second
 // copy of the conv's output, no transposition of B and C, no padding of the token count, and prompts of any length
 // run on the same kernels.
+#include "gemv.hpp"
 #include "mixer_common.hpp"
 #include "ssd_common.hpp"
 
@@ -78,6 +79,25 @@ bool linear_ok(const QaLinearParams& w) {
     return (w.bits == 8 || w.bits == 4) && w.n > 0 && w.k > 0 && w.weight && w.col_scale && w.row_scale;
 }
 
+// in_proj of a decode step with the conv's step behind it in one launch (QA_ERR_UNSUPPORTED: two launches)
+int project_conv(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows, int8_t* d, int ch0, const QaConv2Params& conv, void* stream) {
+    const GemvConv f = {ch0, conv};
+    if (rows > kGemvRows || !gemv_conv_ok(f)) return QA_ERR_UNSUPPORTED;
+    if (w.k % 16 != 0 || lda % 16 != 0 || !aligned16(a) || !aligned16(w.weight)) return QA_ERR_UNSUPPORTED;
+    if (w.bits == 4 && (!w.s_group || w.n % 4 != 0 || w.k % 128 != 0 || (reinterpret_cast<uintptr_t>(w.s_group) & 7u))) return QA_ERR_UNSUPPORTED;
+    GemvParams g = {};
+    g.m = rows; g.n = w.n; g.k = w.k; g.bits = w.bits;
+    g.out_type = QA_OUT_I8;
+    g.rule = kGemvRowOuter;
+    if (w.bits == 8 && rows == 1 && w.row_rule == QA_ROW_ALPHA) { g.rule = kGemvAlpha; g.alpha = w.alpha; }
+    if (w.bits == 8 && rows == 1 && w.row_rule == QA_ROW_HALF_AWAY) { g.rule = kGemvHalfAway; g.half_away = 1; }
+    g.row_numel = 1; g.col_numel = w.bits == 4 ? w.n : w.col_numel;
+    g.lda = lda; g.ldw = w.bits == 4 ? w.k / 2 : w.k; g.ldd = w.n;
+    g.a = a; g.w = w.weight; g.s_group = static_cast<const __half*>(w.s_group);
+    g.row_scale = w.row_scale; g.col_scale = w.col_scale; g.d = d;
+    return gemv_launch(g, &f, static_cast<hipStream_t>(stream));
+}
+
 int hadamard(const void* y, int8_t* out, int rows, int dim, float scale, void* stream) {
     QaHadamardParams h = {};
     h.rows = rows; h.dim = dim; h.in_type = 0; h.scale = scale;
@@ -125,6 +145,24 @@ Mamba1Buffers carve(const QaMamba1Params& p, void* base) {
     b.scan.p = c.take<uint8_t>(b.scan.bytes);
     b.total = c.off;
     return b;
+}
+
+// the Mamba1 conv in the terms of the Mamba2 one: every channel an x channel, one output scale
+QaConv2Params conv_of(const QaMamba1Params& p, const Mamba1Buffers& b) {
+    QaConv2Params c = {};
+    const int64_t len = p.seqlen;
+    const int d = p.d_inner;
+    c.batch = p.batch; c.dim = d; c.seqlen = p.seqlen; c.width = p.d_conv;
+    c.silu_activation = 1;
+    c.x_dim = d; c.x_headdim = d; c.d_state = 1; c.n_groups = 1;
+    c.conv_state_len = p.conv_state_len;
+    c.xBC_batch_stride = len * 2 * d; c.xBC_l_stride = 2 * d; c.xBC_c_stride = 1;
+    c.x_batch_stride = len * d; c.x_l_stride = d; c.x_c_stride = 1;
+    c.weight_c_stride = p.d_conv; c.weight_width_stride = 1;
+    c.conv_state_batch_stride = p.conv_state_batch_stride; c.conv_state_c_stride = p.conv_state_c_stride; c.conv_state_l_stride = p.conv_state_l_stride;
+    c.xBC = b.xz; c.weight = p.conv_weight; c.bias = p.conv_bias; c.x = b.x; c.conv_state = p.conv_state;
+    c.scale_x = p.conv_scale_x; c.scale_wx = p.conv_scale_w; c.scale_bx = p.conv_scale_b; c.x_out_scale = p.conv_scale_out;
+    return c;
 }
 
 int validate(const QaMamba1Params* p) {
@@ -274,18 +312,7 @@ extern "C" int qa_mamba1_forward(const QaMamba1Params* p, void* stream) {
     const int64_t len = p->seqlen;
     QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.xz, QA_OUT_I8, true, b.w8, stream));
 
-    QaConv2Params c = {};                    // every channel an x channel with one output scale
-    c.batch = p->batch; c.dim = d; c.seqlen = p->seqlen; c.width = p->d_conv;
-    c.silu_activation = 1;
-    c.x_dim = d; c.x_headdim = d; c.d_state = 1; c.n_groups = 1;
-    c.conv_state_len = p->conv_state_len;
-    c.xBC_batch_stride = len * 2 * d; c.xBC_l_stride = 2 * d; c.xBC_c_stride = 1;
-    c.x_batch_stride = len * d; c.x_l_stride = d; c.x_c_stride = 1;
-    c.weight_c_stride = p->d_conv; c.weight_width_stride = 1;
-    c.conv_state_batch_stride = p->conv_state_batch_stride; c.conv_state_c_stride = p->conv_state_c_stride; c.conv_state_l_stride = p->conv_state_l_stride;
-    c.xBC = b.xz; c.weight = p->conv_weight; c.bias = p->conv_bias; c.x = b.x; c.conv_state = p->conv_state;
-    c.scale_x = p->conv_scale_x; c.scale_wx = p->conv_scale_w; c.scale_bx = p->conv_scale_b; c.x_out_scale = p->conv_scale_out;
-    QA_TRY(conv_channel_last_fwd(c, static_cast<hipStream_t>(stream)));
+    QA_TRY(conv_channel_last_fwd(conv_of(*p, b), static_cast<hipStream_t>(stream)));
 
     QA_TRY(project(p->x_proj, b.x, d, rows, b.x_dbl, QA_OUT_I8, false, b.w8, stream));
     QA_TRY(project(p->dt_proj, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, true, b.w8, stream));
@@ -322,6 +349,8 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
     if (p->seqlen != 1) return QA_ERR_SHAPE;
     const Mamba1Buffers b = carve(*p, p->workspace);
     const int rows = p->batch, d = p->d_inner;
+    const int fused = project_conv(p->in_proj, p->hidden, p->d_model, rows, b.xz, 0, conv_of(*p, b), stream);
+    if (fused == QA_ERR_UNSUPPORTED) {
     QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.xz, QA_OUT_I8, false, b.w8, stream));
 
     QaConvParams c = {};
@@ -335,6 +364,9 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
     c.x = b.xz; c.weight = p->conv_weight; c.bias = p->conv_bias; c.out = b.x; c.conv_state = p->conv_state;
     c.scale_x = p->conv_scale_x; c.scale_w = p->conv_scale_w; c.scale_b = p->conv_scale_b; c.scale_out = p->conv_scale_out;
     QA_TRY(qa_causal_conv1d_update(&c, stream));
+    } else if (fused != QA_OK) {
+        return fused;
+    }
 
     QA_TRY(project(p->x_proj, b.x, d, rows, b.x_dbl, QA_OUT_I8, false, b.w8, stream));
     QA_TRY(project(p->dt_proj, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, false, b.w8, stream));
@@ -403,9 +435,14 @@ extern "C" int qa_mamba2_step(const QaMamba2Params* p, void* stream) {
     if (p->seqlen != 1) return QA_ERR_SHAPE;
     const Mamba2Buffers b = carve(*p, p->workspace, true);
     const int rows = p->batch, heads = heads_of(*p);
-    QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.zxbcdt, QA_OUT_I8, false, b.w8, stream));
     const QaConv2Params c = conv2_of(*p, b);
-    QA_TRY(qa_quamba2_conv1d_update(&c, stream));
+    const int fused = project_conv(p->in_proj, p->hidden, p->d_model, rows, b.zxbcdt, p->d_inner, c, stream);
+    if (fused == QA_ERR_UNSUPPORTED) {
+        QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.zxbcdt, QA_OUT_I8, false, b.w8, stream));
+        QA_TRY(qa_quamba2_conv1d_update(&c, stream));
+    } else if (fused != QA_OK) {
+        return fused;
+    }
 
     QaSsmUpdateParams u = {};
     const int64_t bc = static_cast<int64_t>(p->ngroups) * p->d_state;
