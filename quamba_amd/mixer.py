@@ -95,11 +95,11 @@ class W8A8QMamba(nn.Module):
         return mods
 
     def _scalars(self):
+        """(dict, key) of everything a plan depends on that is no buffer."""
         m = self._modules
-        c, s, h = m["conv1d"], m["selective_scan"], m["had"]
-        return (c.input_scale, c.weight_scale, c.bias_scale, c.output_scale, id(c.bias), s.delta_softplus, h.x_H_scale, h.had_scale,
-                getattr(m["in_proj"], "alpha", 0.0), getattr(m["x_proj"], "alpha", 0.0), m["dt_proj"].alpha,
-                getattr(m["out_proj"], "alpha", 0.0))
+        c, s, h = (m[k].__dict__ for k in ("conv1d", "selective_scan", "had"))
+        return (tuple((c, k) for k in ("input_scale", "weight_scale", "bias_scale", "output_scale", "bias")) + ((s, "delta_softplus"),)
+                + tuple((h, k) for k in ("x_H_scale", "had_scale")) + tuple((m[k].__dict__, "alpha") for k in ("in_proj", "x_proj", "dt_proj", "out_proj")))
 
     def _native_block(self, dev):
         p, D, N = _lib.QaMamba1Params(), self.d_inner, self.d_state
@@ -122,15 +122,14 @@ class W8A8QMamba(nn.Module):
     def forward(self, hidden_states, inference_params=None, conv_state=None, ssm_state=None):
         """hidden_states int8 (B, L, d_model) -> fp16 (B, L, d_model).  With conv_state / ssm_state (or an
         inference_params cache) the states after the last token are stored into them."""
-        batch, seqlen, _ = hidden_states.shape
         if inference_params is not None:
-            conv_state, ssm_state = self._get_states_from_cache(inference_params, batch)
+            conv_state, ssm_state = self._get_states_from_cache(inference_params, hidden_states.shape[0])
             if inference_params.seqlen_offset > 0:
                 out, _, _ = self.step(hidden_states, conv_state, ssm_state)
                 return out
         out = _layer_call.call(self, hidden_states, conv_state, ssm_state, False)
         if out is not None:
-            return out.view(batch, seqlen, -1)
+            return out
         return self._forward_modules(hidden_states, conv_state, ssm_state)
 
     @torch.no_grad()
@@ -164,11 +163,11 @@ class W8A8QMamba(nn.Module):
         return self.out_proj(self.had(y))                               # (B, L, d_model) fp16
 
     def step(self, hidden_states, conv_state, ssm_state):
-        assert hidden_states.shape[1] == 1, "Only support decoding with 1 token at a time for now"
+        assert hidden_states.size(1) == 1, "Only support decoding with 1 token at a time for now"
         out = _layer_call.call(self, hidden_states, conv_state, ssm_state, True)
         if out is None:
-            out = self._step_modules(hidden_states, conv_state, ssm_state)
-        return out.unsqueeze(1), conv_state, ssm_state
+            out = self._step_modules(hidden_states, conv_state, ssm_state).unsqueeze(1)
+        return out, conv_state, ssm_state
 
     @torch.no_grad()
     def _step_modules(self, hidden_states, conv_state, ssm_state):
@@ -272,12 +271,15 @@ class W4A8QMamba2(nn.Module):
         return mods
 
     def _scalars(self):
+        """(dict, key) of everything a plan depends on that is no buffer."""
         m = self._modules
-        c, s, n, h = m["conv1d"], m["qchunk_scan"], m["norm"], m["had"]
-        return (c.x_scale, c.B_scale, c.C_scale, c.wx_scale, c.wB_scale, c.wC_scale, c.bx_scale, c.bB_scale, c.bC_scale, id(c.bias),
-                id(c.x_head_group_range), id(c.x_dim_group_range), id(s.x_head_group_range), id(s.x_dim_group_range), s.chunk_size,
-                s.delta_softplus, s.dt_limit, s.D_has_hdim, n.eps, n.z_scale, n.group_size, n.norm_before_gate, n.use_float16_output,
-                h.x_H_scale, h.had_scale, getattr(m["out_proj"], "alpha", 0.0))
+        c, s, n, h = (m[k].__dict__ for k in ("conv1d", "qchunk_scan", "norm", "had"))
+        conv = ("x_scale", "B_scale", "C_scale", "wx_scale", "wB_scale", "wC_scale", "bx_scale", "bB_scale", "bC_scale", "bias",
+                "x_head_group_range", "x_dim_group_range")
+        scan = ("x_head_group_range", "x_dim_group_range", "chunk_size", "delta_softplus", "dt_limit", "D_has_hdim", "B_scale", "C_scale", "dt_scale")
+        norm = ("eps", "z_scale", "group_size", "norm_before_gate", "use_float16_output", "bias")
+        return (tuple((c, k) for k in conv) + tuple((s, k) for k in scan) + tuple((n, k) for k in norm)
+                + tuple((h, k) for k in ("x_H_scale", "had_scale")) + ((m["out_proj"].__dict__, "alpha"),))
 
     def _native_block(self, dev):
         p, D, N, G, H = _lib.QaMamba2Params(), self.d_ssm, self.d_state, self.ngroups, self.nheads
@@ -320,14 +322,14 @@ class W4A8QMamba2(nn.Module):
         p.x_scales = _ptr(s.x_scales, torch.float32, G * sg if sg else 1, dev)
         p.B_scale, p.C_scale = (_ptr(t, torch.float32, G if sg else 1, dev) for t in (s.B_scale, s.C_scale))
         p.ssm_state_scale = _ptr(s.ssm_state_scale, torch.float32, G * sg * N if sg else 1, dev)
-        return p, (conv_dim, (H, self.headdim, N), ((self.d_conv,), (self.d_conv, self.d_conv - 1)))
+        return p, (conv_dim, (H, self.headdim, N), ((self.d_conv, self.d_conv), (self.d_conv, self.d_conv - 1)))
 
     def forward(self, u, conv_state=None, ssm_state=None):
         """u int8 (B, L, d_model) -> fp16 (B, L, d_model); conv_state / ssm_state receive the states after
         the last token when given."""
         out = _layer_call.call(self, u, conv_state, ssm_state, False)
         if out is not None:
-            return out.view(u.shape[0], u.shape[1], -1)
+            return out
         return self._forward_modules(u, conv_state, ssm_state)
 
     @torch.no_grad()
@@ -356,11 +358,11 @@ class W4A8QMamba2(nn.Module):
         return self.had(self.norm(y, z))
 
     def step(self, hidden_states, conv_state, ssm_state):
-        assert hidden_states.shape[1] == 1, "Only support decoding with 1 token at a time for now"
+        assert hidden_states.size(1) == 1, "Only support decoding with 1 token at a time for now"
         out = _layer_call.call(self, hidden_states, conv_state, ssm_state, True)
         if out is None:
-            out = self._step_modules(hidden_states, conv_state, ssm_state)
-        return out.unsqueeze(1), conv_state, ssm_state
+            out = self._step_modules(hidden_states, conv_state, ssm_state).unsqueeze(1)
+        return out, conv_state, ssm_state
 
     @torch.no_grad()
     def _step_modules(self, hidden_states, conv_state, ssm_state):

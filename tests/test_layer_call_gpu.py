@@ -5,9 +5,17 @@ import pytest
 import torch
 
 from quamba_amd import W4A8QMamba, W4A8QMamba2, W8A8QMamba, W8A8QMamba2, _layer_call
-from tests.test_mixer_variants_gpu import _mamba1, _mamba2, _ri
+from tests import test_mixer_variants_gpu as variants
+from tests.test_mixer_variants_gpu import _mamba2, _ri
 
 pytestmark = pytest.mark.gpu
+
+
+def _mamba1(cls, dev, seed, d_model=256):
+    sized = lambda width, *a, **k: cls(d_model, *a, **k)       # (the shared builder is for one width)
+    return variants._mamba1(sized, dev, seed)
+
+
 MIXERS = [(W8A8QMamba, _mamba1), (W4A8QMamba, _mamba1), (W8A8QMamba2, _mamba2), (W4A8QMamba2, _mamba2)]
 
 
@@ -44,8 +52,8 @@ def test_forward(dev, cls, build, batch, seqlen, dtype, width):
     out = _layer_call.call(m, h, conv, ssm, False)
     assert out is not None, "the library call has to take this"
     want = m._forward_modules(h, conv2, ssm2)
-    _close(out.view(batch, seqlen, -1), want, (conv, conv2), (ssm, ssm2))
-    assert torch.equal(m.forward(h), out.view(batch, seqlen, -1))          # without states
+    _close(out, want, (conv, conv2), (ssm, ssm2))
+    assert torch.equal(m.forward(h), out)          # without states
 
 
 @pytest.mark.parametrize("cls,build", MIXERS)
@@ -58,7 +66,19 @@ def test_step(dev, cls, build, batch, dtype, width):
     out = _layer_call.call(m, h, conv, ssm, True)
     assert out is not None, "the library call has to take this"
     want = m._step_modules(h, conv2, ssm2)
-    _close(out, want, (conv, conv2), (ssm, ssm2))
+    _close(out[:, 0], want, (conv, conv2), (ssm, ssm2))
+
+
+@pytest.mark.parametrize("d_model", [768, 2048])
+def test_step_of_a_wide_layer(dev, d_model):
+    """in_proj and the conv in one launch, with the weight rows' K split over waves (2048) and not (768)."""
+    m, g = _mamba1(W8A8QMamba, dev, seed=1, d_model=d_model)
+    for batch in (1, 5):
+        h = _ri(dev, g, batch, 1, d_model)
+        conv, ssm = _states(m, dev, g, batch, torch.int8, 4)
+        conv2, ssm2 = conv.clone(), ssm.clone()
+        out = _layer_call.call(m, h, conv, ssm, True)
+        _close(out[:, 0], m._step_modules(h, conv2, ssm2), (conv, conv2), (ssm, ssm2))
 
 
 @pytest.mark.parametrize("cls,build", MIXERS[:1] + MIXERS[3:])
