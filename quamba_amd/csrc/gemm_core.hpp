@@ -220,9 +220,9 @@ __device__ __forceinline__ void mma_tile_paced(const uint8_t* sa, const uint8_t*
 #pragma unroll
             for (int j = 0; j < TM; ++j) {
                 acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[kk & 1][i], fa[kk & 1][j], acc[i][j], 0, 0, 0);
-                if ((i * TM + j) % 2 == 1) {
+                if (TM * TN == 1 || (i * TM + j) % 2 == 1) {
                     __builtin_amdgcn_sched_barrier(0);
-                    hook(kk * (TM * TN / 2) + (i * TM + j) / 2);
+                    hook(TM * TN == 1 ? kk : kk * (TM * TN / 2) + (i * TM + j) / 2);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -454,13 +454,28 @@ constexpr int epilogue_lds_bytes() {
 template <int TM, int WAVES>
 constexpr int skinny_lds_bytes() { return WAVES * (1 + TM) * 32 * kBK + TM * 16 * 64 * 4; }
 
+// Tile of workgroup `linear`, row blocks of 32 TM by column blocks of 32.  With many column blocks the row blocks of one of
+// them go to one XCD (eight workgroups apart), whose L2 then holds their weights.
+template <int TM>
+__device__ __forceinline__ void skinny_tile_of_workgroup(int linear, int m, int n, int& m0, int& n0) {
+    const int blocks_m = (m + 32 * TM - 1) / (32 * TM), blocks_n = (n + 31) / 32, whole = blocks_n / 8 * 8 * blocks_m;
+    if (linear < whole) {
+        n0 = ((linear / (8 * blocks_m)) * 8 + linear % 8) * 32;
+        m0 = (linear / 8) % blocks_m * (32 * TM);
+    } else {
+        const int rest = linear - whole, columns = blocks_n % 8;
+        n0 = (blocks_n / 8 * 8 + rest % columns) * 32;
+        m0 = rest / columns * (32 * TM);
+    }
+}
+
 // Adds the waves' partial accumulators in `red` (TM*16*64 ints, zeroed by the caller before any
 // barrier it has passed), then every thread scales and writes four consecutive columns of one row.
 // Lane l of the accumulator layout holds row (l & 31) and, in registers 4q..4q+3, the columns
 // 8q + 4*(l >> 5) + (0..3): one unit = (row block, q, lane).
 template <int TM, int OUT, bool FLEX, bool TRANS>
 __device__ __forceinline__ void skinny_reduce_store(const Epilogue& e, v16i (&acc)[TM], int* red, int m, int n,
-                                                    int n0, int tid, int threads) {
+                                                    int m0, int n0, int tid, int threads) {
     const int lane = tid & 63;
     __syncthreads();                                       // red is zero
 #pragma unroll
@@ -477,7 +492,7 @@ __device__ __forceinline__ void skinny_reduce_store(const Epilogue& e, v16i (&ac
     const bool vec_ok = !TRANS && e.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(e.d) & (4 * kElt - 1)) == 0;
     for (int u = tid; u < TM * 4 * 64; u += threads) {
         const int ul = u & 63, j = u >> 8, q = (u >> 6) & 3;
-        const int mm = j * 32 + (ul & 31);
+        const int mm = m0 + j * 32 + (ul & 31);
         const int nn = n0 + 8 * q + 4 * (ul >> 5);
         if (mm >= m || nn >= n) continue;
         const float s_row = use_alpha ? e.alpha : e.row_scale[e.row_numel == 1 ? 0 : mm];

@@ -114,10 +114,12 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
         const uint8_t* stage = lds + (kt & 1) * C::kStageBytes;
         // the activation requests for the next tile go out one at a time between the multiplications
         const uint32_t nbase = lds_base + ((kt + 1) & 1) * C::kStageBytes;
-        static_assert(C::kAInstr <= 4 * TM * TN / 2, "more requests than slots");
+        constexpr int kSlots = TM * TN == 1 ? 4 : 4 * (TM * TN / 2), kPerSlot = (C::kAInstr + kSlots - 1) / kSlots;
         mma_tile_paced<TM, TN>(stage + (wm * TM * 32) * kBK, stage + BM * kBK + (wn * TN * 32) * kBK, frow, fhalf, acc,
                                [&](int slot) {
-                                   if (slot < C::kAInstr) load_a.template issue_one<WAVES>(slot, rsrc_a, (kt + 1) * kBK, p.k, nbase, wave);
+#pragma unroll
+                                   for (int r = slot * kPerSlot; r < (slot + 1) * kPerSlot; ++r)
+                                       if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, (kt + 1) * kBK, p.k, nbase, wave);
                                });
         if (more) store_w((kt + 1) & 1);
     }
@@ -179,7 +181,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_w4a8_skinny_kernel(QaGemmW4A8
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int frow = lane & 31, fhalf = lane >> 5;
-    const int n0 = blockIdx.x * 32;
+    int m0, n0;
+    skinny_tile_of_workgroup<TM>(blockIdx.x, p.m, p.n, m0, n0);
     const bool grouped = p.group_size > 0;
     for (int i = tid; i < TM * 16 * 64; i += kThreads) red[i] = 0;
     uint8_t* stage = lds + wave * ((2 + TM) * kTile);          // two weight halves, TM activation tiles
@@ -206,7 +209,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_w4a8_skinny_kernel(QaGemmW4A8
         if (i < AI) {
 #pragma unroll
             for (int j = 0; j < TM; ++j) {
-                const int arow = j * 32 + 8 * i + lrow;
+                const int arow = m0 + j * 32 + 8 * i + lrow;
                 a_off[j][i] = arow < p.m ? static_cast<int>(arow * p.lda) + lchunk * 16 : -1;
             }
         }
@@ -304,7 +307,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_w4a8_skinny_kernel(QaGemmW4A8
     e.row_numel = p.tok_scale_numel; e.col_numel = p.n;
     e.use_alpha = 0; e.alpha = 0.0f; e.round_mode = QA_ROUND_RNE; e.col_outer = 0;
     e.ldd = p.ldd; e.d = p.d;
-    skinny_reduce_store<TM, OUT, false, TRANS>(e, acc, red, p.m, p.n, n0, tid, kThreads);
+    skinny_reduce_store<TM, OUT, false, TRANS>(e, acc, red, p.m, p.n, m0, n0, tid, kThreads);
 }
 
 template <int TM, int AI, int WAVES, int DEPTH, int OUT, bool TRANS>
@@ -317,7 +320,8 @@ int launch_skinny_one(const QaGemmW4A8Params& p, hipStream_t stream) {
             return check_launch();
         }
     }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((p.n + 31) / 32)), dim3(64 * WAVES), kLds, stream, p);
+    const int64_t blocks = static_cast<int64_t>((p.m + 32 * TM - 1) / (32 * TM)) * ((p.n + 31) / 32);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES), kLds, stream, p);
     return check_launch();
 }
 
@@ -331,15 +335,15 @@ int launch_skinny(const QaGemmW4A8Params& p, hipStream_t stream) {
                               : launch_skinny_one<TM, AI, WAVES, DEPTH, QA_OUT_F16, false>(p, stream);
 }
 
+int64_t tiles_of(const QaGemmW4A8Params& p, int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); }
+
 int dispatch_skinny(const QaGemmW4A8Params& p, hipStream_t stream) {
-    // four waves per workgroup once the columns give a workgroup per CU, else eight when K is long enough
-    const bool wide = (p.n + 31) / 32 < 256 && p.k >= 16 * 2 * kBK;
+    // eight waves share K when there is at most a workgroup per CU and K is long, else four (4096 x 8192 at 64 rows: 13.8
+    // against 15.8 us; 18560 x 4096 at 16 rows: 23.0 against 19.1)
+    const bool wide = tiles_of(p, 32, 32) <= 256 && p.k >= 2048;
     // activation rows are fetched eight at a time: up to 8 rows need one fetch per tile, up to 32 four
     if (p.m <= 8) return wide ? launch_skinny<1, 1, 8, 3>(p, stream) : launch_skinny<1, 1, 4, 3>(p, stream);
-    if (p.m <= 32) return wide ? launch_skinny<1, 4, 8, 2>(p, stream) : launch_skinny<1, 4, 4, 2>(p, stream);
-    // two row blocks: a wave's registers allow one workgroup of eight waves or two of four per CU, and
-    // eight waves measured faster whenever K has at least two pieces per wave
-    return (wide || p.k >= 16 * 2 * kBK) ? launch_skinny<2, 4, 8, 2>(p, stream) : launch_skinny<2, 4, 4, 2>(p, stream);
+    return wide ? launch_skinny<1, 4, 8, 2>(p, stream) : launch_skinny<1, 4, 4, 2>(p, stream);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -398,10 +402,23 @@ extern "C" int qa_gemm_w4a8(const QaGemmW4A8Params* p, void* stream_) {
         g.row_scale = p->s_token; g.col_scale = p->s_channel; g.d = p->d;
         return gemv_launch(g, nullptr, stream);
     }
-    if (p->m <= 64 && static_cast<int64_t>(p->n) * (p->k / 2) < 0x70000000LL) return dispatch_skinny(*p, stream);
+    const bool addressable = static_cast<int64_t>(p->n) * (p->k / 2) < 0x70000000LL;
+    if (p->m <= 64 && addressable) return dispatch_skinny(*p, stream);
     const int64_t w8_bytes = static_cast<int64_t>(p->n) * p->k;
-    if (p->w8_workspace && p->w8_workspace_bytes >= w8_bytes && aligned16(p->w8_workspace) && w8_bytes < 0x70000000LL &&
-        (!p->output_transpose || p->n > 64)) {
+    const bool expandable = p->w8_workspace && p->w8_workspace_bytes >= w8_bytes && aligned16(p->w8_workspace) && w8_bytes < 0x70000000LL;
+    if (!p->output_transpose) {
+        // Between the kernel for few rows and the weights expanded once (a pass of its own: 2 us and 1.5 bytes a weight) lie
+        // the shapes in which expanding inside the product is the cheaper way, measured at 96 .. 1000 rows: 32 x 32 tiles
+        // with K split over the waves up to two a CU (192 x 5120: 8.3 us where 128 x 128 tiles took 38; 2560 x 5120 at 128
+        // rows 14.7, expanded once 23.6), then 64 x 64 tiles while they are few and the expansion's latency has either a
+        // short K or other tiles to hide behind (10240 x 2560 at 256 rows 23.4 against 26.1 us, 6144 x 1536 at 512 rows 14.2
+        // against 20.4), 128 x 128 tiles for the rest of the short K.
+        const int64_t t32 = tiles_of(*p, 32, 32), t64 = tiles_of(*p, 64, 64);
+        if (t32 <= 512 && addressable) return dispatch_skinny(*p, stream);
+        if (t64 <= 768 && (p->k <= 1536 || (t64 > 256 && p->k <= 4096))) return launch_gemm<1, 1, 2, 2>(*p, stream);
+        if (p->k <= 1536 && p->m < 1024) return launch_gemm<2, 2, 2, 2>(*p, stream);
+    }
+    if (expandable && (!p->output_transpose || p->n > 64)) {
         int8_t* w8 = static_cast<int8_t*>(p->w8_workspace);
         const int64_t threads = static_cast<int64_t>(p->n) * (p->k / 32);
         hipLaunchKernelGGL(w4_expand_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, *p, w8);

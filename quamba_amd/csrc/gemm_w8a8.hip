@@ -123,12 +123,15 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
         // (past the end of K every lane is out of range and stores zeros)
         const int nt = kt + STAGES - 1;
         const uint32_t nbase = lds_base + (nt % STAGES) * C::kStageBytes;
-        static_assert(C::kAInstr + C::kWInstr <= 4 * TM * TN / 2, "more requests than slots");
+        constexpr int kSlots = TM * TN == 1 ? 4 : 4 * (TM * TN / 2), kPerSlot = (C::kAInstr + C::kWInstr + kSlots - 1) / kSlots;
         mma_tile_paced<TM, TN>(stage + (wm * TM * 32) * kBK, stage + BM * kBK + (wn * TN * 32) * kBK, frow, fhalf, acc,
                                [&](int slot) {
-                                   if (slot < C::kAInstr) load_a.template issue_one<WAVES>(slot, rsrc_a, nt * kBK, p.k, nbase, wave);
-                                   else if (slot < C::kAInstr + C::kWInstr)
-                                       load_w.template issue_one<WAVES>(slot - C::kAInstr, rsrc_w, nt * kBK, p.k, nbase + BM * kBK, wave);
+#pragma unroll
+                                   for (int r = slot * kPerSlot; r < (slot + 1) * kPerSlot; ++r) {
+                                       if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, nt * kBK, p.k, nbase, wave);
+                                       else if (r < C::kAInstr + C::kWInstr)
+                                           load_w.template issue_one<WAVES>(r - C::kAInstr, rsrc_w, nt * kBK, p.k, nbase + BM * kBK, wave);
+                                   }
                                });
     }
     }
@@ -196,7 +199,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_w8a8_skinny_kernel(QaGemmW8A8
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int frow = lane & 31, fhalf = lane >> 5;
-    const int n0 = blockIdx.x * 32;
+    int m0, n0;
+    skinny_tile_of_workgroup<TM>(blockIdx.x, p.m, p.n, m0, n0);
     for (int i = tid; i < TM * 16 * 64; i += kThreads) red[i] = 0;
 
     const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_w8a8_skinny_kernel(QaGemmW8A8
         w_off[i] = row < p.n ? static_cast<int>(row * p.ldw) + lchunk * 16 : -1;
 #pragma unroll
         for (int j = 0; j < TM; ++j) {
-            const int arow = j * 32 + 8 * i + lrow;
+            const int arow = m0 + j * 32 + 8 * i + lrow;
             a_off[j][i] = arow < p.m ? static_cast<int>(arow * p.lda) + lchunk * 16 : -1;
         }
     }
@@ -277,7 +281,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_w8a8_skinny_kernel(QaGemmW8A8
     e.row_numel = p.a_scale_numel; e.col_numel = p.w_scale_numel;
     e.use_alpha = p.use_alpha; e.alpha = p.alpha; e.round_mode = p.round_mode; e.col_outer = p.scale_order;
     e.ldd = p.ldd; e.d = p.d;
-    skinny_reduce_store<TM, OUT, FLEX, false>(e, acc, red, p.m, p.n, n0, tid, kThreads);
+    skinny_reduce_store<TM, OUT, FLEX, false>(e, acc, red, p.m, p.n, m0, n0, tid, kThreads);
 }
 
 template <int TM, int WAVES, int OUT, bool FLEX>
@@ -290,7 +294,8 @@ int launch_skinny_one(const QaGemmW8A8Params& p, hipStream_t stream) {
             return check_launch();
         }
     }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((p.n + 31) / 32)), dim3(64 * WAVES), kLds, stream, p);
+    const int64_t blocks = static_cast<int64_t>((p.m + 32 * TM - 1) / (32 * TM)) * ((p.n + 31) / 32);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES), kLds, stream, p);
     return check_launch();
 }
 
@@ -303,12 +308,35 @@ int launch_skinny(const QaGemmW8A8Params& p, hipStream_t stream) {
 
 template <bool FLEX>
 int dispatch_skinny(const QaGemmW8A8Params& p, hipStream_t stream) {
-    // Four waves per workgroup once there is at least one workgroup per CU (measured: more, smaller
-    // shares only add per-workgroup overhead); eight when the columns alone give too few workgroups
-    // and K is long enough to split further.
-    const bool wide = (p.n + 31) / 32 < 256 && p.k >= 16 * kBK;
-    if (p.m <= 32) return wide ? launch_skinny<1, 8, FLEX>(p, stream) : launch_skinny<1, 4, FLEX>(p, stream);
-    return wide ? launch_skinny<2, 8, FLEX>(p, stream) : launch_skinny<2, 4, FLEX>(p, stream);
+    return launch_skinny<1, 4, FLEX>(p, stream);
+}
+
+// Tile of a launch: the smallest whose tiles fit the part in one round.  With at most one tile per CU a launch takes a
+// tile's own time - about 2.5 us and, per 128 bytes of K, 0.115 us (32 x 32, K split over the waves), 0.20 (64 x 64), 0.31
+// (128 x 64), 0.48 (128 x 128, four stages), 0.68 (128 x 256), 1.15 (256 x 256) - so smaller tiles win until a second round
+// starts.  Measured at M 16 .. 16384 with ten of the projections' N and K: this choice is the fastest or
+// within 8 % of it.  Against 128 x 128 tiles up to 192 tiles of 256 x 256 (rows x outputs x K, us): 512 x 80 x 1536 9.6 ->
+// 4.1, 3063 x 192 x 5120 21.0 -> 11.7, 512 x 1536 x 3072 14.6 -> 7.7, 777 x 10240 x 2560 45 -> 38, 6144 x 1536 x 3072 47 -> 35.
+int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
+        cus = 256;
+    }
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
+    if (tiles(32, 32) <= cus) return dispatch_skinny<false>(p, stream);
+    if (tiles(64, 64) <= cus) return launch_gemm<1, 1, 2, 2, 4, false>(p, stream);
+    if (tiles(128, 64) <= cus) return launch_gemm<2, 1, 2, 2, 4, false>(p, stream);
+    if (tiles(128, 128) <= cus) return launch_gemm<2, 2, 2, 2, 4, false>(p, stream);
+    if (tiles(128, 256) <= cus) return launch_gemm<2, 2, 2, 4, 3, false>(p, stream);
+    // More than a round: what counts is rounds times the tile's work (128 x 256 at six fifths of its share).
+    auto cost = [&](int64_t bm, int64_t bn) { return ((tiles(bm, bn) + cus - 1) / cus) * bm * bn; };
+    const int64_t c_sq = cost(256, 256), c_wide = cost(256, 320), c_tall = cost(320, 256), c_half = cost(128, 256) * 6 / 5;
+    if (c_half < c_sq && c_half < c_wide && c_half < c_tall) return launch_gemm<2, 2, 2, 4, 3, false>(p, stream);
+    if (c_wide < c_sq && c_wide <= c_tall) return launch_gemm<2, 5, 4, 2, 2, false>(p, stream);
+    // at equal arithmetic the larger tile has fewer rounds, each with its own start and epilogue
+    if (c_tall <= c_sq) return launch_gemm<5, 2, 2, 4, 2, false>(p, stream);
+    return launch_gemm<4, 2, 2, 4, 2, false>(p, stream);                             // 256x256 tile, 8 waves
 }
 
 }  // namespace
@@ -346,33 +374,7 @@ extern "C" int qa_gemm_w8a8(const QaGemmW8A8Params* p, void* stream_) {
         g.a = p->a; g.w = p->w; g.row_scale = p->a_scale; g.col_scale = p->w_scale; g.d = p->d;
         return gemv_launch(g, nullptr, stream);
     }
-    if (p->m <= 64) return flex ? dispatch_skinny<true>(*p, stream) : dispatch_skinny<false>(*p, stream);
     // the single-row rules (host alpha, round-half-away) only ever come with tiny M
-    if (flex) return launch_gemm<2, 2, 2, 2, 2, true>(*p, stream);
-    const int64_t big_tiles = static_cast<int64_t>((p->m + 255) / 256) * ((p->n + 255) / 256);
-    if (big_tiles >= 192) {
-        // One workgroup per CU at a time: the launch runs in rounds of `cus` tiles, so a tile count
-        // just above a multiple of the CU count wastes most of a round.  A 256x320 tile (same 8 waves,
-        // 64x160 each) is taken when it needs fewer tile-rounds' worth of arithmetic.
-        int dev = 0, cus = 256;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
-            cus = 256;
-        }
-        auto cost = [&](int64_t bm, int64_t bn) {
-            const int64_t tiles = ((p->m + bm - 1) / bm) * ((p->n + bn - 1) / bn);
-            return ((tiles + cus - 1) / cus) * bm * bn;
-        };
-        const int64_t c_sq = cost(256, 256), c_wide = cost(256, 320), c_tall = cost(320, 256);
-        if (c_wide < c_sq && c_wide <= c_tall) return launch_gemm<2, 5, 4, 2, 2, false>(*p, stream);
-        // at equal arithmetic the larger tile has fewer rounds, each with its own start and epilogue
-        if (c_tall <= c_sq) return launch_gemm<5, 2, 2, 4, 2, false>(*p, stream);
-        return launch_gemm<4, 2, 2, 4, 2, false>(*p, stream);                        // 256x256 tile, 8 waves
-    }
-    // 128x128 tile, 4 waves.  Two stages (64 KB) let two workgroups share a CU; when there is at most one
-    // workgroup per CU anyway and K is long (x_proj: 16384 x 5120 -> 192), four stages keep three k-tiles
-    // in flight instead of one (36 -> 28 us for that shape).
-    const int64_t small_tiles = static_cast<int64_t>((p->m + 127) / 128) * ((p->n + 127) / 128);
-    if (small_tiles <= 256 && p->k >= 8 * gemm::kBK) return launch_gemm<2, 2, 2, 2, 4, false>(*p, stream);
-    return launch_gemm<2, 2, 2, 2, 2, false>(*p, stream);
+    if (flex) return p->m <= 64 ? dispatch_skinny<true>(*p, stream) : launch_gemm<2, 2, 2, 2, 2, true>(*p, stream);
+    return dispatch_tiles(*p, stream);
 }

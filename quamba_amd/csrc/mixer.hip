@@ -18,7 +18,8 @@
 namespace qa {
 namespace {
 
-constexpr int kExpandOnceRows = 1024;     // 4-bit weights are expanded once per call from this many rows on
+constexpr int kFusedDtRows = 16;
+constexpr int kExpandOnceRows = 65;       // from this many rows on the product may want the 4-bit weights expanded once (qa_gemm_w4a8 decides)
 
 // Sections of the workspace, each 256-byte aligned.
 struct Carver {
@@ -369,7 +370,6 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
     }
 
     QA_TRY(project(p->x_proj, b.x, d, rows, b.x_dbl, QA_OUT_I8, false, b.w8, stream));
-    QA_TRY(project(p->dt_proj, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, false, b.w8, stream));
 
     QaSsmUpdateParams u = {};
     u.batch = rows; u.nheads = 1; u.dim = d; u.dstate = p->d_state; u.ngroups = 1;
@@ -391,7 +391,19 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
     u.x_scale = p->u_scale; u.dt_scale = p->dt_scale; u.dt_bias_scale = p->dt_bias_scale; u.A_log_scale = p->A_scale;
     u.state_scale = p->ssm_state_scale; u.B_scale = p->B_scale; u.C_scale = p->C_scale; u.D_scale = p->D_scale; u.z_scale = p->z_scale;
     u.out = b.y;
-    QA_TRY(qa_ssm_state_update(&u, stream));
+    const QaLinearParams& dt = p->dt_proj;
+    int st = QA_ERR_UNSUPPORTED;
+    // (every batch entry reads the weights again, a row per lane: past a few entries a product of its own is the faster one)
+    if (rows <= kFusedDtRows && dt.bits == 8 && dt.k % 16 == 0) {
+        const SsmDtProj proj = {static_cast<const int8_t*>(dt.weight), b.x_dbl, p->x_proj.n, dt.row_scale, dt.col_scale, dt.k / 16, dt.col_numel,
+                                rows == 1 && dt.row_rule == QA_ROW_ALPHA, dt.alpha};
+        st = ssm_update_with_dt(u, proj, static_cast<hipStream_t>(stream));
+    }
+    if (st == QA_ERR_UNSUPPORTED) {
+        QA_TRY(project(dt, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, false, b.w8, stream));
+        st = qa_ssm_state_update(&u, stream);
+    }
+    QA_TRY(st);
 
     QA_TRY(hadamard(b.y, b.yq, rows, d, p->had_scale, stream));
     return project(p->out_proj, b.yq, d, rows, p->out, QA_OUT_F16, false, b.w8, stream);

@@ -8,6 +8,20 @@ namespace qa {
 // sscan.hip: bytes of scratch qa_sscan_fwd can use for these sizes with token-major inputs (0: none)
 int64_t sscan_token_major_workspace(const QaSScanParams& p);
 
+// sscan.hip: the single-token state update of a Mamba1 layer with dt_proj in front of it: the step size code of channel d is
+// the projection of `x` (16 * pieces codes a batch entry, x_batch_stride apart) with row d of `w` (contiguous rows), scaled
+// and rounded as the int8 product does it.  p.dt is not read.  QA_ERR_UNSUPPORTED where the layer's layout is not the one
+// the fixed-shape update takes.
+struct SsmDtProj {
+    const int8_t *w, *x;
+    int64_t x_batch_stride;
+    const float *row_scale, *col_scale;
+    int pieces, col_numel, use_alpha;
+    float alpha;
+};
+constexpr int kSsmDtPieces = 10;       // up to 160 inputs
+int ssm_update_with_dt(const QaSsmUpdateParams& p, const SsmDtProj& dt, hipStream_t stream);
+
 // conv2.hip: the channel-contiguous forward conv.  Without x_out_scales every channel is an x channel with the one
 // output scale `x_out_scale` (the Mamba1 conv); with conv_state the last inputs of every channel are left there.
 int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream);

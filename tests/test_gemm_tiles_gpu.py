@@ -1,0 +1,56 @@
+"""Every tile the W8A8 and W4A8 products choose from, at sizes with remainders in rows, columns and K, against the oracle."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from quamba_amd import _lib, ops
+from quamba_amd import w4a8_utils as wu
+
+pytestmark = pytest.mark.gpu
+
+
+def _t(a, dev):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+
+
+# 32 x 32 (K over the waves), 64 x 64, 128 x 64, 128 x 128, 128 x 256 in one round and in three, 256 x 256, 320-wide
+@pytest.mark.parametrize("M,N,K", [(130, 60, 272), (9, 2100, 2064), (300, 1000, 528), (900, 1200, 400), (1000, 2100, 384), (2100, 2100, 272),
+                                   (4700, 4700, 144), (4000, 4000, 160), (4200, 4900, 128)])
+@pytest.mark.parametrize("order", [0, 1])
+def test_int8_weights(dev, M, N, K, order):
+    g = np.random.default_rng(M + N + K)
+    a, w = g.integers(-128, 128, (M, K)).astype(np.int8), g.integers(-128, 128, (N, K)).astype(np.int8)
+    sa, sb = (g.uniform(0.5, 1.5, M) * 0.02).astype(np.float32), (g.uniform(0.5, 1.5, N) * 0.6 / np.sqrt(K)).astype(np.float32)
+    acc = oracle.gemm_w8a8(a, w, sa, sb)[0].astype(np.float32)
+    v = sb[None] * (sa[:, None] * acc) if order else sa[:, None] * (sb[None] * acc)
+    want = np.clip(np.rint(v), -128, 127).astype(np.int8)
+    got = torch.empty((M, N), dtype=torch.int8, device=dev)
+    ta, tw, tsa, tsb = _t(a, dev), _t(w, dev), _t(sa, dev), _t(sb, dev)
+    p = _lib.QaGemmW8A8Params()
+    p.m, p.n, p.k, p.a_scale_numel, p.w_scale_numel, p.scale_order = M, N, K, M, N, order
+    p.lda = p.ldw = K
+    p.ldd = N
+    p.a, p.w, p.a_scale, p.w_scale, p.d = (t.data_ptr() for t in (ta, tw, tsa, tsb, got))
+    _lib.check(_lib.lib().qa_gemm_w8a8(ctypes.byref(p), _lib.current_stream(dev)), "gemm_w8a8")
+    np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+# 32 x 32 with four and eight waves, 64 x 64 and 128 x 128 expanding inside, 256 x 256, expanded once
+@pytest.mark.parametrize("M,N,K,workspace", [(70, 200, 2176, False), (100, 1000, 384, False), (600, 2100, 256, False), (300, 4200, 1664, False),
+                                             (900, 6100, 128, False), (4000, 3300, 1664, False), (500, 4200, 1664, True)])
+def test_4_bit_weights(dev, M, N, K, workspace):
+    g = np.random.default_rng(M + N + K)
+    a, codes = g.integers(-128, 128, (M, K)).astype(np.int8), g.integers(0, 16, (N, K)).astype(np.uint8)
+    sg = g.uniform(2.0, 15.8, (K // 128, N)).astype(np.float16)
+    sc, st = (g.uniform(0.5, 1.5, N) * 0.06 / np.sqrt(K) / 8).astype(np.float32), g.uniform(0.5, 1.5, M).astype(np.float32)
+    want = oracle.gemm_w4a8(a, codes, sg, sc, st)[3]
+    packed = wu.pack_w4a8(torch.from_numpy(codes.T.astype(np.int32))).to(dev)
+    rows, ops.W4A8_EXPAND_ONCE_ROWS = ops.W4A8_EXPAND_ONCE_ROWS, 65 if workspace else 1 << 30
+    try:
+        got = ops.w4a8o8_gemm(_t(a, dev), packed, _t(st, dev), _t(sc[None], dev), _t(sg, dev), None, M, N, K)
+    finally:
+        ops.W4A8_EXPAND_ONCE_ROWS = rows
+    np.testing.assert_array_equal(got.cpu().numpy(), want)
