@@ -26,7 +26,7 @@ constexpr int kBatchLoads = 8;    // loads in flight per lane
 
 // grid: x = blocks of 256 channels, y = blocks of 4 runs of `run` steps (one run per wave), z = batch
 template <bool SILU>
-__global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, int run) {
+__global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, int run, int packed) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));   // the same in every lane: the step
                                                                                           // counters below stay in scalar registers
@@ -60,12 +60,23 @@ __global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, in
     uint32_t taps[4];
     float bias_f[4], s_out[4], inv_s_out[4];
     bool exact_only[4];
+    if (packed) {
+        // four taps a channel, back to back: the lane's taps are one 16-byte piece, its biases one word
+        const uint4 w = *reinterpret_cast<const uint4*>(p.weight + ch0 * 4);
+        taps[0] = w.x; taps[1] = w.y; taps[2] = w.z; taps[3] = w.w;
+        const uint32_t b4 = p.bias ? *reinterpret_cast<const uint32_t*>(p.bias + ch0) : 0u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bias_f[e] = part.s_bias * static_cast<float>(static_cast<int8_t>(b4 >> (8 * e)));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            taps[e] = pack_taps(p.weight + (ch0 + e) * p.weight_c_stride, p.weight_width_stride, p.width);
+            bias_f[e] = p.bias ? part.s_bias * static_cast<float>(p.bias[ch0 + e]) : 0.0f;
+        }
+    }
+    out_scales4_of(p, part, ch0, s_out);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const int ch = ch0 + e;
-        taps[e] = pack_taps(p.weight + ch * p.weight_c_stride, p.weight_width_stride, p.width);
-        bias_f[e] = p.bias ? part.s_bias * static_cast<float>(p.bias[ch]) : 0.0f;
-        s_out[e] = out_scale_of(p, part, ch);
         inv_s_out[e] = 1.0f / s_out[e];
         exact_only[e] = conv_needs_exact_route(s_out[e]);
     }
@@ -179,6 +190,58 @@ __global__ __launch_bounds__(kThreads) void conv2_update_kernel(QaConv2Params p)
     out[0] = conv_epilogue(v, out_scale_of(p, part, ch), p.silu_activation);
 }
 
+// The single-step update of four neighbouring channels per lane, for words in every operand: four taps a channel back to
+// back, inputs and outputs with unit channel stride, and a state that is either channel-contiguous (a word per step: the
+// Mamba2 layer's buffer) or four codes a channel (a 16-byte piece: the Mamba1 layer's).  grid: x quads of channels, y batch.
+template <bool CHANNEL_ROWS>
+__global__ __launch_bounds__(kThreads) void conv2_update4_kernel(QaConv2Params p) {
+    const int ch0 = (blockIdx.x * kThreads + threadIdx.x) * 4, b = blockIdx.y;
+    if (ch0 >= p.dim) return;
+    int8_t* st = p.conv_state + b * p.conv_state_batch_stride + ch0 * p.conv_state_c_stride;
+    const uint32_t x_new = *reinterpret_cast<const uint32_t*>(p.xBC + b * p.xBC_batch_stride + ch0);
+    const uint4 w = *reinterpret_cast<const uint4*>(p.weight + ch0 * 4);
+    const uint32_t taps[4] = {w.x, w.y, w.z, w.w};
+    const uint32_t b4 = p.bias ? *reinterpret_cast<const uint32_t*>(p.bias + ch0) : 0u;
+    uint32_t win[4];                                              // byte j of win[e]: input t - 3 + j of channel ch0 + e
+    if constexpr (CHANNEL_ROWS) {
+        const int drop = p.conv_state_len - 3;
+        uint32_t d[4];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) d[i] = *reinterpret_cast<const uint32_t*>(st + (drop + i) * p.conv_state_l_stride);
+        d[3] = x_new;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (i >= 4 - p.conv_state_len) *reinterpret_cast<uint32_t*>(st + (i - (4 - p.conv_state_len)) * p.conv_state_l_stride) = d[i];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t pick = 0x0c0c0000u | ((4u + e) << 8) | e;     // byte e of two words, side by side
+            win[e] = __builtin_amdgcn_perm(d[1], d[0], pick) | (__builtin_amdgcn_perm(d[3], d[2], pick) << 16);
+        }
+    } else {
+        const uint4 h = *reinterpret_cast<const uint4*>(st);
+        const uint32_t held[4] = {h.x, h.y, h.z, h.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) win[e] = (held[e] >> 8) | (((x_new >> (8 * e)) & 0xffu) << 24);
+        *reinterpret_cast<uint4*>(st) = make_uint4(win[0], win[1], win[2], win[3]);
+    }
+    const Part part = part_of(p, ch0);
+    float s_out[4], inv_s_out[4], v[4];
+    bool exact_only[4];
+    out_scales4_of(p, part, ch0, s_out);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        inv_s_out[e] = 1.0f / s_out[e];
+        exact_only[e] = conv_needs_exact_route(s_out[e]);
+        v[e] = part.s_bias * static_cast<float>(static_cast<int8_t>(b4 >> (8 * e)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            v[e] = __builtin_fmaf(part.s_in * static_cast<float>(static_cast<int8_t>(taps[e] >> (8 * i))), static_cast<float>(static_cast<int8_t>(win[e] >> (8 * i))), v[e]);
+    }
+    const ConvQuantRegs kq(__builtin_fminf(__builtin_fminf(s_out[0], s_out[1]), __builtin_fminf(s_out[2], s_out[3])));
+    int64_t out_ls, out_cs;
+    *reinterpret_cast<uint32_t*>(out_ptr(p, part, b, ch0, &out_ls, &out_cs)) = conv_quant4(v, s_out, inv_s_out, p.silu_activation, exact_only, kq);
+}
+
 int validate(const QaConv2Params* p, bool update) {
     if (!p) return QA_ERR_NULL;
     if (p->batch < 0 || p->dim < 0 || p->seqlen < 0 || p->batch > 65535) return QA_ERR_SHAPE;
@@ -219,8 +282,34 @@ int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
     const int64_t run_blocks = (p.seqlen + 4 * run - 1) / (4 * run);
     if (run_blocks > 65535) return QA_ERR_SHAPE;
     dim3 grid((p.dim + 255) / 256, static_cast<unsigned>(run_blocks), p.batch);
-    if (p.silu_activation) hipLaunchKernelGGL(conv2_fwd_kernel<true>, grid, dim3(kThreads), 0, stream, p, run);
-    else hipLaunchKernelGGL(conv2_fwd_kernel<false>, grid, dim3(kThreads), 0, stream, p, run);
+    const int packed = p.width == 4 && p.weight_width_stride == 1 && p.weight_c_stride == 4 && aligned16(p.weight) && aligned4(p.bias);
+    if (p.silu_activation) hipLaunchKernelGGL(conv2_fwd_kernel<true>, grid, dim3(kThreads), 0, stream, p, run, packed);
+    else hipLaunchKernelGGL(conv2_fwd_kernel<false>, grid, dim3(kThreads), 0, stream, p, run, packed);
+    return check_launch();
+}
+}  // namespace qa
+
+namespace qa {
+int conv_single_update(const QaConv2Params& p, hipStream_t stream) {
+    auto mult4 = [](int64_t v) { return v % 4 == 0; };
+    const int64_t bc = static_cast<int64_t>(p.d_state) * p.n_groups;
+    const bool all_x = p.x_dim == p.dim;                          // (the Mamba1 conv: no B and C parts)
+    const bool words = p.width == 4 && p.weight_width_stride == 1 && p.weight_c_stride == 4 && aligned16(p.weight) && aligned4(p.bias) &&
+                       p.xBC_c_stride == 1 && mult4(p.xBC_batch_stride) && aligned4(p.xBC) && mult4(p.x_dim) && (all_x || mult4(bc)) &&
+                       p.x_c_stride == 1 && mult4(p.x_batch_stride) && aligned4(p.x) &&
+                       (all_x || (p.B_c_stride == 1 && mult4(p.B_batch_stride) && aligned4(p.B) && p.C_c_stride == 1 && mult4(p.C_batch_stride) && aligned4(p.C)));
+    const dim3 grid4(static_cast<unsigned>((p.dim / 4 + kThreads - 1) / kThreads), static_cast<unsigned>(p.batch));
+    if (words && p.conv_state_c_stride == 1 && mult4(p.conv_state_l_stride) && mult4(p.conv_state_batch_stride) && aligned4(p.conv_state)) {
+        hipLaunchKernelGGL(conv2_update4_kernel<true>, grid4, dim3(kThreads), 0, stream, p);
+        return check_launch();
+    }
+    if (words && p.conv_state_len == 4 && p.conv_state_l_stride == 1 && p.conv_state_c_stride == 4 && p.conv_state_batch_stride % 16 == 0 && aligned16(p.conv_state)) {
+        hipLaunchKernelGGL(conv2_update4_kernel<false>, grid4, dim3(kThreads), 0, stream, p);
+        return check_launch();
+    }
+    const int64_t blocks = (static_cast<int64_t>(p.batch) * p.dim + kThreads - 1) / kThreads;
+    if (blocks > 0x7fffffffLL) return QA_ERR_SHAPE;
+    hipLaunchKernelGGL(conv2_update_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream, p);
     return check_launch();
 }
 }  // namespace qa
@@ -254,8 +343,5 @@ extern "C" int qa_quamba2_conv1d_update(const QaConv2Params* p, void* stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const int64_t total = static_cast<int64_t>(p->batch) * p->dim;
     if (total == 0) return QA_OK;
-    const int64_t blocks = (total + kThreads - 1) / kThreads;
-    if (blocks > 0x7fffffffLL) return QA_ERR_SHAPE;
-    hipLaunchKernelGGL(conv2_update_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream, *p);
-    return check_launch();
+    return conv_single_update(*p, stream);
 }

@@ -59,6 +59,49 @@ __device__ __forceinline__ float out_scale_of(const QaConv2Params& p, const Part
     return s;
 }
 
+// The same for the four channels ch .. ch + 3 (of one part, ch a multiple of four).  Range tables of up to kRangeUnroll
+// entries and whole quads of channels per head: every entry of a level is requested at once - three round trips instead
+// of a chain of up to a dozen dependent loads per channel, which took longer than a short run's steps.
+constexpr int kRangeUnroll = 8;
+__device__ __forceinline__ void out_scales4_of(const QaConv2Params& p, const Part& part, int ch, float (&s)[4]) {
+    const bool grouped = p.x_head_group_range != nullptr && p.x_dim_group_range != nullptr;
+    if (!p.x_out_scales || !grouped || part.index != 0) {
+        // one scale, or one per ssd group
+        if (!p.x_out_scales || !grouped) {
+            const float one = out_scale_of(p, part, ch);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = one;
+        } else {
+            const float* scales = part.index == 1 ? p.B_out_scales : p.C_out_scales;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = scales[(ch + e - part.offset) / p.d_state];
+        }
+        return;
+    }
+    if (p.nhead_groups > kRangeUnroll || p.ndim_groups > kRangeUnroll || p.x_headdim % 4 != 0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = out_scale_of(p, part, ch + e);
+        return;
+    }
+    const int group_size = p.x_dim / p.n_groups, g = ch / group_size, head = (ch % group_size) / p.x_headdim, d = ch % p.x_headdim;
+    const int32_t* hr = p.x_head_group_range + g * p.nhead_groups;
+    int ends[kRangeUnroll], hg = 0;
+#pragma unroll
+    for (int j = 0; j < kRangeUnroll - 1; ++j) ends[j] = hr[min(j, p.nhead_groups - 1)];
+#pragma unroll
+    for (int j = 0; j < kRangeUnroll - 1; ++j) hg += j < p.nhead_groups - 1 && head >= ends[j] ? 1 : 0;
+    const int row = (g * p.nhead_groups + hg) * p.ndim_groups;
+#pragma unroll
+    for (int j = 0; j < kRangeUnroll - 1; ++j) ends[j] = p.x_dim_group_range[row + min(j, p.ndim_groups - 1)];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        int dg = 0;
+#pragma unroll
+        for (int j = 0; j < kRangeUnroll - 1; ++j) dg += j < p.ndim_groups - 1 && d + e >= ends[j] ? 1 : 0;
+        s[e] = p.x_out_scales[row + dg];
+    }
+}
+
 __device__ __forceinline__ int8_t* out_ptr(const QaConv2Params& p, const Part& part, int b, int ch,
                                             int64_t* l_stride, int64_t* c_stride) {
     const int local = ch - part.offset;

@@ -352,19 +352,8 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
     const int rows = p->batch, d = p->d_inner;
     const int fused = project_conv(p->in_proj, p->hidden, p->d_model, rows, b.xz, 0, conv_of(*p, b), stream);
     if (fused == QA_ERR_UNSUPPORTED) {
-    QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.xz, QA_OUT_I8, false, b.w8, stream));
-
-    QaConvParams c = {};
-    c.batch = rows; c.dim = d; c.seqlen = 1; c.width = p->d_conv;
-    c.silu_activation = 1;
-    c.x_batch_stride = 2 * d; c.x_c_stride = 1; c.x_l_stride = 1;
-    c.out_batch_stride = d; c.out_c_stride = 1; c.out_l_stride = 1;
-    c.weight_c_stride = p->d_conv; c.weight_width_stride = 1;
-    c.conv_state_batch_stride = p->conv_state_batch_stride; c.conv_state_c_stride = p->conv_state_c_stride; c.conv_state_l_stride = p->conv_state_l_stride;
-    c.conv_state_len = p->conv_state_len;
-    c.x = b.xz; c.weight = p->conv_weight; c.bias = p->conv_bias; c.out = b.x; c.conv_state = p->conv_state;
-    c.scale_x = p->conv_scale_x; c.scale_w = p->conv_scale_w; c.scale_b = p->conv_scale_b; c.scale_out = p->conv_scale_out;
-    QA_TRY(qa_causal_conv1d_update(&c, stream));
+        QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.xz, QA_OUT_I8, false, b.w8, stream));
+        QA_TRY(conv_single_update(conv_of(*p, b), static_cast<hipStream_t>(stream)));
     } else if (fused != QA_OK) {
         return fused;
     }

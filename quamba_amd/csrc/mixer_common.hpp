@@ -25,5 +25,7 @@ int ssm_update_with_dt(const QaSsmUpdateParams& p, const SsmDtProj& dt, hipStrea
 // conv2.hip: the channel-contiguous forward conv.  Without x_out_scales every channel is an x channel with the one
 // output scale `x_out_scale` (the Mamba1 conv); with conv_state the last inputs of every channel are left there.
 int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream);
+// the single-step update in the same terms
+int conv_single_update(const QaConv2Params& p, hipStream_t stream);
 
 }  // namespace qa
