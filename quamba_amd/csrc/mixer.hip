@@ -316,7 +316,10 @@ extern "C" int qa_mamba1_forward(const QaMamba1Params* p, void* stream) {
     QA_TRY(conv_channel_last_fwd(conv_of(*p, b), static_cast<hipStream_t>(stream)));
 
     QA_TRY(project(p->x_proj, b.x, d, rows, b.x_dbl, QA_OUT_I8, false, b.w8, stream));
-    QA_TRY(project(p->dt_proj, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, true, b.w8, stream));
+    const QaLinearParams& dtp = p->dt_proj;
+    const bool fused_dt = dtp.bits == 8 && dtp.k % 16 == 0 && dtp.k <= kSscanDtRank && p->x_proj.n % 16 == 0 &&
+                          len * static_cast<int64_t>(p->x_proj.n) < 1 << 30;
+    if (!fused_dt) QA_TRY(project(dtp, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, true, b.w8, stream));
 
     QaSScanParams s = scan_sizes(*p);
     const int64_t dbl = p->x_proj.n;
@@ -338,7 +341,8 @@ extern "C" int qa_mamba1_forward(const QaMamba1Params* p, void* stream) {
     if (p->state_is_fp32) s.last_state_f32 = static_cast<float*>(p->ssm_state);
     else s.last_state_i8 = static_cast<int8_t*>(p->ssm_state);
     s.workspace = b.scan.p; s.workspace_bytes = b.scan.bytes;
-    QA_TRY(qa_sscan_fwd(&s, stream));
+    const SscanDtProj proj = {static_cast<const int8_t*>(dtp.weight), b.x_dbl, len * dbl, dbl, dtp.row_scale, dtp.col_scale, dtp.k, dtp.col_numel};
+    QA_TRY(sscan_token_major_fwd(s, fused_dt ? &proj : nullptr, static_cast<hipStream_t>(stream)));
 
     QA_TRY(hadamard(b.y, b.yq, rows, d, p->had_scale, stream));
     return project(p->out_proj, b.yq, d, rows, p->out, QA_OUT_F16, false, b.w8, stream);

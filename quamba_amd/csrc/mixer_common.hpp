@@ -5,7 +5,18 @@
 
 namespace qa {
 
-// sscan.hip: bytes of scratch qa_sscan_fwd can use for these sizes with token-major inputs (0: none)
+// sscan_tm.hip: qa_sscan_fwd for token-major inputs.  With `dt` the step size codes are not read but made in the scan:
+// dt_proj's product of x (x_proj's rows, x_l_stride apart) with w (d_inner rows of `rank` codes, a multiple of 16 up to 192),
+// scaled col * (row * acc) and rounded as the int8 product does it.  seqlen * x_l_stride below 2^30.
+struct SscanDtProj {
+    const int8_t *w, *x;
+    int64_t x_batch_stride, x_l_stride;
+    const float *row_scale, *col_scale;
+    int rank, col_numel;
+};
+constexpr int kSscanDtRank = 192;
+int sscan_token_major_fwd(const QaSScanParams& p, const SscanDtProj* dt, hipStream_t stream);
+// bytes of scratch it can use for these sizes (0: none)
 int64_t sscan_token_major_workspace(const QaSScanParams& p);
 
 // sscan.hip: the single-token state update of a Mamba1 layer with dt_proj in front of it: the step size code of channel d is

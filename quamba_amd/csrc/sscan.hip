@@ -22,107 +22,10 @@
 #include "qa_common.hpp"
 #include "conv_common.hpp"
 #include "mixer_common.hpp"
-
-#include <algorithm>
+#include "sscan_common.hpp"
 
 namespace qa {
 namespace {
-
-// A sequence cut into `count` segments of `len` steps (the last may be shorter) that are scanned side by side: one
-// pass for every segment's end state from a zero state and the sum of its step sizes, one that starts every segment
-// from the state its predecessors chain up to.
-struct SscanSegments {
-    int count, len;
-};
-inline int64_t sscan_segment_bytes(const QaSScanParams& p, const SscanSegments& s) {
-    return static_cast<int64_t>(p.batch) * (s.count - 1) * p.dim * (1 + p.dstate) * 4;
-}
-
-constexpr float kLog2e = 1.44269504088896341f;
-
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-__device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
-__device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-
-// float(int8 code in byte n of w) in one instruction (the sub-dword operand select converts the byte in place; the
-// compiler, left to itself, shifts and sign-extends the byte out first)
-__device__ __forceinline__ float code_byte_to_float(uint32_t w, int n) {
-    float r;
-    switch (n) {
-        case 0: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(r) : "v"(w)); break;
-        case 1: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(r) : "v"(w)); break;
-        case 2: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(r) : "v"(w)); break;
-        default: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(r) : "v"(w)); break;
-    }
-    return r;
-}
-
-// softplus with the reference's threshold; log1p evaluated so that small exp(x) keeps full
-// relative accuracy (series below 2^-6, log2 above).
-__device__ __forceinline__ float softplus20(float x) {
-    if (x > 20.0f) return x;
-    const float e = fast_exp2(x * kLog2e);
-    const float series = e * __builtin_fmaf(e, __builtin_fmaf(e, __builtin_fmaf(e, -0.25f, 1.0f / 3.0f), -0.5f), 1.0f);
-    const float big = fast_log2(1.0f + e) * 0.693147180559945309f;
-    return e < 0.015625f ? series : big;
-}
-
-// The same function without a branch and with one rounding compensated instead of a series:
-//   softplus(x) = max(x, 0) + log1p(e),  e = exp(-|x|) in (0, 1]
-//   u = fl(1 + e) = 1 + e + r with r = (u - 1) - e exact, so log1p(e) = ln(u - r) = ln u - r / u + ..., and with
-//   u in [1, 2] taking r for r / u is wrong by less than 2^-24 of the result.
-// Above the threshold the second term is below half an ulp of x, so x comes back exactly, as the reference returns it.
-__device__ __forceinline__ float softplus20_flat(float x) {
-    const float e = fast_exp2(__builtin_fabsf(x) * -kLog2e);
-    const float u = 1.0f + e;
-    const float r = (u - 1.0f) - e;
-    const float sp = __builtin_fmaf(fast_log2(u), 0.693147180559945309f, -r);
-    float pos;                                        // max(x, 0): written out, because the builtins put a second
-    asm("v_max_f32 %0, 0, %1" : "=v"(pos) : "v"(x));  // maximum of x with itself in front of it (quieting of NaNs)
-    return pos + sp;
-}
-
-__device__ __forceinline__ float silu_gate(float z) {
-    return z * fast_rcp(1.0f + fast_exp2(-z * kLog2e));
-}
-
-// Value of `v` in the lane of this quad that holds slice SRC of the same channel (NSPLIT lanes per
-// channel, NSPLIT in {1,2,4}), as a DPP quad permutation that the compiler folds into the consumer.
-template <int NSPLIT, int SRC>
-__device__ __forceinline__ float quad_bcast(float v) {
-    if (NSPLIT == 1) return v;
-    constexpr int ctrl = NSPLIT == 4 ? (SRC | (SRC << 2) | (SRC << 4) | (SRC << 6))
-                                     : (SRC | (SRC << 2) | ((2 + SRC) << 4) | ((2 + SRC) << 6));
-    const int r = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, false);
-    return __builtin_bit_cast(float, r);
-}
-// Same with a source slice that is a constant only after loop unrolling.
-template <int NSPLIT>
-__device__ __forceinline__ float quad_bcast_sel(float v, int src) {
-    switch (src) {
-        case 0: return quad_bcast<NSPLIT, 0>(v);
-        case 1: return quad_bcast<NSPLIT, 1>(v);
-        case 2: return quad_bcast<NSPLIT, (NSPLIT > 2 ? 2 : 0)>(v);
-        default: return quad_bcast<NSPLIT, (NSPLIT > 2 ? 3 : 1)>(v);
-    }
-}
-// Value of `v` in lane (lane ^ M) of the quad, M in {1,2}.
-template <int M>
-__device__ __forceinline__ float quad_xor(float v) {
-    constexpr int ctrl = M == 1 ? (1 | (0 << 2) | (3 << 4) | (2 << 6)) : (2 | (3 << 2) | (0 << 4) | (1 << 6));
-    const int r = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, false);
-    return __builtin_bit_cast(float, r);
-}
-
-// Value of `v` in the lane four above, inside a row of sixteen lanes (zero past its end).
-__device__ __forceinline__ float row_from_4_up(float v) {
-    const int r = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x104, 0xf, 0xf, true);     // row_shl:4
-    return __builtin_bit_cast(float, r);
-}
-
-__device__ __forceinline__ float i8_of(uint32_t word, int j) {
-    return static_cast<float>(static_cast<int8_t>((word >> (8 * j)) & 0xffu));
-}
 
 // 16 bytes starting at row[t]; bytes at or beyond t_end read as zero.
 __device__ __forceinline__ uint4 load16(const int8_t* row, int t, int t_end, bool vec) {
@@ -531,13 +434,8 @@ __device__ __forceinline__ void load_bytes(uint32_t (&w)[BYTES / 4], const int8_
     }
 }
 
-// TM: u, delta, z and B | C are token-major (channels contiguous, QaSScanParams.token_major).  A wave then stages its own
-// channels with dword loads of four channels and one step: a lane evaluates four channels at one or two steps instead of
-// one channel at eight or four.  Tails need no path of their own: steps past the end read the last step and are given
-// step size zero.  With segments, entry y of the grid is segment y % segments of batch entry y / segments.
-// OUT false: only the end state and the sum of the step sizes (the first pass over the segments).
-template <int NPL, int NSPLIT, int WAVES, bool HAS_Z, bool TM = false, bool OUT = true>
-__device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int vec_in, int vec_bc, int vec_out, int c0, int y,
+template <int NPL, int NSPLIT, int WAVES, bool HAS_Z>
+__device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int vec_in, int vec_bc, int vec_out, int c0, int b,
                                                    PreSmem<PreCfg<NPL, NSPLIT, WAVES>>& sm) {
     using Cfg = PreCfg<NPL, NSPLIT, WAVES>;
     constexpr int T = Cfg::T, kThreads = Cfg::kThreads, kCh = Cfg::kCh, kNP = Cfg::kNP, kStage = Cfg::kStage;
@@ -552,12 +450,8 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
     const int c = c0 + c_local;
     const bool c_ok = c < p.dim;
     const int cc = c_ok ? c : p.dim - 1;                   // clamped channel for parameter loads
-    const int g = TM ? 0 : c0 / (p.dim / p.n_groups);
-    const int segments = TM ? max(p.segments, 1) : 1;
-    const int per_entry = OUT ? segments : segments - 1;   // the last segment's end state is nobody's start
-    const int b = TM ? y / per_entry : y, seg_i = TM ? y - b * per_entry : 0;
-    const int t_base = seg_i * p.segment_len;              // (0 without segments)
-    const int L = TM && segments > 1 ? min(p.segment_len, p.seqlen - t_base) : p.seqlen;
+    const int g = c0 / (p.dim / p.n_groups);
+    const int L = p.seqlen;
     const bool softplus = p.delta_softplus != 0;
 
     const float s_u = *p.scale_u, s_dt = *p.scale_delta, s_A = *p.scale_A, s_B = *p.scale_B, s_C = *p.scale_C;
@@ -575,9 +469,9 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
                     ? -expf(s_A * static_cast<float>(p.A_log[cc * p.A_d_stride + n * p.A_dstate_stride])) * kLog2e
                     : 0.0f;
     }
-    if (OUT && p.carry_state) {          // segments of one sequence side by side, see sscan_fwd_body
-        const int first = TM ? b * (segments - 1) : 0, seg = TM ? first + seg_i : p.carry_first + b;
-        for (int sp = first; sp < seg; ++sp) {
+    if (p.carry_state) {                 // segments of one sequence side by side, see sscan_fwd_body
+        const int seg = p.carry_first + b;
+        for (int sp = 0; sp < seg; ++sp) {
             const float sd = p.carry_dt_sum[static_cast<int64_t>(sp) * p.dim + cc];
 #pragma unroll
             for (int j = 0; j < NPL; ++j) {
@@ -607,7 +501,7 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
     const int8_t* bc_row[kBcPieces];
     float bc_factor[kBcPieces];
 #pragma unroll
-    for (int i = 0; i < (TM ? 0 : kBcPieces); ++i) {
+    for (int i = 0; i < kBcPieces; ++i) {
         int which, n, col;
         bc_piece(tid + i * kThreads, which, n, col);
         const int nn = min(n, p.dstate - 1);
@@ -620,45 +514,7 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
     // A tile that lies inside the sequence, of rows that allow vector loads, is requested without a branch per lane: the
     // requests then stay in flight until stage() needs them.  (With the byte-wise alternative in the same control
     // flow the compiler waits for every request where the two paths join.)
-    // TM: this lane's share of a wave's tile: four channels from lc4 on, kSteps steps from ls * kSteps on
-    constexpr int kQuads = 64 / NSPLIT / 4, kSteps = kStage / 4;
-    const int lane = tid & 63, lc4 = (tid >> 6) * (64 / NSPLIT) + 4 * (lane % kQuads), ls = lane / kQuads;
-    const int ch4 = min(c0 + lc4, p.dim - 4);              // channels past the last read the last four; nothing of theirs is stored
-    float db4[TM ? 4 : 1], dt_sum4[TM ? 4 : 1] = {};
-    const int8_t *u_tm = nullptr, *d_tm = nullptr, *z_tm = nullptr, *bc_tm = nullptr;
-    int bc_step = 0;
-    float bc_scale = 0.0f;
-    int64_t bc_ls = 0;
-    if constexpr (TM) {
-        u_tm = p.u + b * p.u_batch_stride + t_base * p.u_l_stride + ch4;
-        d_tm = p.delta + b * p.delta_batch_stride + t_base * p.delta_l_stride + ch4;
-        if constexpr (HAS_Z && OUT) z_tm = p.z + b * p.z_batch_stride + t_base * p.z_l_stride + ch4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) db4[e] = p.delta_bias ? *p.scale_delta_bias * static_cast<float>(p.delta_bias[ch4 + e]) : 0.0f;
-        // B | C: dword tid % 8 of a step's sixteen B and sixteen C codes
-        static_assert(kThreads % 8 == 0, "whole steps of B and C per pass");
-        const int dw = tid & 7;
-        bc_step = tid >> 3;
-        bc_ls = dw < 4 ? p.B_l_stride : p.C_l_stride;
-        bc_tm = (dw < 4 ? p.B + b * p.B_batch_stride + t_base * p.B_l_stride : p.C + b * p.C_batch_stride + t_base * p.C_l_stride) + 4 * (dw & 3);
-        bc_scale = dw < 4 ? s_B * s_u : s_C;
-    }
     auto issue_loads = [&](int t0) {
-        if constexpr (TM) {
-#pragma unroll
-            for (int i = 0; i < kSteps; ++i) {
-                const int64_t t = min(t0 + ls * kSteps + i, L - 1);
-                r_u[i] = *reinterpret_cast<const uint32_t*>(u_tm + t * p.u_l_stride);
-                r_d[i] = *reinterpret_cast<const uint32_t*>(d_tm + t * p.delta_l_stride);
-                if constexpr (HAS_Z && OUT) r_z[i] = *reinterpret_cast<const uint32_t*>(z_tm + t * p.z_l_stride);
-            }
-#pragma unroll
-            for (int i = 0; i < kBcPieces; ++i) {
-                const int64_t t = min(t0 + bc_step + i * (kThreads / 8), L - 1);
-                r_bc[i] = *reinterpret_cast<const uint32_t*>(bc_tm + t * bc_ls);
-            }
-            return;
-        }
         const int t = t0 + slice * kStage;
         const bool whole = t0 + T <= L;
         // rows past the last channel read the last channel's bytes; nothing of theirs is stored
@@ -702,63 +558,6 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
     // Writes the staged tile.  Per step of this lane's share of its channel: step size (bias, softplus), step
     // size x input, skip term and gate - everything the time loop needs that does not depend on the state.
     auto stage = [&](int t0, int into) {
-        if constexpr (TM) {
-            float dv[kSteps][4], duv[kSteps][4];
-#pragma unroll
-            for (int i = 0; i < kSteps; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) dv[i][e] = __builtin_fmaf(s_dt, i8_of(r_d[i], e), db4[e]);
-            if (softplus) {
-#pragma unroll
-                for (int i = 0; i < kSteps; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) dv[i][e] = softplus20_flat(dv[i][e]);
-            }
-            if (t0 + T > L) {
-#pragma unroll
-                for (int i = 0; i < kSteps; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) dv[i][e] = t0 + ls * kSteps + i < L ? dv[i][e] : 0.0f;
-            }
-#pragma unroll
-            for (int i = 0; i < kSteps; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if constexpr (!OUT) dt_sum4[e] += dv[i][e];
-                    duv[i][e] = dv[i][e] * i8_of(r_u[i], e);
-                }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int t = ls * kSteps;
-                if constexpr (kSteps == 2) {
-                    *reinterpret_cast<float2*>(&sm.d[lc4 + e][t]) = make_float2(dv[0][e], dv[1][e]);
-                    *reinterpret_cast<float2*>(&sm.du[lc4 + e][t]) = make_float2(duv[0][e], duv[1][e]);
-                } else {
-                    sm.d[lc4 + e][t] = dv[0][e];
-                    sm.du[lc4 + e][t] = duv[0][e];
-                }
-                if constexpr (OUT) {
-                    // (u z) of this channel's steps, bytewise
-                    const uint32_t sel = 0x0c0c0400u + 0x0101u * e;
-                    const uint32_t c_first = __builtin_amdgcn_perm(HAS_Z ? r_z[0] : 0u, r_u[0], sel);
-                    if constexpr (kSteps == 2) {
-                        const uint32_t c_second = __builtin_amdgcn_perm(HAS_Z ? r_z[1] : 0u, r_u[1], sel);
-                        *reinterpret_cast<uint32_t*>(&sm.uz[lc4 + e][t]) = c_first | (c_second << 16);
-                    } else {
-                        sm.uz[lc4 + e][t] = static_cast<uint16_t>(c_first);
-                    }
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < kBcPieces; ++i) {
-                const int t = bc_step + i * (kThreads / 8);
-                if (kBcPieces * kThreads / 8 == T || t < T) {
-                    *reinterpret_cast<float4*>(&sm.bc[into][t][4 * (tid & 7)]) =
-                        make_float4(bc_scale * i8_of(r_bc[i], 0), bc_scale * i8_of(r_bc[i], 1), bc_scale * i8_of(r_bc[i], 2), bc_scale * i8_of(r_bc[i], 3));
-                }
-            }
-            return;
-        }
         float dv[kStage], duv[kStage];
 #pragma unroll
         for (int e = 0; e < kStage; ++e) dv[e] = __builtin_fmaf(s_dt, i8_of(r_d[e >> 2], e & 3), db);
@@ -814,11 +613,7 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const float* row = sm.bc[from][tq * 4 + j];
-            if constexpr (!OUT) {
-                // (the first pass over segments needs no C)
-#pragma unroll
-                for (int n = 0; n < NPL; ++n) o.B[j][n] = row[slice * NPL + n];
-            } else if constexpr (NPL == 2) {
+            if constexpr (NPL == 2) {
                 const float2 Bv = *reinterpret_cast<const float2*>(row + slice * NPL);
                 const float2 Cv = *reinterpret_cast<const float2*>(row + kNP + slice * NPL);
                 o.B[j][0] = Bv.x; o.B[j][1] = Bv.y; o.C[j][0] = Cv.x; o.C[j][1] = Cv.y;
@@ -829,12 +624,12 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
                 o.C[j][0] = Cv.x; o.C[j][1] = Cv.y; o.C[j][2] = Cv.z; o.C[j][3] = Cv.w;
             }
         }
-        if constexpr (OUT) o.code = sm.uz[c_local][tq * 4 + qslice];
+        o.code = sm.uz[c_local][tq * 4 + qslice];
     };
 
     const int n_tiles = (L + T - 1) / T;
     issue_loads(0);
-    if constexpr (HAS_Z && OUT) {
+    if constexpr (HAS_Z) {
         for (int i = tid; i < 256; i += kThreads) sm.gate_table[i] = silu_gate(s_z * static_cast<float>(static_cast<int8_t>(i)));
         __syncthreads();
     }
@@ -864,7 +659,7 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
             __builtin_amdgcn_sched_barrier(0);
             // the gate of the step this lane owns: looked up now, used when the group's sums are complete
             float gate = 1.0f;
-            if constexpr (HAS_Z && OUT) gate = sm.gate_table[(o.code >> 8) & 0xffu];
+            if constexpr (HAS_Z) gate = sm.gate_table[(o.code >> 8) & 0xffu];
             float acc[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -873,10 +668,9 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
                 for (int n = 0; n < NPL; ++n) {
                     const float a = fast_exp2(o.d[j] * A2[n]);
                     h[n] = __builtin_fmaf(a, h[n], o.B[j][n] * o.du[j]);
-                    if constexpr (OUT) acc[j] = __builtin_fmaf(h[n], o.C[j][n], acc[j]);
+                    acc[j] = __builtin_fmaf(h[n], o.C[j][n], acc[j]);
                 }
             }
-            if constexpr (!OUT) continue;
             // each lane of a quad completes the step it owns: a transposing reduction (keep one half, hand the
             // other half to the neighbour) instead of four full ones
             const bool odd = qslice & 1, hi = qslice & 2;
@@ -885,19 +679,19 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
             float own_sum = (hi ? w23 : w01) + quad_xor<2>(hi ? w01 : w23);
             // eight lanes per channel: the other quad holds the other half of the states.  The first quad takes them
             // with a row shift inside the addition (a lane permute through LDS would be a round trip in every group)
-            if constexpr (NSPLIT == 8) own_sum += row_from_4_up(own_sum);
-            float out_v = own_sum + D_u * code_byte_to_float(o.code, 0);
-            if constexpr (HAS_Z) out_v *= gate;
-            sm.out[buf][tq * 4 + qslice][out_col] = __float2half(out_v);
+            if constexpr (NSPLIT == 8) own_sum += row_from_up<4>(own_sum);
+            float y = own_sum + D_u * code_byte_to_float(o.code, 0);
+            if constexpr (HAS_Z) y *= gate;
+            sm.out[buf][tq * 4 + qslice][out_col] = __float2half(y);
         }
         // the next tile goes into the other copy (every wave left it at the barrier of the tile before)
         if (tile + 1 < n_tiles) stage(t0 + T, buf ^ 1);
         __syncthreads();   // this tile's outputs and the next tile's B / C are complete
 
         // write the tile's output rows: (t, kCh channels) contiguous along channels
-        if constexpr (OUT) {
+        {
             constexpr int kChunksPerRow = kCh / 8;
-            __half* out_b = static_cast<__half*>(p.out) + b * p.out_batch_stride + t_base * p.out_l_stride;
+            __half* out_b = static_cast<__half*>(p.out) + b * p.out_batch_stride;
             for (int piece = tid; piece < nt * kChunksPerRow; piece += kThreads) {
                 const int t = piece / kChunksPerRow, ch8 = (piece % kChunksPerRow) * 8;
                 __half* dst = out_b + (t0 + t) * p.out_l_stride + (c0 + ch8) * p.out_d_stride;
@@ -913,23 +707,7 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
         buf ^= 1;
     }
 
-    if constexpr (TM && !OUT) {
-        // first pass over the segments: the sum of the step sizes of each channel, and its end state, as fp32
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-#pragma unroll
-            for (int m = kQuads; m < 64; m <<= 1) dt_sum4[e] += __shfl_xor(dt_sum4[e], m);
-            if (ls == 0 && c0 + lc4 < p.dim) p.dt_sum_out[static_cast<int64_t>(y) * p.dim + c0 + lc4 + e] = dt_sum4[e];
-        }
-        if (c_ok) {
-            float* to = const_cast<float*>(p.carry_state) + (static_cast<int64_t>(y) * p.dim + c) * p.dstate + slice * NPL;
-#pragma unroll
-            for (int j = 0; j < NPL; ++j) to[j] = h[j];
-        }
-        return;
-    }
-    if (TM && seg_i != segments - 1) return;
-    if (!TM && p.dt_sum_out) {
+    if (p.dt_sum_out) {
         // the lanes of a channel staged different steps
         dt_sum += quad_xor<1>(dt_sum);
         dt_sum += quad_xor<2>(dt_sum);
@@ -950,11 +728,11 @@ __device__ __forceinline__ void sscan_fwd_pre_body(const QaSScanParams& p, int v
     }
 }
 
-template <int NPL, int NSPLIT, int WAVES, bool HAS_Z, bool TM = false, bool OUT = true>
+template <int NPL, int NSPLIT, int WAVES, bool HAS_Z>
 __global__ __launch_bounds__(64 * WAVES) void sscan_fwd_pre_kernel(QaSScanParams p, int vec_in, int vec_bc, int vec_out) {
     using Cfg = PreCfg<NPL, NSPLIT, WAVES>;
     __shared__ PreSmem<Cfg> sm;
-    sscan_fwd_pre_body<NPL, NSPLIT, WAVES, HAS_Z, TM, OUT>(p, vec_in, vec_bc, vec_out, blockIdx.x * Cfg::kCh, blockIdx.y, sm);
+    sscan_fwd_pre_body<NPL, NSPLIT, WAVES, HAS_Z>(p, vec_in, vec_bc, vec_out, blockIdx.x * Cfg::kCh, blockIdx.y, sm);
 }
 
 // Two kinds of workgroup in one launch, for d_state 16: the first `blocks_a` workgroups of a batch entry take
@@ -963,7 +741,7 @@ __global__ __launch_bounds__(64 * WAVES) void sscan_fwd_pre_kernel(QaSScanParams
 // time does not depend on how many of its lanes are busy, so what counts is the number of waves per SIMD: when
 // the four-lane mapping alone would leave half of the SIMDs with one wave more than the others, the tail of the
 // channels goes to the short kind and every SIMD gets the same mix.
-template <bool HAS_Z, bool TM = false>
+template <bool HAS_Z>
 __global__ __launch_bounds__(256) void sscan_fwd_mixed_kernel(QaSScanParams p, int vec_in, int vec_bc, int vec_out, int blocks_a) {
     using CfgA = PreCfg<4, 4, 4>;
     using CfgB = PreCfg<2, 8, 4>;
@@ -974,9 +752,9 @@ __global__ __launch_bounds__(256) void sscan_fwd_mixed_kernel(QaSScanParams p, i
     } sm;
     const int bx = blockIdx.x;
     if (bx < blocks_a) {
-        sscan_fwd_pre_body<4, 4, 4, HAS_Z, TM>(p, vec_in, vec_bc, vec_out, bx * CfgA::kCh, blockIdx.y, sm.a);
+        sscan_fwd_pre_body<4, 4, 4, HAS_Z>(p, vec_in, vec_bc, vec_out, bx * CfgA::kCh, blockIdx.y, sm.a);
     } else {
-        sscan_fwd_pre_body<2, 8, 4, HAS_Z, TM>(p, vec_in, vec_bc, vec_out, blocks_a * CfgA::kCh + (bx - blocks_a) * CfgB::kCh, blockIdx.y, sm.b);
+        sscan_fwd_pre_body<2, 8, 4, HAS_Z>(p, vec_in, vec_bc, vec_out, blocks_a * CfgA::kCh + (bx - blocks_a) * CfgB::kCh, blockIdx.y, sm.b);
     }
 }
 
@@ -1048,63 +826,6 @@ int choose_mapping16(const QaSScanParams& p) {
     return QA_SSCAN_MAPPING(4, 4);
 }
 
-// Token-major inputs (sixteen states, one group).  With a workspace and few waves the sequence is scanned as segments.
-SscanSegments plan_segments(const QaSScanParams& p) {
-    SscanSegments r = {1, p.seqlen};
-    const int64_t simds = 4LL * 256, waves = static_cast<int64_t>(p.batch) * p.dim / 8;       // eight lanes per channel
-    if (2 * waves > 3 * simds || p.seqlen < 256) return r;
-    int segs = static_cast<int>(std::min<int64_t>(3 * simds / waves, 16));
-    segs = std::min(segs, p.seqlen / 128);
-    if (segs < 2) return r;
-    r.len = ((p.seqlen + segs - 1) / segs + 31) / 32 * 32;
-    r.count = (p.seqlen + r.len - 1) / r.len;
-    return r;
-}
-
-int launch_token_major(const QaSScanParams& p_in, hipStream_t stream) {
-    QaSScanParams p = p_in;
-    const auto mult4 = [](int64_t v) { return v % 4 == 0; };
-    if (p.dstate != 16 || p.n_groups != 1 || p.dim < 4 || !mult4(p.dim) || p.carry_state || p.dt_sum_out) return QA_ERR_UNSUPPORTED;
-    if (p.u_d_stride != 1 || p.delta_d_stride != 1 || (p.z && p.z_d_stride != 1) || p.B_dstate_stride != 1 || p.C_dstate_stride != 1) return QA_ERR_STRIDE;
-    if (!aligned4(p.u) || !aligned4(p.delta) || !aligned4(p.z) || !aligned4(p.B) || !aligned4(p.C)) return QA_ERR_STRIDE;
-    for (const int64_t v : {p.u_batch_stride, p.u_l_stride, p.delta_batch_stride, p.delta_l_stride, p.z ? p.z_batch_stride : 0,
-                            p.z ? p.z_l_stride : 0, p.B_batch_stride, p.B_l_stride, p.C_batch_stride, p.C_l_stride})
-        if (!mult4(v)) return QA_ERR_STRIDE;
-    const int vec_out = p.out_d_stride == 1 && aligned16(p.out) && p.out_batch_stride % 8 == 0 && p.out_l_stride % 8 == 0;
-    p.segments = 1;
-    p.segment_len = 0;
-    const SscanSegments seg = plan_segments(p);
-    if (seg.count > 1 && p.workspace && p.workspace_bytes >= sscan_segment_bytes(p, seg)) {
-        const int64_t entries = static_cast<int64_t>(p.batch) * (seg.count - 1);
-        if (static_cast<int64_t>(p.batch) * seg.count > 65535) return QA_ERR_SHAPE;
-        p.segments = seg.count;
-        p.segment_len = seg.len;
-        p.dt_sum_out = static_cast<float*>(p.workspace);
-        p.carry_dt_sum = p.dt_sum_out;
-        p.carry_state = p.dt_sum_out + entries * p.dim;
-        hipLaunchKernelGGL((sscan_fwd_pre_kernel<2, 8, 4, true, true, false>), dim3((p.dim + 31) / 32, static_cast<unsigned>(entries)), dim3(256), 0, stream, p, 1, 1, vec_out);
-        const dim3 grid((p.dim + 31) / 32, static_cast<unsigned>(p.batch * seg.count));
-        if (p.z) hipLaunchKernelGGL((sscan_fwd_pre_kernel<2, 8, 4, true, true>), grid, dim3(256), 0, stream, p, 1, 1, vec_out);
-        else hipLaunchKernelGGL((sscan_fwd_pre_kernel<2, 8, 4, false, true>), grid, dim3(256), 0, stream, p, 1, 1, vec_out);
-        return check_launch();
-    }
-    const int mapping = choose_mapping16(p);
-    const int lanes = (mapping >> 20) & 0xff, arg = mapping & 0xfffff;
-    if (lanes == 0) {
-        const dim3 grid(arg + (p.dim - 64 * arg + 31) / 32, p.batch);
-        if (p.z) hipLaunchKernelGGL((sscan_fwd_mixed_kernel<true, true>), grid, dim3(256), 0, stream, p, 1, 1, vec_out, arg);
-        else hipLaunchKernelGGL((sscan_fwd_mixed_kernel<false, true>), grid, dim3(256), 0, stream, p, 1, 1, vec_out, arg);
-    } else if (lanes == 8) {
-        const dim3 grid((p.dim + 31) / 32, p.batch);
-        if (p.z) hipLaunchKernelGGL((sscan_fwd_pre_kernel<2, 8, 4, true, true>), grid, dim3(256), 0, stream, p, 1, 1, vec_out);
-        else hipLaunchKernelGGL((sscan_fwd_pre_kernel<2, 8, 4, false, true>), grid, dim3(256), 0, stream, p, 1, 1, vec_out);
-    } else {
-        const dim3 grid((p.dim + 63) / 64, p.batch);
-        if (p.z) hipLaunchKernelGGL((sscan_fwd_pre_kernel<4, 4, 4, true, true>), grid, dim3(256), 0, stream, p, 1, 1, vec_out);
-        else hipLaunchKernelGGL((sscan_fwd_pre_kernel<4, 4, 4, false, true>), grid, dim3(256), 0, stream, p, 1, 1, vec_out);
-    }
-    return check_launch();
-}
 // ---------------------------------------------------------------------------------------------
 // Single-token update.  LPR lanes share one (batch, head, channel) row, up to sixteen states per lane
 // in pieces of four, so consecutive lanes touch consecutive 16-byte (fp32 state) or 4-byte (int8
@@ -1479,11 +1200,6 @@ int launch_update(const QaSsmUpdateParams& p, hipStream_t stream, const QaConvPa
 }  // namespace
 }  // namespace qa
 
-int64_t qa::sscan_token_major_workspace(const QaSScanParams& p) {
-    const SscanSegments seg = plan_segments(p);
-    return seg.count > 1 ? sscan_segment_bytes(p, seg) : 0;
-}
-
 extern "C" int qa_sscan_chosen_mapping(const QaSScanParams* p) {
     if (!p) return QA_ERR_NULL;
     if (p->batch < 1 || p->dim < 1 || p->dstate < 1 || p->dstate > 256) return QA_ERR_SHAPE;
@@ -1514,7 +1230,7 @@ extern "C" int qa_sscan_fwd(const QaSScanParams* p, void* stream_) {
     if ((p->D && !p->scale_D) || (p->delta_bias && !p->scale_delta_bias) || (p->z && !p->scale_z)) return QA_ERR_NULL;
     if (p->last_state_i8 && !p->scale_ssm_state) return QA_ERR_NULL;
     if (p->batch > 65535) return QA_ERR_SHAPE;
-    if (p->token_major) return launch_token_major(*p, stream);
+    if (p->token_major) return sscan_token_major_fwd(*p, nullptr, stream);
 
     auto ok16 = [](const void* ptr, std::initializer_list<int64_t> strides) {
         if (!aligned16(ptr)) return 0;

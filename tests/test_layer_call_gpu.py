@@ -81,6 +81,18 @@ def test_step_of_a_wide_layer(dev, d_model):
         _close(out[:, 0], m._step_modules(h, conv2, ssm2), (conv, conv2), (ssm, ssm2))
 
 
+@pytest.mark.parametrize("d_model,batch,seqlen", [(768, 1, 65), (768, 16, 33), (1536, 1, 515), (1536, 12, 70), (2560, 16, 31), (3072, 3, 100)])
+def test_forward_of_a_wide_layer(dev, d_model, batch, seqlen):
+    """dt_proj inside the scan: ranks of 48, 96, 160 and 192, sixteen, eight and four lanes per channel, both at once."""
+    m, g = _mamba1(W8A8QMamba, dev, seed=seqlen, d_model=d_model)
+    h = _ri(dev, g, batch, seqlen, d_model)
+    conv, ssm = _states(m, dev, g, batch, torch.float32, 4)
+    conv2, ssm2 = conv.clone(), ssm.clone()
+    out = _layer_call.call(m, h, conv, ssm, False)
+    want = m._forward_modules(h, conv2, ssm2)
+    _close(out, want, (conv, conv2), (ssm, ssm2))
+
+
 @pytest.mark.parametrize("cls,build", MIXERS[:1] + MIXERS[3:])
 def test_changed_modules_are_seen(dev, cls, build):
     m, g = build(cls, dev, seed=5)

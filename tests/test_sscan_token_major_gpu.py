@@ -20,7 +20,7 @@ def _inputs(dev, batch, dim, seqlen, seed):
     return d, s
 
 
-def _token_major(d, s, state_dtype, with_z, workspace_bytes):
+def _token_major(d, s, state_dtype, with_z, workspace_bytes, lanes=None):
     batch, L, dim = d["u"].shape
     out = torch.empty((batch, L, dim), dtype=torch.float16, device=d["u"].device)
     state = torch.empty((batch, dim, 16), dtype=state_dtype, device=out.device)
@@ -42,26 +42,28 @@ def _token_major(d, s, state_dtype, with_z, workspace_bytes):
     p.out = out.data_ptr()
     setattr(p, "last_state_i8" if state_dtype == torch.int8 else "last_state_f32", state.data_ptr())
     p.workspace, p.workspace_bytes = ws.data_ptr(), workspace_bytes
+    p.mapping = 0 if lanes is None else 0x40000000 | lanes << 20
     _lib.check(_lib.lib().qa_sscan_fwd(C.byref(p), _lib.current_stream(out.device)), "sscan_fwd")
     return out, state
 
 
 @pytest.mark.parametrize("batch,dim,seqlen,dtype,with_z,ws", [
-    (1, 64, 1, torch.int8, True, 0), (2, 36, 31, torch.float32, True, 0), (3, 1036, 33, torch.int8, False, 0),      # eight lanes
+    (1, 64, 1, torch.int8, True, 0), (2, 36, 31, torch.float32, True, 0), (3, 1036, 33, torch.int8, False, 0),      # few channels
     (40, 1024, 40, torch.float32, True, 0), (40, 1024, 65, torch.int8, False, 0),                                   # two kinds of workgroup
     (48, 1024, 37, torch.float32, True, 0), (48, 1028, 64, torch.int8, False, 0),                                   # four lanes
     (1, 512, 256, torch.float32, True, 1 << 22), (2, 1540, 515, torch.int8, True, 1 << 22), (1, 96, 2049, torch.float32, False, 1 << 22)])
 def test_token_major(dev, batch, dim, seqlen, dtype, with_z, ws):
     d, s = _inputs(dev, batch, dim, seqlen, seed=dim + seqlen)
-    out, state = _token_major(d, s, dtype, with_z, ws)
     rows = lambda a: a.transpose(1, 2).contiguous()
     B, Cm = rows(d["bc"][:, :, 8:24])[:, None], rows(d["bc"][:, :, 24:40])[:, None]
     want, st = ops.sscan_fwd(rows(d["u"]), s["u"], rows(d["dt"]), s["dt"], d["A"], s["A"], B, s["B"], Cm, s["C"], s["st"], d["D"], s["D"],
                              rows(d["z"]) if with_z else None, s["z"] if with_z else None, d["db"], s["db"], True, state_dtype=dtype)
-    diff = (out.float() - want.float()).abs()
-    assert bool((diff <= 1e-3 + 2e-3 * want.float().abs()).all())
-    a, b = state.float(), st[:, :, 0].float()
-    if dtype == torch.int8:
-        assert float((a - b).abs().max()) <= 1
-    else:
-        assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max())
+    for lanes in (None,) if ws else (None, 4, 8, 16):
+        out, state = _token_major(d, s, dtype, with_z, ws, lanes)
+        diff = (out.float() - want.float()).abs()
+        assert bool((diff <= 1e-3 + 2e-3 * want.float().abs()).all())
+        a, b = state.float(), st[:, :, 0].float()
+        if dtype == torch.int8:
+            assert float((a - b).abs().max()) <= 1
+        else:
+            assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max())
