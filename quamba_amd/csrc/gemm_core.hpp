@@ -136,20 +136,22 @@ __device__ __forceinline__ v4i make_rsrc(const void* base, int num_bytes) {
 }
 
 // 16 bytes per lane from buffer offset `voff` straight into LDS at lds_addr + lane*16 (lds_addr is
-// wave-uniform); lanes whose offset is outside the buffer deliver zeros.  Written as assembly so
+// wave-uniform; `soff`, also uniform, is added to the offset); lanes whose offset is outside the buffer deliver zeros.  Written as assembly so
 // that the vector-memory counter stays under this kernel's control: a tile's loads stay in flight
 // during the arithmetic and are waited for with an explicit s_waitcnt just before the barrier.
-__device__ __forceinline__ void buffer_load_lds_b128(v4i rsrc, uint32_t lds_addr, int voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+__device__ __forceinline__ void buffer_load_lds_b128(v4i rsrc, uint32_t lds_addr, int voff, int soff = 0) {
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
-                 : "s"(lds_addr), "v"(voff), "s"(rsrc)
+                 : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
                  : "memory");
 }
 
-__device__ __forceinline__ uint4 buffer_load_b128(v4i rsrc, int voff) {
-    uint4 v;
-    asm volatile("buffer_load_dwordx4 %0, %1, %2, 0 offen" : "=v"(v) : "v"(voff), "s"(rsrc) : "memory");
-    return v;
+// The same with 4 bytes per lane.
+__device__ __forceinline__ void buffer_load_lds_b32(v4i rsrc, uint32_t lds_addr, int voff) {
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(voff), "s"(rsrc)
+                 : "memory");
 }
 
 __device__ __forceinline__ uint32_t lds_offset_of(const void* p) {
@@ -187,48 +189,6 @@ struct TileLoader {
     }
 };
 
-// Accumulates one 128-byte k tile with the instruction order pinned: sa / sw point at this wave's rows of the
-// staged operands.  The fragments of step kk+1 are requested
-// before the multiplications of step kk are issued, and `hook(slot)` runs after every second
-// multiplication (slot = 0 .. 4*TM*TN/2 - 1): the caller places its global -> LDS requests for the
-// next tile there, one at a time, so that the wave never waits on a full memory queue with
-// multiplications behind it in program order.  sched_barrier keeps the compiler from regrouping.
-template <int TM, int TN, class Hook>
-__device__ __forceinline__ void mma_tile_paced(const uint8_t* sa, const uint8_t* sw, int frow, int fhalf,
-                                               v16i (&acc)[TN][TM], Hook&& hook) {
-    v4i fa[2][TM], fw[2][TN];
-    auto fetch = [&](int kk, int buf) {
-#pragma unroll
-        for (int i = 0; i < TN; ++i) {
-            const int row = i * 32 + frow;
-            fw[buf][i] = *reinterpret_cast<const v4i*>(sw + row * kBK + swz(row, kk * 2 + fhalf) * 16);
-        }
-#pragma unroll
-        for (int j = 0; j < TM; ++j) {
-            const int row = j * 32 + frow;
-            fa[buf][j] = *reinterpret_cast<const v4i*>(sa + row * kBK + swz(row, kk * 2 + fhalf) * 16);
-        }
-    };
-    fetch(0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int kk = 0; kk < kBK / 32; ++kk) {
-        if (kk + 1 < kBK / 32) fetch(kk + 1, (kk + 1) & 1);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < TN; ++i)
-#pragma unroll
-            for (int j = 0; j < TM; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[kk & 1][i], fa[kk & 1][j], acc[i][j], 0, 0, 0);
-                if (TM * TN == 1 || (i * TM + j) % 2 == 1) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    hook(TM * TN == 1 ? kk : kk * (TM * TN / 2) + (i * TM + j) / 2);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-    }
-}
-
 // The fragments of k step kk of this wave's rows (sa: TM row blocks of the a operand, sw: TN of the w operand).
 template <int TM, int TN>
 __device__ __forceinline__ void fetch_fragments(const uint8_t* sa, const uint8_t* sw, int kk, int frow, int fhalf,
@@ -242,6 +202,40 @@ __device__ __forceinline__ void fetch_fragments(const uint8_t* sa, const uint8_t
     for (int j = 0; j < TM; ++j) {
         const int row = j * 32 + frow;
         fa[j] = *reinterpret_cast<const v4i*>(sa + row * kBK + swz(row, kk * 2 + fhalf) * 16);
+    }
+}
+
+// Accumulates one 128-byte k tile with the instruction order pinned: sa / sw point at this wave's rows of the
+// staged operands.  The fragments of step kk+1 are requested
+// before the multiplications of step kk are issued, and `hook(slot)` runs after every second
+// multiplication (slot = 0 .. 4*TM*TN/2 - 1): the caller places its global -> LDS requests for the
+// next tile there, one at a time, so that the wave never waits on a full memory queue with
+// multiplications behind it in program order.  sched_barrier keeps the compiler from regrouping.
+template <int TM, int TN, class Hook>
+__device__ __forceinline__ void mma_tile_paced(const uint8_t* sa, const uint8_t* sw, int frow, int fhalf,
+                                               v16i (&acc)[TN][TM], Hook&& hook) {
+    // (a lone multiplication per step does not cover the time its fragments take: all four steps' are fetched at once)
+    constexpr int kAhead = TM * TN == 1 ? 3 : 1, kBufs = TM * TN == 1 ? 4 : 2;
+    v4i fa[kBufs][TM], fw[kBufs][TN];
+    auto fetch = [&](int kk) { fetch_fragments<TM, TN>(sa, sw, kk, frow, fhalf, fa[kk % kBufs], fw[kk % kBufs]); };
+#pragma unroll
+    for (int kk = 0; kk < kAhead; ++kk) fetch(kk);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk < kBK / 32; ++kk) {
+        if (kk + kAhead < kBK / 32) fetch(kk + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j) {
+                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[kk % kBufs][i], fa[kk % kBufs][j], acc[i][j], 0, 0, 0);
+                if (TM * TN == 1 || (i * TM + j) % 2 == 1) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    hook(TM * TN == 1 ? kk : kk * (TM * TN / 2) + (i * TM + j) / 2);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
     }
 }
 

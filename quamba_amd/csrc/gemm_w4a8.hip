@@ -10,27 +10,47 @@
 // Weight storage (this library's own): uint8 (N, K/2).  Each aligned group of 8 codes of a row is
 // one 32-bit word whose byte i holds code[8w+i] in the low nibble and code[8w+4+i] in the high
 // nibble, so that the fp16 exponent trick below yields the int8 bytes in k order.
-// The expansion to int8 runs in registers on the way from global memory to LDS (once per
-// workgroup, not once per wave): (word & 0x000f000f) | 0x6400_6400 is the half2 (1024+c0, 1024+c2);
-// subtracting 1032 gives c-8 exactly; one packed FMA with the group scale and the constant 1280
-// leaves rne((c-8)*s) as a two's-complement byte in the low byte of each half; v_perm gathers four
-// of them.  Everything else is the shared core in gemm_core.hpp.
+// The expansion to int8 is arithmetic in registers: (word & 0x000f000f) | 0x6400_6400 is the half2 (1024+c0, 1024+c2);
+// subtracting 1032 gives c-8 exactly; one packed FMA with the group scale and the constant 1280 leaves rne((c-8)*s) as a
+// two's-complement byte in the low byte of each half; v_perm gathers four of them: fifteen vector instructions for eight
+// codes and lane, four to five cycles each, where a product of 32 x 32 x 32 takes 32 cycles of the matrix cores.  How often
+// a code is expanded - once per row block of the output - and on how many of the chip's SIMDs at once is what the kernels
+// below trade: every one of them is bound by it from about a hundred activation rows on.
 #include "gemm_core.hpp"
 #include "gemv.hpp"
 #include "w4_expand.hpp"
+
+#include <algorithm>
+#include <cmath>
 
 namespace qa {
 namespace {
 
 using namespace gemm;
 
-template <int TM, int TN, int WGM, int WGN, int OUT, bool TRANS>
-__global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Params p) {
-    constexpr int STAGES = 2;
+// The tile kernel.  Everything that comes from memory goes straight to LDS, STAGES - 1 tiles ahead and counted by hand: the
+// activations as the fragments want them, the packed weights and their group scales as each thread's own 16 bytes and word
+// (no other lane reads those: they are registers that a load in flight does not occupy).  During the multiplications of tile
+// t a thread expands its codes of tile t + 1, a word behind every multiplication or two, into the one of two int8 weight
+// tiles that is not being read: the vector units work in the shadow of the matrix cores.  (Behind all multiplications of a
+// tile instead, with a tile's loads issued one tile ahead, a 64 x 64 tile on a CU of its own took 0.67 us per 128 of K; now
+// 0.38, of which the expansion is 0.15 and the LDS traffic of fragments, codes and tiles about as much.)
+template <int TM, int TN, int WGM, int WGN, int STAGES>
+struct W4Cfg {
     using C = Cfg<TM, TN, WGM, WGN, STAGES>;
-    constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves, THREADS = C::kThreads;
-    constexpr int kWPacked = BN * 4 / THREADS;      // 16-byte packed chunks (32 codes) per thread per tile
-    static_assert(epilogue_lds_bytes<TM, TN, WAVES>() <= C::kLdsBytes, "epilogue staging does not fit");
+    static constexpr int kWPacked = C::kBN * 4 / C::kThreads;      // 16-byte packed chunks (32 codes) per thread per tile
+    static constexpr int kSlots = STAGES - 1;                      // tiles of packed weights
+    static constexpr int kABytes = C::kBM * kBK, kWBytes = C::kBN * kBK;
+    static constexpr int kPackedBytes = C::kBN * (kBK / 2), kScaleBytes = kWPacked * C::kThreads * 4;
+    static constexpr int kLdsBytes = STAGES * kABytes + 2 * kWBytes + kSlots * (kPackedBytes + kScaleBytes);
+};
+
+template <int TM, int TN, int WGM, int WGN, int STAGES, bool GROUPED, int OUT>
+__global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Params p) {
+    using W = W4Cfg<TM, TN, WGM, WGN, STAGES>;
+    using C = typename W::C;
+    constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves, THREADS = C::kThreads, kWPacked = W::kWPacked;
+    static_assert(kWPacked * THREADS == BN * 4 && epilogue_lds_bytes<TM, TN, WAVES>() <= W::kLdsBytes, "tile shape");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
     const int tid = threadIdx.x;
@@ -41,54 +61,68 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
     int tile_m, tile_n;
     tile_of_workgroup<BM, BN>(blockIdx.x, tiles_m, tiles_n, tile_m, tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
-    const bool grouped = p.group_size > 0;
+    const int k_tiles = p.k / kBK, ldw = p.k / 2;
 
-    const v4i rsrc_a = make_rsrc(p.a, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k));
     const uint32_t lds_base = lds_offset_of(lds);
+    constexpr int kAtW = STAGES * W::kABytes, kAtPacked = kAtW + 2 * W::kWBytes, kAtScale = kAtPacked + W::kSlots * W::kPackedBytes;
+    const v4i rsrc_a = make_rsrc(p.a, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k));
+    const v4i rsrc_w = make_rsrc(p.w_packed + static_cast<int64_t>(n0) * ldw, min(BN, p.n - n0) * ldw);
+    // group scales are fetched as aligned words of two; `s_first` is the first scale's place in the first word
+    const uintptr_t s_addr = reinterpret_cast<uintptr_t>(p.s_group);
+    const int s_first = static_cast<int>((s_addr >> 1) & 1);
+    v4i rsrc_s = {};
+    if constexpr (GROUPED) rsrc_s = make_rsrc(reinterpret_cast<const void*>(s_addr & ~uintptr_t{3}), static_cast<int>((static_cast<int64_t>(k_tiles) * p.n + s_first + 1) / 2 * 4));
+    // (K is whole tiles: a tile is an offset the whole wave shares.  Requests past the last tile repeat it.)
     TileLoader<C::kAInstr> load_a;
     load_a.template init<WAVES>(m0, p.m, p.lda, wave, lane);
+    const int last = k_tiles - 1;
+    auto issue_a = [&](int r, int tile, int stage) {
+        buffer_load_lds_b128(rsrc_a, lds_base + stage * W::kABytes + (r * WAVES + wave) * 1024, load_a.voff[r], min(tile, last) * kBK);
+    };
 
-    // this thread's packed chunks of the weight tile: (row, 32-code quarter)
-    const int64_t ldw = p.k / 2;
-    const uint8_t* w_src[kWPacked];
-    int w_row[kWPacked], w_quarter[kWPacked];
+    // this thread's packed chunks of the weight tile: row id / 4, codes 32 (id % 4) .. + 31
+    int w_off[kWPacked], s_col[kWPacked];
+    uint32_t s_pick[kWPacked];                             // the half of the fetched word, twice
+    uint8_t* to_w[kWPacked][2];
 #pragma unroll
     for (int i = 0; i < kWPacked; ++i) {
-        const int id = tid + i * THREADS;
-        w_row[i] = id >> 2;
-        w_quarter[i] = id & 3;
-        const int nn = min(n0 + w_row[i], p.n - 1);
-        w_src[i] = p.w_packed + nn * ldw + w_quarter[i] * 16;
+        const int id = tid + i * THREADS, row = id >> 2, quarter = id & 3;
+        w_off[i] = row * ldw + quarter * 16;
+        s_col[i] = s_first + min(n0 + row, p.n - 1);
+        s_pick[i] = 0x01000100u + (s_col[i] & 1) * 0x02020202u;
+        to_w[i][0] = lds + kAtW + row * kBK + swz(row, 2 * quarter) * 16;
+        to_w[i][1] = lds + kAtW + row * kBK + swz(row, 2 * quarter + 1) * 16;
     }
-    const __half* sg = static_cast<const __half*>(p.s_group);
-
-    uint4 wreg[kWPacked];
-    __half wscale[kWPacked];
-    auto load_w = [&](int tile) {
+    const uint32_t s_flip = p.n & 1 ? 0x02020202u : 0u;
+    auto issue_w = [&](int tile, int slot) {
+        const int t = min(tile, last);
 #pragma unroll
         for (int i = 0; i < kWPacked; ++i) {
-            wreg[i] = *reinterpret_cast<const uint4*>(w_src[i] + static_cast<int64_t>(tile) * (kBK / 2));
-            if (grouped) wscale[i] = sg[static_cast<int64_t>(tile) * p.n + min(n0 + w_row[i], p.n - 1)];
+            buffer_load_lds_b128(rsrc_w, lds_base + kAtPacked + slot * W::kPackedBytes + (i * WAVES + wave) * 1024, w_off[i], t * (kBK / 2));
+            if constexpr (GROUPED) buffer_load_lds_b32(rsrc_s, lds_base + kAtScale + slot * W::kScaleBytes + (i * WAVES + wave) * 256, ((s_col[i] + t * p.n) << 1) & ~3);
         }
     };
-    auto store_w = [&](int stage) {
-        uint8_t* sw = lds + stage * C::kStageBytes + BM * kBK;
+    uint4 wreg[kWPacked];
+    __half2 s2[kWPacked];
+    auto fetch_w = [&](int slot) {                         // tile after tile
 #pragma unroll
         for (int i = 0; i < kWPacked; ++i) {
-            const uint32_t w[4] = {wreg[i].x, wreg[i].y, wreg[i].z, wreg[i].w};
-            uint2 e[4];
-            if (grouped) {
-                const __half2 s2 = __half2half2(wscale[i]);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) e[t] = expand_grouped(w[t], s2);
-            } else {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) e[t] = expand_per_channel(w[t]);
+            wreg[i] = *reinterpret_cast<const uint4*>(lds + kAtPacked + slot * W::kPackedBytes + (i * THREADS + tid) * 16);
+            if constexpr (GROUPED) {
+                const uint32_t word = *reinterpret_cast<const uint32_t*>(lds + kAtScale + slot * W::kScaleBytes + (i * THREADS + tid) * 4);
+                s2[i] = bits_h2(__builtin_amdgcn_perm(word, word, s_pick[i]));
+                s_pick[i] ^= s_flip;
             }
-            const int row = w_row[i], c0 = w_quarter[i] * 2;
-            *reinterpret_cast<uint4*>(sw + row * kBK + swz(row, c0) * 16) = make_uint4(e[0].x, e[0].y, e[1].x, e[1].y);
-            *reinterpret_cast<uint4*>(sw + row * kBK + swz(row, c0 + 1) * 16) = make_uint4(e[2].x, e[2].y, e[3].x, e[3].y);
         }
+    };
+    // word `w` of this thread's kWPacked * 4 (a pair is written when its second one is done)
+    uint2 done;
+    auto expand_w = [&](int w, int to) {
+        const int i = w / 4, t = w % 4;
+        const uint32_t packed = t == 0 ? wreg[i].x : t == 1 ? wreg[i].y : t == 2 ? wreg[i].z : wreg[i].w;
+        const uint2 e = GROUPED ? expand_grouped(packed, s2[i]) : expand_per_channel(packed);
+        if (t % 2 == 0) done = e;
+        else *reinterpret_cast<uint4*>(to_w[i][t / 2] + to * W::kWBytes) = make_uint4(done.x, done.y, e.x, e.y);
     };
 
     v16i acc[TN][TM];
@@ -99,29 +133,51 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
-    const int k_tiles = p.k / kBK;
-    load_a.template issue<WAVES>(rsrc_a, 0, p.k, lds_base, wave);
     if (k_tiles > 0) {
-        load_w(0);
-        store_w(0);
-    }
-    const int frow = lane & 31, fhalf = lane >> 5;
-    for (int kt = 0; kt < k_tiles; ++kt) {
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        __syncthreads();
-        const bool more = kt + 1 < k_tiles;
-        if (more) load_w(kt + 1);
-        const uint8_t* stage = lds + (kt & 1) * C::kStageBytes;
-        // the activation requests for the next tile go out one at a time between the multiplications
-        const uint32_t nbase = lds_base + ((kt + 1) & 1) * C::kStageBytes;
-        constexpr int kSlots = TM * TN == 1 ? 4 : 4 * (TM * TN / 2), kPerSlot = (C::kAInstr + kSlots - 1) / kSlots;
-        mma_tile_paced<TM, TN>(stage + (wm * TM * 32) * kBK, stage + BM * kBK + (wn * TN * 32) * kBK, frow, fhalf, acc,
-                               [&](int slot) {
+        // Requests go out in the order W(0) A(0) W(1) A(1) ..., the first tile's weights being expanded before the loop
+        issue_w(0, 0);
 #pragma unroll
-                                   for (int r = slot * kPerSlot; r < (slot + 1) * kPerSlot; ++r)
-                                       if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, (kt + 1) * kBK, p.k, nbase, wave);
-                               });
-        if (more) store_w((kt + 1) & 1);
+        for (int s = 0; s < STAGES - 1; ++s) {
+#pragma unroll
+            for (int r = 0; r < C::kAInstr; ++r) issue_a(r, s, s);
+            if (s + 1 < STAGES - 1) issue_w(s + 1, s + 1);
+        }
+        constexpr int kLoads = C::kAInstr + (GROUPED ? 2 : 1) * kWPacked;      // requests of a wave per tile
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 2) * kLoads + C::kAInstr));
+        wave_lds_sync();
+        fetch_w(0);
+#pragma unroll
+        for (int w = 0; w < 4 * kWPacked; ++w) expand_w(w, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        issue_w(STAGES - 1, 0);
+        const int frow = lane & 31, fhalf = lane >> 5;
+        static_assert(STAGES == 2 || STAGES == 3, "the unrolled tiles have to cover whole turns of stages, slots and weight tiles");
+        constexpr int kUnroll = STAGES == 2 ? 2 : 6;
+        for (int base = 0; base < k_tiles; base += kUnroll) {
+            static_for<0, kUnroll>([&](auto u_c) {
+                constexpr int u = decltype(u_c)::value;
+                const int kt = base + u;
+                if (kt >= k_tiles) return;
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 2) * kLoads));   // A(kt) and W(kt + 1) are here
+                __syncthreads();
+                fetch_w((u + 1) % W::kSlots);
+                __builtin_amdgcn_sched_barrier(0);
+                constexpr int kSteps = TM * TN == 1 ? 4 : 4 * (TM * TN / 2), kPerStep = (C::kAInstr + kSteps - 1) / kSteps;
+                constexpr int kWords = (4 * kWPacked + kSteps - 1) / kSteps;
+                mma_tile_paced<TM, TN>(lds + (u % STAGES) * W::kABytes + (wm * TM * 32) * kBK, lds + kAtW + (u % 2) * W::kWBytes + (wn * TN * 32) * kBK, frow, fhalf, acc,
+                                       [&](int step) {
+                                           // (the fragments of the multiplication before this were read after fetch_w's
+                                           // words, so these are in their registers and the slot they came from is free)
+                                           if (step == 0) issue_w(kt + STAGES, (u + STAGES) % W::kSlots);
+#pragma unroll
+                                           for (int r = step * kPerStep; r < (step + 1) * kPerStep; ++r)
+                                               if (r < C::kAInstr) issue_a(r, kt + STAGES - 1, (u + STAGES - 1) % STAGES);
+#pragma unroll
+                                           for (int w = step * kWords; w < (step + 1) * kWords; ++w)
+                                               if (w < 4 * kWPacked) expand_w(w, (u + 1) % 2);
+                                       });
+            });
+        }
     }
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     __syncthreads();
@@ -131,37 +187,199 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
     e.row_numel = p.tok_scale_numel; e.col_numel = p.n;
     e.use_alpha = 0; e.alpha = 0.0f; e.round_mode = QA_ROUND_RNE; e.col_outer = 0;
     e.ldd = p.ldd; e.d = p.d;
-    epilogue<TM, TN, OUT, false, TRANS>(e, acc, lds, p.m, p.n, m0 + wm * TM * 32, n0 + wn * TN * 32, wave, lane);
+    epilogue<TM, TN, OUT, false, false>(e, acc, lds, p.m, p.n, m0 + wm * TM * 32, n0 + wn * TN * 32, wave, lane);
 }
 
-template <int TM, int TN, int WGM, int WGN, int OUT, bool TRANS>
-int launch_one(const QaGemmW4A8Params& p, hipStream_t stream) {
-    using C = Cfg<TM, TN, WGM, WGN, 2>;
+template <int OUT>
+int launch_tile(const QaGemmW4A8Params& p, hipStream_t stream) {
+    constexpr int TM = 1, TN = 1, WGM = 2, WGN = 2, STAGES = 3;
+    using W = W4Cfg<TM, TN, WGM, WGN, STAGES>;
+    using C = typename W::C;
     const int64_t tiles = static_cast<int64_t>((p.m + C::kBM - 1) / C::kBM) * ((p.n + C::kBN - 1) / C::kBN);
-    if (tiles > 0x7fffffffLL) return QA_ERR_SHAPE;
-    auto kernel = gemm_w4a8_kernel<TM, TN, WGM, WGN, OUT, TRANS>;
-    if (C::kLdsBytes > 65536) {
+    if (tiles > 0x7fffffffLL || static_cast<int64_t>(C::kBN) * p.k > 0x7fffffffLL || static_cast<int64_t>(p.n) * p.k > 64LL * 0x7fffff00LL) return QA_ERR_SHAPE;
+    auto kernel = p.group_size > 0 ? gemm_w4a8_kernel<TM, TN, WGM, WGN, STAGES, true, OUT> : gemm_w4a8_kernel<TM, TN, WGM, WGN, STAGES, false, OUT>;
+    if (W::kLdsBytes > 65536) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                C::kLdsBytes) != hipSuccess) {
+                                W::kLdsBytes) != hipSuccess) {
             return check_launch();
         }
     }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(C::kThreads), C::kLdsBytes, stream, p);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(C::kThreads), W::kLdsBytes, stream, p);
     return check_launch();
 }
 
-template <int TM, int TN, int WGM, int WGN>
-int launch_gemm(const QaGemmW4A8Params& p, hipStream_t stream) {
-    if (p.out_type == QA_OUT_I8) {
-        return p.output_transpose ? launch_one<TM, TN, WGM, WGN, QA_OUT_I8, true>(p, stream)
-                                  : launch_one<TM, TN, WGM, WGN, QA_OUT_I8, false>(p, stream);
+// ---------------------------------------------------------------------------------------------
+// Weights that never pass through LDS.  A wave owns 32 output columns and all BM = 32 TM rows of the tile; the packed codes
+// go from memory into the registers of the lane whose fragment they become, and are expanded there between the
+// multiplications.  A tile of K is KT codes (KT / 2 for either half of the lanes, which is 32 or 64 consecutive bytes of a
+// packed row - the order of K inside a tile is free as long as both operands agree); weights are requested two tiles ahead
+// (registers in three sets), activations one, straight to LDS.  The four waves share the activations.  No code is expanded
+// twice in a tile and none costs LDS bandwidth, so this goes further than the tile kernel above: 777 x 6144 x 1536 in 192
+// rows takes 16.0 us, in 64 x 64 tiles 20.9 and did 22.8 in the 128 x 128 tiles it replaces.
+// ---------------------------------------------------------------------------------------------
+template <int TM, int NW, int KT>
+struct RegCfg {
+    static constexpr int kThreads = 64 * NW;
+    static constexpr int kBM = 32 * TM, kBN = 32 * NW;
+    static constexpr int kRowChunks = KT / 16;
+    static constexpr int kABytes = kBM * KT;
+    static constexpr int kAInstr = kABytes / 1024 / NW;            // direct-to-LDS requests of a wave per tile
+    static constexpr int kWLoads = KT / 64;                        // 16-byte pieces of packed weights per lane and tile
+    static constexpr int kEpilogue = epilogue_lds_bytes<TM, 1, NW>();
+    static constexpr int kLdsBytes = 2 * kABytes > kEpilogue ? 2 * kABytes : kEpilogue;
+};
+
+template <int TM, int NW, int KT, bool GROUPED, int OUT, bool TRANS>
+__global__ __launch_bounds__(64 * NW) void gemm_w4a8_reg_kernel(QaGemmW4A8Params p) {
+    using R = RegCfg<TM, NW, KT>;
+    static_assert(R::kAInstr * NW * 1024 == R::kABytes && (KT == 128 || KT == 256), "tile shape");
+    constexpr int kOob = 0x7ffffff0;                               // beyond any buffer: the load returns zeros
+    constexpr int kSteps = KT / 32, kSets = 3, kLoads = R::kWLoads + (GROUPED ? 1 : 0);
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int frow = lane & 31, fhalf = lane >> 5;
+    const int tiles_m = (p.m + R::kBM - 1) / R::kBM, tiles_n = (p.n + R::kBN - 1) / R::kBN;
+    int tile_m, tile_n;
+    tile_of_workgroup<R::kBM, R::kBN>(blockIdx.x, tiles_m, tiles_n, tile_m, tile_n);
+    const int m0 = tile_m * R::kBM, n0 = tile_n * R::kBN + wave * 32;
+    const int ldw = p.k / 2, k_tiles = (p.k + KT - 1) / KT;
+
+    // activations: request j of a wave fills LDS bytes [(j NW + wave) 1024, + 1024) of the tile, i.e. 1024 / KT rows; the
+    // 16-byte pieces of a row are exchanged by the row's low bits, so that a column of pieces covers all banks
+    const v4i rsrc_a = make_rsrc(p.a, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k));
+    const uint32_t lds_a = lds_offset_of(lds);
+    int a_off[R::kAInstr], a_k[R::kAInstr];
+#pragma unroll
+    for (int j = 0; j < R::kAInstr; ++j) {
+        const int piece = (j * NW + wave) * 64 + lane, row = piece / R::kRowChunks, c = (piece % R::kRowChunks) ^ (row % R::kRowChunks);
+        a_k[j] = c * 16;
+        a_off[j] = m0 + row < p.m ? static_cast<int>((m0 + row) * p.lda) + c * 16 : 0x70000000;
     }
-    return p.output_transpose ? launch_one<TM, TN, WGM, WGN, QA_OUT_F16, true>(p, stream)
-                              : launch_one<TM, TN, WGM, WGN, QA_OUT_F16, false>(p, stream);
+    auto issue_a = [&](int tile, int stage) {
+        const int k0 = min(tile, k_tiles - 1) * KT;                                  // (past the last tile: that one again)
+#pragma unroll
+        for (int j = 0; j < R::kAInstr; ++j) {
+            const int off = KT == 128 || k0 + a_k[j] < p.k ? a_off[j] : kOob;        // (K is a multiple of 128)
+            buffer_load_lds_b128(rsrc_a, lds_a + stage * R::kABytes + (j * NW + wave) * 1024, off, k0);
+        }
+    };
+
+    // weights: this lane's row, its half of the tile's codes
+    const int rows_left = p.n - n0;
+    const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.w_packed) + static_cast<int64_t>(n0) * ldw, 0,
+                                                                           rows_left > 0 ? min(32, rows_left) * ldw : 0, kRsrcFlags);
+    const __half* sg = GROUPED ? static_cast<const __half*>(p.s_group) + min(n0 + frow, p.n - 1) : nullptr;
+    v4u fw[kSets][R::kWLoads];
+    uint16_t fs[kSets];
+    auto load_w = [&](int t, auto set_c) {
+        constexpr int set = decltype(set_c)::value;
+        const int tile = min(t, k_tiles - 1);
+#pragma unroll
+        for (int l = 0; l < R::kWLoads; ++l) fw[set][l] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, frow * ldw + fhalf * (KT / 4) + tile * (KT / 2) + 16 * l, 0, 0);
+        if constexpr (GROUPED) fs[set] = __half_as_ushort(sg[static_cast<int64_t>(min(KT == 256 ? 2 * tile + fhalf : tile, p.k / 128 - 1)) * p.n]);
+    };
+
+    v16i acc[1][TM];
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][j][r] = 0;
+
+    if (k_tiles > 0) {
+        load_w(0, std::integral_constant<int, 0>{});
+        __builtin_amdgcn_sched_barrier(0);
+        issue_a(0, 0);
+        load_w(1, std::integral_constant<int, 1>{});
+        for (int base = 0; base < k_tiles; base += 6) {
+            static_for<0, 6>([&](auto u_c) {
+                constexpr int u = decltype(u_c)::value, set = u % kSets, stage = u % 2;
+                const int tile = base + u;
+                if (tile >= k_tiles) return;
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(kLoads));     // this tile's activations (and weights) are here
+                __syncthreads();
+                const uint8_t* sa = lds + stage * R::kABytes;
+                v4i fa[2][TM], w8[2];
+                auto fetch = [&](int kk) {
+#pragma unroll
+                    for (int j = 0; j < TM; ++j) {
+                        const int row = j * 32 + frow, c = (fhalf * kSteps + kk) ^ (row % R::kRowChunks);
+                        fa[kk & 1][j] = *reinterpret_cast<const v4i*>(sa + row * KT + c * 16);
+                    }
+                };
+                __half2 s2;
+                auto expand = [&](int kk, int half) {
+                    const v4u piece = fw[set][kk / 2];
+                    const uint32_t word = piece[2 * (kk & 1) + half];
+                    const uint2 e = GROUPED ? expand_grouped(word, s2) : expand_per_channel(word);
+                    w8[kk & 1][2 * half] = static_cast<int>(e.x);
+                    w8[kk & 1][2 * half + 1] = static_cast<int>(e.y);
+                };
+                fetch(0);
+                if constexpr (GROUPED) s2 = bits_h2(static_cast<uint32_t>(fs[set]) * 0x10001u);
+#pragma unroll
+                for (int l = 0; l < R::kWLoads; ++l) asm volatile("" : "+v"(fw[set][l]));      // (all of the set is waited for here)
+                expand(0, 0);
+                expand(0, 1);
+                __builtin_amdgcn_sched_barrier(0);
+                // activations before weights: the wait for the next tile's weights then never includes the tile after it
+                issue_a(tile + 1, stage ^ 1);
+                load_w(tile + 2, std::integral_constant<int, (u + 2) % kSets>{});
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int kk = 0; kk < kSteps; ++kk) {
+                    if (kk + 1 < kSteps) fetch(kk + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int x = 0; x < TM; ++x) {
+                        acc[0][x] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w8[kk & 1], fa[kk & 1][x], acc[0][x], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (kk + 1 < kSteps) {
+#pragma unroll
+                            for (int w = x * 2 / TM; w < (x + 1) * 2 / TM; ++w) expand(kk + 1, w);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            });
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    __syncthreads();
+
+    Epilogue e;
+    e.row_scale = p.s_token; e.col_scale = p.s_channel;
+    e.row_numel = p.tok_scale_numel; e.col_numel = p.n;
+    e.use_alpha = 0; e.alpha = 0.0f; e.round_mode = QA_ROUND_RNE; e.col_outer = 0;
+    e.ldd = p.ldd; e.d = p.d;
+    epilogue<TM, 1, OUT, false, TRANS>(e, acc, lds, p.m, p.n, m0, n0, wave, lane);
+}
+
+template <int TM, int NW, int KT, int OUT, bool TRANS>
+int launch_reg_one(const QaGemmW4A8Params& p, hipStream_t stream) {
+    using R = RegCfg<TM, NW, KT>;
+    const int64_t tiles = static_cast<int64_t>((p.m + R::kBM - 1) / R::kBM) * ((p.n + R::kBN - 1) / R::kBN);
+    if (tiles > 0x7fffffffLL || 16LL * p.k > 0x7fffffffLL) return QA_ERR_SHAPE;
+    auto kernel = p.group_size > 0 ? gemm_w4a8_reg_kernel<TM, NW, KT, true, OUT, TRANS> : gemm_w4a8_reg_kernel<TM, NW, KT, false, OUT, TRANS>;
+    if (R::kLdsBytes > 65536) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                R::kLdsBytes) != hipSuccess) {
+            return check_launch();
+        }
+    }
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(R::kThreads), R::kLdsBytes, stream, p);
+    return check_launch();
+}
+
+template <int TM, int NW, int KT>
+int launch_reg(const QaGemmW4A8Params& p, hipStream_t stream) {
+    return p.out_type == QA_OUT_I8 ? launch_reg_one<TM, NW, KT, QA_OUT_I8, false>(p, stream) : launch_reg_one<TM, NW, KT, QA_OUT_F16, false>(p, stream);
 }
 
 // ---------------------------------------------------------------------------------------------
-// Few activation rows (M <= 64, the decode step): a stream over the packed weights.  A workgroup
+// Few activation rows or few columns: a stream over the packed weights.  A workgroup
 // owns 32 output columns and all rows; its WAVES waves split K between them in interleaved pieces
 // of 256 codes, i.e. one full 128-byte line of packed weights per row.  A wave fetches a piece with
 // eight lanes per row (DEPTH pieces in flight in registers), expands its 32 codes per lane to int8
@@ -337,10 +555,12 @@ int launch_skinny(const QaGemmW4A8Params& p, hipStream_t stream) {
 
 int64_t tiles_of(const QaGemmW4A8Params& p, int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); }
 
+// eight waves share K when there is at most a workgroup per CU and K is long, else four (4096 x 8192 at 64 rows: 13.8
+// against 15.8 us; 18560 x 4096 at 16 rows: 23.0 against 19.1)
+bool skinny_is_wide(const QaGemmW4A8Params& p) { return tiles_of(p, 32, 32) <= 256 && p.k >= 2048; }
+
 int dispatch_skinny(const QaGemmW4A8Params& p, hipStream_t stream) {
-    // eight waves share K when there is at most a workgroup per CU and K is long, else four (4096 x 8192 at 64 rows: 13.8
-    // against 15.8 us; 18560 x 4096 at 16 rows: 23.0 against 19.1)
-    const bool wide = tiles_of(p, 32, 32) <= 256 && p.k >= 2048;
+    const bool wide = skinny_is_wide(p);
     // activation rows are fetched eight at a time: up to 8 rows need one fetch per tile, up to 32 four
     if (p.m <= 8) return wide ? launch_skinny<1, 1, 8, 3>(p, stream) : launch_skinny<1, 1, 4, 3>(p, stream);
     return wide ? launch_skinny<1, 4, 8, 2>(p, stream) : launch_skinny<1, 4, 4, 2>(p, stream);
@@ -370,6 +590,37 @@ __global__ __launch_bounds__(256) void w4_expand_kernel(QaGemmW4A8Params p, int8
     int8_t* dst = w8 + static_cast<int64_t>(n) * p.k + piece * 32;
     *reinterpret_cast<uint4*>(dst) = make_uint4(e[0].x, e[0].y, e[1].x, e[1].y);
     *reinterpret_cast<uint4*>(dst + 16) = make_uint4(e[2].x, e[2].y, e[3].x, e[3].y);
+}
+
+// Which kernel a product without transposed output takes: the one whose cost, in microseconds as measured over 16 .. 4096
+// rows of 768 .. 18560 columns and K from 768 to 8192, is the least.  A launch goes in rounds of one workgroup per CU, and
+// r workgroups on the busiest CU take a fixed time and one that grows with r per 128 of K; the kernels differ in the size of
+// their tiles - large ones expand each code fewer times, small ones spread over the chip earlier - and the weights expanded
+// once, in a pass of their own, cost that pass.
+enum Way { kWaySkinny, kWay64x64, kWay64x128, kWay128x128, kWay192x128, kWayExpandOnce };
+
+int cheapest_way(const QaGemmW4A8Params& p, bool addressable, bool expandable) {
+    const double k_tiles = p.k / 128, kCus = 256;
+    auto rounds = [&](int64_t bm, int64_t bn) { return std::ceil(static_cast<double>(tiles_of(p, bm, bn)) / kCus); };
+    double best = 1e30;
+    int way = kWay128x128;
+    auto offer = [&](int w, double cost) {
+        if (cost < best) { best = cost; way = w; }
+    };
+    if (addressable) {
+        const bool wide = skinny_is_wide(p);
+        offer(kWaySkinny, 3.0 + std::ceil(k_tiles / (wide ? 8 : 4)) * (wide ? 1.35 : 0.75 + 0.38 * rounds(32, 32)));
+    }
+    offer(kWay64x64, 3.0 + k_tiles * (0.10 + 0.28 * rounds(64, 64)));
+    offer(kWay64x128, 3.0 + k_tiles * (0.08 + 0.42 * rounds(64, 128)));
+    offer(kWay128x128, 3.0 + k_tiles * std::max(0.73, 0.10 + 0.57 * rounds(128, 128)));
+    offer(kWay192x128, 3.0 + k_tiles * (0.05 + 0.84 * rounds(192, 128)));
+    if (expandable) {
+        // (the int8 x int8 kernel takes the smallest tile that fits one round, see there)
+        const double step = rounds(64, 64) <= 1 ? 0.25 : rounds(128, 64) <= 1 ? 0.33 : rounds(128, 128) <= 1 ? 0.50 : rounds(128, 256) <= 1 ? 0.75 : 1.55 * rounds(256, 256);
+        offer(kWayExpandOnce, 2.5 + static_cast<double>(p.n) * p.k / 3.1e6 + 5.0 + step * k_tiles);
+    }
+    return way;
 }
 
 }  // namespace
@@ -403,20 +654,16 @@ extern "C" int qa_gemm_w4a8(const QaGemmW4A8Params* p, void* stream_) {
         return gemv_launch(g, nullptr, stream);
     }
     const bool addressable = static_cast<int64_t>(p->n) * (p->k / 2) < 0x70000000LL;
-    if (p->m <= 64 && addressable) return dispatch_skinny(*p, stream);
     const int64_t w8_bytes = static_cast<int64_t>(p->n) * p->k;
     const bool expandable = p->w8_workspace && p->w8_workspace_bytes >= w8_bytes && aligned16(p->w8_workspace) && w8_bytes < 0x70000000LL;
+    if (p->output_transpose ? p->m <= 64 && addressable : p->m <= kGemvRows && addressable) return dispatch_skinny(*p, stream);
     if (!p->output_transpose) {
-        // Between the kernel for few rows and the weights expanded once (a pass of its own: 2 us and 1.5 bytes a weight) lie
-        // the shapes in which expanding inside the product is the cheaper way, measured at 96 .. 1000 rows: 32 x 32 tiles
-        // with K split over the waves up to two a CU (192 x 5120: 8.3 us where 128 x 128 tiles took 38; 2560 x 5120 at 128
-        // rows 14.7, expanded once 23.6), then 64 x 64 tiles while they are few and the expansion's latency has either a
-        // short K or other tiles to hide behind (10240 x 2560 at 256 rows 23.4 against 26.1 us, 6144 x 1536 at 512 rows 14.2
-        // against 20.4), 128 x 128 tiles for the rest of the short K.
-        const int64_t t32 = tiles_of(*p, 32, 32), t64 = tiles_of(*p, 64, 64);
-        if (t32 <= 512 && addressable) return dispatch_skinny(*p, stream);
-        if (t64 <= 768 && (p->k <= 1536 || (t64 > 256 && p->k <= 4096))) return launch_gemm<1, 1, 2, 2>(*p, stream);
-        if (p->k <= 1536 && p->m < 1024) return launch_gemm<2, 2, 2, 2>(*p, stream);
+        const int way = cheapest_way(*p, addressable, expandable);
+        if (way == kWaySkinny) return dispatch_skinny(*p, stream);
+        if (way == kWay64x64) return p->out_type == QA_OUT_I8 ? launch_tile<QA_OUT_I8>(*p, stream) : launch_tile<QA_OUT_F16>(*p, stream);
+        if (way == kWay64x128) return launch_reg<2, 4, 256>(*p, stream);
+        if (way == kWay128x128) return launch_reg<4, 4, 128>(*p, stream);
+        if (way == kWay192x128) return launch_reg<6, 4, 128>(*p, stream);
     }
     if (expandable && (!p->output_transpose || p->n > 64)) {
         int8_t* w8 = static_cast<int8_t*>(p->w8_workspace);
@@ -445,7 +692,5 @@ extern "C" int qa_gemm_w4a8(const QaGemmW4A8Params* p, void* stream_) {
         }
         return qa_gemm_w8a8(&q, stream_);
     }
-    const int64_t big_tiles = static_cast<int64_t>((p->m + 255) / 256) * ((p->n + 255) / 256);
-    if (big_tiles >= 192) return launch_gemm<4, 2, 2, 4>(*p, stream);
-    return launch_gemm<2, 2, 2, 2>(*p, stream);
+    return p->out_type == QA_OUT_I8 ? launch_reg_one<4, 4, 128, QA_OUT_I8, true>(*p, stream) : launch_reg_one<4, 4, 128, QA_OUT_F16, true>(*p, stream);
 }

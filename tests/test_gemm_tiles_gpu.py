@@ -38,9 +38,10 @@ def test_int8_weights(dev, M, N, K, order):
     np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
-# 32 x 32 with four and eight waves, 64 x 64 and 128 x 128 expanding inside, 256 x 256, expanded once
-@pytest.mark.parametrize("M,N,K,workspace", [(70, 200, 2176, False), (100, 1000, 384, False), (600, 2100, 256, False), (300, 4200, 1664, False),
-                                             (900, 6100, 128, False), (4000, 3300, 1664, False), (500, 4200, 1664, True)])
+# 32 x 32 with four and eight waves, 64 x 64, 64 x 128, 128 x 128, 192 x 128, expanded once
+@pytest.mark.parametrize("M,N,K,workspace", [(70, 200, 2176, False), (100, 1000, 384, False), (130, 2050, 1664, False), (250, 2500, 1152, False),
+                                             (600, 2100, 256, False), (300, 4200, 1664, False), (70, 9000, 128, False), (700, 3100, 1152, False),
+                                             (900, 6100, 128, False), (950, 6100, 896, False), (4000, 3300, 1664, False), (4000, 3300, 1664, True)])
 def test_4_bit_weights(dev, M, N, K, workspace):
     g = np.random.default_rng(M + N + K)
     a, codes = g.integers(-128, 128, (M, K)).astype(np.int8), g.integers(0, 16, (N, K)).astype(np.uint8)
