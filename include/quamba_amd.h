@@ -179,8 +179,8 @@ int qa_hadamard_quant(const QaHadamardParams* p, void* stream);
  * `norm`: rows, dim, group_size, norm_before_gate, eps, z_scale, x, weight, qz and their strides as for
  * qa_rmsnorm_gated; out_mode must be QA_NORM_OUT_F16; out, out_row_stride, out_scale, dyn_scale unused.
  * `had`: rows, dim (equal to the norm's), scale, out, out_row_stride; x, x_row_stride, in_type unused.
- * Supported: dim 2048, 4096 or 8192 with group_size 512, 1024 or 2048, 16-byte aligned rows;
- * anything else returns QA_ERR_UNSUPPORTED (callers then make the two calls). */
+ * Supported: dim 2048, 4096 or 8192 with group_size 512, 1024 or 2048, and dim 1536, 3072, 5120 or 10240
+ * with group_size == dim; 16-byte aligned rows; anything else returns QA_ERR_UNSUPPORTED (callers then make the two calls). */
 int qa_rmsnorm_gated_hadamard_quant(const QaNormGatedParams* norm, const QaHadamardParams* had, void* stream);
 
 /* ------------------------------------------------------------------------------------------

@@ -199,10 +199,7 @@ struct Mamba2Buffers {
 
 int heads_of(const QaMamba2Params& p) { return p.d_inner / p.headdim; }
 
-bool norm_fuses(const QaMamba2Params& p) {
-    const int d = p.d_inner, g = p.norm_group_size;
-    return (d == 2048 || d == 4096 || d == 8192) && (g == 512 || g == 1024 || g == 2048) && d % g == 0;
-}
+bool norm_fuses(const QaMamba2Params& p) { return norm_hadamard_fuses(p.d_inner, p.norm_group_size); }
 
 QaSsdParams ssd_sizes(const QaMamba2Params& p) {
     QaSsdParams s = {};

@@ -5,6 +5,9 @@
 
 namespace qa {
 
+// hadamard.hip: whether qa_rmsnorm_gated_hadamard_quant takes rows of `dim` columns in norm groups of `group`
+bool norm_hadamard_fuses(int dim, int group);
+
 // sscan_tm.hip: qa_sscan_fwd for token-major inputs.  With `dt` the step size codes are not read but made in the scan:
 // dt_proj's product of x (x_proj's rows, x_l_stride apart) with w (d_inner rows of `rank` codes, a multiple of 16 up to 192),
 // scaled col * (row * acc) and rounded as the int8 product does it.  seqlen * x_l_stride below 2^30.
