@@ -221,7 +221,7 @@ Mamba2Buffers carve(const QaMamba2Params& p, void* base, bool step) {
     b.yn = c.take<__half>(norm_fuses(p) ? 0 : t * p.d_inner * 2);
     b.w8.bytes = std::max(expanded_bytes(p.in_proj, t), expanded_bytes(p.out_proj, t));
     b.w8.p = c.take<uint8_t>(b.w8.bytes);
-    b.ssd.bytes = step ? 0 : ssd_workspace_layout(ssd_sizes(p)).total;
+    b.ssd.bytes = step ? 0 : ssd_workspace_layout(ssd_sizes(p)).total + ssd_workspace_layout(ssd_sizes(p)).sums_bytes;
     b.ssd.p = c.take<uint8_t>(b.ssd.bytes);
     b.total = c.off;
     return b;

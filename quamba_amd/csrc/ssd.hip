@@ -105,18 +105,43 @@ __global__ __launch_bounds__(256) void ssd_cumsum_kernel(QaSsdParams p, float* d
 // ---------------------------------------------------------------------------------------------
 __device__ __forceinline__ v4f mfma16(v8h a, v8h b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ float ubyte_of(uint32_t w, int j) { return static_cast<float>((w >> (8 * j)) & 0xffu); }
+// float(int8 byte j of w) in one instruction (left to itself the compiler shifts and sign-extends the byte out first)
+__device__ __forceinline__ float sbyte_of(uint32_t w, int j) {
+    float r;
+    switch (j) {
+        case 0: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(r) : "v"(w)); break;
+        case 1: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(r) : "v"(w)); break;
+        case 2: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(r) : "v"(w)); break;
+        default: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(r) : "v"(w)); break;
+    }
+    return r;
+}
 constexpr uint32_t kBias = 0x80808080u;
 __device__ __forceinline__ uint32_t word_of(const uint4& v, int d) { return d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w; }
 __device__ __forceinline__ float lane_of(const float4& v, int d) { return d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w; }
 
-// A thread's share of a chunk's x tile, steps 4 kb .. 4 kb + 3 of channels 16 pb .. 16 pb + 15 (four 16-byte loads,
-// biased bytes), goes to the transposed fp16 tile: sixteen 8-byte stores, rows in slot order.
-template <int XP>
-__device__ __forceinline__ void stage_x_share(_Float16 (*xt)[XP], const uint4 (&xr)[4], const float* xs, int pb, int kb) {
+// A thread's share of a chunk's x tile, steps 4 kb .. 4 kb + 3 of the CH (8 or 16) channels from c0 on (four loads of as many
+// bytes), goes to the transposed fp16 tile: CH 8-byte stores, rows in slot order.
+template <int CH>
+struct XShare { uint32_t w[CH / 4]; };
+template <int CH>
+__device__ __forceinline__ XShare<CH> load_x_share(const int8_t* from) {
+    XShare<CH> r;
+    if constexpr (CH == 16) {
+        const uint4 v = *reinterpret_cast<const uint4*>(from);
+        r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
+    } else {
+        const uint2 v = *reinterpret_cast<const uint2*>(from);
+        r.w[0] = v.x; r.w[1] = v.y;
+    }
+    return r;
+}
+template <int XP, int CH>
+__device__ __forceinline__ void stage_x_share(_Float16 (*xt)[XP], const XShare<CH> (&xr)[4], const float* xs, int c0, int kb) {
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        const float4 s4 = *reinterpret_cast<const float4*>(xs + 16 * pb + 4 * d);
-        const uint32_t w0 = word_of(xr[0], d) ^ kBias, w1 = word_of(xr[1], d) ^ kBias, w2 = word_of(xr[2], d) ^ kBias, w3 = word_of(xr[3], d) ^ kBias;
+    for (int d = 0; d < CH / 4; ++d) {
+        const float4 s4 = *reinterpret_cast<const float4*>(xs + c0 + 4 * d);
+        const uint32_t w0 = xr[0].w[d] ^ kBias, w1 = xr[1].w[d] ^ kBias, w2 = xr[2].w[d] ^ kBias, w3 = xr[3].w[d] ^ kBias;
 #pragma unroll
         for (int cc = 0; cc < 4; ++cc) {
             const float sc = lane_of(s4, cc), nsc = -128.0f * sc;
@@ -125,7 +150,7 @@ __device__ __forceinline__ void stage_x_share(_Float16 (*xt)[XP], const uint4 (&
             v[1] = static_cast<_Float16>(__builtin_fmaf(ubyte_of(w1, cc), sc, nsc));
             v[2] = static_cast<_Float16>(__builtin_fmaf(ubyte_of(w2, cc), sc, nsc));
             v[3] = static_cast<_Float16>(__builtin_fmaf(ubyte_of(w3, cc), sc, nsc));
-            *reinterpret_cast<v4h*>(&xt[cc * 16 + 4 * pb + d][kb * 4]) = v;          // row slot(16 pb + 4 d + cc)
+            *reinterpret_cast<v4h*>(&xt[cc * 16 + c0 / 4 + d][kb * 4]) = v;              // row slot(c0 + 4 d + cc)
         }
     }
 }
@@ -147,34 +172,39 @@ __device__ __forceinline__ void unit_head_part(int linear, int units, int hpg, i
 
 // ---------------------------------------------------------------------------------------------
 // Stages 2, 3 and 6 (quamba/triton/quant_chunk_state.py:76-89, quant_state_passing.py:60-83, quant_ssm_states.py
-// :43,119): a workgroup of four waves per (batch, head, 64 state columns) walks the chunks in order with its part
-// of the running state P (64 x 64 of headdim x dstate, fp32) in registers; the fp32 chunk states never travel
-// through memory.  A wave owns 16 columns n and all rows p.  Its B operand, f16((s_B q_B[k,n]) w_k) with the
+// :43,119): a workgroup of N / 16 waves per (batch, head) walks the chunks in order with the running state P
+// (64 x N of headdim x dstate, fp32) in registers; the fp32 chunk states never travel
+// through memory.  A wave owns 16 columns n and all rows p.  Its B operand, f16(q_B[k,n] (s_B w_k)) with the
 // per-head weight w_k = exp(dA_last - dA_k) dt_k, is built in registers from the transposed int8 B tile in LDS
 // (rows n of 4-byte-aligned pitch with an odd number of dwords: conflict-free for the transposing dword stores
 // and for the operand reads); its A operand is the transposed x tile.  The tiles of chunk c+1 are fetched into
 // registers while chunk c is multiplied.  The state entering chunk c >= 1 is stored as fp16, rows in slot order.
+// Bound by vector issue (converting x and B to fp16 operands) and by the LDS reads of the x tile, which every wave makes: with
+// one workgroup for all N columns x is staged once; as a workgroup per 64 columns, which also formed s_B q_B and the product
+// with w_k apart, 16 x 1024 steps of 128 heads took 146 us, now 122.  (Four waves of 32 columns instead of eight of 16 read
+// x half as often and take 138: too few waves for the latencies of a chunk.)
 // ---------------------------------------------------------------------------------------------
-template <int Q>
+template <int N, int Q>
 struct StateSmem {
     static constexpr int XP = Q + 8;        // halves per row of the transposed x tile
     static constexpr int BP = Q + 4;        // bytes per row of the transposed B tile
     __attribute__((aligned(16))) _Float16 xt[kP][XP];
-    __attribute__((aligned(16))) int8_t b8[64][BP];
+    __attribute__((aligned(16))) int8_t b8[N][BP];
     __attribute__((aligned(16))) float w[Q];
     __attribute__((aligned(16))) float xs[kP];    // x scale per channel
     int32_t srow[kP];                             // the channel's row of the grouped state scales
 };
 
-template <int N, int Q>
-__global__ __launch_bounds__(256, 3) void ssd_state_kernel(QaSsdParams p, const float* dt_ws, const float* dA_ws, __half* prev, const float* xs_ws,
-                                                          const int32_t* srow_ws, int nc) {
-    using S = StateSmem<Q>;
+template <int N, int Q, bool WALK>
+__global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSsdParams p, const float* dt_ws, const float* dA_ws, __half* prev, float* sums,
+                                                                              const float* xs_ws, const int32_t* srow_ws, int nc) {
+    using S = StateSmem<N, Q>;
     extern __shared__ __attribute__((aligned(16))) unsigned char ssd_smem_raw[];
     S& sm = *reinterpret_cast<S*>(ssd_smem_raw);
-    constexpr int kThreads = 256;
-    constexpr int PARTS = N / 64;                                 // workgroups per (batch, head)
-    static_assert(Q <= kThreads, "a thread stages at most one share of the chunk's tiles");
+    constexpr int kThreads = 4 * N;
+    constexpr int CH = N == 128 ? 8 : 16;                         // channels of a thread's share of x
+    constexpr int kSharesX = Q / 4 * (kP / CH), kSharesB = Q / 4 * (N / 16);
+    static_assert(kSharesX <= kThreads && kSharesB <= kThreads && Q <= kThreads, "a thread stages at most one share of the chunk's tiles");
 
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);    // the same in every lane: kept in a scalar register
@@ -183,27 +213,26 @@ __global__ __launch_bounds__(256, 3) void ssd_state_kernel(QaSsdParams p, const 
     const int split = p.headdim / kP;
     const int G = p.ngroups, H = p.nheads * split, L = p.seqlen;
     int unit, hig, part;
-    unit_head_part(blockIdx.x, p.batch * G, H / G, PARTS, unit, hig, part);
+    unit_head_part(blockIdx.x, p.batch * (WALK ? 1 : nc) * G, H / G, 1, unit, hig, part);
     const int h = (unit % G) * (H / G) + hig;
     const int hp = h / split, ch0 = (h % split) * kP;
-    const int b = unit / G;
+    const int b = WALK ? unit / G : unit / (G * nc), my_chunk = WALK ? 0 : unit / G % nc;
     const int g = hp / (p.nheads / G);
     const bool grouped = p.nhead_groups > 0;
     const float sB = grouped ? p.B_scale[g] : p.B_scale[0];
-    const float nsB = -128.0f * sB;
     const uint32_t xrow = static_cast<uint32_t>(H) * kP;          // bytes between steps of x
     const uint32_t brow = static_cast<uint32_t>(G) * N;           // bytes between steps of B
     const int64_t rows0 = (static_cast<int64_t>(b) * p.nheads + hp) * nc;
-    // this thread's share of a chunk's tiles: steps 4 kb .. 4 kb + 3, sixteen columns from 16 pb (of x: channels; of
-    // B: state columns of this workgroup's part)
-    const int pb = tid % 4, kb = tid / 4;
-    const bool mine = Q == 256 || tid < Q;
-    const uint32_t voff_x = static_cast<uint32_t>(4 * kb) * xrow + 16 * pb, voff_b = static_cast<uint32_t>(4 * kb) * brow + 16 * pb;
+    // this thread's share of a chunk's tiles: steps 4 kb .. 4 kb + 3 of CH channels of x and of sixteen state columns of B
+    const int xc = tid % (kP / CH) * CH, xkb = tid / (kP / CH), bc = tid % (N / 16) * 16, bkb = tid / (N / 16);
+    const bool mine_x = kSharesX == kThreads || tid < kSharesX, mine_b = kSharesB == kThreads || tid < kSharesB;
+    const uint32_t voff_x = static_cast<uint32_t>(4 * xkb) * xrow + xc, voff_b = static_cast<uint32_t>(4 * bkb) * brow + bc;
     if (tid < kP) {
         sm.xs[tid] = xs_ws[hp * p.headdim + ch0 + tid];
         sm.srow[tid] = srow_ws[hp * p.headdim + ch0 + tid];
     }
-    uint4 xr[4], br[4];
+    XShare<CH> xr[4];
+    uint4 br[4];
     float r_dt = 0.0f, r_dA = 0.0f, r_last = 0.0f;
     int valid_loaded = Q;                                         // steps of the chunk whose tiles are in xr / br
     // One path for whole and ragged chunks: rows past the end of the sequence read the last row (the loads stay inside
@@ -215,14 +244,15 @@ __global__ __launch_bounds__(256, 3) void ssd_state_kernel(QaSsdParams p, const 
         valid_loaded = valid;
         // uniform row addresses plus one per-thread offset: the address arithmetic stays in scalar registers
         const int8_t* xsrc = p.x + (static_cast<int64_t>(b) * L + t0) * xrow + static_cast<int64_t>(h) * kP;
-        const int8_t* bsrc = p.B + (static_cast<int64_t>(b) * L + t0) * brow + static_cast<int64_t>(g) * N + part * 64;
-        if (mine) {
-            const uint32_t last_x = static_cast<uint32_t>(valid - 1) * xrow + 16 * pb, last_b = static_cast<uint32_t>(valid - 1) * brow + 16 * pb;
+        const int8_t* bsrc = p.B + (static_cast<int64_t>(b) * L + t0) * brow + static_cast<int64_t>(g) * N;
+        const uint32_t last_x = static_cast<uint32_t>(valid - 1) * xrow + xc, last_b = static_cast<uint32_t>(valid - 1) * brow + bc;
+        if (mine_x) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                xr[r] = *reinterpret_cast<const uint4*>(xsrc + static_cast<uint64_t>(min(voff_x + static_cast<uint32_t>(r) * xrow, last_x)));
-                br[r] = *reinterpret_cast<const uint4*>(bsrc + static_cast<uint64_t>(min(voff_b + static_cast<uint32_t>(r) * brow, last_b)));
-            }
+            for (int r = 0; r < 4; ++r) xr[r] = load_x_share<CH>(xsrc + static_cast<uint64_t>(min(voff_x + static_cast<uint32_t>(r) * xrow, last_x)));
+        }
+        if (mine_b) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) br[r] = *reinterpret_cast<const uint4*>(bsrc + static_cast<uint64_t>(min(voff_b + static_cast<uint32_t>(r) * brow, last_b)));
         }
         const float* dA_row = dA_ws + (rows0 + c) * Q;
         r_last = dA_row[Q - 1];
@@ -232,51 +262,53 @@ __global__ __launch_bounds__(256, 3) void ssd_state_kernel(QaSsdParams p, const 
         }
     };
     auto stage_chunk = [&]() {
-        if (mine) {
-            if (valid_loaded < Q) {
-                // ragged last chunk: steps past the end of the sequence count as zero
+        if (valid_loaded < Q) {
+            // ragged last chunk: steps past the end of the sequence count as zero
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (4 * kb + r >= valid_loaded) xr[r] = br[r] = make_uint4(0u, 0u, 0u, 0u);
-                }
+            for (int r = 0; r < 4; ++r) {
+                if (4 * xkb + r >= valid_loaded) xr[r] = XShare<CH>{};
+                if (4 * bkb + r >= valid_loaded) br[r] = make_uint4(0u, 0u, 0u, 0u);
             }
-            stage_x_share<S::XP>(sm.xt, xr, sm.xs, pb, kb);
+        }
+        if (mine_x) stage_x_share<S::XP, CH>(sm.xt, xr, sm.xs, xc, xkb);
+        if (mine_b) {
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
                 // 4x4 byte transpose: rows k (registers) x columns n (bytes) -> rows n x bytes k
-                const uint32_t r0 = word_of(br[0], d) ^ kBias, r1 = word_of(br[1], d) ^ kBias, r2 = word_of(br[2], d) ^ kBias, r3 = word_of(br[3], d) ^ kBias;
+                const uint32_t r0 = word_of(br[0], d), r1 = word_of(br[1], d), r2 = word_of(br[2], d), r3 = word_of(br[3], d);
                 const uint32_t lo01 = __builtin_amdgcn_perm(r1, r0, 0x05010400u);   // r0.b0 r1.b0 r0.b1 r1.b1
                 const uint32_t hi01 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);   // r0.b2 r1.b2 r0.b3 r1.b3
                 const uint32_t lo23 = __builtin_amdgcn_perm(r3, r2, 0x05010400u);
                 const uint32_t hi23 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
-                const int n4 = 16 * pb + 4 * d;
-                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 0][kb * 4]) = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 1][kb * 4]) = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 2][kb * 4]) = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 3][kb * 4]) = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+                const int n4 = bc + 4 * d;
+                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 0][bkb * 4]) = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 1][bkb * 4]) = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 2][bkb * 4]) = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 3][bkb * 4]) = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
             }
         }
-        if (tid < Q) sm.w[tid] = fexp(r_last - r_dA) * r_dt;        // weight of step k in the chunk's state
+        if (tid < Q) sm.w[tid] = sB * (fexp(r_last - r_dA) * r_dt);        // weight of step k in the chunk's state
     };
 
-    // the running state: columns n = 64 part + 16 wave + lane % 16; tile j, register r: channel p = 4 (4 (lane / 16) + r) + j
-    const int n_col = part * 64 + 16 * wave + l16;
+    // the running state: columns n = 16 wave + lane % 16; tile j, register r: channel p = 4 (4 (lane / 16) + r) + j
+    const int n_col = 16 * wave + l16;
     v4f run[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) run[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-    load_chunk(0);
+    load_chunk(my_chunk);
     __syncthreads();                                              // the table of x scales
     stage_chunk();
     float dA_last = r_last;                                       // of the chunk about to be multiplied
     __syncthreads();
 
-    for (int c = 0; c < nc; ++c) {
-        const bool more = c + 1 < nc;
+    const int chunks = WALK ? nc : 1;
+    for (int c = 0; c < chunks; ++c) {
+        const bool more = c + 1 < chunks;
         // in flight during the products.  Unconditional (the last chunk is requested once more and never staged): a
         // conditional request leaves the tile registers with two possible sources, which the compiler merges by
         // copies right behind the loads, i.e. by waiting for them where they are issued
-        load_chunk(min(c + 1, nc - 1));
+        if constexpr (WALK) load_chunk(min(c + 1, nc - 1));
         __builtin_amdgcn_sched_barrier(0);                         // (the scheduler would sink the requests below the products)
         v4f accs[4];
 #pragma unroll
@@ -293,9 +325,17 @@ __global__ __launch_bounds__(256, 3) void ssd_state_kernel(QaSsdParams p, const 
             const float wk[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
             v8h bw;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) bw[e] = static_cast<_Float16>(__builtin_fmaf(ubyte_of(e < 4 ? b0 : b1, e & 3), sB, nsB) * wk[e]);
+            for (int e = 0; e < 8; ++e) bw[e] = static_cast<_Float16>(sbyte_of(e < 4 ? b0 : b1, e & 3) * wk[e]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) accs[j] = mfma16(fx[j], bw, accs[j]);
+        }
+        if constexpr (!WALK) {
+            float* to = sums + (((static_cast<int64_t>(b) * nc + my_chunk) * H + h) * kP) * N + n_col;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) to[(j * 16 + 4 * lq + r) * N] = accs[j][r];
+            return;
         }
         // P <- exp(dA_last) P + S
         const float decay = fexp(dA_last);
@@ -334,6 +374,63 @@ __global__ __launch_bounds__(256, 3) void ssd_state_kernel(QaSsdParams p, const 
                     static_cast<int8_t*>(p.final_states)[fo] = ssd_quantize_state(p, sm.srow[pp], n_col, sv);
                 }
             }
+    }
+}
+
+// The same with few heads in flight: a workgroup per chunk (WALK false) leaves the chunk's own sums S_c in memory as fp32, rows
+// in slot order, and this kernel runs the recurrence over them, four states a thread: the same values in the same order.
+template <int N>
+__global__ __launch_bounds__(256) void ssd_pass_kernel(QaSsdParams p, const float* dA_ws, __half* prev, const float* sums, const int32_t* srow_ws, int nc) {
+    constexpr int kPieces = kP * N / 4;                           // of one head of 64 channels
+    const int split = p.headdim / kP, H = p.nheads * split;
+    const unsigned bh = blockIdx.x / (kPieces / 256);
+    const int piece = (blockIdx.x % (kPieces / 256)) * 256 + threadIdx.x;
+    const int b = bh / H, h = bh % H, hp = h / split, ch0 = (h % split) * kP;
+    const int slot = piece / (N / 4), n = piece % (N / 4) * 4;
+    const int64_t step = static_cast<int64_t>(H) * kP * N, first = ((static_cast<int64_t>(b) * nc) * H + h) * kP * N + piece * 4;
+    const float* dA = dA_ws + (static_cast<int64_t>(b) * p.nheads + hp) * nc * p.chunk_size + p.chunk_size - 1;
+    constexpr int kAhead = 8;
+    float4 s[kAhead];
+    float d[kAhead];
+    auto load = [&](int c, int at) {
+        const int cc = min(c, nc - 1);
+        s[at] = *reinterpret_cast<const float4*>(sums + first + cc * step);
+        d[at] = dA[static_cast<int64_t>(cc) * p.chunk_size];
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) load(i, i);
+    float4 run = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int c0 = 0; c0 < nc; c0 += kAhead) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const int c = c0 + i;
+            if (c < nc) {
+                const float decay = fexp(d[i]);
+                run.x = decay * run.x + s[i].x;
+                run.y = decay * run.y + s[i].y;
+                run.z = decay * run.z + s[i].z;
+                run.w = decay * run.w + s[i].w;
+                load(c + kAhead, i);
+                if (c + 1 < nc) {
+                    v4h o;
+                    o[0] = static_cast<_Float16>(run.x); o[1] = static_cast<_Float16>(run.y);
+                    o[2] = static_cast<_Float16>(run.z); o[3] = static_cast<_Float16>(run.w);
+                    *reinterpret_cast<v4h*>(prev + first + (c + 1) * step) = o;
+                }
+            }
+        }
+    }
+    if (p.final_states) {
+        const int pp = 4 * (slot % 16) + slot / 16;
+        const int64_t fo = ((static_cast<int64_t>(b) * H + h) * kP + pp) * N + n;
+        if (p.final_state_is_fp32) {
+            *reinterpret_cast<float4*>(static_cast<float*>(p.final_states) + fo) = run;
+        } else {
+            const int srow = srow_ws[hp * p.headdim + ch0 + pp];
+            const float v[4] = {run.x, run.y, run.z, run.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) static_cast<int8_t*>(p.final_states)[fo + i] = ssd_quantize_state(p, srow, n + i, v[i]);
+        }
     }
 }
 
@@ -474,11 +571,11 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
         // (one path for whole and ragged chunks: rows past the end of the sequence read the last row and are zeroed
         // when the tile is staged; with a second path beside it the compiler merges the two sets of destination
         // registers by copies right behind the loads and so waits for them before the requests below are issued)
-        uint4 xr[4];
+        XShare<16> xr[4];
         if (mine) {
             const uint32_t last_x = static_cast<uint32_t>(lim - 1) * xrow + 16 * pb, voff_x = static_cast<uint32_t>(4 * kb) * xrow + 16 * pb;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) xr[r] = *reinterpret_cast<const uint4*>(xbase + static_cast<uint64_t>(min(voff_x + static_cast<uint32_t>(r) * xrow, last_x)));
+            for (int r = 0; r < 4; ++r) xr[r] = load_x_share<16>(xbase + static_cast<uint64_t>(min(voff_x + static_cast<uint32_t>(r) * xrow, last_x)));
         }
         if (tid < kP) {
             sm.xs[tid] = xs_ws[hp * p.headdim + ch0 + tid];
@@ -513,10 +610,10 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                 // ragged last chunk: steps past the end of the sequence count as zero
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    if (4 * kb + r >= lim) xr[r] = make_uint4(0u, 0u, 0u, 0u);
+                    if (4 * kb + r >= lim) xr[r] = XShare<16>{};
                 }
             }
-            stage_x_share<S::XP>(sm.xt, xr, sm.xs, pb, kb);
+            stage_x_share<S::XP, 16>(sm.xt, xr, sm.xs, 16 * pb, kb);
         }
     }
     __syncthreads();
@@ -675,10 +772,9 @@ int validate(const QaSsdParams* p) {
     if (p->headdim < 1 || p->headdim > 256 || p->dstate < 1 || p->dstate > 1024 || p->chunk_size < 1 || p->chunk_size > 1024) return QA_ERR_UNSUPPORTED;
     const int64_t nc = (static_cast<int64_t>(p->seqlen) + p->chunk_size - 1) / p->chunk_size;
     if (ssd_fast_shape(*p)) {
-        // every launch is a one-dimensional grid: one workgroup per (batch, chunk, head) or per (batch, head, 64 states)
+        // every launch is a one-dimensional grid: one workgroup per (batch, chunk, head) or per (batch, head)
         const int64_t heads = static_cast<int64_t>(p->nheads) * (p->headdim / 64);       // heads of 64 channels
         if (static_cast<int64_t>(p->batch) * nc * heads > 0x7fffffffLL) return QA_ERR_SHAPE;
-        if (static_cast<int64_t>(p->batch) * heads * (p->dstate / 64) > 0x7fffffffLL) return QA_ERR_SHAPE;
     } else {
         const int st = ssd_general_grid_check(*p);
         if (st != QA_OK) return st;
@@ -691,7 +787,8 @@ int validate(const QaSsdParams* p) {
 
 extern "C" int64_t qa_ssd_workspace_bytes(const QaSsdParams* p) {
     if (qa::validate(p) != QA_OK) return 0;
-    return qa::ssd_workspace_layout(*p).total;
+    const qa::SsdWorkspace ws = qa::ssd_workspace_layout(*p);
+    return ws.total + ws.sums_bytes;
 }
 
 extern "C" int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream_) {
@@ -724,7 +821,7 @@ extern "C" int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream_) {
     hipLaunchKernelGGL(ssd_cumsum_kernel, dim3(static_cast<unsigned>((bch + 3) / 4)), dim3(256), 0, stream, *p, dt_ws,
                        dA_ws, xs_ws, srow_ws, nc);
     const int heads64 = p->nheads * (p->headdim / 64);          // the kernels see a head of 64 s channels as s heads of 64
-    const dim3 hgrid(static_cast<unsigned>(p->batch * heads64 * (p->dstate / 64)));
+    const dim3 hgrid(static_cast<unsigned>(p->batch * heads64));
     int status = QA_OK;
     // more LDS than a kernel gets by default: raise the limit (idempotent)
     auto lds_ok = [&](const void* kernel, size_t lds) {
@@ -733,12 +830,19 @@ extern "C" int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream_) {
         if (status == QA_OK) status = QA_ERR_LAUNCH;
         return false;
     };
-    auto launch = [&](auto state_kernel, size_t state_lds, auto scan_kernel, size_t scan_lds, int scan_threads) {
+    float* sums_ws = ws.sums_bytes && p->workspace_bytes >= ws.sums + ws.sums_bytes ? reinterpret_cast<float*>(base + ws.sums) : nullptr;
+    auto launch = [&](auto state_kernel, auto chunk_state_kernel, auto pass_kernel, size_t state_lds, auto scan_kernel, size_t scan_lds, int scan_threads) {
         if (!lds_ok(reinterpret_cast<const void*>(state_kernel), state_lds) || !lds_ok(reinterpret_cast<const void*>(scan_kernel), scan_lds)) return;
-        hipLaunchKernelGGL(state_kernel, hgrid, dim3(256), state_lds, stream, *p, dt_ws, dA_ws, prev_ws, xs_ws, srow_ws, nc);
+        if (sums_ws) {
+            if (!lds_ok(reinterpret_cast<const void*>(chunk_state_kernel), state_lds)) return;
+            hipLaunchKernelGGL(chunk_state_kernel, dim3(hgrid.x * nc), dim3(4 * p->dstate), state_lds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws, srow_ws, nc);
+            hipLaunchKernelGGL(pass_kernel, dim3(hgrid.x * (p->dstate / 16)), dim3(256), 0, stream, *p, dA_ws, prev_ws, sums_ws, srow_ws, nc);
+        } else {
+            hipLaunchKernelGGL(state_kernel, hgrid, dim3(4 * p->dstate), state_lds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws, srow_ws, nc);
+        }
         hipLaunchKernelGGL(scan_kernel, dim3(static_cast<unsigned>(bch * (p->headdim / 64))), dim3(scan_threads), scan_lds, stream, *p, dt_ws, dA_ws, prev_ws, xs_ws, nc);
     };
-#define QA_SSD_LAUNCH(N_, Q_) launch(ssd_state_kernel<N_, Q_>, sizeof(StateSmem<Q_>), ssd_chunk_scan_kernel<N_, Q_>, \
+#define QA_SSD_LAUNCH(N_, Q_) launch(ssd_state_kernel<N_, Q_, true>, ssd_state_kernel<N_, Q_, false>, ssd_pass_kernel<N_>, sizeof(StateSmem<N_, Q_>), ssd_chunk_scan_kernel<N_, Q_>, \
                                      sizeof(ScanSmem<N_, Q_>), 64 * scan_waves_of(Q_))
     if (p->dstate == 128) {
         if (p->chunk_size == 256) QA_SSD_LAUNCH(128, 256);

@@ -16,7 +16,19 @@ __device__ __forceinline__ int ssd_dt_stride(const QaSsdParams& p) { return p.dt
 
 struct SsdWorkspace {            // sections of the workspace (byte offsets), see qa_ssd_workspace_bytes
     int64_t dt, dA, prev, xs, srow, total;
+    int64_t sums, sums_bytes;    // behind `total`, used when the caller's workspace holds it (see ssd_chunks_apart)
 };
+
+// Whether the chunks' states are summed by a workgroup each and chained by a pass of its own (matrix-core shapes): with few
+// heads in flight.  Walking, a workgroup takes about 5 us per chunk of 256 steps (a lone one; 6.4 in two rounds); apart, each
+// chunk and head costs 24 ns of the whole chip and the second launch 6 us: 6 chunks of 80 heads 30 against 19 us, 16 chunks
+// of 320 heads 102 against 129.
+inline bool ssd_chunks_apart(const QaSsdParams& p) {
+    const double nc = static_cast<double>((p.seqlen + p.chunk_size - 1) / p.chunk_size), q = p.chunk_size / 256.0;
+    const double heads = static_cast<double>(p.batch) * p.nheads * (p.headdim / 64);
+    const double rounds = heads <= 256 ? 5.0 : heads <= 512 ? 6.4 : heads / 80.0;
+    return nc >= 2 && nc * heads * (0.008 * q + 0.016) * (p.dstate / 128.0) + 6.0 < nc * rounds * q;
+}
 
 __host__ __device__ inline int64_t ssd_align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
@@ -24,7 +36,7 @@ __host__ __device__ inline int64_t ssd_align256(int64_t v) { return (v + 255) & 
 // fp16 [batch, chunks, nheads, headdim, dstate]; the x scale of every channel, fp32 [nheads, headdim], and the row of
 // the grouped state scales it quantises its final state with, int32 [nheads, headdim] (both looked up once from the
 // group ranges by the first kernel: the others read them with one load instead of a chain of dependent ones)
-__host__ __device__ inline SsdWorkspace ssd_workspace_layout(const QaSsdParams& p) {
+inline SsdWorkspace ssd_workspace_layout(const QaSsdParams& p) {
     const int64_t nc = (p.seqlen + p.chunk_size - 1) / p.chunk_size;
     const int64_t B = p.batch, H = p.nheads, Q = p.chunk_size, N = p.dstate, P = p.headdim;
     SsdWorkspace w;
@@ -35,6 +47,8 @@ __host__ __device__ inline SsdWorkspace ssd_workspace_layout(const QaSsdParams& 
     w.xs = off; off = ssd_align256(off + H * P * 4);
     w.srow = off; off = ssd_align256(off + H * P * 4);
     w.total = off;
+    w.sums = off;
+    w.sums_bytes = p.headdim % 64 == 0 && (p.dstate == 64 || p.dstate == 128) && ssd_chunks_apart(p) ? B * nc * H * P * N * 4 : 0;
     return w;
 }
 
