@@ -225,6 +225,8 @@ struct RegCfg {
     static constexpr int kABytes = kBM * KT;
     static constexpr int kAInstr = kABytes / 1024 / NW;            // direct-to-LDS requests of a wave per tile
     static constexpr int kWLoads = KT / 64;                        // 16-byte pieces of packed weights per lane and tile
+    // what a row's 16-byte pieces are exchanged by: sixteen neighbouring rows of one column of pieces then cover all banks
+    __device__ static __forceinline__ int exchange(int row) { return KT == 256 ? row & 15 : (row >> 1) & 7; }
     static constexpr int kEpilogue = epilogue_lds_bytes<TM, 1, NW>();
     static constexpr int kLdsBytes = 2 * kABytes > kEpilogue ? 2 * kABytes : kEpilogue;
 };
@@ -246,14 +248,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4a8_reg_kernel(QaGemmW4A8Params
     const int m0 = tile_m * R::kBM, n0 = tile_n * R::kBN + wave * 32;
     const int ldw = p.k / 2, k_tiles = (p.k + KT - 1) / KT;
 
-    // activations: request j of a wave fills LDS bytes [(j NW + wave) 1024, + 1024) of the tile, i.e. 1024 / KT rows; the
-    // 16-byte pieces of a row are exchanged by the row's low bits, so that a column of pieces covers all banks
+    // activations: request j of a wave fills LDS bytes [(j NW + wave) 1024, + 1024) of the tile, i.e. 1024 / KT rows
     const v4i rsrc_a = make_rsrc(p.a, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k));
     const uint32_t lds_a = lds_offset_of(lds);
     int a_off[R::kAInstr], a_k[R::kAInstr];
 #pragma unroll
     for (int j = 0; j < R::kAInstr; ++j) {
-        const int piece = (j * NW + wave) * 64 + lane, row = piece / R::kRowChunks, c = (piece % R::kRowChunks) ^ (row % R::kRowChunks);
+        const int piece = (j * NW + wave) * 64 + lane, row = piece / R::kRowChunks, c = (piece % R::kRowChunks) ^ R::exchange(row);
         a_k[j] = c * 16;
         a_off[j] = m0 + row < p.m ? static_cast<int>((m0 + row) * p.lda) + c * 16 : 0x70000000;
     }
@@ -305,7 +306,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4a8_reg_kernel(QaGemmW4A8Params
                 auto fetch = [&](int kk) {
 #pragma unroll
                     for (int j = 0; j < TM; ++j) {
-                        const int row = j * 32 + frow, c = (fhalf * kSteps + kk) ^ (row % R::kRowChunks);
+                        const int row = j * 32 + frow, c = (fhalf * kSteps + kk) ^ R::exchange(row);
                         fa[kk & 1][j] = *reinterpret_cast<const v4i*>(sa + row * KT + c * 16);
                     }
                 };
