@@ -15,6 +15,7 @@
 #include "conv2_common.hpp"
 #include "gemm_core.hpp"
 #include "gemv.hpp"
+#include "hadamard_core.hpp"
 #include "w4_expand.hpp"
 
 namespace qa {
@@ -282,6 +283,129 @@ int pick(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
     if (groups <= 2816 && p.k >= 2048) return launch<BITS, M, 2, B2>(p, conv, stream);
     return launch<BITS, M, 1, B1>(p, conv, stream);
 }
+// ---------------------------------------------------------------------------------------------
+// One activation row that the kernel makes itself: the Hadamard transform and quantisation that as a launch of its own keeps
+// one workgroup busy for 3 to 5 us while the weights wait.  Here every workgroup transforms the row in its own LDS, in the
+// order of the stand-alone kernel and so to the same bits, with its share of the weights on the way.  Eight waves a workgroup
+// and at most about one workgroup per CU, so that no CU transforms the row twice; KS waves share four weight rows.  A decode
+// step of one sequence (one launch less to make and to wait for): d_inner 1536 21.0 -> 18.0 us, 3072 20.5 -> 17.3, 4096 21.9
+// -> 19.7, 5120 25.7 -> 23.6; 8192 33.5 -> 34.0, so up to 5120 only.  (With the gated norm in front as well it was slower
+// than the two kernels at every width.)
+// ---------------------------------------------------------------------------------------------
+constexpr int kRotThreads = 512, kRotWaves = kRotThreads / 64, kRotDim = 5120;
+
+struct RotShape {
+    int log_m, ks;
+};
+
+template <int BITS, int S>
+__global__ __launch_bounds__(kRotThreads) void gemv_rotated_kernel(GemvParams p, GemvRotate r, RotShape shape) {
+    constexpr int kLaneCodes = BITS == 8 ? 16 : 32, kPieceCodes = 64 * kLaneCodes, AQ = kLaneCodes / 16, BATCH = BITS == 8 ? 4 : 2;
+    extern __shared__ __attribute__((aligned(16))) float buf[];
+    __shared__ int parts[kRotWaves][64];
+    const int tid = threadIdx.x, lane = tid & 63, dim = p.k;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ks = shape.ks, part_k = wave % ks;
+    const int n0 = (blockIdx.x * (kRotWaves / ks) + wave / ks) * kRows;
+    int8_t* codes = reinterpret_cast<int8_t*>(buf + (dim + (dim >> 5) + 4) / 4 * 4);
+    const int share = (dim / kLaneCodes + ks - 1) / ks * kLaneCodes;
+    const int k_first = part_k * share, k_end = min(k_first + share, dim);
+    const int pieces = (k_end - k_first + kPieceCodes - 1) / kPieceCodes;
+
+    const uint8_t* w_row[kRows];
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) w_row[q] = static_cast<const uint8_t*>(p.w) + static_cast<int64_t>(min(n0 + q, p.n - 1)) * p.ldw;
+    v4u fw[BATCH][kRows];
+    uint2 fs[BATCH];
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) {
+            const int k0 = k_first + (c0 + b) * kPieceCodes + lane * kLaneCodes, kk = k0 < k_end ? k0 : 0;
+#pragma unroll
+            for (int q = 0; q < kRows; ++q) fw[b][q] = *reinterpret_cast<const v4u*>(w_row[q] + kk * BITS / 8);
+            if constexpr (BITS == 4) fs[b] = *reinterpret_cast<const uint2*>(p.s_group + static_cast<int64_t>(kk / 128) * p.n + min(n0, p.n - 4));
+            if (c0 + b + 1 >= pieces) break;
+        }
+    };
+    // The row first: loads return in order, and what waits for it must not wait for the weights
+    constexpr int kRowPieces = (kRotDim / 8 + kRotThreads - 1) / kRotThreads;
+    uint4 yr[kRowPieces];
+#pragma unroll
+    for (int i = 0; i < kRowPieces; ++i)
+        if ((tid + i * kRotThreads) * 8 < dim) yr[i] = *reinterpret_cast<const uint4*>(r.y + (tid + i * kRotThreads) * 8);
+    __builtin_amdgcn_sched_barrier(0);
+    load(0);
+    const int quarter = lane >> 4, my_n = min(n0 + quarter, p.n - 1);
+    const bool mine = (lane & 15) == 0 && n0 + quarter < p.n;
+    const float s_row = p.rule == kGemvAlpha ? p.alpha : p.row_scale[0];
+    const float s_col = p.rule == kGemvAlpha ? 1.0f : p.col_scale[p.col_numel == 1 ? 0 : my_n];
+    __builtin_amdgcn_sched_barrier(0);
+
+#pragma unroll
+    for (int i = 0; i < kRowPieces; ++i) {
+        const int e0 = (tid + i * kRotThreads) * 8;
+        if (e0 < dim) {
+            const __half* h = reinterpret_cast<const __half*>(&yr[i]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) buf[phys(e0 + j)] = __half2float(h[j]);
+        }
+    }
+    __syncthreads();
+    fwht_passes<kRotThreads, __half>(buf, nullptr, dim, shape.log_m, true, tid);
+    if constexpr (S > 1) {
+        s_point_quantised<S, kRotThreads, 4>(buf, codes, shape.log_m, r.had_scale, tid);
+    } else {
+        for (int e0 = tid * 16; e0 < dim; e0 += kRotThreads * 16) {
+            uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int j = 0; j < 16; ++j) w[j >> 2] |= static_cast<uint32_t>(sat8_half_away(buf[phys(e0 + j)] * r.had_scale) & 0xff) << (8 * (j & 3));
+            *reinterpret_cast<uint4*>(codes + e0) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
+    __syncthreads();
+
+    int acc[kRows] = {0, 0, 0, 0};
+    for (int c0 = 0; c0 < pieces; c0 += BATCH) {
+        if (c0) load(c0);
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) {
+            if (c0 + b >= pieces) break;
+            const int k0 = k_first + (c0 + b) * kPieceCodes + lane * kLaneCodes;
+            v4u fa[AQ];
+#pragma unroll
+            for (int q = 0; q < AQ; ++q) fa[q] = k0 < k_end ? *reinterpret_cast<const v4u*>(codes + k0 + 16 * q) : v4u{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int row = 0; row < kRows; ++row) {
+                if constexpr (BITS == 8) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) acc[row] = __builtin_amdgcn_sdot4(static_cast<int>(fw[b][row][q]), static_cast<int>(fa[0][q]), acc[row], false);
+                } else {
+                    const uint32_t pair = row & 2 ? fs[b].y : fs[b].x;
+                    const uint32_t one = row & 1 ? pair >> 16 : pair & 0xffffu;
+                    const __half2 s2 = bits_h2(one | (one << 16));
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const uint2 e = expand_grouped(fw[b][row][q], s2);
+                        acc[row] = __builtin_amdgcn_sdot4(static_cast<int>(e.x), static_cast<int>(fa[q / 2][2 * (q & 1)]), acc[row], false);
+                        acc[row] = __builtin_amdgcn_sdot4(static_cast<int>(e.y), static_cast<int>(fa[q / 2][2 * (q & 1) + 1]), acc[row], false);
+                    }
+                }
+            }
+        }
+    }
+    int sum = row_sum(fold16(fold32(acc[0], acc[2]), fold32(acc[1], acc[3])));          // of row `lane / 16`
+    if (ks > 1) {
+        if (part_k) parts[wave][lane] = sum;
+        __syncthreads();
+        if (part_k) return;
+        for (int i = 1; i < ks; ++i) sum += parts[wave + i][lane];
+    }
+    if (!mine) return;
+    const float accf = static_cast<float>(sum);
+    float y = p.rule == kGemvHalfAway ? (s_col * s_row) * accf : p.rule == kGemvColOuter ? s_col * (s_row * accf)
+            : p.rule == kGemvAlpha ? s_row * accf : s_row * (s_col * accf);
+    asm volatile("" : "+v"(y));                                  // the fp32 product is rounded on its own
+    static_cast<uint16_t*>(p.d)[my_n] = one_f16_or_bf16<QA_OUT_F16>(y);
+}
 }  // namespace
 
 int gemv_launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
@@ -295,6 +419,23 @@ int gemv_launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
     if (p.m == 2) return pick<4, 2, 2, 1, 1>(p, conv, stream);
     if (p.m <= 4) return pick<4, 4, 2, 1, 1>(p, conv, stream);
     return pick<4, 8, 1, 1, 1>(p, conv, stream);
+}
+
+int gemv_rotated_launch(const GemvParams& p, const GemvRotate& r, hipStream_t stream) {
+    const HadamardShape h = hadamard_shape(p.k);
+    const int64_t groups = (static_cast<int64_t>(p.n) + kRows - 1) / kRows;
+    if (p.m != 1 || p.out_type != QA_OUT_F16 || h.s == 0 || h.log_m < 5 || p.k > kRotDim || groups > 2048) return QA_ERR_UNSUPPORTED;
+    if (!aligned16(r.y) || !aligned16(p.w) || p.ldw % 16 != 0 || (p.bits == 4 && (p.k % 128 != 0 || p.n % 4 != 0 || (reinterpret_cast<uintptr_t>(p.s_group) & 7u)))) return QA_ERR_UNSUPPORTED;
+    const RotShape shape = {h.log_m, groups <= 512 ? 4 : groups <= 1024 ? 2 : 1};
+    const int per_block = kRotWaves / shape.ks;
+    const dim3 grid(static_cast<unsigned>((groups + per_block - 1) / per_block));
+    const int lds = (p.k + (p.k >> 5) + 4) / 4 * 16 + p.k;           // (below 64 KB)
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kRotThreads), lds, stream, p, r, shape);
+        return check_launch();
+    };
+    if (p.bits == 8) return h.s == 12 ? go(gemv_rotated_kernel<8, 12>) : h.s == 40 ? go(gemv_rotated_kernel<8, 40>) : go(gemv_rotated_kernel<8, 1>);
+    return h.s == 12 ? go(gemv_rotated_kernel<4, 12>) : h.s == 40 ? go(gemv_rotated_kernel<4, 40>) : go(gemv_rotated_kernel<4, 1>);
 }
 
 }  // namespace qa

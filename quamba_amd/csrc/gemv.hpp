@@ -45,4 +45,12 @@ inline bool gemv_conv_ok(const GemvConv& f) {
 
 int gemv_launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream);
 
+// One activation row that is made on the spot: sat8(round_half_away(H y * had_scale)) of a row y of k fp16 values
+// (qa_hadamard_quant); fp16 results.  QA_ERR_UNSUPPORTED: not for these sizes (the caller then makes the two calls).
+struct GemvRotate {
+    const __half* y;
+    float had_scale;
+};
+int gemv_rotated_launch(const GemvParams& p, const GemvRotate& r, hipStream_t stream);
+
 }  // namespace qa

@@ -107,6 +107,22 @@ int hadamard(const void* y, int8_t* out, int rows, int dim, float scale, void* s
     return qa_hadamard_quant(&h, stream);
 }
 
+// out_proj of one row with the transform that makes its activations in the same launch (QA_ERR_UNSUPPORTED: apart)
+int project_rotated(const QaLinearParams& w, const GemvRotate& r, void* out, void* stream) {
+    if (w.bits == 4 && !w.s_group) return QA_ERR_UNSUPPORTED;
+    GemvParams g = {};
+    g.m = 1; g.n = w.n; g.k = w.k; g.bits = w.bits;
+    g.out_type = QA_OUT_F16;
+    g.rule = kGemvRowOuter;
+    if (w.bits == 8 && w.row_rule == QA_ROW_ALPHA) { g.rule = kGemvAlpha; g.alpha = w.alpha; }
+    if (w.bits == 8 && w.row_rule == QA_ROW_HALF_AWAY) g.rule = kGemvHalfAway;
+    g.row_numel = 1; g.col_numel = w.bits == 4 ? w.n : w.col_numel;
+    g.ldw = w.bits == 4 ? w.k / 2 : w.k; g.ldd = w.n;
+    g.w = w.weight; g.s_group = static_cast<const __half*>(w.s_group);
+    g.row_scale = w.row_scale; g.col_scale = w.col_scale; g.d = out;
+    return gemv_rotated_launch(g, r, static_cast<hipStream_t>(stream));
+}
+
 #define QA_TRY(call)                       \
     do {                                   \
         const int st_ = (call);            \
@@ -395,6 +411,11 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
     }
     QA_TRY(st);
 
+    if (rows == 1) {
+        const GemvRotate r = {b.y, p->had_scale};
+        st = project_rotated(p->out_proj, r, p->out, stream);
+        if (st != QA_ERR_UNSUPPORTED) return st;
+    }
     QA_TRY(hadamard(b.y, b.yq, rows, d, p->had_scale, stream));
     return project(p->out_proj, b.yq, d, rows, p->out, QA_OUT_F16, false, b.w8, stream);
 }

@@ -69,9 +69,10 @@ def test_step(dev, cls, build, batch, dtype, width):
     _close(out[:, 0], want, (conv, conv2), (ssm, ssm2))
 
 
-@pytest.mark.parametrize("d_model", [768, 2048])
+@pytest.mark.parametrize("d_model", [768, 2048, 2560])
 def test_step_of_a_wide_layer(dev, d_model):
-    """in_proj and the conv in one launch, with the weight rows' K split over waves (2048) and not (768)."""
+    """in_proj and the conv in one launch, with the weight rows' K split over waves (2048) and not (768); for one row the
+    transform and out_proj in one launch, with 12, 1 and 40 column blocks."""
     m, g = _mamba1(W8A8QMamba, dev, seed=1, d_model=d_model)
     for batch in (1, 5):
         h = _ri(dev, g, batch, 1, d_model)
