@@ -21,8 +21,11 @@
 //     until the tile has been consumed, then written to LDS.
 #include "qa_common.hpp"
 #include "conv_common.hpp"
+#include "gemm_core.hpp"
 #include "mixer_common.hpp"
 #include "sscan_common.hpp"
+
+#include <algorithm>
 
 namespace qa {
 namespace {
@@ -832,6 +835,26 @@ int choose_mapping16(const QaSScanParams& p) {
 // state) pieces.
 // Reference: quamba/triton/selective_state_update.py:83-126 and :303-362.
 // ---------------------------------------------------------------------------------------------
+// sat8_rne(fl(h k) / fl(s k)) of four states, packed.  The IEEE quotient is twelve instructions a state and was most of a
+// lane's arithmetic; a product with the reciprocal is within 2^-21 of it, so the integers agree unless the product lies within
+// 1e-4 of a rounding tie (values up to 128; beyond, both saturate), and only a wave that holds such a state divides.
+// (inv: rcp of fl(s k))
+__device__ __forceinline__ uint32_t requantise4(const float (&h)[4], const float (&s)[4], const float (&inv)[4], float k) {
+    float t[4], num[4];
+    bool tie = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        num[e] = h[e] * k;
+        t[e] = num[e] * inv[e];
+        tie |= !(__builtin_fabsf(t[e] - __builtin_rintf(t[e])) < 0.4999f);         // (NaN and infinities divide)
+    }
+    if (__builtin_amdgcn_ballot_w64(tie)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = num[e] / (s[e] * k);
+    }
+    return gemm::pack4_rne_sat8(t[0], t[1], t[2], t[3]);
+}
+
 // VEC: the state axis has unit stride in state, A_log, B and C and every row piece of four states is
 // naturally aligned, so a lane moves its four states with one load and one store per operand.
 // A wave's life here is a chain of memory round trips, not arithmetic, so optional operands are read
@@ -843,15 +866,16 @@ int choose_mapping16(const QaSScanParams& p) {
 // A_log codes are one aligned 16-byte row, per-tensor scales, no fp16 bias, four taps), so the lane's work is one
 // run of loads, arithmetic and stores without loops or branches on the parameter block.
 // CONV_STATE: with CONV and FAST, the codes per row of the conv state (4: a word per row; 3: rows back to back).
+// A_ONE: A_log has one value for all states of a row (Mamba2: one per head), and the decay is evaluated once.
 // DT, with FAST: the step size code is dt_proj's output, evaluated here (a row of up to 160 int8 weights per lane against the
 // batch entry's row of x_proj's output, which is the same for the whole wave and comes through scalar loads).
-template <int LPR, bool VEC, bool FP32, bool CONV, bool FAST = false, int CONV_STATE = 4, bool DT = false>
+template <int LPR, bool VEC, bool FP32, bool CONV, bool FAST = false, int CONV_STATE = 4, bool DT = false, bool A_ONE = false>
 __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, const QaConvParams* cp, const SsmDtProj* dp = nullptr) {
     static_assert(!CONV || LPR == 1, "the conv step needs one lane per row");
     static_assert(!FAST || (LPR == 1 && VEC), "the fixed shape has one lane per row and whole pieces");
     const int dstate = FAST ? 16 : p.dstate;
     // grid: x over the channels of one head, y = head, z = batch (no integer division on the way in)
-    const int gid = blockIdx.x * 256 + threadIdx.x;
+    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     const int sub = gid % LPR;
     const bool row_ok = gid / LPR < p.dim;
     const int d = row_ok ? gid / LPR : p.dim - 1;
@@ -932,7 +956,9 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
             // dstate is a multiple of four here, so the piece is whole.  A_log alone may be a broadcast view
             // (one value per head, stride 0 along the states, as Mamba2 passes it): it is read through its
             // stride, the state and B, C with one load per piece
-            if (a_row16) {
+            if constexpr (A_ONE) {
+                if (k == 0) a8[0][0] = *Ap;
+            } else if (a_row16) {
                 if (k == 0) {
                     const uint4 row = *reinterpret_cast<const uint4*>(Ap);
                     if constexpr (FAST) { a_word[0] = row.x; a_word[1] = row.y; a_word[2] = row.z; a_word[3] = row.w; }
@@ -1062,7 +1088,12 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
     float dt = dt_scale * dtq;
     dt += bias_i8 ? bias_scale * b8 : (bias_f16 ? b16 : 0.0f);
     if (p.dt_softplus) dt = softplus20_flat(dt);
-    float acc = 0.0f;
+    float acc = 0.0f, dA = 0.0f;
+    auto decay = [&](float a_code) {
+        const float A = -__expf(A_scale * a_code);
+        return __expf(A * dt);
+    };
+    if constexpr (A_ONE) dA = decay(static_cast<float>(a8[0][0]));
 #pragma unroll
     for (int k = 0; k < kPieces; ++k) {
         const int n0 = (sub + k * LPR) * 4;
@@ -1070,9 +1101,7 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             if constexpr (!FP32) hv[k][e] = sc[k][e] * static_cast<float>(s8[k][e]);
-            const float a_code = FAST ? code_byte_to_float(a_word[k], e) : static_cast<float>(a8[k][e]);
-            const float A = -__expf(A_scale * a_code);
-            const float dA = __expf(A * dt);
+            if constexpr (!A_ONE) dA = decay(FAST ? code_byte_to_float(a_word[k], e) : static_cast<float>(a8[k][e]));
             const float Bv = FAST ? bvf[k][e] : B_scale * static_cast<float>(b8v[k][e]);
             const float Cv = FAST ? cvf[k][e] : C_scale * static_cast<float>(c8[k][e]);
             hv[k][e] = hv[k][e] * dA + (Bv * dt) * xv;
@@ -1086,9 +1115,10 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
                 *reinterpret_cast<float4*>(static_cast<float*>(p.state) + st_base + n0) =
                     make_float4(hv[k][0], hv[k][1], hv[k][2], hv[k][3]);
             } else {
+                float inv[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) s8[k][e] = sat8_rne((hv[k][e] * requant_k) / (sc[k][e] * requant_k));
-                *reinterpret_cast<int32_t*>(static_cast<int8_t*>(p.state) + st_base + n0) = *reinterpret_cast<const int32_t*>(s8[k]);
+                for (int e = 0; e < 4; ++e) inv[e] = __builtin_amdgcn_rcpf(sc[k][e] * requant_k);
+                *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(p.state) + st_base + n0) = requantise4(hv[k], sc[k], inv, requant_k);
             }
         } else {
 #pragma unroll
@@ -1126,9 +1156,9 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
     }
 }
 
-template <int LPR, bool VEC, bool FP32, bool FAST = false>
+template <int LPR, bool VEC, bool FP32, bool FAST = false, bool A_ONE = false>
 __global__ __launch_bounds__(256) void ssm_update_kernel(QaSsmUpdateParams p) {
-    ssm_update_body<LPR, VEC, FP32, false, FAST>(p, nullptr);
+    ssm_update_body<LPR, VEC, FP32, false, FAST, 4, false, A_ONE>(p, nullptr);
 }
 
 template <bool FP32>
@@ -1140,6 +1170,132 @@ __global__ __launch_bounds__(256) void ssm_update_dt_kernel(QaSsmUpdateParams p,
 template <bool VEC, bool FP32, bool FAST, int CONV_STATE = 4>
 __global__ __launch_bounds__(256) void decode_step_kernel(QaSsmUpdateParams p, QaConvParams cp) {
     ssm_update_body<1, VEC, FP32, true, FAST, CONV_STATE>(p, &cp);
+}
+
+// ---------------------------------------------------------------------------------------------
+// The update of int8 states of heads with one A each (Mamba2), for several batch entries at a time.  The bytes are few, so
+// arithmetic and set-up are what takes the time: a lane owns sixteen states in a row (one 16-byte load and store) of one
+// channel and walks `per` batch entries with everything that does not depend on them in registers - state scales and their
+// reciprocals, decay, skip weight, bias, the group lookup; B and C of an entry, the same for all channels of the head, are
+// scaled once per workgroup into LDS; the operands of the next entry are on their way while one is computed.  Same
+// expressions as ssm_update_body; only the order of a row's output sum differs.  A decode step of 64 sequences, 128 heads of 64
+// channels x 128 states, in_proj to out_proj: 186 us with the kernel above and its divisions, 140 with requantise4 and one
+// decay per lane, 104 with this one; 128 sequences 243 -> 168 from the second of these, one 31.9 -> 30.7.
+// ---------------------------------------------------------------------------------------------
+template <int LPR>
+__global__ __launch_bounds__(256) void ssm_update_heads_i8_kernel(QaSsmUpdateParams p, int per) {
+    constexpr int N = 16 * LPR;
+    __shared__ __attribute__((aligned(16))) float bc[2][2][N];
+    const int tid = threadIdx.x, gid = blockIdx.x * 256 + tid, sub = gid % LPR, hd = blockIdx.y;
+    const bool row_ok = gid / LPR < p.dim;
+    const int d = row_ok ? gid / LPR : p.dim - 1;
+    const int b0 = blockIdx.z * per, b1 = min(b0 + per, p.batch);
+    const int heads_per_group = p.nheads / p.ngroups, g = hd / heads_per_group;
+    const bool grouped = p.nhead_groups > 0;
+    int sidx = 0;
+    if (grouped) {
+        int hg = 0, dg = 0;
+        const int hrel = hd % heads_per_group;
+        for (int j = 0; j < p.nhead_groups; ++j) hg += hrel >= p.x_head_group_range[g * p.nhead_groups + j] ? 1 : 0;
+        hg = min(hg, p.nhead_groups - 1);
+        const int32_t* dr = p.x_dim_group_range + (g * p.nhead_groups + hg) * p.ndim_groups;
+        for (int j = 0; j < p.ndim_groups; ++j) dg += d >= dr[j] ? 1 : 0;
+        dg = min(dg, p.ndim_groups - 1);
+        sidx = (g * p.nhead_groups + hg) * p.ndim_groups + dg;
+    }
+    const float K = grouped ? 1e6f : 1e2f;
+    float sc[4][4], inv[4][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (grouped) __builtin_memcpy(sc[k], p.state_scale + static_cast<int64_t>(sidx) * N + 16 * sub + 4 * k, 16);
+        else sc[k][0] = sc[k][1] = sc[k][2] = sc[k][3] = *p.state_scale;
+    }
+    const float x_scale = p.x_scale[sidx], B_scale = p.B_scale[grouped ? g : 0], C_scale = p.C_scale[grouped ? g : 0];
+    const float dt_scale = *p.dt_scale, A_scale = *p.A_log_scale, z_scale = p.z ? *p.z_scale : 0.0f;
+    const float A = -__expf(A_scale * static_cast<float>(p.A_log[hd * p.A_head_stride + d * p.A_dim_stride]));
+    const int64_t bias_i = hd * p.dt_bias_head_stride + d * p.dt_bias_dim_stride;
+    float bias = 0.0f;
+    if (p.dt_bias) bias = p.dt_bias_is_fp16 ? __half2float(static_cast<const __half*>(p.dt_bias)[bias_i]) : *p.dt_bias_scale * static_cast<float>(static_cast<const int8_t*>(p.dt_bias)[bias_i]);
+    const float skip = p.D ? *p.D_scale * static_cast<float>(p.D[hd * p.D_head_stride + d * p.D_dim_stride]) : 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) inv[k][e] = __builtin_amdgcn_rcpf(sc[k][e] * K);
+
+    int8_t* const st0 = static_cast<int8_t*>(p.state) + hd * p.state_head_stride + d * p.state_dim_stride + 16 * sub;
+    const int8_t* const x0 = p.x + hd * p.x_head_stride + d * p.x_dim_stride;
+    const int8_t* const dt0 = p.dt + hd * p.dt_head_stride + d * p.dt_dim_stride;
+    const int8_t* const z0 = p.z ? p.z + hd * p.z_head_stride + d * p.z_dim_stride : x0;
+    const int64_t z_batch = p.z ? p.z_batch_stride : p.x_batch_stride;
+    // (threads past the 2 N codes of B and C read the last one)
+    const int code = min(tid, 2 * N - 1);
+    const int8_t* const bc0 = code < N ? p.B + g * p.B_group_stride + code : p.C + g * p.C_group_stride + (code - N);
+    const int64_t bc_batch = code < N ? p.B_batch_stride : p.C_batch_stride;
+    const float bc_scale = code < N ? B_scale : C_scale;
+
+    uint4 state, state_next;
+    int xq, dtq, zq, bcq, xn, dtn, zn, bcn;
+    auto load = [&](int64_t b, uint4& s, int& x, int& t, int& z, int& c) {
+        s = *reinterpret_cast<const uint4*>(st0 + b * p.state_batch_stride);
+        x = x0[b * p.x_batch_stride];
+        t = dt0[b * p.dt_batch_stride];
+        z = z0[b * z_batch];
+        c = bc0[b * bc_batch];
+    };
+    load(b0, state_next, xn, dtn, zn, bcn);
+    for (int b = b0; b < b1; ++b) {
+        state = state_next; xq = xn; dtq = dtn; zq = zn; bcq = bcn;
+        float* const turn = &bc[(b - b0) & 1][0][0];
+        if (tid < 2 * N) turn[tid] = bc_scale * static_cast<float>(bcq);
+        __syncthreads();                               // (the other copy: every wave left it before this barrier)
+        if (b + 1 < b1) load(b + 1, state_next, xn, dtn, zn, bcn);
+        const float xv = x_scale * static_cast<float>(xq);
+        float dt = dt_scale * static_cast<float>(dtq);
+        dt += bias;
+        if (p.dt_softplus) dt = softplus20_flat(dt);
+        const float dA = __expf(A * dt);
+        float acc = 0.0f;
+        const uint32_t word[4] = {state.x, state.y, state.z, state.w};
+        uint32_t out[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float4 Bq = *reinterpret_cast<const float4*>(&turn[16 * sub + 4 * k]), Cq = *reinterpret_cast<const float4*>(&turn[N + 16 * sub + 4 * k]);
+            const float Bv[4] = {Bq.x, Bq.y, Bq.z, Bq.w}, Cv[4] = {Cq.x, Cq.y, Cq.z, Cq.w};
+            float h[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                h[e] = sc[k][e] * code_byte_to_float(word[k], e);
+                h[e] = h[e] * dA + (Bv[e] * dt) * xv;
+                acc += h[e] * Cv[e];
+            }
+            out[k] = requantise4(h, sc[k], inv[k], K);
+        }
+        if (row_ok) *reinterpret_cast<uint4*>(st0 + b * p.state_batch_stride) = make_uint4(out[0], out[1], out[2], out[3]);
+#pragma unroll
+        for (int m = 1; m < LPR; m <<= 1) acc += __shfl_xor(acc, m);
+        if (row_ok && sub == 0) {
+            if (p.D) acc += xv * skip;
+            if (p.z) {
+                const float zv = z_scale * static_cast<float>(zq);
+                acc *= zv * (1.0f / (1.0f + expf(-zv)));
+            }
+            static_cast<__half*>(p.out)[b * p.out_batch_stride + hd * p.out_head_stride + d * p.out_dim_stride] = __float2half(acc);
+        }
+    }
+}
+
+// Whether that kernel takes an update, and how many batch entries a workgroup then walks: as many as leave the part four waves
+// per SIMD.
+template <int LPR>
+bool launch_heads_i8(const QaSsmUpdateParams& p, hipStream_t stream) {
+    auto mult16 = [](int64_t v) { return v % 16 == 0; };
+    if (p.state_is_fp32 || p.A_dstate_stride != 0 || p.dstate != 16 * LPR || p.state_dstate_stride != 1 || p.B_dstate_stride != 1 || p.C_dstate_stride != 1) return false;
+    if (!aligned16(p.state) || !mult16(p.state_batch_stride) || !mult16(p.state_head_stride) || !mult16(p.state_dim_stride)) return false;
+    const int64_t waves = static_cast<int64_t>(p.batch) * p.nheads * ((static_cast<int64_t>(p.dim) * LPR + 255) / 256) * 4;
+    const int per = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(waves / 4096, 8)));
+    const dim3 grid(static_cast<unsigned>((static_cast<int64_t>(p.dim) * LPR + 255) / 256), static_cast<unsigned>(p.nheads), static_cast<unsigned>((p.batch + per - 1) / per));
+    hipLaunchKernelGGL(ssm_update_heads_i8_kernel<LPR>, grid, dim3(256), 0, stream, p, per);
+    return true;
 }
 
 template <int LPR>
@@ -1165,8 +1321,11 @@ int launch_update(const QaSsmUpdateParams& p, hipStream_t stream, const QaConvPa
                                  !(p.dt_bias && p.dt_bias_is_fp16);
         if (dt) {
             if (!fast_update || dt->pieces > kSsmDtPieces || !aligned16(dt->w) || !aligned4(dt->x) || dt->x_batch_stride % 4 != 0) return QA_ERR_UNSUPPORTED;
-            if (p.state_is_fp32) hipLaunchKernelGGL(ssm_update_dt_kernel<true>, grid, dim3(256), 0, stream, p, *dt);
-            else hipLaunchKernelGGL(ssm_update_dt_kernel<false>, grid, dim3(256), 0, stream, p, *dt);
+            // a wave per workgroup: the rows' step size weights, 16 bytes a lane at a stride, are slow work for a CU's memory
+            // path, and few sequences have few waves
+            const dim3 waves(static_cast<unsigned>((p.dim + 63) / 64), 1, static_cast<unsigned>(p.batch));
+            if (p.state_is_fp32) hipLaunchKernelGGL(ssm_update_dt_kernel<true>, waves, dim3(64), 0, stream, p, *dt);
+            else hipLaunchKernelGGL(ssm_update_dt_kernel<false>, waves, dim3(64), 0, stream, p, *dt);
             return check_launch();
         }
         if (!conv && fast_update) {
@@ -1192,6 +1351,13 @@ int launch_update(const QaSsmUpdateParams& p, hipStream_t stream, const QaConvPa
         }
     }
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, p); };
+    if constexpr (LPR == 4 || LPR == 8) {
+        if (launch_heads_i8<LPR>(p, stream)) return check_launch();
+    }
+    if (vec && LPR > 1 && p.A_dstate_stride == 0) {
+        p.state_is_fp32 ? go(ssm_update_kernel<LPR, true, true, false, true>) : go(ssm_update_kernel<LPR, true, false, false, true>);
+        return check_launch();
+    }
     if (p.state_is_fp32) vec ? go(ssm_update_kernel<LPR, true, true>) : go(ssm_update_kernel<LPR, false, true>);
     else vec ? go(ssm_update_kernel<LPR, true, false>) : go(ssm_update_kernel<LPR, false, false>);
     return check_launch();
