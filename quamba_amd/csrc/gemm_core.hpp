@@ -282,15 +282,36 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The scales of a workgroup's tile, BN column scales and BM row scales, fetched into LDS in front of everything else: loaded
+// where they are used, they cost the end of every tile two memory round trips and, with a scale per column, 150 instructions
+// of addresses.  (One scale for all columns or rows is read into each of its places; rows and columns outside read zero.)
+template <int BM, int BN, int WAVES>
+struct TileScales {
+    static constexpr int kBytes = (BM + BN) * 4;
+    static_assert(BM % 64 == 0 || BM == 32, "whole requests");
+    // call once before the first tile's requests; complete with them
+    static __device__ __forceinline__ void request(uint32_t lds_addr, const float* row_scale, int row_numel, int m, int m0, const float* col_scale, int col_numel, int n, int n0, int wave, int lane) {
+        constexpr int kCols = BN / 64, kRows = (BM + 63) / 64;
+        const v4i rsrc_c = make_rsrc(col_scale, (col_numel == 1 ? 1 : n) * 4), rsrc_r = make_rsrc(row_scale, (row_numel == 1 ? 1 : m) * 4);
+#pragma unroll
+        for (int i = 0; i < kCols + kRows; ++i) {
+            if (i % WAVES != wave) continue;
+            if (i < kCols) buffer_load_lds_b32(rsrc_c, lds_addr + i * 256, col_numel == 1 ? 0 : (n0 + i * 64 + lane) * 4);
+            else buffer_load_lds_b32(rsrc_r, lds_addr + BN * 4 + (i - kCols) * 256, row_numel == 1 ? 0 : (m0 + (i - kCols) * 64 + lane) * 4);
+        }
+    }
+};
+
 // In acc[i][j] lane l holds output row m = j*32 + (l & 31) and, in register r, column
 // n = i*32 + 8*(r/4) + 4*(l/32) + (r%4).
 // FLEX = false compiles the common rule only (d = cast_rne(s_row * (s_col * acc))); FLEX = true also
 // honours use_alpha and the round-half-away GEMV rule at run time.  TRANS selects the (N,M) output.
 // COL_OUTER (the column scale applied last) is a compile-time choice: selecting the association per
 // element costs two extra instructions on each of the 128 outputs of a lane.
+// s_lds: the scales of the workgroup's tile in LDS (TileScales), this wave's first row and column at row_at and col_at.
 template <int TM, int TN, int OUT, bool FLEX, bool TRANS, bool COL_OUTER = false>
 __device__ __forceinline__ void epilogue(const Epilogue& e, v16i (&acc)[TN][TM], uint8_t* lds, int m, int n,
-                                         int wave_m0, int wave_n0, int wave, int lane) {
+                                         int wave_m0, int wave_n0, int wave, int lane, const float* s_lds, int row_at, int col_at) {
     constexpr int kElt = OUT == QA_OUT_I8 ? 1 : 2;
     const int frow = lane & 31, fhalf = lane >> 5;
     const bool vec_ok = (e.ldd * kElt) % 16 == 0 && aligned16(e.d);
@@ -298,34 +319,18 @@ __device__ __forceinline__ void epilogue(const Epilogue& e, v16i (&acc)[TN][TM],
     const bool away = FLEX && e.round_mode == QA_ROUND_HALF_AWAY;
     const int round_mode = FLEX ? e.round_mode : QA_ROUND_RNE;
 
-    // this lane's column scales: 4 consecutive columns per (i, q), loaded once
+    // this lane's column scales: 4 consecutive columns per (i, q)
     float s_col[TN][4][4];
-    if (use_alpha || e.col_numel == 1) {
-        // one scale for every column: a single (scalar) fetch instead of one per column and lane
-        const float one = use_alpha ? 1.0f : e.col_scale[0];
 #pragma unroll
-        for (int i = 0; i < TN; ++i)
+    for (int i = 0; i < TN; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) s_col[i][q][t] = one;
-    } else {
-#pragma unroll
-        for (int i = 0; i < TN; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int nn = wave_n0 + i * 32 + 8 * q + 4 * fhalf + t;
-                    s_col[i][q][t] = e.col_scale[min(nn, n - 1)];
-                }
-    }
+        for (int q = 0; q < 4; ++q) {
+            const float4 v = *reinterpret_cast<const float4*>(s_lds + col_at + i * 32 + 8 * q + 4 * fhalf);
+            s_col[i][q][0] = v.x; s_col[i][q][1] = v.y; s_col[i][q][2] = v.z; s_col[i][q][3] = v.w;
+        }
     float s_row[TM];
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-        const int mm = wave_m0 + j * 32 + frow;
-        s_row[j] = use_alpha ? e.alpha : e.row_scale[e.row_numel == 1 ? 0 : min(mm, m - 1)];
-    }
+    for (int j = 0; j < TM; ++j) s_row[j] = use_alpha ? e.alpha : s_lds[row_at + j * 32 + frow];
     auto scaled = [&](int i, int j, int q, int t) -> float {
         const float accf = static_cast<float>(acc[i][j][q * 4 + t]);
         float v;
@@ -342,6 +347,10 @@ __device__ __forceinline__ void epilogue(const Epilogue& e, v16i (&acc)[TN][TM],
     if (!TRANS) {
         constexpr int kPitch = TN * 32 * kElt + 16;
         uint8_t* stg = lds + wave * (32 * kPitch);
+        // a tile that lies inside the output altogether: no bounds to look at, 32-bit offsets from one address
+        const bool whole = vec_ok && wave_m0 + TM * 32 <= m && wave_n0 + TN * 32 <= n && e.ldd * kElt < (1 << 23);
+        uint8_t* const first = static_cast<uint8_t*>(e.d) + (static_cast<int64_t>(wave_m0) * e.ldd + wave_n0) * kElt;
+        const uint32_t row_bytes = static_cast<uint32_t>(e.ldd * kElt);
 #pragma unroll
         for (int j = 0; j < TM; ++j) {
 #pragma unroll
@@ -371,6 +380,15 @@ __device__ __forceinline__ void epilogue(const Epilogue& e, v16i (&acc)[TN][TM],
             }
             wave_lds_sync();
             constexpr int kPiecesPerRow = TN * 32 * kElt / 16;
+            if (whole) {
+#pragma unroll
+                for (int piece = lane; piece < 32 * kPiecesPerRow; piece += 64) {
+                    const uint32_t r = piece / kPiecesPerRow, cb = (piece % kPiecesPerRow) * 16;
+                    *reinterpret_cast<uint4*>(first + ((j * 32 + r) * row_bytes + cb)) = *reinterpret_cast<const uint4*>(stg + r * kPitch + cb);
+                }
+                wave_lds_sync();
+                continue;
+            }
 #pragma unroll
             for (int piece = lane; piece < 32 * kPiecesPerRow; piece += 64) {
                 const int r = piece / kPiecesPerRow, cb = (piece % kPiecesPerRow) * 16;

@@ -42,7 +42,8 @@ struct W4Cfg {
     static constexpr int kSlots = STAGES - 1;                      // tiles of packed weights
     static constexpr int kABytes = C::kBM * kBK, kWBytes = C::kBN * kBK;
     static constexpr int kPackedBytes = C::kBN * (kBK / 2), kScaleBytes = kWPacked * C::kThreads * 4;
-    static constexpr int kLdsBytes = STAGES * kABytes + 2 * kWBytes + kSlots * (kPackedBytes + kScaleBytes);
+    static constexpr int kScalesAt = STAGES * kABytes + 2 * kWBytes + kSlots * (kPackedBytes + kScaleBytes);
+    static constexpr int kLdsBytes = kScalesAt + TileScales<C::kBM, C::kBN, C::kWaves>::kBytes;
 };
 
 template <int TM, int TN, int WGM, int WGN, int STAGES, bool GROUPED, int OUT>
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
     using W = W4Cfg<TM, TN, WGM, WGN, STAGES>;
     using C = typename W::C;
     constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves, THREADS = C::kThreads, kWPacked = W::kWPacked;
-    static_assert(kWPacked * THREADS == BN * 4 && epilogue_lds_bytes<TM, TN, WAVES>() <= W::kLdsBytes, "tile shape");
+    static_assert(kWPacked * THREADS == BN * 4 && epilogue_lds_bytes<TM, TN, WAVES>() <= W::kScalesAt, "tile shape");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
     const int tid = threadIdx.x;
@@ -64,6 +65,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
     const int k_tiles = p.k / kBK, ldw = p.k / 2;
 
     const uint32_t lds_base = lds_offset_of(lds);
+    TileScales<BM, BN, WAVES>::request(lds_base + W::kScalesAt, p.s_token, p.tok_scale_numel, p.m, m0, p.s_channel, p.n, p.n, n0, wave, lane);
     constexpr int kAtW = STAGES * W::kABytes, kAtPacked = kAtW + 2 * W::kWBytes, kAtScale = kAtPacked + W::kSlots * W::kPackedBytes;
     const v4i rsrc_a = make_rsrc(p.a, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k));
     const v4i rsrc_w = make_rsrc(p.w_packed + static_cast<int64_t>(n0) * ldw, min(BN, p.n - n0) * ldw);
@@ -183,11 +185,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
     __syncthreads();
 
     Epilogue e;
-    e.row_scale = p.s_token; e.col_scale = p.s_channel;
-    e.row_numel = p.tok_scale_numel; e.col_numel = p.n;
     e.use_alpha = 0; e.alpha = 0.0f; e.round_mode = QA_ROUND_RNE; e.col_outer = 0;
     e.ldd = p.ldd; e.d = p.d;
-    epilogue<TM, TN, OUT, false, false>(e, acc, lds, p.m, p.n, m0 + wm * TM * 32, n0 + wn * TN * 32, wave, lane);
+    epilogue<TM, TN, OUT, false, false>(e, acc, lds, p.m, p.n, m0 + wm * TM * 32, n0 + wn * TN * 32, wave, lane,
+                                          reinterpret_cast<const float*>(lds + W::kScalesAt), BN + wm * TM * 32, wn * TN * 32);
 }
 
 template <int OUT>
@@ -228,7 +229,8 @@ struct RegCfg {
     // what a row's 16-byte pieces are exchanged by: sixteen neighbouring rows of one column of pieces then cover all banks
     __device__ static __forceinline__ int exchange(int row) { return KT == 256 ? row & 15 : (row >> 1) & 7; }
     static constexpr int kEpilogue = epilogue_lds_bytes<TM, 1, NW>();
-    static constexpr int kLdsBytes = 2 * kABytes > kEpilogue ? 2 * kABytes : kEpilogue;
+    static constexpr int kScalesAt = 2 * kABytes > kEpilogue ? 2 * kABytes : kEpilogue;
+    static constexpr int kLdsBytes = kScalesAt + TileScales<kBM, kBN, NW>::kBytes;
 };
 
 template <int TM, int NW, int KT, bool GROUPED, int OUT, bool TRANS>
@@ -251,6 +253,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4a8_reg_kernel(QaGemmW4A8Params
     // activations: request j of a wave fills LDS bytes [(j NW + wave) 1024, + 1024) of the tile, i.e. 1024 / KT rows
     const v4i rsrc_a = make_rsrc(p.a, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k));
     const uint32_t lds_a = lds_offset_of(lds);
+    TileScales<R::kBM, R::kBN, NW>::request(lds_a + R::kScalesAt, p.s_token, p.tok_scale_numel, p.m, m0, p.s_channel, p.n, p.n, tile_n * R::kBN, wave, lane);
     int a_off[R::kAInstr], a_k[R::kAInstr];
 #pragma unroll
     for (int j = 0; j < R::kAInstr; ++j) {
@@ -351,11 +354,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4a8_reg_kernel(QaGemmW4A8Params
     __syncthreads();
 
     Epilogue e;
-    e.row_scale = p.s_token; e.col_scale = p.s_channel;
-    e.row_numel = p.tok_scale_numel; e.col_numel = p.n;
     e.use_alpha = 0; e.alpha = 0.0f; e.round_mode = QA_ROUND_RNE; e.col_outer = 0;
     e.ldd = p.ldd; e.d = p.d;
-    epilogue<TM, 1, OUT, false, TRANS>(e, acc, lds, p.m, p.n, m0, n0, wave, lane);
+    epilogue<TM, 1, OUT, false, TRANS>(e, acc, lds, p.m, p.n, m0, n0, wave, lane, reinterpret_cast<const float*>(lds + R::kScalesAt), R::kBN, wave * 32);
 }
 
 template <int TM, int NW, int KT, int OUT, bool TRANS>

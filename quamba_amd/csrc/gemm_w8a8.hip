@@ -57,6 +57,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
     const v4i rsrc_w = make_rsrc(p.w, static_cast<int>((static_cast<int64_t>(p.n) - 1) * p.ldw + p.k));
     const uint32_t lds_base = lds_offset_of(lds);
 
+    using Scales = TileScales<BM, BN, WAVES>;
+    if (!p.use_alpha) Scales::request(lds_base + C::kLdsBytes, p.a_scale, p.a_scale_numel, p.m, m0, p.w_scale, p.w_scale_numel, p.n, n0, wave, lane);
     TileLoader<C::kAInstr> load_a;
     TileLoader<C::kWInstr> load_w;
     load_a.template init<WAVES>(m0, p.m, p.lda, wave, lane);
@@ -140,11 +142,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
     CLK_MARK(2);
 
     Epilogue e;
-    e.row_scale = p.a_scale; e.col_scale = p.w_scale;
-    e.row_numel = p.a_scale_numel; e.col_numel = p.w_scale_numel;
     e.use_alpha = p.use_alpha; e.alpha = p.alpha; e.round_mode = p.round_mode; e.col_outer = p.scale_order;
     e.ldd = p.ldd; e.d = p.d;
-    epilogue<TM, TN, OUT, FLEX, false, COL_OUTER>(e, acc, lds, p.m, p.n, m0 + wm * TM * 32, n0 + wn * TN * 32, wave, lane);
+    epilogue<TM, TN, OUT, FLEX, false, COL_OUTER>(e, acc, lds, p.m, p.n, m0 + wm * TM * 32, n0 + wn * TN * 32, wave, lane,
+                                                  reinterpret_cast<const float*>(lds + C::kLdsBytes), BN + wm * TM * 32, wn * TN * 32);
     CLK_MARK(3);
 }
 
@@ -157,14 +158,15 @@ int launch_one(const QaGemmW8A8Params& p, hipStream_t stream) {
     const int64_t tiles = static_cast<int64_t>((p.m + C::kBM - 1) / C::kBM) * ((p.n + C::kBN - 1) / C::kBN);
     if (tiles > 0x7fffffffLL) return QA_ERR_SHAPE;
     auto kernel = gemm_w8a8_kernel<TM, TN, WGM, WGN, STAGES, OUT, FLEX, COL_OUTER>;
-    if (C::kLdsBytes > 65536) {
+    constexpr int kLds = C::kLdsBytes + TileScales<C::kBM, C::kBN, C::kWaves>::kBytes;
+    if (kLds > 65536) {
         // allowing more than 64 KiB of dynamic LDS is a per-function attribute; setting it is idempotent
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                C::kLdsBytes) != hipSuccess) {
+                                kLds) != hipSuccess) {
             return check_launch();
         }
     }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(C::kThreads), C::kLdsBytes, stream, p);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(C::kThreads), kLds, stream, p);
     return check_launch();
 }
 
