@@ -319,6 +319,9 @@ int dispatch_skinny(const QaGemmW8A8Params& p, hipStream_t stream) {
 // starts.  Measured at M 16 .. 16384 with ten of the projections' N and K: this choice is the fastest or
 // within 8 % of it.  Against 128 x 128 tiles up to 192 tiles of 256 x 256 (rows x outputs x K, us): 512 x 80 x 1536 9.6 ->
 // 4.1, 3063 x 192 x 5120 21.0 -> 11.7, 512 x 1536 x 3072 14.6 -> 7.7, 777 x 10240 x 2560 45 -> 38, 6144 x 1536 x 3072 47 -> 35.
+// From 128 x 64 on a tile is divided over eight waves: a CU that holds one tile then has two waves per SIMD, and one issues
+// while the other waits.  Four waves against eight (us): 1531 x 768 x 1536 6.9 -> 6.3, 1024 x 1536 x 3072 10.2 -> 9.8 with
+// 128 x 64; 3063 x 768 x 1536 9.2 -> 7.8, 1531 x 1536 x 3072 14.0 -> 12.1, 1531 x 2560 x 5120 28.0 -> 27.8 with 128 x 128.
 int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -328,8 +331,8 @@ int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
     auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
     if (tiles(32, 32) <= cus) return dispatch_skinny<false>(p, stream);
     if (tiles(64, 64) <= cus) return launch_gemm<1, 1, 2, 2, 4, false>(p, stream);
-    if (tiles(128, 64) <= cus) return launch_gemm<2, 1, 2, 2, 4, false>(p, stream);
-    if (tiles(128, 128) <= cus) return launch_gemm<2, 2, 2, 2, 4, false>(p, stream);
+    if (tiles(128, 64) <= cus) return launch_gemm<1, 1, 4, 2, 4, false>(p, stream);
+    if (tiles(128, 128) <= cus) return launch_gemm<2, 1, 2, 4, 4, false>(p, stream);
     if (tiles(128, 256) <= cus) return launch_gemm<2, 2, 2, 4, 3, false>(p, stream);
     // More than a round: what counts is rounds times the tile's work (128 x 256 at six fifths of its share).
     auto cost = [&](int64_t bm, int64_t bn) { return ((tiles(bm, bn) + cus - 1) / cus) * bm * bn; };
