@@ -69,19 +69,44 @@ __device__ __forceinline__ int ssd_dim_group_of(const QaSsdParams& p, int g, int
     for (int j = 0; j < p.ndim_groups; ++j) dg += ch >= dr[j] ? 1 : 0;
     return min(dg, p.ndim_groups - 1);
 }
-__device__ __forceinline__ float ssd_x_scale_of(const QaSsdParams& p, int g, int hg, int ch) {
-    if (p.nhead_groups == 0) return p.x_scale[0];
-    return p.x_scale[(g * p.nhead_groups + hg) * p.ndim_groups + ssd_dim_group_of(p, g, hg, ch)];
-}
 
-// The per-channel tables: called by the wave that handles (batch 0, chunk 0, head h) in the first kernel.
-// srow: index of the first state's scale in state_scale for this channel (0 with one scale for everything)
+// The per-channel tables of head h, written by one whole wave of the first kernel (h is the same in all its lanes).
+// srow: index of the first state's scale in state_scale for this channel (0 with one scale for everything).
+// The bounds of the groups come from memory once, a bound per lane, and are compared out of registers: a walk that loads
+// one bound after another waits for memory at every step, which was longer than the rest of that kernel.
 __device__ __forceinline__ void ssd_write_channel_tables(const QaSsdParams& p, int h, int lane, float* xs_out, int32_t* srow_out) {
+    if (p.nhead_groups == 0) {
+        const float xs = p.x_scale[0];
+        for (int ch = lane; ch < p.headdim; ch += 64) {
+            xs_out[h * p.headdim + ch] = xs;
+            srow_out[h * p.headdim + ch] = 0;
+        }
+        return;
+    }
     int g, hg;
-    ssd_group_of(p, h, g, hg);
-    for (int ch = lane; ch < p.headdim; ch += 64) {
-        xs_out[h * p.headdim + ch] = ssd_x_scale_of(p, g, hg, ch);
-        srow_out[h * p.headdim + ch] = p.nhead_groups > 0 ? ((g * p.nhead_groups + hg) * p.ndim_groups + ssd_dim_group_of(p, g, hg, ch)) * p.dstate : 0;
+    const int hpg = p.nheads / p.ngroups;
+    if (p.nhead_groups <= 64) {
+        g = h / hpg;
+        const int bound = lane < p.nhead_groups ? p.x_head_group_range[g * p.nhead_groups + lane] : 0;
+        hg = min(__popcll(__ballot(lane < p.nhead_groups && h % hpg >= bound)), p.nhead_groups - 1);
+    } else {
+        ssd_group_of(p, h, g, hg);
+    }
+    const int group = (g * p.nhead_groups + hg) * p.ndim_groups;
+    const int bound = lane < p.ndim_groups ? p.x_dim_group_range[group + lane] : 0;
+    for (int ch0 = 0; ch0 < p.headdim; ch0 += 64) {
+        const int ch = ch0 + lane;
+        int dg = 0;
+        if (p.ndim_groups <= 64) {
+            for (int j = 0; j < p.ndim_groups; ++j) dg += ch >= __builtin_amdgcn_readlane(bound, j) ? 1 : 0;
+            dg = min(dg, p.ndim_groups - 1);
+        } else if (ch < p.headdim) {
+            dg = ssd_dim_group_of(p, g, hg, ch);
+        }
+        if (ch < p.headdim) {
+            xs_out[h * p.headdim + ch] = p.x_scale[group + dg];
+            srow_out[h * p.headdim + ch] = (group + dg) * p.dstate;
+        }
     }
 }
 
