@@ -3,7 +3,8 @@
 //   acc[m,n] = sum_k a[m,k] * w[n,k]   (int32)      a: (M,K) int8, K-contiguous
 //   d[m,n]   = cast(s_row[m|0] * (s_col[n|0] * float(acc)))          w: (N,K) int8, K-contiguous (W8A8)
 //                                                                       or 4-bit codes + group scales (W4A8)
-// Structure: WGM x WGN waves per workgroup, each wave TM x TN tiles of v_mfma_i32_32x32x32_i8; block
+// Structure: WGM x WGN waves per workgroup, each wave TM x TN blocks of 32 x 32 (v_mfma_i32_32x32x32_i8, or
+// v_mfma_i32_16x16x64_i8 in the two-stage main loop of the large tiles, see RotatedMma); block
 // tile (WGM*TM*32) x (WGN*TN*32) x 128 k-bytes.  The k extent of 128 bytes is one full cache line
 // per operand row: measured on MI355X, 64-byte row pieces halve the L1 load rate.  Operand tiles live
 // in LDS as rows of eight 16-byte chunks, the chunk index XOR-swizzled with bits 1..3 of the row
@@ -179,6 +180,11 @@ struct TileLoader {
         const int off = (k0 + kc[j] < k_end) ? voff[j] + k0 : 0x7ffffff0;
         buffer_load_lds_b128(rsrc, dst + (j * WAVES + wave) * 1024, off);
     }
+    // a tile whose 128 bytes all lie inside K
+    template <int WAVES>
+    __device__ __forceinline__ void issue_whole(int j, v4i rsrc, int k0, uint32_t dst, int wave) const {
+        buffer_load_lds_b128(rsrc, dst + (j * WAVES + wave) * 1024, voff[j], k0);
+    }
     template <int WAVES>
     __device__ __forceinline__ void issue(v4i rsrc, int k0, int k_end, uint32_t dst, int wave) const {
 #pragma unroll
@@ -239,40 +245,82 @@ __device__ __forceinline__ void mma_tile_paced(const uint8_t* sa, const uint8_t*
     }
 }
 
-// One k tile of a main loop whose workgroup barrier sits before the last k step instead of between tiles.  On entry
-// the fragments of k step 0 of the tile at `sa`/`sw` are in fa[0]/fw[0].  Steps 0..2 fetch the fragments of the step
-// after them; before the multiplications of step 3 the wave waits for its own global -> LDS requests, meets the
-// others at the barrier - every wave then holds all fragments of this tile, so this stage may be overwritten, and
-// the next tile's stage is complete - and fetches step 0 of the next tile from `na`/`nw`.  The matrix pipe has the
-// multiplications of step 3 queued behind the barrier, so it does not drain while the first fragments of the next
-// tile travel.  `hook(idx)` runs after every multiplication, idx counted from the barrier: 0 .. TM*TN-1 during
-// step 3 of this tile, the following 3*TM*TN during steps 0..2 of the next one; the caller places its global ->
-// LDS requests behind the multiplications it chooses (a hook that does nothing costs nothing).
-template <int TM, int TN, class Hook>
-__device__ __forceinline__ void mma_tile_rotated(const uint8_t* sa, const uint8_t* sw, const uint8_t* na, const uint8_t* nw,
-                                                 int frow, int fhalf, v4i (&fa)[2][TM], v4i (&fw)[2][TN],
-                                                 v16i (&acc)[TN][TM], Hook&& hook) {
+// The main loop of the large tiles, on v_mfma_i32_16x16x64_i8.  These launches run at the power limit of the part - their
+// clock is what the energy of a multiplication leaves - and registers full of random int8 operands multiply at 4.0 POP/s
+// with this shape against 3.3 with 32x32x32 (both 4.9 with zeros): half as many accumulators are read and written per product.
+//
+// A k tile of 128 bytes is two steps of 64.  Of the two operands' fragments (16 rows x 64 bytes) a wave keeps the smaller
+// set, `held`, for a whole step and walks through the other one, a fragment at a time with all held ones: `Walk` is true when
+// the w operand is walked.  A walked fragment is fetched three positions ahead into a ring of four, the held ones of the next
+// step during the last three positions of a step, each fetch behind a multiplication of its own - fetched in a block
+// between the steps they left the matrix pipe idle (256 x 256 tiles, K 8192: 158900 -> 144000 cycles).  The barrier
+// stands where the last fetch from this tile's stage has been made, three positions before the end: there the wave waits for its own
+// global -> LDS requests and meets the others, so the next tile's stage is complete and this one may be overwritten.
+// `hook(idx)` runs after every multiplication, idx counted from the barrier, through kPerTile; the caller places its
+// requests behind the multiplications it chooses.
+// Against 32x32x32 with block fetches (rows x outputs x K, us): 16384 x 18560 x 4096 1030 -> 965, 16384 x 4096 x 8192
+// 434 -> 388, 16384 x 10240 x 2560 375 -> 333.  Four waves of 128 x 128 instead of eight of 128 x 64 or so read a third less from
+// LDS, but one wave per SIMD does not hide its own requests: 520 us where the eight take 388.
+template <int TM, int TN>
+struct RotatedMma {
+    static constexpr bool kWalkW = TN > TM;
+    static constexpr int kHeld = 2 * (kWalkW ? TM : TN), kWalk = 2 * (kWalkW ? TN : TM), kRing = 4, kAhead = 3;
+    static constexpr int kPerTile = 2 * kWalk * kHeld, kBehindBarrier = kAhead * kHeld;     // multiplications
+    static_assert(2 * kWalk % kRing == 0 && kHeld <= kAhead * (kHeld - 1), "");
+    v4i acc[2 * TN][2 * TM];      // lane l: row 16 j + (l & 15), columns 16 i + 4 (l >> 4) + 0..3
+    v4i held[2][kHeld], ring[kRing];
+    int at;                       // this lane's 16 bytes of fragment 0, step 0, in a stage's rows
+
+    __device__ __forceinline__ void init(int lane) {
+        at = (lane & 15) * kBK + swz(lane & 15, lane >> 4) * 16;
 #pragma unroll
-    for (int kk = 0; kk < kBK / 32; ++kk) {
-        if (kk + 1 < kBK / 32) {
-            fetch_fragments<TM, TN>(sa, sw, kk + 1, frow, fhalf, fa[(kk + 1) & 1], fw[(kk + 1) & 1]);
-        } else {
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-            __syncthreads();
-            fetch_fragments<TM, TN>(na, nw, 0, frow, fhalf, fa[0], fw[0]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < 2 * TN; ++i)
 #pragma unroll
-        for (int i = 0; i < TN; ++i)
+            for (int j = 0; j < 2 * TM; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+    }
+    // step 1 is four chunks further, which the swizzle turns into an exchange of bit 6
+    __device__ __forceinline__ v4i fragment(const uint8_t* rows, int step, int f) const {
+        return *reinterpret_cast<const v4i*>(rows + ((at ^ (step * 64)) + f * 16 * kBK));
+    }
+    // sa / sw: this wave's rows of the first tile's stage
+    __device__ __forceinline__ void start(const uint8_t* sa, const uint8_t* sw) {
 #pragma unroll
-            for (int j = 0; j < TM; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[kk & 1][i], fa[kk & 1][j], acc[i][j], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-                hook(((kk + 1) % (kBK / 32)) * (TM * TN) + i * TM + j);
+        for (int h = 0; h < kHeld; ++h) held[0][h] = fragment(kWalkW ? sa : sw, 0, h);
+#pragma unroll
+        for (int g = 0; g < kAhead; ++g) ring[g] = fragment(kWalkW ? sw : sa, 0, g);
+    }
+    template <class Hook>
+    __device__ __forceinline__ void tile(const uint8_t* sa, const uint8_t* sw, const uint8_t* na, const uint8_t* nw, Hook&& hook) {
+        const uint8_t* const h0 = kWalkW ? sa : sw;
+        const uint8_t* const h1 = kWalkW ? na : nw;
+        const uint8_t* const w0 = kWalkW ? sw : sa;
+        const uint8_t* const w1 = kWalkW ? nw : na;
+#pragma unroll
+        for (int g = 0; g < 2 * kWalk; ++g) {
+            const int step = g / kWalk, pos = g % kWalk, from_end = kWalk - pos;
+            if (g == 2 * kWalk - kAhead) {
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+                __syncthreads();
                 __builtin_amdgcn_sched_barrier(0);
             }
+#pragma unroll
+            for (int h = 0; h < kHeld; ++h) {
+                v4i& c = kWalkW ? acc[pos][h] : acc[h][pos];
+                c = __builtin_amdgcn_mfma_i32_16x16x64_i8(kWalkW ? ring[g % kRing] : held[step][h], kWalkW ? held[step][h] : ring[g % kRing], c, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (h == 0) {
+                    const int n = g + kAhead;
+                    ring[n % kRing] = n < 2 * kWalk ? fragment(w0, n / kWalk, n % kWalk) : fragment(w1, 0, n - 2 * kWalk);
+                } else if (from_end <= kAhead) {
+                    const int f = (kAhead - from_end) * (kHeld - 1) + h - 1;
+                    if (f < kHeld) held[1 - step][f] = step == 0 ? fragment(h0, 1, f) : fragment(h1, 0, f);
+                }
+                hook((g * kHeld + h + kBehindBarrier) % kPerTile);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
     }
-}
+};
 
 // Orders this wave's LDS writes before its later LDS reads (the staging area is private to the
 // wave, and one wave's LDS operations execute in order, so no workgroup barrier is needed).
@@ -302,49 +350,57 @@ struct TileScales {
     }
 };
 
-// In acc[i][j] lane l holds output row m = j*32 + (l & 31) and, in register r, column
-// n = i*32 + 8*(r/4) + 4*(l/32) + (r%4).
+// Accumulators as the two matrix instructions leave them, seen as quads: in quad u of row block b a lane holds four
+// consecutive output columns, from column_of(u), of row row_of() of the block.  Of 32x32x32: acc[i][j], row l & 31 of block
+// j, columns i*32 + 8*(r/4) + 4*(l/32) + (r%4) in register r; of 16x16x64: acc[i][j], row l & 15, columns i*16 + 4*(l/16) + r.
+template <class V>
+struct QuadView {
+    static constexpr int kRows = sizeof(V) == 16 ? 16 : 32, kQuadsPer = sizeof(V) / 16;
+    template <int NI, int NJ>
+    static __device__ __forceinline__ float value(const V (&acc)[NI][NJ], int u, int b, int t) { return static_cast<float>(acc[u / kQuadsPer][b][u % kQuadsPer * 4 + t]); }
+    static __device__ __forceinline__ int row_of(int lane) { return lane & (kRows - 1); }
+    static __device__ __forceinline__ int column_of(int u, int lane) { return kRows == 16 ? u * 16 + 4 * (lane >> 4) : u / 4 * 32 + 8 * (u % 4) + 4 * (lane >> 5); }
+};
+
 // FLEX = false compiles the common rule only (d = cast_rne(s_row * (s_col * acc))); FLEX = true also
 // honours use_alpha and the round-half-away GEMV rule at run time.  TRANS selects the (N,M) output.
 // COL_OUTER (the column scale applied last) is a compile-time choice: selecting the association per
 // element costs two extra instructions on each of the 128 outputs of a lane.
 // s_lds: the scales of the workgroup's tile in LDS (TileScales), this wave's first row and column at row_at and col_at.
-template <int TM, int TN, int OUT, bool FLEX, bool TRANS, bool COL_OUTER = false>
-__device__ __forceinline__ void epilogue(const Epilogue& e, v16i (&acc)[TN][TM], uint8_t* lds, int m, int n,
+template <int TM, int TN, int OUT, bool FLEX, bool TRANS, bool COL_OUTER = false, class V, int NI, int NJ>
+__device__ __forceinline__ void epilogue(const Epilogue& e, V (&acc)[NI][NJ], uint8_t* lds, int m, int n,
                                          int wave_m0, int wave_n0, int wave, int lane, const float* s_lds, int row_at, int col_at) {
-    constexpr int kElt = OUT == QA_OUT_I8 ? 1 : 2;
-    const int frow = lane & 31, fhalf = lane >> 5;
+    using Q = QuadView<V>;
+    constexpr int kElt = OUT == QA_OUT_I8 ? 1 : 2, kQuads = TN * 32 / (256 / Q::kRows) , kRowBlocks = TM * 32 / Q::kRows;
+    static_assert(NI * Q::kQuadsPer == kQuads && NJ == kRowBlocks, "accumulators of another tile");
     const bool vec_ok = (e.ldd * kElt) % 16 == 0 && aligned16(e.d);
     const bool use_alpha = FLEX && e.use_alpha;
     const bool away = FLEX && e.round_mode == QA_ROUND_HALF_AWAY;
     const int round_mode = FLEX ? e.round_mode : QA_ROUND_RNE;
 
-    // this lane's column scales: 4 consecutive columns per (i, q)
-    float s_col[TN][4][4];
+    float s_col[kQuads][4];
 #pragma unroll
-    for (int i = 0; i < TN; ++i)
+    for (int u = 0; u < kQuads; ++u) {
+        const float4 v = *reinterpret_cast<const float4*>(s_lds + col_at + Q::column_of(u, lane));
+        s_col[u][0] = v.x; s_col[u][1] = v.y; s_col[u][2] = v.z; s_col[u][3] = v.w;
+    }
+    float s_row[kRowBlocks];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 v = *reinterpret_cast<const float4*>(s_lds + col_at + i * 32 + 8 * q + 4 * fhalf);
-            s_col[i][q][0] = v.x; s_col[i][q][1] = v.y; s_col[i][q][2] = v.z; s_col[i][q][3] = v.w;
-        }
-    float s_row[TM];
-#pragma unroll
-    for (int j = 0; j < TM; ++j) s_row[j] = use_alpha ? e.alpha : s_lds[row_at + j * 32 + frow];
-    auto scaled = [&](int i, int j, int q, int t) -> float {
-        const float accf = static_cast<float>(acc[i][j][q * 4 + t]);
+    for (int b = 0; b < kRowBlocks; ++b) s_row[b] = use_alpha ? e.alpha : s_lds[row_at + b * Q::kRows + Q::row_of(lane)];
+    auto scaled = [&](int u, int b, int t) -> float {
+        const float accf = Q::value(acc, u, b, t);
         float v;
-        if (use_alpha) v = s_row[j] * accf;
+        if (use_alpha) v = s_row[b] * accf;
         // GEMV rule (round-half-away mode): the two scales are multiplied first
-        else if (COL_OUTER) v = s_col[i][q][t] * (s_row[j] * accf);
-        else v = away ? (s_col[i][q][t] * s_row[j]) * accf : s_row[j] * (s_col[i][q][t] * accf);
+        else if (COL_OUTER) v = s_col[u][t] * (s_row[b] * accf);
+        else v = away ? (s_col[u][t] * s_row[b]) * accf : s_row[b] * (s_col[u][t] * accf);
         // keep the fp32 product a value of its own: folding the multiply into a mixed-precision
         // convert would round once instead of twice and change the fp16 result in rare cases
         asm volatile("" : "+v"(v));
         return v;
     };
 
-    if (!TRANS) {
+    if constexpr (!TRANS) {
         constexpr int kPitch = TN * 32 * kElt + 16;
         uint8_t* stg = lds + wave * (32 * kPitch);
         // a tile that lies inside the output altogether: no bounds to look at, 32-bit offsets from one address
@@ -354,12 +410,13 @@ __device__ __forceinline__ void epilogue(const Epilogue& e, v16i (&acc)[TN][TM],
 #pragma unroll
         for (int j = 0; j < TM; ++j) {
 #pragma unroll
-            for (int i = 0; i < TN; ++i) {
+            for (int sub = 0; sub < 32 / Q::kRows; ++sub) {
+                const int b = j * (32 / Q::kRows) + sub, row = sub * Q::kRows + Q::row_of(lane);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int nl = i * 32 + 8 * q + 4 * fhalf;
-                    const float v0 = scaled(i, j, q, 0), v1 = scaled(i, j, q, 1);
-                    const float v2 = scaled(i, j, q, 2), v3 = scaled(i, j, q, 3);
+                for (int u = 0; u < kQuads; ++u) {
+                    const int nl = Q::column_of(u, lane);
+                    const float v0 = scaled(u, b, 0), v1 = scaled(u, b, 1);
+                    const float v2 = scaled(u, b, 2), v3 = scaled(u, b, 3);
                     if (OUT == QA_OUT_I8) {
                         uint32_t word;
                         if (!away) {
@@ -369,12 +426,12 @@ __device__ __forceinline__ void epilogue(const Epilogue& e, v16i (&acc)[TN][TM],
                             const uint32_t b2 = quant8(v2, round_mode) & 0xff, b3 = quant8(v3, round_mode);
                             word = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
                         }
-                        *reinterpret_cast<uint32_t*>(stg + frow * kPitch + nl) = word;
+                        *reinterpret_cast<uint32_t*>(stg + row * kPitch + nl) = word;
                     } else {
                         uint2 pk;
                         pk.x = pack2_f16_or_bf16<OUT>(v0, v1);
                         pk.y = pack2_f16_or_bf16<OUT>(v2, v3);
-                        *reinterpret_cast<uint2*>(stg + frow * kPitch + nl * 2) = pk;
+                        *reinterpret_cast<uint2*>(stg + row * kPitch + nl * 2) = pk;
                     }
                 }
             }
@@ -409,6 +466,8 @@ __device__ __forceinline__ void epilogue(const Epilogue& e, v16i (&acc)[TN][TM],
         }
     } else {
         // transposed output d[n][m]: stage 32 columns n x (TM*32) rows m per pass
+        static_assert(Q::kRows == 32, "only of 32x32x32");
+        const int frow = lane & 31, fhalf = lane >> 5;
         constexpr int kPitch = TM * 32 * kElt + 16;
         uint8_t* stg = lds + wave * (32 * kPitch);
 #pragma unroll
@@ -420,7 +479,7 @@ __device__ __forceinline__ void epilogue(const Epilogue& e, v16i (&acc)[TN][TM],
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
                         const int nl = 8 * q + 4 * fhalf + t;          // column inside this 32-column tile
-                        const float v = scaled(i, j, q, t);
+                        const float v = scaled(i * 4 + q, j, t);
                         if (OUT == QA_OUT_I8) {
                             *reinterpret_cast<int8_t*>(stg + nl * kPitch + j * 32 + frow) =
                                 static_cast<int8_t>(quant8(v, round_mode));

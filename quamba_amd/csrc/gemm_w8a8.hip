@@ -64,25 +64,27 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
     load_a.template init<WAVES>(m0, p.m, p.lda, wave, lane);
     load_w.template init<WAVES>(n0, p.n, p.ldw, wave, lane);
 
-    v16i acc[TN][TM];
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int j = 0; j < TM; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-
     const int k_tiles = (p.k + kBK - 1) / kBK;
-    const int frow = lane & 31, fhalf = lane >> 5;
+    Epilogue e;
+    e.use_alpha = p.use_alpha; e.alpha = p.alpha; e.round_mode = p.round_mode; e.col_outer = p.scale_order;
+    e.ldd = p.ldd; e.d = p.d;
+    auto finish = [&](auto& acc) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        __syncthreads();
+        CLK_MARK(2);
+        epilogue<TM, TN, OUT, FLEX, false, COL_OUTER>(e, acc, lds, p.m, p.n, m0 + wm * TM * 32, n0 + wn * TN * 32, wave, lane,
+                                                      reinterpret_cast<const float*>(lds + C::kLdsBytes), BN + wm * TM * 32, wn * TN * 32);
+        CLK_MARK(3);
+    };
     CLK_MARK(0);
     if constexpr (STAGES == 2) {
-        // Two stages, the barrier before the last k step of a tile (mma_tile_rotated).  The requests for a tile go
-        // out one at a time behind every second multiplication, counted from that barrier: the ones that fit into
-        // the last k step of tile t - 2, the rest during the first three steps of tile t - 1.  Past the end of K
-        // every lane is out of range and stores zeros.
-        constexpr int kReq = C::kAInstr + C::kWInstr, kPerStep = TM * TN;
-        constexpr int kEarly = kPerStep / 2 < kReq ? kPerStep / 2 : kReq;      // positions inside the last k step
-        static_assert(kReq <= 4 * kPerStep / 2, "more requests than positions");
+        // Two stages (RotatedMma).  The requests for a tile go out one at a time, one per kPace multiplications counted from
+        // the barrier: those that fit behind it for tile t + 2, the rest during the next tile for t + 1.  Past the end
+        // of K every lane is out of range and stores zeros.
+        using Mma = RotatedMma<TM, TN>;
+        constexpr int kReq = C::kAInstr + C::kWInstr, kPace = 4;
+        constexpr int kEarly = Mma::kBehindBarrier / kPace < kReq ? Mma::kBehindBarrier / kPace : kReq;
+        static_assert(kReq <= Mma::kPerTile / kPace, "more requests than positions");
         auto request = [&](int r, int tile) {
             const uint32_t base = lds_base + (tile & 1) * C::kStageBytes;
             if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, tile * kBK, p.k, base, wave);
@@ -96,19 +98,36 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
         __syncthreads();
         const uint8_t* my_a = lds + (wm * TM * 32) * kBK;
         const uint8_t* my_w = lds + BM * kBK + (wn * TN * 32) * kBK;
-        v4i fa[2][TM], fw[2][TN];
-        fetch_fragments<TM, TN>(my_a, my_w, 0, frow, fhalf, fa[0], fw[0]);
+        Mma mma;
+        mma.init(lane);
+        mma.start(my_a, my_w);
         CLK_MARK(1);
-        for (int kt = 0; kt < k_tiles; ++kt) {
+        auto multiply = [&](int kt, auto&& req) {
             const int cur = (kt & 1) * C::kStageBytes, nxt = C::kStageBytes - cur;
-            mma_tile_rotated<TM, TN>(my_a + cur, my_w + cur, my_a + nxt, my_w + nxt, frow, fhalf, fa, fw, acc,
-                                     [&](int idx) {
-                                         if (idx % 2 != 1) return;
-                                         const int r = idx / 2;
-                                         request(r, r < kEarly ? kt + 2 : kt + 1);
-                                     });
-        }
+            mma.tile(my_a + cur, my_w + cur, my_a + nxt, my_w + nxt, [&](int idx) {
+                if (idx % kPace != kPace - 1) return;
+                const int r = idx / kPace;
+                req(r, r < kEarly ? kt + 2 : kt + 1);
+            });
+        };
+        auto request_whole = [&](int r, int tile) {
+            const uint32_t base = lds_base + (tile & 1) * C::kStageBytes;
+            if (r < C::kAInstr) load_a.template issue_whole<WAVES>(r, rsrc_a, tile * kBK, base, wave);
+            else if (r < kReq) load_w.template issue_whole<WAVES>(r - C::kAInstr, rsrc_w, tile * kBK, base + BM * kBK, wave);
+        };
+        int kt = 0;
+        for (const int whole = p.k / kBK - 2; kt < whole; ++kt) multiply(kt, request_whole);
+        for (; kt < k_tiles; ++kt) multiply(kt, request);
+        finish(mma.acc);
     } else {
+    const int frow = lane & 31, fhalf = lane >> 5;
+    v16i acc[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
     auto issue = [&](int tile) {
         const uint32_t base = lds_base + (tile % STAGES) * C::kStageBytes;
         load_a.template issue<WAVES>(rsrc_a, tile * kBK, p.k, base, wave);
@@ -136,17 +155,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
                                    }
                                });
     }
+    finish(acc);
     }
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    __syncthreads();
-    CLK_MARK(2);
-
-    Epilogue e;
-    e.use_alpha = p.use_alpha; e.alpha = p.alpha; e.round_mode = p.round_mode; e.col_outer = p.scale_order;
-    e.ldd = p.ldd; e.d = p.d;
-    epilogue<TM, TN, OUT, FLEX, false, COL_OUTER>(e, acc, lds, p.m, p.n, m0 + wm * TM * 32, n0 + wn * TN * 32, wave, lane,
-                                                  reinterpret_cast<const float*>(lds + C::kLdsBytes), BN + wm * TM * 32, wn * TN * 32);
-    CLK_MARK(3);
 }
 
 template <int TM, int TN, int WGM, int WGN, int STAGES, int OUT, bool FLEX, bool COL_OUTER = false>
