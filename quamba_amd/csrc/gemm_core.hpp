@@ -4,7 +4,7 @@
 //   d[m,n]   = cast(s_row[m|0] * (s_col[n|0] * float(acc)))          w: (N,K) int8, K-contiguous (W8A8)
 //                                                                       or 4-bit codes + group scales (W4A8)
 // Structure: WGM x WGN waves per workgroup, each wave TM x TN blocks of 32 x 32 (v_mfma_i32_32x32x32_i8, or
-// v_mfma_i32_16x16x64_i8 in the two-stage main loop of the large tiles, see RotatedMma); block
+// v_mfma_i32_16x16x64_i8 in the main loop of tiles of 128 x 128 and more, see RotatedMma); block
 // tile (WGM*TM*32) x (WGN*TN*32) x 128 k-bytes.  The k extent of 128 bytes is one full cache line
 // per operand row: measured on MI355X, 64-byte row pieces halve the L1 load rate.  Operand tiles live
 // in LDS as rows of eight 16-byte chunks, the chunk index XOR-swizzled with bits 1..3 of the row
@@ -256,6 +256,7 @@ __device__ __forceinline__ void mma_tile_paced(const uint8_t* sa, const uint8_t*
 // between the steps they left the matrix pipe idle (256 x 256 tiles, K 8192: 158900 -> 144000 cycles).  The barrier
 // stands where the last fetch from this tile's stage has been made, three positions before the end: there the wave waits for its own
 // global -> LDS requests and meets the others, so the next tile's stage is complete and this one may be overwritten.
+// IN_FLIGHT: requests, the last ones made, that need not be complete at the barrier (those of tiles after the next).
 // `hook(idx)` runs after every multiplication, idx counted from the barrier, through kPerTile; the caller places its
 // requests behind the multiplications it chooses.
 // Against 32x32x32 with block fetches (rows x outputs x K, us): 16384 x 18560 x 4096 1030 -> 965, 16384 x 4096 x 8192
@@ -266,7 +267,7 @@ struct RotatedMma {
     static constexpr bool kWalkW = TN > TM;
     static constexpr int kHeld = 2 * (kWalkW ? TM : TN), kWalk = 2 * (kWalkW ? TN : TM), kRing = 4, kAhead = 3;
     static constexpr int kPerTile = 2 * kWalk * kHeld, kBehindBarrier = kAhead * kHeld;     // multiplications
-    static_assert(2 * kWalk % kRing == 0 && kHeld <= kAhead * (kHeld - 1), "");
+    static_assert(2 * kWalk % kRing == 0 && kAhead < kWalk && kHeld <= kAhead * (kHeld - 1), "the order of the fetches");
     v4i acc[2 * TN][2 * TM];      // lane l: row 16 j + (l & 15), columns 16 i + 4 (l >> 4) + 0..3
     v4i held[2][kHeld], ring[kRing];
     int at;                       // this lane's 16 bytes of fragment 0, step 0, in a stage's rows
@@ -289,7 +290,7 @@ struct RotatedMma {
 #pragma unroll
         for (int g = 0; g < kAhead; ++g) ring[g] = fragment(kWalkW ? sw : sa, 0, g);
     }
-    template <class Hook>
+    template <int IN_FLIGHT, class Hook>
     __device__ __forceinline__ void tile(const uint8_t* sa, const uint8_t* sw, const uint8_t* na, const uint8_t* nw, Hook&& hook) {
         const uint8_t* const h0 = kWalkW ? sa : sw;
         const uint8_t* const h1 = kWalkW ? na : nw;
@@ -299,7 +300,7 @@ struct RotatedMma {
         for (int g = 0; g < 2 * kWalk; ++g) {
             const int step = g / kWalk, pos = g % kWalk, from_end = kWalk - pos;
             if (g == 2 * kWalk - kAhead) {
-                __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(IN_FLIGHT));
                 __syncthreads();
                 __builtin_amdgcn_sched_barrier(0);
             }

@@ -77,24 +77,32 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
         CLK_MARK(3);
     };
     CLK_MARK(0);
-    if constexpr (STAGES == 2) {
-        // Two stages (RotatedMma).  The requests for a tile go out one at a time, one per kPace multiplications counted from
-        // the barrier: those that fit behind it for tile t + 2, the rest during the next tile for t + 1.  Past the end
-        // of K every lane is out of range and stores zeros.
+    if constexpr (TM * TN > 1) {
+        // The requests for a tile go out one at a time, one per kPace multiplications counted from the barrier (RotatedMma): those
+        // that fit behind it, whose stage it has just freed, for tile t + STAGES, the rest during the next tile.  Past the
+        // end of K every lane is out of range and stores zeros.
+        // (Workgroups that go from one output tile to the next without a pause, the next one's first k tile requested
+        // during the last ones of this one, gained nothing: the clock falls by what the matrix cores are busier.)
+        // 128 x 256 tiles, three stages, against 32x32x32 with block fetches (us): 3063 x 2560 x 5120 42.8 -> 40.8, 3063 x
+        // 1536 x 3072 20.6 -> 18.6, 16384 x 1536 x 3072 77.6 -> 68.2.
         using Mma = RotatedMma<TM, TN>;
-        constexpr int kReq = C::kAInstr + C::kWInstr, kPace = 4;
+        constexpr int kReq = C::kAInstr + C::kWInstr, kPace = kReq <= Mma::kPerTile / 4 ? 4 : Mma::kPerTile / kReq;
         constexpr int kEarly = Mma::kBehindBarrier / kPace < kReq ? Mma::kBehindBarrier / kPace : kReq;
-        static_assert(kReq <= Mma::kPerTile / kPace, "more requests than positions");
-        auto request = [&](int r, int tile) {
-            const uint32_t base = lds_base + (tile & 1) * C::kStageBytes;
-            if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, tile * kBK, p.k, base, wave);
-            else if (r < kReq) load_w.template issue_one<WAVES>(r - C::kAInstr, rsrc_w, tile * kBK, p.k, base + BM * kBK, wave);
+        auto request = [&](int r, int tile, uint32_t stage) {
+            if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, tile * kBK, p.k, lds_base + stage, wave);
+            else if (r < kReq) load_w.template issue_one<WAVES>(r - C::kAInstr, rsrc_w, tile * kBK, p.k, lds_base + stage + BM * kBK, wave);
+        };
+        auto request_whole = [&](int r, int tile, uint32_t stage) {
+            if (r < C::kAInstr) load_a.template issue_whole<WAVES>(r, rsrc_a, tile * kBK, lds_base + stage, wave);
+            else if (r < kReq) load_w.template issue_whole<WAVES>(r - C::kAInstr, rsrc_w, tile * kBK, lds_base + stage + BM * kBK, wave);
         };
 #pragma unroll
-        for (int r = 0; r < kReq; ++r) request(r, 0);
+        for (int t = 0; t < STAGES - 1; ++t)
 #pragma unroll
-        for (int r = 0; r < kEarly; ++r) request(r, 1);
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(kEarly));
+            for (int r = 0; r < kReq; ++r) request(r, t, t * C::kStageBytes);
+#pragma unroll
+        for (int r = 0; r < kEarly; ++r) request(r, STAGES - 1, (STAGES - 1) * C::kStageBytes);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 2) * kReq + kEarly));
         __syncthreads();
         const uint8_t* my_a = lds + (wm * TM * 32) * kBK;
         const uint8_t* my_w = lds + BM * kBK + (wn * TN * 32) * kBK;
@@ -102,21 +110,20 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
         mma.init(lane);
         mma.start(my_a, my_w);
         CLK_MARK(1);
+        uint32_t cur = 0, late = (STAGES - 1) * C::kStageBytes;        // stages of this tile and of the tile STAGES - 1 further
         auto multiply = [&](int kt, auto&& req) {
-            const int cur = (kt & 1) * C::kStageBytes, nxt = C::kStageBytes - cur;
-            mma.tile(my_a + cur, my_w + cur, my_a + nxt, my_w + nxt, [&](int idx) {
+            const uint32_t nxt = cur + C::kStageBytes == C::kLdsBytes ? 0 : cur + C::kStageBytes;
+            mma.template tile<(STAGES - 2) * kReq>(my_a + cur, my_w + cur, my_a + nxt, my_w + nxt, [&](int idx) {
                 if (idx % kPace != kPace - 1) return;
                 const int r = idx / kPace;
-                req(r, r < kEarly ? kt + 2 : kt + 1);
+                if (r < kEarly) req(r, kt + STAGES, cur);
+                else req(r, kt + STAGES - 1, late);
             });
-        };
-        auto request_whole = [&](int r, int tile) {
-            const uint32_t base = lds_base + (tile & 1) * C::kStageBytes;
-            if (r < C::kAInstr) load_a.template issue_whole<WAVES>(r, rsrc_a, tile * kBK, base, wave);
-            else if (r < kReq) load_w.template issue_whole<WAVES>(r - C::kAInstr, rsrc_w, tile * kBK, base + BM * kBK, wave);
+            late = cur;
+            cur = nxt;
         };
         int kt = 0;
-        for (const int whole = p.k / kBK - 2; kt < whole; ++kt) multiply(kt, request_whole);
+        for (const int whole = p.k / kBK - STAGES; kt < whole; ++kt) multiply(kt, request_whole);
         for (; kt < k_tiles; ++kt) multiply(kt, request);
         finish(mma.acc);
     } else {
