@@ -306,8 +306,9 @@ struct RotatedMma {
             }
 #pragma unroll
             for (int h = 0; h < kHeld; ++h) {
-                v4i& c = kWalkW ? acc[pos][h] : acc[h][pos];
-                c = __builtin_amdgcn_mfma_i32_16x16x64_i8(kWalkW ? ring[g % kRing] : held[step][h], kWalkW ? held[step][h] : ring[g % kRing], c, 0, 0, 0);
+                const int x = g % 2 ? kHeld - 1 - h : h;               // there and back: one operand stays at every turn, 0.7 % of the time
+                v4i& c = kWalkW ? acc[pos][x] : acc[x][pos];
+                c = __builtin_amdgcn_mfma_i32_16x16x64_i8(kWalkW ? ring[g % kRing] : held[step][x], kWalkW ? held[step][x] : ring[g % kRing], c, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 if (h == 0) {
                     const int n = g + kAhead;
