@@ -325,13 +325,74 @@ int launch_skinny(const QaGemmW8A8Params& p, hipStream_t stream) {
     return launch_skinny_one<TM, WAVES, QA_OUT_F16, FLEX>(p, stream);
 }
 
+// ---------------------------------------------------------------------------------------------
+// Products of so few outputs that even tiles of 32 x 32 leave most CUs idle (the step-size and B, C projection of a decode
+// batch or a short prompt): 16 x 16 outputs per workgroup, K over sixteen waves.  What bounds them is latency - a CU fetches
+// its operand rows at about 64 bytes a clock, and every trip to memory counts - so the outputs go to four times the CUs, a wave asks
+// for all its fragments (16 rows x 64 bytes, straight into the operand registers of 16x16x64) before it multiplies, and the
+// sixteen partial sums meet in LDS with one store and sixteen loads each.
+// Against 32 x 32 with K over four waves (rows x outputs x K, us): 64 x 192 x 5120 7.5 -> 6.8, 64 x 80 x 1536 4.0 -> 3.2, 512 x 80
+// x 1536 4.7 -> 3.8, 512 x 128 x 3072 5.7 -> 5.1, 16 x 2560 x 5120 9.4 -> 8.7, 16 x 3072 x 768 4.2 -> 3.2.
+// ---------------------------------------------------------------------------------------------
+template <int OUT>
+__global__ __launch_bounds__(1024) void gemm_w8a8_narrow_kernel(QaGemmW8A8Params p) {
+    constexpr int kWaves = 16, kUnits = 3;                 // units of 128 bytes of K at a time, all in flight
+    __shared__ __align__(16) int red[kWaves][256];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int blocks_m = (p.m + 15) / 16;
+    const int m0 = static_cast<int>(blockIdx.x) % blocks_m * 16, n0 = static_cast<int>(blockIdx.x) / blocks_m * 16;
+    const int chunk = (lane >> 4) * 16;
+    // rows outside repeat the last one: their outputs are not written
+    const int8_t* a = p.a + static_cast<int64_t>(min(m0 + (lane & 15), p.m - 1)) * p.lda;
+    const int8_t* w = p.w + static_cast<int64_t>(min(n0 + (lane & 15), p.n - 1)) * p.ldw;
+    v4i acc = {0, 0, 0, 0};
+    for (int k0 = wave * kBK; k0 < p.k; k0 += kUnits * kWaves * kBK) {
+        v4i fa[2 * kUnits], fw[2 * kUnits];
+#pragma unroll
+        for (int s = 0; s < 2 * kUnits; ++s) {
+            const int k = k0 + s / 2 * (kWaves * kBK) + s % 2 * 64 + chunk;
+            fa[s] = fw[s] = v4i{0, 0, 0, 0};
+            if (k < p.k) {
+                fw[s] = *reinterpret_cast<const v4i*>(w + k);
+                fa[s] = *reinterpret_cast<const v4i*>(a + k);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 2 * kUnits; ++s) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[s], fa[s], acc, 0, 0, 0);
+    }
+    *reinterpret_cast<v4i*>(&red[wave][lane * 4]) = acc;
+    __syncthreads();
+    if (threadIdx.x >= 256) return;
+    // thread t: row (t >> 2) & 15, column 4 (t >> 6) + (t & 3)
+    const int t = threadIdx.x, mm = m0 + ((t >> 2) & 15), nn = n0 + (t >> 6) * 4 + (t & 3);
+    if (mm >= p.m || nn >= p.n) return;
+    const float s_row = p.a_scale[p.a_scale_numel == 1 ? 0 : mm], s_col = p.w_scale[p.w_scale_numel == 1 ? 0 : nn];
+    int sum = 0;
+#pragma unroll
+    for (int x = 0; x < kWaves; ++x) sum += red[x][t];
+    const float accf = static_cast<float>(sum);
+    float v = p.scale_order ? s_col * (s_row * accf) : s_row * (s_col * accf);
+    asm volatile("" : "+v"(v));                            // the fp32 product is rounded on its own
+    const int64_t at = static_cast<int64_t>(mm) * p.ldd + nn;
+    if (OUT == QA_OUT_I8) static_cast<int8_t*>(p.d)[at] = static_cast<int8_t>(quant8(v, QA_ROUND_RNE));
+    else static_cast<uint16_t*>(p.d)[at] = one_f16_or_bf16<OUT>(v);
+}
+
+int launch_narrow(const QaGemmW8A8Params& p, hipStream_t stream) {
+    const int64_t blocks = static_cast<int64_t>((p.m + 15) / 16) * ((p.n + 15) / 16);
+    auto kernel = p.out_type == QA_OUT_I8 ? gemm_w8a8_narrow_kernel<QA_OUT_I8> : p.out_type == QA_OUT_BF16 ? gemm_w8a8_narrow_kernel<QA_OUT_BF16> : gemm_w8a8_narrow_kernel<QA_OUT_F16>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(1024), 0, stream, p);
+    return check_launch();
+}
+
 template <bool FLEX>
 int dispatch_skinny(const QaGemmW8A8Params& p, hipStream_t stream) {
     return launch_skinny<1, 4, FLEX>(p, stream);
 }
 
 // Tile of a launch: the smallest whose tiles fit the part in one round.  With at most one tile per CU a launch takes a
-// tile's own time - about 2.5 us and, per 128 bytes of K, 0.115 us (32 x 32, K split over the waves), 0.20 (64 x 64), 0.31
+// tile's own time - about 2.5 us and, per 128 bytes of K, 0.105 us (16 x 16, K split over the waves), 0.125 (32 x 32, the same), 0.20 (64 x 64), 0.31
 // (128 x 64), 0.48 (128 x 128, four stages), 0.68 (128 x 256), 1.15 (256 x 256) - so smaller tiles win until a second round
 // starts.  Measured at M 16 .. 16384 with ten of the projections' N and K: this choice is the fastest or
 // within 8 % of it.  Against 128 x 128 tiles up to 192 tiles of 256 x 256 (rows x outputs x K, us): 512 x 80 x 1536 9.6 ->
@@ -346,6 +407,7 @@ int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
         cus = 256;
     }
     auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
+    if (tiles(16, 16) <= cus) return launch_narrow(p, stream);                       // (two rounds of these: slower than one of 32 x 32)
     if (tiles(32, 32) <= cus) return dispatch_skinny<false>(p, stream);
     if (tiles(64, 64) <= cus) return launch_gemm<1, 1, 2, 2, 4, false>(p, stream);
     if (tiles(128, 64) <= cus) return launch_gemm<1, 1, 4, 2, 4, false>(p, stream);

@@ -38,6 +38,14 @@ def test_int8_weights(dev, M, N, K, order):
     np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
+# 16 x 16 tiles: one k step and part of one, more units of K than a wave takes at once, rows and columns with remainders, the
+# largest number of tiles (and one more: 32 x 32)
+@pytest.mark.parametrize("M,N,K", [(9, 5, 16), (17, 33, 80), (16, 48, 6160), (100, 30, 12304), (256, 250, 144), (257, 250, 144)])
+@pytest.mark.parametrize("order", [0, 1])
+def test_int8_weights_of_few_outputs(dev, M, N, K, order):
+    test_int8_weights(dev, M, N, K, order)
+
+
 # 32 x 32 with four and eight waves, 64 x 64, 64 x 128, 128 x 128, 192 x 128, expanded once
 @pytest.mark.parametrize("M,N,K,workspace", [(70, 200, 2176, False), (100, 1000, 384, False), (130, 2050, 1664, False), (250, 2500, 1152, False),
                                              (600, 2100, 256, False), (300, 4200, 1664, False), (70, 9000, 128, False), (700, 3100, 1152, False),
