@@ -413,12 +413,13 @@ int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
     if (tiles(128, 64) <= cus) return launch_gemm<1, 1, 4, 2, 4, false>(p, stream);
     if (tiles(128, 128) <= cus) return launch_gemm<2, 1, 2, 4, 4, false>(p, stream);
     if (tiles(128, 256) <= cus) return launch_gemm<2, 2, 2, 4, 3, false>(p, stream);
-    // More than a round: what counts is rounds times the tile's work (128 x 256 at six fifths of its share).
+    // More than a round: what counts is rounds times the tile's work, 128 x 256 at six fifths of its share and the 320-wide
+    // ones at 24/25: they move a tenth less per product through the caches, which at the power limit is time (against
+    // 256 x 256 at equal arithmetic 16384 x 10240 x 2560 321 -> 309 us, at 2 % more 16384 x 10576 x 2560 346 -> 339).
     auto cost = [&](int64_t bm, int64_t bn) { return ((tiles(bm, bn) + cus - 1) / cus) * bm * bn; };
-    const int64_t c_sq = cost(256, 256), c_wide = cost(256, 320), c_tall = cost(320, 256), c_half = cost(128, 256) * 6 / 5;
+    const int64_t c_sq = cost(256, 256), c_wide = cost(256, 320) * 24 / 25, c_tall = cost(320, 256) * 24 / 25, c_half = cost(128, 256) * 6 / 5;
     if (c_half < c_sq && c_half < c_wide && c_half < c_tall) return launch_gemm<2, 2, 2, 4, 3, false>(p, stream);
-    if (c_wide < c_sq && c_wide <= c_tall) return launch_gemm<2, 5, 4, 2, 2, false>(p, stream);
-    // at equal arithmetic the larger tile has fewer rounds, each with its own start and epilogue
+    if (c_wide <= c_sq && c_wide <= c_tall) return launch_gemm<2, 5, 4, 2, 2, false>(p, stream);
     if (c_tall <= c_sq) return launch_gemm<5, 2, 2, 4, 2, false>(p, stream);
     return launch_gemm<4, 2, 2, 4, 2, false>(p, stream);                             // 256x256 tile, 8 waves
 }
