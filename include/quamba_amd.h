@@ -33,7 +33,11 @@ typedef enum QaStatus {
 
 /* Human-readable text for a status code (static storage). */
 const char* qa_status_string(int status);
-/* ABI version, bumped on any incompatible change of the structs below. */
+/* ABI version of the structs below: bumped on any change of their fields, of what a field means or of which fields a call
+ * reads.  A caller compares its own QA_ABI_VERSION with qa_abi_version() before the first call.
+ * 3: QaSScanParams has the token-major fields at its end, QaConv2Params x_out_scale and QaSsdParams dt_row_stride in the
+ *    place of a reserved field; the forward Mamba2 conv writes conv_state; the layer blocks. */
+#define QA_ABI_VERSION 3
 int qa_abi_version(void);
 /* Last HIP error code seen by a failed launch on this thread (0 if none). */
 int qa_last_hip_error(void);

@@ -24,6 +24,9 @@ def _plan_class():
             from . import _host as native
         except ImportError as e:
             raise RuntimeError("quamba_amd/_host.so is missing or does not load: build it with `python -m quamba_amd.build`") from e
+        if getattr(native, "ABI_VERSION", None) != _lib.ABI_VERSION:
+            raise RuntimeError("quamba_amd/_host.so is built for another layout of the parameter blocks: rebuild it with "
+                               "`python -m quamba_amd.build --force`")
         _host = native
     return _host.Plan
 

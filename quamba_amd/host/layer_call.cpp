@@ -327,5 +327,6 @@ PyMODINIT_FUNC PyInit__host() {
     if (!m) return nullptr;
     Py_INCREF(&PlanType);
     if (PyModule_AddObject(m, "Plan", reinterpret_cast<PyObject*>(&PlanType)) < 0) return nullptr;
+    if (PyModule_AddIntConstant(m, "ABI_VERSION", QA_ABI_VERSION) < 0) return nullptr;      // of the blocks a plan holds
     return m;
 }

@@ -1,6 +1,7 @@
 """CPU-side checks of the C ABI: the library loads and exports every declared symbol, the ctypes
 structs match the header's layout, and argument validation returns the documented codes."""
 import ctypes as C
+import hashlib
 import os
 import re
 import subprocess
@@ -30,10 +31,34 @@ def test_library_exports_every_declared_symbol():
 
 def test_abi_version_and_status_strings():
     l = _lib.lib()
-    assert l.qa_abi_version() == _lib.ABI_VERSION == 2
+    assert l.qa_abi_version() == _lib.ABI_VERSION == 3
     assert l.qa_status_string(0) == b"ok"
     for code in (-1, -2, -3, -4, -5, -6):
         assert l.qa_status_string(code) not in (b"ok", b"unknown status")
+
+
+# what the header's parameter blocks looked like at each version (comments and spacing aside)
+BLOCKS_OF_VERSION = {2: "ef5cba8d0ff46858", 3: "7acd57262ac5b05b"}
+
+
+def test_a_changed_block_has_another_version():
+    """The version is all that keeps a caller built against other blocks out of the library: no version stands for two
+    layouts, and a change of any block fails here until the version is another one."""
+    text = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S)
+    blocks = re.findall(r"typedef struct (?:Qa\w+Params) \{.*?\} \w+;", text, flags=re.S)
+    assert len(blocks) == len(_param_structs())
+    found = hashlib.sha256(re.sub(r"\s+", " ", " ".join(blocks)).encode()).hexdigest()[:16]
+    assert BLOCKS_OF_VERSION[_lib.lib().qa_abi_version()] == found
+    assert int(re.search(r"#define QA_ABI_VERSION (\d+)", text).group(1)) == _lib.ABI_VERSION
+
+
+def test_a_host_extension_of_another_version_is_refused(monkeypatch):
+    from quamba_amd import _host, _layer_call
+    assert _host.ABI_VERSION == _lib.ABI_VERSION
+    monkeypatch.setattr(_layer_call, "_host", None)
+    monkeypatch.setattr(_lib, "ABI_VERSION", _lib.ABI_VERSION + 1)
+    with pytest.raises(RuntimeError, match="another layout"):
+        _layer_call._plan_class()
 
 
 def _param_structs():
