@@ -1,10 +1,10 @@
 """One library call per mixer call: qa_mamba1_* / qa_mamba2_* behind the mixers.
 
 A mixer's weights, scales and sizes are gathered into the library's parameter block once and kept, in a native object
-(quamba_amd._host.Plan, host/layer_call.cpp), for as long as its sub-modules, their buffers (the tensor objects and their
-addresses) and their scalars are the ones the block was made from; running the plan verifies that, allocates output and
-workspace and enqueues the layer.  Mixers, tensors or states the library call does not cover (other sub-module classes,
-forward hooks, views with gaps, unusual sizes) yield None, and the mixer runs its modules one by one.
+(quamba_amd._host.Plan, host/layer_call.cpp), for as long as its sub-modules and everything they hold - attributes, buffers
+and parameters, tensors with their addresses - are the ones the block was made from; running the plan verifies that,
+allocates output and workspace and enqueues the layer.  Mixers, tensors or states the library call does not cover (other
+sub-module classes, forward hooks, views with gaps, unusual sizes) yield None, and the mixer runs its modules one by one.
 """
 import ctypes as C
 
@@ -88,17 +88,19 @@ def _native(mixer):
 
 
 def _make(mixer):
-    """The mixer's plan, or None where its sub-modules are not the stock ones."""
-    mods = mixer._native_modules()
-    if mods is None:
-        return None
-    names = tuple(next(k for k, v in mixer._modules.items() if v is md) for md in mods)
-    hooks = tuple(getattr(_module, k) for k in ("_global_forward_hooks", "_global_forward_pre_hooks"))
+    """The mixer's plan (one that only ever yields None where the library does not cover the mixer)."""
+    mods = [m for m in mixer._modules.values() if m is not None]
+    watched = [mixer._modules]
+    hooks = [getattr(_module, k) for k in ("_global_forward_hooks", "_global_forward_pre_hooks")]
+    for m in mods:
+        watched += [m.__dict__, m._buffers, m._parameters]
+        hooks += [m._forward_hooks, m._forward_pre_hooks]
     try:
+        _need(mixer._native_modules() is not None)
         native = _native(mixer)
     except _Unsupported:
         native = None
-    return _plan_class()(mixer._modules, names, mixer._scalars(), hooks, native)
+    return _plan_class()(tuple(watched), tuple(hooks), native)
 
 
 def call(mixer, hidden, conv_state, ssm_state, step):
@@ -107,8 +109,6 @@ def call(mixer, hidden, conv_state, ssm_state, step):
     out = plan.run(hidden, conv_state, ssm_state, step) if plan is not None else False
     if out is False:
         plan = mixer.__dict__["_plan"] = _make(mixer)
-        if plan is None:
-            return None
         out = plan.run(hidden, conv_state, ssm_state, step)
         if out is False:
             return None

@@ -2,9 +2,13 @@
 //
 // One decode step of one sequence is four to six kernels of 3-5 us; gathering the layer's tensors, checking that nothing
 // has changed and filling the parameter block cost 13-17 us of that in Python.  A Plan holds the parameter block of a
-// layer (qa_mamba1_* / qa_mamba2_*, include/quamba_amd.h) together with what it was made from - the sub-modules, their
-// buffers (the tensor objects and their addresses), the scalars they carry, their hooks - and run() verifies all of it,
+// layer (qa_mamba1_* / qa_mamba2_*, include/quamba_amd.h) together with what it was made from, and run() verifies all of it,
 // allocates output and workspace, and enqueues the layer.
+//
+// What it was made from is a list of dicts - the mixer's sub-modules, and of each of them its attributes, buffers and
+// parameters - as they were, entry by entry: a tensor whose address is in the block is in one of them wherever the module
+// keeps it, the entry keeps it alive, and every call compares the entries with what the dicts hold now (values by identity,
+// numbers by value, tensors by their address as well).
 //
 // run(hidden, conv_state, ssm_state, step) returns the output tensor; None when the library call does not cover these
 // arguments (the mixer then runs its modules one by one); False when the layer is not the one the plan was made from any
@@ -24,28 +28,34 @@
 
 namespace {
 
-struct Buffer {
-    PyObject* object;          // a tensor or None
-    const void* address;
+struct Entry {
+    PyObject *key, *value;
+    bool tensor;
+    const void* address;       // of a tensor's memory
 };
 
-struct Module {
-    PyObject *name, *module, *dict, *buffers_dict;
-    std::vector<Buffer> buffers;
+struct Watch {
+    PyObject* dict;
+    uint64_t version;
+    std::vector<Entry> entries;
 };
 
-struct Scalar {
-    PyObject *dict, *key, *value;
-};
+// The number the interpreter gives a dict anew with every change of it (0: this interpreter has none).
+uint64_t version_of(PyObject* dict) {
+#if PY_VERSION_HEX < 0x030C0000
+    return reinterpret_cast<PyDictObject*>(dict)->ma_version_tag;
+#else
+    return 0;
+#endif
+}
 
 using Forward = int (*)(const void*, void*);
 using Workspace = int64_t (*)(const void*, int);
 
 struct State {
-    PyObject* modules = nullptr;               // the mixer's own dict of sub-modules
-    std::vector<Module> parts;
-    std::vector<Scalar> scalars;
-    std::vector<PyObject*> no_hooks;           // dicts that have to be empty: global hooks
+    std::vector<Watch> watches;
+    std::vector<Entry> tensors;                // the entries that are tensors, once more (borrowed)
+    std::vector<PyObject*> no_hooks;           // dicts that have to be empty: hooks
     bool usable = false;
     int family = 1;
     QaMamba1Params m1;
@@ -65,9 +75,7 @@ struct PlanObject {
     State* s;
 };
 
-PyObject *s_buffers, *s_hooks, *s_pre_hooks;   // interned attribute names
-
-const void* address_of(PyObject* t) { return t == Py_None ? nullptr : THPVariable_Unpack(t).const_data_ptr(); }
+const void* address_of(PyObject* t) { return THPVariable_Unpack(t).const_data_ptr(); }
 
 // ---- making a plan ------------------------------------------------------------------------------------------------
 PyObject* keep(PyObject* o) {
@@ -77,52 +85,40 @@ PyObject* keep(PyObject* o) {
 
 void plan_free(State* s) {
     if (!s) return;
-    Py_XDECREF(s->modules);
-    for (auto& m : s->parts) {
-        Py_XDECREF(m.name); Py_XDECREF(m.module); Py_XDECREF(m.dict); Py_XDECREF(m.buffers_dict);
-        for (auto& b : m.buffers) Py_XDECREF(b.object);
+    for (auto& w : s->watches) {
+        Py_XDECREF(w.dict);
+        for (auto& e : w.entries) { Py_XDECREF(e.key); Py_XDECREF(e.value); }
     }
-    for (auto& c : s->scalars) { Py_XDECREF(c.dict); Py_XDECREF(c.key); Py_XDECREF(c.value); }
     for (PyObject* d : s->no_hooks) Py_XDECREF(d);
     Py_XDECREF(s->get_device); Py_XDECREF(s->set_device); Py_XDECREF(s->get_stream); Py_XDECREF(s->oom);
     delete s;
 }
 
-// Plan(modules_dict, names, scalars, global_hook_dicts, native): scalars are (dict, key) pairs; native is None for a layer
-// the library does not cover, or (family, block bytes, (forward, step, workspace) addresses, (conv channels, state shape,
+// Plan(watched, hooks, native): the dicts the layer was made from, the dicts that have to be empty, and None for a layer the
+// library does not cover, or (family, block bytes, (forward, step, workspace) addresses, (conv channels, state shape,
 // (forward widths, step widths)), output padding, a tensor on the layer's device, (get_device, set_device, get_stream, out-of-memory error)).
 int plan_init(PlanObject* self, PyObject* args, PyObject*) {
-    PyObject *modules, *names, *scalars, *hooks, *native;
-    if (!PyArg_ParseTuple(args, "O!O!O!O!O", &PyDict_Type, &modules, &PyTuple_Type, &names, &PyTuple_Type, &scalars, &PyTuple_Type, &hooks, &native)) return -1;
+    PyObject *watched, *hooks, *native;
+    if (!PyArg_ParseTuple(args, "O!O!O", &PyTuple_Type, &watched, &PyTuple_Type, &hooks, &native)) return -1;
+    for (PyObject* dicts : {watched, hooks})
+        for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(dicts); ++i)
+            if (!PyDict_Check(PyTuple_GET_ITEM(dicts, i))) {
+                PyErr_SetString(PyExc_TypeError, "a plan is made from dicts");
+                return -1;
+            }
     State* s = new State;
     plan_free(self->s);
     self->s = s;
-    s->modules = keep(modules);
-    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(names); ++i) {
-        Module m = {};
-        m.name = keep(PyTuple_GET_ITEM(names, i));
-        m.module = keep(PyDict_GetItem(modules, m.name));
-        m.dict = m.module ? PyObject_GenericGetDict(m.module, nullptr) : nullptr;
-        m.buffers_dict = m.dict ? keep(PyDict_GetItem(m.dict, s_buffers)) : nullptr;
-        s->parts.push_back(m);
-        if (!m.buffers_dict || !PyDict_Check(m.buffers_dict)) {
-            PyErr_SetString(PyExc_TypeError, "not a module of the layer");
-            return -1;
-        }
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(watched); ++i) {
+        PyObject* dict = keep(PyTuple_GET_ITEM(watched, i));
+        s->watches.push_back({dict, version_of(dict), {}});
         PyObject *key, *value;
         Py_ssize_t pos = 0;
-        while (PyDict_Next(m.buffers_dict, &pos, &key, &value)) {
-            if (value != Py_None && !THPVariable_Check(value)) {
-                PyErr_SetString(PyExc_TypeError, "a buffer that is no tensor");
-                return -1;
-            }
-            s->parts.back().buffers.push_back({keep(value), address_of(value)});
+        while (PyDict_Next(dict, &pos, &key, &value)) {
+            const bool tensor = THPVariable_Check(value);
+            s->watches.back().entries.push_back({keep(key), keep(value), tensor, tensor ? address_of(value) : nullptr});
+            if (tensor) s->tensors.push_back(s->watches.back().entries.back());
         }
-    }
-    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(scalars); ++i) {
-        PyObject *dict, *key;
-        if (!PyArg_ParseTuple(PyTuple_GET_ITEM(scalars, i), "O!O", &PyDict_Type, &dict, &key)) return -1;
-        s->scalars.push_back({keep(dict), keep(key), keep(PyDict_GetItem(dict, key))});
     }
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(hooks); ++i) s->no_hooks.push_back(keep(PyTuple_GET_ITEM(hooks, i)));
     if (native == Py_None) return 0;
@@ -162,36 +158,34 @@ int plan_init(PlanObject* self, PyObject* args, PyObject*) {
 // ---- using it -----------------------------------------------------------------------------------------------------
 bool same_value(PyObject* a, PyObject* b) {
     if (a == b) return true;
-    if (!a || !b) return false;
     if (PyFloat_CheckExact(a) && PyFloat_CheckExact(b)) return PyFloat_AS_DOUBLE(a) == PyFloat_AS_DOUBLE(b);
     if (PyLong_CheckExact(a) && PyLong_CheckExact(b)) return PyObject_RichCompareBool(a, b, Py_EQ) == 1;
     return false;
 }
 
-bool hooked(PyObject* dict, PyObject* name) {
-    PyObject* d = PyDict_GetItem(dict, name);
-    return d && PyDict_Check(d) && PyDict_GET_SIZE(d) != 0;
+// The dict holds what it held.  (Most calls end at the version; scanning the twenty dicts of a layer takes about 1 us.)
+bool same_entries(Watch& w) {
+    const uint64_t version = version_of(w.dict);
+    if (version && version == w.version) return true;
+    if (PyDict_GET_SIZE(w.dict) != static_cast<Py_ssize_t>(w.entries.size())) return false;
+    PyObject *key, *value;
+    Py_ssize_t pos = 0;
+    const Entry* e = w.entries.data();
+    for (; PyDict_Next(w.dict, &pos, &key, &value); ++e)
+        if (key != e->key || !same_value(value, e->value)) return false;
+    w.version = version;
+    return true;
 }
 
 // 1: the layer the plan was made from; 0: it has changed; -1: unchanged but hooked
-int verify(const State& s) {
-    bool with_hooks = false;
-    for (PyObject* d : s.no_hooks) with_hooks = with_hooks || PyDict_GET_SIZE(d) != 0;
-    for (const Module& m : s.parts) {
-        if (PyDict_GetItem(s.modules, m.name) != m.module || PyDict_GetItem(m.dict, s_buffers) != m.buffers_dict) return 0;
-        if (PyDict_GET_SIZE(m.buffers_dict) != static_cast<Py_ssize_t>(m.buffers.size())) return 0;
-        PyObject *key, *value;
-        Py_ssize_t pos = 0;
-        size_t i = 0;
-        while (PyDict_Next(m.buffers_dict, &pos, &key, &value)) {
-            const Buffer& b = m.buffers[i++];
-            if (value != b.object || (value != Py_None && address_of(value) != b.address)) return 0;
-        }
-        with_hooks = with_hooks || hooked(m.dict, s_hooks) || hooked(m.dict, s_pre_hooks);
-    }
-    for (const Scalar& c : s.scalars)
-        if (!same_value(PyDict_GetItem(c.dict, c.key), c.value)) return 0;
-    return with_hooks ? -1 : 1;
+int verify(State& s) {
+    for (Watch& w : s.watches)
+        if (!same_entries(w)) return 0;
+    for (const Entry& e : s.tensors)
+        if (address_of(e.value) != e.address) return 0;
+    for (PyObject* d : s.no_hooks)
+        if (PyDict_GET_SIZE(d) != 0) return -1;
+    return 1;
 }
 
 template <class Params>
@@ -296,8 +290,28 @@ PyObject* plan_run(PlanObject* self, PyObject* const* args, Py_ssize_t nargs) {
 // Copies and pickles of a layer start without a plan.
 PyObject* plan_reduce(PyObject*, PyObject*) { return Py_BuildValue("(O())", reinterpret_cast<PyObject*>(Py_TYPE(Py_None))); }
 
+// (an attribute of a sub-module may lead back to the mixer and from there to the plan)
+int plan_traverse(PlanObject* self, visitproc visit, void* arg) {
+    if (!self->s) return 0;
+    for (const Watch& w : self->s->watches) {
+        Py_VISIT(w.dict);
+        for (const Entry& e : w.entries) { Py_VISIT(e.key); Py_VISIT(e.value); }
+    }
+    for (PyObject* d : self->s->no_hooks) Py_VISIT(d);
+    for (PyObject* o : {self->s->get_device, self->s->set_device, self->s->get_stream, self->s->oom}) Py_VISIT(o);
+    return 0;
+}
+
+int plan_clear(PlanObject* self) {
+    State* s = self->s;
+    self->s = nullptr;
+    plan_free(s);
+    return 0;
+}
+
 void plan_dealloc(PlanObject* self) {
-    plan_free(self->s);
+    PyObject_GC_UnTrack(self);
+    plan_clear(self);
     Py_TYPE(self)->tp_free(reinterpret_cast<PyObject*>(self));
 }
 
@@ -312,13 +326,13 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Host side of the mixe
 }  // namespace
 
 PyMODINIT_FUNC PyInit__host() {
-    s_buffers = PyUnicode_InternFromString("_buffers");
-    s_hooks = PyUnicode_InternFromString("_forward_hooks");
-    s_pre_hooks = PyUnicode_InternFromString("_forward_pre_hooks");
     PlanType.tp_name = "quamba_amd._host.Plan";
     PlanType.tp_basicsize = sizeof(PlanObject);
-    PlanType.tp_flags = Py_TPFLAGS_DEFAULT;
+    PlanType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
     PlanType.tp_new = PyType_GenericNew;
+    PlanType.tp_traverse = reinterpret_cast<traverseproc>(plan_traverse);
+    PlanType.tp_clear = reinterpret_cast<inquiry>(plan_clear);
+    PlanType.tp_free = PyObject_GC_Del;
     PlanType.tp_init = reinterpret_cast<initproc>(plan_init);
     PlanType.tp_dealloc = reinterpret_cast<destructor>(plan_dealloc);
     PlanType.tp_methods = plan_methods;

@@ -94,13 +94,6 @@ class W8A8QMamba(nn.Module):
                 return None
         return mods
 
-    def _scalars(self):
-        """(dict, key) of everything a plan depends on that is no buffer."""
-        m = self._modules
-        c, s, h = (m[k].__dict__ for k in ("conv1d", "selective_scan", "had"))
-        return (tuple((c, k) for k in ("input_scale", "weight_scale", "bias_scale", "output_scale", "bias")) + ((s, "delta_softplus"),)
-                + tuple((h, k) for k in ("x_H_scale", "had_scale")) + tuple((m[k].__dict__, "alpha") for k in ("in_proj", "x_proj", "dt_proj", "out_proj")))
-
     def _native_block(self, dev):
         p, D, N = _lib.QaMamba1Params(), self.d_inner, self.d_state
         c, s = self.conv1d, self.selective_scan
@@ -269,17 +262,6 @@ class W4A8QMamba2(nn.Module):
             if type(md) is not cls:
                 return None
         return mods
-
-    def _scalars(self):
-        """(dict, key) of everything a plan depends on that is no buffer."""
-        m = self._modules
-        c, s, n, h = (m[k].__dict__ for k in ("conv1d", "qchunk_scan", "norm", "had"))
-        conv = ("x_scale", "B_scale", "C_scale", "wx_scale", "wB_scale", "wC_scale", "bx_scale", "bB_scale", "bC_scale", "bias",
-                "x_head_group_range", "x_dim_group_range")
-        scan = ("x_head_group_range", "x_dim_group_range", "chunk_size", "delta_softplus", "dt_limit", "D_has_hdim", "B_scale", "C_scale", "dt_scale")
-        norm = ("eps", "z_scale", "group_size", "norm_before_gate", "use_float16_output", "bias")
-        return (tuple((c, k) for k in conv) + tuple((s, k) for k in scan) + tuple((n, k) for k in norm)
-                + tuple((h, k) for k in ("x_H_scale", "had_scale")) + ((m["out_proj"].__dict__, "alpha"),))
 
     def _native_block(self, dev):
         p, D, N, G, H = _lib.QaMamba2Params(), self.d_ssm, self.d_state, self.ngroups, self.nheads

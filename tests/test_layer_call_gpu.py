@@ -109,3 +109,24 @@ def test_changed_modules_are_seen(dev, cls, build):
     hook = m.conv1d.register_forward_hook(lambda *a: seen.append(1))
     assert torch.equal(m.forward(h), third) and seen           # hooked modules run one by one
     hook.remove()
+
+
+@pytest.mark.parametrize("cls,build", MIXERS)
+def test_weights_held_as_parameters_are_followed(dev, cls, build):
+    """A weight that is a Parameter (no buffer) when the first call is made, replaced before the second."""
+    m, g = build(cls, dev, seed=6)
+    h = _ri(dev, g, 2, 20, 256)
+    outs = []
+    for turn in range(3):
+        w = m.out_proj.weight
+        # (int8 weights are the transposed view of contiguous rows)
+        w = w.roll(turn, 0) if w.dtype == torch.uint8 else w.t().roll(turn, 0).contiguous().t()
+        if turn == 0:
+            del m.out_proj._buffers["weight"]
+        m.out_proj.weight = torch.nn.Parameter(w, requires_grad=False)
+        outs.append(_layer_call.call(m, h, None, None, False))
+        want = m._forward_modules(h, None, None)
+        # (as in _close: fp16 scan outputs may differ in the last place; other rows of the weight differ by the whole range)
+        assert outs[-1] is not None and float((outs[-1].float() - want.float()).abs().max()) <= 2e-2 * float(want.float().abs().max()), turn
+        del w
+    assert not torch.equal(outs[0], outs[1]) and not torch.equal(outs[1], outs[2])

@@ -1,0 +1,88 @@
+"""The plan behind a mixer call (quamba_amd._host.Plan) on the host alone: what it notices about a layer, what it keeps."""
+import gc
+import weakref
+
+import pytest
+import torch
+import torch.nn as nn
+
+from quamba_amd import W4A8QMamba, W4A8QMamba2, W8A8QMamba, W8A8QMamba2, _layer_call
+
+MIXERS = [W8A8QMamba, W4A8QMamba, W8A8QMamba2, W4A8QMamba2]
+HIDDEN = torch.zeros(1, 1, 256, dtype=torch.int8)
+
+
+def _mixer(cls):
+    if cls in (W8A8QMamba, W4A8QMamba):
+        return cls(256, 16, 4, device="cpu")
+    return cls(256, 64, 4, 2, 64, ngroups=2, chunk_size=64, device="cpu", x_nhead_group=2, x_ndim_group=2)
+
+
+def _unchanged(plan):
+    """None: the plan's layer (which the library does not cover, on the CPU); False: not that layer any more."""
+    return plan.run(HIDDEN, None, None, False) is None
+
+
+def _tensors(mixer):
+    return [(m, name) for m in mixer._modules.values() for name, t in m._buffers.items() if t is not None]
+
+
+@pytest.mark.parametrize("cls", MIXERS)
+@pytest.mark.parametrize("held", ["buffer", "parameter", "attribute"])
+def test_every_tensor_is_watched_wherever_the_module_holds_it(cls, held):
+    m = _mixer(cls)
+
+    def hold(module, name, t):
+        for d in (module._buffers, module._parameters, module.__dict__):
+            d.pop(name, None)
+        if held == "buffer":
+            module.register_buffer(name, t)
+        elif held == "parameter":
+            module.register_parameter(name, nn.Parameter(t, requires_grad=False))
+        else:
+            module.__dict__[name] = t
+
+    for module, name in _tensors(m):
+        hold(module, name, getattr(module, name))
+    plan = _layer_call._make(m)
+    assert _unchanged(plan)
+    for module, name in _tensors(m) + [(mod, n) for mod in m._modules.values() for n, t in {**mod._parameters, **mod.__dict__}.items() if torch.is_tensor(t)]:
+        old = getattr(module, name)
+        gone = weakref.ref(old)
+        new = old.clone().contiguous()
+        if held == "attribute":
+            module.__dict__[name] = new
+        else:
+            setattr(module, name, nn.Parameter(new, requires_grad=False) if held == "parameter" else new)
+        del old, new
+        assert not _unchanged(plan), name
+        assert gone() is not None, f"{name}: its address is in the plan's block"
+        plan = _layer_call._make(m)
+        assert _unchanged(plan), name
+
+
+@pytest.mark.parametrize("cls", [W8A8QMamba, W8A8QMamba2])
+def test_replaced_modules_numbers_and_memory_are_seen(cls):
+    m = _mixer(cls)
+    plan = _layer_call._make(m)
+    m.had.x_H_scale = float(m.had.x_H_scale) + 0.0           # another object, the same number
+    assert _unchanged(plan)
+    m.had.x_H_scale = 3.0
+    assert not _unchanged(plan)
+    plan = _layer_call._make(m)
+    m.out_proj.weight.data = m.out_proj.weight.clone()       # the same object, other memory
+    assert not _unchanged(plan)
+    plan = _layer_call._make(m)
+    m.had = type(m.had)(m.had.dim)
+    assert not _unchanged(plan)
+
+
+def test_a_plan_does_not_keep_its_mixer():
+    m = _mixer(W8A8QMamba)
+    m.__dict__["_plan"] = _layer_call._make(m)
+    m.conv1d.__dict__["owner"] = m                           # leads from the plan back to the mixer
+    m.__dict__["_plan"] = _layer_call._make(m)
+    gone = weakref.ref(m)
+    del m
+    gc.collect()
+    assert gone() is None
