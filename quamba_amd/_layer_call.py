@@ -45,7 +45,10 @@ def _ptr(t, dtype, numel, device, align=1):
     if t is None:
         return None
     _need(t.dtype == dtype and t.numel() == numel and t.device == device and t.is_contiguous())
-    a = t.data_ptr()
+    try:
+        a = t.data_ptr()
+    except RuntimeError as e:                  # no memory of its own (under vmap, say)
+        raise _Unsupported from e
     _need(a % align == 0)
     return a
 

@@ -75,7 +75,16 @@ struct PlanObject {
     State* s;
 };
 
-const void* address_of(PyObject* t) { return THPVariable_Unpack(t).const_data_ptr(); }
+// Where a tensor's memory is.  One that only stands for others (under vmap, say, or a fake one) has none of its own: a layer
+// that holds such a tensor runs module by module.
+const char kNoMemory = 0;
+const void* address_of(PyObject* t) noexcept {
+    try {
+        return THPVariable_Unpack(t).const_data_ptr();
+    } catch (...) {
+        return &kNoMemory;
+    }
+}
 
 // ---- making a plan ------------------------------------------------------------------------------------------------
 PyObject* keep(PyObject* o) {
@@ -97,7 +106,7 @@ void plan_free(State* s) {
 // Plan(watched, hooks, native): the dicts the layer was made from, the dicts that have to be empty, and None for a layer the
 // library does not cover, or (family, block bytes, (forward, step, workspace) addresses, (conv channels, state shape,
 // (forward widths, step widths)), output padding, a tensor on the layer's device, (get_device, set_device, get_stream, out-of-memory error)).
-int plan_init(PlanObject* self, PyObject* args, PyObject*) {
+int make_plan(PlanObject* self, PyObject* args) {
     PyObject *watched, *hooks, *native;
     if (!PyArg_ParseTuple(args, "O!O!O", &PyTuple_Type, &watched, &PyTuple_Type, &hooks, &native)) return -1;
     for (PyObject* dicts : {watched, hooks})
@@ -122,6 +131,10 @@ int plan_init(PlanObject* self, PyObject* args, PyObject*) {
     }
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(hooks); ++i) s->no_hooks.push_back(keep(PyTuple_GET_ITEM(hooks, i)));
     if (native == Py_None) return 0;
+    if (!PyTuple_Check(native)) {
+        PyErr_SetString(PyExc_TypeError, "the native part of a plan is a tuple or None");
+        return -1;
+    }
 
     const char* block;
     Py_ssize_t block_len;
@@ -150,9 +163,30 @@ int plan_init(PlanObject* self, PyObject* args, PyObject*) {
     s->d_model = s->family == 1 ? s->m1.d_model : s->m2.d_model;
     s->n_out = s->family == 1 ? s->m1.out_proj.n : s->m2.out_proj.n;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(shape); ++i) s->ssm_shape.push_back(PyLong_AsLongLong(PyTuple_GET_ITEM(shape, i)));
+    if (PyErr_Occurred()) return -1;
     s->device = THPVariable_Unpack(anchor).device();
     s->usable = true;
+    for (const Entry& e : s->tensors) s->usable = s->usable && e.address != &kNoMemory;
     return 0;
+}
+
+// No C++ exception passes through the interpreter.
+template <class Result, class Body>
+Result guarded(const State* s, Result failed, Body&& body) {
+    try {
+        return body();
+    } catch (const c10::OutOfMemoryError& e) {
+        PyErr_SetString(s && s->oom ? s->oom : PyExc_MemoryError, e.what_without_backtrace());
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    } catch (...) {
+        PyErr_SetString(PyExc_RuntimeError, "unknown C++ exception");
+    }
+    return failed;
+}
+
+int plan_init(PlanObject* self, PyObject* args, PyObject*) {
+    return guarded(nullptr, -1, [&] { return make_plan(self, args); });
 }
 
 // ---- using it -----------------------------------------------------------------------------------------------------
@@ -271,20 +305,14 @@ PyObject* plan_run(PlanObject* self, PyObject* const* args, Py_ssize_t nargs) {
     State& s = *self->s;
     const int step = PyObject_IsTrue(args[3]);
     if (step < 0) return nullptr;
-    const int same = verify(s);
-    if (same == 0) Py_RETURN_FALSE;
-    if (same < 0 || !s.usable || !THPVariable_Check(args[0])) Py_RETURN_NONE;
-    for (int i = 1; i < 3; ++i)
-        if (args[i] != Py_None && !THPVariable_Check(args[i])) Py_RETURN_NONE;
-    try {
+    return guarded(&s, static_cast<PyObject*>(nullptr), [&]() -> PyObject* {
+        const int same = verify(s);
+        if (same == 0) Py_RETURN_FALSE;
+        if (same < 0 || !s.usable || !THPVariable_Check(args[0])) Py_RETURN_NONE;
+        for (int i = 1; i < 3; ++i)
+            if (args[i] != Py_None && !THPVariable_Check(args[i])) Py_RETURN_NONE;
         return run_on_device(s, args[0], args[1], args[2], step);
-    } catch (const c10::OutOfMemoryError& e) {
-        PyErr_SetString(s.oom, e.what_without_backtrace());
-        return nullptr;
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
-    }
+    });
 }
 
 // Copies and pickles of a layer start without a plan.

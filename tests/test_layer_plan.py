@@ -86,3 +86,33 @@ def test_a_plan_does_not_keep_its_mixer():
     del m
     gc.collect()
     assert gone() is None
+
+
+@pytest.mark.parametrize("cls", MIXERS)
+def test_a_tensor_without_memory_of_its_own(cls):
+    """Under vmap a buffer stands for a batch of tensors and has no address: the plan yields to the modules (once, and
+    without a plan made anew on each call), and an existing plan sees the exchange."""
+    m = _mixer(cls)
+    plan = _layer_call._make(m)
+    held = m.out_proj._buffers["weight"]
+    seen = []
+
+    def body(w):
+        m.out_proj._buffers["weight"] = w
+        inner = _layer_call._make(m)
+        seen.extend([_unchanged(plan), _unchanged(inner), _layer_call.call(m, HIDDEN, None, None, False), _unchanged(m.__dict__["_plan"])])
+        return w
+
+    torch.vmap(body)(torch.stack([held, held]))
+    m.out_proj._buffers["weight"] = held
+    assert seen == [False, True, None, True]
+    assert not _unchanged(m.__dict__["_plan"])
+
+
+def test_a_plan_made_of_the_wrong_things_is_an_error():
+    plan = _layer_call._plan_class()
+    for args in ((), ((), ()), ((), (), 3), ((3,), (), None), ((), (3,), None), ((), (), (1, b"", (1, 2, 3)))):
+        with pytest.raises(TypeError):
+            plan(*args)
+    with pytest.raises(TypeError):
+        plan.__new__(plan).run(HIDDEN, None, None, False)
