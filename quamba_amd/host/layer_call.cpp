@@ -272,29 +272,46 @@ PyObject* enqueue(State& s, Params p, const at::Tensor& hidden, PyObject* conv_o
     return THPVariable_Wrap(out);
 }
 
+// The layer's device for as long as this stands, however the call ends.
+class OnDevice {
+  public:
+    explicit OnDevice(const State& s) : s_(s) {
+        PyObject* at = PyObject_CallNoArgs(s.get_device);
+        if (!at) return;
+        back_ = PyLong_AsLong(at);
+        Py_DECREF(at);
+        if (PyErr_Occurred()) return;
+        ok = back_ == s.device.index();
+        if (!ok) ok = moved_ = set(s.device.index());
+    }
+    ~OnDevice() {
+        if (!moved_) return;
+        PyObject *type, *value, *trace;
+        PyErr_Fetch(&type, &value, &trace);
+        if (!set(back_)) PyErr_WriteUnraisable(s_.set_device);
+        PyErr_Restore(type, value, trace);
+    }
+    OnDevice(const OnDevice&) = delete;
+    bool ok = false;               // otherwise an error is set
+
+  private:
+    bool set(long device) {
+        PyObject* r = PyObject_CallFunction(s_.set_device, "l", device);
+        Py_XDECREF(r);
+        return r != nullptr;
+    }
+    const State& s_;
+    long back_ = 0;
+    bool moved_ = false;
+};
+
 PyObject* run_on_device(State& s, PyObject* hidden_o, PyObject* conv_o, PyObject* ssm_o, int step) {
     const at::Tensor& hidden = THPVariable_Unpack(hidden_o);
     if (hidden.scalar_type() != at::kChar || hidden.device() != s.device || hidden.dim() != 3 || !hidden.is_contiguous() ||
         hidden.size(2) != s.d_model || hidden.size(0) == 0 || hidden.size(1) == 0 || hidden.size(0) > 65535 || hidden.size(1) > 0x7fffffff) Py_RETURN_NONE;
-    PyObject* at_o = PyObject_CallNoArgs(s.get_device);
-    if (!at_o) return nullptr;
-    const long at_dev = PyLong_AsLong(at_o);
-    Py_DECREF(at_o);
-    const bool move = at_dev != s.device.index();
-    if (move) {
-        PyObject* r = PyObject_CallFunction(s.set_device, "i", static_cast<int>(s.device.index()));
-        if (!r) return nullptr;
-        Py_DECREF(r);
-    }
-    PyObject* out = s.family == 1 ? enqueue(s, s.m1, hidden, conv_o, ssm_o, step) : enqueue(s, s.m2, hidden, conv_o, ssm_o, step);
-    if (move) {
-        PyObject *type, *value, *trace;
-        PyErr_Fetch(&type, &value, &trace);
-        PyObject* r = PyObject_CallFunction(s.set_device, "l", at_dev);
-        Py_XDECREF(r);
-        PyErr_Restore(type, value, trace);
-    }
-    return out;
+    const OnDevice on(s);
+    if (!on.ok) return nullptr;
+    return s.family == 1 ? enqueue(s, s.m1, hidden, conv_o, ssm_o, step) : enqueue(s, s.m2, hidden, conv_o, ssm_o, step);
 }
 
 PyObject* plan_run(PlanObject* self, PyObject* const* args, Py_ssize_t nargs) {

@@ -1,4 +1,5 @@
 """The plan behind a mixer call (quamba_amd._host.Plan) on the host alone: what it notices about a layer, what it keeps."""
+import ctypes as C
 import gc
 import weakref
 
@@ -6,7 +7,7 @@ import pytest
 import torch
 import torch.nn as nn
 
-from quamba_amd import W4A8QMamba, W4A8QMamba2, W8A8QMamba, W8A8QMamba2, _layer_call
+from quamba_amd import W4A8QMamba, W4A8QMamba2, W8A8QMamba, W8A8QMamba2, _layer_call, _lib
 
 MIXERS = [W8A8QMamba, W4A8QMamba, W8A8QMamba2, W4A8QMamba2]
 HIDDEN = torch.zeros(1, 1, 256, dtype=torch.int8)
@@ -116,3 +117,53 @@ def test_a_plan_made_of_the_wrong_things_is_an_error():
             plan(*args)
     with pytest.raises(TypeError):
         plan.__new__(plan).run(HIDDEN, None, None, False)
+
+
+class _Runtime:
+    """A plan over host functions in place of the library's and the device's, for what the plan does around them."""
+    FORWARD = C.CFUNCTYPE(C.c_int, C.POINTER(_lib.QaMamba1Params), C.c_void_p)
+    WORKSPACE = C.CFUNCTYPE(C.c_int64, C.POINTER(_lib.QaMamba1Params), C.c_int)
+
+    def __init__(self, status=0, workspace=256, stream=0, current=3):
+        self.current, self.calls, self.blocks = current, [], []
+        self.device, self.stream = current, stream
+        self.fns = self.FORWARD(lambda p, s: self.enter("forward", p, status)), self.FORWARD(lambda p, s: self.enter("step", p, status))
+        self.workspace = self.WORKSPACE(lambda p, step: workspace)
+        block = _lib.QaMamba1Params()
+        block.d_model, block.out_proj.n = 256, 256
+        addresses = tuple(C.cast(f, C.c_void_p).value for f in self.fns + (self.workspace,))
+        runtime = (lambda: self.device, self.set_device, self.get_stream, MemoryError)
+        self.plan = _layer_call._plan_class()((), (), (1, bytes(block), addresses, (512, (512, 16), ((4, 3), (4, 3))), 0, torch.empty(0), runtime))
+
+    def enter(self, what, p, status):
+        self.calls.append((what, self.device))
+        self.blocks.append(_lib.QaMamba1Params.from_buffer_copy(p.contents))
+        return status
+
+    def set_device(self, index):
+        self.device = index
+
+    def get_stream(self, index):
+        if isinstance(self.stream, Exception):
+            raise self.stream
+        return self.stream
+
+
+def test_the_current_device_comes_back_however_the_call_ends():
+    here = -1                                                # (the index of a device without one)
+    r = _Runtime()
+    assert r.plan.run(HIDDEN, None, None, False).shape == (1, 1, 256) and r.calls == [("forward", here)] and r.device == 3
+    r = _Runtime(status=-5)
+    assert r.plan.run(HIDDEN, None, None, True) == -5 and r.calls == [("step", here)] and r.device == 3
+    r = _Runtime(workspace=1 << 60)                          # more than there is: the allocation throws
+    with pytest.raises(RuntimeError):
+        r.plan.run(HIDDEN, None, None, False)
+    assert not r.calls and r.device == 3
+    r = _Runtime(stream=KeyError("no stream"))
+    with pytest.raises(KeyError):
+        r.plan.run(HIDDEN, None, None, False)
+    assert r.device == 3
+    r = _Runtime(current=here)                               # on the layer's device already
+    assert torch.is_tensor(r.plan.run(HIDDEN, None, None, False)) and r.device == here
+    r = _Runtime()
+    assert r.plan.run(HIDDEN.float(), None, None, False) is None and not r.calls and r.device == 3
