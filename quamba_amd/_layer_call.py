@@ -4,7 +4,8 @@ A mixer's weights, scales and sizes are gathered into the library's parameter bl
 (quamba_amd._host.Plan, host/layer_call.cpp), for as long as its sub-modules and everything they hold - attributes, buffers
 and parameters, tensors with their addresses - are the ones the block was made from; running the plan verifies that,
 allocates output and workspace and enqueues the layer.  Mixers, tensors or states the library call does not cover (other
-sub-module classes, forward hooks, views with gaps, unusual sizes) yield None, and the mixer runs its modules one by one.
+sub-module classes or replaced methods, forward hooks, views with gaps, unusual sizes) yield None, and the mixer runs its
+modules one by one.
 """
 import ctypes as C
 
@@ -90,6 +91,33 @@ def _native(mixer):
     return family, bytes(block), fns, dims, mixer.out_proj.pad_out, mixer.out_proj.weight, runtime
 
 
+# class -> what is callable in it, as it was when this package was imported
+_CODE = {}
+
+
+def _code_of(cls):
+    return {n: f for n, f in vars(cls).items() if callable(f) or isinstance(f, (classmethod, staticmethod, property))}
+
+
+def remember(*classes):
+    """The library call stands for the methods of these classes as they are now."""
+    for cls in classes:
+        for c in cls.__mro__:
+            if c.__module__.split(".")[0] == __package__ or c is torch.nn.Module:
+                _CODE[c] = _code_of(c)
+
+
+def _own_code(module):
+    """Whether calling the module's methods runs the code of its class: no method replaced on the instance (as offloading
+    and tracing tools wrap modules) or on the class, no compiled form in their place."""
+    if module.__dict__.get("_compiled_call_impl") is not None:
+        return False
+    for c in type(module).__mro__:
+        if c in _CODE and _code_of(c) != _CODE[c]:
+            return False
+    return not any(callable(getattr(type(module), n, None)) for n in module.__dict__)
+
+
 def _make(mixer):
     """The mixer's plan (one that only ever yields None where the library does not cover the mixer)."""
     mods = [m for m in mixer._modules.values() if m is not None]
@@ -98,8 +126,9 @@ def _make(mixer):
     for m in mods:
         watched += [m.__dict__, m._buffers, m._parameters]
         hooks += [m._forward_hooks, m._forward_pre_hooks]
+    watched += {c: None for m in mods for c in type(m).__mro__ if c in _CODE}
     try:
-        _need(mixer._native_modules() is not None)
+        _need(mixer._native_modules() is not None and all(_own_code(m) for m in mods))
         native = _native(mixer)
     except _Unsupported:
         native = None

@@ -5,8 +5,8 @@
 // layer (qa_mamba1_* / qa_mamba2_*, include/quamba_amd.h) together with what it was made from, and run() verifies all of it,
 // allocates output and workspace, and enqueues the layer.
 //
-// What it was made from is a list of dicts - the mixer's sub-modules, and of each of them its attributes, buffers and
-// parameters - as they were, entry by entry: a tensor whose address is in the block is in one of them wherever the module
+// What it was made from is a list of dicts - the mixer's sub-modules, of each of them its attributes, buffers and
+// parameters, and their classes (another function in the place of a method is another layer) - as they were, entry by entry: a tensor whose address is in the block is in one of them wherever the module
 // keeps it, the entry keeps it alive, and every call compares the entries with what the dicts hold now (values by identity,
 // numbers by value, tensors by their address as well).
 //
@@ -103,7 +103,7 @@ void plan_free(State* s) {
     delete s;
 }
 
-// Plan(watched, hooks, native): the dicts the layer was made from, the dicts that have to be empty, and None for a layer the
+// Plan(watched, hooks, native): the dicts and classes the layer was made from, the dicts that have to be empty, and None for a layer the
 // library does not cover, or (family, block bytes, (forward, step, workspace) addresses, (conv channels, state shape,
 // (forward widths, step widths)), output padding, a tensor on the layer's device, (get_device, set_device, get_stream, out-of-memory error)).
 int make_plan(PlanObject* self, PyObject* args) {
@@ -111,15 +111,16 @@ int make_plan(PlanObject* self, PyObject* args) {
     if (!PyArg_ParseTuple(args, "O!O!O", &PyTuple_Type, &watched, &PyTuple_Type, &hooks, &native)) return -1;
     for (PyObject* dicts : {watched, hooks})
         for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(dicts); ++i)
-            if (!PyDict_Check(PyTuple_GET_ITEM(dicts, i))) {
-                PyErr_SetString(PyExc_TypeError, "a plan is made from dicts");
+            if (!PyDict_Check(PyTuple_GET_ITEM(dicts, i)) && (dicts == hooks || !PyType_Check(PyTuple_GET_ITEM(dicts, i)))) {
+                PyErr_SetString(PyExc_TypeError, "a plan is made from dicts and classes");
                 return -1;
             }
     State* s = new State;
     plan_free(self->s);
     self->s = s;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(watched); ++i) {
-        PyObject* dict = keep(PyTuple_GET_ITEM(watched, i));
+        PyObject* from = PyTuple_GET_ITEM(watched, i);
+        PyObject* dict = keep(PyType_Check(from) ? reinterpret_cast<PyTypeObject*>(from)->tp_dict : from);
         s->watches.push_back({dict, version_of(dict), {}});
         PyObject *key, *value;
         Py_ssize_t pos = 0;

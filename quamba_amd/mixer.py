@@ -17,13 +17,18 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _layer_call, _lib
+from . import _layer_call, _lib, ops
 from ._layer_call import _need, _ptr, linear_block
-from .conv import QCausalConv1D
+from .chunk_scan import Quamba2ChunkScan
+from .conv import QCausalConv1D, Quamb2Conv1D
 from .hadamard import QHadamard
 from .linear import (W4A8B8O8Linear, W4A8B8O8LinearParallel, W4A8B16O16Linear, W8A8B8O8Linear, W8A8B8O8LinearParallel,
                      W8A8B16O16Linear)
+from .norm import QRMSNormGated
 from .sscan import QSScan
+
+_layer_call.remember(W4A8B8O8Linear, W4A8B8O8LinearParallel, W4A8B16O16Linear, W8A8B8O8Linear, W8A8B8O8LinearParallel, W8A8B16O16Linear,
+                     QCausalConv1D, Quamb2Conv1D, QSScan, Quamba2ChunkScan, QRMSNormGated, QHadamard)
 
 
 class W8A8QMamba(nn.Module):
@@ -108,6 +113,7 @@ class W8A8QMamba(nn.Module):
         p.D, p.dt_bias = _ptr(s.D, torch.int8, D, dev), _ptr(s.dt_bias, torch.int8, D, dev)
         for name in ("A_scale", "D_scale", "dt_bias_scale", "u_scale", "dt_scale", "B_scale", "C_scale", "z_scale", "ssm_state_scale"):
             setattr(p, name, _ptr(getattr(s, name), torch.float32, 1, dev))
+        _need(self.had.transform_fn is ops.hadamard_quant)
         p.had_scale = self.had.had_scale / float(self.had.x_H_scale)
         widths = (self.d_conv, self.d_conv - 1)                        # of the conv state, in forward and in step
         return p, (D, (D, N), (widths, widths))
@@ -218,9 +224,6 @@ class W4A8QMamba2(nn.Module):
                  chunk_size=256, use_had_transform=True, layer_idx=None, device=None, state_dtype=torch.int8,
                  x_nhead_group=4, x_ndim_group=4, **kwargs):
         super().__init__()
-        from .chunk_scan import Quamba2ChunkScan
-        from .conv import Quamb2Conv1D
-        from .norm import QRMSNormGated
         assert bias is False, "Only support bias=False for now"
         assert rmsnorm, "Only support Mamba2 block with rmsnorm"
         assert use_had_transform, "the mixer is built with the Hadamard + quantisation op in front of out_proj"
@@ -252,9 +255,6 @@ class W4A8QMamba2(nn.Module):
 
     def _native_modules(self):
         """The sub-modules in the order of the library call, or None when one of them is not the stock class."""
-        from .chunk_scan import Quamba2ChunkScan
-        from .conv import Quamb2Conv1D
-        from .norm import QRMSNormGated
         m = self._modules
         mods = (m["in_proj"], m["conv1d"], m["qchunk_scan"], m["norm"], m["had"], m["out_proj"])
         want = (self._in_proj_cls, Quamb2Conv1D, Quamba2ChunkScan, QRMSNormGated, QHadamard, self._out_proj_cls)
@@ -295,6 +295,7 @@ class W4A8QMamba2(nn.Module):
         p.norm_eps, p.norm_z_scale, p.norm_before_gate = n.eps, float(n.z_scale), int(bool(n.norm_before_gate))
         p.norm_group_size = D if n.group_size is None else n.group_size
         p.norm_weight = _ptr(n.weight, torch.float16, D, dev)
+        _need(self.had.transform_fn is ops.hadamard_quant)
         p.had_scale = self.had.had_scale / float(self.had.x_H_scale)
         p.A_log = _ptr(s.A_log, torch.int8, H, dev)
         p.D = _ptr(s.D, torch.int8, D if s.D_has_hdim else H, dev)

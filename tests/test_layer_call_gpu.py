@@ -130,3 +130,36 @@ def test_weights_held_as_parameters_are_followed(dev, cls, build):
         assert outs[-1] is not None and float((outs[-1].float() - want.float()).abs().max()) <= 2e-2 * float(want.float().abs().max()), turn
         del w
     assert not torch.equal(outs[0], outs[1]) and not torch.equal(outs[1], outs[2])
+
+
+@pytest.mark.parametrize("cls,build", MIXERS)
+def test_replaced_methods_are_called(dev, cls, build, monkeypatch):
+    m, g = build(cls, dev, seed=7)
+    h = _ri(dev, g, 2, 20, 256)
+    first, seen = m.forward(h), []
+
+    def noting(f):
+        return lambda *a, **k: (seen.append(f), f(*a, **k))[1]
+
+    def runs_the_modules():
+        seen.clear()
+        out = m.forward(h)
+        # (as in _close: fp16 scan outputs may differ in the last place)
+        assert seen and float((out.float() - first.float()).abs().max()) <= 2e-2 * float(first.float().abs().max())
+
+    m.conv1d.forward = noting(m.conv1d.forward)                # on the instance
+    runs_the_modules()
+    del m.conv1d.forward
+    m.out_proj._call_impl = noting(m.out_proj._call_impl)
+    runs_the_modules()
+    del m.out_proj._call_impl
+    if not hasattr(m, "norm"):
+        kept = m.had.transform_fn
+        m.had.transform_fn = noting(kept)
+        runs_the_modules()
+        m.had.transform_fn = kept
+    with monkeypatch.context() as patch:                       # on the class
+        patch.setattr(type(m.conv1d), "forward", noting(type(m.conv1d).forward))
+        runs_the_modules()
+    seen.clear()
+    assert torch.equal(m.forward(h), first) and not seen and _layer_call.call(m, h, None, None, False) is not None
