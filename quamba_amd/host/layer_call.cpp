@@ -229,6 +229,7 @@ PyObject* enqueue(State& s, Params p, const at::Tensor& hidden, PyObject* conv_o
     p.batch = static_cast<int32_t>(batch);
     p.seqlen = static_cast<int32_t>(len);
     p.hidden = hidden.const_data_ptr<int8_t>();
+    if (reinterpret_cast<uintptr_t>(p.hidden) % 16 != 0) Py_RETURN_NONE;
     if (conv_o != Py_None) {
         const at::Tensor& c = THPVariable_Unpack(conv_o);
         if (c.scalar_type() != at::kChar || c.device() != s.device || c.dim() != 3 || c.size(0) != batch || c.size(1) != s.conv_dim ||

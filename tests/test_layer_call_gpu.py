@@ -163,3 +163,25 @@ def test_replaced_methods_are_called(dev, cls, build, monkeypatch):
         runs_the_modules()
     seen.clear()
     assert torch.equal(m.forward(h), first) and not seen and _layer_call.call(m, h, None, None, False) is not None
+
+
+@pytest.mark.parametrize("cls,build", MIXERS)
+def test_unaligned_hidden_states(dev, cls, build):
+    """Contiguous, 8 bytes off: the W8A8 Mamba1 forward pads token counts that are no multiple of 16 and so takes it; where the
+    modules refuse it, so does the mixer, with the states as they were."""
+    m, g = build(cls, dev, seed=8)
+    for batch, seqlen in ((2, 21), (1, 32)):
+        h = torch.empty(batch * seqlen * 256 + 8, dtype=torch.int8, device=dev)[8:].view(batch, seqlen, 256)
+        h.copy_(_ri(dev, g, batch, seqlen, 256))
+        assert h.is_contiguous() and h.data_ptr() % 16 == 8
+        if cls is W8A8QMamba and seqlen == 21:
+            want = m.forward(h.clone())
+            assert float((m.forward(h).float() - want.float()).abs().max()) <= 2e-2 * float(want.float().abs().max())
+        else:
+            with pytest.raises(RuntimeError):
+                m.forward(h)
+    conv, ssm = _states(m, dev, g, 2, torch.int8, 4)
+    kept = conv.clone(), ssm.clone()
+    with pytest.raises(RuntimeError):
+        m.step(h[:, :2].reshape(2, 1, 256), conv, ssm)
+    assert torch.equal(conv, kept[0]) and torch.equal(ssm, kept[1])

@@ -149,6 +149,17 @@ class _Runtime:
         return self.stream
 
 
+def test_hidden_states_the_products_cannot_read_go_to_the_modules():
+    """Contiguous but not 16-byte aligned: refused before anything is enqueued, whatever the token count."""
+    r = _Runtime()
+    room = torch.zeros(5 * 256 + 16, dtype=torch.int8)
+    start = -room.data_ptr() % 16
+    for tokens, offset in ((1, 1), (3, 8), (5, 4)):
+        h = room[start + offset:][:tokens * 256].view(1, tokens, 256)
+        assert h.is_contiguous() and r.plan.run(h, None, None, False) is None and not r.calls
+    assert torch.is_tensor(r.plan.run(room[start:][:256].view(1, 1, 256), None, None, False))
+
+
 def test_the_current_device_comes_back_however_the_call_ends():
     here = -1                                                # (the index of a device without one)
     r = _Runtime()
