@@ -139,7 +139,7 @@ int qa_quamba2_conv1d_update(const QaConv2Params* p, void* stream);
 enum { QA_NORM_OUT_F16 = 0, QA_NORM_OUT_I8_STATIC = 1, QA_NORM_OUT_I8_DYNAMIC = 2 };
 
 typedef struct QaNormGatedParams {
-    int32_t rows, dim, group_size;   /* dim % group_size == 0, group_size % 8 == 0, group_size <= 8192 */
+    int32_t rows, dim, group_size;   /* dim % group_size == 0, group_size % 8 == 0, group_size <= 32768 */
     int32_t norm_before_gate;
     int32_t out_mode;
     float eps, z_scale, out_scale;
@@ -475,6 +475,8 @@ int qa_ssd_chunk_scan_fwd_noalloc(const QaSsdParams* p, void* stream);
  * caller-supplied workspace.  forward: a prompt from zero states (quamba/qMambaLayer.py:895-943, qMamba2.py:905-985);
  * step: one token per sequence, both states advanced in place (qMambaLayer.py:945-1010, qMamba2.py:987-1068).
  * Activations stay row-major (token, channel) from in_proj to out_proj.
+ * A call is refused (any status but QA_ERR_LAUNCH) before its first launch, with both states as they were: sizes the
+ * kernels do not take give workspace_bytes 0 as well; hidden and the norm's weight are 16-byte aligned.
  * ---------------------------------------------------------------------------------------- */
 /* a projection with one row of activations: the rule its module applies then */
 typedef enum QaRowRule { QA_ROW_SCALES = 0, QA_ROW_ALPHA = 1, QA_ROW_HALF_AWAY = 2 } QaRowRule;

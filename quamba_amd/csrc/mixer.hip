@@ -9,7 +9,11 @@
 // channels per lane, the scan stages token-major rows, x_proj and dt_proj are plain row-major products - so no second
 // copy of the conv's output, no transposition of B and C, no padding of the token count, and prompts of any length
 // run on the same kernels.
+//
+// A call is refused before its first launch or not at all (validate, ready): a step advances both states in place, and one
+// that stopped half way could not be made again another way.
 #include "gemv.hpp"
+#include "hadamard_core.hpp"
 #include "mixer_common.hpp"
 #include "ssd_common.hpp"
 
@@ -76,9 +80,20 @@ int project(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows, voi
     return qa_gemm_w8a8(&p, stream);
 }
 
-bool linear_ok(const QaLinearParams& w) {
-    return (w.bits == 8 || w.bits == 4) && w.n > 0 && w.k > 0 && w.weight && w.col_scale && w.row_scale;
+// what the products would refuse: `rows` rows of activations, lda apart and 16-byte aligned, against w
+int linear_check(const QaLinearParams& w, int64_t rows, int64_t lda) {
+    if ((w.bits != 8 && w.bits != 4) || w.n < 1 || w.k < 1 || !w.weight || !w.col_scale || !w.row_scale) return QA_ERR_NULL;
+    if (w.k % (w.bits == 8 ? 16 : 128) != 0 || (w.bits == 8 && w.col_numel != 1 && w.col_numel != w.n)) return QA_ERR_SHAPE;
+    if (lda % 16 != 0 || lda < w.k || !aligned16(w.weight)) return QA_ERR_STRIDE;
+    // 32-bit offsets (4-bit weights from the tile's first row)
+    const int64_t weights = static_cast<int64_t>(w.n) * w.k;
+    if (rows * lda >= 0x70000000LL || (w.bits == 8 ? weights >= 0x70000000LL : 64LL * w.k > 0x7fffffffLL || weights > 64LL * 0x7fffff00LL)) return QA_ERR_SHAPE;
+    return QA_OK;
 }
+
+int hadamard_check(int dim) { return dim <= 32768 && hadamard_shape(dim).s != 0 ? QA_OK : QA_ERR_UNSUPPORTED; }
+
+constexpr int64_t kConvSteps = 65535LL * 4 * 256;       // of a sequence: the grid of the forward conv
 
 // in_proj of a decode step with the conv's step behind it in one launch (QA_ERR_UNSUPPORTED: two launches)
 int project_conv(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows, int8_t* d, int ch0, const QaConv2Params& conv, void* stream) {
@@ -184,23 +199,91 @@ QaConv2Params conv_of(const QaMamba1Params& p, const Mamba1Buffers& b) {
 
 int validate(const QaMamba1Params* p) {
     if (!p) return QA_ERR_NULL;
-    if (p->batch < 1 || p->seqlen < 1 || p->batch > 65535 || static_cast<int64_t>(p->batch) * p->seqlen > 0x7fffffff) return QA_ERR_SHAPE;
-    if (p->d_state != 16 || p->d_conv < 2 || p->d_conv > 4 || p->d_inner % 16 != 0 || p->dt_rank % 4 != 0) return QA_ERR_UNSUPPORTED;
-    for (const QaLinearParams* w : {&p->in_proj, &p->x_proj, &p->dt_proj, &p->out_proj})
-        if (!linear_ok(*w)) return QA_ERR_NULL;
+    if (p->batch < 1 || p->seqlen < 1 || p->batch > 65535 || p->seqlen > kConvSteps || static_cast<int64_t>(p->batch) * p->seqlen > 0x7fffffff) return QA_ERR_SHAPE;
+    if (p->d_state != 16 || p->d_conv < 2 || p->d_conv > 4 || p->d_inner < 16 || p->d_inner % 16 != 0 || p->dt_rank % 4 != 0) return QA_ERR_UNSUPPORTED;
     if (p->in_proj.k != p->d_model || p->in_proj.n != 2 * p->d_inner || p->x_proj.k != p->d_inner ||
         p->x_proj.n < p->dt_rank + 2 * p->d_state || p->x_proj.n % 4 != 0 || p->dt_proj.k != p->dt_rank ||
         p->dt_proj.n != p->d_inner || p->out_proj.k != p->d_inner) return QA_ERR_SHAPE;
     if (p->conv_state_len != p->d_conv && p->conv_state_len != p->d_conv - 1) return QA_ERR_SHAPE;
-    return QA_OK;
+    const int64_t t = static_cast<int64_t>(p->batch) * p->seqlen;
+    QA_TRY(linear_check(p->in_proj, t, p->d_model));
+    QA_TRY(linear_check(p->x_proj, t, p->d_inner));
+    QA_TRY(linear_check(p->dt_proj, t, p->x_proj.n));
+    QA_TRY(linear_check(p->out_proj, t, p->d_inner));
+    return hadamard_check(p->d_inner);
 }
 
-int ready(const QaMamba1Params* p, bool states) {
+// dt_proj inside the scan (sscan_tm.hip) or as a product of its own
+bool dt_in_scan(const QaMamba1Params& p) {
+    return p.dt_proj.bits == 8 && p.dt_proj.k <= kSscanDtRank && p.x_proj.n % 16 == 0 && p.seqlen * static_cast<int64_t>(p.x_proj.n) < 1 << 30;
+}
+
+SscanDtProj scan_dt_of(const QaMamba1Params& p, const Mamba1Buffers& b) {
+    const QaLinearParams& w = p.dt_proj;
+    const int64_t dbl = p.x_proj.n;
+    return {static_cast<const int8_t*>(w.weight), b.x_dbl, p.seqlen * dbl, dbl, w.row_scale, w.col_scale, w.k, w.col_numel};
+}
+
+QaSScanParams scan_of(const QaMamba1Params& p, const Mamba1Buffers& b) {
+    QaSScanParams s = scan_sizes(p);
+    const int64_t dbl = p.x_proj.n, len = p.seqlen, d = p.d_inner;
+    s.delta_softplus = p.delta_softplus;
+    s.token_major = 1;
+    s.u_batch_stride = len * d; s.u_l_stride = d; s.u_d_stride = 1;
+    s.delta_batch_stride = len * d; s.delta_l_stride = d; s.delta_d_stride = 1;
+    s.z_batch_stride = len * 2 * d; s.z_l_stride = 2 * d; s.z_d_stride = 1;
+    s.B_batch_stride = s.C_batch_stride = len * dbl;
+    s.B_l_stride = s.C_l_stride = dbl;
+    s.B_dstate_stride = s.C_dstate_stride = 1;
+    s.A_d_stride = p.d_state; s.A_dstate_stride = 1;
+    s.out_batch_stride = len * d; s.out_l_stride = d; s.out_d_stride = 1;
+    s.u = b.x; s.delta = b.dt; s.A_log = p.A_log; s.B = b.x_dbl + p.dt_rank; s.C = s.B + p.d_state;
+    s.D = p.D; s.delta_bias = p.dt_bias; s.z = b.xz + d;
+    s.scale_u = p.u_scale; s.scale_delta = p.dt_scale; s.scale_A = p.A_scale; s.scale_B = p.B_scale; s.scale_C = p.C_scale;
+    s.scale_D = p.D_scale; s.scale_delta_bias = p.dt_bias_scale; s.scale_z = p.z_scale; s.scale_ssm_state = p.ssm_state_scale;
+    s.out = b.y;
+    if (p.state_is_fp32) s.last_state_f32 = static_cast<float*>(p.ssm_state);
+    else s.last_state_i8 = static_cast<int8_t*>(p.ssm_state);
+    s.workspace = b.scan.p; s.workspace_bytes = b.scan.bytes;
+    return s;
+}
+
+QaSsmUpdateParams update_of(const QaMamba1Params& p, const Mamba1Buffers& b) {
+    QaSsmUpdateParams u = {};
+    const int64_t d = p.d_inner;
+    u.batch = p.batch; u.nheads = 1; u.dim = p.d_inner; u.dstate = p.d_state; u.ngroups = 1;
+    u.dt_softplus = p.delta_softplus;
+    u.state_is_fp32 = p.state_is_fp32;
+    u.state_batch_stride = d * p.d_state; u.state_head_stride = u.state_batch_stride;
+    u.state_dim_stride = p.d_state; u.state_dstate_stride = 1;
+    u.x_batch_stride = u.x_head_stride = d; u.x_dim_stride = 1;
+    u.dt_batch_stride = u.dt_head_stride = d; u.dt_dim_stride = 1;
+    u.dt_bias_head_stride = d; u.dt_bias_dim_stride = 1;
+    u.A_head_stride = u.state_batch_stride; u.A_dim_stride = p.d_state; u.A_dstate_stride = 1;
+    u.B_batch_stride = u.B_group_stride = p.x_proj.n; u.B_dstate_stride = 1;
+    u.C_batch_stride = u.C_group_stride = p.x_proj.n; u.C_dstate_stride = 1;
+    u.D_head_stride = d; u.D_dim_stride = 1;
+    u.z_batch_stride = u.z_head_stride = 2 * d; u.z_dim_stride = 1;
+    u.out_batch_stride = u.out_head_stride = d; u.out_dim_stride = 1;
+    u.state = p.ssm_state; u.x = b.x; u.dt = b.dt; u.dt_bias = p.dt_bias; u.A_log = p.A_log;
+    u.B = b.x_dbl + p.dt_rank; u.C = u.B + p.d_state; u.D = p.D; u.z = b.xz + d;
+    u.x_scale = p.u_scale; u.dt_scale = p.dt_scale; u.dt_bias_scale = p.dt_bias_scale; u.A_log_scale = p.A_scale;
+    u.state_scale = p.ssm_state_scale; u.B_scale = p.B_scale; u.C_scale = p.C_scale; u.D_scale = p.D_scale; u.z_scale = p.z_scale;
+    u.out = b.y;
+    return u;
+}
+
+// b: the workspace's sections
+int ready(const QaMamba1Params* p, bool step, Mamba1Buffers& b) {
     QA_TRY(validate(p));
     if (!p->hidden || !p->out || !p->workspace || !p->conv_weight || !p->A_log) return QA_ERR_NULL;
-    if (states && (!p->conv_state || !p->ssm_state)) return QA_ERR_NULL;
-    if (p->workspace_bytes < carve(*p, nullptr).total || (reinterpret_cast<uintptr_t>(p->workspace) & 255u)) return QA_ERR_STRIDE;
-    return QA_OK;
+    if (step && (!p->conv_state || !p->ssm_state)) return QA_ERR_NULL;
+    if (step && p->seqlen != 1) return QA_ERR_SHAPE;
+    b = carve(*p, p->workspace);
+    if (p->workspace_bytes < b.total || (reinterpret_cast<uintptr_t>(p->workspace) & 255u) || !aligned16(p->hidden)) return QA_ERR_STRIDE;
+    if (step) return ssm_update_check(update_of(*p, b));
+    const SscanDtProj dt = scan_dt_of(*p, b);
+    return sscan_token_major_check(scan_of(*p, b), dt_in_scan(*p) ? &dt : nullptr);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -243,27 +326,22 @@ Mamba2Buffers carve(const QaMamba2Params& p, void* base, bool step) {
     return b;
 }
 
-int validate(const QaMamba2Params* p) {
+int validate(const QaMamba2Params* p, bool step) {
     if (!p) return QA_ERR_NULL;
-    if (p->batch < 1 || p->seqlen < 1 || p->batch > 65535 || static_cast<int64_t>(p->batch) * p->seqlen > 0x7fffffff) return QA_ERR_SHAPE;
-    if (p->headdim < 1 || p->d_inner % p->headdim != 0 || p->ngroups < 1 || heads_of(*p) % p->ngroups != 0) return QA_ERR_SHAPE;
-    if (p->d_conv < 2 || p->d_conv > 4 || p->d_inner % 16 != 0 || (p->ngroups * p->d_state) % 4 != 0) return QA_ERR_UNSUPPORTED;
-    for (const QaLinearParams* w : {&p->in_proj, &p->out_proj})
-        if (!linear_ok(*w)) return QA_ERR_NULL;
+    if (p->batch < 1 || p->seqlen < 1 || p->batch > 65535 || p->seqlen > kConvSteps || static_cast<int64_t>(p->batch) * p->seqlen > 0x7fffffff) return QA_ERR_SHAPE;
+    if (p->d_inner < 16 || p->headdim < 1 || p->d_inner % p->headdim != 0 || p->ngroups < 1 || heads_of(*p) % p->ngroups != 0) return QA_ERR_SHAPE;
+    if (p->d_conv < 2 || p->d_conv > 4 || p->d_inner % 16 != 0 || p->d_state < 1 || (p->ngroups * p->d_state) % 4 != 0) return QA_ERR_UNSUPPORTED;
+    // the limits of the scan (qa_ssd_chunk_scan_fwd) and of the state update
+    if (step ? p->d_state > 256 || heads_of(*p) > 65535 : p->headdim > 256 || p->d_state > 1024 || p->chunk_size < 1 || p->chunk_size > 1024) return QA_ERR_UNSUPPORTED;
     const int64_t used = 2LL * p->d_inner + 2LL * p->ngroups * p->d_state + heads_of(*p);
-    if (p->in_proj.k != p->d_model || p->in_proj.n < used || p->in_proj.n % 4 != 0 || p->out_proj.k != p->d_inner) return QA_ERR_SHAPE;
+    if (p->in_proj.k != p->d_model || p->in_proj.n < used || p->in_proj.n % 8 != 0 || p->out_proj.k != p->d_inner) return QA_ERR_SHAPE;
     if (p->conv_state_len != p->d_conv && p->conv_state_len != p->d_conv - 1) return QA_ERR_SHAPE;
     if (p->norm_group_size < 1 || p->d_inner % p->norm_group_size != 0) return QA_ERR_SHAPE;
-    return QA_OK;
-}
-
-int ready(const QaMamba2Params* p, bool step) {
-    QA_TRY(validate(p));
-    if (!p->hidden || !p->out || !p->workspace || !p->conv_weight || !p->A_log || !p->norm_weight) return QA_ERR_NULL;
-    if (!p->x_out_scales || !p->B_out_scales || !p->C_out_scales) return QA_ERR_NULL;
-    if (step && (!p->conv_state || !p->ssm_state)) return QA_ERR_NULL;
-    if (p->workspace_bytes < carve(*p, nullptr, step).total || (reinterpret_cast<uintptr_t>(p->workspace) & 255u)) return QA_ERR_STRIDE;
-    return QA_OK;
+    if (p->norm_group_size % 8 != 0 || p->norm_group_size > kNormGroup) return QA_ERR_UNSUPPORTED;
+    const int64_t t = static_cast<int64_t>(p->batch) * p->seqlen;
+    QA_TRY(linear_check(p->in_proj, t, p->d_model));
+    QA_TRY(linear_check(p->out_proj, t, p->d_inner));
+    return hadamard_check(p->d_inner);
 }
 
 QaConv2Params conv2_of(const QaMamba2Params& p, const Mamba2Buffers& b) {
@@ -288,6 +366,65 @@ QaConv2Params conv2_of(const QaMamba2Params& p, const Mamba2Buffers& b) {
     c.scale_wx = p.scale_wx; c.scale_wB = p.scale_wB; c.scale_wC = p.scale_wC;
     c.scale_bx = p.scale_bx; c.scale_bB = p.scale_bB; c.scale_bC = p.scale_bC;
     return c;
+}
+
+QaSsdParams ssd_of(const QaMamba2Params& p, const Mamba2Buffers& b) {
+    QaSsdParams s = ssd_sizes(p);
+    s.dt_softplus = p.delta_softplus;
+    s.D_has_hdim = p.D_has_hdim;
+    s.nhead_groups = p.nhead_groups; s.ndim_groups = p.ndim_groups;
+    s.final_state_is_fp32 = p.state_is_fp32;
+    s.dt_row_stride = p.in_proj.n;
+    s.dt_min = p.dt_min; s.dt_max = p.dt_max;
+    s.x = b.x; s.B = b.B; s.C = b.C;
+    s.dt = b.zxbcdt + 2 * p.d_inner + 2 * p.ngroups * p.d_state;
+    s.A_log = p.A_log; s.D = p.D; s.dt_bias = p.dt_bias;
+    s.x_scale = p.x_scales; s.dt_scale = p.dt_scale; s.A_log_scale = p.A_log_scale; s.B_scale = p.B_scale; s.C_scale = p.C_scale;
+    s.D_scale = p.D_scale; s.state_scale = p.ssm_state_scale;
+    s.x_head_group_range = p.head_range; s.x_dim_group_range = p.dim_range;
+    s.out = b.y; s.final_states = p.ssm_state;
+    s.workspace = b.ssd.p; s.workspace_bytes = b.ssd.bytes;
+    return s;
+}
+
+QaSsmUpdateParams update_of(const QaMamba2Params& p, const Mamba2Buffers& b) {
+    QaSsmUpdateParams u = {};
+    const int heads = heads_of(p);
+    const int64_t bc = static_cast<int64_t>(p.ngroups) * p.d_state;
+    u.batch = p.batch; u.nheads = heads; u.dim = p.headdim; u.dstate = p.d_state; u.ngroups = p.ngroups;
+    u.dt_softplus = p.delta_softplus;
+    u.state_is_fp32 = p.state_is_fp32;
+    u.dt_bias_is_fp16 = 1;
+    u.nhead_groups = p.nhead_groups; u.ndim_groups = p.ndim_groups;
+    u.state_dstate_stride = 1; u.state_dim_stride = p.d_state;
+    u.state_head_stride = static_cast<int64_t>(p.headdim) * p.d_state; u.state_batch_stride = u.state_head_stride * heads;
+    u.x_batch_stride = p.d_inner; u.x_head_stride = p.headdim; u.x_dim_stride = 1;
+    u.dt_batch_stride = p.in_proj.n; u.dt_head_stride = 1;
+    u.dt_bias_head_stride = 1;
+    u.A_head_stride = 1;
+    u.B_batch_stride = u.C_batch_stride = bc; u.B_group_stride = u.C_group_stride = p.d_state; u.B_dstate_stride = u.C_dstate_stride = 1;
+    u.D_head_stride = p.D_has_hdim ? p.headdim : 1; u.D_dim_stride = p.D_has_hdim ? 1 : 0;
+    u.out_batch_stride = p.d_inner; u.out_head_stride = p.headdim; u.out_dim_stride = 1;
+    u.state = p.ssm_state; u.x = b.x; u.dt = b.zxbcdt + 2 * p.d_inner + 2 * bc; u.dt_bias = p.dt_bias; u.A_log = p.A_log;
+    u.B = b.B; u.C = b.C; u.D = p.D;
+    u.x_scale = p.x_scales; u.dt_scale = p.dt_scale; u.A_log_scale = p.A_log_scale; u.state_scale = p.ssm_state_scale;
+    u.B_scale = p.B_scale; u.C_scale = p.C_scale; u.D_scale = p.D_scale;
+    u.x_head_group_range = p.head_range; u.x_dim_group_range = p.dim_range;
+    u.out = b.y;
+    return u;
+}
+
+int ready(const QaMamba2Params* p, bool step, Mamba2Buffers& b) {
+    QA_TRY(validate(p, step));
+    if (!p->hidden || !p->out || !p->workspace || !p->conv_weight || !p->A_log || !p->norm_weight) return QA_ERR_NULL;
+    if (!p->x_out_scales || !p->B_out_scales || !p->C_out_scales) return QA_ERR_NULL;
+    if ((p->conv_head_range == nullptr) != (p->conv_dim_range == nullptr)) return QA_ERR_NULL;
+    if (p->conv_head_range && (p->conv_nhead_groups < 1 || p->conv_ndim_groups < 1)) return QA_ERR_SHAPE;
+    if (step && (!p->conv_state || !p->ssm_state)) return QA_ERR_NULL;
+    if (step && p->seqlen != 1) return QA_ERR_SHAPE;
+    b = carve(*p, p->workspace, step);
+    if (p->workspace_bytes < b.total || (reinterpret_cast<uintptr_t>(p->workspace) & 255u) || !aligned16(p->hidden) || !aligned16(p->norm_weight)) return QA_ERR_STRIDE;
+    return step ? ssm_update_check(update_of(*p, b)) : ssd_check(ssd_of(*p, b));
 }
 
 // gated norm, Hadamard rotation and quantisation, out_proj
@@ -320,42 +457,18 @@ extern "C" int64_t qa_mamba1_workspace_bytes(const QaMamba1Params* p, int) {
 
 extern "C" int qa_mamba1_forward(const QaMamba1Params* p, void* stream) {
     using namespace qa;
-    QA_TRY(ready(p, false));
-    const Mamba1Buffers b = carve(*p, p->workspace);
+    Mamba1Buffers b;
+    QA_TRY(ready(p, false, b));
     const int rows = p->batch * p->seqlen, d = p->d_inner;
-    const int64_t len = p->seqlen;
     QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.xz, QA_OUT_I8, true, b.w8, stream));
 
     QA_TRY(conv_channel_last_fwd(conv_of(*p, b), static_cast<hipStream_t>(stream)));
 
     QA_TRY(project(p->x_proj, b.x, d, rows, b.x_dbl, QA_OUT_I8, false, b.w8, stream));
-    const QaLinearParams& dtp = p->dt_proj;
-    const bool fused_dt = dtp.bits == 8 && dtp.k % 16 == 0 && dtp.k <= kSscanDtRank && p->x_proj.n % 16 == 0 &&
-                          len * static_cast<int64_t>(p->x_proj.n) < 1 << 30;
-    if (!fused_dt) QA_TRY(project(dtp, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, true, b.w8, stream));
-
-    QaSScanParams s = scan_sizes(*p);
-    const int64_t dbl = p->x_proj.n;
-    s.delta_softplus = p->delta_softplus;
-    s.token_major = 1;
-    s.u_batch_stride = len * d; s.u_l_stride = d; s.u_d_stride = 1;
-    s.delta_batch_stride = len * d; s.delta_l_stride = d; s.delta_d_stride = 1;
-    s.z_batch_stride = len * 2 * d; s.z_l_stride = 2 * d; s.z_d_stride = 1;
-    s.B_batch_stride = s.C_batch_stride = len * dbl;
-    s.B_l_stride = s.C_l_stride = dbl;
-    s.B_dstate_stride = s.C_dstate_stride = 1;
-    s.A_d_stride = p->d_state; s.A_dstate_stride = 1;
-    s.out_batch_stride = len * d; s.out_l_stride = d; s.out_d_stride = 1;
-    s.u = b.x; s.delta = b.dt; s.A_log = p->A_log; s.B = b.x_dbl + p->dt_rank; s.C = s.B + p->d_state;
-    s.D = p->D; s.delta_bias = p->dt_bias; s.z = b.xz + d;
-    s.scale_u = p->u_scale; s.scale_delta = p->dt_scale; s.scale_A = p->A_scale; s.scale_B = p->B_scale; s.scale_C = p->C_scale;
-    s.scale_D = p->D_scale; s.scale_delta_bias = p->dt_bias_scale; s.scale_z = p->z_scale; s.scale_ssm_state = p->ssm_state_scale;
-    s.out = b.y;
-    if (p->state_is_fp32) s.last_state_f32 = static_cast<float*>(p->ssm_state);
-    else s.last_state_i8 = static_cast<int8_t*>(p->ssm_state);
-    s.workspace = b.scan.p; s.workspace_bytes = b.scan.bytes;
-    const SscanDtProj proj = {static_cast<const int8_t*>(dtp.weight), b.x_dbl, len * dbl, dbl, dtp.row_scale, dtp.col_scale, dtp.k, dtp.col_numel};
-    QA_TRY(sscan_token_major_fwd(s, fused_dt ? &proj : nullptr, static_cast<hipStream_t>(stream)));
+    const bool fused_dt = dt_in_scan(*p);
+    if (!fused_dt) QA_TRY(project(p->dt_proj, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, true, b.w8, stream));
+    const SscanDtProj dt = scan_dt_of(*p, b);
+    QA_TRY(sscan_token_major_fwd(scan_of(*p, b), fused_dt ? &dt : nullptr, static_cast<hipStream_t>(stream)));
 
     QA_TRY(hadamard(b.y, b.yq, rows, d, p->had_scale, stream));
     return project(p->out_proj, b.yq, d, rows, p->out, QA_OUT_F16, false, b.w8, stream);
@@ -363,9 +476,8 @@ extern "C" int qa_mamba1_forward(const QaMamba1Params* p, void* stream) {
 
 extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
     using namespace qa;
-    QA_TRY(ready(p, true));
-    if (p->seqlen != 1) return QA_ERR_SHAPE;
-    const Mamba1Buffers b = carve(*p, p->workspace);
+    Mamba1Buffers b;
+    QA_TRY(ready(p, true, b));
     const int rows = p->batch, d = p->d_inner;
     const int fused = project_conv(p->in_proj, p->hidden, p->d_model, rows, b.xz, 0, conv_of(*p, b), stream);
     if (fused == QA_ERR_UNSUPPORTED) {
@@ -377,30 +489,11 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
 
     QA_TRY(project(p->x_proj, b.x, d, rows, b.x_dbl, QA_OUT_I8, false, b.w8, stream));
 
-    QaSsmUpdateParams u = {};
-    u.batch = rows; u.nheads = 1; u.dim = d; u.dstate = p->d_state; u.ngroups = 1;
-    u.dt_softplus = p->delta_softplus;
-    u.state_is_fp32 = p->state_is_fp32;
-    u.state_batch_stride = static_cast<int64_t>(d) * p->d_state; u.state_head_stride = u.state_batch_stride;
-    u.state_dim_stride = p->d_state; u.state_dstate_stride = 1;
-    u.x_batch_stride = u.x_head_stride = d; u.x_dim_stride = 1;
-    u.dt_batch_stride = u.dt_head_stride = d; u.dt_dim_stride = 1;
-    u.dt_bias_head_stride = d; u.dt_bias_dim_stride = 1;
-    u.A_head_stride = u.state_batch_stride; u.A_dim_stride = p->d_state; u.A_dstate_stride = 1;
-    u.B_batch_stride = u.B_group_stride = p->x_proj.n; u.B_dstate_stride = 1;
-    u.C_batch_stride = u.C_group_stride = p->x_proj.n; u.C_dstate_stride = 1;
-    u.D_head_stride = d; u.D_dim_stride = 1;
-    u.z_batch_stride = u.z_head_stride = 2 * d; u.z_dim_stride = 1;
-    u.out_batch_stride = u.out_head_stride = d; u.out_dim_stride = 1;
-    u.state = p->ssm_state; u.x = b.x; u.dt = b.dt; u.dt_bias = p->dt_bias; u.A_log = p->A_log;
-    u.B = b.x_dbl + p->dt_rank; u.C = u.B + p->d_state; u.D = p->D; u.z = b.xz + d;
-    u.x_scale = p->u_scale; u.dt_scale = p->dt_scale; u.dt_bias_scale = p->dt_bias_scale; u.A_log_scale = p->A_scale;
-    u.state_scale = p->ssm_state_scale; u.B_scale = p->B_scale; u.C_scale = p->C_scale; u.D_scale = p->D_scale; u.z_scale = p->z_scale;
-    u.out = b.y;
+    const QaSsmUpdateParams u = update_of(*p, b);
     const QaLinearParams& dt = p->dt_proj;
     int st = QA_ERR_UNSUPPORTED;
     // (every batch entry reads the weights again, a row per lane: past a few entries a product of its own is the faster one)
-    if (rows <= kFusedDtRows && dt.bits == 8 && dt.k % 16 == 0) {
+    if (rows <= kFusedDtRows && dt.bits == 8) {
         const SsmDtProj proj = {static_cast<const int8_t*>(dt.weight), b.x_dbl, p->x_proj.n, dt.row_scale, dt.col_scale, dt.k / 16, dt.col_numel,
                                 rows == 1 && dt.row_rule == QA_ROW_ALPHA, dt.alpha};
         st = ssm_update_with_dt(u, proj, static_cast<hipStream_t>(stream));
@@ -422,42 +515,26 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
 
 extern "C" int64_t qa_mamba2_workspace_bytes(const QaMamba2Params* p, int step) {
     using namespace qa;
-    return validate(p) == QA_OK ? carve(*p, nullptr, step != 0).total : 0;
+    return validate(p, step != 0) == QA_OK ? carve(*p, nullptr, step != 0).total : 0;
 }
 
 extern "C" int qa_mamba2_forward(const QaMamba2Params* p, void* stream) {
     using namespace qa;
-    QA_TRY(ready(p, false));
-    const Mamba2Buffers b = carve(*p, p->workspace, false);
+    Mamba2Buffers b;
+    QA_TRY(ready(p, false, b));
     const int rows = p->batch * p->seqlen;
     QA_TRY(project(p->in_proj, p->hidden, p->d_model, rows, b.zxbcdt, QA_OUT_I8, false, b.w8, stream));
     QA_TRY(conv_channel_last_fwd(conv2_of(*p, b), static_cast<hipStream_t>(stream)));
-
-    QaSsdParams s = ssd_sizes(*p);
-    s.dt_softplus = p->delta_softplus;
-    s.D_has_hdim = p->D_has_hdim;
-    s.nhead_groups = p->nhead_groups; s.ndim_groups = p->ndim_groups;
-    s.final_state_is_fp32 = p->state_is_fp32;
-    s.dt_row_stride = p->in_proj.n;
-    s.dt_min = p->dt_min; s.dt_max = p->dt_max;
-    s.x = b.x; s.B = b.B; s.C = b.C;
-    s.dt = b.zxbcdt + 2 * p->d_inner + 2 * p->ngroups * p->d_state;
-    s.A_log = p->A_log; s.D = p->D; s.dt_bias = p->dt_bias;
-    s.x_scale = p->x_scales; s.dt_scale = p->dt_scale; s.A_log_scale = p->A_log_scale; s.B_scale = p->B_scale; s.C_scale = p->C_scale;
-    s.D_scale = p->D_scale; s.state_scale = p->ssm_state_scale;
-    s.x_head_group_range = p->head_range; s.x_dim_group_range = p->dim_range;
-    s.out = b.y; s.final_states = p->ssm_state;
-    s.workspace = b.ssd.p; s.workspace_bytes = b.ssd.bytes;
+    const QaSsdParams s = ssd_of(*p, b);
     QA_TRY(qa_ssd_chunk_scan_fwd(&s, stream));
     return mamba2_tail(*p, b, stream);
 }
 
 extern "C" int qa_mamba2_step(const QaMamba2Params* p, void* stream) {
     using namespace qa;
-    QA_TRY(ready(p, true));
-    if (p->seqlen != 1) return QA_ERR_SHAPE;
-    const Mamba2Buffers b = carve(*p, p->workspace, true);
-    const int rows = p->batch, heads = heads_of(*p);
+    Mamba2Buffers b;
+    QA_TRY(ready(p, true, b));
+    const int rows = p->batch;
     const QaConv2Params c = conv2_of(*p, b);
     const int fused = project_conv(p->in_proj, p->hidden, p->d_model, rows, b.zxbcdt, p->d_inner, c, stream);
     if (fused == QA_ERR_UNSUPPORTED) {
@@ -466,29 +543,7 @@ extern "C" int qa_mamba2_step(const QaMamba2Params* p, void* stream) {
     } else if (fused != QA_OK) {
         return fused;
     }
-
-    QaSsmUpdateParams u = {};
-    const int64_t bc = static_cast<int64_t>(p->ngroups) * p->d_state;
-    u.batch = rows; u.nheads = heads; u.dim = p->headdim; u.dstate = p->d_state; u.ngroups = p->ngroups;
-    u.dt_softplus = p->delta_softplus;
-    u.state_is_fp32 = p->state_is_fp32;
-    u.dt_bias_is_fp16 = 1;
-    u.nhead_groups = p->nhead_groups; u.ndim_groups = p->ndim_groups;
-    u.state_dstate_stride = 1; u.state_dim_stride = p->d_state;
-    u.state_head_stride = static_cast<int64_t>(p->headdim) * p->d_state; u.state_batch_stride = u.state_head_stride * heads;
-    u.x_batch_stride = p->d_inner; u.x_head_stride = p->headdim; u.x_dim_stride = 1;
-    u.dt_batch_stride = p->in_proj.n; u.dt_head_stride = 1;
-    u.dt_bias_head_stride = 1;
-    u.A_head_stride = 1;
-    u.B_batch_stride = u.C_batch_stride = bc; u.B_group_stride = u.C_group_stride = p->d_state; u.B_dstate_stride = u.C_dstate_stride = 1;
-    u.D_head_stride = p->D_has_hdim ? p->headdim : 1; u.D_dim_stride = p->D_has_hdim ? 1 : 0;
-    u.out_batch_stride = p->d_inner; u.out_head_stride = p->headdim; u.out_dim_stride = 1;
-    u.state = p->ssm_state; u.x = b.x; u.dt = b.zxbcdt + 2 * p->d_inner + 2 * bc; u.dt_bias = p->dt_bias; u.A_log = p->A_log;
-    u.B = b.B; u.C = b.C; u.D = p->D;
-    u.x_scale = p->x_scales; u.dt_scale = p->dt_scale; u.A_log_scale = p->A_log_scale; u.state_scale = p->ssm_state_scale;
-    u.B_scale = p->B_scale; u.C_scale = p->C_scale; u.D_scale = p->D_scale;
-    u.x_head_group_range = p->head_range; u.x_dim_group_range = p->dim_range;
-    u.out = b.y;
+    const QaSsmUpdateParams u = update_of(*p, b);
     QA_TRY(qa_ssm_state_update(&u, stream));
     return mamba2_tail(*p, b, stream);
 }

@@ -18,6 +18,7 @@ struct SscanDtProj {
     int rank, col_numel;
 };
 constexpr int kSscanDtRank = 192;
+int sscan_token_major_check(const QaSScanParams& p, const SscanDtProj* dt);       // what it refuses, without a launch
 int sscan_token_major_fwd(const QaSScanParams& p, const SscanDtProj* dt, hipStream_t stream);
 // bytes of scratch it can use for these sizes (0: none)
 int64_t sscan_token_major_workspace(const QaSScanParams& p);
@@ -35,6 +36,14 @@ struct SsmDtProj {
 };
 constexpr int kSsmDtPieces = 10;       // up to 160 inputs
 int ssm_update_with_dt(const QaSsmUpdateParams& p, const SsmDtProj& dt, hipStream_t stream);
+// what qa_ssm_state_update refuses, without a launch
+int ssm_update_check(const QaSsmUpdateParams& p);
+
+// ssd.hip: what qa_ssd_chunk_scan_fwd refuses about sizes and tensors, without a launch
+int ssd_check(const QaSsdParams& p);
+
+// normgated.hip: columns of the widest group
+constexpr int kNormGroup = 32768;
 
 // conv2.hip: the channel-contiguous forward conv.  Without x_out_scales every channel is an x channel with the one
 // output scale `x_out_scale` (the Mamba1 conv); with conv_state the last inputs of every channel are left there.

@@ -14,13 +14,14 @@
 // (W waves per group), so every load and store of a wave is one contiguous run.
 // The gate has 256 possible values (one per int8 code): a workgroup evaluates them once into LDS and
 // every element looks its gate up, which gives the same bits as evaluating it per element.
+#include "mixer_common.hpp"
 #include "normgated_core.hpp"
 
 namespace qa {
 namespace {
 
 constexpr int kWavesPerBlock = 4;
-constexpr int kMaxPieces = 16;      // per lane: 16 pieces * 4 waves * 64 lanes * 8 columns = 32768 columns per group
+static_assert(kNormGroup == 16 * kWavesPerBlock * 512, "a lane holds up to 16 pieces of 8 columns");
 
 template <int PIECES, int WPI, bool GATE_LAST>
 __global__ __launch_bounds__(64 * kWavesPerBlock) void rmsnorm_gated_kernel(QaNormGatedParams p) {
@@ -144,7 +145,7 @@ extern "C" int qa_rmsnorm_gated(const QaNormGatedParams* p, void* stream_) {
     if (p->rows > 0 && p->out_mode == QA_NORM_OUT_I8_DYNAMIC && !p->dyn_scale) return QA_ERR_NULL;
     if (p->out_mode < 0 || p->out_mode > 2) return QA_ERR_UNSUPPORTED;
     if (p->rows < 0 || p->dim < 1 || p->group_size < 1 || p->dim % p->group_size != 0) return QA_ERR_SHAPE;
-    if (p->group_size % 8 != 0 || p->group_size > kMaxPieces * kWavesPerBlock * 512) return QA_ERR_UNSUPPORTED;
+    if (p->group_size % 8 != 0 || p->group_size > kNormGroup) return QA_ERR_UNSUPPORTED;
     if (p->x_row_stride % 8 != 0 || p->out_row_stride % 8 != 0 || (p->qz && p->z_row_stride % 8 != 0)) return QA_ERR_STRIDE;
     if (!aligned16(p->x) || !aligned16(p->weight) || !aligned16(p->out) ||
         (p->qz && (reinterpret_cast<uintptr_t>(p->qz) & 7u))) return QA_ERR_STRIDE;

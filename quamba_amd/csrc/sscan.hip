@@ -1298,10 +1298,14 @@ bool launch_heads_i8(const QaSsmUpdateParams& p, hipStream_t stream) {
     return true;
 }
 
+bool update_fits_grid(const QaSsmUpdateParams& p, int lanes_per_row = 16) {
+    return (static_cast<int64_t>(p.dim) * lanes_per_row + 255) / 256 <= 0x7fffffffLL / 256 && p.nheads <= 65535 && p.batch <= 65535;
+}
+
 template <int LPR>
 int launch_update(const QaSsmUpdateParams& p, hipStream_t stream, const QaConvParams* conv = nullptr, const SsmDtProj* dt = nullptr) {
     const int64_t blocks = (static_cast<int64_t>(p.dim) * LPR + 255) / 256;
-    if (blocks > 0x7fffffffLL / 256 || p.nheads > 65535 || p.batch > 65535) return QA_ERR_SHAPE;
+    if (!update_fits_grid(p, LPR)) return QA_ERR_SHAPE;
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(p.nheads), static_cast<unsigned>(p.batch));
     const int64_t st_align = p.state_is_fp32 ? 16 : 4;      // bytes of one lane's four states
     const int64_t st_el = p.state_is_fp32 ? 4 : 1;
@@ -1478,6 +1482,11 @@ int validate_update(const QaSsmUpdateParams* p, bool needs_x) {
 }
 }  // namespace
 }  // namespace qa
+
+int qa::ssm_update_check(const QaSsmUpdateParams& p) {
+    const int st = validate_update(&p, true);
+    return st != QA_OK ? st : update_fits_grid(p) ? QA_OK : QA_ERR_SHAPE;
+}
 
 int qa::ssm_update_with_dt(const QaSsmUpdateParams& p, const SsmDtProj& dt, hipStream_t stream) { return launch_update<1>(p, stream, nullptr, &dt); }
 

@@ -560,7 +560,7 @@ int launch(const QaSScanParams& p_in, const SscanDtProj& dtp, hipStream_t stream
 
 }  // namespace
 
-int sscan_token_major_fwd(const QaSScanParams& p, const SscanDtProj* dt, hipStream_t stream) {
+int sscan_token_major_check(const QaSScanParams& p, const SscanDtProj* dt) {
     const auto mult4 = [](int64_t v) { return v % 4 == 0; };
     if (p.dstate != 16 || p.n_groups != 1 || p.dim < 4 || !mult4(p.dim) || p.carry_state || p.dt_sum_out || p.segments < 0) return QA_ERR_UNSUPPORTED;
     if (p.mapping != 0 && ((p.mapping & ~0x0fffffff) != 0x40000000 || (((p.mapping >> 20) & 0xff) == 0 && 64LL * (p.mapping & 0xfffff) > p.dim))) return QA_ERR_UNSUPPORTED;
@@ -571,11 +571,22 @@ int sscan_token_major_fwd(const QaSScanParams& p, const SscanDtProj* dt, hipStre
         if (!mult4(v) || v < 0) return QA_ERR_STRIDE;
     for (const int64_t v : {p.u_l_stride, dt ? dt->x_l_stride : p.delta_l_stride, p.z ? p.z_l_stride : 0, p.B_l_stride, p.C_l_stride})
         if (v >= 1 << 24) return QA_ERR_STRIDE;                        // a tile is addressed with 32-bit offsets
-    const SscanDtProj none = {};
-    if (!dt) return p.z ? launch<true, 0>(p, none, stream) : launch<false, 0>(p, none, stream);
+    if (!p.u || (!dt && !p.delta) || !p.A_log || !p.B || !p.C || !p.out) return QA_ERR_NULL;
+    if (!p.scale_u || !p.scale_delta || !p.scale_A || !p.scale_B || !p.scale_C) return QA_ERR_NULL;
+    if ((p.D && !p.scale_D) || (p.delta_bias && !p.scale_delta_bias) || (p.z && !p.scale_z) || (p.last_state_i8 && !p.scale_ssm_state)) return QA_ERR_NULL;
+    if (!dt) return QA_OK;
+    if (!dt->w || !dt->x || !dt->row_scale || !dt->col_scale) return QA_ERR_NULL;
     if (!p.z || dt->rank < 16 || dt->rank % 16 != 0 || dt->rank > kSscanDtRank) return QA_ERR_UNSUPPORTED;
     if (static_cast<int64_t>(p.seqlen) * dt->x_l_stride >= 1 << 30) return QA_ERR_UNSUPPORTED;       // 32-bit buffer offsets
     if (!aligned16(dt->w) || !aligned16(dt->x) || dt->x_l_stride % 16 != 0 || dt->x_batch_stride % 16 != 0) return QA_ERR_STRIDE;
+    return QA_OK;
+}
+
+int sscan_token_major_fwd(const QaSScanParams& p, const SscanDtProj* dt, hipStream_t stream) {
+    const int st = sscan_token_major_check(p, dt);
+    if (st != QA_OK) return st;
+    const SscanDtProj none = {};
+    if (!dt) return p.z ? launch<true, 0>(p, none, stream) : launch<false, 0>(p, none, stream);
     if (dt->rank <= 64) return launch<true, 1>(p, *dt, stream);
     if (dt->rank <= 128) return launch<true, 2>(p, *dt, stream);
     return launch<true, 3>(p, *dt, stream);

@@ -16,7 +16,7 @@
 #include <atomic>
 #include <mutex>
 
-#include "qa_common.hpp"
+#include "mixer_common.hpp"
 #include "ssd_common.hpp"
 
 namespace qa {
@@ -824,6 +824,8 @@ int validate(const QaSsdParams* p) {
 }
 
 }  // namespace
+
+int ssd_check(const QaSsdParams& p) { return validate(&p); }
 }  // namespace qa
 
 extern "C" int64_t qa_ssd_workspace_bytes(const QaSsdParams* p) {

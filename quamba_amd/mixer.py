@@ -113,6 +113,8 @@ class W8A8QMamba(nn.Module):
         p.D, p.dt_bias = _ptr(s.D, torch.int8, D, dev), _ptr(s.dt_bias, torch.int8, D, dev)
         for name in ("A_scale", "D_scale", "dt_bias_scale", "u_scale", "dt_scale", "B_scale", "C_scale", "z_scale", "ssm_state_scale"):
             setattr(p, name, _ptr(getattr(s, name), torch.float32, 1, dev))
+        _need(all((p.conv_weight, p.A_log, p.A_scale, p.u_scale, p.dt_scale, p.B_scale, p.C_scale, p.z_scale, p.ssm_state_scale)))
+        _need((p.D_scale or not p.D) and (p.dt_bias_scale or not p.dt_bias))
         _need(self.had.transform_fn is ops.hadamard_quant)
         p.had_scale = self.had.had_scale / float(self.had.x_H_scale)
         widths = (self.d_conv, self.d_conv - 1)                        # of the conv state, in forward and in step
@@ -294,7 +296,7 @@ class W4A8QMamba2(nn.Module):
         p.dt_min, p.dt_max = float(s.dt_limit[0]), float(min(s.dt_limit[1], 3.0e38))
         p.norm_eps, p.norm_z_scale, p.norm_before_gate = n.eps, float(n.z_scale), int(bool(n.norm_before_gate))
         p.norm_group_size = D if n.group_size is None else n.group_size
-        p.norm_weight = _ptr(n.weight, torch.float16, D, dev)
+        p.norm_weight = _ptr(n.weight, torch.float16, D, dev, 16)
         _need(self.had.transform_fn is ops.hadamard_quant)
         p.had_scale = self.had.had_scale / float(self.had.x_H_scale)
         p.A_log = _ptr(s.A_log, torch.int8, H, dev)
@@ -305,6 +307,8 @@ class W4A8QMamba2(nn.Module):
         p.x_scales = _ptr(s.x_scales, torch.float32, G * sg if sg else 1, dev)
         p.B_scale, p.C_scale = (_ptr(t, torch.float32, G if sg else 1, dev) for t in (s.B_scale, s.C_scale))
         p.ssm_state_scale = _ptr(s.ssm_state_scale, torch.float32, G * sg * N if sg else 1, dev)
+        _need(all((p.conv_weight, p.x_out_scales, p.B_out_scales, p.C_out_scales, p.A_log, p.A_log_scale, p.dt_scale, p.x_scales, p.B_scale,
+                   p.C_scale, p.ssm_state_scale, p.norm_weight)) and (p.D_scale or not p.D))
         return p, (conv_dim, (H, self.headdim, N), ((self.d_conv, self.d_conv), (self.d_conv, self.d_conv - 1)))
 
     def forward(self, u, conv_state=None, ssm_state=None):
