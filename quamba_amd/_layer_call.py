@@ -8,6 +8,7 @@ sub-module classes or replaced methods, forward hooks, views with gaps, unusual 
 modules one by one.
 """
 import ctypes as C
+import numbers
 
 import torch
 import torch.nn.modules.module as _module
@@ -54,6 +55,13 @@ def _ptr(t, dtype, numel, device, align=1):
     return a
 
 
+def _number(v):
+    """A value that goes into the block as a number: one that only changes by becoming another object.  (A tensor or an array
+    of one element can change in place, which the plan would not see: the modules read it on every call.)"""
+    _need(isinstance(v, numbers.Real))
+    return v
+
+
 def linear_block(lin, device):
     """QaLinearParams of one of the linear modules."""
     p = _lib.QaLinearParams()
@@ -73,7 +81,7 @@ def linear_block(lin, device):
         p.col_scale = _ptr(lin.b, torch.float32, lin.b.numel(), device)
         p.row_scale = _ptr(lin.a, torch.float32, 1, device)
         if hasattr(lin, "alpha"):
-            p.row_rule, p.alpha = _lib.QA_ROW_ALPHA, lin.alpha
+            p.row_rule, p.alpha = _lib.QA_ROW_ALPHA, _number(lin.alpha)
         else:
             p.row_rule = _lib.QA_ROW_HALF_AWAY
     return p

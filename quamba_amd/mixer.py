@@ -18,7 +18,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _layer_call, _lib, ops
-from ._layer_call import _need, _ptr, linear_block
+from ._layer_call import _need, _number, _ptr, linear_block
 from .chunk_scan import Quamba2ChunkScan
 from .conv import QCausalConv1D, Quamb2Conv1D
 from .hadamard import QHadamard
@@ -104,11 +104,12 @@ class W8A8QMamba(nn.Module):
         c, s = self.conv1d, self.selective_scan
         p.d_model, p.d_inner, p.d_state, p.d_conv, p.dt_rank = self.d_model, D, N, self.d_conv, self.dt_rank
         p.conv_state_len = self.d_conv
-        p.delta_softplus = int(bool(s.delta_softplus))
+        p.delta_softplus = int(bool(_number(s.delta_softplus)))
         for name in ("in_proj", "x_proj", "dt_proj", "out_proj"):
             setattr(p, name, linear_block(getattr(self, name), dev))
         p.conv_weight, p.conv_bias = _ptr(c.weight, torch.int8, D * self.d_conv, dev), _ptr(c.bias, torch.int8, D, dev)
-        p.conv_scale_x, p.conv_scale_w, p.conv_scale_b, p.conv_scale_out = c.input_scale, c.weight_scale, c.bias_scale, c.output_scale
+        p.conv_scale_x, p.conv_scale_w, p.conv_scale_b, p.conv_scale_out = (
+            _number(v) for v in (c.input_scale, c.weight_scale, c.bias_scale, c.output_scale))
         p.A_log = _ptr(s.A_log, torch.int8, D * N, dev)
         p.D, p.dt_bias = _ptr(s.D, torch.int8, D, dev), _ptr(s.dt_bias, torch.int8, D, dev)
         for name in ("A_scale", "D_scale", "dt_bias_scale", "u_scale", "dt_scale", "B_scale", "C_scale", "z_scale", "ssm_state_scale"):
@@ -116,7 +117,7 @@ class W8A8QMamba(nn.Module):
         _need(all((p.conv_weight, p.A_log, p.A_scale, p.u_scale, p.dt_scale, p.B_scale, p.C_scale, p.z_scale, p.ssm_state_scale)))
         _need((p.D_scale or not p.D) and (p.dt_bias_scale or not p.dt_bias))
         _need(self.had.transform_fn is ops.hadamard_quant)
-        p.had_scale = self.had.had_scale / float(self.had.x_H_scale)
+        p.had_scale = _number(self.had.had_scale) / float(_number(self.had.x_H_scale))
         widths = (self.d_conv, self.d_conv - 1)                        # of the conv state, in forward and in step
         return p, (D, (D, N), (widths, widths))
 
@@ -272,8 +273,8 @@ class W4A8QMamba2(nn.Module):
         # the kernels' state counts: others run padded, module by module
         _need(self.headdim % 64 != 0 or N in (64, 128) or N > 128 or s.chunk_size not in (64, 128, 256))
         p.d_model, p.d_inner, p.d_state, p.d_conv, p.headdim, p.ngroups = self.d_model, D, N, self.d_conv, self.headdim, G
-        p.chunk_size, p.conv_state_len = s.chunk_size, self.d_conv
-        p.delta_softplus, p.D_has_hdim = int(bool(s.delta_softplus)), int(bool(s.D_has_hdim))
+        p.chunk_size, p.conv_state_len = _number(s.chunk_size), self.d_conv
+        p.delta_softplus, p.D_has_hdim = int(bool(_number(s.delta_softplus))), int(bool(_number(s.D_has_hdim)))
         p.in_proj, p.out_proj = linear_block(self.in_proj, dev), linear_block(self.out_proj, dev)
         conv_dim = D + 2 * G * N
         p.conv_weight, p.conv_bias = _ptr(c.weight, torch.int8, conv_dim * self.d_conv, dev), _ptr(c.bias, torch.int8, conv_dim, dev)
@@ -290,15 +291,17 @@ class W4A8QMamba2(nn.Module):
         p.x_out_scales = _ptr(c.x_out_scales, torch.float32, G * cg if cg else 1, dev)
         p.B_out_scales, p.C_out_scales = (_ptr(t, torch.float32, G if cg else 1, dev) for t in (c.B_out_scales, c.C_out_scales))
         for name in ("x", "B", "C"):
-            setattr(p, "scale_" + name, getattr(c, name + "_scale"))
-            setattr(p, "scale_w" + name, getattr(c, "w" + name + "_scale"))
-            setattr(p, "scale_b" + name, getattr(c, "b" + name + "_scale") or 0.0)
-        p.dt_min, p.dt_max = float(s.dt_limit[0]), float(min(s.dt_limit[1], 3.0e38))
-        p.norm_eps, p.norm_z_scale, p.norm_before_gate = n.eps, float(n.z_scale), int(bool(n.norm_before_gate))
-        p.norm_group_size = D if n.group_size is None else n.group_size
+            setattr(p, "scale_" + name, _number(getattr(c, name + "_scale")))
+            setattr(p, "scale_w" + name, _number(getattr(c, "w" + name + "_scale")))
+            bias_scale = getattr(c, "b" + name + "_scale")
+            setattr(p, "scale_b" + name, 0.0 if bias_scale is None else _number(bias_scale))
+        _need(type(s.dt_limit) is tuple)
+        p.dt_min, p.dt_max = float(_number(s.dt_limit[0])), float(min(_number(s.dt_limit[1]), 3.0e38))
+        p.norm_eps, p.norm_z_scale, p.norm_before_gate = _number(n.eps), float(_number(n.z_scale)), int(bool(_number(n.norm_before_gate)))
+        p.norm_group_size = D if n.group_size is None else _number(n.group_size)
         p.norm_weight = _ptr(n.weight, torch.float16, D, dev, 16)
         _need(self.had.transform_fn is ops.hadamard_quant)
-        p.had_scale = self.had.had_scale / float(self.had.x_H_scale)
+        p.had_scale = _number(self.had.had_scale) / float(_number(self.had.x_H_scale))
         p.A_log = _ptr(s.A_log, torch.int8, H, dev)
         p.D = _ptr(s.D, torch.int8, D if s.D_has_hdim else H, dev)
         p.dt_bias = _ptr(s.dt_bias, torch.float16, H, dev)

@@ -46,7 +46,7 @@ class QRMSNormGated(torch.nn.Module):
         return state_dict
 
     def _load_scales(self, state_dict, prefix, local_metadata, strict, missing_keys, unexpected_keys, error_msgs):
-        self.z_scale = state_dict.pop(prefix + "z_scale")
+        self.z_scale = float(state_dict.pop(prefix + "z_scale"))
         self.output_scale = state_dict.pop(prefix + "output_scale")
 
     @torch.no_grad()

@@ -185,3 +185,19 @@ def test_unaligned_hidden_states(dev, cls, build):
     with pytest.raises(RuntimeError):
         m.step(h[:, :2].reshape(2, 1, 256), conv, ssm)
     assert torch.equal(conv, kept[0]) and torch.equal(ssm, kept[1])
+
+
+@pytest.mark.parametrize("cls,build", MIXERS)
+def test_a_scale_held_as_a_tensor_may_change_in_place(dev, cls, build):
+    m, g = build(cls, dev, seed=9)
+    h = _ri(dev, g, 2, 20, 256)
+    want = [m.forward(h)]
+    m.had.x_H_scale *= 2.0
+    want.append(m.forward(h))
+    m.had.x_H_scale = torch.tensor(m.had.x_H_scale / 2.0)
+    got = [m.forward(h)]
+    m.had.x_H_scale.mul_(2.0)
+    got.append(m.forward(h))
+    for a, b in zip(got, want):                              # (as in _close: fp16 scan outputs may differ in the last place)
+        assert float((a.float() - b.float()).abs().max()) <= 2e-2 * float(b.float().abs().max())
+    assert not torch.equal(got[0], got[1])

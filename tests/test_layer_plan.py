@@ -3,6 +3,7 @@ import ctypes as C
 import gc
 import weakref
 
+import numpy as np
 import pytest
 import torch
 import torch.nn as nn
@@ -117,6 +118,29 @@ def test_a_plan_made_of_the_wrong_things_is_an_error():
             plan(*args)
     with pytest.raises(TypeError):
         plan.__new__(plan).run(HIDDEN, None, None, False)
+
+
+@pytest.mark.parametrize("cls", MIXERS)
+def test_a_number_that_can_change_in_place_is_left_to_the_modules(cls):
+    m = _mixer(cls)
+    cpu = torch.device("cpu")
+    m._native_block(cpu)
+    names = [("had", "x_H_scale"), ("had", "had_scale"), ("out_proj", "alpha")] + (
+        [("norm", "z_scale"), ("norm", "eps"), ("conv1d", "x_scale"), ("conv1d", "wB_scale"), ("conv1d", "bC_scale"), ("qchunk_scan", "dt_limit")]
+        if hasattr(m, "norm") else [("conv1d", n) for n in ("input_scale", "weight_scale", "bias_scale", "output_scale")])
+    for module, name in names:
+        md = m._modules[module]
+        if name not in md.__dict__:
+            continue                                         # (4-bit projections have no alpha)
+        kept = getattr(md, name)
+        for held in ([torch.tensor(v) for v in (kept, 1.0)] if name != "dt_limit" else [[0.0, 1.0], (torch.tensor(0.0), 1.0)]):
+            setattr(md, name, held)
+            with pytest.raises(_layer_call._Unsupported):
+                m._native_block(cpu)
+        setattr(md, name, kept)
+    m._native_block(cpu)
+    m.had.x_H_scale = np.float32(0.5)                        # (a number like any other)
+    m._native_block(cpu)
 
 
 class _Runtime:
