@@ -14,6 +14,7 @@ import torch
 import torch.nn.modules.module as _module
 
 from . import _lib
+from .linear import _AlphaHooks, _W4A8Base
 
 _host = None
 
@@ -58,14 +59,14 @@ def _ptr(t, dtype, numel, device, align=1):
 def _number(v):
     """A value that goes into the block as a number: one that only changes by becoming another object.  (A tensor or an array
     of one element can change in place, which the plan would not see: the modules read it on every call.)"""
-    _need(isinstance(v, numbers.Real))
+    _need(type(v) in (float, int, bool) or isinstance(v, numbers.Real))
     return v
 
 
 def linear_block(lin, device):
     """QaLinearParams of one of the linear modules."""
     p = _lib.QaLinearParams()
-    if hasattr(lin, "s_group"):
+    if isinstance(lin, _W4A8Base):
         n, k = lin.size_n, lin.size_k
         p.n, p.k, p.bits, p.col_numel = n, k, 4, n
         p.weight = _ptr(lin.weight, torch.uint8, n * (k // 2), device, 16)
@@ -80,7 +81,7 @@ def linear_block(lin, device):
         p.weight = _ptr(lin.weight.t(), torch.int8, n * k, device, 16)
         p.col_scale = _ptr(lin.b, torch.float32, lin.b.numel(), device)
         p.row_scale = _ptr(lin.a, torch.float32, 1, device)
-        if hasattr(lin, "alpha"):
+        if isinstance(lin, _AlphaHooks):
             p.row_rule, p.alpha = _lib.QA_ROW_ALPHA, _number(lin.alpha)
         else:
             p.row_rule = _lib.QA_ROW_HALF_AWAY
@@ -99,31 +100,35 @@ def _native(mixer):
     return family, bytes(block), fns, dims, mixer.out_proj.pad_out, mixer.out_proj.weight, runtime
 
 
-# class -> what is callable in it, as it was when this package was imported
-_CODE = {}
-
-
-def _code_of(cls):
-    return {n: f for n, f in vars(cls).items() if callable(f) or isinstance(f, (classmethod, staticmethod, property))}
+# The classes whose methods the library call stands for, as they were when this package was imported: what each of them
+# holds itself, and the names under which it and its bases hold something callable.
+_HELD, _CALLABLE = {}, {}
 
 
 def remember(*classes):
     """The library call stands for the methods of these classes as they are now."""
     for cls in classes:
+        _CALLABLE[cls] = frozenset(n for n in dir(cls) if callable(getattr(cls, n, None)))
         for c in cls.__mro__:
             if c.__module__.split(".")[0] == __package__ or c is torch.nn.Module:
-                _CODE[c] = _code_of(c)
+                _HELD[c] = dict(vars(c))
 
 
-def _own_code(module):
-    """Whether calling the module's methods runs the code of its class: no method replaced on the instance (as offloading
+def _code_of(held):
+    return {n: f for n, f in held.items() if callable(f) or isinstance(f, (classmethod, staticmethod, property))}
+
+
+def _classes_of(modules):
+    return list({c: None for m in modules for c in type(m).__mro__ if c in _HELD})
+
+
+def _own_code(modules, classes):
+    """Whether calling the modules' methods runs the code of their classes: no method replaced on the instance (as offloading
     and tracing tools wrap modules) or on the class, no compiled form in their place."""
-    if module.__dict__.get("_compiled_call_impl") is not None:
-        return False
-    for c in type(module).__mro__:
-        if c in _CODE and _code_of(c) != _CODE[c]:
+    for c in classes:
+        if vars(c) != _HELD[c] and _code_of(vars(c)) != _code_of(_HELD[c]):
             return False
-    return not any(callable(getattr(type(module), n, None)) for n in module.__dict__)
+    return all(type(m) in _CALLABLE and _CALLABLE[type(m)].isdisjoint(m.__dict__) and m.__dict__.get("_compiled_call_impl") is None for m in modules)
 
 
 def _make(mixer):
@@ -132,11 +137,13 @@ def _make(mixer):
     watched = [mixer._modules]
     hooks = [getattr(_module, k) for k in ("_global_forward_hooks", "_global_forward_pre_hooks")]
     for m in mods:
-        watched += [m.__dict__, m._buffers, m._parameters]
-        hooks += [m._forward_hooks, m._forward_pre_hooks]
-    watched += {c: None for m in mods for c in type(m).__mro__ if c in _CODE}
+        held = m.__dict__
+        watched += [held, held["_buffers"], held["_parameters"]]
+        hooks += [held["_forward_hooks"], held["_forward_pre_hooks"]]
+    classes = _classes_of(mods)
+    watched += classes
     try:
-        _need(mixer._native_modules() is not None and all(_own_code(m) for m in mods))
+        _need(mixer._native_modules() is not None and _own_code(mods, classes))
         native = _native(mixer)
     except _Unsupported:
         native = None

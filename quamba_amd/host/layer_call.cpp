@@ -122,10 +122,12 @@ int make_plan(PlanObject* self, PyObject* args) {
         PyObject* from = PyTuple_GET_ITEM(watched, i);
         PyObject* dict = keep(PyType_Check(from) ? reinterpret_cast<PyTypeObject*>(from)->tp_dict : from);
         s->watches.push_back({dict, version_of(dict), {}});
+        s->watches.back().entries.reserve(PyDict_GET_SIZE(dict));
         PyObject *key, *value;
         Py_ssize_t pos = 0;
         while (PyDict_Next(dict, &pos, &key, &value)) {
-            const bool tensor = THPVariable_Check(value);
+            // (by type: THPVariable_Check asks the metaclass about everything that is no tensor)
+            const bool tensor = PyObject_TypeCheck(value, reinterpret_cast<PyTypeObject*>(THPVariableClass));
             s->watches.back().entries.push_back({keep(key), keep(value), tensor, tensor ? address_of(value) : nullptr});
             if (tensor) s->tensors.push_back(s->watches.back().entries.back());
         }

@@ -204,6 +204,10 @@ def test_the_current_device_comes_back_however_the_call_ends():
     assert r.plan.run(HIDDEN.float(), None, None, False) is None and not r.calls and r.device == 3
 
 
+def _own_code(*modules):
+    return _layer_call._own_code(modules, _layer_call._classes_of(modules))
+
+
 def _public(module):
     return [n for c in type(module).__mro__ if c.__module__.startswith("quamba_amd") for n, f in vars(c).items() if callable(f) and not n.startswith("__")]
 
@@ -211,15 +215,15 @@ def _public(module):
 @pytest.mark.parametrize("cls", MIXERS)
 def test_a_method_replaced_on_a_module_is_another_layer(cls):
     m = _mixer(cls)
-    assert all(_layer_call._own_code(module) for module in m._modules.values())
+    assert _own_code(*m._modules.values())
     for module in m._modules.values():
         names = _public(module)
         assert "forward" in names
         for name in names + ["_call_impl", "_compiled_call_impl"]:
             plan = _layer_call._make(m)
-            assert _unchanged(plan) and _layer_call._own_code(module)
+            assert _unchanged(plan) and _own_code(module)
             module.__dict__[name] = lambda *a, **k: None
-            assert not _unchanged(plan) and not _layer_call._own_code(module), name
+            assert not _unchanged(plan) and not _own_code(module), name
             del module.__dict__[name]
     plan = _layer_call._make(m)
     m.had.transform_fn = lambda x, s: x
@@ -233,8 +237,8 @@ def test_a_method_replaced_on_a_class_is_another_layer(cls, monkeypatch):
         for c in (type(module), torch.nn.Module):
             name = "forward" if c is not torch.nn.Module else "__call__"
             plan = _layer_call._make(m)
-            assert _unchanged(plan) and _layer_call._own_code(module)
+            assert _unchanged(plan) and _own_code(module)
             with monkeypatch.context() as patch:
                 patch.setattr(c, name, lambda *a, **k: None)
-                assert not _unchanged(plan) and not _layer_call._own_code(module)
-            assert _layer_call._own_code(module)
+                assert not _unchanged(plan) and not _own_code(module)
+            assert _own_code(module)
