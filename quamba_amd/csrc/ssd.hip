@@ -215,15 +215,16 @@ __device__ __forceinline__ void unit_head_part(int linear, int units, int hpg, i
 // Stages 2, 3 and 6 (quamba/triton/quant_chunk_state.py:76-89, quant_state_passing.py:60-83, quant_ssm_states.py
 // :43,119): a workgroup of N / 16 waves per (batch, head) walks the chunks in order with the running state P
 // (64 x N of headdim x dstate, fp32) in registers; the fp32 chunk states never travel
-// through memory.  A wave owns 16 columns n and all rows p.  Its B operand, f16(q_B[k,n] (s_B w_k)) with the
+// through memory.  A wave owns 16 columns n and all rows p.  Its B operand, f16((s_B q_B[k,n]) w_k) with the
 // per-head weight w_k = exp(dA_last - dA_k) dt_k, is built in registers from the transposed int8 B tile in LDS
 // (rows n of 4-byte-aligned pitch with an odd number of dwords: conflict-free for the transposing dword stores
 // and for the operand reads); its A operand is the transposed x tile.  The tiles of chunk c+1 are fetched into
 // registers while chunk c is multiplied.  The state entering chunk c >= 1 is stored as fp16, rows in slot order.
 // Bound by vector issue (converting x and B to fp16 operands) and by the LDS reads of the x tile, which every wave makes: with
-// one workgroup for all N columns x is staged once; as a workgroup per 64 columns, which also formed s_B q_B and the product
-// with w_k apart, 16 x 1024 steps of 128 heads took 146 us, now 122.  (Four waves of 32 columns instead of eight of 16 read
-// x half as often and take 138: too few waves for the latencies of a chunk.)
+// one workgroup for all N columns x is staged once: as a workgroup per 64 columns 16 x 1024 steps of 128 heads took 146 us, now
+// 129.  (Four waves of 32 columns instead of eight of 16 read x half as often and take 138: too few waves for the latencies
+// of a chunk.  With s_B in the weight, q_B (s_B w_k), a product less per value: 128, but at fp16 ties another value than the
+// reference's; the general kernels round the same one.)
 // ---------------------------------------------------------------------------------------------
 template <int N, int Q>
 struct StateSmem {
@@ -328,7 +329,7 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
                 *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 3][bkb * 4]) = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
             }
         }
-        if (tid < Q) sm.w[tid] = sB * (fexp(r_last - r_dA) * r_dt);        // weight of step k in the chunk's state
+        if (tid < Q) sm.w[tid] = fexp(r_last - r_dA) * r_dt;        // weight of step k in the chunk's state
     };
 
     // the running state: columns n = 16 wave + lane % 16; tile j, register r: channel p = 4 (4 (lane / 16) + r) + j
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
             const float wk[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
             v8h bw;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) bw[e] = static_cast<_Float16>(sbyte_of(e < 4 ? b0 : b1, e & 3) * wk[e]);
+            for (int e = 0; e < 8; ++e) bw[e] = static_cast<_Float16>((sB * sbyte_of(e < 4 ? b0 : b1, e & 3)) * wk[e]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) accs[j] = mfma16(fx[j], bw, accs[j]);
         }
