@@ -63,3 +63,55 @@ def test_4_bit_weights(dev, M, N, K, workspace):
     finally:
         ops.W4A8_EXPAND_ONCE_ROWS = rows
     np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+# 128 x 128 with four stages, 128 x 256 with three, 256 x 256, 256 x 320 and 320 x 256 with two: K of as many k tiles as there
+# are stages and one more, and of so many that the ring of stages goes round several times, with and without a remainder
+LARGE = [(1500, 2500), (1500, 5000), (4090, 4090), (4090, 5100), (5100, 4090)]
+
+
+@pytest.mark.parametrize("M,N", LARGE)
+@pytest.mark.parametrize("K", [384, 512, 640, 1712, 2560])
+@pytest.mark.parametrize("order,dtype", [(0, torch.int8), (1, torch.int8), (0, torch.float16), (0, torch.bfloat16)])
+def test_large_tiles_over_a_long_k(dev, M, N, K, order, dtype):
+    """Sums of integers below 2^53 are exact in float64 whatever their order, the epilogue is two fp32 products and a rounding."""
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    a, w = (torch.randint(-128, 128, s, dtype=torch.int8, device=dev, generator=g) for s in ((M, K), (N, K)))
+    sa, sb = torch.rand(M, device=dev, generator=g) * 0.02 + 0.01, (torch.rand(N, device=dev, generator=g) + 0.5) * 0.6 / K ** 0.5
+    acc = (a.double() @ w.double().t()).float()
+    v = sb * (sa[:, None] * acc) if order else sa[:, None] * (sb * acc)
+    want = v.round().clamp(-128, 127).to(torch.int8) if dtype == torch.int8 else v.to(dtype)
+    got = torch.empty((M, N), dtype=dtype, device=dev)
+    p = _lib.QaGemmW8A8Params()
+    p.m, p.n, p.k, p.a_scale_numel, p.w_scale_numel, p.scale_order = M, N, K, M, N, order
+    p.out_type = {torch.int8: _lib.QA_OUT_I8, torch.float16: _lib.QA_OUT_F16, torch.bfloat16: _lib.QA_OUT_BF16}[dtype]
+    p.lda = p.ldw = K
+    p.ldd = N
+    p.a, p.w, p.a_scale, p.w_scale, p.d = (t.data_ptr() for t in (a, w, sa, sb, got))
+    _lib.check(_lib.lib().qa_gemm_w8a8(ctypes.byref(p), _lib.current_stream(dev)), "gemm_w8a8")
+    assert torch.equal(got, want)
+    if dtype == torch.int8:
+        assert int(want.max()) - int(want.min()) > 100
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 300, 640), (1500, 2500, 1712)])
+def test_the_single_row_rules_with_many_rows(dev, M, N, K):
+    """128 x 128 with two stages: the host's scalar, and rounding half away from zero."""
+    g = torch.Generator(device=dev).manual_seed(K)
+    a, w = (torch.randint(-128, 128, s, dtype=torch.int8, device=dev, generator=g) for s in ((M, K), (N, K)))
+    acc = (a.double() @ w.double().t()).float()
+    got = torch.empty((M, N), dtype=torch.int8, device=dev)
+    p = _lib.QaGemmW8A8Params()
+    p.m, p.n, p.k, p.a_scale_numel, p.w_scale_numel = M, N, K, 1, N
+    p.lda = p.ldw = K
+    p.ldd = N
+    alpha = torch.tensor(0.012 / K ** 0.5, device=dev)
+    p.use_alpha, p.alpha = 1, float(alpha)
+    p.a, p.w, p.d = a.data_ptr(), w.data_ptr(), got.data_ptr()
+    _lib.check(_lib.lib().qa_gemm_w8a8(ctypes.byref(p), _lib.current_stream(dev)), "gemm_w8a8")
+    assert torch.equal(got, (alpha * acc).round().clamp(-128, 127).to(torch.int8))
+    sa, sb = torch.tensor([0.5], device=dev), (torch.rand(N, device=dev, generator=g) + 0.5) * 0.025 / K ** 0.5
+    p.use_alpha, p.round_mode, p.a_scale, p.w_scale = 0, _lib.QA_ROUND_HALF_AWAY, sa.data_ptr(), sb.data_ptr()
+    _lib.check(_lib.lib().qa_gemm_w8a8(ctypes.byref(p), _lib.current_stream(dev)), "gemm_w8a8")
+    v = ((sb * sa) * acc).double()
+    assert torch.equal(got, (v.sign() * (v.abs() + 0.5).floor()).clamp(-128, 127).to(torch.int8))
