@@ -195,53 +195,31 @@ struct TileLoader {
     }
 };
 
-// The fragments of k step kk of this wave's rows (sa: TM row blocks of the a operand, sw: TN of the w operand).
-template <int TM, int TN>
-__device__ __forceinline__ void fetch_fragments(const uint8_t* sa, const uint8_t* sw, int kk, int frow, int fhalf,
-                                                v4i (&fa)[TM], v4i (&fw)[TN]) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
-        const int row = i * 32 + frow;
-        fw[i] = *reinterpret_cast<const v4i*>(sw + row * kBK + swz(row, kk * 2 + fhalf) * 16);
-    }
-#pragma unroll
-    for (int j = 0; j < TM; ++j) {
-        const int row = j * 32 + frow;
-        fa[j] = *reinterpret_cast<const v4i*>(sa + row * kBK + swz(row, kk * 2 + fhalf) * 16);
-    }
-}
-
-// Accumulates one 128-byte k tile with the instruction order pinned: sa / sw point at this wave's rows of the
-// staged operands.  The fragments of step kk+1 are requested
-// before the multiplications of step kk are issued, and `hook(slot)` runs after every second
-// multiplication (slot = 0 .. 4*TM*TN/2 - 1): the caller places its global -> LDS requests for the
-// next tile there, one at a time, so that the wave never waits on a full memory queue with
-// multiplications behind it in program order.  sched_barrier keeps the compiler from regrouping.
-template <int TM, int TN, class Hook>
-__device__ __forceinline__ void mma_tile_paced(const uint8_t* sa, const uint8_t* sw, int frow, int fhalf,
-                                               v16i (&acc)[TN][TM], Hook&& hook) {
-    // (a lone multiplication per step does not cover the time its fragments take: all four steps' are fetched at once)
-    constexpr int kAhead = TM * TN == 1 ? 3 : 1, kBufs = TM * TN == 1 ? 4 : 2;
-    v4i fa[kBufs][TM], fw[kBufs][TN];
-    auto fetch = [&](int kk) { fetch_fragments<TM, TN>(sa, sw, kk, frow, fhalf, fa[kk % kBufs], fw[kk % kBufs]); };
+// Accumulates one 128-byte k tile of one 32 x 32 block with the instruction order pinned: sa / sw point at this wave's rows of
+// the staged operands.  A lone multiplication per step does not cover the time its fragments take: three of the four steps'
+// are requested ahead of the first one, the last behind it in program order, and `hook(step)` runs after every multiplication:
+// the caller places its global -> LDS requests for the next tile there, one at a time, so that the wave never waits on a full
+// memory queue with multiplications behind it in program order.  sched_barrier keeps the compiler from regrouping.
+template <class Hook>
+__device__ __forceinline__ void mma_tile_paced(const uint8_t* sa, const uint8_t* sw, int frow, int fhalf, v16i& acc, Hook&& hook) {
+    constexpr int kSteps = kBK / 32, kAhead = 3;
+    v4i fa[kSteps], fw[kSteps];
+    auto fetch = [&](int kk) {
+        const int at = frow * kBK + swz(frow, kk * 2 + fhalf) * 16;
+        fw[kk] = *reinterpret_cast<const v4i*>(sw + at);
+        fa[kk] = *reinterpret_cast<const v4i*>(sa + at);
+    };
 #pragma unroll
     for (int kk = 0; kk < kAhead; ++kk) fetch(kk);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int kk = 0; kk < kBK / 32; ++kk) {
-        if (kk + kAhead < kBK / 32) fetch(kk + kAhead);
+    for (int kk = 0; kk < kSteps; ++kk) {
+        if (kk + kAhead < kSteps) fetch(kk + kAhead);
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < TN; ++i)
-#pragma unroll
-            for (int j = 0; j < TM; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[kk % kBufs][i], fa[kk % kBufs][j], acc[i][j], 0, 0, 0);
-                if (TM * TN == 1 || (i * TM + j) % 2 == 1) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    hook(TM * TN == 1 ? kk : kk * (TM * TN / 2) + (i * TM + j) / 2);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[kk], fa[kk], acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        hook(kk);
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 

@@ -28,36 +28,35 @@ namespace {
 
 using namespace gemm;
 
-// The tile kernel.  Everything that comes from memory goes straight to LDS, STAGES - 1 tiles ahead and counted by hand: the
+// The tile kernel, 64 x 64 outputs over four waves of 32 x 32.  Everything that comes from memory goes straight to LDS, STAGES - 1 tiles ahead and counted by hand: the
 // activations as the fragments want them, the packed weights and their group scales as each thread's own 16 bytes and word
 // (no other lane reads those: they are registers that a load in flight does not occupy).  During the multiplications of tile
-// t a thread expands its codes of tile t + 1, a word behind every multiplication or two, into the one of two int8 weight
+// t a thread expands its codes of tile t + 1, a word behind every multiplication, into the one of two int8 weight
 // tiles that is not being read: the vector units work in the shadow of the matrix cores.  (Behind all multiplications of a
 // tile instead, with a tile's loads issued one tile ahead, a 64 x 64 tile on a CU of its own took 0.67 us per 128 of K; now
 // 0.38, of which the expansion is 0.15 and the LDS traffic of fragments, codes and tiles about as much.)
-template <int TM, int TN, int WGM, int WGN, int STAGES>
-struct W4Cfg {
-    using C = Cfg<TM, TN, WGM, WGN, STAGES>;
-    static constexpr int kWPacked = C::kBN * 4 / C::kThreads;      // 16-byte packed chunks (32 codes) per thread per tile
-    static constexpr int kSlots = STAGES - 1;                      // tiles of packed weights
+struct W4Tile {
+    static constexpr int kStages = 3;
+    using C = Cfg<1, 1, 2, 2, kStages>;
+    static constexpr int kSlots = kStages - 1;                     // tiles of packed weights
     static constexpr int kABytes = C::kBM * kBK, kWBytes = C::kBN * kBK;
-    static constexpr int kPackedBytes = C::kBN * (kBK / 2), kScaleBytes = kWPacked * C::kThreads * 4;
-    static constexpr int kScalesAt = STAGES * kABytes + 2 * kWBytes + kSlots * (kPackedBytes + kScaleBytes);
+    static constexpr int kPackedBytes = C::kBN * (kBK / 2), kScaleBytes = C::kThreads * 4;      // a thread: 16 bytes (32 codes), a word
+    static constexpr int kScalesAt = kStages * kABytes + 2 * kWBytes + kSlots * (kPackedBytes + kScaleBytes);
     static constexpr int kLdsBytes = kScalesAt + TileScales<C::kBM, C::kBN, C::kWaves>::kBytes;
+    static_assert(kPackedBytes == 16 * C::kThreads && epilogue_lds_bytes<1, 1, C::kWaves>() <= kScalesAt, "tile shape");
 };
 
-template <int TM, int TN, int WGM, int WGN, int STAGES, bool GROUPED, int OUT>
-__global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Params p) {
-    using W = W4Cfg<TM, TN, WGM, WGN, STAGES>;
-    using C = typename W::C;
-    constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves, THREADS = C::kThreads, kWPacked = W::kWPacked;
-    static_assert(kWPacked * THREADS == BN * 4 && epilogue_lds_bytes<TM, TN, WAVES>() <= W::kScalesAt, "tile shape");
+template <bool GROUPED, int OUT>
+__global__ __launch_bounds__(W4Tile::C::kThreads) void gemm_w4a8_kernel(QaGemmW4A8Params p) {
+    using W = W4Tile;
+    using C = W::C;
+    constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves, STAGES = W::kStages;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave % WGM, wn = wave / WGM;
+    const int wm = wave & 1, wn = wave >> 1;
     const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
     int tile_m, tile_n;
     tile_of_workgroup<BM, BN>(blockIdx.x, tiles_m, tiles_n, tile_m, tile_n);
@@ -82,58 +81,39 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
         buffer_load_lds_b128(rsrc_a, lds_base + stage * W::kABytes + (r * WAVES + wave) * 1024, load_a.voff[r], min(tile, last) * kBK);
     };
 
-    // this thread's packed chunks of the weight tile: row id / 4, codes 32 (id % 4) .. + 31
-    int w_off[kWPacked], s_col[kWPacked];
-    uint32_t s_pick[kWPacked];                             // the half of the fetched word, twice
-    uint8_t* to_w[kWPacked][2];
-#pragma unroll
-    for (int i = 0; i < kWPacked; ++i) {
-        const int id = tid + i * THREADS, row = id >> 2, quarter = id & 3;
-        w_off[i] = row * ldw + quarter * 16;
-        s_col[i] = s_first + min(n0 + row, p.n - 1);
-        s_pick[i] = 0x01000100u + (s_col[i] & 1) * 0x02020202u;
-        to_w[i][0] = lds + kAtW + row * kBK + swz(row, 2 * quarter) * 16;
-        to_w[i][1] = lds + kAtW + row * kBK + swz(row, 2 * quarter + 1) * 16;
-    }
+    // this thread's packed chunk of the weight tile: row tid / 4, codes 32 (tid % 4) .. + 31
+    const int row = tid >> 2, quarter = tid & 3;
+    const int w_off = row * ldw + quarter * 16, s_col = s_first + min(n0 + row, p.n - 1);
+    uint32_t s_pick = 0x01000100u + (s_col & 1) * 0x02020202u;     // the half of the fetched word, twice
+    uint8_t* const to_w[2] = {lds + kAtW + row * kBK + swz(row, 2 * quarter) * 16, lds + kAtW + row * kBK + swz(row, 2 * quarter + 1) * 16};
     const uint32_t s_flip = p.n & 1 ? 0x02020202u : 0u;
     auto issue_w = [&](int tile, int slot) {
         const int t = min(tile, last);
-#pragma unroll
-        for (int i = 0; i < kWPacked; ++i) {
-            buffer_load_lds_b128(rsrc_w, lds_base + kAtPacked + slot * W::kPackedBytes + (i * WAVES + wave) * 1024, w_off[i], t * (kBK / 2));
-            if constexpr (GROUPED) buffer_load_lds_b32(rsrc_s, lds_base + kAtScale + slot * W::kScaleBytes + (i * WAVES + wave) * 256, ((s_col[i] + t * p.n) << 1) & ~3);
-        }
+        buffer_load_lds_b128(rsrc_w, lds_base + kAtPacked + slot * W::kPackedBytes + wave * 1024, w_off, t * (kBK / 2));
+        if constexpr (GROUPED) buffer_load_lds_b32(rsrc_s, lds_base + kAtScale + slot * W::kScaleBytes + wave * 256, ((s_col + t * p.n) << 1) & ~3);
     };
-    uint4 wreg[kWPacked];
-    __half2 s2[kWPacked];
+    uint4 wreg;
+    __half2 s2;
     auto fetch_w = [&](int slot) {                         // tile after tile
-#pragma unroll
-        for (int i = 0; i < kWPacked; ++i) {
-            wreg[i] = *reinterpret_cast<const uint4*>(lds + kAtPacked + slot * W::kPackedBytes + (i * THREADS + tid) * 16);
-            if constexpr (GROUPED) {
-                const uint32_t word = *reinterpret_cast<const uint32_t*>(lds + kAtScale + slot * W::kScaleBytes + (i * THREADS + tid) * 4);
-                s2[i] = bits_h2(__builtin_amdgcn_perm(word, word, s_pick[i]));
-                s_pick[i] ^= s_flip;
-            }
+        wreg = *reinterpret_cast<const uint4*>(lds + kAtPacked + slot * W::kPackedBytes + tid * 16);
+        if constexpr (GROUPED) {
+            const uint32_t word = *reinterpret_cast<const uint32_t*>(lds + kAtScale + slot * W::kScaleBytes + tid * 4);
+            s2 = bits_h2(__builtin_amdgcn_perm(word, word, s_pick));
+            s_pick ^= s_flip;
         }
     };
-    // word `w` of this thread's kWPacked * 4 (a pair is written when its second one is done)
+    // word `w` of this thread's four (a pair is written when its second one is done)
     uint2 done;
     auto expand_w = [&](int w, int to) {
-        const int i = w / 4, t = w % 4;
-        const uint32_t packed = t == 0 ? wreg[i].x : t == 1 ? wreg[i].y : t == 2 ? wreg[i].z : wreg[i].w;
-        const uint2 e = GROUPED ? expand_grouped(packed, s2[i]) : expand_per_channel(packed);
-        if (t % 2 == 0) done = e;
-        else *reinterpret_cast<uint4*>(to_w[i][t / 2] + to * W::kWBytes) = make_uint4(done.x, done.y, e.x, e.y);
+        const uint32_t packed = w == 0 ? wreg.x : w == 1 ? wreg.y : w == 2 ? wreg.z : wreg.w;
+        const uint2 e = GROUPED ? expand_grouped(packed, s2) : expand_per_channel(packed);
+        if (w % 2 == 0) done = e;
+        else *reinterpret_cast<uint4*>(to_w[w / 2] + to * W::kWBytes) = make_uint4(done.x, done.y, e.x, e.y);
     };
 
-    v16i acc[TN][TM];
+    v16i acc[1][1];
 #pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int j = 0; j < TM; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    for (int r = 0; r < 16; ++r) acc[0][0][r] = 0;
 
     if (k_tiles > 0) {
         // Requests go out in the order W(0) A(0) W(1) A(1) ..., the first tile's weights being expanded before the loop
@@ -144,17 +124,17 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
             for (int r = 0; r < C::kAInstr; ++r) issue_a(r, s, s);
             if (s + 1 < STAGES - 1) issue_w(s + 1, s + 1);
         }
-        constexpr int kLoads = C::kAInstr + (GROUPED ? 2 : 1) * kWPacked;      // requests of a wave per tile
+        constexpr int kLoads = C::kAInstr + (GROUPED ? 2 : 1);                 // requests of a wave per tile
         __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 2) * kLoads + C::kAInstr));
         wave_lds_sync();
         fetch_w(0);
 #pragma unroll
-        for (int w = 0; w < 4 * kWPacked; ++w) expand_w(w, 0);
+        for (int w = 0; w < 4; ++w) expand_w(w, 0);
         __builtin_amdgcn_sched_barrier(0);
         issue_w(STAGES - 1, 0);
         const int frow = lane & 31, fhalf = lane >> 5;
-        static_assert(STAGES == 2 || STAGES == 3, "the unrolled tiles have to cover whole turns of stages, slots and weight tiles");
-        constexpr int kUnroll = STAGES == 2 ? 2 : 6;
+        constexpr int kUnroll = 6;                                             // whole turns of stages, slots and weight tiles
+        static_assert(kUnroll % STAGES == 0 && kUnroll % W::kSlots == 0 && kUnroll % 2 == 0 && C::kAInstr <= 4, "a request behind each of four multiplications");
         for (int base = 0; base < k_tiles; base += kUnroll) {
             static_for<0, kUnroll>([&](auto u_c) {
                 constexpr int u = decltype(u_c)::value;
@@ -164,20 +144,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
                 __syncthreads();
                 fetch_w((u + 1) % W::kSlots);
                 __builtin_amdgcn_sched_barrier(0);
-                constexpr int kSteps = TM * TN == 1 ? 4 : 4 * (TM * TN / 2), kPerStep = (C::kAInstr + kSteps - 1) / kSteps;
-                constexpr int kWords = (4 * kWPacked + kSteps - 1) / kSteps;
-                mma_tile_paced<TM, TN>(lds + (u % STAGES) * W::kABytes + (wm * TM * 32) * kBK, lds + kAtW + (u % 2) * W::kWBytes + (wn * TN * 32) * kBK, frow, fhalf, acc,
-                                       [&](int step) {
-                                           // (the fragments of the multiplication before this were read after fetch_w's
-                                           // words, so these are in their registers and the slot they came from is free)
-                                           if (step == 0) issue_w(kt + STAGES, (u + STAGES) % W::kSlots);
-#pragma unroll
-                                           for (int r = step * kPerStep; r < (step + 1) * kPerStep; ++r)
-                                               if (r < C::kAInstr) issue_a(r, kt + STAGES - 1, (u + STAGES - 1) % STAGES);
-#pragma unroll
-                                           for (int w = step * kWords; w < (step + 1) * kWords; ++w)
-                                               if (w < 4 * kWPacked) expand_w(w, (u + 1) % 2);
-                                       });
+                mma_tile_paced(lds + (u % STAGES) * W::kABytes + wm * 32 * kBK, lds + kAtW + (u % 2) * W::kWBytes + wn * 32 * kBK, frow, fhalf, acc[0][0],
+                               [&](int step) {
+                                   // (the fragments of the multiplication before this were read after fetch_w's
+                                   // words, so these are in their registers and the slot they came from is free)
+                                   if (step == 0) issue_w(kt + STAGES, (u + STAGES) % W::kSlots);
+                                   if (step < C::kAInstr) issue_a(step, kt + STAGES - 1, (u + STAGES - 1) % STAGES);
+                                   expand_w(step, (u + 1) % 2);
+                               });
             });
         }
     }
@@ -187,24 +161,18 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w4a8_kernel(QaGemmW4A8Par
     Epilogue e;
     e.use_alpha = 0; e.alpha = 0.0f; e.round_mode = QA_ROUND_RNE; e.col_outer = 0;
     e.ldd = p.ldd; e.d = p.d;
-    epilogue<TM, TN, OUT, false, false>(e, acc, lds, p.m, p.n, m0 + wm * TM * 32, n0 + wn * TN * 32, wave, lane,
-                                          reinterpret_cast<const float*>(lds + W::kScalesAt), BN + wm * TM * 32, wn * TN * 32);
+    epilogue<1, 1, OUT, false, false>(e, acc, lds, p.m, p.n, m0 + wm * 32, n0 + wn * 32, wave, lane,
+                                      reinterpret_cast<const float*>(lds + W::kScalesAt), BN + wm * 32, wn * 32);
 }
 
 template <int OUT>
 int launch_tile(const QaGemmW4A8Params& p, hipStream_t stream) {
-    constexpr int TM = 1, TN = 1, WGM = 2, WGN = 2, STAGES = 3;
-    using W = W4Cfg<TM, TN, WGM, WGN, STAGES>;
-    using C = typename W::C;
+    using W = W4Tile;
+    using C = W::C;
     const int64_t tiles = static_cast<int64_t>((p.m + C::kBM - 1) / C::kBM) * ((p.n + C::kBN - 1) / C::kBN);
     if (tiles > 0x7fffffffLL || static_cast<int64_t>(C::kBN) * p.k > 0x7fffffffLL || static_cast<int64_t>(p.n) * p.k > 64LL * 0x7fffff00LL) return QA_ERR_SHAPE;
-    auto kernel = p.group_size > 0 ? gemm_w4a8_kernel<TM, TN, WGM, WGN, STAGES, true, OUT> : gemm_w4a8_kernel<TM, TN, WGM, WGN, STAGES, false, OUT>;
-    if (W::kLdsBytes > 65536) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                W::kLdsBytes) != hipSuccess) {
-            return check_launch();
-        }
-    }
+    static_assert(W::kLdsBytes <= 65536, "more LDS than a launch gets by default");
+    auto kernel = p.group_size > 0 ? gemm_w4a8_kernel<true, OUT> : gemm_w4a8_kernel<false, OUT>;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(C::kThreads), W::kLdsBytes, stream, p);
     return check_launch();
 }

@@ -128,13 +128,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
         finish(mma.acc);
     } else {
     const int frow = lane & 31, fhalf = lane >> 5;
-    v16i acc[TN][TM];
+    v16i acc[1][1];
 #pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int j = 0; j < TM; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    for (int r = 0; r < 16; ++r) acc[0][0][r] = 0;
     auto issue = [&](int tile) {
         const uint32_t base = lds_base + (tile % STAGES) * C::kStageBytes;
         load_a.template issue<WAVES>(rsrc_a, tile * kBK, p.k, base, wave);
@@ -151,16 +147,11 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
         // (past the end of K every lane is out of range and stores zeros)
         const int nt = kt + STAGES - 1;
         const uint32_t nbase = lds_base + (nt % STAGES) * C::kStageBytes;
-        constexpr int kSlots = TM * TN == 1 ? 4 : 4 * (TM * TN / 2), kPerSlot = (C::kAInstr + C::kWInstr + kSlots - 1) / kSlots;
-        mma_tile_paced<TM, TN>(stage + (wm * TM * 32) * kBK, stage + BM * kBK + (wn * TN * 32) * kBK, frow, fhalf, acc,
-                               [&](int slot) {
-#pragma unroll
-                                   for (int r = slot * kPerSlot; r < (slot + 1) * kPerSlot; ++r) {
-                                       if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, nt * kBK, p.k, nbase, wave);
-                                       else if (r < C::kAInstr + C::kWInstr)
-                                           load_w.template issue_one<WAVES>(r - C::kAInstr, rsrc_w, nt * kBK, p.k, nbase + BM * kBK, wave);
-                                   }
-                               });
+        static_assert(C::kAInstr + C::kWInstr <= 4, "a request behind each of four multiplications");
+        mma_tile_paced(stage + wm * 32 * kBK, stage + BM * kBK + wn * 32 * kBK, frow, fhalf, acc[0][0], [&](int r) {
+            if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, nt * kBK, p.k, nbase, wave);
+            else if (r < C::kAInstr + C::kWInstr) load_w.template issue_one<WAVES>(r - C::kAInstr, rsrc_w, nt * kBK, p.k, nbase + BM * kBK, wave);
+        });
     }
     finish(acc);
     }
