@@ -160,20 +160,25 @@ QaSScanParams scan_sizes(const QaMamba1Params& p) {
     return s;
 }
 
-Mamba1Buffers carve(const QaMamba1Params& p, void* base) {
+// dt_proj inside the scan (sscan_tm.hip) or as a product of its own
+bool dt_in_scan(const QaMamba1Params& p) {
+    return p.dt_proj.bits == 8 && p.dt_proj.k <= kSscanDtRank && p.x_proj.n % 16 == 0 && p.seqlen * static_cast<int64_t>(p.x_proj.n) < 1 << 30;
+}
+
+Mamba1Buffers carve(const QaMamba1Params& p, void* base, bool step) {
     const int64_t t = static_cast<int64_t>(p.batch) * p.seqlen;
     Carver c{static_cast<uint8_t*>(base)};
     Mamba1Buffers b;
     b.xz = c.take<int8_t>(t * p.in_proj.n);
     b.x = c.take<int8_t>(t * p.d_inner);
     b.x_dbl = c.take<int8_t>(t * p.x_proj.n);
-    b.dt = c.take<int8_t>(t * p.dt_proj.n);
+    b.dt = c.take<int8_t>(!step && dt_in_scan(p) ? 0 : t * p.dt_proj.n);       // (8 x 2048 tokens of 5120 channels: 84 MB)
     b.yq = c.take<int8_t>(t * p.d_inner);
     b.y = c.take<__half>(t * p.d_inner * 2);
     b.w8.bytes = std::max(std::max(expanded_bytes(p.in_proj, t), expanded_bytes(p.x_proj, t)),
                           std::max(expanded_bytes(p.dt_proj, t), expanded_bytes(p.out_proj, t)));
     b.w8.p = c.take<uint8_t>(b.w8.bytes);
-    b.scan.bytes = sscan_token_major_workspace(scan_sizes(p));
+    b.scan.bytes = step ? 0 : sscan_token_major_workspace(scan_sizes(p));
     b.scan.p = c.take<uint8_t>(b.scan.bytes);
     b.total = c.off;
     return b;
@@ -211,11 +216,6 @@ int validate(const QaMamba1Params* p) {
     QA_TRY(linear_check(p->dt_proj, t, p->x_proj.n));
     QA_TRY(linear_check(p->out_proj, t, p->d_inner));
     return hadamard_check(p->d_inner);
-}
-
-// dt_proj inside the scan (sscan_tm.hip) or as a product of its own
-bool dt_in_scan(const QaMamba1Params& p) {
-    return p.dt_proj.bits == 8 && p.dt_proj.k <= kSscanDtRank && p.x_proj.n % 16 == 0 && p.seqlen * static_cast<int64_t>(p.x_proj.n) < 1 << 30;
 }
 
 SscanDtProj scan_dt_of(const QaMamba1Params& p, const Mamba1Buffers& b) {
@@ -279,7 +279,7 @@ int ready(const QaMamba1Params* p, bool step, Mamba1Buffers& b) {
     if (!p->hidden || !p->out || !p->workspace || !p->conv_weight || !p->A_log) return QA_ERR_NULL;
     if (step && (!p->conv_state || !p->ssm_state)) return QA_ERR_NULL;
     if (step && p->seqlen != 1) return QA_ERR_SHAPE;
-    b = carve(*p, p->workspace);
+    b = carve(*p, p->workspace, step);
     if (p->workspace_bytes < b.total || (reinterpret_cast<uintptr_t>(p->workspace) & 255u) || !aligned16(p->hidden)) return QA_ERR_STRIDE;
     if (step) return ssm_update_check(update_of(*p, b));
     const SscanDtProj dt = scan_dt_of(*p, b);
@@ -450,9 +450,9 @@ int mamba2_tail(const QaMamba2Params& p, const Mamba2Buffers& b, void* stream) {
 }  // namespace
 }  // namespace qa
 
-extern "C" int64_t qa_mamba1_workspace_bytes(const QaMamba1Params* p, int) {
+extern "C" int64_t qa_mamba1_workspace_bytes(const QaMamba1Params* p, int step) {
     using namespace qa;
-    return validate(p) == QA_OK ? carve(*p, nullptr).total : 0;
+    return validate(p) == QA_OK ? carve(*p, nullptr, step != 0).total : 0;
 }
 
 extern "C" int qa_mamba1_forward(const QaMamba1Params* p, void* stream) {

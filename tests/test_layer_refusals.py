@@ -76,6 +76,16 @@ def test_refused_before_the_first_launch(family, build, change, status, call):
     assert getattr(_lib.lib(), f"qa_mamba{family}_{call}")(C.byref(p), None) == status
 
 
+def test_the_step_sizes_made_in_the_scan_need_no_workspace():
+    """A codes' section for them only where dt_proj is a product of its own."""
+    l, tokens = _lib.lib(), 8 * 640
+    p = _mamba1()
+    p.batch, p.seqlen = 8, 640
+    in_scan = l.qa_mamba1_workspace_bytes(C.byref(p), 0)
+    p.x_proj, p.dt_rank, p.dt_proj = _linear(240, 512), 208, _linear(512, 208)             # a rank the scan does not take
+    assert l.qa_mamba1_workspace_bytes(C.byref(p), 0) - in_scan == tokens * (240 - 48) + tokens * 512
+
+
 def test_sizes_no_kernel_takes_need_no_workspace():
     """Zero bytes: the caller runs the operators one by one, or tells its user."""
     l = _lib.lib()
