@@ -527,10 +527,10 @@ int64_t tiles_of(const QaGemmW4A8Params& p, int64_t bm, int64_t bn) { return ((p
 
 // eight waves share K when there is at most a workgroup per CU and K is long, else four (4096 x 8192 at 64 rows: 13.8
 // against 15.8 us; 18560 x 4096 at 16 rows: 23.0 against 19.1)
-bool skinny_is_wide(const QaGemmW4A8Params& p) { return tiles_of(p, 32, 32) <= 256 && p.k >= 2048; }
+bool skinny_is_wide(const QaGemmW4A8Params& p, int cus) { return tiles_of(p, 32, 32) <= cus && p.k >= 2048; }
 
-int dispatch_skinny(const QaGemmW4A8Params& p, hipStream_t stream) {
-    const bool wide = skinny_is_wide(p);
+int dispatch_skinny(const QaGemmW4A8Params& p, int cus, hipStream_t stream) {
+    const bool wide = skinny_is_wide(p, cus);
     // activation rows are fetched eight at a time: up to 8 rows need one fetch per tile, up to 32 four
     if (p.m <= 8) return wide ? launch_skinny<1, 1, 8, 3>(p, stream) : launch_skinny<1, 1, 4, 3>(p, stream);
     return wide ? launch_skinny<1, 4, 8, 2>(p, stream) : launch_skinny<1, 4, 4, 2>(p, stream);
@@ -569,16 +569,16 @@ __global__ __launch_bounds__(256) void w4_expand_kernel(QaGemmW4A8Params p, int8
 // once, in a pass of their own, cost that pass.
 enum Way { kWaySkinny, kWay64x64, kWay64x128, kWay128x128, kWay192x128, kWayExpandOnce };
 
-int cheapest_way(const QaGemmW4A8Params& p, bool addressable, bool expandable) {
-    const double k_tiles = p.k / 128, kCus = 256;
-    auto rounds = [&](int64_t bm, int64_t bn) { return std::ceil(static_cast<double>(tiles_of(p, bm, bn)) / kCus); };
+int cheapest_way(const QaGemmW4A8Params& p, int cus, bool addressable, bool expandable) {
+    const double k_tiles = p.k / 128;
+    auto rounds = [&](int64_t bm, int64_t bn) { return static_cast<double>((tiles_of(p, bm, bn) + cus - 1) / cus); };
     double best = 1e30;
     int way = kWay128x128;
     auto offer = [&](int w, double cost) {
         if (cost < best) { best = cost; way = w; }
     };
     if (addressable) {
-        const bool wide = skinny_is_wide(p);
+        const bool wide = skinny_is_wide(p, cus);
         offer(kWaySkinny, 3.0 + std::ceil(k_tiles / (wide ? 8 : 4)) * (wide ? 1.35 : 0.75 + 0.38 * rounds(32, 32)));
     }
     offer(kWay64x64, 3.0 + k_tiles * (0.10 + 0.28 * rounds(64, 64)));
@@ -626,10 +626,11 @@ extern "C" int qa_gemm_w4a8(const QaGemmW4A8Params* p, void* stream_) {
     const bool addressable = static_cast<int64_t>(p->n) * (p->k / 2) < 0x70000000LL;
     const int64_t w8_bytes = static_cast<int64_t>(p->n) * p->k;
     const bool expandable = p->w8_workspace && p->w8_workspace_bytes >= w8_bytes && aligned16(p->w8_workspace) && w8_bytes < 0x70000000LL;
-    if (p->output_transpose ? p->m <= 64 && addressable : p->m <= kGemvRows && addressable) return dispatch_skinny(*p, stream);
+    const int cus = compute_units();
+    if (p->output_transpose ? p->m <= 64 && addressable : p->m <= kGemvRows && addressable) return dispatch_skinny(*p, cus, stream);
     if (!p->output_transpose) {
-        const int way = cheapest_way(*p, addressable, expandable);
-        if (way == kWaySkinny) return dispatch_skinny(*p, stream);
+        const int way = cheapest_way(*p, cus, addressable, expandable);
+        if (way == kWaySkinny) return dispatch_skinny(*p, cus, stream);
         if (way == kWay64x64) return p->out_type == QA_OUT_I8 ? launch_tile<QA_OUT_I8>(*p, stream) : launch_tile<QA_OUT_F16>(*p, stream);
         if (way == kWay64x128) return launch_reg<2, 4, 256>(*p, stream);
         if (way == kWay128x128) return launch_reg<4, 4, 128>(*p, stream);

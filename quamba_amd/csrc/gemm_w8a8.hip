@@ -392,11 +392,7 @@ int dispatch_skinny(const QaGemmW8A8Params& p, hipStream_t stream) {
 // while the other waits.  Four waves against eight (us): 1531 x 768 x 1536 6.9 -> 6.3, 1024 x 1536 x 3072 10.2 -> 9.8 with
 // 128 x 64; 3063 x 768 x 1536 9.2 -> 7.8, 1531 x 1536 x 3072 14.0 -> 12.1, 1531 x 2560 x 5120 28.0 -> 27.8 with 128 x 128.
 int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
-        cus = 256;
-    }
+    const int cus = compute_units();
     auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
     if (tiles(16, 16) <= cus) return launch_narrow(p, stream);                       // (two rounds of these: slower than one of 32 x 32)
     if (tiles(32, 32) <= cus) return dispatch_skinny<false>(p, stream);

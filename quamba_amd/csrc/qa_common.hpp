@@ -27,6 +27,13 @@ inline int check_launch() {
     return QA_OK;
 }
 
+// compute units of the current device (256 where there is none to ask)
+inline int compute_units() {
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
+    return cus;
+}
+
 // f(integral_constant<int, I>) for I = FIRST .. LAST-1: a loop whose index is a compile-time constant
 template <int FIRST, int LAST, typename F>
 __host__ __device__ __forceinline__ void static_for(F&& f) {

@@ -807,11 +807,7 @@ int choose_mapping16(const QaSScanParams& p) {
     // Waves per SIMD with four lanes per channel: q + f.  With 0 < f <= 1/2 the last f/(q+f) of the
     // channels of every batch entry go to the eight-lane kind (see sscan_fwd_mixed_kernel), as long as
     // both parts stay whole workgroups and, with channel groups, whole groups.
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
-        cus = 256;
-    }
+    const int cus = compute_units();
     const int64_t simds = 4LL * cus;
     const int64_t waves_a = static_cast<int64_t>(p.batch) * p.dim / 16;
     const int64_t q = waves_a / simds, rem_waves = waves_a % simds;

@@ -471,11 +471,7 @@ int step_cost(int lanes, bool out, int64_t waves) {
 
 TmPlan plan_of(const QaSScanParams& p) {
     TmPlan r = {4, 0, 1, p.seqlen};
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
-        cus = 256;
-    }
+    const int cus = compute_units();
     const int64_t simds = 4LL * cus, rows = static_cast<int64_t>(p.batch) * p.dim;
     const int64_t waves4 = rows / 16, q = waves4 / simds, rest = waves4 % simds;
     auto cut = [&](int segments) {
