@@ -10,7 +10,10 @@ shape (batch 8, seqlen 2048, d_model 2560, d_inner 5120, d_state 16, conv width 
 
 Inputs are resident in HBM before the timed region.  dt, B and C (produced by x_proj / dt_proj in
 the full layer) and out_proj's int8 input (produced by the Hadamard-quantise op) are synthetic
-tensors of the right shape and layout.  Prints one JSON line.
+tensors of the right shape and layout.  The step calls the four operators as the reference's layer does, with
+seqlen-last activations between them; the assembled layer (W8A8QMamba.forward, one library call with row-major
+activations and dt_proj inside its scan) runs other kernels for in_proj's output, the conv and the scan and is one of
+the workloads of --other-workloads.  Prints one JSON line.
 """
 import argparse
 import json
@@ -634,16 +637,26 @@ def valu_calibration(dev, ops_list=None, launches=4):
 # Vector instructions a wave of the selective scan issues per group of four steps, counted in the compiled kernel
 # (time loop + staging of the next tile + output store, divided by the eight groups of a 32-step tile): the kind with
 # four lanes per channel and four states per lane, and the short kind with eight lanes per channel and two states.
-# The counts belong to one state of the kernel source: `source_sha256` is the hash of quamba_amd/csrc/sscan.hip they
-# were counted at; when the file has changed since, the line says so (`stale`) instead of passing them off as current.
+# The counts belong to one state of the kernel sources (source_fingerprint); when those have changed since, the line says
+# so (`stale`) instead of passing them off as current.
 SCAN_MIX = {"four_lane": {"plain": 96, "transcendental": 18}, "eight_lane": {"plain": 57, "transcendental": 9}}
-SCAN_MIX_SOURCE_SHA256 = "e70cab8ddcf16e14fb332f9d44a854577bfdeee217b5a47359992baa1c18e961"
+SCAN_MIX_SOURCES = ("sscan.hip", "sscan_common.hpp")
+SCAN_MIX_FINGERPRINT = "1620c750a8173a42"
+
+
+def source_fingerprint(names, root=os.path.join(ROOT, "quamba_amd", "csrc")):
+    """What figures about a kernel's compiled code are tied to: its source files without comments and spacing."""
+    import hashlib
+    import re
+    h = hashlib.sha256()
+    for name in names:
+        text = open(os.path.join(root, name)).read()
+        h.update(re.sub(r"\s+", "", re.sub(r"//[^\n]*|/\*.*?\*/", "", text, flags=re.S)).encode())
+    return h.hexdigest()[:16]
 
 
 def scan_mix_is_stale():
-    import hashlib
-    path = os.path.join(ROOT, "quamba_amd", "csrc", "sscan.hip")
-    return hashlib.sha256(open(path, "rb").read()).hexdigest() != SCAN_MIX_SOURCE_SHA256
+    return source_fingerprint(SCAN_MIX_SOURCES) != SCAN_MIX_FINGERPRINT
 
 
 def peaks_measured(dev):
@@ -785,8 +798,9 @@ def scan_issue_bound(dev, B, D, L):
 
 def load_traffic(path):
     """HBM bytes per launch from the rocprofv3 counter runs summarised in profiles/hbm_traffic_counters.md: the file
-    names the git head it was measured at and, per entry, the kernels it sums.  An entry whose kernels no longer exist
-    in the library under those names is dropped (its figure would belong to other code)."""
+    names the git head it was measured at and, per entry, the kernels it sums and the fingerprint of their sources.  An
+    entry whose kernels no longer exist in the library under those names, or whose sources have changed, is dropped (its
+    figure would belong to other code)."""
     if not os.path.exists(path):
         return {}, None
     from quamba_amd import _lib
@@ -794,7 +808,7 @@ def load_traffic(path):
     image = open(_lib.LIB_PATH, "rb").read()
     out = {}
     for name, entry in doc.get("entries", {}).items():
-        if all(sym.encode() in image for sym in entry["kernel_symbols"]):
+        if all(sym.encode() in image for sym in entry["kernel_symbols"]) and entry.get("fingerprint") == source_fingerprint(entry.get("sources", ())):
             out[name] = entry["bytes"]
     return out, doc.get("head")
 
@@ -917,7 +931,7 @@ def main():
         # the bound that binds this kernel is vector-ALU issue, not HBM: how far the launch is from it
         ib = scan_issue_bound(dev, B, CFG["d_inner"], L)
         if ib["stale"]:
-            roofline["issue_bound_stale"] = "quamba_amd/csrc/sscan.hip has changed since the instruction mix was counted"
+            roofline["issue_bound_stale"] = f"{', '.join(SCAN_MIX_SOURCES)} changed since the instruction mix was counted"
         else:
             roofline["issue_bound_us"] = round(ib["issue_bound_us"], 2)
             roofline["frac_of_issue_bound"] = round(ib["issue_bound_us"] / dom["avg_us"], 4)
