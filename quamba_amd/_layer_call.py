@@ -8,6 +8,7 @@ sub-module classes or replaced methods, forward hooks, views with gaps, unusual 
 modules one by one.
 """
 import ctypes as C
+import functools
 import numbers
 
 import torch
@@ -43,16 +44,24 @@ def _need(cond):
         raise _Unsupported
 
 
+def _held(module):
+    """What a module holds, by name, as attribute access finds it (at a fraction of the time of some fifty of them)."""
+    d = module.__dict__
+    return {**d["_buffers"], **d["_parameters"], **d}
+
+
 def _ptr(t, dtype, numel, device, align=1):
     """Address of a dense tensor of `numel` elements on the layer's device (None stays None)."""
     if t is None:
         return None
-    _need(t.dtype == dtype and t.numel() == numel and t.device == device and t.is_contiguous())
+    if t.dtype is not dtype or t.numel() != numel or t.device != device or not t.is_contiguous():
+        raise _Unsupported
     try:
         a = t.data_ptr()
     except RuntimeError as e:                  # no memory of its own (under vmap, say)
         raise _Unsupported from e
-    _need(a % align == 0)
+    if a % align:
+        raise _Unsupported
     return a
 
 
@@ -65,27 +74,32 @@ def _number(v):
 
 def linear_block(lin, device):
     """QaLinearParams of one of the linear modules."""
-    p = _lib.QaLinearParams()
+    p, held = _lib.QaLinearParams(), _held(lin)
+    weight = held["weight"]
     if isinstance(lin, _W4A8Base):
-        n, k = lin.size_n, lin.size_k
+        n, k, s_group = lin.size_n, lin.size_k, held["s_group"]
         p.n, p.k, p.bits, p.col_numel = n, k, 4, n
-        p.weight = _ptr(lin.weight, torch.uint8, n * (k // 2), device, 16)
-        p.s_group = _ptr(lin.s_group, torch.float16, (k // 128) * n, device) if lin.s_group.numel() else None
-        p.col_scale = _ptr(lin.s_channel, torch.float32, n, device)
-        p.row_scale = _ptr(lin.input_scale, torch.float32, 1, device)
+        p.weight = _ptr(weight, torch.uint8, n * (k // 2), device, 16)
+        p.s_group = _ptr(s_group, torch.float16, (k // 128) * n, device) if s_group.numel() else None
+        p.col_scale = _ptr(held["s_channel"], torch.float32, n, device)
+        p.row_scale = _ptr(held["input_scale"], torch.float32, 1, device)
         _need(k % 128 == 0)
     else:
-        n, k = lin.out_features + lin.pad_out, lin.in_features
-        p.n, p.k, p.bits, p.col_numel = n, k, 8, lin.b.numel()
-        _need(tuple(lin.weight.shape) == (k, n) and p.col_numel in (1, n))
-        p.weight = _ptr(lin.weight.t(), torch.int8, n * k, device, 16)
-        p.col_scale = _ptr(lin.b, torch.float32, lin.b.numel(), device)
-        p.row_scale = _ptr(lin.a, torch.float32, 1, device)
+        n, k, b = lin.out_features + lin.pad_out, lin.in_features, held["b"]
+        cols = b.numel()
+        p.n, p.k, p.bits, p.col_numel = n, k, 8, cols
+        _need(weight.shape == (k, n) and cols in (1, n))
+        p.weight = _ptr(weight.t(), torch.int8, n * k, device, 16)
+        p.col_scale = _ptr(b, torch.float32, cols, device)
+        p.row_scale = _ptr(held["a"], torch.float32, 1, device)
         if isinstance(lin, _AlphaHooks):
             p.row_rule, p.alpha = _lib.QA_ROW_ALPHA, _number(lin.alpha)
         else:
             p.row_rule = _lib.QA_ROW_HALF_AWAY
     return p
+
+
+_ENTRIES = {}          # family -> addresses of its entry points in the loaded library
 
 
 def _native(mixer):
@@ -95,9 +109,10 @@ def _native(mixer):
     block, dims = mixer._native_block(device)
     lib = _lib.lib()
     family = 1 if type(block) is _lib.QaMamba1Params else 2
-    fns = tuple(C.cast(getattr(lib, f"qa_mamba{family}{s}"), C.c_void_p).value for s in ("_forward", "_step", "_workspace_bytes"))
+    if family not in _ENTRIES:
+        _ENTRIES[family] = tuple(C.cast(getattr(lib, f"qa_mamba{family}{s}"), C.c_void_p).value for s in ("_forward", "_step", "_workspace_bytes"))
     runtime = (torch.cuda.current_device, torch.cuda.set_device, torch._C._cuda_getCurrentRawStream, torch.cuda.OutOfMemoryError)
-    return family, bytes(block), fns, dims, mixer.out_proj.pad_out, mixer.out_proj.weight, runtime
+    return family, bytes(block), _ENTRIES[family], dims, mixer.out_proj.pad_out, mixer.out_proj.weight, runtime
 
 
 # The classes whose methods the library call stands for, as they were when this package was imported: what each of them
@@ -118,8 +133,10 @@ def _code_of(held):
     return {n: f for n, f in held.items() if callable(f) or isinstance(f, (classmethod, staticmethod, property))}
 
 
-def _classes_of(modules):
-    return list({c: None for m in modules for c in type(m).__mro__ if c in _HELD})
+@functools.lru_cache(maxsize=64)
+def _classes_of(types):
+    """The remembered classes among these and their bases."""
+    return tuple({c: None for t in types for c in t.__mro__ if c in _HELD})
 
 
 def _own_code(modules, classes):
@@ -140,7 +157,7 @@ def _make(mixer):
         held = m.__dict__
         watched += [held, held["_buffers"], held["_parameters"]]
         hooks += [held["_forward_hooks"], held["_forward_pre_hooks"]]
-    classes = _classes_of(mods)
+    classes = _classes_of(tuple(map(type, mods)))
     watched += classes
     try:
         _need(mixer._native_modules() is not None and _own_code(mods, classes))

@@ -18,7 +18,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _layer_call, _lib, ops
-from ._layer_call import _need, _number, _ptr, linear_block
+from ._layer_call import _held, _need, _number, _ptr, linear_block
 from .chunk_scan import Quamba2ChunkScan
 from .conv import QCausalConv1D, Quamb2Conv1D
 from .hadamard import QHadamard
@@ -101,23 +101,23 @@ class W8A8QMamba(nn.Module):
 
     def _native_block(self, dev):
         p, D, N = _lib.QaMamba1Params(), self.d_inner, self.d_state
-        c, s = self.conv1d, self.selective_scan
+        c, s, had = self.conv1d, _held(self.selective_scan), self.had
         p.d_model, p.d_inner, p.d_state, p.d_conv, p.dt_rank = self.d_model, D, N, self.d_conv, self.dt_rank
         p.conv_state_len = self.d_conv
-        p.delta_softplus = int(bool(_number(s.delta_softplus)))
+        p.delta_softplus = int(bool(_number(s["delta_softplus"])))
         for name in ("in_proj", "x_proj", "dt_proj", "out_proj"):
             setattr(p, name, linear_block(getattr(self, name), dev))
         p.conv_weight, p.conv_bias = _ptr(c.weight, torch.int8, D * self.d_conv, dev), _ptr(c.bias, torch.int8, D, dev)
         p.conv_scale_x, p.conv_scale_w, p.conv_scale_b, p.conv_scale_out = (
             _number(v) for v in (c.input_scale, c.weight_scale, c.bias_scale, c.output_scale))
-        p.A_log = _ptr(s.A_log, torch.int8, D * N, dev)
-        p.D, p.dt_bias = _ptr(s.D, torch.int8, D, dev), _ptr(s.dt_bias, torch.int8, D, dev)
+        p.A_log = _ptr(s["A_log"], torch.int8, D * N, dev)
+        p.D, p.dt_bias = _ptr(s["D"], torch.int8, D, dev), _ptr(s["dt_bias"], torch.int8, D, dev)
         for name in ("A_scale", "D_scale", "dt_bias_scale", "u_scale", "dt_scale", "B_scale", "C_scale", "z_scale", "ssm_state_scale"):
-            setattr(p, name, _ptr(getattr(s, name), torch.float32, 1, dev))
+            setattr(p, name, _ptr(s[name], torch.float32, 1, dev))
         _need(all((p.conv_weight, p.A_log, p.A_scale, p.u_scale, p.dt_scale, p.B_scale, p.C_scale, p.z_scale, p.ssm_state_scale)))
         _need((p.D_scale or not p.D) and (p.dt_bias_scale or not p.dt_bias))
-        _need(self.had.transform_fn is ops.hadamard_quant)
-        p.had_scale = _number(self.had.had_scale) / float(_number(self.had.x_H_scale))
+        _need(had.transform_fn is ops.hadamard_quant)
+        p.had_scale = _number(had.had_scale) / float(_number(had.x_H_scale))
         widths = (self.d_conv, self.d_conv - 1)                        # of the conv state, in forward and in step
         return p, (D, (D, N), (widths, widths))
 

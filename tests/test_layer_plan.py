@@ -205,7 +205,7 @@ def test_the_current_device_comes_back_however_the_call_ends():
 
 
 def _own_code(*modules):
-    return _layer_call._own_code(modules, _layer_call._classes_of(modules))
+    return _layer_call._own_code(modules, _layer_call._classes_of(tuple(map(type, modules))))
 
 
 def _public(module):
