@@ -150,7 +150,9 @@ def _own_code(modules, classes):
 
 def _make(mixer):
     """The mixer's plan (one that only ever yields None where the library does not cover the mixer)."""
-    mods = [m for m in mixer._modules.values() if m is not None]
+    mods = mixer._native_modules()
+    if mods is None:                           # (whatever stands there need not be held together like an ordinary module)
+        return _plan_class()((mixer._modules,), (), None)
     watched = [mixer._modules]
     hooks = [getattr(_module, k) for k in ("_global_forward_hooks", "_global_forward_pre_hooks")]
     for m in mods:
@@ -160,7 +162,7 @@ def _make(mixer):
     classes = _classes_of(tuple(map(type, mods)))
     watched += classes
     try:
-        _need(mixer._native_modules() is not None and _own_code(mods, classes))
+        _need(_own_code(mods, classes))
         native = _native(mixer)
     except _Unsupported:
         native = None

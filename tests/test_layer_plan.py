@@ -79,6 +79,26 @@ def test_replaced_modules_numbers_and_memory_are_seen(cls):
     assert not _unchanged(plan)
 
 
+def test_other_modules_in_the_mixer():
+    """In the place of one of its own: the modules run, whatever it is made of.  Beside them: nothing to the call."""
+    m = _mixer(W8A8QMamba)
+    stock = m.had
+    m.had = torch.jit.script(nn.Identity())                  # (keeps no dicts of buffers and parameters)
+    plan = _layer_call._make(m)
+    assert _unchanged(plan) and m._native_modules() is None
+    m.had = stock
+    assert not _unchanged(plan)
+    m.observer = nn.Linear(1, 1)
+    m.observer.forward = lambda x: x
+    native = []
+    kept, _layer_call._native = _layer_call._native, lambda mixer: native.append(mixer)
+    try:
+        _layer_call._make(m)
+    finally:
+        _layer_call._native = kept
+    assert native == [m]
+
+
 def test_a_plan_does_not_keep_its_mixer():
     m = _mixer(W8A8QMamba)
     m.__dict__["_plan"] = _layer_call._make(m)
