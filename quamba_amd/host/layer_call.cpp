@@ -236,6 +236,9 @@ PyObject* enqueue(State& s, Params p, const at::Tensor& hidden, PyObject* conv_o
         const at::Tensor& c = THPVariable_Unpack(conv_o);
         if (c.scalar_type() != at::kChar || c.device() != s.device || c.dim() != 3 || c.size(0) != batch || c.size(1) != s.conv_dim ||
             (c.size(2) != s.widths[step][0] && c.size(2) != s.widths[step][1])) Py_RETURN_NONE;
+        // (rows that lie on each other: the modules' copy refuses them)
+        for (int i = 0; i < 3; ++i)
+            if (c.stride(i) == 0 && c.size(i) > 1) Py_RETURN_NONE;
         p.conv_state = c.data_ptr<int8_t>();
         p.conv_state_len = static_cast<int32_t>(c.size(2));
         p.conv_state_batch_stride = c.stride(0); p.conv_state_c_stride = c.stride(1); p.conv_state_l_stride = c.stride(2);

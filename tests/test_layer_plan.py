@@ -204,6 +204,20 @@ def test_hidden_states_the_products_cannot_read_go_to_the_modules():
     assert torch.is_tensor(r.plan.run(room[start:][:256].view(1, 1, 256), None, None, False))
 
 
+def test_states_the_call_does_not_write():
+    r = _Runtime()
+    conv, ssm = torch.zeros(1, 512, 4, dtype=torch.int8), torch.zeros(1, 512, 16)
+    assert torch.is_tensor(r.plan.run(HIDDEN, conv, ssm, False)) and r.blocks[-1].state_is_fp32 == 1 and r.blocks[-1].conv_state == conv.data_ptr()
+    assert torch.is_tensor(r.plan.run(HIDDEN, conv[..., 1:], ssm.to(torch.int8), True)) and r.blocks[-1].conv_state_len == 3
+    room = torch.zeros(512 * 16 + 4)
+    off = room[(-room.data_ptr() // 4) % 4 + 1:][:512 * 16].view(1, 512, 16)
+    for c, s in ((conv[:, :1].expand(1, 512, 4), ssm), (conv[:, :511], ssm), (conv.float(), ssm), (conv.expand(2, 512, 4), ssm), (conv[..., :2], ssm),
+                 (conv, ssm.half()), (conv, ssm.transpose(1, 2).contiguous().transpose(1, 2)), (conv, ssm[:, :511]), (conv, off)):
+        for step in (False, True):
+            assert r.plan.run(HIDDEN, c, s, step) is None
+    assert len(r.calls) == 2
+
+
 def test_the_current_device_comes_back_however_the_call_ends():
     here = -1                                                # (the index of a device without one)
     r = _Runtime()
