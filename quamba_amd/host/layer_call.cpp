@@ -5,10 +5,11 @@
 // layer (qa_mamba1_* / qa_mamba2_*, include/quamba_amd.h) together with what it was made from, and run() verifies all of it,
 // allocates output and workspace, and enqueues the layer.
 //
-// What it was made from is a list of dicts - the mixer's sub-modules, of each of them its attributes, buffers and
-// parameters, and their classes (another function in the place of a method is another layer) - as they were, entry by entry: a tensor whose address is in the block is in one of them wherever the module
+// What it was made from is a list of dicts - the mixer's sub-modules, and of each of them its attributes, buffers and
+// parameters - as they were, entry by entry: a tensor whose address is in the block is in one of them wherever the module
 // keeps it, the entry keeps it alive, and every call compares the entries with what the dicts hold now (values by identity,
-// numbers by value, tensors by their address as well).
+// numbers by value, tensors by their address as well).  The modules' classes belong to it too: another function in the place
+// of a method is another layer.
 //
 // run(hidden, conv_state, ssm_state, step) returns the output tensor; None when the library call does not cover these
 // arguments (the mixer then runs its modules one by one); False when the layer is not the one the plan was made from any
@@ -37,6 +38,7 @@ struct Entry {
 struct Watch {
     PyObject* dict;
     uint64_t version;
+    bool entire;                   // held entry by entry (a class is not, where its dict has a version)
     std::vector<Entry> entries;
 };
 
@@ -121,7 +123,8 @@ int make_plan(PlanObject* self, PyObject* args) {
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(watched); ++i) {
         PyObject* from = PyTuple_GET_ITEM(watched, i);
         PyObject* dict = keep(PyType_Check(from) ? reinterpret_cast<PyTypeObject*>(from)->tp_dict : from);
-        s->watches.push_back({dict, version_of(dict), {}});
+        s->watches.push_back({dict, version_of(dict), dict == from || version_of(dict) == 0, {}});
+        if (!s->watches.back().entire) continue;
         s->watches.back().entries.reserve(PyDict_GET_SIZE(dict));
         PyObject *key, *value;
         Py_ssize_t pos = 0;
@@ -204,6 +207,7 @@ bool same_value(PyObject* a, PyObject* b) {
 bool same_entries(Watch& w) {
     const uint64_t version = version_of(w.dict);
     if (version && version == w.version) return true;
+    if (!w.entire) return false;
     if (PyDict_GET_SIZE(w.dict) != static_cast<Py_ssize_t>(w.entries.size())) return false;
     PyObject *key, *value;
     Py_ssize_t pos = 0;
@@ -372,8 +376,19 @@ PyMethodDef plan_methods[] = {
     {"__reduce__", plan_reduce, METH_NOARGS, "Pickles as None."},
     {nullptr, nullptr, 0, nullptr}};
 
+// class_version(cls): the version of a class's own dict (0: none)
+PyObject* class_version(PyObject*, PyObject* cls) {
+    if (!PyType_Check(cls)) {
+        PyErr_SetString(PyExc_TypeError, "class_version(cls)");
+        return nullptr;
+    }
+    return PyLong_FromUnsignedLongLong(version_of(reinterpret_cast<PyTypeObject*>(cls)->tp_dict));
+}
+
+PyMethodDef module_methods[] = {{"class_version", class_version, METH_O, "Version of a class's own dict."}, {nullptr, nullptr, 0, nullptr}};
+
 PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
-PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Host side of the mixers' library calls.", -1, nullptr};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Host side of the mixers' library calls.", -1, module_methods};
 
 }  // namespace
 

@@ -104,16 +104,16 @@ class W8A8QMamba(nn.Module):
         c, s, had = self.conv1d, _held(self.selective_scan), self.had
         p.d_model, p.d_inner, p.d_state, p.d_conv, p.dt_rank = self.d_model, D, N, self.d_conv, self.dt_rank
         p.conv_state_len = self.d_conv
-        p.delta_softplus = int(bool(_number(s["delta_softplus"])))
+        p.delta_softplus = int(bool(_number(s("delta_softplus"))))
         for name in ("in_proj", "x_proj", "dt_proj", "out_proj"):
             setattr(p, name, linear_block(getattr(self, name), dev))
         p.conv_weight, p.conv_bias = _ptr(c.weight, torch.int8, D * self.d_conv, dev), _ptr(c.bias, torch.int8, D, dev)
         p.conv_scale_x, p.conv_scale_w, p.conv_scale_b, p.conv_scale_out = (
             _number(v) for v in (c.input_scale, c.weight_scale, c.bias_scale, c.output_scale))
-        p.A_log = _ptr(s["A_log"], torch.int8, D * N, dev)
-        p.D, p.dt_bias = _ptr(s["D"], torch.int8, D, dev), _ptr(s["dt_bias"], torch.int8, D, dev)
+        p.A_log = _ptr(s("A_log"), torch.int8, D * N, dev)
+        p.D, p.dt_bias = _ptr(s("D"), torch.int8, D, dev), _ptr(s("dt_bias"), torch.int8, D, dev)
         for name in ("A_scale", "D_scale", "dt_bias_scale", "u_scale", "dt_scale", "B_scale", "C_scale", "z_scale", "ssm_state_scale"):
-            setattr(p, name, _ptr(s[name], torch.float32, 1, dev))
+            setattr(p, name, _ptr(s(name), torch.float32, 1, dev))
         _need(all((p.conv_weight, p.A_log, p.A_scale, p.u_scale, p.dt_scale, p.B_scale, p.C_scale, p.z_scale, p.ssm_state_scale)))
         _need((p.D_scale or not p.D) and (p.dt_bias_scale or not p.dt_bias))
         _need(had.transform_fn is ops.hadamard_quant)
