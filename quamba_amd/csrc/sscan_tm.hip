@@ -6,7 +6,8 @@
 // and C are converted once per workgroup; the time loop is the recurrence alone.  What differs:
 //
 // Bound by vector issue: at 8 x 2048 steps x 5120 channels the recurrence is 16 exponentials (a quarter of the rate) and 64
-// multiplies and adds per channel and step, 384 us of which about 300 are issue; the bytes would take 60.
+// multiplies and adds per channel and step, 391 us of which about 300 are issue; the bytes would take 60.  With B x (step size
+// x input) as matrix instructions and the sums over lanes by swaps 377 (16 x 512 x 5120, four lanes for all, 176 -> 168).
 //
 // Staging.  A wave stages its own channels with dword loads of four channels and one step.  Tails need no path of their
 // own: steps past the end read the last step and get step size zero.
@@ -37,6 +38,7 @@ namespace {
 
 constexpr int kThreads = 256;
 using gemm::v4i;
+typedef float v16f __attribute__((ext_vector_type(16)));
 
 template <int NSPLIT>
 struct TmCfg {
@@ -66,13 +68,18 @@ struct TmSmem {
     float gate_table[256];             // SiLU gate per z code (indexed by the raw byte)
 };
 
-// DTK: 64-code pieces of dt_proj's K (0: the step size codes are read from p.delta)
-template <int NSPLIT, bool HAS_Z, bool OUT, int DTK>
+// DTK: 64-code pieces of dt_proj's K (0: the step size codes are read from p.delta).  SPREAD: a channel's lanes are 16 apart
+// (and 8, when there are eight), not neighbours.
+template <int NSPLIT, bool HAS_Z, bool OUT, int DTK, bool SPREAD>
 __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const SscanDtProj& dtp, int vec_out, int c0, int y, TmSmem<TmCfg<NSPLIT>, DTK>& sm) {
     using Cfg = TmCfg<NSPLIT>;
     constexpr int T = Cfg::T, NPL = Cfg::NPL, kCh = Cfg::kCh, kSteps = Cfg::kSteps;
+    constexpr bool kOuter = NSPLIT == 4;                   // B x (step size x input) on the matrix cores
+    static_assert(SPREAD ? NSPLIT <= 8 : !kOuter, "lanes as 16 x 16 products leave them");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int c_local = tid / NSPLIT, slice = tid % NSPLIT, qslice = slice & 3;
+    constexpr int kWaveCh = Cfg::kWaveCh;
+    const int c_local = SPREAD ? wave * kWaveCh + lane % kWaveCh : tid / NSPLIT;
+    const int slice = SPREAD ? (lane & 15) / kWaveCh * 4 + (lane >> 4) : tid % NSPLIT, qslice = slice & 3;
     const int c = c0 + c_local;
     const bool c_ok = c < p.dim;
     const int cc = c_ok ? c : p.dim - 1;                   // clamped channel for parameter loads
@@ -283,19 +290,39 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
 
     // operands of one group of four steps
     struct Group {
-        float d[4], du[4], B[NPL][4];
+        float d[4], du[kOuter ? 1 : 4], B[kOuter ? 1 : NPL][kOuter ? 1 : 4];
+        v16f bdu;                       // with kOuter B x du instead, step s and state n of this lane in 4 s + n
         uint32_t code;                  // of the step this lane owns: u in byte 0, z in byte 1
+    };
+    // Four lanes per channel: these products on the matrix cores.  A 16 x 16 x 1 instruction of four blocks, a block per step,
+    // multiplies the B of sixteen states (rows) with the du of sixteen channels (columns) and leaves four rows of a column - a
+    // lane's states and channel - in each lane, rounded as the sixteen multiplications it stands for; a group's are made
+    // during the group before.  The instruction keeps the vector units from about eight of their own (16 x 512 steps x 5120
+    // channels 162 -> 157 us, 8 x 2048 x 4096 274 -> 263); with eight lanes per channel, where a group takes two of them for
+    // eight multiplications, it loses (4 x 2048 x 5120 225 -> 256).
+    struct Factors {                    // B of state j, du of this channel, both of step g
+        float b, du;
+    };
+    auto fetch_factors = [&](Factors& o, int tq, int from) {
+        o.b = sm.bc[from][tq][0][j][g];
+        o.du = sm.du[c_local][tq * 4 + g];
+    };
+    auto multiply = [&](Group& o, const Factors& x) {
+        constexpr v16f zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        o.bdu = __builtin_amdgcn_mfma_f32_16x16x1f32(x.b, x.du, zero, 0, 0, 0);
     };
     auto fetch = [&](Group& o, int tq, int from) {
         if constexpr (OUT) o.code = sm.uz[c_local][tq * 4 + qslice];
         const float4 d4 = *reinterpret_cast<const float4*>(&sm.d[c_local][tq * 4]);
-        const float4 du4 = *reinterpret_cast<const float4*>(&sm.du[c_local][tq * 4]);
         o.d[0] = d4.x; o.d[1] = d4.y; o.d[2] = d4.z; o.d[3] = d4.w;
-        o.du[0] = du4.x; o.du[1] = du4.y; o.du[2] = du4.z; o.du[3] = du4.w;
+        if constexpr (!kOuter) {
+            const float4 du4 = *reinterpret_cast<const float4*>(&sm.du[c_local][tq * 4]);
+            o.du[0] = du4.x; o.du[1] = du4.y; o.du[2] = du4.z; o.du[3] = du4.w;
 #pragma unroll
-        for (int n = 0; n < NPL; ++n) {
-            const float4 Bv = *reinterpret_cast<const float4*>(sm.bc[from][tq][0][slice * NPL + n]);
-            o.B[n][0] = Bv.x; o.B[n][1] = Bv.y; o.B[n][2] = Bv.z; o.B[n][3] = Bv.w;
+            for (int n = 0; n < NPL; ++n) {
+                const float4 Bv = *reinterpret_cast<const float4*>(sm.bc[from][tq][0][slice * NPL + n]);
+                o.B[n][0] = Bv.x; o.B[n][1] = Bv.y; o.B[n][2] = Bv.z; o.B[n][3] = Bv.w;
+            }
         }
     };
     // the column of the output tile a lane writes: with more than four lanes per channel only the first quad's sums are
@@ -308,7 +335,13 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
     auto compute = [&](int from) {
         __half* const out_at = &sm.out[from][qslice][out_col];
         Group grp[2];
+        Factors fac[2];
         fetch(grp[0], 0, from);
+        if constexpr (kOuter) {
+            fetch_factors(fac[0], 0, from);
+            fetch_factors(fac[1], 1, from);
+            multiply(grp[0], fac[0]);
+        }
 #pragma unroll
         for (int tq = 0; tq < T / 4; ++tq) {
             Group& o = grp[tq & 1];
@@ -324,6 +357,10 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
                 if constexpr (HAS_Z) gate = sm.gate_table[o.code >> 8];
             }
             if (tq + 1 < T / 4) fetch(grp[(tq + 1) & 1], tq + 1, from);
+            if constexpr (kOuter) {
+                if (tq + 2 < T / 4) fetch_factors(fac[tq & 1], tq + 2, from);
+                if (tq + 1 < T / 4) multiply(grp[(tq + 1) & 1], fac[(tq + 1) & 1]);
+            }
             // keep the reads above ahead of this group's arithmetic (the scheduler would sink them to their first use, and a
             // wave would then wait for LDS once or twice per group)
             __builtin_amdgcn_sched_barrier(0);
@@ -334,7 +371,8 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
 #pragma unroll
                 for (int n = 0; n < NPL; ++n) {
                     const float a = fast_exp2(o.d[s] * A2[n]);
-                    h[n] = __builtin_fmaf(a, h[n], o.B[n][s] * o.du[s]);
+                    if constexpr (kOuter) h[n] = __builtin_fmaf(a, h[n], o.bdu[4 * s + n]);
+                    else h[n] = __builtin_fmaf(a, h[n], o.B[n][s] * o.du[s]);
                     if constexpr (OUT) acc[s] = n == 0 ? h[n] * C[n][s] : __builtin_fmaf(h[n], C[n][s], acc[s]);
                 }
             }
@@ -343,15 +381,30 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
                 for (int n = 0; n < NPL; ++n) asm volatile("" : "+v"(h[n]));      // (no output holds a group's arithmetic in its place)
                 continue;
             }
-            // each lane of a quad completes the step it owns: a transposing reduction (keep one half, hand the other half to
-            // the neighbour) instead of four full ones; the sums of a channel's other quads arrive by row shifts inside the
-            // additions
-            const bool odd = qslice & 1, hi = qslice & 2;
-            const float w01 = (odd ? acc[1] : acc[0]) + quad_xor<1>(odd ? acc[0] : acc[1]);
-            const float w23 = (odd ? acc[3] : acc[2]) + quad_xor<1>(odd ? acc[2] : acc[3]);
-            float own_sum = (hi ? w23 : w01) + quad_xor<2>(hi ? w01 : w23);
-            if constexpr (NSPLIT >= 8) own_sum += row_from_up<4>(own_sum);
-            if constexpr (NSPLIT == 16) own_sum += row_from_up<8>(own_sum);
+            // each of four lanes completes the step it owns: a transposing reduction (keep one half, hand the other half over)
+            // instead of four full ones.  Lanes 32 and 16 apart exchange halves with one swap for two values; neighbours, which
+            // select what they keep and what they hand over, take half as many instructions again (four lanes 278 -> 274 us at
+            // 8 x 2048 x 4096; both kinds of workgroup at 8 x 2048 x 5120 359 -> 351; eight lanes in a launch of their own, whose
+            // waves wait for more than instructions, 3 x 1021 x 5120 100 -> 99 and short segments 13.0 -> 13.5: left as
+            // neighbours).  The sums of a channel's other quads arrive by row shifts inside the additions.
+            float own_sum;
+            if constexpr (SPREAD) {
+                const auto fold32 = [](float a, float b) {
+                    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+                    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+                };
+                const float w02 = fold32(acc[0], acc[2]), w13 = fold32(acc[1], acc[3]);
+                const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(w02), __float_as_uint(w13), false, false);
+                own_sum = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+                if constexpr (NSPLIT == 8) own_sum += row_from_up<8>(own_sum);
+            } else {
+                const bool odd = qslice & 1, hi = qslice & 2;
+                const float w01 = (odd ? acc[1] : acc[0]) + quad_xor<1>(odd ? acc[0] : acc[1]);
+                const float w23 = (odd ? acc[3] : acc[2]) + quad_xor<1>(odd ? acc[2] : acc[3]);
+                own_sum = (hi ? w23 : w01) + quad_xor<2>(hi ? w01 : w23);
+                own_sum += row_from_up<4>(own_sum);
+                if constexpr (NSPLIT == 16) own_sum += row_from_up<8>(own_sum);
+            }
             float out_v = own_sum + D_u * code_byte_to_float(o.code, 0);
             if constexpr (HAS_Z) out_v *= gate;
             out_at[tq * 4 * Cfg::kOutPitch] = __float2half(out_v);
@@ -438,7 +491,7 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
 template <int NSPLIT, bool HAS_Z, bool OUT, int DTK>
 __global__ __launch_bounds__(kThreads, 3) void scan_tm_kernel(QaSScanParams p, SscanDtProj dtp, int vec_out) {
     __shared__ TmSmem<TmCfg<NSPLIT>, DTK> sm;
-    scan_tm_body<NSPLIT, HAS_Z, OUT, DTK>(p, dtp, vec_out, blockIdx.x * TmCfg<NSPLIT>::kCh, blockIdx.y, sm);
+    scan_tm_body<NSPLIT, HAS_Z, OUT, DTK, NSPLIT == 4>(p, dtp, vec_out, blockIdx.x * TmCfg<NSPLIT>::kCh, blockIdx.y, sm);
 }
 
 // Two kinds of workgroup in one launch: the first `blocks_a` of a batch entry take 64 channels each with four lanes per
@@ -451,8 +504,8 @@ __global__ __launch_bounds__(kThreads, 3) void scan_tm_mixed_kernel(QaSScanParam
         __device__ Smem() {}
     } sm;
     const int bx = blockIdx.x;
-    if (bx < blocks_a) scan_tm_body<4, HAS_Z, true, DTK>(p, dtp, vec_out, bx * 64, blockIdx.y, sm.a);
-    else scan_tm_body<8, HAS_Z, true, DTK>(p, dtp, vec_out, blocks_a * 64 + (bx - blocks_a) * 32, blockIdx.y, sm.b);
+    if (bx < blocks_a) scan_tm_body<4, HAS_Z, true, DTK, true>(p, dtp, vec_out, bx * 64, blockIdx.y, sm.a);
+    else scan_tm_body<8, HAS_Z, true, DTK, true>(p, dtp, vec_out, blocks_a * 64 + (bx - blocks_a) * 32, blockIdx.y, sm.b);
 }
 
 // How a launch is laid out: lanes per channel (0: two kinds of workgroup, `blocks_a` of the first) and segments.
