@@ -505,18 +505,18 @@ constexpr int epilogue_lds_bytes() {
 template <int TM, int WAVES>
 constexpr int skinny_lds_bytes() { return WAVES * (1 + TM) * 32 * kBK + TM * 16 * 64 * 4; }
 
-// Tile of workgroup `linear`, row blocks of 32 TM by column blocks of 32.  With many column blocks the row blocks of one of
+// Tile of workgroup `linear`, row blocks of BM by column blocks of BN.  With many column blocks the row blocks of one of
 // them go to one XCD (eight workgroups apart), whose L2 then holds their weights.
-template <int TM>
-__device__ __forceinline__ void skinny_tile_of_workgroup(int linear, int m, int n, int& m0, int& n0) {
-    const int blocks_m = (m + 32 * TM - 1) / (32 * TM), blocks_n = (n + 31) / 32, whole = blocks_n / 8 * 8 * blocks_m;
+template <int BM, int BN = BM>
+__device__ __forceinline__ void split_tile_of_workgroup(int linear, int m, int n, int& m0, int& n0) {
+    const int blocks_m = (m + BM - 1) / BM, blocks_n = (n + BN - 1) / BN, whole = blocks_n / 8 * 8 * blocks_m;
     if (linear < whole) {
-        n0 = ((linear / (8 * blocks_m)) * 8 + linear % 8) * 32;
-        m0 = (linear / 8) % blocks_m * (32 * TM);
+        n0 = ((linear / (8 * blocks_m)) * 8 + linear % 8) * BN;
+        m0 = (linear / 8) % blocks_m * BM;
     } else {
         const int rest = linear - whole, columns = blocks_n % 8;
-        n0 = (blocks_n / 8 * 8 + rest % columns) * 32;
-        m0 = rest / columns * (32 * TM);
+        n0 = (blocks_n / 8 * 8 + rest % columns) * BN;
+        m0 = rest / columns * BM;
     }
 }
 

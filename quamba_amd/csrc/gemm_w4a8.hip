@@ -370,7 +370,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_w4a8_skinny_kernel(QaGemmW4A8
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int frow = lane & 31, fhalf = lane >> 5;
     int m0, n0;
-    skinny_tile_of_workgroup<TM>(blockIdx.x, p.m, p.n, m0, n0);
+    split_tile_of_workgroup<32 * TM, 32>(blockIdx.x, p.m, p.n, m0, n0);
     const bool grouped = p.group_size > 0;
     for (int i = tid; i < TM * 16 * 64; i += kThreads) red[i] = 0;
     uint8_t* stage = lds + wave * ((2 + TM) * kTile);          // two weight halves, TM activation tiles

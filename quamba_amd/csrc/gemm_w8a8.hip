@@ -186,204 +186,144 @@ int launch_gemm(const QaGemmW8A8Params& p, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Few activation rows (M <= 64, the decode step): the product is a stream over the weight matrix
-// and HBM-bound, so the shape of the launch is chosen for memory parallelism rather than reuse.
-// A workgroup owns 32 output columns and all rows; its WAVES waves split K between them in
-// interleaved 128-byte tiles.  A wave fetches its tiles with eight lanes per 128-byte row piece
-// (whole cache lines; fetching MFMA fragments directly would touch 64 lines per instruction),
-// DEPTH tiles in flight in registers, and turns a tile into fragments through a staging area in
-// LDS that is private to the wave, so the main loop has no workgroup barrier.  The small
-// activation matrix takes the same route and is served by the caches.  The partial sums of the
-// waves are added in LDS (integers: the order does not matter), then every thread scales and
-// writes four consecutive columns of one row.
+// Products of few outputs (the projections of a decode batch or a short prompt): B x B outputs per workgroup, K over its
+// waves, 128 bytes of every row at a time.
+// What bounds them is how fast a CU fetches its operand rows and the trips to memory that wait for each other.  A wave
+// fetches with eight lanes per 128-byte row piece straight to its own part of LDS - eight lines per instruction; the
+// fragments of 16x16x64 fetched into registers directly touch sixteen rows with consecutive lanes, which a CU takes at about
+// 16 bytes a clock - up to DEPTH units ahead; the scales are requested in front of everything else; the waves meet only for
+// their partial sums, which take the fetched units' place in LDS.
+// Eight waves: sixteen are as fast, but need more than the 64 KB that a launch gets by default and that two workgroups of a CU
+// can have.
+// Before, 16 x 16 with fragments fetched into registers by sixteen waves and 32 x 32 staged through registers by four (rows x
+// outputs x K, us): 64 x 192 x 5120 6.7 -> 3.8, 16 x 2560 x 5120 6.9 -> 4.9, 512 x 128 x 3072 4.8 -> 3.6, 64 x 80 x 1536 3.4 -> 3.4
+// (which is a launch); 64 x 2560 x 5120 7.8 -> 6.7, 100 x 1024 x 2048 5.2 -> 3.9, 40 x 3352 x 768 4.0 -> 3.5.  In 64 x 64 outputs a
+// wave's share of K is too little: 64 x 10240 x 2560 7.2 -> 9.7, and the tile kernel above stays.
 // ---------------------------------------------------------------------------------------------
-template <int TM, int WAVES, int DEPTH, int OUT, bool FLEX>
-__global__ __launch_bounds__(64 * WAVES) void gemm_w8a8_skinny_kernel(QaGemmW8A8Params p) {
-    constexpr int kThreads = 64 * WAVES;
-    constexpr int kOob = 0x7ffffff0;                       // beyond any buffer: the load returns zeros
-    constexpr int kTile = 32 * kBK;                        // one staged 32-row tile
+template <int B, int WAVES, int DEPTH>
+struct SplitCfg {
+    static constexpr int kThreads = 64 * WAVES, kBlocks = B / 16;
+    static constexpr int kRequests = B / 8;                        // per operand and unit
+    static constexpr int kUnit = 2 * B * kBK;                      // a rows, then w rows
+    static constexpr int kOutputs = (B * B + kThreads - 1) / kThreads;         // per thread
+    static constexpr int kRing = WAVES * DEPTH * kUnit, kSums = WAVES * B * B * 4;
+    static constexpr int kLdsBytes = kRing > kSums ? kRing : kSums;
+};
+
+template <int B, int WAVES, int DEPTH, int OUT>
+__global__ __launch_bounds__(64 * WAVES) void gemm_w8a8_split_kernel(QaGemmW8A8Params p) {
+    using C = SplitCfg<B, WAVES, DEPTH>;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    int* red = reinterpret_cast<int*>(lds + WAVES * (1 + TM) * kTile);   // [row block][acc register][lane]
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int frow = lane & 31, fhalf = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int m0, n0;
-    skinny_tile_of_workgroup<TM>(blockIdx.x, p.m, p.n, m0, n0);
-    for (int i = tid; i < TM * 16 * 64; i += kThreads) red[i] = 0;
+    split_tile_of_workgroup<B>(blockIdx.x, p.m, p.n, m0, n0);
 
-    const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<int8_t*>(p.w), 0, static_cast<int>((static_cast<int64_t>(p.n) - 1) * p.ldw + p.k), kRsrcFlags);
-    const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<int8_t*>(p.a), 0, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k), kRsrcFlags);
-    // fetch mapping: instruction i, lane l -> tile row 8i + l/8, 16-byte chunk l%8
-    const int lrow = lane >> 3, lchunk = lane & 7;
-    int w_off[4], a_off[TM][4];
+    // output o of this thread: element tid + o * kThreads of the blocks' accumulators, 256 each: of lane l, register r row
+    // l % 16 and column 4 (l / 16) + r
+    int mm[C::kOutputs], nn[C::kOutputs];
+    float s_row[C::kOutputs], s_col[C::kOutputs];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = n0 + 8 * i + lrow;
-        w_off[i] = row < p.n ? static_cast<int>(row * p.ldw) + lchunk * 16 : -1;
-#pragma unroll
-        for (int j = 0; j < TM; ++j) {
-            const int arow = m0 + j * 32 + 8 * i + lrow;
-            a_off[j][i] = arow < p.m ? static_cast<int>(arow * p.lda) + lchunk * 16 : -1;
+    for (int o = 0; o < C::kOutputs; ++o) {
+        const int t = tid + o * C::kThreads, block = t >> 8;
+        mm[o] = m0 + block / C::kBlocks * 16 + ((t >> 2) & 15);
+        nn[o] = t < B * B ? n0 + block % C::kBlocks * 16 + ((t >> 6) & 3) * 4 + (t & 3) : p.n;
+        s_row[o] = s_col[o] = p.alpha;
+        if (!p.use_alpha && mm[o] < p.m && nn[o] < p.n) {
+            s_row[o] = p.a_scale[p.a_scale_numel == 1 ? 0 : mm[o]];
+            s_col[o] = p.w_scale[p.w_scale_numel == 1 ? 0 : nn[o]];
         }
     }
 
-    const int k_tiles = (p.k + kBK - 1) / kBK;
-    const int my_tiles = (k_tiles - wave + WAVES - 1) / WAVES;      // tiles wave, wave + WAVES, ...
-    v4u fw[DEPTH][4], fa[DEPTH][TM][4];
-    auto load = [&](int i_tile, auto buf_c) {
-        constexpr int buf = decltype(buf_c)::value;
-        const int k0 = (wave + i_tile * WAVES) * kBK;
-        const bool k_ok = k0 + lchunk * 16 < p.k;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            fw[buf][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, (k_ok && w_off[i] >= 0) ? w_off[i] + k0 : kOob, 0, 0);
-#pragma unroll
-            for (int j = 0; j < TM; ++j) {
-                fa[buf][j][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (k_ok && a_off[j][i] >= 0) ? a_off[j][i] + k0 : kOob, 0, 0);
-            }
-        }
+    const v4i rsrc_a = make_rsrc(p.a, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k));
+    const v4i rsrc_w = make_rsrc(p.w, static_cast<int>((static_cast<int64_t>(p.n) - 1) * p.ldw + p.k));
+    TileLoader<C::kRequests> load_a, load_w;
+    load_a.template init<1>(m0, p.m, p.lda, 0, lane);
+    load_w.template init<1>(n0, p.n, p.ldw, 0, lane);
+    uint8_t* const mine = lds + wave * DEPTH * C::kUnit;
+    const uint32_t at = lds_offset_of(mine);
+    const int units = (p.k + kBK - 1) / kBK, my_units = (units - wave + WAVES - 1) / WAVES;       // units wave, wave + WAVES, ...
+    auto issue = [&](int u, int slot) {
+        const int k0 = (wave + u * WAVES) * kBK;
+        load_w.template issue<1>(rsrc_w, k0, p.k, at + slot * C::kUnit + B * kBK, 0);
+        load_a.template issue<1>(rsrc_a, k0, p.k, at + slot * C::kUnit, 0);
     };
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u)
+        if (u < my_units) issue(u, u);
 
-    v16i acc[TM];
+    v4i acc[C::kBlocks][C::kBlocks];                       // [rows][columns]
 #pragma unroll
-    for (int j = 0; j < TM; ++j)
+    for (int i = 0; i < C::kBlocks; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[j][r] = 0;
-
-    uint8_t* stage = lds + wave * ((1 + TM) * kTile);
-    static_for<0, DEPTH - 1>([&](auto s) { load(decltype(s)::value, s); });
-    for (int base = 0; base < my_tiles; base += DEPTH) {
-        static_for<0, DEPTH>([&](auto s_c) {
-            constexpr int s = decltype(s_c)::value;
-            // tiles past this wave's share are outside K: their loads touch no memory
-            load(base + s + DEPTH - 1, std::integral_constant<int, (s + DEPTH - 1) % DEPTH>{});
-            if (base + s < my_tiles) {
+        for (int j = 0; j < C::kBlocks; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+    for (int base = 0; base < my_units; base += DEPTH) {
+        static_for<0, DEPTH>([&](auto slot_c) {
+            constexpr int slot = decltype(slot_c)::value;
+            const int u = base + slot;
+            if (u >= my_units) return;
+            if (u + DEPTH <= my_units) __builtin_amdgcn_s_waitcnt(vmcnt_imm((DEPTH - 1) * 2 * C::kRequests));
+            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            wave_lds_sync();
+            const uint8_t* sa = mine + slot * C::kUnit;
+            v4i fa[2][C::kBlocks], fw[2][C::kBlocks];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int row = 8 * i + lrow;
-                    *reinterpret_cast<v4u*>(stage + row * kBK + swz(row, lchunk) * 16) = fw[s][i];
+            for (int step = 0; step < 2; ++step) {
+                const int off = (lane & 15) * kBK + swz(lane & 15, 4 * step + (lane >> 4)) * 16;
 #pragma unroll
-                    for (int j = 0; j < TM; ++j)
-                        *reinterpret_cast<v4u*>(stage + (1 + j) * kTile + row * kBK + swz(row, lchunk) * 16) = fa[s][j][i];
+                for (int i = 0; i < C::kBlocks; ++i) {
+                    fa[step][i] = *reinterpret_cast<const v4i*>(sa + off + i * 16 * kBK);
+                    fw[step][i] = *reinterpret_cast<const v4i*>(sa + B * kBK + off + i * 16 * kBK);
                 }
-                wave_lds_sync();
-#pragma unroll
-                for (int kk = 0; kk < 4; ++kk) {
-                    const int off = frow * kBK + swz(frow, kk * 2 + fhalf) * 16;
-                    const v4i bw = *reinterpret_cast<const v4i*>(stage + off);
-#pragma unroll
-                    for (int j = 0; j < TM; ++j) {
-                        const v4i ba = *reinterpret_cast<const v4i*>(stage + (1 + j) * kTile + off);
-                        acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bw, ba, acc[j], 0, 0, 0);
-                    }
-                }
-                wave_lds_sync();
             }
+#pragma unroll
+            for (int step = 0; step < 2; ++step)
+#pragma unroll
+                for (int i = 0; i < C::kBlocks; ++i)
+#pragma unroll
+                    for (int j = 0; j < C::kBlocks; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[step][j], fa[step][i], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);             // (the fragments are in registers: the slot is free)
+            if (u + DEPTH < my_units) issue(u + DEPTH, slot);
         });
     }
 
-    Epilogue e;
-    e.row_scale = p.a_scale; e.col_scale = p.w_scale;
-    e.row_numel = p.a_scale_numel; e.col_numel = p.w_scale_numel;
-    e.use_alpha = p.use_alpha; e.alpha = p.alpha; e.round_mode = p.round_mode; e.col_outer = p.scale_order;
-    e.ldd = p.ldd; e.d = p.d;
-    skinny_reduce_store<TM, OUT, FLEX, false>(e, acc, red, p.m, p.n, m0, n0, tid, kThreads);
-}
-
-template <int TM, int WAVES, int OUT, bool FLEX>
-int launch_skinny_one(const QaGemmW8A8Params& p, hipStream_t stream) {
-    constexpr int kLds = skinny_lds_bytes<TM, WAVES>();
-    auto kernel = gemm_w8a8_skinny_kernel<TM, WAVES, 3, OUT, FLEX>;
-    if (kLds > 65536) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                kLds) != hipSuccess) {
-            return check_launch();
-        }
-    }
-    const int64_t blocks = static_cast<int64_t>((p.m + 32 * TM - 1) / (32 * TM)) * ((p.n + 31) / 32);
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * WAVES), kLds, stream, p);
-    return check_launch();
-}
-
-template <int TM, int WAVES, bool FLEX>
-int launch_skinny(const QaGemmW8A8Params& p, hipStream_t stream) {
-    if (p.out_type == QA_OUT_I8) return launch_skinny_one<TM, WAVES, QA_OUT_I8, FLEX>(p, stream);
-    if (p.out_type == QA_OUT_BF16) return launch_skinny_one<TM, WAVES, QA_OUT_BF16, FLEX>(p, stream);
-    return launch_skinny_one<TM, WAVES, QA_OUT_F16, FLEX>(p, stream);
-}
-
-// ---------------------------------------------------------------------------------------------
-// Products of so few outputs that even tiles of 32 x 32 leave most CUs idle (the step-size and B, C projection of a decode
-// batch or a short prompt): 16 x 16 outputs per workgroup, K over sixteen waves.  What bounds them is latency - a CU fetches
-// its operand rows at about 64 bytes a clock, and every trip to memory counts - so the outputs go to four times the CUs, a wave asks
-// for all its fragments (16 rows x 64 bytes, straight into the operand registers of 16x16x64) before it multiplies, and the
-// sixteen partial sums meet in LDS with one store and sixteen loads each.
-// Against 32 x 32 with K over four waves (rows x outputs x K, us): 64 x 192 x 5120 7.5 -> 6.8, 64 x 80 x 1536 4.0 -> 3.2, 512 x 80
-// x 1536 4.7 -> 3.8, 512 x 128 x 3072 5.7 -> 5.1, 16 x 2560 x 5120 9.4 -> 8.7, 16 x 3072 x 768 4.2 -> 3.2.
-// ---------------------------------------------------------------------------------------------
-template <int OUT>
-__global__ __launch_bounds__(1024) void gemm_w8a8_narrow_kernel(QaGemmW8A8Params p) {
-    constexpr int kWaves = 16, kUnits = 3;                 // units of 128 bytes of K at a time, all in flight
-    __shared__ __align__(16) int red[kWaves][256];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int blocks_m = (p.m + 15) / 16;
-    const int m0 = static_cast<int>(blockIdx.x) % blocks_m * 16, n0 = static_cast<int>(blockIdx.x) / blocks_m * 16;
-    const int chunk = (lane >> 4) * 16;
-    // rows outside repeat the last one: their outputs are not written
-    const int8_t* a = p.a + static_cast<int64_t>(min(m0 + (lane & 15), p.m - 1)) * p.lda;
-    const int8_t* w = p.w + static_cast<int64_t>(min(n0 + (lane & 15), p.n - 1)) * p.ldw;
-    v4i acc = {0, 0, 0, 0};
-    for (int k0 = wave * kBK; k0 < p.k; k0 += kUnits * kWaves * kBK) {
-        v4i fa[2 * kUnits], fw[2 * kUnits];
+    __syncthreads();                                       // every wave is done with its units
+    int* const sums = reinterpret_cast<int*>(lds);
 #pragma unroll
-        for (int s = 0; s < 2 * kUnits; ++s) {
-            const int k = k0 + s / 2 * (kWaves * kBK) + s % 2 * 64 + chunk;
-            fa[s] = fw[s] = v4i{0, 0, 0, 0};
-            if (k < p.k) {
-                fw[s] = *reinterpret_cast<const v4i*>(w + k);
-                fa[s] = *reinterpret_cast<const v4i*>(a + k);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < C::kBlocks; ++i)
 #pragma unroll
-        for (int s = 0; s < 2 * kUnits; ++s) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[s], fa[s], acc, 0, 0, 0);
-    }
-    *reinterpret_cast<v4i*>(&red[wave][lane * 4]) = acc;
+        for (int j = 0; j < C::kBlocks; ++j) *reinterpret_cast<v4i*>(&sums[wave * B * B + (i * C::kBlocks + j) * 256 + lane * 4]) = acc[i][j];
     __syncthreads();
-    if (threadIdx.x >= 256) return;
-    // thread t: row (t >> 2) & 15, column 4 (t >> 6) + (t & 3)
-    const int t = threadIdx.x, mm = m0 + ((t >> 2) & 15), nn = n0 + (t >> 6) * 4 + (t & 3);
-    if (mm >= p.m || nn >= p.n) return;
-    const float s_row = p.a_scale[p.a_scale_numel == 1 ? 0 : mm], s_col = p.w_scale[p.w_scale_numel == 1 ? 0 : nn];
-    int sum = 0;
 #pragma unroll
-    for (int x = 0; x < kWaves; ++x) sum += red[x][t];
-    const float accf = static_cast<float>(sum);
-    float v = p.scale_order ? s_col * (s_row * accf) : s_row * (s_col * accf);
-    asm volatile("" : "+v"(v));                            // the fp32 product is rounded on its own
-    const int64_t at = static_cast<int64_t>(mm) * p.ldd + nn;
-    if (OUT == QA_OUT_I8) static_cast<int8_t*>(p.d)[at] = static_cast<int8_t>(quant8(v, QA_ROUND_RNE));
-    else static_cast<uint16_t*>(p.d)[at] = one_f16_or_bf16<OUT>(v);
+    for (int o = 0; o < C::kOutputs; ++o) {
+        if (mm[o] >= p.m || nn[o] >= p.n) continue;
+        int sum = 0;
+#pragma unroll
+        for (int x = 0; x < WAVES; ++x) sum += sums[x * B * B + tid + o * C::kThreads];
+        const float accf = static_cast<float>(sum);
+        float v;
+        if (p.use_alpha) v = s_row[o] * accf;
+        else if (p.scale_order) v = s_col[o] * (s_row[o] * accf);
+        else if (p.round_mode == QA_ROUND_HALF_AWAY) v = (s_col[o] * s_row[o]) * accf;      // the rule of single rows
+        else v = s_row[o] * (s_col[o] * accf);
+        asm volatile("" : "+v"(v));                        // the fp32 product is rounded on its own
+        const int64_t to = static_cast<int64_t>(mm[o]) * p.ldd + nn[o];
+        if (OUT == QA_OUT_I8) static_cast<int8_t*>(p.d)[to] = static_cast<int8_t>(quant8(v, p.round_mode));
+        else static_cast<uint16_t*>(p.d)[to] = one_f16_or_bf16<OUT>(v);
+    }
 }
 
-int launch_narrow(const QaGemmW8A8Params& p, hipStream_t stream) {
-    const int64_t blocks = static_cast<int64_t>((p.m + 15) / 16) * ((p.n + 15) / 16);
-    auto kernel = p.out_type == QA_OUT_I8 ? gemm_w8a8_narrow_kernel<QA_OUT_I8> : p.out_type == QA_OUT_BF16 ? gemm_w8a8_narrow_kernel<QA_OUT_BF16> : gemm_w8a8_narrow_kernel<QA_OUT_F16>;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(1024), 0, stream, p);
+template <int B, int WAVES, int DEPTH>
+int launch_split(const QaGemmW8A8Params& p, hipStream_t stream) {
+    using C = SplitCfg<B, WAVES, DEPTH>;
+    const int64_t blocks = static_cast<int64_t>((p.m + B - 1) / B) * ((p.n + B - 1) / B);
+    auto kernel = p.out_type == QA_OUT_I8 ? gemm_w8a8_split_kernel<B, WAVES, DEPTH, QA_OUT_I8> : p.out_type == QA_OUT_BF16 ? gemm_w8a8_split_kernel<B, WAVES, DEPTH, QA_OUT_BF16> : gemm_w8a8_split_kernel<B, WAVES, DEPTH, QA_OUT_F16>;
+    if (C::kLdsBytes > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, C::kLdsBytes) != hipSuccess) return check_launch();
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(C::kThreads), C::kLdsBytes, stream, p);
     return check_launch();
-}
-
-template <bool FLEX>
-int dispatch_skinny(const QaGemmW8A8Params& p, hipStream_t stream) {
-    return launch_skinny<1, 4, FLEX>(p, stream);
 }
 
 // Tile of a launch: the smallest whose tiles fit the part in one round.  With at most one tile per CU a launch takes a
-// tile's own time - about 2.5 us and, per 128 bytes of K, 0.105 us (16 x 16, K split over the waves), 0.125 (32 x 32, the same), 0.20 (64 x 64), 0.31
+// tile's own time - about 2.5 us and, per 128 bytes of K, 0.04 us (16 x 16, K split over the waves), 0.10 (32 x 32, the same), 0.20 (64 x 64), 0.31
 // (128 x 64), 0.48 (128 x 128, four stages), 0.68 (128 x 256), 1.15 (256 x 256) - so smaller tiles win until a second round
 // starts.  Measured at M 16 .. 16384 with ten of the projections' N and K: this choice is the fastest or
 // within 8 % of it.  Against 128 x 128 tiles up to 192 tiles of 256 x 256 (rows x outputs x K, us): 512 x 80 x 1536 9.6 ->
@@ -394,8 +334,8 @@ int dispatch_skinny(const QaGemmW8A8Params& p, hipStream_t stream) {
 int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
     const int cus = compute_units();
     auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
-    if (tiles(16, 16) <= cus) return launch_narrow(p, stream);                       // (two rounds of these: slower than one of 32 x 32)
-    if (tiles(32, 32) <= cus) return dispatch_skinny<false>(p, stream);
+    if (tiles(16, 16) <= cus) return launch_split<16, 8, 2>(p, stream);              // (two rounds of these: slower than one of 32 x 32)
+    if (tiles(32, 32) <= cus) return launch_split<32, 8, 1>(p, stream);
     if (tiles(64, 64) <= cus) return launch_gemm<1, 1, 2, 2, 4, false>(p, stream);
     if (tiles(128, 64) <= cus) return launch_gemm<1, 1, 4, 2, 4, false>(p, stream);
     if (tiles(128, 128) <= cus) return launch_gemm<2, 1, 2, 4, 4, false>(p, stream);
@@ -447,6 +387,6 @@ extern "C" int qa_gemm_w8a8(const QaGemmW8A8Params* p, void* stream_) {
         return gemv_launch(g, nullptr, stream);
     }
     // the single-row rules (host alpha, round-half-away) only ever come with tiny M
-    if (flex) return p->m <= 64 ? dispatch_skinny<true>(*p, stream) : launch_gemm<2, 2, 2, 2, 2, true>(*p, stream);
+    if (flex) return p->m <= 64 ? launch_split<32, 8, 1>(*p, stream) : launch_gemm<2, 2, 2, 2, 2, true>(*p, stream);
     return dispatch_tiles(*p, stream);
 }

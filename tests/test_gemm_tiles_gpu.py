@@ -46,6 +46,15 @@ def test_int8_weights_of_few_outputs(dev, M, N, K, order):
     test_int8_weights(dev, M, N, K, order)
 
 
+# K over the waves of a workgroup, 16 x 16 and 32 x 32 outputs: fewer 128-byte units of K than waves, one each, one more, the
+# ring of two units round several times, all with and without a remainder of K
+@pytest.mark.parametrize("M,N", [(9, 200), (20, 1000), (70, 1900)])
+@pytest.mark.parametrize("K", [16, 128, 1008, 1024, 1040, 2048, 2064, 3200, 4112])
+@pytest.mark.parametrize("order,dtype", [(0, torch.int8), (1, torch.int8), (0, torch.float16), (0, torch.bfloat16)])
+def test_k_split_over_the_waves(dev, M, N, K, order, dtype):
+    test_large_tiles_over_a_long_k(dev, M, N, K, order, dtype)
+
+
 # 32 x 32 with four and eight waves, 64 x 64, 64 x 128, 128 x 128, 192 x 128, expanded once
 @pytest.mark.parametrize("M,N,K,workspace", [(70, 200, 2176, False), (100, 1000, 384, False), (130, 2050, 1664, False), (250, 2500, 1152, False),
                                              (600, 2100, 256, False), (300, 4200, 1664, False), (70, 9000, 128, False), (700, 3100, 1152, False),
@@ -94,9 +103,9 @@ def test_large_tiles_over_a_long_k(dev, M, N, K, order, dtype):
         assert int(want.max()) - int(want.min()) > 100
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 300, 640), (1500, 2500, 1712)])
+@pytest.mark.parametrize("M,N,K", [(9, 37, 1040), (64, 300, 640), (65, 300, 640), (1500, 2500, 1712)])
 def test_the_single_row_rules_with_many_rows(dev, M, N, K):
-    """128 x 128 with two stages: the host's scalar, and rounding half away from zero."""
+    """32 x 32 with K over the waves and 128 x 128 with two stages: the host's scalar, and rounding half away from zero."""
     g = torch.Generator(device=dev).manual_seed(K)
     a, w = (torch.randint(-128, 128, s, dtype=torch.int8, device=dev, generator=g) for s in ((M, K), (N, K)))
     acc = (a.double() @ w.double().t()).float()
