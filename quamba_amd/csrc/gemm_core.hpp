@@ -79,9 +79,6 @@ __device__ __forceinline__ uint16_t one_f16_or_bf16(float v) {
 }
 
 struct Epilogue {
-    const float* row_scale;   // s_row, numel 1 or M (unused with use_alpha)
-    const float* col_scale;   // s_col, numel 1 or N
-    int row_numel, col_numel;
     int use_alpha;            // d = cast(alpha * acc)
     float alpha;
     int round_mode;           // QaRound
@@ -498,13 +495,6 @@ constexpr int epilogue_lds_bytes() {
     return WAVES * 32 * ((TM > TN ? TM : TN) * 32 * 2 + 16);
 }
 
-// ---------------------------------------------------------------------------------------------
-// Pieces shared by the kernels for few activation rows (one 32-column block per workgroup, K split
-// over the waves, a wave-private staging area of one weight tile and TM activation tiles).
-// ---------------------------------------------------------------------------------------------
-template <int TM, int WAVES>
-constexpr int skinny_lds_bytes() { return WAVES * (1 + TM) * 32 * kBK + TM * 16 * 64 * 4; }
-
 // Tile of workgroup `linear`, row blocks of BM by column blocks of BN.  With many column blocks the row blocks of one of
 // them go to one XCD (eight workgroups apart), whose L2 then holds their weights.
 template <int BM, int BN = BM>
@@ -517,69 +507,6 @@ __device__ __forceinline__ void split_tile_of_workgroup(int linear, int m, int n
         const int rest = linear - whole, columns = blocks_n % 8;
         n0 = (blocks_n / 8 * 8 + rest % columns) * BN;
         m0 = rest / columns * BM;
-    }
-}
-
-// Adds the waves' partial accumulators in `red` (TM*16*64 ints, zeroed by the caller before any
-// barrier it has passed), then every thread scales and writes four consecutive columns of one row.
-// Lane l of the accumulator layout holds row (l & 31) and, in registers 4q..4q+3, the columns
-// 8q + 4*(l >> 5) + (0..3): one unit = (row block, q, lane).
-template <int TM, int OUT, bool FLEX, bool TRANS>
-__device__ __forceinline__ void skinny_reduce_store(const Epilogue& e, v16i (&acc)[TM], int* red, int m, int n,
-                                                    int m0, int n0, int tid, int threads) {
-    const int lane = tid & 63;
-    __syncthreads();                                       // red is zero
-#pragma unroll
-    for (int j = 0; j < TM; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            __hip_atomic_fetch_add(&red[(j * 16 + r) * 64 + lane], acc[j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __syncthreads();
-
-    constexpr int kElt = OUT == QA_OUT_I8 ? 1 : 2;
-    const bool use_alpha = FLEX && e.use_alpha;
-    const bool away = FLEX && e.round_mode == QA_ROUND_HALF_AWAY;
-    const int round_mode = FLEX ? e.round_mode : QA_ROUND_RNE;
-    const bool vec_ok = !TRANS && e.ldd % 4 == 0 && (reinterpret_cast<uintptr_t>(e.d) & (4 * kElt - 1)) == 0;
-    for (int u = tid; u < TM * 4 * 64; u += threads) {
-        const int ul = u & 63, j = u >> 8, q = (u >> 6) & 3;
-        const int mm = m0 + j * 32 + (ul & 31);
-        const int nn = n0 + 8 * q + 4 * (ul >> 5);
-        if (mm >= m || nn >= n) continue;
-        const float s_row = use_alpha ? e.alpha : e.row_scale[e.row_numel == 1 ? 0 : mm];
-        float v[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const float accf = static_cast<float>(red[(j * 16 + q * 4 + t) * 64 + ul]);
-            const float s_col = use_alpha ? 1.0f : e.col_scale[e.col_numel == 1 ? 0 : min(nn + t, n - 1)];
-            if (use_alpha) v[t] = s_row * accf;
-            else if (e.col_outer) v[t] = s_col * (s_row * accf);
-            else v[t] = away ? (s_col * s_row) * accf : s_row * (s_col * accf);
-            asm volatile("" : "+v"(v[t]));                 // the fp32 product is rounded on its own
-        }
-        const int cols = min(4, n - nn);
-        const int64_t step = TRANS ? e.ldd : 1;            // distance between consecutive columns
-        const int64_t at = TRANS ? static_cast<int64_t>(nn) * e.ldd + mm : static_cast<int64_t>(mm) * e.ldd + nn;
-        if (OUT == QA_OUT_I8) {
-            int8_t* dst = static_cast<int8_t*>(e.d) + at;
-            if (vec_ok && cols == 4) {
-                const uint32_t b0 = quant8(v[0], round_mode) & 0xff, b1 = quant8(v[1], round_mode) & 0xff;
-                const uint32_t b2 = quant8(v[2], round_mode) & 0xff, b3 = quant8(v[3], round_mode);
-                *reinterpret_cast<uint32_t*>(dst) = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
-            } else {
-                for (int t = 0; t < cols; ++t) dst[t * step] = static_cast<int8_t>(quant8(v[t], round_mode));
-            }
-        } else {
-            uint16_t* dst = static_cast<uint16_t*>(e.d) + at;
-            if (vec_ok && cols == 4) {
-                uint2 pk;
-                pk.x = pack2_f16_or_bf16<OUT>(v[0], v[1]);
-                pk.y = pack2_f16_or_bf16<OUT>(v[2], v[3]);
-                *reinterpret_cast<uint2*>(dst) = pk;
-            } else {
-                for (int t = 0; t < cols; ++t) dst[t * step] = one_f16_or_bf16<OUT>(v[t]);
-            }
-        }
     }
 }
 

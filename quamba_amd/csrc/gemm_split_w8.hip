@@ -1,0 +1,6 @@
+// The products of some activation rows with int8 weights (gemm_split.hpp).
+#include "gemm_split.hpp"
+
+namespace qa {
+int split_launch_w8(const GemvParams& p, int shape, hipStream_t stream) { return split::launch_shape<8>(p, shape, stream); }
+}  // namespace qa

@@ -349,14 +349,46 @@ int launch_reg(const QaGemmW4A8Params& p, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Few activation rows or few columns: a stream over the packed weights.  A workgroup
+// Few activation rows, transposed output: a stream over the packed weights.  A workgroup
 // owns 32 output columns and all rows; its WAVES waves split K between them in interleaved pieces
 // of 256 codes, i.e. one full 128-byte line of packed weights per row.  A wave fetches a piece with
 // eight lanes per row (DEPTH pieces in flight in registers), expands its 32 codes per lane to int8
 // and passes them through a staging area in LDS that is private to the wave; the activation tiles
 // take the same route, one 128-byte half at a time.  Partial sums meet in LDS at the end.
 // ---------------------------------------------------------------------------------------------
-template <int TM, int AI, int WAVES, int DEPTH, int OUT, bool TRANS>
+template <int TM, int WAVES>
+constexpr int skinny_lds_bytes() { return WAVES * (2 + TM) * 32 * kBK + TM * 16 * 64 * 4; }      // (2 + TM) tiles per wave, TM reduction blocks
+
+// Adds the waves' partial accumulators in `red` (TM*16*64 ints, zeroed by the caller before any
+// barrier it has passed), then every thread scales and writes four columns of one row.
+// Lane l of the accumulator layout holds row (l & 31) and, in registers 4q..4q+3, the columns
+// 8q + 4*(l >> 5) + (0..3): one unit = (row block, q, lane).
+template <int TM, int OUT>
+__device__ __forceinline__ void skinny_reduce_store(const QaGemmW4A8Params& p, v16i (&acc)[TM], int* red, int m0, int n0, int tid, int threads) {
+    const int lane = tid & 63;
+    __syncthreads();                                       // red is zero
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            __hip_atomic_fetch_add(&red[(j * 16 + r) * 64 + lane], acc[j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __syncthreads();
+    for (int u = tid; u < TM * 4 * 64; u += threads) {
+        const int ul = u & 63, j = u >> 8, q = (u >> 6) & 3;
+        const int mm = m0 + j * 32 + (ul & 31), nn = n0 + 8 * q + 4 * (ul >> 5);
+        if (mm >= p.m || nn >= p.n) continue;
+        const float s_row = p.s_token[p.tok_scale_numel == 1 ? 0 : mm];
+        for (int t = 0; t < min(4, p.n - nn); ++t) {
+            float v = s_row * (p.s_channel[nn + t] * static_cast<float>(red[(j * 16 + q * 4 + t) * 64 + ul]));
+            asm volatile("" : "+v"(v));                    // the fp32 product is rounded on its own
+            const int64_t at = static_cast<int64_t>(nn + t) * p.ldd + mm;
+            if (OUT == QA_OUT_I8) static_cast<int8_t*>(p.d)[at] = static_cast<int8_t>(quant8(v, QA_ROUND_RNE));
+            else static_cast<uint16_t*>(p.d)[at] = one_f16_or_bf16<OUT>(v);
+        }
+    }
+}
+
+template <int TM, int AI, int WAVES, int DEPTH, int OUT>
 __global__ __launch_bounds__(64 * WAVES) void gemm_w4a8_skinny_kernel(QaGemmW4A8Params p) {
     constexpr int kThreads = 64 * WAVES;
     constexpr int kOob = 0x7ffffff0;                       // beyond any buffer: the load returns zeros
@@ -490,18 +522,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_w4a8_skinny_kernel(QaGemmW4A8
         });
     }
 
-    Epilogue e;
-    e.row_scale = p.s_token; e.col_scale = p.s_channel;
-    e.row_numel = p.tok_scale_numel; e.col_numel = p.n;
-    e.use_alpha = 0; e.alpha = 0.0f; e.round_mode = QA_ROUND_RNE; e.col_outer = 0;
-    e.ldd = p.ldd; e.d = p.d;
-    skinny_reduce_store<TM, OUT, false, TRANS>(e, acc, red, p.m, p.n, m0, n0, tid, kThreads);
+    skinny_reduce_store<TM, OUT>(p, acc, red, m0, n0, tid, kThreads);
 }
 
-template <int TM, int AI, int WAVES, int DEPTH, int OUT, bool TRANS>
+template <int TM, int AI, int WAVES, int DEPTH, int OUT>
 int launch_skinny_one(const QaGemmW4A8Params& p, hipStream_t stream) {
-    constexpr int kLds = skinny_lds_bytes<TM + 1, WAVES>() - 16 * 64 * 4;   // (2 + TM) tiles per wave, TM reduction blocks
-    auto kernel = gemm_w4a8_skinny_kernel<TM, AI, WAVES, DEPTH, OUT, TRANS>;
+    constexpr int kLds = skinny_lds_bytes<TM, WAVES>();
+    auto kernel = gemm_w4a8_skinny_kernel<TM, AI, WAVES, DEPTH, OUT>;
     if (kLds > 65536) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 kLds) != hipSuccess) {
@@ -515,22 +542,14 @@ int launch_skinny_one(const QaGemmW4A8Params& p, hipStream_t stream) {
 
 template <int TM, int AI, int WAVES, int DEPTH>
 int launch_skinny(const QaGemmW4A8Params& p, hipStream_t stream) {
-    if (p.out_type == QA_OUT_I8) {
-        return p.output_transpose ? launch_skinny_one<TM, AI, WAVES, DEPTH, QA_OUT_I8, true>(p, stream)
-                                  : launch_skinny_one<TM, AI, WAVES, DEPTH, QA_OUT_I8, false>(p, stream);
-    }
-    return p.output_transpose ? launch_skinny_one<TM, AI, WAVES, DEPTH, QA_OUT_F16, true>(p, stream)
-                              : launch_skinny_one<TM, AI, WAVES, DEPTH, QA_OUT_F16, false>(p, stream);
+    return p.out_type == QA_OUT_I8 ? launch_skinny_one<TM, AI, WAVES, DEPTH, QA_OUT_I8>(p, stream) : launch_skinny_one<TM, AI, WAVES, DEPTH, QA_OUT_F16>(p, stream);
 }
 
 int64_t tiles_of(const QaGemmW4A8Params& p, int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); }
 
-// eight waves share K when there is at most a workgroup per CU and K is long, else four (4096 x 8192 at 64 rows: 13.8
-// against 15.8 us; 18560 x 4096 at 16 rows: 23.0 against 19.1)
-bool skinny_is_wide(const QaGemmW4A8Params& p, int cus) { return tiles_of(p, 32, 32) <= cus && p.k >= 2048; }
-
 int dispatch_skinny(const QaGemmW4A8Params& p, int cus, hipStream_t stream) {
-    const bool wide = skinny_is_wide(p, cus);
+    // eight waves share K when there is at most a workgroup per CU and K is long, else four
+    const bool wide = tiles_of(p, 32, 32) <= cus && p.k >= 2048;
     // activation rows are fetched eight at a time: up to 8 rows need one fetch per tile, up to 32 four
     if (p.m <= 8) return wide ? launch_skinny<1, 1, 8, 3>(p, stream) : launch_skinny<1, 1, 4, 3>(p, stream);
     return wide ? launch_skinny<1, 4, 8, 2>(p, stream) : launch_skinny<1, 4, 4, 2>(p, stream);
@@ -567,9 +586,9 @@ __global__ __launch_bounds__(256) void w4_expand_kernel(QaGemmW4A8Params p, int8
 // r workgroups on the busiest CU take a fixed time and one that grows with r per 128 of K; the kernels differ in the size of
 // their tiles - large ones expand each code fewer times, small ones spread over the chip earlier - and the weights expanded
 // once, in a pass of their own, cost that pass.
-enum Way { kWaySkinny, kWay64x64, kWay64x128, kWay128x128, kWay192x128, kWayExpandOnce };
+enum Way { kWaySplit, kWay64x64, kWay64x128, kWay128x128, kWay192x128, kWayExpandOnce };
 
-int cheapest_way(const QaGemmW4A8Params& p, int cus, bool addressable, bool expandable) {
+int cheapest_way(const QaGemmW4A8Params& p, int cus, const SplitChoice& split, bool expandable) {
     const double k_tiles = p.k / 128;
     auto rounds = [&](int64_t bm, int64_t bn) { return static_cast<double>((tiles_of(p, bm, bn) + cus - 1) / cus); };
     double best = 1e30;
@@ -577,10 +596,7 @@ int cheapest_way(const QaGemmW4A8Params& p, int cus, bool addressable, bool expa
     auto offer = [&](int w, double cost) {
         if (cost < best) { best = cost; way = w; }
     };
-    if (addressable) {
-        const bool wide = skinny_is_wide(p, cus);
-        offer(kWaySkinny, 3.0 + std::ceil(k_tiles / (wide ? 8 : 4)) * (wide ? 1.35 : 0.75 + 0.38 * rounds(32, 32)));
-    }
+    if (split.shape >= 0) offer(kWaySplit, split.us);
     offer(kWay64x64, 3.0 + k_tiles * (0.10 + 0.28 * rounds(64, 64)));
     offer(kWay64x128, 3.0 + k_tiles * (0.08 + 0.42 * rounds(64, 128)));
     offer(kWay128x128, 3.0 + k_tiles * std::max(0.73, 0.10 + 0.57 * rounds(128, 128)));
@@ -612,25 +628,24 @@ extern "C" int qa_gemm_w4a8(const QaGemmW4A8Params* p, void* stream_) {
     if (p->m == 0 || p->n == 0) return QA_OK;
     if (static_cast<int64_t>(p->m) * p->lda >= 0x70000000LL) return QA_ERR_SHAPE;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    if (p->m <= kGemvRows && !p->output_transpose && p->group_size == 128 && p->n % 4 == 0 && (reinterpret_cast<uintptr_t>(p->s_group) & 7u) == 0) {
+    const bool addressable = static_cast<int64_t>(p->n) * (p->k / 2) < 0x70000000LL;
+    const int64_t w8_bytes = static_cast<int64_t>(p->n) * p->k;
+    const bool expandable = p->w8_workspace && p->w8_workspace_bytes >= w8_bytes && aligned16(p->w8_workspace) && w8_bytes < 0x70000000LL;
+    const int cus = compute_units();
+    if (p->output_transpose && p->m <= 64 && addressable) return dispatch_skinny(*p, cus, stream);
+    if (!p->output_transpose) {
         GemvParams g = {};
         g.m = p->m; g.n = p->n; g.k = p->k; g.bits = 4;
         g.out_type = p->out_type;
         g.rule = kGemvRowOuter;
         g.row_numel = p->tok_scale_numel; g.col_numel = p->n;
         g.lda = p->lda; g.ldw = p->k / 2; g.ldd = p->ldd;
-        g.a = p->a; g.w = p->w_packed; g.s_group = static_cast<const __half*>(p->s_group);
+        g.a = p->a; g.w = p->w_packed; g.s_group = p->group_size == 128 ? static_cast<const __half*>(p->s_group) : nullptr;
         g.row_scale = p->s_token; g.col_scale = p->s_channel; g.d = p->d;
-        return gemv_launch(g, nullptr, stream);
-    }
-    const bool addressable = static_cast<int64_t>(p->n) * (p->k / 2) < 0x70000000LL;
-    const int64_t w8_bytes = static_cast<int64_t>(p->n) * p->k;
-    const bool expandable = p->w8_workspace && p->w8_workspace_bytes >= w8_bytes && aligned16(p->w8_workspace) && w8_bytes < 0x70000000LL;
-    const int cus = compute_units();
-    if (p->output_transpose ? p->m <= 64 && addressable : p->m <= kGemvRows && addressable) return dispatch_skinny(*p, cus, stream);
-    if (!p->output_transpose) {
-        const int way = cheapest_way(*p, cus, addressable, expandable);
-        if (way == kWaySkinny) return dispatch_skinny(*p, cus, stream);
+        if (gemv_is_faster(p->m, p->n, p->k) && g.s_group && p->n % 4 == 0 && (reinterpret_cast<uintptr_t>(p->s_group) & 7u) == 0) return gemv_launch(g, nullptr, stream);
+        const SplitChoice split = split_addressable_w4(p->n, p->k) ? split_choice(4, p->m, p->n, p->k, cus) : SplitChoice{-1, 0.0f};
+        const int way = cheapest_way(*p, cus, split, expandable);
+        if (way == kWaySplit) return split_launch_w4(g, split.shape, stream);
         if (way == kWay64x64) return p->out_type == QA_OUT_I8 ? launch_tile<QA_OUT_I8>(*p, stream) : launch_tile<QA_OUT_F16>(*p, stream);
         if (way == kWay64x128) return launch_reg<2, 4, 256>(*p, stream);
         if (way == kWay128x128) return launch_reg<4, 4, 128>(*p, stream);

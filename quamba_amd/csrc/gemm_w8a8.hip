@@ -185,157 +185,37 @@ int launch_gemm(const QaGemmW8A8Params& p, hipStream_t stream) {
     return launch_one<TM, TN, WGM, WGN, STAGES, QA_OUT_F16, FLEX>(p, stream);
 }
 
-// ---------------------------------------------------------------------------------------------
-// Products of few outputs (the projections of a decode batch or a short prompt): B x B outputs per workgroup, K over its
-// waves, 128 bytes of every row at a time.
-// What bounds them is how fast a CU fetches its operand rows and the trips to memory that wait for each other.  A wave
-// fetches with eight lanes per 128-byte row piece straight to its own part of LDS - eight lines per instruction; the
-// fragments of 16x16x64 fetched into registers directly touch sixteen rows with consecutive lanes, which a CU takes at about
-// 16 bytes a clock - up to DEPTH units ahead; the scales are requested in front of everything else; the waves meet only for
-// their partial sums, which take the fetched units' place in LDS.
-// Eight waves: sixteen are as fast, but need more than the 64 KB that a launch gets by default and that two workgroups of a CU
-// can have.
-// Before, 16 x 16 with fragments fetched into registers by sixteen waves and 32 x 32 staged through registers by four (rows x
-// outputs x K, us): 64 x 192 x 5120 6.7 -> 3.8, 16 x 2560 x 5120 6.9 -> 4.9, 512 x 128 x 3072 4.8 -> 3.6, 64 x 80 x 1536 3.4 -> 3.4
-// (which is a launch); 64 x 2560 x 5120 7.8 -> 6.7, 100 x 1024 x 2048 5.2 -> 3.9, 40 x 3352 x 768 4.0 -> 3.5.  In 64 x 64 outputs a
-// wave's share of K is too little: 64 x 10240 x 2560 7.2 -> 9.7, and the tile kernel above stays.
-// ---------------------------------------------------------------------------------------------
-template <int B, int WAVES, int DEPTH>
-struct SplitCfg {
-    static constexpr int kThreads = 64 * WAVES, kBlocks = B / 16;
-    static constexpr int kRequests = B / 8;                        // per operand and unit
-    static constexpr int kUnit = 2 * B * kBK;                      // a rows, then w rows
-    static constexpr int kOutputs = (B * B + kThreads - 1) / kThreads;         // per thread
-    static constexpr int kRing = WAVES * DEPTH * kUnit, kSums = WAVES * B * B * 4;
-    static constexpr int kLdsBytes = kRing > kSums ? kRing : kSums;
-};
-
-template <int B, int WAVES, int DEPTH, int OUT>
-__global__ __launch_bounds__(64 * WAVES) void gemm_w8a8_split_kernel(QaGemmW8A8Params p) {
-    using C = SplitCfg<B, WAVES, DEPTH>;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int m0, n0;
-    split_tile_of_workgroup<B>(blockIdx.x, p.m, p.n, m0, n0);
-
-    // output o of this thread: element tid + o * kThreads of the blocks' accumulators, 256 each: of lane l, register r row
-    // l % 16 and column 4 (l / 16) + r
-    int mm[C::kOutputs], nn[C::kOutputs];
-    float s_row[C::kOutputs], s_col[C::kOutputs];
-#pragma unroll
-    for (int o = 0; o < C::kOutputs; ++o) {
-        const int t = tid + o * C::kThreads, block = t >> 8;
-        mm[o] = m0 + block / C::kBlocks * 16 + ((t >> 2) & 15);
-        nn[o] = t < B * B ? n0 + block % C::kBlocks * 16 + ((t >> 6) & 3) * 4 + (t & 3) : p.n;
-        s_row[o] = s_col[o] = p.alpha;
-        if (!p.use_alpha && mm[o] < p.m && nn[o] < p.n) {
-            s_row[o] = p.a_scale[p.a_scale_numel == 1 ? 0 : mm[o]];
-            s_col[o] = p.w_scale[p.w_scale_numel == 1 ? 0 : nn[o]];
-        }
-    }
-
-    const v4i rsrc_a = make_rsrc(p.a, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k));
-    const v4i rsrc_w = make_rsrc(p.w, static_cast<int>((static_cast<int64_t>(p.n) - 1) * p.ldw + p.k));
-    TileLoader<C::kRequests> load_a, load_w;
-    load_a.template init<1>(m0, p.m, p.lda, 0, lane);
-    load_w.template init<1>(n0, p.n, p.ldw, 0, lane);
-    uint8_t* const mine = lds + wave * DEPTH * C::kUnit;
-    const uint32_t at = lds_offset_of(mine);
-    const int units = (p.k + kBK - 1) / kBK, my_units = (units - wave + WAVES - 1) / WAVES;       // units wave, wave + WAVES, ...
-    auto issue = [&](int u, int slot) {
-        const int k0 = (wave + u * WAVES) * kBK;
-        load_w.template issue<1>(rsrc_w, k0, p.k, at + slot * C::kUnit + B * kBK, 0);
-        load_a.template issue<1>(rsrc_a, k0, p.k, at + slot * C::kUnit, 0);
-    };
-#pragma unroll
-    for (int u = 0; u < DEPTH; ++u)
-        if (u < my_units) issue(u, u);
-
-    v4i acc[C::kBlocks][C::kBlocks];                       // [rows][columns]
-#pragma unroll
-    for (int i = 0; i < C::kBlocks; ++i)
-#pragma unroll
-        for (int j = 0; j < C::kBlocks; ++j) acc[i][j] = v4i{0, 0, 0, 0};
-    for (int base = 0; base < my_units; base += DEPTH) {
-        static_for<0, DEPTH>([&](auto slot_c) {
-            constexpr int slot = decltype(slot_c)::value;
-            const int u = base + slot;
-            if (u >= my_units) return;
-            if (u + DEPTH <= my_units) __builtin_amdgcn_s_waitcnt(vmcnt_imm((DEPTH - 1) * 2 * C::kRequests));
-            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-            wave_lds_sync();
-            const uint8_t* sa = mine + slot * C::kUnit;
-            v4i fa[2][C::kBlocks], fw[2][C::kBlocks];
-#pragma unroll
-            for (int step = 0; step < 2; ++step) {
-                const int off = (lane & 15) * kBK + swz(lane & 15, 4 * step + (lane >> 4)) * 16;
-#pragma unroll
-                for (int i = 0; i < C::kBlocks; ++i) {
-                    fa[step][i] = *reinterpret_cast<const v4i*>(sa + off + i * 16 * kBK);
-                    fw[step][i] = *reinterpret_cast<const v4i*>(sa + B * kBK + off + i * 16 * kBK);
-                }
-            }
-#pragma unroll
-            for (int step = 0; step < 2; ++step)
-#pragma unroll
-                for (int i = 0; i < C::kBlocks; ++i)
-#pragma unroll
-                    for (int j = 0; j < C::kBlocks; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[step][j], fa[step][i], acc[i][j], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);             // (the fragments are in registers: the slot is free)
-            if (u + DEPTH < my_units) issue(u + DEPTH, slot);
-        });
-    }
-
-    __syncthreads();                                       // every wave is done with its units
-    int* const sums = reinterpret_cast<int*>(lds);
-#pragma unroll
-    for (int i = 0; i < C::kBlocks; ++i)
-#pragma unroll
-        for (int j = 0; j < C::kBlocks; ++j) *reinterpret_cast<v4i*>(&sums[wave * B * B + (i * C::kBlocks + j) * 256 + lane * 4]) = acc[i][j];
-    __syncthreads();
-#pragma unroll
-    for (int o = 0; o < C::kOutputs; ++o) {
-        if (mm[o] >= p.m || nn[o] >= p.n) continue;
-        int sum = 0;
-#pragma unroll
-        for (int x = 0; x < WAVES; ++x) sum += sums[x * B * B + tid + o * C::kThreads];
-        const float accf = static_cast<float>(sum);
-        float v;
-        if (p.use_alpha) v = s_row[o] * accf;
-        else if (p.scale_order) v = s_col[o] * (s_row[o] * accf);
-        else if (p.round_mode == QA_ROUND_HALF_AWAY) v = (s_col[o] * s_row[o]) * accf;      // the rule of single rows
-        else v = s_row[o] * (s_col[o] * accf);
-        asm volatile("" : "+v"(v));                        // the fp32 product is rounded on its own
-        const int64_t to = static_cast<int64_t>(mm[o]) * p.ldd + nn[o];
-        if (OUT == QA_OUT_I8) static_cast<int8_t*>(p.d)[to] = static_cast<int8_t>(quant8(v, p.round_mode));
-        else static_cast<uint16_t*>(p.d)[to] = one_f16_or_bf16<OUT>(v);
-    }
-}
-
-template <int B, int WAVES, int DEPTH>
-int launch_split(const QaGemmW8A8Params& p, hipStream_t stream) {
-    using C = SplitCfg<B, WAVES, DEPTH>;
-    const int64_t blocks = static_cast<int64_t>((p.m + B - 1) / B) * ((p.n + B - 1) / B);
-    auto kernel = p.out_type == QA_OUT_I8 ? gemm_w8a8_split_kernel<B, WAVES, DEPTH, QA_OUT_I8> : p.out_type == QA_OUT_BF16 ? gemm_w8a8_split_kernel<B, WAVES, DEPTH, QA_OUT_BF16> : gemm_w8a8_split_kernel<B, WAVES, DEPTH, QA_OUT_F16>;
-    if (C::kLdsBytes > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, C::kLdsBytes) != hipSuccess) return check_launch();
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(C::kThreads), C::kLdsBytes, stream, p);
-    return check_launch();
+GemvParams as_gemv(const QaGemmW8A8Params& p) {
+    GemvParams g = {};
+    g.m = p.m; g.n = p.n; g.k = p.k; g.bits = 8;
+    g.out_type = p.out_type;
+    g.rule = p.use_alpha ? kGemvAlpha : p.round_mode != QA_ROUND_RNE ? kGemvHalfAway : p.scale_order == 1 ? kGemvColOuter : kGemvRowOuter;
+    g.alpha = p.alpha;
+    g.half_away = p.round_mode != QA_ROUND_RNE;
+    g.row_numel = p.a_scale_numel; g.col_numel = p.w_scale_numel;
+    g.lda = p.lda; g.ldw = p.ldw; g.ldd = p.ldd;
+    g.a = p.a; g.w = p.w; g.row_scale = p.a_scale; g.col_scale = p.w_scale; g.d = p.d;
+    return g;
 }
 
 // Tile of a launch: the smallest whose tiles fit the part in one round.  With at most one tile per CU a launch takes a
-// tile's own time - about 2.5 us and, per 128 bytes of K, 0.04 us (16 x 16, K split over the waves), 0.10 (32 x 32, the same), 0.20 (64 x 64), 0.31
-// (128 x 64), 0.48 (128 x 128, four stages), 0.68 (128 x 256), 1.15 (256 x 256) - so smaller tiles win until a second round
-// starts.  Measured at M 16 .. 16384 with ten of the projections' N and K: this choice is the fastest or
-// within 8 % of it.  Against 128 x 128 tiles up to 192 tiles of 256 x 256 (rows x outputs x K, us): 512 x 80 x 1536 9.6 ->
-// 4.1, 3063 x 192 x 5120 21.0 -> 11.7, 512 x 1536 x 3072 14.6 -> 7.7, 777 x 10240 x 2560 45 -> 38, 6144 x 1536 x 3072 47 -> 35.
+// tile's own time - about 2.5 us and, per 128 bytes of K, 0.20 us (64 x 64), 0.31 (128 x 64), 0.48 (128 x 128, four stages),
+// 0.68 (128 x 256), 1.15 (256 x 256) - so smaller tiles win until a second round starts; below that K split over the waves
+// (gemm_split.hpp) where its cost is the smaller one.  Measured at M 16 .. 16384 with ten of the projections' N and K: this choice is the fastest or
+// within 8 % of it.  Against 128 x 128 tiles up to 192 tiles of 256 x 256 (rows x outputs x K, us): 512 x 1536 x 3072 14.6 ->
+// 7.7, 777 x 10240 x 2560 45 -> 38, 6144 x 1536 x 3072 47 -> 35.
 // From 128 x 64 on a tile is divided over eight waves: a CU that holds one tile then has two waves per SIMD, and one issues
 // while the other waits.  Four waves against eight (us): 1531 x 768 x 1536 6.9 -> 6.3, 1024 x 1536 x 3072 10.2 -> 9.8 with
 // 128 x 64; 3063 x 768 x 1536 9.2 -> 7.8, 1531 x 1536 x 3072 14.0 -> 12.1, 1531 x 2560 x 5120 28.0 -> 27.8 with 128 x 128.
 int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
     const int cus = compute_units();
     auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
-    if (tiles(16, 16) <= cus) return launch_split<16, 8, 2>(p, stream);              // (two rounds of these: slower than one of 32 x 32)
-    if (tiles(32, 32) <= cus) return launch_split<32, 8, 1>(p, stream);
+    const float units = static_cast<float>((p.k + kBK - 1) / kBK);
+    if (tiles(128, 128) <= cus) {
+        const float whole = 2.5f + units * (tiles(64, 64) <= cus ? 0.20f : tiles(128, 64) <= cus ? 0.31f : 0.48f);
+        const SplitChoice split = split_choice(8, p.m, p.n, p.k, cus);
+        if (split.us < whole) return split_launch_w8(as_gemv(p), split.shape, stream);
+    }
     if (tiles(64, 64) <= cus) return launch_gemm<1, 1, 2, 2, 4, false>(p, stream);
     if (tiles(128, 64) <= cus) return launch_gemm<1, 1, 4, 2, 4, false>(p, stream);
     if (tiles(128, 128) <= cus) return launch_gemm<2, 1, 2, 4, 4, false>(p, stream);
@@ -374,19 +254,9 @@ extern "C" int qa_gemm_w8a8(const QaGemmW8A8Params* p, void* stream_) {
     if (static_cast<int64_t>(p->m) * p->lda >= 0x70000000LL || static_cast<int64_t>(p->n) * p->ldw >= 0x70000000LL) return QA_ERR_SHAPE;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const bool flex = p->use_alpha || p->round_mode != QA_ROUND_RNE;
-    if (p->m <= kGemvRows) {
-        GemvParams g = {};
-        g.m = p->m; g.n = p->n; g.k = p->k; g.bits = 8;
-        g.out_type = p->out_type;
-        g.rule = p->use_alpha ? kGemvAlpha : p->round_mode != QA_ROUND_RNE ? kGemvHalfAway : p->scale_order == 1 ? kGemvColOuter : kGemvRowOuter;
-        g.alpha = p->alpha;
-        g.half_away = p->round_mode != QA_ROUND_RNE;
-        g.row_numel = p->a_scale_numel; g.col_numel = p->w_scale_numel;
-        g.lda = p->lda; g.ldw = p->ldw; g.ldd = p->ldd;
-        g.a = p->a; g.w = p->w; g.row_scale = p->a_scale; g.col_scale = p->w_scale; g.d = p->d;
-        return gemv_launch(g, nullptr, stream);
-    }
+    if (gemv_is_faster(p->m, p->n, p->k)) return gemv_launch(as_gemv(*p), nullptr, stream);
     // the single-row rules (host alpha, round-half-away) only ever come with tiny M
-    if (flex) return p->m <= 64 ? launch_split<32, 8, 1>(*p, stream) : launch_gemm<2, 2, 2, 2, 2, true>(*p, stream);
+    if (flex && p->m <= 64) return split_launch_w8(as_gemv(*p), split_choice(8, p->m, p->n, p->k, compute_units()).shape, stream);
+    if (flex) return launch_gemm<2, 2, 2, 2, 2, true>(*p, stream);
     return dispatch_tiles(*p, stream);
 }

@@ -1,9 +1,9 @@
-// Up to eight activation rows against a weight matrix: a stream over the weights.
+// Up to four activation rows against a weight matrix: a stream over the weights.
 //
 // A wave owns four rows of the weight and the whole of K: a lane takes 16 bytes of each row out of every 1024 (int8: 16
 // codes; 4 bits: 32 codes), so a load of the wave is 1 KB in one piece, and the loads of up to five such pieces of all
-// four rows go out before the first is used.  The matrix cores have nothing to give here - a tile of 32 activation rows
-// would be seven eighths or more empty - and their fragments would have to pass through LDS; the products are 4-way int8
+// four rows go out before the first is used.  The matrix cores have nothing to give here - a tile of 16 activation rows
+// would be three quarters or more empty - and their fragments would have to pass through LDS; the products are 4-way int8
 // dot products in the lane that loaded the codes, and LDS is not used at all.  The lanes' partial sums meet through lane
 // swaps (two stages, four values at a time) and row permutes.
 //
@@ -412,13 +412,11 @@ int gemv_launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
     if (p.bits == 8) {
         if (p.m == 1) return pick<8, 1, 4, 2, 2>(p, conv, stream);
         if (p.m == 2) return pick<8, 2, 3, 2, 2>(p, conv, stream);
-        if (p.m <= 4) return pick<8, 4, 3, 2, 2>(p, conv, stream);
-        return pick<8, 8, 2, 2, 2>(p, conv, stream);
+        return pick<8, 4, 3, 2, 2>(p, conv, stream);
     }
     if (p.m == 1) return pick<4, 1, 2, 1, 1>(p, conv, stream);
     if (p.m == 2) return pick<4, 2, 2, 1, 1>(p, conv, stream);
-    if (p.m <= 4) return pick<4, 4, 2, 1, 1>(p, conv, stream);
-    return pick<4, 8, 1, 1, 1>(p, conv, stream);
+    return pick<4, 4, 2, 1, 1>(p, conv, stream);
 }
 
 int gemv_rotated_launch(const GemvParams& p, const GemvRotate& r, hipStream_t stream) {

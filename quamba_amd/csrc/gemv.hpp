@@ -1,10 +1,12 @@
-// Products with very few activation rows (one decode step of a few sequences): see gemv.hip.
+// Products with few activation rows (a decode step): one to four of them in gemv.hip, more in gemm_split.hpp.
 #pragma once
 #include "qa_common.hpp"
 
+#include <algorithm>
+
 namespace qa {
 
-constexpr int kGemvRows = 8;
+constexpr int kGemvRows = 4;
 constexpr int kGemvConvGroups = 8;     // head groups and dim groups of the conv's output scales, at most
 
 enum GemvRule {
@@ -44,6 +46,48 @@ inline bool gemv_conv_ok(const GemvConv& f) {
 }
 
 int gemv_launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream);
+
+// gemm_split_w8.hip, gemm_split_w4.hip: K over the eight waves of a workgroup, in one of these tiles.  What a launch takes, in
+// us with `units` of 128 codes of K, is 2.9 and rounds (of one workgroup per CU) x (fixed + per_unit x units), as measured over
+// 1 .. 200 rows of 80 .. 18560 columns and K from 160 to 8192 with the weights coming from beyond the L2s; the fixed part is
+// the sums of the larger tiles, which all meet at the end (negative: another tile is always the faster one).
+struct SplitShape {
+    int rows, cols;
+    float fixed[2], per_unit[2];       // int8, 4 bits
+};
+constexpr SplitShape kSplitShapes[] = {
+    {16, 16, {0.0f, 0.0f}, {0.045f, 0.045f}}, {16, 32, {0.0f, 0.0f}, {0.07f, 0.075f}},  {16, 48, {0.0f, 0.0f}, {0.1f, 0.115f}},
+    {32, 32, {0.0f, 0.0f}, {0.09f, 0.1f}},    {32, 48, {0.3f, 0.2f}, {0.125f, 0.135f}}, {32, 80, {1.2f, 1.0f}, {0.155f, 0.22f}},
+    {64, 48, {-1.0f, 1.6f}, {0.0f, 0.165f}}, {64, 80, {2.6f, 2.5f}, {0.2f, 0.31f}},
+};
+struct SplitChoice {
+    int shape;
+    float us;
+};
+inline SplitChoice split_choice(int bits, int m, int n, int k, int cus) {
+    SplitChoice best = {-1, 1e30f};
+    for (int i = 0; i < static_cast<int>(sizeof(kSplitShapes) / sizeof(kSplitShapes[0])); ++i) {
+        const SplitShape& s = kSplitShapes[i];
+        if (s.fixed[bits == 4] < 0.0f) continue;
+        const int64_t tiles = static_cast<int64_t>((m + s.rows - 1) / s.rows) * ((n + s.cols - 1) / s.cols);
+        const float rounds = static_cast<float>((tiles + cus - 1) / cus), units = static_cast<float>((k + 127) / 128);
+        const float us = 2.9f + rounds * (s.fixed[bits == 4] + s.per_unit[bits == 4] * units);
+        if (tiles <= 0x7fffffff && us < best.us) best = {i, us};
+    }
+    return best;
+}
+// Operands as the products' entry points take them (16-byte aligned rows; K a multiple of 16, or of 128 with 4 bits; with 8
+// bits every offset below 2^31).  4 bits: a tile's rows and the group scales (null: per channel) are addressed with 32 bits.
+inline bool split_addressable_w4(int n, int k) { return 40LL * k <= 0x7fffffffLL && static_cast<int64_t>(n) * (k / 128) < 1 << 29; }
+int split_launch_w8(const GemvParams& p, int shape, hipStream_t stream);
+int split_launch_w4(const GemvParams& p, int shape, hipStream_t stream);
+
+// Which of the two a product of up to kGemvRows rows takes.  A row is work for the vector units in gemv.hip and free in a
+// block of sixteen here: one and two rows there, three and four only where the outputs are so few that the split leaves the
+// waves a long K each (us at 1 / 2 / 3 rows, gemv against split: int8 10240 x 2560 5.8 / 6.1 / 6.8 against 6.3, 192 x 5120 3.0 /
+// 3.1 / 3.1 against 3.6; 4 bits 10240 x 2560 5.7 / 6.4 / 7.5 against 5.4, 4096 x 8192 5.5 / 6.2 / 7.4 against 6.9, 192 x 5120 3.1 /
+// 3.1 / 3.2 against 4.4; at five to eight rows, where it takes twice the registers, 9.1 and 10.0 against 6.3 and 5.4).
+inline bool gemv_is_faster(int m, int n, int k) { return m <= 2 || (m <= kGemvRows && n <= 512 && k > 2048); }
 
 // One activation row that is made on the spot: sat8(round_half_away(H y * had_scale)) of a row y of k fp16 values
 // (qa_hadamard_quant); fp16 results.  QA_ERR_UNSUPPORTED: not for these sizes (the caller then makes the two calls).

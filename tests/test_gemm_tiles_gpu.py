@@ -38,24 +38,56 @@ def test_int8_weights(dev, M, N, K, order):
     np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
-# 16 x 16 tiles: one k step and part of one, more units of K than a wave takes at once, rows and columns with remainders, the
-# largest number of tiles (and one more: 32 x 32)
+# K over the waves, 16 x 16 and 32 x 32 outputs: one k step and part of one, a ring of units that goes round, rows and columns
+# with remainders
 @pytest.mark.parametrize("M,N,K", [(9, 5, 16), (17, 33, 80), (16, 48, 6160), (100, 30, 12304), (256, 250, 144), (257, 250, 144)])
 @pytest.mark.parametrize("order", [0, 1])
 def test_int8_weights_of_few_outputs(dev, M, N, K, order):
     test_int8_weights(dev, M, N, K, order)
 
 
-# K over the waves of a workgroup, 16 x 16 and 32 x 32 outputs: fewer 128-byte units of K than waves, one each, one more, the
-# ring of two units round several times, all with and without a remainder of K
-@pytest.mark.parametrize("M,N", [(9, 200), (20, 1000), (70, 1900)])
-@pytest.mark.parametrize("K", [16, 128, 1008, 1024, 1040, 2048, 2064, 3200, 4112])
+# K over the waves of a workgroup: fewer 128-byte units of K than waves, one each, one more, the ring of two units round several
+# times, all with and without a remainder of K; then every other tile, at the K where the dispatch takes it
+@pytest.mark.parametrize("M,N,K", [(m, n, k) for m, n in [(9, 200), (20, 1000), (70, 1900)] for k in (16, 128, 1008, 1024, 1040, 2048, 2064, 3200, 4112)] +
+                         [(16, 4201, 2192), (3, 12210, 2176), (64, 6001, 2192), (200, 2510, 2176), (61, 18500, 2064)])
 @pytest.mark.parametrize("order,dtype", [(0, torch.int8), (1, torch.int8), (0, torch.float16), (0, torch.bfloat16)])
 def test_k_split_over_the_waves(dev, M, N, K, order, dtype):
     test_large_tiles_over_a_long_k(dev, M, N, K, order, dtype)
 
 
-# 32 x 32 with four and eight waves, 64 x 64, 64 x 128, 128 x 128, 192 x 128, expanded once
+# the same with 4-bit weights, groups of 128 and one scale per channel; an odd number of columns, group scales two bytes off a word
+@pytest.mark.parametrize("M,N,K", [(9, 200, 128), (9, 201, 1024), (33, 500, 1152), (20, 1000, 4352), (16, 4201, 2176), (3, 12210, 2176), (70, 1900, 1280),
+                                   (64, 6001, 2176), (30, 20001, 2176), (61, 10201, 2176), (64, 18500, 2048), (130, 60, 2176)])
+@pytest.mark.parametrize("grouped", [True, False])
+@pytest.mark.parametrize("dtype", [torch.int8, torch.float16])
+def test_k_split_over_the_waves_with_4_bits(dev, M, N, K, grouped, dtype):
+    """Codes times a group scale are exact in fp32, so rounding them there is the single rounding of the expansion."""
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    a = torch.randint(-128, 128, (M, K), dtype=torch.int8, device=dev, generator=g)
+    codes = torch.randint(0, 16, (N, K), dtype=torch.uint8, device=dev, generator=g)
+    words = codes.view(N, K // 8, 2, 4)
+    packed = (words[:, :, 0] | words[:, :, 1] << 4).reshape(N, K // 2).contiguous()
+    scales = torch.empty(K // 128 * N + 1, dtype=torch.float16, device=dev)
+    sg = scales[1:].view(K // 128, N)
+    sg.copy_(torch.rand(sg.shape, device=dev, generator=g) * 13 + 2)
+    if grouped:
+        w8 = ((codes.float() - 8) * sg.t().float().repeat_interleave(128, 1)).round().double()
+    else:
+        w8 = (codes.to(torch.int8) << 4).double()
+    sc, st = (torch.rand(N, device=dev, generator=g) + 0.5) * 0.006 / K ** 0.5, torch.rand(M, device=dev, generator=g) + 0.5
+    v = st[:, None] * (sc * (a.double() @ w8.t()).float())
+    want = v.round().clamp(-128, 127).to(torch.int8) if dtype == torch.int8 else v.half()
+    got = torch.empty((M, N), dtype=dtype, device=dev)
+    p = _lib.QaGemmW4A8Params()
+    p.m, p.n, p.k, p.tok_scale_numel, p.group_size, p.lda, p.ldd = M, N, K, M, 128 if grouped else -1, K, N
+    p.out_type = _lib.QA_OUT_I8 if dtype == torch.int8 else _lib.QA_OUT_F16
+    p.a, p.w_packed, p.s_channel, p.s_token, p.d = (t.data_ptr() for t in (a, packed, sc, st, got))
+    p.s_group = sg.data_ptr() if grouped else None
+    _lib.check(_lib.lib().qa_gemm_w4a8(ctypes.byref(p), _lib.current_stream(dev)), "gemm_w4a8")
+    assert torch.equal(got, want)
+
+
+# K over the waves, 64 x 64, 64 x 128, 128 x 128, 192 x 128, expanded once
 @pytest.mark.parametrize("M,N,K,workspace", [(70, 200, 2176, False), (100, 1000, 384, False), (130, 2050, 1664, False), (250, 2500, 1152, False),
                                              (600, 2100, 256, False), (300, 4200, 1664, False), (70, 9000, 128, False), (700, 3100, 1152, False),
                                              (900, 6100, 128, False), (950, 6100, 896, False), (4000, 3300, 1664, False), (4000, 3300, 1664, True)])
