@@ -190,56 +190,17 @@ __global__ __launch_bounds__(kThreads) void conv2_update_kernel(QaConv2Params p)
     out[0] = conv_epilogue(v, out_scale_of(p, part, ch), p.silu_activation);
 }
 
-// The single-step update of four neighbouring channels per lane, for words in every operand: four taps a channel back to
-// back, inputs and outputs with unit channel stride, and a state that is either channel-contiguous (a word per step: the
-// Mamba2 layer's buffer) or four codes a channel (a 16-byte piece: the Mamba1 layer's).  grid: x quads of channels, y batch.
+// The single-step update of four neighbouring channels per lane.  grid: x quads of channels, y batch.
 template <bool CHANNEL_ROWS>
 __global__ __launch_bounds__(kThreads) void conv2_update4_kernel(QaConv2Params p) {
     const int ch0 = (blockIdx.x * kThreads + threadIdx.x) * 4, b = blockIdx.y;
     if (ch0 >= p.dim) return;
-    int8_t* st = p.conv_state + b * p.conv_state_batch_stride + ch0 * p.conv_state_c_stride;
     const uint32_t x_new = *reinterpret_cast<const uint32_t*>(p.xBC + b * p.xBC_batch_stride + ch0);
-    const uint4 w = *reinterpret_cast<const uint4*>(p.weight + ch0 * 4);
-    const uint32_t taps[4] = {w.x, w.y, w.z, w.w};
-    const uint32_t b4 = p.bias ? *reinterpret_cast<const uint32_t*>(p.bias + ch0) : 0u;
-    uint32_t win[4];                                              // byte j of win[e]: input t - 3 + j of channel ch0 + e
-    if constexpr (CHANNEL_ROWS) {
-        const int drop = p.conv_state_len - 3;
-        uint32_t d[4];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) d[i] = *reinterpret_cast<const uint32_t*>(st + (drop + i) * p.conv_state_l_stride);
-        d[3] = x_new;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (i >= 4 - p.conv_state_len) *reinterpret_cast<uint32_t*>(st + (i - (4 - p.conv_state_len)) * p.conv_state_l_stride) = d[i];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t pick = 0x0c0c0000u | ((4u + e) << 8) | e;     // byte e of two words, side by side
-            win[e] = __builtin_amdgcn_perm(d[1], d[0], pick) | (__builtin_amdgcn_perm(d[3], d[2], pick) << 16);
-        }
-    } else {
-        const uint4 h = *reinterpret_cast<const uint4*>(st);
-        const uint32_t held[4] = {h.x, h.y, h.z, h.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) win[e] = (held[e] >> 8) | (((x_new >> (8 * e)) & 0xffu) << 24);
-        *reinterpret_cast<uint4*>(st) = make_uint4(win[0], win[1], win[2], win[3]);
-    }
+    const ConvHeld<CHANNEL_ROWS> held = conv_held4<CHANNEL_ROWS>(p, b, ch0);
     const Part part = part_of(p, ch0);
-    float s_out[4], inv_s_out[4], v[4];
-    bool exact_only[4];
-    out_scales4_of(p, part, ch0, s_out);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        inv_s_out[e] = 1.0f / s_out[e];
-        exact_only[e] = conv_needs_exact_route(s_out[e]);
-        v[e] = part.s_bias * static_cast<float>(static_cast<int8_t>(b4 >> (8 * e)));
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            v[e] = __builtin_fmaf(part.s_in * static_cast<float>(static_cast<int8_t>(taps[e] >> (8 * i))), static_cast<float>(static_cast<int8_t>(win[e] >> (8 * i))), v[e]);
-    }
-    const ConvQuantRegs kq(__builtin_fminf(__builtin_fminf(s_out[0], s_out[1]), __builtin_fminf(s_out[2], s_out[3])));
+    const ConvQuad quad = conv_quad(p, part, ch0);
     int64_t out_ls, out_cs;
-    *reinterpret_cast<uint32_t*>(out_ptr(p, part, b, ch0, &out_ls, &out_cs)) = conv_quant4(v, s_out, inv_s_out, p.silu_activation, exact_only, kq);
+    *reinterpret_cast<uint32_t*>(out_ptr(p, part, b, ch0, &out_ls, &out_cs)) = conv_step4<CHANNEL_ROWS>(p, b, ch0, part, quad, held, x_new);
 }
 
 int validate(const QaConv2Params* p, bool update) {
@@ -291,19 +252,13 @@ int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
 
 namespace qa {
 int conv_single_update(const QaConv2Params& p, hipStream_t stream) {
-    auto mult4 = [](int64_t v) { return v % 4 == 0; };
-    const int64_t bc = static_cast<int64_t>(p.d_state) * p.n_groups;
-    const bool all_x = p.x_dim == p.dim;                          // (the Mamba1 conv: no B and C parts)
-    const bool words = p.width == 4 && p.weight_width_stride == 1 && p.weight_c_stride == 4 && aligned16(p.weight) && aligned4(p.bias) &&
-                       p.xBC_c_stride == 1 && mult4(p.xBC_batch_stride) && aligned4(p.xBC) && mult4(p.x_dim) && (all_x || mult4(bc)) &&
-                       p.x_c_stride == 1 && mult4(p.x_batch_stride) && aligned4(p.x) &&
-                       (all_x || (p.B_c_stride == 1 && mult4(p.B_batch_stride) && aligned4(p.B) && p.C_c_stride == 1 && mult4(p.C_batch_stride) && aligned4(p.C)));
+    const bool words = conv_words_ok(p) && p.xBC_c_stride == 1 && p.xBC_batch_stride % 4 == 0 && aligned4(p.xBC);
     const dim3 grid4(static_cast<unsigned>((p.dim / 4 + kThreads - 1) / kThreads), static_cast<unsigned>(p.batch));
-    if (words && p.conv_state_c_stride == 1 && mult4(p.conv_state_l_stride) && mult4(p.conv_state_batch_stride) && aligned4(p.conv_state)) {
+    if (words && conv_state_in_rows(p)) {
         hipLaunchKernelGGL(conv2_update4_kernel<true>, grid4, dim3(kThreads), 0, stream, p);
         return check_launch();
     }
-    if (words && p.conv_state_len == 4 && p.conv_state_l_stride == 1 && p.conv_state_c_stride == 4 && p.conv_state_batch_stride % 16 == 0 && aligned16(p.conv_state)) {
+    if (words && conv_state_in_words(p)) {
         hipLaunchKernelGGL(conv2_update4_kernel<false>, grid4, dim3(kThreads), 0, stream, p);
         return check_launch();
     }

@@ -111,4 +111,85 @@ __device__ __forceinline__ int8_t* out_ptr(const QaConv2Params& p, const Part& p
     return p.C + b * p.C_batch_stride + local * p.C_c_stride;
 }
 
+// The single-step update of four neighbouring channels of a part, for words in every operand: four taps a channel back to
+// back, inputs and outputs with unit channel stride, and a state that is either channel-contiguous (a word per step: the
+// Mamba2 layer's buffer) or four codes a channel (a 16-byte piece: the Mamba1 layer's).
+struct ConvQuad {
+    uint32_t taps[4], bias;            // bias: four codes (zero without one)
+    float s_out[4];
+};
+__device__ __forceinline__ ConvQuad conv_quad(const QaConv2Params& p, const Part& part, int ch0) {
+    ConvQuad q;
+    const uint4 w = *reinterpret_cast<const uint4*>(p.weight + ch0 * 4);
+    q.taps[0] = w.x; q.taps[1] = w.y; q.taps[2] = w.z; q.taps[3] = w.w;
+    q.bias = p.bias ? *reinterpret_cast<const uint32_t*>(p.bias + ch0) : 0u;
+    out_scales4_of(p, part, ch0, q.s_out);
+    return q;
+}
+// the state, as loaded: a word per step of the three that the window keeps, or a word per channel
+template <bool CHANNEL_ROWS>
+struct ConvHeld {
+    uint32_t w[CHANNEL_ROWS ? 3 : 4];
+};
+template <bool CHANNEL_ROWS>
+__device__ __forceinline__ ConvHeld<CHANNEL_ROWS> conv_held4(const QaConv2Params& p, int b, int ch0) {
+    const int8_t* st = p.conv_state + b * p.conv_state_batch_stride + ch0 * p.conv_state_c_stride;
+    ConvHeld<CHANNEL_ROWS> h;
+    if constexpr (CHANNEL_ROWS) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) h.w[i] = *reinterpret_cast<const uint32_t*>(st + (p.conv_state_len - 3 + i) * p.conv_state_l_stride);
+    } else {
+        const uint4 v = *reinterpret_cast<const uint4*>(st);
+        h.w[0] = v.x; h.w[1] = v.y; h.w[2] = v.z; h.w[3] = v.w;
+    }
+    return h;
+}
+// x_new: the new inputs, a byte per channel.  The state moves on; returns the four outputs.
+template <bool CHANNEL_ROWS>
+__device__ __forceinline__ uint32_t conv_step4(const QaConv2Params& p, int b, int ch0, const Part& part, const ConvQuad& q, const ConvHeld<CHANNEL_ROWS>& h, uint32_t x_new) {
+    int8_t* st = p.conv_state + b * p.conv_state_batch_stride + ch0 * p.conv_state_c_stride;
+    uint32_t win[4];                                              // byte j of win[e]: input t - 3 + j of channel ch0 + e
+    if constexpr (CHANNEL_ROWS) {
+        const uint32_t d[4] = {h.w[0], h.w[1], h.w[2], x_new};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (i >= 4 - p.conv_state_len) *reinterpret_cast<uint32_t*>(st + (i - (4 - p.conv_state_len)) * p.conv_state_l_stride) = d[i];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t pick = 0x0c0c0000u | ((4u + e) << 8) | e;     // byte e of two words, side by side
+            win[e] = __builtin_amdgcn_perm(d[1], d[0], pick) | (__builtin_amdgcn_perm(d[3], d[2], pick) << 16);
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) win[e] = (h.w[e] >> 8) | (((x_new >> (8 * e)) & 0xffu) << 24);
+        *reinterpret_cast<uint4*>(st) = make_uint4(win[0], win[1], win[2], win[3]);
+    }
+    float inv_s_out[4], v[4];
+    bool exact_only[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        inv_s_out[e] = p.silu_activation ? 0.0f : 1.0f / q.s_out[e];     // (SiLU divides by both at once)
+        exact_only[e] = conv_needs_exact_route(q.s_out[e]);
+        v[e] = part.s_bias * static_cast<float>(static_cast<int8_t>(q.bias >> (8 * e)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            v[e] = __builtin_fmaf(part.s_in * static_cast<float>(static_cast<int8_t>(q.taps[e] >> (8 * i))), static_cast<float>(static_cast<int8_t>(win[e] >> (8 * i))), v[e]);
+    }
+    const ConvQuantRegs kq(__builtin_fminf(__builtin_fminf(q.s_out[0], q.s_out[1]), __builtin_fminf(q.s_out[2], q.s_out[3])));
+    return conv_quant4(v, q.s_out, inv_s_out, p.silu_activation, exact_only, kq);
+}
+// the layouts these take: words everywhere but in the state and in the inputs ...
+inline bool conv_words_ok(const QaConv2Params& p) {
+    auto mult4 = [](int64_t v) { return v % 4 == 0; };
+    return p.width == 4 && p.weight_width_stride == 1 && p.weight_c_stride == 4 && aligned16(p.weight) && aligned4(p.bias) && mult4(p.x_dim) &&
+           p.x_c_stride == 1 && mult4(p.x_batch_stride) && aligned4(p.x) &&
+           (p.x_dim == p.dim ||                                   // (the Mamba1 conv: no B and C parts)
+            (mult4(static_cast<int64_t>(p.d_state) * p.n_groups) && p.B_c_stride == 1 && mult4(p.B_batch_stride) && aligned4(p.B) && p.C_c_stride == 1 && mult4(p.C_batch_stride) && aligned4(p.C)));
+}
+// ... and the two layouts of the state
+inline bool conv_state_in_rows(const QaConv2Params& p) { return p.conv_state_c_stride == 1 && p.conv_state_l_stride % 4 == 0 && p.conv_state_batch_stride % 4 == 0 && aligned4(p.conv_state); }
+inline bool conv_state_in_words(const QaConv2Params& p) {
+    return p.conv_state_len == 4 && p.conv_state_l_stride == 1 && p.conv_state_c_stride == 4 && p.conv_state_batch_stride % 16 == 0 && aligned16(p.conv_state);
+}
+
 }  // namespace qa

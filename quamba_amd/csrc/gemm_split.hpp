@@ -17,7 +17,11 @@
 // 64 x 4096 x 8192 12.3 -> 9.3, 24 x 10240 x 2560 9.7 -> 6.4, 64 x 18560 x 4096 18.6 -> 16.6.  What is left of a small one is the
 // launch (2.9); the large ones wait for their units, of which a CU holds 100 KB at a time (int8 64 x 10240 x 2560: 64 x 64
 // tiles that stream K past one ring take 7.2, 64 x 48 of these 9.4).
+//
+// With a conv behind the product (GemvConv) a thread that has the new inputs of four channels makes their conv step as well:
+// the state arrives during the product, and a launch and a round trip through memory are saved.
 #pragma once
+#include "conv2_common.hpp"
 #include "gemm_core.hpp"
 #include "gemv.hpp"
 #include "w4_expand.hpp"
@@ -40,14 +44,18 @@ struct Cfg {
     static constexpr int kRing = kWaves * DEPTH * kUnit, kSums = kWaves * kPassRows * kPitch * 4;
     static constexpr int kColScales = (BN + 63) / 64 * 64, kRowScales = 64;
     static constexpr int kScalesAt = kRing > kSums ? kRing : kSums;
-    static constexpr int kLdsBytes = kScalesAt + (kColScales + kRowScales) * 4;
-    static_assert(BM <= 64 && kLdsBytes <= 160 * 1024, "tile shape");
+    static constexpr int kColumnsAt = kScalesAt + (kColScales + kRowScales) * 4;
+    static constexpr int kLdsBytes = kColumnsAt + BN / 4 * static_cast<int>(sizeof(ConvQuad));
+    static constexpr int kQuads = (kPass / 4 + kThreads - 1) / kThreads;               // of outputs in a pass, per thread
+    static_assert(BM <= 64 && BN <= 256 && kLdsBytes <= 160 * 1024, "tile shape");
 };
 
-template <int BITS, int BM, int BN, int DEPTH, int OUT>
-__global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_split_kernel(GemvParams p) {
+enum ConvKind { kNoConv, kConvWords, kConvRows };       // the layouts of the conv's state (conv_state_in_words, conv_state_in_rows)
+
+template <int BITS, int BM, int BN, int DEPTH, int OUT, ConvKind CONV>
+__global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_split_kernel(GemvParams p, GemvConv f) {
     using C = Cfg<BITS, BM, BN, DEPTH>;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[C::kLdsBytes];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int m0, n0;
     split_tile_of_workgroup<BM, BN>(blockIdx.x, p.m, p.n, m0, n0);
@@ -114,6 +122,26 @@ __global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_spl
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u)
         if (u < my_units) issue(u, u);
+
+    // With a conv a thread finishes four neighbouring outputs at a time: quad t = tid + q * kThreads of a pass, row t / (BN / 4).
+    // The conv state of its row and channels is on its way from here on.
+    ConvHeld<CONV == kConvRows> held[CONV ? C::kPasses : 1][CONV ? C::kQuads : 1];
+    ConvQuad* const quads = reinterpret_cast<ConvQuad*>(lds + C::kColumnsAt);
+    auto is_conv = [&](int n) { return n >= f.ch0 && n < f.ch0 + f.conv.dim; };
+    if constexpr (CONV != kNoConv) {
+        const QaConv2Params& c = f.conv;
+#pragma unroll
+        for (int i = 0; i < C::kPasses; ++i)
+#pragma unroll
+            for (int q = 0; q < C::kQuads; ++q) {
+                // (columns and rows that are not the conv's read some that are)
+                const int t = tid + q * C::kThreads, ch = min(max(n0 + t % (BN / 4) * 4 - f.ch0, 0), c.dim - 4);
+                held[i][q] = conv_held4<CONV == kConvRows>(c, min(m0 + C::kPassRows * i + t / (BN / 4), p.m - 1), ch);
+            }
+        // the columns' taps and scales (a chain of loads), by the last wave, which has the fewest units
+        const int quad = tid - (C::kThreads - 64), n = n0 + 4 * quad;
+        if (quad >= 0 && quad < BN / 4 && is_conv(n)) quads[quad] = conv_quad(c, part_of(c, n - f.ch0), n - f.ch0);
+    }
 
     v4i acc[C::kRowBlocks][C::kColBlocks];
 #pragma unroll
@@ -191,13 +219,7 @@ __global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_spl
             for (int b = 0; b < C::kColBlocks; ++b)
                 *reinterpret_cast<v4i*>(&sums[(wave * C::kPassRows + r * 16 + frow) * C::kPitch + b * 16 + 4 * quarter]) = acc[i * (C::kPassRows / 16) + r][b];
         __syncthreads();
-#pragma unroll
-        for (int o = 0; o < C::kOutputs; ++o) {
-            const int t = tid + o * C::kThreads, row = t / BN, col = t % BN, m = m0 + C::kPassRows * i + row, n = n0 + col;
-            if (t >= C::kPass || m >= p.m || n >= p.n) continue;
-            int sum = 0;
-#pragma unroll
-            for (int x = 0; x < C::kWaves; ++x) sum += sums[(x * C::kPassRows + row) * C::kPitch + col];
+        auto scaled = [&](int sum, int row, int col) {
             const float accf = static_cast<float>(sum), sr = s_row[C::kPassRows * i + row], sc = s_col[col];
             float y;
             if (p.rule == kGemvAlpha) y = p.alpha * accf;
@@ -205,6 +227,37 @@ __global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_spl
             else if (p.rule == kGemvHalfAway) y = (sc * sr) * accf;
             else y = sr * (sc * accf);
             asm volatile("" : "+v"(y));                            // the fp32 product is rounded on its own
+            return y;
+        };
+        if constexpr (CONV != kNoConv) {
+#pragma unroll
+            for (int q = 0; q < C::kQuads; ++q) {
+                const int t = tid + q * C::kThreads, row = t / (BN / 4), quad = t % (BN / 4), m = m0 + C::kPassRows * i + row, n = n0 + 4 * quad;
+                if (t >= C::kPass / 4 || m >= p.m || n >= p.n) continue;
+                v4i sum = {0, 0, 0, 0};
+#pragma unroll
+                for (int x = 0; x < C::kWaves; ++x) sum += *reinterpret_cast<const v4i*>(&sums[(x * C::kPassRows + row) * C::kPitch + 4 * quad]);
+                uint32_t word = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) word |= static_cast<uint32_t>(quant8(scaled(sum[e], row, 4 * quad + e), QA_ROUND_RNE) & 0xff) << (8 * e);
+                if (!is_conv(n)) {
+                    *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(p.d) + m * p.ldd + n) = word;
+                    continue;
+                }
+                const Part part = part_of(f.conv, n - f.ch0);
+                int64_t ls, cs;
+                *reinterpret_cast<uint32_t*>(out_ptr(f.conv, part, m, n - f.ch0, &ls, &cs)) = conv_step4<CONV == kConvRows>(f.conv, m, n - f.ch0, part, quads[quad], held[i][q], word);
+            }
+            continue;
+        }
+#pragma unroll
+        for (int o = 0; o < C::kOutputs; ++o) {
+            const int t = tid + o * C::kThreads, row = t / BN, col = t % BN, m = m0 + C::kPassRows * i + row, n = n0 + col;
+            if (t >= C::kPass || m >= p.m || n >= p.n) continue;
+            int sum = 0;
+#pragma unroll
+            for (int x = 0; x < C::kWaves; ++x) sum += sums[(x * C::kPassRows + row) * C::kPitch + col];
+            const float y = scaled(sum, row, col);
             if constexpr (OUT == QA_OUT_I8) {
                 static_cast<int8_t*>(p.d)[m * p.ldd + n] = static_cast<int8_t>(quant8(y, p.half_away ? QA_ROUND_HALF_AWAY : QA_ROUND_RNE));
             } else {
@@ -215,30 +268,29 @@ __global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_spl
 }
 
 template <int BITS, int BM, int BN, int DEPTH>
-int launch(const GemvParams& p, hipStream_t stream) {
+int launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
     using C = Cfg<BITS, BM, BN, DEPTH>;
     const int64_t blocks = static_cast<int64_t>((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
-    auto kernel = gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8>;
-    if (p.out_type == QA_OUT_F16) kernel = gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_F16>;
-    else if constexpr (BITS == 8) { if (p.out_type == QA_OUT_BF16) kernel = gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_BF16>; }
-    // (allowing more than 64 KiB of dynamic LDS is a per-function attribute; setting it is idempotent)
-    if (C::kLdsBytes > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, C::kLdsBytes) != hipSuccess) return check_launch();
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(C::kThreads), C::kLdsBytes, stream, p);
+    auto kernel = gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8, kNoConv>;
+    if (conv) kernel = conv_state_in_words(conv->conv) ? gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8, kConvWords> : gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8, kConvRows>;
+    else if (p.out_type == QA_OUT_F16) kernel = gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_F16, kNoConv>;
+    else if constexpr (BITS == 8) { if (p.out_type == QA_OUT_BF16) kernel = gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_BF16, kNoConv>; }
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(C::kThreads), 0, stream, p, conv ? *conv : GemvConv{});
     return check_launch();
 }
 
 // the tile shapes in the order of kSplitShapes
 template <int BITS>
-int launch_shape(const GemvParams& p, int shape, hipStream_t stream) {
+int launch_shape(const GemvParams& p, int shape, const GemvConv* conv, hipStream_t stream) {
     switch (shape) {
-        case 0: return launch<BITS, 16, 16, 2>(p, stream);
-        case 1: return launch<BITS, 16, 32, 1>(p, stream);
-        case 2: return launch<BITS, 16, 48, 1>(p, stream);
-        case 3: return launch<BITS, 32, 32, 1>(p, stream);
-        case 4: return launch<BITS, 32, 48, 1>(p, stream);
-        case 5: return launch<BITS, 32, 80, 1>(p, stream);
-        case 6: if constexpr (BITS == 4) return launch<BITS, 64, 48, 1>(p, stream); else break;
-        case 7: return launch<BITS, 64, 80, 1>(p, stream);
+        case 0: return launch<BITS, 16, 16, 2>(p, conv, stream);
+        case 1: return launch<BITS, 16, 32, 1>(p, conv, stream);
+        case 2: return launch<BITS, 16, 48, 1>(p, conv, stream);
+        case 3: return launch<BITS, 32, 32, 1>(p, conv, stream);
+        case 4: return launch<BITS, 32, 48, 1>(p, conv, stream);
+        case 5: return launch<BITS, 32, 80, 1>(p, conv, stream);
+        case 6: if constexpr (BITS == 4) return launch<BITS, 64, 48, 1>(p, conv, stream); else break;
+        case 7: return launch<BITS, 64, 80, 1>(p, conv, stream);
     }
     return QA_ERR_UNSUPPORTED;
 }

@@ -2,5 +2,5 @@
 #include "gemm_split.hpp"
 
 namespace qa {
-int split_launch_w4(const GemvParams& p, int shape, hipStream_t stream) { return split::launch_shape<4>(p, shape, stream); }
+int split_launch_w4(const GemvParams& p, int shape, const GemvConv* conv, hipStream_t stream) { return split::launch_shape<4>(p, shape, conv, stream); }
 }  // namespace qa

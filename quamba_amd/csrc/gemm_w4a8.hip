@@ -587,29 +587,41 @@ __global__ __launch_bounds__(256) void w4_expand_kernel(QaGemmW4A8Params p, int8
 // their tiles - large ones expand each code fewer times, small ones spread over the chip earlier - and the weights expanded
 // once, in a pass of their own, cost that pass.
 enum Way { kWaySplit, kWay64x64, kWay64x128, kWay128x128, kWay192x128, kWayExpandOnce };
+struct WayChoice {
+    int way;
+    double us;
+    void offer(int w, double cost) {
+        if (cost < us) *this = {w, cost};
+    }
+};
+
+WayChoice cheapest_tile(int m, int n, int k, int cus) {
+    const double k_tiles = k / 128;
+    auto rounds = [&](int64_t bm, int64_t bn) { return static_cast<double>((((m + bm - 1) / bm) * ((n + bn - 1) / bn) + cus - 1) / cus); };
+    WayChoice best = {kWay128x128, 1e30};
+    best.offer(kWay64x64, 3.0 + k_tiles * (0.10 + 0.28 * rounds(64, 64)));
+    best.offer(kWay64x128, 3.0 + k_tiles * (0.08 + 0.42 * rounds(64, 128)));
+    best.offer(kWay128x128, 3.0 + k_tiles * std::max(0.73, 0.10 + 0.57 * rounds(128, 128)));
+    best.offer(kWay192x128, 3.0 + k_tiles * (0.05 + 0.84 * rounds(192, 128)));
+    return best;
+}
 
 int cheapest_way(const QaGemmW4A8Params& p, int cus, const SplitChoice& split, bool expandable) {
-    const double k_tiles = p.k / 128;
-    auto rounds = [&](int64_t bm, int64_t bn) { return static_cast<double>((tiles_of(p, bm, bn) + cus - 1) / cus); };
-    double best = 1e30;
-    int way = kWay128x128;
-    auto offer = [&](int w, double cost) {
-        if (cost < best) { best = cost; way = w; }
-    };
-    if (split.shape >= 0) offer(kWaySplit, split.us);
-    offer(kWay64x64, 3.0 + k_tiles * (0.10 + 0.28 * rounds(64, 64)));
-    offer(kWay64x128, 3.0 + k_tiles * (0.08 + 0.42 * rounds(64, 128)));
-    offer(kWay128x128, 3.0 + k_tiles * std::max(0.73, 0.10 + 0.57 * rounds(128, 128)));
-    offer(kWay192x128, 3.0 + k_tiles * (0.05 + 0.84 * rounds(192, 128)));
+    WayChoice best = cheapest_tile(p.m, p.n, p.k, cus);
+    if (split.shape >= 0) best.offer(kWaySplit, split.us);
     if (expandable) {
         // (the int8 x int8 kernel takes the smallest tile that fits one round, see there)
+        auto rounds = [&](int64_t bm, int64_t bn) { return static_cast<double>((tiles_of(p, bm, bn) + cus - 1) / cus); };
         const double step = rounds(64, 64) <= 1 ? 0.25 : rounds(128, 64) <= 1 ? 0.33 : rounds(128, 128) <= 1 ? 0.50 : rounds(128, 256) <= 1 ? 0.75 : 1.55 * rounds(256, 256);
-        offer(kWayExpandOnce, 2.5 + static_cast<double>(p.n) * p.k / 3.1e6 + 5.0 + step * k_tiles);
+        best.offer(kWayExpandOnce, 2.5 + static_cast<double>(p.n) * p.k / 3.1e6 + 5.0 + step * (p.k / 128));
     }
-    return way;
+    return best.way;
 }
 
 }  // namespace
+
+float tiles_us_w4(int m, int n, int k, int cus) { return static_cast<float>(cheapest_tile(m, n, k, cus).us); }
+
 }  // namespace qa
 
 extern "C" int qa_gemm_w4a8(const QaGemmW4A8Params* p, void* stream_) {
@@ -645,7 +657,7 @@ extern "C" int qa_gemm_w4a8(const QaGemmW4A8Params* p, void* stream_) {
         if (gemv_is_faster(p->m, p->n, p->k) && g.s_group && p->n % 4 == 0 && (reinterpret_cast<uintptr_t>(p->s_group) & 7u) == 0) return gemv_launch(g, nullptr, stream);
         const SplitChoice split = split_addressable_w4(p->n, p->k) ? split_choice(4, p->m, p->n, p->k, cus) : SplitChoice{-1, 0.0f};
         const int way = cheapest_way(*p, cus, split, expandable);
-        if (way == kWaySplit) return split_launch_w4(g, split.shape, stream);
+        if (way == kWaySplit) return split_launch_w4(g, split.shape, nullptr, stream);
         if (way == kWay64x64) return p->out_type == QA_OUT_I8 ? launch_tile<QA_OUT_I8>(*p, stream) : launch_tile<QA_OUT_F16>(*p, stream);
         if (way == kWay64x128) return launch_reg<2, 4, 256>(*p, stream);
         if (way == kWay128x128) return launch_reg<4, 4, 128>(*p, stream);

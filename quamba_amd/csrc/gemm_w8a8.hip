@@ -210,11 +210,9 @@ GemvParams as_gemv(const QaGemmW8A8Params& p) {
 int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
     const int cus = compute_units();
     auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
-    const float units = static_cast<float>((p.k + kBK - 1) / kBK);
     if (tiles(128, 128) <= cus) {
-        const float whole = 2.5f + units * (tiles(64, 64) <= cus ? 0.20f : tiles(128, 64) <= cus ? 0.31f : 0.48f);
         const SplitChoice split = split_choice(8, p.m, p.n, p.k, cus);
-        if (split.us < whole) return split_launch_w8(as_gemv(p), split.shape, stream);
+        if (split.us < tiles_us_w8(p.m, p.n, p.k, cus)) return split_launch_w8(as_gemv(p), split.shape, nullptr, stream);
     }
     if (tiles(64, 64) <= cus) return launch_gemm<1, 1, 2, 2, 4, false>(p, stream);
     if (tiles(128, 64) <= cus) return launch_gemm<1, 1, 4, 2, 4, false>(p, stream);
@@ -232,6 +230,12 @@ int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
 }
 
 }  // namespace
+
+float tiles_us_w8(int m, int n, int k, int cus) {
+    auto fits = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn) <= cus; };
+    return 2.5f + static_cast<float>((k + gemm::kBK - 1) / gemm::kBK) * (fits(64, 64) ? 0.20f : fits(128, 64) ? 0.31f : fits(128, 128) ? 0.48f : fits(128, 256) ? 0.68f : 1.15f);
+}
+
 }  // namespace qa
 
 extern "C" int qa_gemm_w8a8(const QaGemmW8A8Params* p, void* stream_) {
@@ -256,7 +260,7 @@ extern "C" int qa_gemm_w8a8(const QaGemmW8A8Params* p, void* stream_) {
     const bool flex = p->use_alpha || p->round_mode != QA_ROUND_RNE;
     if (gemv_is_faster(p->m, p->n, p->k)) return gemv_launch(as_gemv(*p), nullptr, stream);
     // the single-row rules (host alpha, round-half-away) only ever come with tiny M
-    if (flex && p->m <= 64) return split_launch_w8(as_gemv(*p), split_choice(8, p->m, p->n, p->k, compute_units()).shape, stream);
+    if (flex && p->m <= 64) return split_launch_w8(as_gemv(*p), split_choice(8, p->m, p->n, p->k, compute_units()).shape, nullptr, stream);
     if (flex) return launch_gemm<2, 2, 2, 2, 2, true>(*p, stream);
     return dispatch_tiles(*p, stream);
 }

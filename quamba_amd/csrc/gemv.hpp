@@ -79,8 +79,12 @@ inline SplitChoice split_choice(int bits, int m, int n, int k, int cus) {
 // Operands as the products' entry points take them (16-byte aligned rows; K a multiple of 16, or of 128 with 4 bits; with 8
 // bits every offset below 2^31).  4 bits: a tile's rows and the group scales (null: per channel) are addressed with 32 bits.
 inline bool split_addressable_w4(int n, int k) { return 40LL * k <= 0x7fffffffLL && static_cast<int64_t>(n) * (k / 128) < 1 << 29; }
-int split_launch_w8(const GemvParams& p, int shape, hipStream_t stream);
-int split_launch_w4(const GemvParams& p, int shape, hipStream_t stream);
+int split_launch_w8(const GemvParams& p, int shape, const GemvConv* conv, hipStream_t stream);
+int split_launch_w4(const GemvParams& p, int shape, const GemvConv* conv, hipStream_t stream);
+
+// us of the products' launches without it, where one round of their tiles is enough (else far more): gemm_w8a8.hip, gemm_w4a8.hip
+float tiles_us_w8(int m, int n, int k, int cus);
+float tiles_us_w4(int m, int n, int k, int cus);
 
 // Which of the two a product of up to kGemvRows rows takes.  A row is work for the vector units in gemv.hip and free in a
 // block of sixteen here: one and two rows there, three and four only where the outputs are so few that the split leaves the

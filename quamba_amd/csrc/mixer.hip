@@ -12,6 +12,7 @@
 //
 // A call is refused before its first launch or not at all (validate, ready): a step advances both states in place, and one
 // that stopped half way could not be made again another way.
+#include "conv2_common.hpp"
 #include "gemv.hpp"
 #include "hadamard_core.hpp"
 #include "mixer_common.hpp"
@@ -95,12 +96,15 @@ int hadamard_check(int dim) { return dim <= 32768 && hadamard_shape(dim).s != 0 
 
 constexpr int64_t kConvSteps = 65535LL * 4 * 256;       // of a sequence: the grid of the forward conv
 
-// in_proj of a decode step with the conv's step behind it in one launch (QA_ERR_UNSUPPORTED: two launches)
+// in_proj of a decode step with the conv's step behind it in one launch (QA_ERR_UNSUPPORTED: two launches).  Behind a product
+// that splits K the conv takes 0.3 us and 1.1 per four outputs of a thread, on the few waves that hold the sums; a launch of its
+// own takes 4.0, with grouped scales, whose table is walked first, 5.5 - and the product may then be another, faster one (us,
+// apart -> together: int8 16 x 10240 x 2560 11.3 -> 8.6, 64 x 10240 x 2560 11.2 -> 10.8, 128 x 10240 x 2560 14.2 -> 15.9; 4 bits 24 x
+// 10240 x 2560 9.9 -> 8.1, 40 x 8480 x 2048 12.4 -> 10.9, 64 x 18560 x 4096 33 -> 31).
 int project_conv(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows, int8_t* d, int ch0, const QaConv2Params& conv, void* stream) {
     const GemvConv f = {ch0, conv};
-    if (rows > kGemvRows || !gemv_conv_ok(f)) return QA_ERR_UNSUPPORTED;
+    if (!gemv_conv_ok(f)) return QA_ERR_UNSUPPORTED;
     if (w.k % 16 != 0 || lda % 16 != 0 || !aligned16(a) || !aligned16(w.weight)) return QA_ERR_UNSUPPORTED;
-    if (w.bits == 4 && (!w.s_group || w.n % 4 != 0 || w.k % 128 != 0 || (reinterpret_cast<uintptr_t>(w.s_group) & 7u))) return QA_ERR_UNSUPPORTED;
     GemvParams g = {};
     g.m = rows; g.n = w.n; g.k = w.k; g.bits = w.bits;
     g.out_type = QA_OUT_I8;
@@ -111,7 +115,18 @@ int project_conv(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows
     g.lda = lda; g.ldw = w.bits == 4 ? w.k / 2 : w.k; g.ldd = w.n;
     g.a = a; g.w = w.weight; g.s_group = static_cast<const __half*>(w.s_group);
     g.row_scale = w.row_scale; g.col_scale = w.col_scale; g.d = d;
-    return gemv_launch(g, &f, static_cast<hipStream_t>(stream));
+    if (w.bits == 4 && (w.k % 128 != 0 || !split_addressable_w4(w.n, w.k))) return QA_ERR_UNSUPPORTED;
+    const bool dot_products = w.bits == 8 || (w.s_group && w.n % 4 == 0 && (reinterpret_cast<uintptr_t>(w.s_group) & 7u) == 0);
+    if (gemv_is_faster(rows, w.n, w.k) && dot_products) return gemv_launch(g, &f, static_cast<hipStream_t>(stream));
+    // (words in every operand and in the columns that are stored)
+    if (!conv_words_ok(conv) || !(conv_state_in_words(conv) || conv_state_in_rows(conv)) || w.n % 4 != 0 || !aligned4(d)) return QA_ERR_UNSUPPORTED;
+    const int cus = compute_units();
+    const SplitChoice split = split_choice(w.bits, rows, w.n, w.k, cus);
+    const float tiles = w.bits == 8 ? tiles_us_w8(rows, w.n, w.k, cus) : tiles_us_w4(rows, w.n, w.k, cus);
+    const SplitShape& shape = kSplitShapes[split.shape];
+    const int quads = (shape.rows * shape.cols / 4 + 511) / 512;
+    if (split.us + 0.3f + 1.1f * static_cast<float>(quads) > std::min(split.us, tiles) + (conv.x_head_group_range ? 5.5f : 4.0f)) return QA_ERR_UNSUPPORTED;
+    return w.bits == 8 ? split_launch_w8(g, split.shape, &f, static_cast<hipStream_t>(stream)) : split_launch_w4(g, split.shape, &f, static_cast<hipStream_t>(stream));
 }
 
 int hadamard(const void* y, int8_t* out, int rows, int dim, float scale, void* stream) {
