@@ -23,7 +23,6 @@
 namespace qa {
 namespace {
 
-constexpr int kFusedDtRows = 16;
 constexpr int kExpandOnceRows = 65;       // from this many rows on the product may want the 4-bit weights expanded once (qa_gemm_w4a8 decides)
 
 // Sections of the workspace, each 256-byte aligned.
@@ -507,11 +506,10 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
     const QaSsmUpdateParams u = update_of(*p, b);
     const QaLinearParams& dt = p->dt_proj;
     int st = QA_ERR_UNSUPPORTED;
-    // (every batch entry reads the weights again, a row per lane: past a few entries a product of its own is the faster one)
-    if (rows <= kFusedDtRows && dt.bits == 8) {
+    if (dt.bits == 8) {
         const SsmDtProj proj = {static_cast<const int8_t*>(dt.weight), b.x_dbl, p->x_proj.n, dt.row_scale, dt.col_scale, dt.k / 16, dt.col_numel,
                                 rows == 1 && dt.row_rule == QA_ROW_ALPHA, dt.alpha};
-        st = ssm_update_with_dt(u, proj, static_cast<hipStream_t>(stream));
+        st = mamba1_step(u, proj, static_cast<hipStream_t>(stream));
     }
     if (st == QA_ERR_UNSUPPORTED) {
         QA_TRY(project(dt, b.x_dbl, p->x_proj.n, rows, b.dt, QA_OUT_I8, false, b.w8, stream));

@@ -23,10 +23,10 @@ int sscan_token_major_fwd(const QaSScanParams& p, const SscanDtProj* dt, hipStre
 // bytes of scratch it can use for these sizes (0: none)
 int64_t sscan_token_major_workspace(const QaSScanParams& p);
 
-// sscan.hip: the single-token state update of a Mamba1 layer with dt_proj in front of it: the step size code of channel d is
-// the projection of `x` (16 * pieces codes a batch entry, x_batch_stride apart) with row d of `w` (contiguous rows), scaled
-// and rounded as the int8 product does it.  p.dt is not read.  QA_ERR_UNSUPPORTED where the layer's layout is not the one
-// the fixed-shape update takes.
+// sscan_step.hip: the single-token state update of a Mamba1 layer with dt_proj in front of it (p.dt is not read): the step size
+// code of channel d is the projection of `x` (16 * pieces codes a batch entry, x_batch_stride apart) with row d of `w`
+// (contiguous rows), scaled and rounded as the int8 product does it.  QA_ERR_UNSUPPORTED where the layout is not the one it
+// takes (contiguous channels and states, whole waves of sixteen channels).
 struct SsmDtProj {
     const int8_t *w, *x;
     int64_t x_batch_stride;
@@ -34,8 +34,8 @@ struct SsmDtProj {
     int pieces, col_numel, use_alpha;
     float alpha;
 };
-constexpr int kSsmDtPieces = 10;       // up to 160 inputs
-int ssm_update_with_dt(const QaSsmUpdateParams& p, const SsmDtProj& dt, hipStream_t stream);
+constexpr int kSsmDtPieces = 12;       // up to 192 inputs
+int mamba1_step(const QaSsmUpdateParams& p, const SsmDtProj& dt, hipStream_t stream);
 // what qa_ssm_state_update refuses, without a launch
 int ssm_update_check(const QaSsmUpdateParams& p);
 

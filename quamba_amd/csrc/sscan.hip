@@ -831,26 +831,6 @@ int choose_mapping16(const QaSScanParams& p) {
 // state) pieces.
 // Reference: quamba/triton/selective_state_update.py:83-126 and :303-362.
 // ---------------------------------------------------------------------------------------------
-// sat8_rne(fl(h k) / fl(s k)) of four states, packed.  The IEEE quotient is twelve instructions a state and was most of a
-// lane's arithmetic; a product with the reciprocal is within 2^-21 of it, so the integers agree unless the product lies within
-// 1e-4 of a rounding tie (values up to 128; beyond, both saturate), and only a wave that holds such a state divides.
-// (inv: rcp of fl(s k))
-__device__ __forceinline__ uint32_t requantise4(const float (&h)[4], const float (&s)[4], const float (&inv)[4], float k) {
-    float t[4], num[4];
-    bool tie = false;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        num[e] = h[e] * k;
-        t[e] = num[e] * inv[e];
-        tie |= !(__builtin_fabsf(t[e] - __builtin_rintf(t[e])) < 0.4999f);         // (NaN and infinities divide)
-    }
-    if (__builtin_amdgcn_ballot_w64(tie)) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) t[e] = num[e] / (s[e] * k);
-    }
-    return gemm::pack4_rne_sat8(t[0], t[1], t[2], t[3]);
-}
-
 // VEC: the state axis has unit stride in state, A_log, B and C and every row piece of four states is
 // naturally aligned, so a lane moves its four states with one load and one store per operand.
 // A wave's life here is a chain of memory round trips, not arithmetic, so optional operands are read
@@ -863,10 +843,8 @@ __device__ __forceinline__ uint32_t requantise4(const float (&h)[4], const float
 // run of loads, arithmetic and stores without loops or branches on the parameter block.
 // CONV_STATE: with CONV and FAST, the codes per row of the conv state (4: a word per row; 3: rows back to back).
 // A_ONE: A_log has one value for all states of a row (Mamba2: one per head), and the decay is evaluated once.
-// DT, with FAST: the step size code is dt_proj's output, evaluated here (a row of up to 160 int8 weights per lane against the
-// batch entry's row of x_proj's output, which is the same for the whole wave and comes through scalar loads).
-template <int LPR, bool VEC, bool FP32, bool CONV, bool FAST = false, int CONV_STATE = 4, bool DT = false, bool A_ONE = false>
-__device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, const QaConvParams* cp, const SsmDtProj* dp = nullptr) {
+template <int LPR, bool VEC, bool FP32, bool CONV, bool FAST = false, int CONV_STATE = 4, bool A_ONE = false>
+__device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, const QaConvParams* cp) {
     static_assert(!CONV || LPR == 1, "the conv step needs one lane per row");
     static_assert(!FAST || (LPR == 1 && VEC), "the fixed shape has one lane per row and whole pieces");
     const int dstate = FAST ? 16 : p.dstate;
@@ -1006,22 +984,11 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
     // FAST: B_scale * B[n] and C_scale * C[n] are the same in every lane of the workgroup (one batch entry), and
     // converting and scaling them in every lane is an eighth of the lane's arithmetic.  Lanes 0-31 of each wave form
     // one value each (same expression, same bits) and the wave reads all 32 back from LDS as broadcasts.
-    uint4 dt_w[DT ? kSsmDtPieces : 1];
-    float dt_col = 0.0f, dt_row = 0.0f;
-    if constexpr (DT) {
-        const uint4* row = reinterpret_cast<const uint4*>(dp->w + static_cast<int64_t>(d) * (16 * dp->pieces));
-#pragma unroll
-        for (int i = 0; i < kSsmDtPieces; ++i)
-            if (i < dp->pieces) dt_w[i] = row[i];
-        dt_row = dp->use_alpha ? dp->alpha : *dp->row_scale;
-        dt_col = dp->use_alpha ? 1.0f : dp->col_scale[dp->col_numel == 1 ? 0 : d];
-    }
     int8_t bc_code = 0;
     if constexpr (FAST) bc_code = ((lane & 16) ? Cp : Bp)[lane & 15];      // every lane loads: no branch, no wait here
     // The row's other operands come after the state's pieces are on their way: with CONV the conv step's own loads,
     // arithmetic and stores then run under the state's round trip instead of before it.
-    float dtq;
-    if constexpr (!DT) dtq = static_cast<float>(*dt_a);
+    const float dtq = static_cast<float>(*dt_a);
     const float zq = static_cast<float>(*z_a), Dq = static_cast<float>(*D_a);
     const float b8 = static_cast<float>(*b8_a), b16 = __half2float(*b16_a);
     float xq;
@@ -1062,23 +1029,6 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
             const float4 v = turn[wv][4 * lane + (k ^ (lane / 4 % 4))];
             hv[k][0] = v.x; hv[k][1] = v.y; hv[k][2] = v.z; hv[k][3] = v.w;
         }
-    }
-    if constexpr (DT) {
-        typedef const __attribute__((address_space(4))) uint32_t* const_words;
-        const const_words x = reinterpret_cast<const_words>(reinterpret_cast<uintptr_t>(dp->x + b * dp->x_batch_stride));
-        int sum = 0;
-#pragma unroll
-        for (int i = 0; i < kSsmDtPieces; ++i) {
-            if (i < dp->pieces) {
-                sum = __builtin_amdgcn_sdot4(static_cast<int>(dt_w[i].x), static_cast<int>(x[4 * i]), sum, false);
-                sum = __builtin_amdgcn_sdot4(static_cast<int>(dt_w[i].y), static_cast<int>(x[4 * i + 1]), sum, false);
-                sum = __builtin_amdgcn_sdot4(static_cast<int>(dt_w[i].z), static_cast<int>(x[4 * i + 2]), sum, false);
-                sum = __builtin_amdgcn_sdot4(static_cast<int>(dt_w[i].w), static_cast<int>(x[4 * i + 3]), sum, false);
-            }
-        }
-        float v = dt_col * static_cast<float>(sum);
-        asm volatile("" : "+v"(v));                   // two products, each rounded (with alpha the first is by one)
-        dtq = static_cast<float>(sat8_rne(dt_row * v));
     }
     const float xv = x_scale * xq;
     float dt = dt_scale * dtq;
@@ -1154,12 +1104,7 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
 
 template <int LPR, bool VEC, bool FP32, bool FAST = false, bool A_ONE = false>
 __global__ __launch_bounds__(256) void ssm_update_kernel(QaSsmUpdateParams p) {
-    ssm_update_body<LPR, VEC, FP32, false, FAST, 4, false, A_ONE>(p, nullptr);
-}
-
-template <bool FP32>
-__global__ __launch_bounds__(256) void ssm_update_dt_kernel(QaSsmUpdateParams p, SsmDtProj dp) {
-    ssm_update_body<1, true, FP32, false, true, 4, true>(p, nullptr, &dp);
+    ssm_update_body<LPR, VEC, FP32, false, FAST, 4, A_ONE>(p, nullptr);
 }
 
 // conv step + state update of one token in one launch (d_state <= 16, one head)
@@ -1299,7 +1244,7 @@ bool update_fits_grid(const QaSsmUpdateParams& p, int lanes_per_row = 16) {
 }
 
 template <int LPR>
-int launch_update(const QaSsmUpdateParams& p, hipStream_t stream, const QaConvParams* conv = nullptr, const SsmDtProj* dt = nullptr) {
+int launch_update(const QaSsmUpdateParams& p, hipStream_t stream, const QaConvParams* conv = nullptr) {
     const int64_t blocks = (static_cast<int64_t>(p.dim) * LPR + 255) / 256;
     if (!update_fits_grid(p, LPR)) return QA_ERR_SHAPE;
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(p.nheads), static_cast<unsigned>(p.batch));
@@ -1319,15 +1264,6 @@ int launch_update(const QaSsmUpdateParams& p, hipStream_t stream, const QaConvPa
                                  p.A_dstate_stride == 1 && p.A_dim_stride % 16 == 0 && aligned16(p.A_log) &&
                                  (!p.state_is_fp32 || (p.state_dim_stride == 16 && p.dim % 64 == 0)) &&
                                  !(p.dt_bias && p.dt_bias_is_fp16);
-        if (dt) {
-            if (!fast_update || dt->pieces > kSsmDtPieces || !aligned16(dt->w) || !aligned4(dt->x) || dt->x_batch_stride % 4 != 0) return QA_ERR_UNSUPPORTED;
-            // a wave per workgroup: the rows' step size weights, 16 bytes a lane at a stride, are slow work for a CU's memory
-            // path, and few sequences have few waves
-            const dim3 waves(static_cast<unsigned>((p.dim + 63) / 64), 1, static_cast<unsigned>(p.batch));
-            if (p.state_is_fp32) hipLaunchKernelGGL(ssm_update_dt_kernel<true>, waves, dim3(64), 0, stream, p, *dt);
-            else hipLaunchKernelGGL(ssm_update_dt_kernel<false>, waves, dim3(64), 0, stream, p, *dt);
-            return check_launch();
-        }
         if (!conv && fast_update) {
             auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, p); };
             p.state_is_fp32 ? go(ssm_update_kernel<1, true, true, true>) : go(ssm_update_kernel<1, true, false, true>);
@@ -1484,7 +1420,6 @@ int qa::ssm_update_check(const QaSsmUpdateParams& p) {
     return st != QA_OK ? st : update_fits_grid(p) ? QA_OK : QA_ERR_SHAPE;
 }
 
-int qa::ssm_update_with_dt(const QaSsmUpdateParams& p, const SsmDtProj& dt, hipStream_t stream) { return launch_update<1>(p, stream, nullptr, &dt); }
 
 extern "C" int qa_ssm_state_update(const QaSsmUpdateParams* p, void* stream_) {
     using namespace qa;

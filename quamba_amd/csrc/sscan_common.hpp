@@ -1,6 +1,7 @@
 // Pieces shared by the selective-scan kernels (sscan.hip, sscan_tm.hip): the transcendental functions as they evaluate
 // them, byte conversions, cross-lane moves.
 #pragma once
+#include "gemm_core.hpp"
 #include "qa_common.hpp"
 
 namespace qa {
@@ -90,6 +91,26 @@ __device__ __forceinline__ float row_from_up(float v) {
 
 __device__ __forceinline__ float i8_of(uint32_t word, int j) {
     return static_cast<float>(static_cast<int8_t>((word >> (8 * j)) & 0xffu));
+}
+
+// sat8_rne(fl(h k) / fl(s k)) of four states, packed.  The IEEE quotient is twelve instructions a state and was most of a
+// lane's arithmetic; a product with the reciprocal is within 2^-21 of it, so the integers agree unless the product lies within
+// 1e-4 of a rounding tie (values up to 128; beyond, both saturate), and only a wave that holds such a state divides.
+// (inv: rcp of fl(s k))
+__device__ __forceinline__ uint32_t requantise4(const float (&h)[4], const float (&s)[4], const float (&inv)[4], float k) {
+    float t[4], num[4];
+    bool tie = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        num[e] = h[e] * k;
+        t[e] = num[e] * inv[e];
+        tie |= !(__builtin_fabsf(t[e] - __builtin_rintf(t[e])) < 0.4999f);         // (NaN and infinities divide)
+    }
+    if (__builtin_amdgcn_ballot_w64(tie)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = num[e] / (s[e] * k);
+    }
+    return gemm::pack4_rne_sat8(t[0], t[1], t[2], t[3]);
 }
 
 }  // namespace qa

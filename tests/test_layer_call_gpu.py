@@ -84,10 +84,13 @@ def test_step_of_a_wide_layer(dev, d_model):
 
 @pytest.mark.parametrize("cls,d_model,batch,width", [(W8A8QMamba, 768, 3, 4), (W8A8QMamba, 2560, 30, 4), (W8A8QMamba, 2560, 61, 4), (W8A8QMamba, 2560, 20, 3),
                                                      (W4A8QMamba, 2560, 24, 4), (W4A8QMamba, 2560, 61, 4), (W8A8QMamba2, 768, 9, 4),
-                                                     (W8A8QMamba2, 2560, 17, 3), (W4A8QMamba2, 2048, 40, 4), (W4A8QMamba2, 4096, 63, 4)])
+                                                     (W8A8QMamba2, 2560, 17, 3), (W8A8QMamba, 3072, 2, 4),
+                                                     (W8A8QMamba, 1024, 4, 4), (W4A8QMamba, 1536, 6, 4), (W4A8QMamba2, 2048, 40, 4), (W4A8QMamba2, 4096, 63, 4)])
 def test_step_of_many_sequences(dev, cls, d_model, batch, width):
     """in_proj and the conv in one launch for more than two rows: each tile of the product, with one and two passes over its
-    sums, the conv's state by channel and by step (three and four codes), rows and columns with remainders."""
+    sums, the conv's state by channel and by step (three and four codes), rows and columns with remainders; in the first family
+    dt_proj in the state update's launch, ranks of 48 to 192, one to four entries a wave."""
+    dtype = torch.float32 if batch % 2 == 0 else torch.int8
     second = cls in (W8A8QMamba2, W4A8QMamba2)
     sized = lambda d, *a, **k: cls(d_model, *a, **k)
     m, g = (_mamba2 if second else variants._mamba1)(sized, dev, seed=batch)
@@ -95,7 +98,7 @@ def test_step_of_many_sequences(dev, cls, d_model, batch, width):
         heads = m.nheads // 2
         m.conv1d.x_head_group_range = m.qchunk_scan.x_head_group_range = torch.tensor([[1, heads], [3, heads]], dtype=torch.int32, device=dev)
     h = _ri(dev, g, batch, 1, d_model)
-    conv, ssm = _states(m, dev, g, batch, torch.int8, width)
+    conv, ssm = _states(m, dev, g, batch, dtype, width)
     conv2, ssm2 = conv.clone(), ssm.clone()
     out = _layer_call.call(m, h, conv, ssm, True)
     assert out is not None
