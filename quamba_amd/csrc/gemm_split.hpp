@@ -53,7 +53,7 @@ struct Cfg {
 enum ConvKind { kNoConv, kConvWords, kConvRows };       // the layouts of the conv's state (conv_state_in_words, conv_state_in_rows)
 
 template <int BITS, int BM, int BN, int DEPTH, int OUT, ConvKind CONV>
-__global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_split_kernel(GemvParams p, GemvConv f) {
+__global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_split_kernel(GemvArgs p, std::conditional_t<CONV != kNoConv, GemvConv, NoGemvConv> f) {
     using C = Cfg<BITS, BM, BN, DEPTH>;
     __shared__ __attribute__((aligned(16))) uint8_t lds[C::kLdsBytes];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -67,16 +67,16 @@ __global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_spl
     float* const s_col = reinterpret_cast<float*>(lds + C::kScalesAt);
     float* const s_row = s_col + C::kColScales;
     if (p.rule != kGemvAlpha) {
-        const v4i rsrc_c = make_rsrc(p.col_scale, (p.col_numel == 1 ? 1 : p.n) * 4), rsrc_r = make_rsrc(p.row_scale, (p.row_numel == 1 ? 1 : p.m) * 4);
+        const v4i rsrc_c = make_rsrc(p.col_scale, (p.one_col_scale ? 1 : p.n) * 4), rsrc_r = make_rsrc(p.row_scale, (p.one_row_scale ? 1 : p.m) * 4);
 #pragma unroll
         for (int i = 0; i < (C::kColScales + C::kRowScales) / 64; ++i) {
             if (i % C::kWaves != wave) continue;
-            if (i < C::kColScales / 64) buffer_load_lds_b32(rsrc_c, lds_base + C::kScalesAt + i * 256, p.col_numel == 1 ? 0 : (n0 + i * 64 + lane) * 4);
-            else buffer_load_lds_b32(rsrc_r, lds_base + C::kScalesAt + i * 256, p.row_numel == 1 ? 0 : (m0 + lane) * 4);
+            if (i < C::kColScales / 64) buffer_load_lds_b32(rsrc_c, lds_base + C::kScalesAt + i * 256, p.one_col_scale ? 0 : (n0 + i * 64 + lane) * 4);
+            else buffer_load_lds_b32(rsrc_r, lds_base + C::kScalesAt + i * 256, p.one_row_scale ? 0 : (m0 + lane) * 4);
         }
     }
 
-    const int ldw = static_cast<int>(p.ldw);
+    const int ldw = p.ldw;
     const v4i rsrc_a = make_rsrc(p.a, static_cast<int>((static_cast<int64_t>(p.m) - 1) * p.lda + p.k));
     const v4i rsrc_w = make_rsrc(static_cast<const uint8_t*>(p.w) + static_cast<int64_t>(n0) * ldw, (min(BN, p.n - n0) - 1) * ldw + p.k * BITS / 8);
     TileLoader<C::kAReq> load_a;
@@ -127,7 +127,10 @@ __global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_spl
     // The conv state of its row and channels is on its way from here on.
     ConvHeld<CONV == kConvRows> held[CONV ? C::kPasses : 1][CONV ? C::kQuads : 1];
     ConvQuad* const quads = reinterpret_cast<ConvQuad*>(lds + C::kColumnsAt);
-    auto is_conv = [&](int n) { return n >= f.ch0 && n < f.ch0 + f.conv.dim; };
+    auto is_conv = [&](int n) {
+        if constexpr (CONV != kNoConv) return n >= f.ch0 && n < f.ch0 + f.conv.dim;
+        else return false;
+    };
     if constexpr (CONV != kNoConv) {
         const QaConv2Params& c = f.conv;
 #pragma unroll
@@ -271,12 +274,16 @@ template <int BITS, int BM, int BN, int DEPTH>
 int launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
     using C = Cfg<BITS, BM, BN, DEPTH>;
     const int64_t blocks = static_cast<int64_t>((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
-    auto kernel = gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8, kNoConv>;
-    if (conv) kernel = conv_state_in_words(conv->conv) ? gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8, kConvWords> : gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8, kConvRows>;
-    else if (p.out_type == QA_OUT_F16) kernel = gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_F16, kNoConv>;
-    else if constexpr (BITS == 8) { if (p.out_type == QA_OUT_BF16) kernel = gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_BF16, kNoConv>; }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(C::kThreads), 0, stream, p, conv ? *conv : GemvConv{});
-    return check_launch();
+    const GemvArgs args(p);
+    auto go = [&](auto kernel, const auto& f) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(C::kThreads), 0, stream, args, f);
+        return check_launch();
+    };
+    if (conv) return conv_state_in_words(conv->conv) ? go(gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8, kConvWords>, *conv) : go(gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8, kConvRows>, *conv);
+    const NoGemvConv none = {};
+    if (p.out_type == QA_OUT_F16) return go(gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_F16, kNoConv>, none);
+    if constexpr (BITS == 8) { if (p.out_type == QA_OUT_BF16) return go(gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_BF16, kNoConv>, none); }
+    return go(gemm_split_kernel<BITS, BM, BN, DEPTH, QA_OUT_I8, kNoConv>, none);
 }
 
 // the tile shapes in the order of kSplitShapes

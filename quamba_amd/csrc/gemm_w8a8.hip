@@ -258,7 +258,7 @@ extern "C" int qa_gemm_w8a8(const QaGemmW8A8Params* p, void* stream_) {
     if (static_cast<int64_t>(p->m) * p->lda >= 0x70000000LL || static_cast<int64_t>(p->n) * p->ldw >= 0x70000000LL) return QA_ERR_SHAPE;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const bool flex = p->use_alpha || p->round_mode != QA_ROUND_RNE;
-    if (gemv_is_faster(p->m, p->n, p->k)) return gemv_launch(as_gemv(*p), nullptr, stream);
+    if (gemv_is_faster(8, p->m, p->n, p->k)) return gemv_launch(as_gemv(*p), nullptr, stream);
     // the single-row rules (host alpha, round-half-away) only ever come with tiny M
     if (flex && p->m <= 64) return split_launch_w8(as_gemv(*p), split_choice(8, p->m, p->n, p->k, compute_units()).shape, nullptr, stream);
     if (flex) return launch_gemm<2, 2, 2, 2, 2, true>(*p, stream);

@@ -93,7 +93,7 @@ __device__ __forceinline__ void uniform_out_scales(const QaConv2Params& p, const
 // BATCH: pieces of K (1 KB of each weight row) whose loads are in flight together.  KS: waves of the workgroup that share
 // four rows, a contiguous part of K each.
 template <int BITS, int M, int KS, int BATCH, int OUT, bool CONV>
-__global__ __launch_bounds__(256) void gemv_kernel(GemvParams p, GemvConv f) {
+__global__ __launch_bounds__(256) void gemv_kernel(GemvArgs p, std::conditional_t<CONV, GemvConv, NoGemvConv> f) {
     constexpr int V = kRows * M, PER = V / 4;                    // values of the wave, and per lane after two folds
     constexpr int kLaneCodes = BITS == 8 ? 16 : 32, kPieceCodes = 64 * kLaneCodes, AQ = kLaneCodes / 16;
     const int lane = threadIdx.x & 63;
@@ -135,8 +135,8 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p, GemvConv f) {
     const int value = (quarter >> 1) * (V / 2) + (quarter & 1) * PER + min(slot, PER - 1);
     const int my_m = min(value / kRows, p.m - 1), my_n = min(n0 + value % kRows, p.n - 1);
     const bool mine = slot < PER && value / kRows < p.m && n0 + value % kRows < p.n;
-    const float s_row = p.rule == kGemvAlpha ? p.alpha : p.row_scale[p.row_numel == 1 ? 0 : my_m];
-    const float s_col = p.rule == kGemvAlpha ? 1.0f : p.col_scale[p.col_numel == 1 ? 0 : my_n];
+    const float s_row = p.rule == kGemvAlpha ? p.alpha : p.row_scale[p.one_row_scale ? 0 : my_m];
+    const float s_col = p.rule == kGemvAlpha ? 1.0f : p.col_scale[p.one_col_scale ? 0 : my_n];
 
     // operands of the conv step of this lane's column
     bool conv_col = false;
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p, GemvConv f) {
     Part part = {};
     bool st_word = false;
     // (the four columns of a wave are all conv channels, of one part and one head, or none is)
-    if (CONV && n0 >= f.ch0 && n0 < f.ch0 + f.conv.dim) {
+    if constexpr (CONV) if (n0 >= f.ch0 && n0 < f.ch0 + f.conv.dim) {
         const QaConv2Params& c = f.conv;
         conv_col = true;
         ch = my_n - f.ch0;
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p, GemvConv f) {
     asm volatile("" : "+v"(y));                                  // the fp32 product is rounded on its own
     if constexpr (OUT == QA_OUT_I8) {
         const int8_t q = static_cast<int8_t>(quant8(y, p.half_away ? QA_ROUND_HALF_AWAY : QA_ROUND_RNE));
-        if (CONV && conv_col) {
+        if constexpr (CONV) if (conv_col) {
             const QaConv2Params& c = f.conv;
             const uint32_t kept = st_word ? held[0] >> 8 : held[0] | (held[1] << 8) | (held[2] << 16);
             const uint32_t win = kept | (static_cast<uint32_t>(static_cast<uint8_t>(q)) << 24);
@@ -264,11 +264,12 @@ int launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
     const int64_t groups = (static_cast<int64_t>(p.n) + kRows - 1) / kRows;
     const int per_block = KS > 1 || groups >= 1024 ? 4 : 1;      // waves; few waves: a workgroup each, spread over the part
     const dim3 grid(static_cast<unsigned>((groups * KS + per_block - 1) / per_block)), block(64 * per_block);
-    const GemvConv none = {};
-    if (conv) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, true>), grid, block, 0, stream, p, *conv);
-    else if (p.out_type == QA_OUT_I8) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, false>), grid, block, 0, stream, p, none);
-    else if (p.out_type == QA_OUT_F16) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_F16, false>), grid, block, 0, stream, p, none);
-    else hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_BF16, false>), grid, block, 0, stream, p, none);
+    const GemvArgs args(p);
+    const NoGemvConv none = {};
+    if (conv) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, true>), grid, block, 0, stream, args, *conv);
+    else if (p.out_type == QA_OUT_I8) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, false>), grid, block, 0, stream, args, none);
+    else if (p.out_type == QA_OUT_F16) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_F16, false>), grid, block, 0, stream, args, none);
+    else hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_BF16, false>), grid, block, 0, stream, args, none);
     return check_launch();
 }
 
@@ -299,7 +300,7 @@ struct RotShape {
 };
 
 template <int BITS, int S>
-__global__ __launch_bounds__(kRotThreads) void gemv_rotated_kernel(GemvParams p, GemvRotate r, RotShape shape) {
+__global__ __launch_bounds__(kRotThreads) void gemv_rotated_kernel(GemvArgs p, GemvRotate r, RotShape shape) {
     constexpr int kLaneCodes = BITS == 8 ? 16 : 32, kPieceCodes = 64 * kLaneCodes, AQ = kLaneCodes / 16, BATCH = BITS == 8 ? 4 : 2;
     extern __shared__ __attribute__((aligned(16))) float buf[];
     __shared__ int parts[kRotWaves][64];
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(kRotThreads) void gemv_rotated_kernel(GemvParams p,
     const int quarter = lane >> 4, my_n = min(n0 + quarter, p.n - 1);
     const bool mine = (lane & 15) == 0 && n0 + quarter < p.n;
     const float s_row = p.rule == kGemvAlpha ? p.alpha : p.row_scale[0];
-    const float s_col = p.rule == kGemvAlpha ? 1.0f : p.col_scale[p.col_numel == 1 ? 0 : my_n];
+    const float s_col = p.rule == kGemvAlpha ? 1.0f : p.col_scale[p.one_col_scale ? 0 : my_n];
     __builtin_amdgcn_sched_barrier(0);
 
 #pragma unroll
@@ -429,7 +430,7 @@ int gemv_rotated_launch(const GemvParams& p, const GemvRotate& r, hipStream_t st
     const dim3 grid(static_cast<unsigned>((groups + per_block - 1) / per_block));
     const int lds = (p.k + (p.k >> 5) + 4) / 4 * 16 + p.k;           // (below 64 KB)
     auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(kRotThreads), lds, stream, p, r, shape);
+        hipLaunchKernelGGL(kernel, grid, dim3(kRotThreads), lds, stream, GemvArgs(p), r, shape);
         return check_launch();
     };
     if (p.bits == 8) return h.s == 12 ? go(gemv_rotated_kernel<8, 12>) : h.s == 40 ? go(gemv_rotated_kernel<8, 40>) : go(gemv_rotated_kernel<8, 1>);

@@ -31,12 +31,33 @@ struct GemvParams {
     void* d;
 };
 
+// The same as the kernels take it.  What a launch costs the host grows with its arguments - 2.8 us up to 64 bytes, 3.4 at 128, 3.7
+// at 256, 3.9 at 512 - and a decode step of one or two sequences is as long as its launches.  (Products of up to 64 rows:
+// operands below 2^31 bytes.)
+struct GemvArgs {
+    const int8_t* a;
+    const void* w;
+    const __half* s_group;
+    const float* row_scale;
+    const float* col_scale;
+    void* d;
+    int64_t ldd;
+    int m, n, k, lda, ldw;
+    float alpha;
+    uint8_t rule, half_away, one_row_scale, one_col_scale;
+    explicit GemvArgs(const GemvParams& p)
+        : a(p.a), w(p.w), s_group(p.s_group), row_scale(p.row_scale), col_scale(p.col_scale), d(p.d), ldd(p.ldd), m(p.m), n(p.n), k(p.k),
+          lda(static_cast<int>(p.lda)), ldw(static_cast<int>(p.ldw)), alpha(p.alpha), rule(static_cast<uint8_t>(p.rule)),
+          half_away(p.half_away != 0), one_row_scale(p.row_numel == 1), one_col_scale(p.col_numel == 1) {}
+};
+
 // The output columns ch0 .. ch0 + conv.dim - 1 are the input of a causal conv's single-step update (width 4): the conv
 // state moves on, the conv's int8 output goes where `conv` says, and the columns themselves are not stored.
 struct GemvConv {
     int ch0;
     QaConv2Params conv;
 };
+struct NoGemvConv {};
 // (four columns a wave: whole quads of channels, inside one part and one head; taps as one word)
 inline bool gemv_conv_ok(const GemvConv& f) {
     const QaConv2Params& c = f.conv;
@@ -87,11 +108,11 @@ float tiles_us_w8(int m, int n, int k, int cus);
 float tiles_us_w4(int m, int n, int k, int cus);
 
 // Which of the two a product of up to kGemvRows rows takes.  A row is work for the vector units in gemv.hip and free in a
-// block of sixteen here: one and two rows there, three and four only where the outputs are so few that the split leaves the
-// waves a long K each (us at 1 / 2 / 3 rows, gemv against split: int8 10240 x 2560 5.8 / 6.1 / 6.8 against 6.3, 192 x 5120 3.0 /
-// 3.1 / 3.1 against 3.6; 4 bits 10240 x 2560 5.7 / 6.4 / 7.5 against 5.4, 4096 x 8192 5.5 / 6.2 / 7.4 against 6.9, 192 x 5120 3.1 /
-// 3.1 / 3.2 against 4.4; at five to eight rows, where it takes twice the registers, 9.1 and 10.0 against 6.3 and 5.4).
-inline bool gemv_is_faster(int m, int n, int k) { return m <= 2 || (m <= kGemvRows && n <= 512 && k > 2048); }
+// block of sixteen here, but a launch of small size is the faster one there: one and two rows, and three and four while the
+// weights are few (in a layer, us with three and four rows, gemv against split: int8 8192 x 2048 with the conv 5.2 against 6.8, 2048 x
+// 4096 3.6 / 4.6, 10240 x 2560 8.0 / 7.7; 4 bits 6144 x 1536 with the conv 5.7 / 6.1, 10240 x 2560 10.3 / 7.5, 8416 x 2048 11.4 / 8.0, 192 x
+// 5120 3.2 / 4.4; at five to eight rows, where it takes twice the registers, int8 10240 x 2560 9.1 / 6.3).
+inline bool gemv_is_faster(int bits, int m, int n, int k) { return m <= 2 || (m <= kGemvRows && static_cast<int64_t>(n) * k < (bits == 8 ? 20000000 : 10000000)); }
 
 // One activation row that is made on the spot: sat8(round_half_away(H y * had_scale)) of a row y of k fp16 values
 // (qa_hadamard_quant); fp16 results.  QA_ERR_UNSUPPORTED: not for these sizes (the caller then makes the two calls).

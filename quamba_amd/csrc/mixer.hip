@@ -116,7 +116,7 @@ int project_conv(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows
     g.row_scale = w.row_scale; g.col_scale = w.col_scale; g.d = d;
     if (w.bits == 4 && (w.k % 128 != 0 || !split_addressable_w4(w.n, w.k))) return QA_ERR_UNSUPPORTED;
     const bool dot_products = w.bits == 8 || (w.s_group && w.n % 4 == 0 && (reinterpret_cast<uintptr_t>(w.s_group) & 7u) == 0);
-    if (gemv_is_faster(rows, w.n, w.k) && dot_products) return gemv_launch(g, &f, static_cast<hipStream_t>(stream));
+    if (gemv_is_faster(w.bits, rows, w.n, w.k) && dot_products) return gemv_launch(g, &f, static_cast<hipStream_t>(stream));
     // (words in every operand and in the columns that are stored)
     if (!conv_words_ok(conv) || !(conv_state_in_words(conv) || conv_state_in_rows(conv)) || w.n % 4 != 0 || !aligned4(d)) return QA_ERR_UNSUPPORTED;
     const int cus = compute_units();

@@ -33,8 +33,20 @@ struct StepSmem {
     __attribute__((aligned(16))) int8_t w[kWaveCh * 16 * kSsmDtPieces], x[NB * 16 * kSsmDtPieces];
 };
 
+// what the kernel takes of QaSsmUpdateParams and SsmDtProj (a launch's arguments are host time, see gemv.hpp)
+struct StepArgs {
+    void* state;
+    __half* out;
+    const int8_t *x, *z, *A_log, *B, *C, *D, *dt_bias, *w, *dt_x;
+    const float *x_scale, *dt_scale, *dt_bias_scale, *A_log_scale, *state_scale, *B_scale, *C_scale, *D_scale, *z_scale, *row_scale, *col_scale;
+    int64_t state_batch_stride;
+    int batch, dim, A_dim_stride, x_batch_stride, z_batch_stride, B_batch_stride, C_batch_stride, out_batch_stride, dt_x_batch_stride, pieces;
+    float alpha;
+    uint8_t softplus, use_alpha, one_col_scale;
+};
+
 template <int NB, bool FP32>
-__global__ __launch_bounds__(kThreads) void mamba1_step_kernel(QaSsmUpdateParams p, SsmDtProj dp) {
+__global__ __launch_bounds__(kThreads) void mamba1_step_kernel(StepArgs p) {
     static_assert(NB == 1 || NB == 2 || NB == 4, "entries per wave");
     __shared__ StepSmem<NB> smem[kWaves];
     __shared__ __attribute__((aligned(16))) float bc_all[kWaves][NB][2][16];
@@ -49,10 +61,10 @@ __global__ __launch_bounds__(kThreads) void mamba1_step_kernel(QaSsmUpdateParams
 
     // the projection's operands first: everything else is needed behind them
     v4u rw[3], rx;
-    const v4u* w = reinterpret_cast<const v4u*>(dp.w + static_cast<int64_t>(c0) * (16 * dp.pieces));
+    const v4u* w = reinterpret_cast<const v4u*>(p.w + static_cast<int64_t>(c0) * (16 * p.pieces));
 #pragma unroll
-    for (int i = 0; i < 3; ++i) rw[i] = w[min(i * 64 + lane, kWaveCh * dp.pieces - 1)];
-    rx = *reinterpret_cast<const v4u*>(dp.x + entry(min(lane >> 4, NB - 1)) * dp.x_batch_stride + 16 * min(lane & 15, dp.pieces - 1));
+    for (int i = 0; i < 3; ++i) rw[i] = w[min(i * 64 + lane, kWaveCh * p.pieces - 1)];
+    rx = *reinterpret_cast<const v4u*>(p.dt_x + entry(min(lane >> 4, NB - 1)) * p.dt_x_batch_stride + 16 * min(lane & 15, p.pieces - 1));
     // B | C: word lane % 8 of an entry's sixteen B and sixteen C codes
     const int bc_b = lane >> 3, bc_w = lane & 7;
     uint32_t bc_codes = 0;
@@ -61,10 +73,10 @@ __global__ __launch_bounds__(kThreads) void mamba1_step_kernel(QaSsmUpdateParams
     const int8_t* const standin = p.x + c;                 // (read where an optional operand is missing)
     const int64_t mine = entry(min(slice, NB - 1));
     const int8_t x_q = p.x[mine * p.x_batch_stride + c], z_q = *(p.z ? p.z + mine * p.z_batch_stride + c : standin);
-    const int8_t D_q = *(p.D ? p.D + c : standin), bias_q = *(p.dt_bias ? static_cast<const int8_t*>(p.dt_bias) + c : standin);
-    const uint32_t A_codes = *reinterpret_cast<const uint32_t*>(p.A_log + c * p.A_dim_stride + 4 * slice);
-    const float dt_row = dp.use_alpha ? dp.alpha : *dp.row_scale;
-    const float dt_col = dp.use_alpha ? 1.0f : dp.col_scale[dp.col_numel == 1 ? 0 : c0 + (lane & 15)];
+    const int8_t D_q = *(p.D ? p.D + c : standin), bias_q = *(p.dt_bias ? p.dt_bias + c : standin);
+    const uint32_t A_codes = *reinterpret_cast<const uint32_t*>(p.A_log + static_cast<int64_t>(c) * p.A_dim_stride + 4 * slice);
+    const float dt_row = p.use_alpha ? p.alpha : *p.row_scale;
+    const float dt_col = p.use_alpha ? 1.0f : p.col_scale[p.one_col_scale ? 0 : c0 + (lane & 15)];
     const int64_t at = static_cast<int64_t>(c) * 16 + 4 * slice;
     float4 st32[FP32 ? NB : 1];
     uint32_t st8[FP32 ? 1 : NB];
@@ -80,7 +92,7 @@ __global__ __launch_bounds__(kThreads) void mamba1_step_kernel(QaSsmUpdateParams
     __builtin_amdgcn_sched_barrier(0);
 
     // (a wave writes and reads only its own part of LDS, where its operations complete in order)
-    const int pieces = dp.pieces;
+    const int pieces = p.pieces;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         const int t = i * 64 + lane;
@@ -118,7 +130,7 @@ __global__ __launch_bounds__(kThreads) void mamba1_step_kernel(QaSsmUpdateParams
     const float my_x = x_scale * static_cast<float>(x_q);
     float my_dt = dt_scale * static_cast<float>(dt_q), gate = 1.0f;
     my_dt += p.dt_bias ? bias_scale * static_cast<float>(bias_q) : 0.0f;
-    if (p.dt_softplus) my_dt = softplus20_flat(my_dt);
+    if (p.softplus) my_dt = softplus20_flat(my_dt);
     if (p.z) {
         const float zv = z_scale * static_cast<float>(z_q);
         gate = zv * (1.0f / (1.0f + expf(-zv)));
@@ -157,18 +169,18 @@ __global__ __launch_bounds__(kThreads) void mamba1_step_kernel(QaSsmUpdateParams
     const float w23 = (odd ? acc[3] : acc[2]) + quad_xor<1>(odd ? acc[2] : acc[3]);
     const float sum = (hi ? w23 : w01) + quad_xor<2>(hi ? w01 : w23);
     const float y = (sum + my_x * (D_scale * static_cast<float>(D_q))) * gate;
-    if (slice < NB && b0 + slice < p.batch) static_cast<__half*>(p.out)[(b0 + slice) * p.out_batch_stride + c] = __float2half(y);
+    if (slice < NB && b0 + slice < p.batch) p.out[static_cast<int64_t>(b0 + slice) * p.out_batch_stride + c] = __float2half(y);
 }
 
 template <bool FP32>
-int launch(const QaSsmUpdateParams& p, const SsmDtProj& dt, hipStream_t stream) {
-    const int64_t blocks = (p.dim / kWaveCh + kWaves - 1) / kWaves;
+int launch(const StepArgs& a, hipStream_t stream) {
+    const int64_t blocks = (a.dim / kWaveCh + kWaves - 1) / kWaves;
     auto go = [&](auto kernel, int nb) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>((p.batch + nb - 1) / nb)), dim3(kThreads), 0, stream, p, dt);
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>((a.batch + nb - 1) / nb)), dim3(kThreads), 0, stream, a);
         return check_launch();
     };
-    if (p.batch == 1) return go(mamba1_step_kernel<1, FP32>, 1);
-    if (p.batch == 2) return go(mamba1_step_kernel<2, FP32>, 2);
+    if (a.batch == 1) return go(mamba1_step_kernel<1, FP32>, 1);
+    if (a.batch == 2) return go(mamba1_step_kernel<2, FP32>, 2);
     return go(mamba1_step_kernel<4, FP32>, 4);
 }
 
@@ -182,7 +194,21 @@ int mamba1_step(const QaSsmUpdateParams& p, const SsmDtProj& dt, hipStream_t str
     if (p.B_dstate_stride != 1 || p.C_dstate_stride != 1 || !mult4(p.B_batch_stride) || !mult4(p.C_batch_stride) || !aligned4(p.B) || !aligned4(p.C)) return QA_ERR_UNSUPPORTED;
     if ((p.D && p.D_dim_stride != 1) || (p.dt_bias && (p.dt_bias_is_fp16 || p.dt_bias_dim_stride != 1))) return QA_ERR_UNSUPPORTED;
     if (dt.pieces < 1 || dt.pieces > kSsmDtPieces || !aligned16(dt.w) || !aligned16(dt.x) || dt.x_batch_stride % 16 != 0) return QA_ERR_UNSUPPORTED;
-    return p.state_is_fp32 ? launch<true>(p, dt, stream) : launch<false>(p, dt, stream);
+    for (const int64_t v : {p.A_dim_stride, p.x_batch_stride, p.z ? p.z_batch_stride : 0, p.B_batch_stride, p.C_batch_stride, p.out_batch_stride, dt.x_batch_stride})
+        if (v < 0 || v > 0x7fffffff) return QA_ERR_UNSUPPORTED;
+    StepArgs a = {};
+    a.state = p.state; a.out = static_cast<__half*>(p.out);
+    a.x = p.x; a.z = p.z; a.A_log = p.A_log; a.B = p.B; a.C = p.C; a.D = p.D; a.dt_bias = static_cast<const int8_t*>(p.dt_bias); a.w = dt.w; a.dt_x = dt.x;
+    a.x_scale = p.x_scale; a.dt_scale = p.dt_scale; a.dt_bias_scale = p.dt_bias_scale; a.A_log_scale = p.A_log_scale; a.state_scale = p.state_scale;
+    a.B_scale = p.B_scale; a.C_scale = p.C_scale; a.D_scale = p.D_scale; a.z_scale = p.z_scale; a.row_scale = dt.row_scale; a.col_scale = dt.col_scale;
+    a.state_batch_stride = p.state_batch_stride;
+    a.batch = p.batch; a.dim = p.dim; a.A_dim_stride = static_cast<int>(p.A_dim_stride);
+    a.x_batch_stride = static_cast<int>(p.x_batch_stride); a.z_batch_stride = static_cast<int>(p.z_batch_stride);
+    a.B_batch_stride = static_cast<int>(p.B_batch_stride); a.C_batch_stride = static_cast<int>(p.C_batch_stride);
+    a.out_batch_stride = static_cast<int>(p.out_batch_stride); a.dt_x_batch_stride = static_cast<int>(dt.x_batch_stride);
+    a.pieces = dt.pieces; a.alpha = dt.alpha;
+    a.softplus = p.dt_softplus != 0; a.use_alpha = dt.use_alpha != 0; a.one_col_scale = dt.col_numel == 1;
+    return p.state_is_fp32 ? launch<true>(a, stream) : launch<false>(a, stream);
 }
 
 }  // namespace qa
