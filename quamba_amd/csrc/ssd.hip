@@ -13,6 +13,7 @@
 // Both fp16 contractions over the time index need x (and B) with time as the fastest-moving index,
 // while memory has channels fastest; the tiles are transposed once on the way into LDS and then read as
 // 16-byte MFMA operands.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -477,9 +478,9 @@ __global__ __launch_bounds__(256) void ssd_pass_kernel(QaSsdParams p, const floa
 }
 
 // ---------------------------------------------------------------------------------------------
-// Stages 4 and 5 (quamba/triton/quant_bmm_chunk.py:60-66, quant_chunk_scan.py:96-171): a workgroup of eight waves
-// per (batch, chunk, head).  A wave owns whole 16-row m-tiles with all 64 channels, a long and a short causal range
-// each (with sixteen tiles: 15 - w and w), the long one first.
+// Stages 4 and 5 (quamba/triton/quant_bmm_chunk.py:60-66, quant_chunk_scan.py:96-171): a workgroup of eight waves takes some
+// heads of one (batch, chunk, group) in turn.  A wave owns whole 16-row m-tiles with all 64 channels, a long and a short
+// causal range each (with sixteen tiles: 15 - w and w).
 // C B^T never exists in memory: the chunk's B codes sit in LDS, a lane holds 32 codes of its row of C, and
 // v_mfma_i32_16x16x64_i8 forms (C B^T)^T in 16 x 16 blocks - exact integers, times s_C s_B in fp32, the value
 // the reference's bmm kernel stores.  A block comes out with a lane per row m and four consecutive steps k, which
@@ -490,43 +491,42 @@ __global__ __launch_bounds__(256) void ssd_pass_kernel(QaSsdParams p, const floa
 // entering state is read in that order.  Below the diagonal the decay factors into exp(dA_m - R) (one exp per
 // lane and piece) and exp(R - dA_k) dt_k (a table per workgroup) with R = dA at the last step of the piece, so
 // that both exponents are <= 0; on the piece that holds the diagonal it is computed per element, in the
-// reference's order.  After the prologue a wave reads global memory only for the bytes of the skip term and gate.
-// With 128 states and chunks of 256 steps two workgroups fit a CU's LDS only if the entering state and the upper
-// half of the B codes share their 16 KB: term 1 of both tiles runs first, then the B codes (held in registers
-// since the prologue) take the state's place.
+// reference's order.  While a head's last tile is computed, what the next head needs from memory is on its way to registers.
+// Moving a head's bytes (the entering state and x in, y out) and computing it take about as long as each other: 89 us of each for
+// 4 x 4096 steps of 80 heads with nothing else in the kernel, and as a workgroup per head, two to a CU, they ran half one
+// after the other.  Walking heads overlaps them and reads the codes of B and C once for all: 158 -> 135 us, 16 x 1024 of
+// 128 257 -> 212, 1 x 1531 of 80 (a head each, so only the shorter code) 21.4 -> 18.9.  The walk has to stay inside 128 registers:
+// with the next head requested ahead of the first tile, or the reads of LDS gathered in front of the products, some values
+// spill, and waiting for a spilled one is waiting for the requests: 144 to 177 us.
+// Two workgroups fit a CU's LDS with 128 states and chunks of 256 steps because the entering state and x take the same place:
+// term 1 of both tiles runs first, x is staged from its registers after it.
 // ---------------------------------------------------------------------------------------------
 template <int N, int Q>
 struct ScanSmem {
-    static constexpr bool ALIAS = N == 128 && Q == 256;
     static constexpr int XP = Q + 8;        // halves per row of the transposed x tile
     static constexpr int NCH = N / 8;       // 16-byte pieces per row of the entering state
     static constexpr int SWZ = (NCH < 16 ? NCH : 16) - 1;
     static constexpr int BSWZ = (N / 16 < 8 ? N / 16 : 8) - 1;
-    static constexpr int BROWS = ALIAS ? Q / 2 : Q;
-    __attribute__((aligned(16))) _Float16 xt[kP][XP];
-    // rows without padding: piece c of row r sits at position c ^ (r & SWZ), so that the sixteen rows of an operand
-    // read fall into different banks
-    __attribute__((aligned(16))) _Float16 prev[kP][N];
-    __attribute__((aligned(16))) int8_t bq[BROWS][N];   // B codes; 16-byte piece c of row k at position c ^ (k & BSWZ)
-    __attribute__((aligned(16))) float dt[Q];
+    // of the head at hand; the entering state first, then x.  The state's rows have no padding: piece c of row r sits
+    // at position c ^ (r & SWZ), so that the sixteen rows of an operand read fall into different banks
+    union {
+        __attribute__((aligned(16))) _Float16 xt[kP][XP];
+        __attribute__((aligned(16))) _Float16 prev[kP][N];
+    };
+    __attribute__((aligned(16))) int8_t bq[Q][N];   // B codes; 16-byte piece c of row k at position c ^ (k & BSWZ)
+    __attribute__((aligned(16))) float dt[Q];   // s_C s_B dt_k
     __attribute__((aligned(16))) float dA[Q];
-    __attribute__((aligned(16))) float gk[Q];   // exp(dA[end of the 32-step piece] - dA_k) dt_k
+    __attribute__((aligned(16))) float gk[Q];   // exp(dA[end of the 32-step piece] - dA_k) s_C s_B dt_k
     __attribute__((aligned(16))) float xs[kP];  // x scale per channel
-    __attribute__((aligned(16))) float Dv[kP];  // skip weight per channel
+    __attribute__((aligned(16))) float xD[kP];  // x scale times skip weight per channel
     __attribute__((aligned(16))) float gate[256];   // SiLU(z_scale code) of the gate's 256 codes, indexed by the code's byte
-    static_assert(!ALIAS || sizeof(_Float16) * kP * N == static_cast<size_t>(Q / 2) * N, "the upper B rows take exactly the state's place");
-    // row k of the B codes
-    __device__ __forceinline__ int8_t* brow(int k) {
-        if (ALIAS && k >= BROWS) return reinterpret_cast<int8_t*>(&prev[0][0]) + (k - BROWS) * N;
-        return bq[k];
-    }
 };
 
 constexpr int scan_waves_of(int Q) { return Q / 16 < 8 ? Q / 16 : 8; }
 
 template <int N, int Q>
 __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kernel(QaSsdParams p, const float* dt_ws, const float* dA_ws,
-                                                                                const __half* prev, const float* xs_ws, int nc) {
+                                                                                const __half* prev, const float* xs_ws, int nc, int heads_each) {
     using S = ScanSmem<N, Q>;
     extern __shared__ __attribute__((aligned(16))) unsigned char ssd_smem_raw[];
     S& sm = *reinterpret_cast<S*>(ssd_smem_raw);
@@ -538,24 +538,23 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
     constexpr int PB = PPC / kThreads;
     constexpr int BPC = Q * N / 16;                               // 16-byte pieces of the B codes
     constexpr int BB = BPC / kThreads;
-    constexpr int BB_NOW = S::ALIAS ? BB / 2 : BB;                // pieces a thread writes in the prologue
-    static_assert(Q <= kThreads, "a thread stages at most one share of the x tile");
-    static_assert(PPC % kThreads == 0 && BPC % kThreads == 0 && (!S::ALIAS || BB % 2 == 0), "whole shares per thread");
+    constexpr int CH = 8;                                         // channels of a thread's share of x
+    constexpr int kShares = Q / 4 * (kP / CH);
+    static_assert(kShares <= kThreads && Q <= kThreads, "a thread stages at most one share of the x tile");
+    static_assert(PPC % kThreads == 0 && BPC % kThreads == 0, "whole shares per thread");
     static_assert(TILES <= 2, "a long and a short tile per wave");
 
-    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lq = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);    // the same in every lane: kept in a scalar register
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);    // the same in every lane: kept in a scalar register
     // (H, h, hp, ch0 as in the state kernel: heads of 64 s channels run as s heads of 64)
     const int split = p.headdim / kP;
     const int G = p.ngroups, H = p.nheads * split, L = p.seqlen;
     // the heads of one (batch, chunk, ssd group) read the same B and C codes: they go to one XCD
-    int unit, hig, part;
-    unit_head_part(blockIdx.x, p.batch * nc * G, H / G, 1, unit, hig, part);
-    const int h = (unit % G) * (H / G) + hig;
-    const int hp = h / split, ch0 = (h % split) * kP;
+    int unit, unused, part;
+    unit_head_part(blockIdx.x, p.batch * nc * G, 1, (H / G + heads_each - 1) / heads_each, unit, unused, part);
+    const int g = unit % G;
     const int c = (unit / G) % nc;
     const int b = unit / (G * nc);
-    const int g = hp / (p.nheads / G);
+    const int h_first = g * (H / G) + part * heads_each, h_last = min(h_first + heads_each, (g + 1) * (H / G)) - 1;
     const bool grouped = p.nhead_groups > 0;
     const float sC = grouped ? p.C_scale[g] : p.C_scale[0];
     const float cb_scale = sC * (grouped ? p.B_scale[g] : p.B_scale[0]);
@@ -563,37 +562,53 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
     const int lim = min(Q, L - t0);
     const uint32_t xrow = static_cast<uint32_t>(H) * kP;          // bytes between steps of x
     const uint32_t crow = static_cast<uint32_t>(G) * N;           // bytes between steps of B and C
-    const int8_t* xbase = p.x + (static_cast<int64_t>(b) * L + t0) * xrow + static_cast<int64_t>(h) * kP;
-    const int8_t* zbase = p.z + (static_cast<int64_t>(b) * L + t0) * xrow + static_cast<int64_t>(h) * kP;       // only read if p.z
+    const int64_t row0 = (static_cast<int64_t>(b) * L + t0) * xrow;
     const int8_t* Bbase = p.B + (static_cast<int64_t>(b) * L + t0) * crow + static_cast<int64_t>(g) * N;
     const int8_t* Cbase = p.C + (static_cast<int64_t>(b) * L + t0) * crow + static_cast<int64_t>(g) * N;
     const float D_scale = p.D ? *p.D_scale : 0.0f;
     const float z_scale = p.z ? *p.z_scale : 0.0f;
-    __half* out = static_cast<__half*>(p.out) + (static_cast<int64_t>(b) * L + t0) * xrow + static_cast<int64_t>(h) * kP;
 
     // tile s of this wave
     auto tile_of = [&](int s) { return (s & 1) == 0 ? NMT - 1 - 8 * (s / 2) - wave : 8 * ((TILES - 1 - s) / 2) + wave; };
 
-    // codes of C of this lane's rows: states 64 i + 16 q .. + 15 (rows past the end of the sequence read the last
-    // row; nothing of theirs is stored)
-    v4i cq[TILES][N / 64];
-    v4i r_b[BB];
-    {
-        // Prologue: every global read is issued before the first LDS write, so that the workgroup waits for memory
-        // once.
-        float r_dt = 0.0f, r_dA = 0.0f, r_end = 0.0f;
-        if (tid < Q) {
+    // what a head needs from memory, fetched into registers while the head before it is computed.  Unconditional (the
+    // last head is requested once more and never staged), and one path for whole and ragged chunks: rows past the end of
+    // the sequence read the last row and are zeroed when the tile is staged.  With a second path beside it the compiler
+    // merges the two sets of destination registers by copies right behind the loads, i.e. waits for them there.
+    float r_dt = 0.0f, r_dA = 0.0f, r_xs = 0.0f, r_D = 0.0f;
+    v4i r_prev[PB];
+    XShare<CH> xr[4];                                             // steps 4 kb .. 4 kb + 3, channels xc .. xc + 7
+    auto fetch_head = [&](int h, int tid) {
+        const int xc = tid % (kP / CH) * CH, kb = tid / (kP / CH);
+        const int hp = h / split, ch0 = (h % split) * kP;
+        if (Q == kThreads || tid < Q) {
             const int64_t row = ((static_cast<int64_t>(b) * p.nheads + hp) * nc + c) * Q;
             r_dt = dt_ws[row + tid];
             r_dA = dA_ws[row + tid];
-            r_end = dA_ws[row + (tid | 31)];
+        }
+        if (tid < kP) {
+            r_xs = xs_ws[hp * p.headdim + ch0 + tid];
+            if (p.D) r_D = static_cast<float>(p.D_has_hdim ? p.D[hp * p.headdim + ch0 + tid] : p.D[hp]);
         }
         // (the first chunk has no entering state: its slot of the workspace is read all the same and never used)
-        v4i r_prev[PB];
         const __half* pst = prev + ((static_cast<int64_t>(b) * nc + c) * H + h) * kP * N;
 #pragma unroll
         for (int i = 0; i < PB; ++i) r_prev[i] = *reinterpret_cast<const v4i*>(pst + (tid + i * kThreads) * 8);
-        // the chunk's B codes
+        if (kShares == kThreads || tid < kShares) {
+            const int8_t* from = p.x + row0 + static_cast<int64_t>(h) * kP;
+            const uint32_t last_x = static_cast<uint32_t>(lim - 1) * xrow + xc, voff_x = static_cast<uint32_t>(4 * kb) * xrow + xc;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) xr[r] = load_x_share<CH>(from + static_cast<uint64_t>(min(voff_x + static_cast<uint32_t>(r) * xrow, last_x)));
+        }
+    };
+
+    // codes of C of this lane's rows: states 64 i + 16 q .. + 15 (rows past the end of the sequence read the last
+    // row; nothing of theirs is stored)
+    v4i cq[TILES][N / 64];
+    {
+        // every global read of the prologue is issued before the first LDS write, so that the workgroup waits once
+        const int tid = threadIdx.x, l16 = tid & 15, lq = (tid & 63) >> 4;
+        v4i r_b[BB];
 #pragma unroll
         for (int i = 0; i < BB; ++i) {
             const int piece = tid + i * kThreads, k = piece / (N / 16), col = piece % (N / 16);
@@ -605,24 +620,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
 #pragma unroll
             for (int i = 0; i < N / 64; ++i) cq[s][i] = *reinterpret_cast<const v4i*>(cp + 64 * i);
         }
-        // (requested last: the compiler moves the loaded words into other registers right behind these loads, i.e.
-        // waits for them here, and everything else is then already on its way)
-        // this thread's share of the x tile: steps 4 kb .. 4 kb + 3, channels 16 pb .. 16 pb + 15
-        const int pb = tid % 4, kb = tid / 4;
-        const bool mine = Q == kThreads || tid < Q;
-        // (one path for whole and ragged chunks: rows past the end of the sequence read the last row and are zeroed
-        // when the tile is staged; with a second path beside it the compiler merges the two sets of destination
-        // registers by copies right behind the loads and so waits for them before the requests below are issued)
-        XShare<16> xr[4];
-        if (mine) {
-            const uint32_t last_x = static_cast<uint32_t>(lim - 1) * xrow + 16 * pb, voff_x = static_cast<uint32_t>(4 * kb) * xrow + 16 * pb;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) xr[r] = load_x_share<16>(xbase + static_cast<uint64_t>(min(voff_x + static_cast<uint32_t>(r) * xrow, last_x)));
-        }
-        if (tid < kP) {
-            sm.xs[tid] = xs_ws[hp * p.headdim + ch0 + tid];
-            sm.Dv[tid] = !p.D ? 0.0f : D_scale * static_cast<float>(p.D_has_hdim ? p.D[hp * p.headdim + ch0 + tid] : p.D[hp]);
-        }
+        fetch_head(h_first, tid);
         if (p.z) {
             // the gate has 256 possible values: evaluated once per workgroup, looked up per output
             for (int i = tid; i < 256; i += kThreads) {
@@ -630,172 +628,186 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                 sm.gate[i] = zv * __builtin_amdgcn_rcpf(1.0f + fexp(-zv));
             }
         }
-        __syncthreads();                                           // the tables per channel (and every load above has landed)
+#pragma unroll
+        for (int i = 0; i < BB; ++i) {
+            const int piece = tid + i * kThreads, k = piece / (N / 16), col = piece % (N / 16);
+            *reinterpret_cast<v4i*>(&sm.bq[k][(col ^ (k & S::BSWZ)) * 16]) = r_b[i];
+        }
+    }
 
+    for (int h = h_first; h <= h_last; ++h) {
+        const int8_t* xbase = p.x + row0 + static_cast<int64_t>(h) * kP;
+        const int8_t* zbase = p.z + row0 + static_cast<int64_t>(h) * kP;       // only read if p.z
+        // (opaque: the addresses of a head's steps, kept from head to head, are more than the registers hold, and so are the codes
+        // of C as fp16)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, l16 = lane & 15, lq = lane >> 4;
+#pragma unroll
+        for (int s = 0; s < TILES; ++s)
+#pragma unroll
+            for (int i = 0; i < N / 64; ++i) asm volatile("" : "+v"(cq[s][i]));
+        __half* out = static_cast<__half*>(p.out) + row0 + static_cast<int64_t>(h) * kP;
+        if (tid < kP) {
+            sm.xs[tid] = r_xs;
+            sm.xD[tid] = r_xs * (D_scale * r_D);
+        }
         if (tid < Q) {
-            sm.dt[tid] = r_dt;
+            const float scaled = cb_scale * r_dt;
+            sm.dt[tid] = scaled;
             sm.dA[tid] = r_dA;
-            sm.gk[tid] = fexp(r_end - r_dA) * r_dt;
+            sm.gk[tid] = fexp(__shfl(r_dA, lane | 31) - r_dA) * scaled;
         }
 #pragma unroll
         for (int i = 0; i < PB; ++i) {
             const int piece = tid + i * kThreads, pr = piece / (N / 8), col = (piece % (N / 8)) * 8;
             *reinterpret_cast<v4i*>(&sm.prev[pr][col ^ ((pr & S::SWZ) * 8)]) = r_prev[i];
         }
+        __syncthreads();
+
+        // term 1 of every tile of the wave: C^ (rows m) x entering state (rows p), zero for the first chunk
+        v4f acc[TILES][4];
 #pragma unroll
-        for (int i = 0; i < BB_NOW; ++i) {
-            const int piece = tid + i * kThreads, k = piece / (N / 16), col = piece % (N / 16);
-            *reinterpret_cast<v4i*>(sm.brow(k) + (col ^ (k & S::BSWZ)) * 16) = r_b[i];
+        for (int s = 0; s < TILES; ++s) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[s][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            if (c > 0) {
+                const int m0 = tile_of(s) * 16;
+#pragma unroll
+                for (int ks = 0; ks < N / 32; ++ks) {
+                    const uint32_t w0 = static_cast<uint32_t>(cq[s][ks / 2][2 * (ks % 2)]), w1 = static_cast<uint32_t>(cq[s][ks / 2][2 * (ks % 2) + 1]);
+                    v8h cf;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        cf[e] = static_cast<_Float16>(sC * sbyte_of(w0, e));
+                        cf[4 + e] = static_cast<_Float16>(sC * sbyte_of(w1, e));
+                    }
+                    const int n0 = 64 * (ks / 2) + 16 * lq + 8 * (ks % 2);     // the states of those eight codes
+                    v8h fs[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) fs[j] = *reinterpret_cast<const v8h*>(&sm.prev[j * 16 + l16][n0 ^ ((l16 & S::SWZ) * 8)]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[s][j] = mfma16(cf, fs[j], acc[s][j]);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float em = fexp(sm.dA[m0 + 4 * lq + r]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[s][j][r] *= em;
+                }
+            }
         }
-        if (mine) {
+        __syncthreads();                                               // everyone is done with the entering state
+        if (kShares == kThreads || tid < kShares) {
+            const int xc = tid % (kP / CH) * CH, kb = tid / (kP / CH);
             if (lim < Q) {
                 // ragged last chunk: steps past the end of the sequence count as zero
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    if (4 * kb + r >= lim) xr[r] = XShare<16>{};
+                    if (4 * kb + r >= lim) xr[r] = XShare<CH>{};
                 }
             }
-            stage_x_share<S::XP, 16>(sm.xt, xr, sm.xs, 16 * pb, kb);
-        }
-    }
-    __syncthreads();
-
-    // term 1 of every tile of the wave: C^ (rows m) x entering state (rows p), zero for the first chunk
-    v4f acc[TILES][4];
-#pragma unroll
-    for (int s = 0; s < TILES; ++s) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[s][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        if (c > 0) {
-            const int m0 = tile_of(s) * 16;
-#pragma unroll
-            for (int ks = 0; ks < N / 32; ++ks) {
-                const uint32_t w0 = static_cast<uint32_t>(cq[s][ks / 2][2 * (ks % 2)]), w1 = static_cast<uint32_t>(cq[s][ks / 2][2 * (ks % 2) + 1]);
-                v8h cf;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    cf[e] = static_cast<_Float16>(sC * static_cast<float>(byte_of(w0, e)));
-                    cf[4 + e] = static_cast<_Float16>(sC * static_cast<float>(byte_of(w1, e)));
-                }
-                const int n0 = 64 * (ks / 2) + 16 * lq + 8 * (ks % 2);     // the states of those eight codes
-                v8h fs[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) fs[j] = *reinterpret_cast<const v8h*>(&sm.prev[j * 16 + l16][n0 ^ ((l16 & S::SWZ) * 8)]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[s][j] = mfma16(cf, fs[j], acc[s][j]);
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float em = fexp(sm.dA[m0 + 4 * lq + r]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[s][j][r] *= em;
-            }
-        }
-    }
-    if constexpr (S::ALIAS) {
-        __syncthreads();                                           // everyone is done with the entering state
-#pragma unroll
-        for (int i = BB_NOW; i < BB; ++i) {
-            const int piece = tid + i * kThreads, k = piece / (N / 16), col = piece % (N / 16);
-            *reinterpret_cast<v4i*>(sm.brow(k) + (col ^ (k & S::BSWZ)) * 16) = r_b[i];
+            stage_x_share<S::XP, CH>(sm.xt, xr, sm.xs, xc, kb);
         }
         __syncthreads();
-    }
 
+        // the short tile first, the next head's requests with the long one: by then the first tile's sums have left their registers
 #pragma unroll
-    for (int s = 0; s < TILES; ++s) {
-        // the most pieces a tile in position s can have (position 0 holds the longest tiles)
-        const int max_tile = (s & 1) == 0 ? NMT - 1 - 8 * (s / 2) : 8 * ((TILES - 1 - s) / 2) + kWaves - 1;
-        const int max_nks = (max_tile + 2) / 2;
-        const int mt = tile_of(s);
-        const int m0 = mt * 16;
-        const int nks = (mt + 2) / 2;                               // 32-step pieces that reach row m0 + 15; the last holds the diagonal
-        const int m_row = m0 + l16;                                 // row of this lane's first operands
-        const float dA_m = sm.dA[m_row];
-        // skip-term operands of this lane's four output rows
-        // (requested now, used in the epilogue: nothing there waits for memory)
-        uint32_t xq[4], zq[4] = {0u, 0u, 0u, 0u};
+        for (int s = TILES - 1; s >= 0; --s) {
+            if (s == 0) {
+                fetch_head(min(h + 1, h_last), tid);
+                __builtin_amdgcn_sched_barrier(0);                     // (the scheduler would sink the requests below the products)
+            }
+            const int mt = tile_of(s);
+            const int m0 = mt * 16;
+            const int nks = (mt + 2) / 2;                               // 32-step pieces that reach row m0 + 15; the last holds the diagonal
+            const int m_row = m0 + l16;                                 // row of this lane's first operands
+            const float dA_m = sm.dA[m_row];
+            // skip-term operands of this lane's four output rows
+            // (requested now, used in the epilogue: nothing there waits for memory)
+            uint32_t xq[4], zq[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t at = static_cast<uint32_t>(min(m0 + 4 * lq + r, lim - 1)) * xrow + 4 * l16;
-            xq[r] = *reinterpret_cast<const uint32_t*>(xbase + at);
-            if (p.z) zq[r] = *reinterpret_cast<const uint32_t*>(zbase + at);
-        }
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t at = static_cast<uint32_t>(min(m0 + 4 * lq + r, lim - 1)) * xrow + 4 * l16;
+                xq[r] = *reinterpret_cast<const uint32_t*>(xbase + at);
+                if (p.z) zq[r] = *reinterpret_cast<const uint32_t*>(zbase + at);
+            }
+            // (C B^T)^T of a 16-step block of piece ks: a lane has four steps of its row
+            auto cb_of = [&](int ks, int blk) {
+                v4i cb = v4i{0, 0, 0, 0};
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            if (ks < max_nks && ks < nks) {
-                // steps of this lane's eight values: ka .. ka + 3 and ka + 16 .. ka + 19
-                const int ka = 32 * ks + 4 * lq;
-                // (C B^T)^T for the two 16-step blocks of the piece
-                v4i cbi[2];
-#pragma unroll
-                for (int blk = 0; blk < 2; ++blk) {
-                    const int k = 32 * ks + 16 * blk + l16;
-                    const int8_t* brow = sm.brow(32 * ks + 16 * blk) + l16 * N;
-                    cbi[blk] = v4i{0, 0, 0, 0};
-#pragma unroll
-                    for (int i = 0; i < N / 64; ++i) {
-                        const v4i bo = *reinterpret_cast<const v4i*>(brow + (((4 * i + lq) ^ (k & S::BSWZ)) * 16));
-                        cbi[blk] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bo, cq[s][i], cbi[blk], 0, 0, 0);
-                    }
+                for (int i = 0; i < N / 64; ++i) {
+                    const v4i bo = *reinterpret_cast<const v4i*>(&sm.bq[32 * ks + 16 * blk + l16][((4 * i + lq) ^ (l16 & S::BSWZ)) * 16]);
+                    cb = __builtin_amdgcn_mfma_i32_16x16x64_i8(bo, cq[s][i], cb, 0, 0, 0);
                 }
-                v8h fx[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const v4h x0 = *reinterpret_cast<const v4h*>(&sm.xt[j * 16 + l16][ka]);
-                    const v4h x1 = *reinterpret_cast<const v4h*>(&sm.xt[j * 16 + l16][ka + 16]);
-                    fx[j] = v8h{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-                }
-                float cv[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) cv[e] = static_cast<float>(cbi[e / 4][e % 4]);
-                float wv[8];
-                if (ks + 1 < nks) {
-                    const float4 g0 = *reinterpret_cast<const float4*>(&sm.gk[ka]), g1 = *reinterpret_cast<const float4*>(&sm.gk[ka + 16]);
-                    const float gk[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-                    const float e_m = cb_scale * fexp(dA_m - sm.dA[32 * ks + 31]);      // the scale of C B^T rides with the row's decay
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) wv[e] = cv[e] * (e_m * gk[e]);
-                } else {
-                    // the piece with the diagonal: steps after row m do not count
-                    const float4 a0 = *reinterpret_cast<const float4*>(&sm.dA[ka]), a1 = *reinterpret_cast<const float4*>(&sm.dA[ka + 16]);
-                    const float4 d0 = *reinterpret_cast<const float4*>(&sm.dt[ka]), d1 = *reinterpret_cast<const float4*>(&sm.dt[ka + 16]);
-                    const float ak[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-                    const float dk[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int k = ka + 16 * (e / 4) + e % 4;
-                        wv[e] = ((k <= m_row ? cb_scale * cv[e] : 0.0f) * fexp(fminf(dA_m - ak[e], 0.0f))) * dk[e];
-                    }
-                }
+                return cb;
+            };
+            // the weights of steps 32 ks + 4 q .. + 3 and 32 ks + 16 + 4 q .. + 3 times x
+            auto times_x = [&](int ks, const float (&wv)[8]) {
                 v8h fl;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) fl[e] = static_cast<_Float16>(wv[e]);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[s][j] = mfma16(fl, fx[j], acc[s][j]);
+                for (int j = 0; j < 4; ++j) {
+                    const v4h x0 = *reinterpret_cast<const v4h*>(&sm.xt[j * 16 + l16][32 * ks + 4 * lq]);
+                    const v4h x1 = *reinterpret_cast<const v4h*>(&sm.xt[j * 16 + l16][32 * ks + 4 * lq + 16]);
+                    acc[s][j] = mfma16(fl, v8h{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, acc[s][j]);
+                }
+            };
+            float wv[8];
+#pragma unroll 1
+            for (int ks = 0; ks + 1 < nks; ++ks) {
+                const int ka = 32 * ks + 4 * lq;
+                const v4i cb[2] = {cb_of(ks, 0), cb_of(ks, 1)};
+                const float4 g0 = *reinterpret_cast<const float4*>(&sm.gk[ka]), g1 = *reinterpret_cast<const float4*>(&sm.gk[ka + 16]);
+                const float gk[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+                const float e_m = fexp(dA_m - sm.dA[32 * ks + 31]);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) wv[e] = static_cast<float>(cb[e / 4][e % 4]) * (e_m * gk[e]);
+                times_x(ks, wv);
+            }
+            // the piece with the diagonal: steps after row m do not count, nor does all of the second block of an even tile
+            auto diagonal = [&](int blk) {
+                const int ka = 32 * (nks - 1) + 16 * blk + 4 * lq;
+                const v4i cb = cb_of(nks - 1, blk);
+                const float4 a4 = *reinterpret_cast<const float4*>(&sm.dA[ka]), d4 = *reinterpret_cast<const float4*>(&sm.dt[ka]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float cv = ka + e <= m_row ? static_cast<float>(cb[e]) : 0.0f;
+                    wv[4 * blk + e] = (cv * fexp(fminf(dA_m - lane_of(a4, e), 0.0f))) * lane_of(d4, e);
+                }
+            };
+            diagonal(0);
+            if (mt & 1) {
+                diagonal(1);
+            } else {
+#pragma unroll
+                for (int e = 4; e < 8; ++e) wv[e] = 0.0f;
+            }
+            times_x(nks - 1, wv);
+            // Epilogue: acc[s][j][r] is row m0 + 4 (lane / 16) + r, channel 4 (lane % 16) + j
+            const float4 xD4 = *reinterpret_cast<const float4*>(&sm.xD[4 * l16]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = m0 + 4 * lq + r;
+                if (m < lim) {
+                    float y[4] = {acc[s][0][r], acc[s][1][r], acc[s][2][r], acc[s][3][r]};
+                    if (p.D) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) y[j] = __builtin_fmaf(sbyte_of(xq[r], j), lane_of(xD4, j), y[j]);
+                    }
+                    if (p.z) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) y[j] *= sm.gate[(zq[r] >> (8 * j)) & 0xffu];
+                    }
+                    v4h o;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) o[j] = static_cast<_Float16>(y[j]);
+                    *reinterpret_cast<v4h*>(out + static_cast<uint32_t>(m) * xrow + 4 * l16) = o;
+                }
             }
         }
-        // Epilogue: acc[s][j][r] is row m0 + 4 (lane / 16) + r, channel 4 (lane % 16) + j
-        const float4 xs4 = *reinterpret_cast<const float4*>(&sm.xs[4 * l16]), Dv4 = *reinterpret_cast<const float4*>(&sm.Dv[4 * l16]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = m0 + 4 * lq + r;
-            if (m < lim) {
-                float y[4] = {acc[s][0][r], acc[s][1][r], acc[s][2][r], acc[s][3][r]};
-                if (p.D) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) y[j] += __builtin_fmaf(ubyte_of(xq[r] ^ kBias, j), lane_of(xs4, j), -128.0f * lane_of(xs4, j)) * lane_of(Dv4, j);
-                }
-                if (p.z) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) y[j] *= sm.gate[(zq[r] >> (8 * j)) & 0xffu];
-                }
-                v4h o;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) o[j] = static_cast<_Float16>(y[j]);
-                *reinterpret_cast<v4h*>(out + static_cast<uint32_t>(m) * xrow + 4 * l16) = o;
-            }
-        }
+        __syncthreads();                                               // everyone is done with this head's tile and tables
     }
 }
 
@@ -889,7 +901,12 @@ extern "C" int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream_) {
         } else {
             hipLaunchKernelGGL(state_kernel, hgrid, dim3(4 * p->dstate), state_lds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws, srow_ws, nc);
         }
-        hipLaunchKernelGGL(scan_kernel, dim3(static_cast<unsigned>(bch * (p->headdim / 64))), dim3(scan_threads), scan_lds, stream, *p, dt_ws, dA_ws, prev_ws, xs_ws, nc);
+        const int hpg = heads64 / p->ngroups, units = static_cast<int>(bch / p->nheads) * p->ngroups;
+        // as many workgroups as the chip holds at once (sixteen waves of up to 128 registers to a CU), each with its share of a group's heads
+        const int64_t places = static_cast<int64_t>(compute_units()) * (1024 / scan_threads);
+        const int heads_each = static_cast<int>(std::min<int64_t>((static_cast<int64_t>(units) * hpg + places - 1) / places, hpg));
+        hipLaunchKernelGGL(scan_kernel, dim3(static_cast<unsigned>(units * ((hpg + heads_each - 1) / heads_each))), dim3(scan_threads), scan_lds, stream, *p, dt_ws, dA_ws, prev_ws, xs_ws, nc,
+                           heads_each);
     };
 #define QA_SSD_LAUNCH(N_, Q_) launch(ssd_state_kernel<N_, Q_, true>, ssd_state_kernel<N_, Q_, false>, ssd_pass_kernel<N_>, sizeof(StateSmem<N_, Q_>), ssd_chunk_scan_kernel<N_, Q_>, \
                                      sizeof(ScanSmem<N_, Q_>), 64 * scan_waves_of(Q_))

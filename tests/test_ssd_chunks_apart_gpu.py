@@ -31,3 +31,26 @@ def test_one_entry_at_a_time(dev, B, L, N, G, Q, final_dtype):
         y1, final1 = run(slice(b, b + 1))
         assert torch.equal(y1[0], y[b]) and torch.equal(final1[0], final[b])
     assert float(y.float().abs().max()) > 0.1
+
+
+# with more heads in flight than the chip holds workgroups, a workgroup walks some heads of a (batch, chunk, group), the last one
+# of a group fewer: every chunk length, heads of 64 and of 128 channels, with and without gate and skip weights per channel
+@pytest.mark.parametrize("B,L,H,P,N,G,Q,per_channel", [(4, 1100, 27, 64, 128, 1, 256, False), (9, 300, 48, 64, 64, 3, 128, True),
+                                                       (5, 500, 56, 64, 128, 2, 64, False), (16, 600, 13, 128, 128, 1, 256, True)])
+def test_heads_walked_by_a_workgroup(dev, B, L, H, P, N, G, Q, per_channel):
+    d = synth.mamba2_ssd_inputs(B, L, H, P, N, G, seed=H, with_z=per_channel)
+    if per_channel:
+        d["D"] = np.random.default_rng(1).integers(-128, 128, (H, P)).astype(np.int8)
+    t = lambda a: None if a is None else torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    s = lambda v: None if v is None else torch.tensor(np.asarray(v, np.float32)).to(dev)
+
+    def run(sel):
+        return ops.ssd_chunk_scan_combined_fwd(
+            t(d["x"][sel]), s(d["x_scale"]), t(d["dt"][sel]), s(d["s_dt"]), t(d["A_log"]), s(d["s_A"]), t(d["B"][sel]), s(d["s_B"]),
+            t(d["C"][sel]), s(d["s_C"]), None, Q, q_D=t(d["D"]), D_scale=s(d["s_D"]), q_z=t(d["z"][sel]) if per_channel else None,
+            z_scale=s(d["s_z"]), dt_bias=t(d["dt_bias"]), dt_softplus=True, final_state_dtype=torch.float32)[0]
+
+    y = run(slice(None))
+    for b in range(B):
+        assert torch.equal(run(slice(b, b + 1))[0], y[b])
+    assert float(y.float().abs().max()) > 0.1
