@@ -610,10 +610,11 @@ int cheapest_way(const QaGemmW4A8Params& p, int cus, const SplitChoice& split, b
     WayChoice best = cheapest_tile(p.m, p.n, p.k, cus);
     if (split.shape >= 0) best.offer(kWaySplit, split.us);
     if (expandable) {
-        // (the int8 x int8 kernel takes the smallest tile that fits one round, see there)
-        auto rounds = [&](int64_t bm, int64_t bn) { return static_cast<double>((tiles_of(p, bm, bn) + cus - 1) / cus); };
-        const double step = rounds(64, 64) <= 1 ? 0.25 : rounds(128, 64) <= 1 ? 0.33 : rounds(128, 128) <= 1 ? 0.50 : rounds(128, 256) <= 1 ? 0.75 : 1.55 * rounds(256, 256);
-        best.offer(kWayExpandOnce, 2.5 + static_cast<double>(p.n) * p.k / 3.1e6 + 5.0 + step * (p.k / 128));
+        // (the int8 x int8 kernel's own estimate up to a round of its 128 x 256 tiles, see there, with weights that come from the
+        // pass before: 777 x 2560 x 5120 takes 6.6 + 21.4 us)
+        const double rounds = static_cast<double>((tiles_of(p, 256, 256) + cus - 1) / cus);
+        const double w8 = tiles_of(p, 128, 256) <= cus ? tiles_us_w8(p.m, p.n, p.k, cus) + 0.6 : 5.0 + 1.55 * rounds * (p.k / 128);
+        best.offer(kWayExpandOnce, 5.1 + static_cast<double>(p.n) * p.k / 3.1e6 + w8);
     }
     return best.way;
 }

@@ -92,7 +92,11 @@ inline SplitChoice split_choice(int bits, int m, int n, int k, int cus) {
         if (s.fixed[bits == 4] < 0.0f) continue;
         const int64_t tiles = static_cast<int64_t>((m + s.rows - 1) / s.rows) * ((n + s.cols - 1) / s.cols);
         const float rounds = static_cast<float>((tiles + cus - 1) / cus), units = static_cast<float>((k + 127) / 128);
-        const float us = 2.9f + rounds * (s.fixed[bits == 4] + s.per_unit[bits == 4] * units);
+        // (workgroups that share a CU expand their codes at the same time, which tells from two of the large tiles and from five of the
+        // others on: 777 x 2560 x 5120 with 4 bits 33.4 us by 64 x 48, 28.0 expanded once; 777 x 1536 x 3072 17.3 by 64 x 48, 18.3 by
+        // 32 x 32, 16.9 in 64 x 128 tiles; 100 x 18560 x 4096 37.5 by 64 x 80, 25.4 in 128 x 128 tiles)
+        const float crowd = bits == 4 && rounds > (s.rows == 64 ? 1.0f : 4.0f) ? 1.3f : 1.0f;
+        const float us = 2.9f + rounds * crowd * (s.fixed[bits == 4] + s.per_unit[bits == 4] * units);
         if (tiles <= 0x7fffffff && us < best.us) best = {i, us};
     }
     return best;
