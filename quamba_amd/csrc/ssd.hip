@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "mixer_common.hpp"
 #include "ssd_common.hpp"
@@ -422,6 +423,7 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
 
 // The same with few heads in flight: a workgroup per chunk (WALK false) leaves the chunk's own sums S_c in memory as fp32, rows
 // in slot order, and this kernel runs the recurrence over them, four states a thread: the same values in the same order.
+// (Up to kChainChunks chunks the chunk scan does it itself.)
 template <int N>
 __global__ __launch_bounds__(256) void ssd_pass_kernel(QaSsdParams p, const float* dA_ws, __half* prev, const float* sums, const int32_t* srow_ws, int nc) {
     constexpr int kPieces = kP * N / 4;                           // of one head of 64 channels
@@ -524,9 +526,18 @@ struct ScanSmem {
 
 constexpr int scan_waves_of(int Q) { return Q / 16 < 8 ? Q / 16 : 8; }
 
-template <int N, int Q>
-__global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kernel(QaSsdParams p, const float* dt_ws, const float* dA_ws,
-                                                                                const __half* prev, const float* xs_ws, int nc, int heads_each) {
+// One head, some in turn, or one whose entering state the workgroup makes itself from the chunks' own sums (the first chunk's
+// workgroup then leaves the final state).
+enum ScanMode { kScanOne, kScanWalk, kScanChain };
+// With few chunks a workgroup per chunk and head reads the sums of the chunks before its own faster than a launch of its own passes
+// the states on (pass and scan against the scan alone, us: 6 chunks of 80 heads 27.2 -> 21.0, 4 of 128 27.5 -> 22.6, 8 of 48 24.1 ->
+// 20.4, 2 of 80 15.5 -> 15.8 and a launch less to make).  What is read grows with the square of the chunks - 16 of 80 heads read 300 MB -
+// and with heads to walk the sums would have no registers.
+constexpr int kChainChunks = 8;
+
+template <int N, int Q, ScanMode MODE>
+__global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kernel(QaSsdParams p, const float* dt_ws, const float* dA_ws, const __half* prev, const float* sums,
+                                                                                const float* xs_ws, const int32_t* srow_ws, int nc, int heads_each) {
     using S = ScanSmem<N, Q>;
     extern __shared__ __attribute__((aligned(16))) unsigned char ssd_smem_raw[];
     S& sm = *reinterpret_cast<S*>(ssd_smem_raw);
@@ -548,9 +559,16 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
     // (H, h, hp, ch0 as in the state kernel: heads of 64 s channels run as s heads of 64)
     const int split = p.headdim / kP;
     const int G = p.ngroups, H = p.nheads * split, L = p.seqlen;
-    // the heads of one (batch, chunk, ssd group) read the same B and C codes: they go to one XCD
+    // the heads of one (batch, chunk, ssd group) read the same B and C codes: they go to one XCD.  Not where a workgroup reads
+    // the chunks before its own: the last chunk's would all draw on one XCD's share of the memory
     int unit, unused, part;
-    unit_head_part(blockIdx.x, p.batch * nc * G, 1, (H / G + heads_each - 1) / heads_each, unit, unused, part);
+    const int parts = (H / G + heads_each - 1) / heads_each;
+    if constexpr (MODE == kScanChain) {
+        unit = blockIdx.x / parts;
+        part = blockIdx.x % parts;
+    } else {
+        unit_head_part(blockIdx.x, p.batch * nc * G, 1, parts, unit, unused, part);
+    }
     const int g = unit % G;
     const int c = (unit / G) % nc;
     const int b = unit / (G * nc);
@@ -590,15 +608,52 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
             r_xs = xs_ws[hp * p.headdim + ch0 + tid];
             if (p.D) r_D = static_cast<float>(p.D_has_hdim ? p.D[hp * p.headdim + ch0 + tid] : p.D[hp]);
         }
-        // (the first chunk has no entering state: its slot of the workspace is read all the same and never used)
-        const __half* pst = prev + ((static_cast<int64_t>(b) * nc + c) * H + h) * kP * N;
+        if constexpr (MODE != kScanChain) {
+            // (the first chunk has no entering state: its slot of the workspace is read all the same and never used)
+            const __half* pst = prev + ((static_cast<int64_t>(b) * nc + c) * H + h) * kP * N;
 #pragma unroll
-        for (int i = 0; i < PB; ++i) r_prev[i] = *reinterpret_cast<const v4i*>(pst + (tid + i * kThreads) * 8);
+            for (int i = 0; i < PB; ++i) r_prev[i] = *reinterpret_cast<const v4i*>(pst + (tid + i * kThreads) * 8);
+        }
         if (kShares == kThreads || tid < kShares) {
             const int8_t* from = p.x + row0 + static_cast<int64_t>(h) * kP;
             const uint32_t last_x = static_cast<uint32_t>(lim - 1) * xrow + xc, voff_x = static_cast<uint32_t>(4 * kb) * xrow + xc;
 #pragma unroll
             for (int r = 0; r < 4; ++r) xr[r] = load_x_share<CH>(from + static_cast<uint64_t>(min(voff_x + static_cast<uint32_t>(r) * xrow, last_x)));
+        }
+    };
+
+    // states 8 (tid + i kThreads) .. + 7 of the state entering chunk `end`, rows in slot order: the recurrence of ssd_pass_kernel, the
+    // same values in the same order
+    auto chain = [&](float (&run)[PB][8], int tid, int end) {
+        constexpr int kAtOnce = 4;                                 // chunks requested together
+        const int64_t step = static_cast<int64_t>(H) * kP * N;
+        const float* from = sums + ((static_cast<int64_t>(b) * nc) * H + h_first) * kP * N + tid * 8;
+        const float* dA_last = dA_ws + (static_cast<int64_t>(b) * p.nheads + h_first / split) * nc * Q + Q - 1;
+#pragma unroll
+        for (int i = 0; i < PB; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) run[i][e] = 0.0f;
+        for (int c0 = 0; c0 < end; c0 += kAtOnce) {
+            float4 sum[kAtOnce][PB][2];
+            float d[kAtOnce];
+#pragma unroll
+            for (int k = 0; k < kAtOnce; ++k) {
+                const int cc = min(c0 + k, end - 1);
+                d[k] = dA_last[static_cast<int64_t>(cc) * Q];
+#pragma unroll
+                for (int i = 0; i < PB; ++i)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) sum[k][i][q] = *reinterpret_cast<const float4*>(from + cc * step + i * (8 * kThreads) + 4 * q);
+            }
+#pragma unroll
+            for (int k = 0; k < kAtOnce; ++k) {
+                if (c0 + k >= end) break;
+                const float decay = fexp(d[k]);
+#pragma unroll
+                for (int i = 0; i < PB; ++i)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) run[i][e] = decay * run[i][e] + lane_of(sum[k][i][e / 4], e % 4);
+            }
         }
     };
 
@@ -621,6 +676,17 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
             for (int i = 0; i < N / 64; ++i) cq[s][i] = *reinterpret_cast<const v4i*>(cp + 64 * i);
         }
         fetch_head(h_first, tid);
+        if constexpr (MODE == kScanChain) {
+            float run[PB][8];
+            chain(run, tid, c);
+#pragma unroll
+            for (int i = 0; i < PB; ++i) {
+                v8h o;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = static_cast<_Float16>(run[i][e]);
+                r_prev[i] = __builtin_bit_cast(v4i, o);
+            }
+        }
         if (p.z) {
             // the gate has 256 possible values: evaluated once per workgroup, looked up per output
             for (int i = tid; i < 256; i += kThreads) {
@@ -714,7 +780,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
         // the short tile first, the next head's requests with the long one: by then the first tile's sums have left their registers
 #pragma unroll
         for (int s = TILES - 1; s >= 0; --s) {
-            if (s == 0) {
+            if (MODE == kScanWalk && s == 0) {
                 fetch_head(min(h + 1, h_last), tid);
                 __builtin_amdgcn_sched_barrier(0);                     // (the scheduler would sink the requests below the products)
             }
@@ -807,7 +873,25 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                 }
             }
         }
-        __syncthreads();                                               // everyone is done with this head's tile and tables
+        if constexpr (MODE == kScanWalk) __syncthreads();              // everyone is done with this head's tile and tables
+    }
+    if constexpr (MODE == kScanChain) {
+        // the first chunk's workgroup, which had nothing to chain up, leaves the state after the last
+        if (c > 0 || !p.final_states) return;
+        const int tid = threadIdx.x;
+        float run[PB][8];
+        chain(run, tid, nc);
+#pragma unroll
+        for (int i = 0; i < PB; ++i) {
+            const int piece = tid + i * kThreads, slot = piece / (N / 8), n = piece % (N / 8) * 8, pp = 4 * (slot % 16) + slot / 16;
+            const int64_t at = ((static_cast<int64_t>(b) * H + h_first) * kP + pp) * N + n;
+            const int srow = p.final_state_is_fp32 ? 0 : srow_ws[h_first / split * p.headdim + (h_first % split) * kP + pp];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (p.final_state_is_fp32) static_cast<float*>(p.final_states)[at + e] = run[i][e];
+                else static_cast<int8_t*>(p.final_states)[at + e] = ssd_quantize_state(p, srow, n + e, run[i][e]);
+            }
+        }
     }
 }
 
@@ -882,7 +966,6 @@ extern "C" int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream_) {
     else if (p->chunk_size == 128) cumsum(ssd_cumsum_kernel<128>, 128);
     else cumsum(ssd_cumsum_kernel<64>, 64);
     const int heads64 = p->nheads * (p->headdim / 64);          // the kernels see a head of 64 s channels as s heads of 64
-    const dim3 hgrid(static_cast<unsigned>(p->batch * heads64));
     int status = QA_OK;
     // more LDS than a kernel gets by default: raise the limit (idempotent)
     auto lds_ok = [&](const void* kernel, size_t lds) {
@@ -892,24 +975,25 @@ extern "C" int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream_) {
         return false;
     };
     float* sums_ws = ws.sums_bytes && p->workspace_bytes >= ws.sums + ws.sums_bytes ? reinterpret_cast<float*>(base + ws.sums) : nullptr;
-    auto launch = [&](auto state_kernel, auto chunk_state_kernel, auto pass_kernel, size_t state_lds, auto scan_kernel, size_t scan_lds, int scan_threads) {
-        if (!lds_ok(reinterpret_cast<const void*>(state_kernel), state_lds) || !lds_ok(reinterpret_cast<const void*>(scan_kernel), scan_lds)) return;
-        if (sums_ws) {
-            if (!lds_ok(reinterpret_cast<const void*>(chunk_state_kernel), state_lds)) return;
-            hipLaunchKernelGGL(chunk_state_kernel, dim3(hgrid.x * nc), dim3(4 * p->dstate), state_lds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws, srow_ws, nc);
-            hipLaunchKernelGGL(pass_kernel, dim3(hgrid.x * (p->dstate / 16)), dim3(256), 0, stream, *p, dA_ws, prev_ws, sums_ws, srow_ws, nc);
-        } else {
-            hipLaunchKernelGGL(state_kernel, hgrid, dim3(4 * p->dstate), state_lds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws, srow_ws, nc);
-        }
+    auto launch = [&](auto n_c, auto q_c) {
+        constexpr int N = decltype(n_c)::value, Q = decltype(q_c)::value, kScanThreads = 64 * scan_waves_of(Q);
+        constexpr size_t kStateLds = sizeof(StateSmem<N, Q>), kScanLds = sizeof(ScanSmem<N, Q>);
+        // as many scan workgroups as the chip holds at once (sixteen waves of up to 128 registers to a CU), each with its share of a
+        // group's heads
         const int hpg = heads64 / p->ngroups, units = static_cast<int>(bch / p->nheads) * p->ngroups;
-        // as many workgroups as the chip holds at once (sixteen waves of up to 128 registers to a CU), each with its share of a group's heads
-        const int64_t places = static_cast<int64_t>(compute_units()) * (1024 / scan_threads);
+        const int64_t places = static_cast<int64_t>(compute_units()) * (1024 / kScanThreads);
         const int heads_each = static_cast<int>(std::min<int64_t>((static_cast<int64_t>(units) * hpg + places - 1) / places, hpg));
-        hipLaunchKernelGGL(scan_kernel, dim3(static_cast<unsigned>(units * ((hpg + heads_each - 1) / heads_each))), dim3(scan_threads), scan_lds, stream, *p, dt_ws, dA_ws, prev_ws, xs_ws, nc,
-                           heads_each);
+        const bool chain = sums_ws && heads_each == 1 && nc <= kChainChunks;
+        auto scan_kernel = chain ? ssd_chunk_scan_kernel<N, Q, kScanChain> : heads_each == 1 ? ssd_chunk_scan_kernel<N, Q, kScanOne> : ssd_chunk_scan_kernel<N, Q, kScanWalk>;
+        auto state_kernel = sums_ws ? ssd_state_kernel<N, Q, false> : ssd_state_kernel<N, Q, true>;
+        if (!lds_ok(reinterpret_cast<const void*>(state_kernel), kStateLds) || !lds_ok(reinterpret_cast<const void*>(scan_kernel), kScanLds)) return;
+        hipLaunchKernelGGL(state_kernel, dim3(static_cast<unsigned>(p->batch * heads64 * (sums_ws ? nc : 1))), dim3(4 * N), kStateLds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws, srow_ws, nc);
+        if (sums_ws && !chain)
+            hipLaunchKernelGGL(ssd_pass_kernel<N>, dim3(static_cast<unsigned>(p->batch * heads64 * (N / 16))), dim3(256), 0, stream, *p, dA_ws, prev_ws, sums_ws, srow_ws, nc);
+        hipLaunchKernelGGL(scan_kernel, dim3(static_cast<unsigned>(units * ((hpg + heads_each - 1) / heads_each))), dim3(kScanThreads), kScanLds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws,
+                           srow_ws, nc, heads_each);
     };
-#define QA_SSD_LAUNCH(N_, Q_) launch(ssd_state_kernel<N_, Q_, true>, ssd_state_kernel<N_, Q_, false>, ssd_pass_kernel<N_>, sizeof(StateSmem<N_, Q_>), ssd_chunk_scan_kernel<N_, Q_>, \
-                                     sizeof(ScanSmem<N_, Q_>), 64 * scan_waves_of(Q_))
+#define QA_SSD_LAUNCH(N_, Q_) launch(std::integral_constant<int, N_>{}, std::integral_constant<int, Q_>{})
     if (p->dstate == 128) {
         if (p->chunk_size == 256) QA_SSD_LAUNCH(128, 256);
         else if (p->chunk_size == 128) QA_SSD_LAUNCH(128, 128);

@@ -21,7 +21,7 @@ struct SsdWorkspace {            // sections of the workspace (byte offsets), se
 
 // Whether the chunks' states are summed by a workgroup each and chained by a pass of its own (matrix-core shapes): with few
 // heads in flight.  Walking, a workgroup takes about 5 us per chunk of 256 steps (a lone one; 6.4 in two rounds); apart, each
-// chunk and head costs 24 ns of the whole chip and the second launch 6 us: 6 chunks of 80 heads 30 against 19 us, 16 chunks
+// chunk and head costs 24 ns of the whole chip and the second launch (or the scan's share of it, see kChainChunks) up to 6 us: 6 chunks of 80 heads 30 against 19 us, 16 chunks
 // of 320 heads 102 against 129.
 inline bool ssd_chunks_apart(const QaSsdParams& p) {
     const double nc = static_cast<double>((p.seqlen + p.chunk_size - 1) / p.chunk_size), q = p.chunk_size / 256.0;

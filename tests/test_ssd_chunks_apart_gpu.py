@@ -33,6 +33,13 @@ def test_one_entry_at_a_time(dev, B, L, N, G, Q, final_dtype):
     assert float(y.float().abs().max()) > 0.1
 
 
+# the most chunks whose sums the scan chains up itself (8), and one more (the pass between the two); last chunks of 128 and 1 steps
+@pytest.mark.parametrize("B,L,N,G,Q", [(5, 1024, 128, 1, 128), (5, 1025, 128, 2, 128), (5, 1025, 64, 1, 128)])
+@pytest.mark.parametrize("final_dtype", [torch.float32, torch.int8])
+def test_one_entry_at_a_time_eight_and_nine_chunks(dev, B, L, N, G, Q, final_dtype):
+    test_one_entry_at_a_time(dev, B, L, N, G, Q, final_dtype)
+
+
 # with more heads in flight than the chip holds workgroups, a workgroup walks some heads of a (batch, chunk, group), the last one
 # of a group fewer: every chunk length, heads of 64 and of 128 channels, with and without gate and skip weights per channel
 @pytest.mark.parametrize("B,L,H,P,N,G,Q,per_channel", [(4, 1100, 27, 64, 128, 1, 256, False), (9, 300, 48, 64, 64, 3, 128, True),
