@@ -47,6 +47,34 @@ __device__ __forceinline__ int8_t byte_of(uint32_t w, int j) { return static_cas
 // ---------------------------------------------------------------------------------------------
 constexpr int kCumHeads = 4;
 
+// the step size of an int8 code with its bias
+__device__ __forceinline__ float step_size(const QaSsdParams& p, float s_dt, int8_t code, float bias) {
+    float v = s_dt * static_cast<float>(code) + bias;
+    if (p.dt_softplus) v = v <= 20.0f ? log1pf(expf(v)) : v;
+    return fminf(fmaxf(v, p.dt_min), p.dt_max);
+}
+__device__ __forceinline__ float decay_rate(const QaSsdParams& p, int h) { return -expf(*p.A_log_scale * static_cast<float>(p.A_log[h])); }
+// In a whole wave, a lane with E consecutive step sizes of a chunk: the inclusive sums of dt A from the chunk's start.
+template <int E>
+__device__ __forceinline__ void chunk_cumsum(const float (&dtv)[E], float A, int lane, float (&cs)[E]) {
+    float local = 0.0f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        local += dtv[e] * A;
+        cs[e] = local;
+    }
+    // exclusive prefix of the lane totals
+    float incl = local;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const float up = __shfl_up(incl, off);
+        if (lane >= off) incl += up;
+    }
+    const float before = incl - local;
+#pragma unroll
+    for (int e = 0; e < E; ++e) cs[e] = before + cs[e];
+}
+
 template <int Q>
 __global__ __launch_bounds__(Q) void ssd_cumsum_kernel(QaSsdParams p, float* dt_out, float* dA_out, float* xs_out, int32_t* srow_out, int nc) {
     constexpr int E = Q / 64;                          // steps per lane, and waves
@@ -84,47 +112,28 @@ __global__ __launch_bounds__(Q) void ssd_cumsum_kernel(QaSsdParams p, float* dt_
             }
             const float s_dt = *p.dt_scale;
 #pragma unroll
-            for (int j = 0; j < kCumHeads; ++j) {
-                v[j] = s_dt * static_cast<float>(byte_of(w, j)) + bias[j];
-                if (p.dt_softplus) v[j] = v[j] <= 20.0f ? log1pf(expf(v[j])) : v[j];
-                v[j] = fminf(fmaxf(v[j], p.dt_min), p.dt_max);
-            }
+            for (int j = 0; j < kCumHeads; ++j) v[j] = step_size(p, s_dt, byte_of(w, j), bias[j]);
         }
 #pragma unroll
         for (int j = 0; j < kCumHeads; ++j) dt_s[j][threadIdx.x] = t < p.seqlen ? v[j] : 0.0f;
     }
     float A[(kCumHeads + E - 1) / E];
 #pragma unroll
-    for (int j = wave, i = 0; i < static_cast<int>(sizeof(A) / 4); j += E, ++i) {
-        const int h = min(h0 + j, p.nheads - 1);
-        A[i] = -expf(*p.A_log_scale * static_cast<float>(p.A_log[h]));
-    }
+    for (int j = wave, i = 0; i < static_cast<int>(sizeof(A) / 4); j += E, ++i) A[i] = decay_rate(p, min(h0 + j, p.nheads - 1));
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < static_cast<int>(sizeof(A) / 4); ++i) {
         const int j = wave + i * E, h = h0 + j;
         if (h >= p.nheads) return;
         float dtv[E], run[E];
-        float local = 0.0f;
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            dtv[e] = dt_s[j][lane * E + e];
-            local += dtv[e] * A[i];
-            run[e] = local;
-        }
-        // exclusive prefix of the lane totals
-        float incl = local;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const float up = __shfl_up(incl, off);
-            if (lane >= off) incl += up;
-        }
-        const float before = incl - local;
+        for (int e = 0; e < E; ++e) dtv[e] = dt_s[j][lane * E + e];
+        chunk_cumsum<E>(dtv, A[i], lane, run);
         const int64_t row = ((static_cast<int64_t>(b) * p.nheads + h) * nc + c) * Q + lane * E;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             dt_out[row + e] = dtv[e];
-            dA_out[row + e] = before + run[e];
+            dA_out[row + e] = run[e];
         }
     }
 }
@@ -159,6 +168,13 @@ __device__ __forceinline__ float sbyte_of(uint32_t w, int j) {
     }
     return r;
 }
+// fp16 of a value that is an fp32 number already.  The empty asm separates the conversion from the multiplication that made the
+// value: where the compiler merges the two into a mixed-precision instruction the exact product is rounded once, which is another
+// number at some ties, and which of the kernels' values it does so with changes with the code around them.
+__device__ __forceinline__ _Float16 rounded(float v) {
+    asm("" : "+v"(v));
+    return static_cast<_Float16>(v);
+}
 constexpr uint32_t kBias = 0x80808080u;
 __device__ __forceinline__ uint32_t word_of(const uint4& v, int d) { return d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w; }
 __device__ __forceinline__ float lane_of(const float4& v, int d) { return d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w; }
@@ -189,10 +205,10 @@ __device__ __forceinline__ void stage_x_share(_Float16 (*xt)[XP], const XShare<C
         for (int cc = 0; cc < 4; ++cc) {
             const float sc = lane_of(s4, cc), nsc = -128.0f * sc;
             v4h v;
-            v[0] = static_cast<_Float16>(__builtin_fmaf(ubyte_of(w0, cc), sc, nsc));
-            v[1] = static_cast<_Float16>(__builtin_fmaf(ubyte_of(w1, cc), sc, nsc));
-            v[2] = static_cast<_Float16>(__builtin_fmaf(ubyte_of(w2, cc), sc, nsc));
-            v[3] = static_cast<_Float16>(__builtin_fmaf(ubyte_of(w3, cc), sc, nsc));
+            v[0] = rounded(__builtin_fmaf(ubyte_of(w0, cc), sc, nsc));
+            v[1] = rounded(__builtin_fmaf(ubyte_of(w1, cc), sc, nsc));
+            v[2] = rounded(__builtin_fmaf(ubyte_of(w2, cc), sc, nsc));
+            v[3] = rounded(__builtin_fmaf(ubyte_of(w3, cc), sc, nsc));
             *reinterpret_cast<v4h*>(&xt[cc * 16 + c0 / 4 + d][kb * 4]) = v;              // row slot(c0 + 4 d + cc)
         }
     }
@@ -240,8 +256,8 @@ struct StateSmem {
 };
 
 template <int N, int Q, bool WALK>
-__global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSsdParams p, const float* dt_ws, const float* dA_ws, __half* prev, float* sums,
-                                                                              const float* xs_ws, const int32_t* srow_ws, int nc) {
+__global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSsdParams p, float* dt_ws, float* dA_ws, __half* prev, float* sums, float* xs_ws,
+                                                                              int32_t* srow_ws, int nc, int own_steps) {
     using S = StateSmem<N, Q>;
     extern __shared__ __attribute__((aligned(16))) unsigned char ssd_smem_raw[];
     S& sm = *reinterpret_cast<S*>(ssd_smem_raw);
@@ -271,7 +287,8 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
     const int xc = tid % (kP / CH) * CH, xkb = tid / (kP / CH), bc = tid % (N / 16) * 16, bkb = tid / (N / 16);
     const bool mine_x = kSharesX == kThreads || tid < kSharesX, mine_b = kSharesB == kThreads || tid < kSharesB;
     const uint32_t voff_x = static_cast<uint32_t>(4 * xkb) * xrow + xc, voff_b = static_cast<uint32_t>(4 * bkb) * brow + bc;
-    if (tid < kP) {
+    const bool steps_made = WALK || !own_steps;                   // step sizes, their sums and the tables: by ssd_cumsum_kernel
+    if (steps_made && tid < kP) {
         sm.xs[tid] = xs_ws[hp * p.headdim + ch0 + tid];
         sm.srow[tid] = srow_ws[hp * p.headdim + ch0 + tid];
     }
@@ -298,11 +315,13 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
 #pragma unroll
             for (int r = 0; r < 4; ++r) br[r] = *reinterpret_cast<const uint4*>(bsrc + static_cast<uint64_t>(min(voff_b + static_cast<uint32_t>(r) * brow, last_b)));
         }
-        const float* dA_row = dA_ws + (rows0 + c) * Q;
-        r_last = dA_row[Q - 1];
-        if (Q == kThreads || tid < Q) {
-            r_dt = dt_ws[(rows0 + c) * Q + tid];
-            r_dA = dA_row[tid];
+        if (steps_made) {
+            const float* dA_row = dA_ws + (rows0 + c) * Q;
+            r_last = dA_row[Q - 1];
+            if (Q == kThreads || tid < Q) {
+                r_dt = dt_ws[(rows0 + c) * Q + tid];
+                r_dA = dA_row[tid];
+            }
         }
     };
     auto stage_chunk = [&]() {
@@ -331,7 +350,7 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
                 *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 3][bkb * 4]) = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
             }
         }
-        if (tid < Q) sm.w[tid] = fexp(r_last - r_dA) * r_dt;        // weight of step k in the chunk's state
+        if (steps_made && tid < Q) sm.w[tid] = fexp(r_last - r_dA) * r_dt;   // weight of step k in the chunk's state
     };
 
     // the running state: columns n = 16 wave + lane % 16; tile j, register r: channel p = 4 (4 (lane / 16) + r) + j
@@ -340,8 +359,72 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
 #pragma unroll
     for (int j = 0; j < 4; ++j) run[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
+    // the final state in the requested form
+    auto store_final = [&](const v4f (&state)[4]) {
+        if (p.final_states) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int pp = 4 * (4 * lq + r) + j;
+                    const int64_t fo = ((static_cast<int64_t>(b) * H + h) * kP + pp) * N + n_col;
+                    const float sv = state[j][r];
+                    if (p.final_state_is_fp32) {
+                        static_cast<float*>(p.final_states)[fo] = sv;
+                    } else {
+                        static_cast<int8_t*>(p.final_states)[fo] = ssd_quantize_state(p, sm.srow[pp], n_col, sv);
+                    }
+                }
+        }
+    };
+
     load_chunk(my_chunk);
-    __syncthreads();                                              // the table of x scales
+    if (!steps_made) {
+        // The chunk's step sizes, their sums and the channels' scales, which this workgroup needs before anyone else does, while its
+        // tiles are on their way
+        constexpr int E = Q / 64;
+        __builtin_amdgcn_sched_barrier(0);
+        if (wave == kThreads / 64 - 1) {
+            const SsdChannel e = ssd_channel(p, hp, lane, ch0);
+            sm.xs[lane] = e.xs;
+            sm.srow[lane] = e.srow;
+            if (b == 0 && my_chunk == 0) {
+                xs_ws[hp * p.headdim + ch0 + lane] = e.xs;
+                srow_ws[hp * p.headdim + ch0 + lane] = e.srow;
+            }
+        }
+        if (tid < Q) {
+            const int t = my_chunk * Q + tid;
+            const int64_t at = (static_cast<int64_t>(b) * L + min(t, L - 1)) * ssd_dt_stride(p) + hp;
+            float v;
+            if (p.dt_is_fp32) {
+                v = static_cast<const float*>(p.dt)[at];
+            } else {
+                const float bias = p.dt_bias ? __half2float(static_cast<const __half*>(p.dt_bias)[hp]) : 0.0f;
+                v = step_size(p, *p.dt_scale, static_cast<const int8_t*>(p.dt)[at], bias);
+            }
+            sm.w[tid] = t < L ? v : 0.0f;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            float dtv[E], cs[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) dtv[e] = sm.w[lane * E + e];
+            chunk_cumsum<E>(dtv, decay_rate(p, hp), lane, cs);
+            const float last = __shfl(cs[E - 1], 63);
+            const int64_t row = (rows0 + my_chunk) * Q + lane * E;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                sm.w[lane * E + e] = fexp(last - cs[e]) * dtv[e];
+                if (h % split == 0) {
+                    dt_ws[row + e] = dtv[e];
+                    dA_ws[row + e] = cs[e];
+                }
+            }
+        }
+    } else {
+        __syncthreads();                                          // the table of x scales
+    }
     stage_chunk();
     float dA_last = r_last;                                       // of the chunk about to be multiplied
     __syncthreads();
@@ -369,11 +452,15 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
             const float wk[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
             v8h bw;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) bw[e] = static_cast<_Float16>((sB * sbyte_of(e < 4 ? b0 : b1, e & 3)) * wk[e]);
+            for (int e = 0; e < 8; ++e) bw[e] = rounded((sB * sbyte_of(e < 4 ? b0 : b1, e & 3)) * wk[e]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) accs[j] = mfma16(fx[j], bw, accs[j]);
         }
         if constexpr (!WALK) {
+            if (nc == 1) {                                         // the only chunk's sums are the final state
+                store_final(accs);
+                return;
+            }
             float* to = sums + (((static_cast<int64_t>(b) * nc + my_chunk) * H + h) * kP) * N + n_col;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
@@ -403,27 +490,12 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
         __syncthreads();
     }
 
-    // final state in the requested form
-    if (p.final_states) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int pp = 4 * (4 * lq + r) + j;
-                const int64_t fo = ((static_cast<int64_t>(b) * H + h) * kP + pp) * N + n_col;
-                const float sv = run[j][r];
-                if (p.final_state_is_fp32) {
-                    static_cast<float*>(p.final_states)[fo] = sv;
-                } else {
-                    static_cast<int8_t*>(p.final_states)[fo] = ssd_quantize_state(p, sm.srow[pp], n_col, sv);
-                }
-            }
-    }
+    store_final(run);
 }
 
 // The same with few heads in flight: a workgroup per chunk (WALK false) leaves the chunk's own sums S_c in memory as fp32, rows
 // in slot order, and this kernel runs the recurrence over them, four states a thread: the same values in the same order.
-// (Up to kChainChunks chunks the chunk scan does it itself.)
+// (Up to kChainChunks chunks the chunk scan does it itself; of one chunk the sums are the final state.)
 template <int N>
 __global__ __launch_bounds__(256) void ssd_pass_kernel(QaSsdParams p, const float* dA_ws, __half* prev, const float* sums, const int32_t* srow_ws, int nc) {
     constexpr int kPieces = kP * N / 4;                           // of one head of 64 channels
@@ -745,8 +817,8 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                     v8h cf;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        cf[e] = static_cast<_Float16>(sC * sbyte_of(w0, e));
-                        cf[4 + e] = static_cast<_Float16>(sC * sbyte_of(w1, e));
+                        cf[e] = rounded(sC * sbyte_of(w0, e));
+                        cf[4 + e] = rounded(sC * sbyte_of(w1, e));
                     }
                     const int n0 = 64 * (ks / 2) + 16 * lq + 8 * (ks % 2);     // the states of those eight codes
                     v8h fs[4];
@@ -812,7 +884,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
             auto times_x = [&](int ks, const float (&wv)[8]) {
                 v8h fl;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) fl[e] = static_cast<_Float16>(wv[e]);
+                for (int e = 0; e < 8; ++e) fl[e] = rounded(wv[e]);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const v4h x0 = *reinterpret_cast<const v4h*>(&sm.xt[j * 16 + l16][32 * ks + 4 * lq]);
@@ -958,13 +1030,6 @@ extern "C" int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream_) {
         ssd_general_launch(*p, dt_ws, dA_ws, prev_ws, xs_ws, srow_ws, nc, stream);
         return check_launch();
     }
-    auto cumsum = [&](auto kernel, int Q) {
-        const int64_t tables = (p->nheads + Q / 64 - 1) / (Q / 64), heads = (p->nheads + kCumHeads - 1) / kCumHeads;
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tables + heads * p->batch * nc)), dim3(Q), 0, stream, *p, dt_ws, dA_ws, xs_ws, srow_ws, nc);
-    };
-    if (p->chunk_size == 256) cumsum(ssd_cumsum_kernel<256>, 256);
-    else if (p->chunk_size == 128) cumsum(ssd_cumsum_kernel<128>, 128);
-    else cumsum(ssd_cumsum_kernel<64>, 64);
     const int heads64 = p->nheads * (p->headdim / 64);          // the kernels see a head of 64 s channels as s heads of 64
     int status = QA_OK;
     // more LDS than a kernel gets by default: raise the limit (idempotent)
@@ -985,9 +1050,20 @@ extern "C" int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream_) {
         const int heads_each = static_cast<int>(std::min<int64_t>((static_cast<int64_t>(units) * hpg + places - 1) / places, hpg));
         const bool chain = sums_ws && heads_each == 1 && nc <= kChainChunks;
         auto scan_kernel = chain ? ssd_chunk_scan_kernel<N, Q, kScanChain> : heads_each == 1 ? ssd_chunk_scan_kernel<N, Q, kScanOne> : ssd_chunk_scan_kernel<N, Q, kScanWalk>;
-        auto state_kernel = sums_ws ? ssd_state_kernel<N, Q, false> : ssd_state_kernel<N, Q, true>;
+        // With a workgroup per chunk and head these make the step sizes, too, in place of a launch in front: once per head instead of once
+        // per four heads' line of bytes, which is cheaper up to some workgroups a CU (us of the two launches against the one:
+        // 2 chunks of 24 heads 11.3 -> 7.4, 6 of 80 17.4 -> 13.7, 8 of 80 19.5 -> 17.4; 16 of 128 38.6 -> 41.7)
+        const int64_t chunk_heads = static_cast<int64_t>(p->batch) * heads64 * nc;
+        const int own_steps = (sums_ws || nc == 1) && chunk_heads <= 4LL * compute_units();
+        const bool apart = sums_ws || (nc == 1 && own_steps);
+        auto state_kernel = apart ? ssd_state_kernel<N, Q, false> : ssd_state_kernel<N, Q, true>;
         if (!lds_ok(reinterpret_cast<const void*>(state_kernel), kStateLds) || !lds_ok(reinterpret_cast<const void*>(scan_kernel), kScanLds)) return;
-        hipLaunchKernelGGL(state_kernel, dim3(static_cast<unsigned>(p->batch * heads64 * (sums_ws ? nc : 1))), dim3(4 * N), kStateLds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws, srow_ws, nc);
+        if (!own_steps) {
+            const int64_t tables = (p->nheads + Q / 64 - 1) / (Q / 64), heads = (p->nheads + kCumHeads - 1) / kCumHeads;
+            hipLaunchKernelGGL(ssd_cumsum_kernel<Q>, dim3(static_cast<unsigned>(tables + heads * p->batch * nc)), dim3(Q), 0, stream, *p, dt_ws, dA_ws, xs_ws, srow_ws, nc);
+        }
+        hipLaunchKernelGGL(state_kernel, dim3(static_cast<unsigned>(apart ? chunk_heads : p->batch * heads64)), dim3(4 * N), kStateLds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws, srow_ws, nc,
+                           own_steps);
         if (sums_ws && !chain)
             hipLaunchKernelGGL(ssd_pass_kernel<N>, dim3(static_cast<unsigned>(p->batch * heads64 * (N / 16))), dim3(256), 0, stream, *p, dA_ws, prev_ws, sums_ws, srow_ws, nc);
         hipLaunchKernelGGL(scan_kernel, dim3(static_cast<unsigned>(units * ((hpg + heads_each - 1) / heads_each))), dim3(kScanThreads), kScanLds, stream, *p, dt_ws, dA_ws, prev_ws, sums_ws, xs_ws,

@@ -19,15 +19,18 @@ struct SsdWorkspace {            // sections of the workspace (byte offsets), se
     int64_t sums, sums_bytes;    // behind `total`, used when the caller's workspace holds it (see ssd_chunks_apart)
 };
 
-// Whether the chunks' states are summed by a workgroup each and chained by a pass of its own (matrix-core shapes): with few
-// heads in flight.  Walking, a workgroup takes about 5 us per chunk of 256 steps (a lone one; 6.4 in two rounds); apart, each
-// chunk and head costs 24 ns of the whole chip and the second launch (or the scan's share of it, see kChainChunks) up to 6 us: 6 chunks of 80 heads 30 against 19 us, 16 chunks
-// of 320 heads 102 against 129.
+// Whether the chunks' states are summed by a workgroup each and chained up afterwards (matrix-core shapes): with few heads in
+// flight.  Walking, a workgroup takes about 5 us per chunk of 256 steps (a lone one; 6.4 in two rounds); apart, each chunk and
+// head costs 24 ns of the whole chip and the launch that passes the states on 6 us: 16 chunks of 320 heads 102 against 129.
+// With few chunks and heads the scan passes the states on and the chunks' workgroups make the step sizes (see kChainChunks and
+// own_steps): no launch more and one less, 3 chunks of 128 heads 39.9 us for the whole
+// scan walking, 30.8 apart.
 inline bool ssd_chunks_apart(const QaSsdParams& p) {
     const double nc = static_cast<double>((p.seqlen + p.chunk_size - 1) / p.chunk_size), q = p.chunk_size / 256.0;
     const double heads = static_cast<double>(p.batch) * p.nheads * (p.headdim / 64);
     const double rounds = heads <= 256 ? 5.0 : heads <= 512 ? 6.4 : heads / 80.0;
-    return nc >= 2 && nc * heads * (0.008 * q + 0.016) * (p.dstate / 128.0) + 6.0 < nc * rounds * q;
+    const double more = nc <= 8 && nc * heads <= 512 ? 1.5 : 6.0;
+    return nc >= 2 && nc * heads * (0.008 * q + 0.016) * (p.dstate / 128.0) + more < nc * rounds * q;
 }
 
 __host__ __device__ inline int64_t ssd_align256(int64_t v) { return (v + 255) & ~int64_t(255); }
@@ -70,19 +73,16 @@ __device__ __forceinline__ int ssd_dim_group_of(const QaSsdParams& p, int g, int
     return min(dg, p.ndim_groups - 1);
 }
 
-// The per-channel tables of head h, written by one whole wave of the first kernel (h is the same in all its lanes).
+// The entries of the per-channel tables for channels ch0 + lane of head h, in one whole wave (h is the same in all its lanes).
 // srow: index of the first state's scale in state_scale for this channel (0 with one scale for everything).
 // The bounds of the groups come from memory once, a bound per lane, and are compared out of registers: a walk that loads
 // one bound after another waits for memory at every step, which was longer than the rest of that kernel.
-__device__ __forceinline__ void ssd_write_channel_tables(const QaSsdParams& p, int h, int lane, float* xs_out, int32_t* srow_out) {
-    if (p.nhead_groups == 0) {
-        const float xs = p.x_scale[0];
-        for (int ch = lane; ch < p.headdim; ch += 64) {
-            xs_out[h * p.headdim + ch] = xs;
-            srow_out[h * p.headdim + ch] = 0;
-        }
-        return;
-    }
+struct SsdChannel {
+    float xs;
+    int32_t srow;
+};
+__device__ __forceinline__ SsdChannel ssd_channel(const QaSsdParams& p, int h, int lane, int ch0) {
+    if (p.nhead_groups == 0) return {p.x_scale[0], 0};
     int g, hg;
     const int hpg = p.nheads / p.ngroups;
     if (p.nhead_groups <= 64) {
@@ -92,20 +92,24 @@ __device__ __forceinline__ void ssd_write_channel_tables(const QaSsdParams& p, i
     } else {
         ssd_group_of(p, h, g, hg);
     }
-    const int group = (g * p.nhead_groups + hg) * p.ndim_groups;
+    const int group = (g * p.nhead_groups + hg) * p.ndim_groups, ch = min(ch0 + lane, p.headdim - 1);
     const int bound = lane < p.ndim_groups ? p.x_dim_group_range[group + lane] : 0;
+    int dg = 0;
+    if (p.ndim_groups <= 64) {
+        for (int j = 0; j < p.ndim_groups; ++j) dg += ch >= __builtin_amdgcn_readlane(bound, j) ? 1 : 0;
+        dg = min(dg, p.ndim_groups - 1);
+    } else {
+        dg = ssd_dim_group_of(p, g, hg, ch);
+    }
+    return {p.x_scale[group + dg], (group + dg) * p.dstate};
+}
+// The tables of head h, written by one whole wave of the first kernel.
+__device__ __forceinline__ void ssd_write_channel_tables(const QaSsdParams& p, int h, int lane, float* xs_out, int32_t* srow_out) {
     for (int ch0 = 0; ch0 < p.headdim; ch0 += 64) {
-        const int ch = ch0 + lane;
-        int dg = 0;
-        if (p.ndim_groups <= 64) {
-            for (int j = 0; j < p.ndim_groups; ++j) dg += ch >= __builtin_amdgcn_readlane(bound, j) ? 1 : 0;
-            dg = min(dg, p.ndim_groups - 1);
-        } else if (ch < p.headdim) {
-            dg = ssd_dim_group_of(p, g, hg, ch);
-        }
-        if (ch < p.headdim) {
-            xs_out[h * p.headdim + ch] = p.x_scale[group + dg];
-            srow_out[h * p.headdim + ch] = (group + dg) * p.dstate;
+        const SsdChannel e = ssd_channel(p, h, lane, ch0);
+        if (ch0 + lane < p.headdim) {
+            xs_out[h * p.headdim + ch0 + lane] = e.xs;
+            srow_out[h * p.headdim + ch0 + lane] = e.srow;
         }
     }
 }

@@ -40,6 +40,13 @@ def test_one_entry_at_a_time_eight_and_nine_chunks(dev, B, L, N, G, Q, final_dty
     test_one_entry_at_a_time(dev, B, L, N, G, Q, final_dtype)
 
 
+# the step sizes by the chunks' own workgroups (an entry alone) and in a launch of their own (all together): 20 chunks, and one
+@pytest.mark.parametrize("B,L,N,G,Q", [(2, 20 * 256 - 3, 128, 1, 256), (23, 256, 128, 1, 256), (23, 17, 64, 2, 64)])
+@pytest.mark.parametrize("final_dtype", [torch.float32, torch.int8])
+def test_one_entry_at_a_time_step_sizes(dev, B, L, N, G, Q, final_dtype):
+    test_one_entry_at_a_time(dev, B, L, N, G, Q, final_dtype)
+
+
 # with more heads in flight than the chip holds workgroups, a workgroup walks some heads of a (batch, chunk, group), the last one
 # of a group fewer: every chunk length, heads of 64 and of 128 channels, with and without gate and skip weights per channel
 @pytest.mark.parametrize("B,L,H,P,N,G,Q,per_channel", [(4, 1100, 27, 64, 128, 1, 256, False), (9, 300, 48, 64, 64, 3, 128, True),
