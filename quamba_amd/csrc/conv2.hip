@@ -226,17 +226,17 @@ int validate(const QaConv2Params* p, bool update) {
 
 namespace qa {
 int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
-    // Steps per wave: 8 to 256, whichever needs the fewest rounds of resident waves (seven per SIMD) times its own length
-    // plus a wave's set-up (taps, scales: about 24 steps' worth).  Batch 16 x 1024 steps x 10240 channels is 10240 waves
-    // of 64 steps on 7168 places - a second round at a third of the occupancy - or 5120 of 128.  A short prompt
-    // (1 x 512 x 1536 channels: 48 waves of 64 steps, one after the other 19 us) takes short runs.
-    int run = kBatchLoads;
+    // Steps per wave: 4 to 256, whichever takes the busiest SIMD's waves the shortest: in ns about 145 a step and 350 for a
+    // wave's set-up (taps, scales, the three inputs ahead), and 100 a step of the last wave with nobody beside it.  Measured
+    // with runs of 4, 8, 16, 32, 64 steps, us: 1 x 512 x 1536 channels 5.5, 6.7, 8.2, 11.1, 17.4; 1 x 777 x 3072 5.9, 6.5, 8.1, 11.4, 18.2;
+    // 1 x 1531 x 5376 14.6, 12.6, 13.1, 14.4, 20.7; 4 x 4096 x 5376 87.7, 64.4, 57.0, 56.5, 60.8; 16 x 1024 x 10240 164, 118, 99, 95, 95.
+    int run = 4;
     {
-        const int64_t ch_blocks = (p.dim + 255) / 256, places = 7 * 4 * 256;
+        const int64_t ch_blocks = (p.dim + 255) / 256, simds = 4LL * compute_units();
         int64_t best = -1;
-        for (int r = kBatchLoads; r <= 256; r *= 2) {
+        for (int r = 4; r <= 256; r *= 2) {
             const int64_t waves = ch_blocks * (((p.seqlen + r - 1) / r + 3) / 4 * 4) * p.batch;
-            const int64_t cost = ((waves + places - 1) / places) * (r + 24);
+            const int64_t cost = (waves + simds - 1) / simds * (145 * r + 350) + 100 * r;
             if (best < 0 || cost < best) { best = cost; run = r; }
         }
     }
