@@ -290,7 +290,9 @@ int pick(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
 // order of the stand-alone kernel and so to the same bits, with its share of the weights on the way.  Eight waves a workgroup
 // and at most about one workgroup per CU, so that no CU transforms the row twice; KS waves share four weight rows.  A decode
 // step of one sequence (one launch less to make and to wait for): d_inner 1536 21.0 -> 18.0 us, 3072 20.5 -> 17.3, 4096 21.9
-// -> 19.7, 5120 25.7 -> 23.6; 8192 33.5 -> 34.0, so up to 5120 only.  (With the gated norm in front as well it was slower
+// -> 19.7, 5120 25.7 -> 23.6; 8192 33.5 -> 34.0, so up to 5120 only.  The transform is most of the kernel: with the first three
+// index bits in the registers the row arrives in and the outputs of a lane chosen for their common beginnings (s_point_quantised) the
+// launch takes 2560 x 5120 with 4 bits 9.6 -> 8.9 us, int8 8.2 -> 7.3, 768 x 1536 4.8 -> 4.4.  (With the gated norm in front as well it was slower
 // than the two kernels at every width.)
 // ---------------------------------------------------------------------------------------------
 constexpr int kRotThreads = 512, kRotWaves = kRotThreads / 64, kRotDim = 5120;
@@ -345,13 +347,27 @@ __global__ __launch_bounds__(kRotThreads) void gemv_rotated_kernel(GemvArgs p, G
     for (int i = 0; i < kRowPieces; ++i) {
         const int e0 = (tid + i * kRotThreads) * 8;
         if (e0 < dim) {
+            // index bits 0-2 in the registers the row arrives in
             const __half* h = reinterpret_cast<const __half*>(&yr[i]);
+            float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) buf[phys(e0 + j)] = __half2float(h[j]);
+            for (int j = 0; j < 8; ++j) v[j] = __half2float(h[j]);
+#pragma unroll
+            for (int s = 1; s < 8; s <<= 1) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    if (j & s) continue;
+                    const float a = v[j], c = v[j | s];
+                    v[j] = a + c;
+                    v[j | s] = a - c;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) buf[phys(e0 + j)] = v[j];
         }
     }
     __syncthreads();
-    fwht_passes<kRotThreads, __half>(buf, nullptr, dim, shape.log_m, true, tid);
+    fwht_passes<kRotThreads, __half>(buf, nullptr, dim, shape.log_m, true, tid, 3);
     if constexpr (S > 1) {
         s_point_quantised<S, kRotThreads, 4>(buf, codes, shape.log_m, r.had_scale, tid);
     } else {

@@ -59,6 +59,26 @@ constexpr std::array<uint64_t, 40> make_h40() {
 constexpr auto kH12 = make_h12();
 constexpr auto kH40 = make_h40();
 
+// The rows in the order of their sign patterns, the first sign taken out: neighbours in it begin with the same signed sum, up to
+// the sign of the whole, and a lane that makes a few neighbours adds up their common beginning once.
+template <size_t S>
+constexpr std::array<int, S> rows_by_pattern(const std::array<uint64_t, S>& rows) {
+    auto pattern = [&](int i) {                                    // the first column in the highest bit
+        uint64_t v = 0;
+        for (size_t k = 0; k < S; ++k) v = v << 1 | (((rows[i] >> k) ^ rows[i]) & 1);
+        return v;
+    };
+    std::array<int, S> order{};
+    for (size_t i = 0; i < S; ++i) {
+        size_t at = i;
+        for (; at > 0 && pattern(order[at - 1]) > pattern(static_cast<int>(i)); --at) order[at] = order[at - 1];
+        order[at] = static_cast<int>(i);
+    }
+    return order;
+}
+constexpr auto kOrder12 = rows_by_pattern(kH12);
+constexpr auto kOrder40 = rows_by_pattern(kH40);
+
 template <int S>
 __device__ __forceinline__ bool minus_at(int i, int j) {
     if constexpr (S == 12) return (kH12[i] >> j) & 1;
@@ -127,13 +147,13 @@ __device__ __forceinline__ void fwht_pass(float* buf, const T* x, int dim, int b
     }
 }
 
-// All index bits of the row (2^log_m per column block), in passes of at most five bits, sizes as even as possible
-// (7 -> 4+3, 13 -> 5+4+4).  Ends with a barrier.
+// The index bits of the row (2^log_m per column block) from `first` on, in passes of at most five bits, sizes as even as
+// possible (7 -> 4+3, 13 -> 5+4+4).  Ends with a barrier.
 template <int NT, typename T>
-__device__ __forceinline__ void fwht_passes(float* buf, const T* x, int dim, int log_m, bool vec, int tid) {
-    const int n_pass = (log_m + 4) / 5;
-    for (int pass = 0, bit0 = 0; pass < n_pass; ++pass) {
-        const int b = log_m / n_pass + (pass < log_m % n_pass ? 1 : 0);
+__device__ __forceinline__ void fwht_passes(float* buf, const T* x, int dim, int log_m, bool vec, int tid, int first = 0) {
+    const int bits = log_m - first, n_pass = (bits + 4) / 5;
+    for (int pass = 0, bit0 = first; pass < n_pass; ++pass) {
+        const int b = bits / n_pass + (pass < bits % n_pass ? 1 : 0);
         switch (b) {
             case 1: fwht_pass<1, NT, T>(buf, x, dim, bit0, vec, tid); break;
             case 2: fwht_pass<2, NT, T>(buf, x, dim, bit0, vec, tid); break;
@@ -146,7 +166,8 @@ __device__ __forceinline__ void fwht_passes(float* buf, const T* x, int dim, int
     }
 }
 
-// The S point transform of every column of the row in buf, quantised: PARTS lanes share the S outputs of a column.
+// The S point transform of every column of the row in buf, quantised: PARTS lanes share the S outputs of a column, neighbours
+// by pattern each (in four parts 283 additions a lane for S = 40, with neighbouring rows 373).
 template <int S, int NT, int PARTS>
 __device__ __forceinline__ void s_point_quantised(const float* buf, int8_t* out, int log_m, float scale, int tid) {
     constexpr int kPer = (S + PARTS - 1) / PARTS;
@@ -160,7 +181,8 @@ __device__ __forceinline__ void s_point_quantised(const float* buf, int8_t* out,
             constexpr int kPart = decltype(part_c)::value;
             if (part == kPart) {
 #pragma unroll
-                for (int i = kPart * kPer; i < (kPart + 1) * kPer && i < S; ++i) {
+                for (int o = kPart * kPer; o < (kPart + 1) * kPer && o < S; ++o) {
+                    const int i = S == 12 ? kOrder12[o % 12] : kOrder40[o];
                     float acc = minus_at<S>(i, 0) ? -v[0] : v[0];
 #pragma unroll
                     for (int j = 1; j < S; ++j) acc = minus_at<S>(i, j) ? acc - v[j] : acc + v[j];
