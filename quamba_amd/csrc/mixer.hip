@@ -453,7 +453,7 @@ int mamba2_tail(const QaMamba2Params& p, const Mamba2Buffers& b, void* stream) {
     if (norm_fuses(p)) {
         QaHadamardParams h = {};
         h.rows = rows; h.dim = p.d_inner; h.scale = p.had_scale; h.out_row_stride = p.d_inner; h.out = b.yq;
-        QA_TRY(qa_rmsnorm_gated_hadamard_quant(&n, &h, stream));
+        QA_TRY(norm_hadamard_quant(&n, &h, true, stream));
     } else {
         QA_TRY(qa_rmsnorm_gated(&n, stream));
         QA_TRY(hadamard(b.yn, b.yq, rows, p.d_inner, p.had_scale, stream));

@@ -5,8 +5,11 @@
 
 namespace qa {
 
-// hadamard.hip: whether qa_rmsnorm_gated_hadamard_quant takes rows of `dim` columns in norm groups of `group`
+// hadamard.hip: whether norm_hadamard_quant takes rows of `dim` columns in norm groups of `group`, and
+// qa_rmsnorm_gated_hadamard_quant itself, which as an entry point of its own leaves rows of 4096 columns in one group to the
+// two kernels (`in_layer` false)
 bool norm_hadamard_fuses(int dim, int group);
+int norm_hadamard_quant(const QaNormGatedParams* n, const QaHadamardParams* h, bool in_layer, void* stream);
 
 // sscan_tm.hip: qa_sscan_fwd for token-major inputs.  With `dt` the step size codes are not read but made in the scan:
 // dt_proj's product of x (x_proj's rows, x_l_stride apart) with w (d_inner rows of `rank` codes, a multiple of 16 up to 192),

@@ -105,6 +105,28 @@ def test_step_of_many_sequences(dev, cls, d_model, batch, width):
     _close(out[:, 0], m._step_modules(h, conv2, ssm2), (conv, conv2), (ssm, ssm2))
 
 
+@pytest.mark.parametrize("batch,seqlen", [(1, 0), (5, 0), (2, 37), (3, 900)])
+@pytest.mark.parametrize("norm_first", [False, True])
+def test_norm_of_whole_rows_of_4096(dev, batch, seqlen, norm_first):
+    """One norm group a row, in the transform's launch: one row, a few, more than the chip holds workgroups (seqlen 0: a step)."""
+    m, g = _mamba2(lambda d, *a, **k: W8A8QMamba2(2048, *a, **{**k, "ngroups": 1}), dev, seed=batch)
+    m.norm.norm_before_gate = norm_first
+    c, q = m.conv1d, m.qchunk_scan                                 # (the tables of two groups: the first one's)
+    c.x_out_scales, c.B_out_scales, c.C_out_scales = c.x_out_scales[:1], c.B_out_scales[:1], c.C_out_scales[:1]
+    c.x_head_group_range = torch.tensor([[1, m.nheads]], dtype=torch.int32, device=dev)
+    c.x_dim_group_range = c.x_dim_group_range[:1].contiguous()
+    q.x_scales, q.B_scale, q.C_scale = c.x_out_scales, c.B_out_scales, c.C_out_scales
+    q.x_head_group_range, q.x_dim_group_range = c.x_head_group_range, c.x_dim_group_range
+    q.ssm_state_scale = q.ssm_state_scale[:1].contiguous()
+    step = seqlen == 0
+    h = _ri(dev, g, batch, max(seqlen, 1), 2048)
+    conv, ssm = _states(m, dev, g, batch, torch.float32, 4)
+    conv2, ssm2 = conv.clone(), ssm.clone()
+    out = _layer_call.call(m, h, conv, ssm, step)
+    assert out is not None and m.norm.group_size in (None, 4096)
+    _close(out[:, 0] if step else out, m._step_modules(h, conv2, ssm2) if step else m._forward_modules(h, conv2, ssm2), (conv, conv2), (ssm, ssm2))
+
+
 @pytest.mark.parametrize("d_model,batch,seqlen", [(768, 1, 65), (768, 16, 33), (1536, 1, 515), (1536, 12, 70), (2560, 16, 31), (3072, 3, 100)])
 def test_forward_of_a_wide_layer(dev, d_model, batch, seqlen):
     """dt_proj inside the scan: ranks of 48, 96, 160 and 192, sixteen, eight and four lanes per channel, both at once."""
