@@ -200,7 +200,7 @@ __global__ __launch_bounds__(kThreads) void conv2_update4_kernel(QaConv2Params p
     const Part part = part_of(p, ch0);
     const ConvQuad quad = conv_quad(p, part, ch0);
     int64_t out_ls, out_cs;
-    *reinterpret_cast<uint32_t*>(out_ptr(p, part, b, ch0, &out_ls, &out_cs)) = conv_step4<CHANNEL_ROWS>(p, b, ch0, part, quad, held, x_new);
+    *reinterpret_cast<uint32_t*>(out_ptr(p, part, b, ch0, &out_ls, &out_cs)) = conv_step4<CHANNEL_ROWS>(p, b, ch0, quad, held, x_new);
 }
 
 int validate(const QaConv2Params* p, bool update) {

@@ -44,7 +44,7 @@ struct Cfg {
     static constexpr int kRing = kWaves * DEPTH * kUnit, kSums = kWaves * kPassRows * kPitch * 4;
     static constexpr int kColScales = (BN + 63) / 64 * 64, kRowScales = 64;
     static constexpr int kScalesAt = kRing > kSums ? kRing : kSums;
-    static constexpr int kColumnsAt = kScalesAt + (kColScales + kRowScales) * 4;
+    static constexpr int kColumnsAt = (kScalesAt + (kColScales + kRowScales) * 4 + 15) / 16 * 16;
     static constexpr int kLdsBytes = kColumnsAt + BN / 4 * static_cast<int>(sizeof(ConvQuad));
     static constexpr int kQuads = (kPass / 4 + kThreads - 1) / kThreads;               // of outputs in a pass, per thread
     static_assert(BM <= 64 && BN <= 256 && kLdsBytes <= 160 * 1024, "tile shape");
@@ -249,7 +249,7 @@ __global__ __launch_bounds__((Cfg<BITS, BM, BN, DEPTH>::kThreads)) void gemm_spl
                 }
                 const Part part = part_of(f.conv, n - f.ch0);
                 int64_t ls, cs;
-                *reinterpret_cast<uint32_t*>(out_ptr(f.conv, part, m, n - f.ch0, &ls, &cs)) = conv_step4<CONV == kConvRows>(f.conv, m, n - f.ch0, part, quads[quad], held[i][q], word);
+                *reinterpret_cast<uint32_t*>(out_ptr(f.conv, part, m, n - f.ch0, &ls, &cs)) = conv_step4<CONV == kConvRows>(f.conv, m, n - f.ch0, quads[quad], held[i][q], word);
             }
             continue;
         }
