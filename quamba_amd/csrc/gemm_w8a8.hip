@@ -9,6 +9,8 @@
 #include "gemm_core.hpp"
 #include "gemv.hpp"
 
+#include <type_traits>
+
 // Built with -DQA_GEMM_CLK (bench.py --gemm-phase-clocks, never the product library) thread 0 of every workgroup of
 // the tiled kernel records the shader clock and the constant 100 MHz clock at four points - start, first fragments
 // in registers, end of the main loop, end of the epilogue - and qa_gemm_clk_read copies the table out.
@@ -37,7 +39,9 @@ namespace {
 
 using namespace gemm;
 
-template <int TM, int TN, int WGM, int WGN, int STAGES, int OUT, bool FLEX, bool COL_OUTER>
+constexpr int kNarrow = 256;           // columns whose whole w a workgroup's XCD holds on to
+
+template <int TM, int TN, int WGM, int WGN, int STAGES, int OUT, bool FLEX, bool COL_OUTER, bool TURN>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Params p) {
     using C = Cfg<TM, TN, WGM, WGN, STAGES>;
     constexpr int BM = C::kBM, BN = C::kBN, WAVES = C::kWaves;
@@ -65,6 +69,17 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
     load_w.template init<WAVES>(n0, p.n, p.ldw, wave, lane);
 
     const int k_tiles = (p.k + kBK - 1) / kBK;
+    // Where in K this workgroup's k tile `tile` lies (past the last one: outside K).  TURN: workgroups do not all start at K's
+    // beginning.  In step, all of them ask for the same 128 bytes of rows that lie K bytes apart, which few of the memory's
+    // channels hold; the order of the sum does not matter, it is exact.  The workgroups of an XCD, which share panels through
+    // its L2, start together, an eighth of K from those of the next; with so few columns that w stays in every L2 each row block
+    // by itself.
+    const int turn = !TURN ? 0 : p.n <= kNarrow ? tile_m * 7 % k_tiles : static_cast<int>(blockIdx.x % 8) * k_tiles / 8;
+    auto k_of = [&](int tile) {
+        if constexpr (!TURN) return tile * kBK;
+        const int t = tile + turn;
+        return tile >= k_tiles ? k_tiles * kBK : (t >= k_tiles ? t - k_tiles : t) * kBK;
+    };
     Epilogue e;
     e.use_alpha = p.use_alpha; e.alpha = p.alpha; e.round_mode = p.round_mode; e.col_outer = p.scale_order;
     e.ldd = p.ldd; e.d = p.d;
@@ -88,20 +103,21 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
         using Mma = RotatedMma<TM, TN>;
         constexpr int kReq = C::kAInstr + C::kWInstr, kPace = kReq <= Mma::kPerTile / 4 ? 4 : Mma::kPerTile / kReq;
         constexpr int kEarly = Mma::kBehindBarrier / kPace < kReq ? Mma::kBehindBarrier / kPace : kReq;
-        auto request = [&](int r, int tile, uint32_t stage) {
-            if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, tile * kBK, p.k, lds_base + stage, wave);
-            else if (r < kReq) load_w.template issue_one<WAVES>(r - C::kAInstr, rsrc_w, tile * kBK, p.k, lds_base + stage + BM * kBK, wave);
+        auto request = [&](int r, int k0, uint32_t stage) {
+            if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, k0, p.k, lds_base + stage, wave);
+            else if (r < kReq) load_w.template issue_one<WAVES>(r - C::kAInstr, rsrc_w, k0, p.k, lds_base + stage + BM * kBK, wave);
         };
-        auto request_whole = [&](int r, int tile, uint32_t stage) {
-            if (r < C::kAInstr) load_a.template issue_whole<WAVES>(r, rsrc_a, tile * kBK, lds_base + stage, wave);
-            else if (r < kReq) load_w.template issue_whole<WAVES>(r - C::kAInstr, rsrc_w, tile * kBK, lds_base + stage + BM * kBK, wave);
+        auto request_whole = [&](int r, int k0, uint32_t stage) {
+            if (r < C::kAInstr) load_a.template issue_whole<WAVES>(r, rsrc_a, k0, lds_base + stage, wave);
+            else if (r < kReq) load_w.template issue_whole<WAVES>(r - C::kAInstr, rsrc_w, k0, lds_base + stage + BM * kBK, wave);
         };
 #pragma unroll
         for (int t = 0; t < STAGES - 1; ++t)
 #pragma unroll
-            for (int r = 0; r < kReq; ++r) request(r, t, t * C::kStageBytes);
+            for (int r = 0; r < kReq; ++r) request(r, k_of(t), t * C::kStageBytes);
+        int k_late = k_of(STAGES - 1);                                 // of the tile STAGES - 1 further than the one at hand
 #pragma unroll
-        for (int r = 0; r < kEarly; ++r) request(r, STAGES - 1, (STAGES - 1) * C::kStageBytes);
+        for (int r = 0; r < kEarly; ++r) request(r, k_late, (STAGES - 1) * C::kStageBytes);
         __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 2) * kReq + kEarly));
         __syncthreads();
         const uint8_t* my_a = lds + (wm * TM * 32) * kBK;
@@ -113,12 +129,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
         uint32_t cur = 0, late = (STAGES - 1) * C::kStageBytes;        // stages of this tile and of the tile STAGES - 1 further
         auto multiply = [&](int kt, auto&& req) {
             const uint32_t nxt = cur + C::kStageBytes == C::kLdsBytes ? 0 : cur + C::kStageBytes;
+            const int k_early = k_of(kt + STAGES);
             mma.template tile<(STAGES - 2) * kReq>(my_a + cur, my_w + cur, my_a + nxt, my_w + nxt, [&](int idx) {
                 if (idx % kPace != kPace - 1) return;
                 const int r = idx / kPace;
-                if (r < kEarly) req(r, kt + STAGES, cur);
-                else req(r, kt + STAGES - 1, late);
+                if (r < kEarly) req(r, k_early, cur);
+                else req(r, k_late, late);
             });
+            k_late = k_early;
             late = cur;
             cur = nxt;
         };
@@ -133,8 +151,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
     for (int r = 0; r < 16; ++r) acc[0][0][r] = 0;
     auto issue = [&](int tile) {
         const uint32_t base = lds_base + (tile % STAGES) * C::kStageBytes;
-        load_a.template issue<WAVES>(rsrc_a, tile * kBK, p.k, base, wave);
-        load_w.template issue<WAVES>(rsrc_w, tile * kBK, p.k, base + BM * kBK, wave);
+        load_a.template issue<WAVES>(rsrc_a, k_of(tile), p.k, base, wave);
+        load_w.template issue<WAVES>(rsrc_w, k_of(tile), p.k, base + BM * kBK, wave);
     };
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s) issue(s);
@@ -147,25 +165,26 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_w8a8_kernel(QaGemmW8A8Par
         // (past the end of K every lane is out of range and stores zeros)
         const int nt = kt + STAGES - 1;
         const uint32_t nbase = lds_base + (nt % STAGES) * C::kStageBytes;
+        const int nk = k_of(nt);
         static_assert(C::kAInstr + C::kWInstr <= 4, "a request behind each of four multiplications");
         mma_tile_paced(stage + wm * 32 * kBK, stage + BM * kBK + wn * 32 * kBK, frow, fhalf, acc[0][0], [&](int r) {
-            if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, nt * kBK, p.k, nbase, wave);
-            else if (r < C::kAInstr + C::kWInstr) load_w.template issue_one<WAVES>(r - C::kAInstr, rsrc_w, nt * kBK, p.k, nbase + BM * kBK, wave);
+            if (r < C::kAInstr) load_a.template issue_one<WAVES>(r, rsrc_a, nk, p.k, nbase, wave);
+            else if (r < C::kAInstr + C::kWInstr) load_w.template issue_one<WAVES>(r - C::kAInstr, rsrc_w, nk, p.k, nbase + BM * kBK, wave);
         });
     }
     finish(acc);
     }
 }
 
-template <int TM, int TN, int WGM, int WGN, int STAGES, int OUT, bool FLEX, bool COL_OUTER = false>
+template <int TM, int TN, int WGM, int WGN, int STAGES, int OUT, bool FLEX, bool TURN, bool COL_OUTER = false>
 int launch_one(const QaGemmW8A8Params& p, hipStream_t stream) {
     using C = Cfg<TM, TN, WGM, WGN, STAGES>;
     if constexpr (!FLEX && !COL_OUTER) {
-        if (p.scale_order == 1) return launch_one<TM, TN, WGM, WGN, STAGES, OUT, FLEX, true>(p, stream);
+        if (p.scale_order == 1) return launch_one<TM, TN, WGM, WGN, STAGES, OUT, FLEX, TURN, true>(p, stream);
     }
     const int64_t tiles = static_cast<int64_t>((p.m + C::kBM - 1) / C::kBM) * ((p.n + C::kBN - 1) / C::kBN);
     if (tiles > 0x7fffffffLL) return QA_ERR_SHAPE;
-    auto kernel = gemm_w8a8_kernel<TM, TN, WGM, WGN, STAGES, OUT, FLEX, COL_OUTER>;
+    auto kernel = gemm_w8a8_kernel<TM, TN, WGM, WGN, STAGES, OUT, FLEX, COL_OUTER, TURN>;
     constexpr int kLds = C::kLdsBytes + TileScales<C::kBM, C::kBN, C::kWaves>::kBytes;
     if (kLds > 65536) {
         // allowing more than 64 KiB of dynamic LDS is a per-function attribute; setting it is idempotent
@@ -178,11 +197,11 @@ int launch_one(const QaGemmW8A8Params& p, hipStream_t stream) {
     return check_launch();
 }
 
-template <int TM, int TN, int WGM, int WGN, int STAGES, bool FLEX>
+template <int TM, int TN, int WGM, int WGN, int STAGES, bool FLEX, bool TURN = false>
 int launch_gemm(const QaGemmW8A8Params& p, hipStream_t stream) {
-    if (p.out_type == QA_OUT_I8) return launch_one<TM, TN, WGM, WGN, STAGES, QA_OUT_I8, FLEX>(p, stream);
-    if (p.out_type == QA_OUT_BF16) return launch_one<TM, TN, WGM, WGN, STAGES, QA_OUT_BF16, FLEX>(p, stream);
-    return launch_one<TM, TN, WGM, WGN, STAGES, QA_OUT_F16, FLEX>(p, stream);
+    if (p.out_type == QA_OUT_I8) return launch_one<TM, TN, WGM, WGN, STAGES, QA_OUT_I8, FLEX, TURN>(p, stream);
+    if (p.out_type == QA_OUT_BF16) return launch_one<TM, TN, WGM, WGN, STAGES, QA_OUT_BF16, FLEX, TURN>(p, stream);
+    return launch_one<TM, TN, WGM, WGN, STAGES, QA_OUT_F16, FLEX, TURN>(p, stream);
 }
 
 GemvParams as_gemv(const QaGemmW8A8Params& p) {
@@ -216,7 +235,11 @@ int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
     }
     if (tiles(64, 64) <= cus) return launch_gemm<1, 1, 2, 2, 4, false>(p, stream);
     if (tiles(128, 64) <= cus) return launch_gemm<1, 1, 4, 2, 4, false>(p, stream);
-    if (tiles(128, 128) <= cus) return launch_gemm<2, 1, 2, 4, 4, false>(p, stream);
+    if (tiles(128, 128) <= cus) {
+        // (16384 x 192 x 5120 34.5 -> 26.2 us, 12000 x 160 x 4096 27.5 -> 19.5)
+        if (p.n <= kNarrow && p.k >= 1024 && p.k % kBK == 0) return launch_gemm<2, 1, 2, 4, 4, false, true>(p, stream);
+        return launch_gemm<2, 1, 2, 4, 4, false>(p, stream);
+    }
     if (tiles(128, 256) <= cus) return launch_gemm<2, 2, 2, 4, 3, false>(p, stream);
     // More than a round: what counts is rounds times the tile's work, 128 x 256 at six fifths of its share and the 320-wide
     // ones at 24/25: they move a tenth less per product through the caches, which at the power limit is time (against
@@ -224,9 +247,17 @@ int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
     auto cost = [&](int64_t bm, int64_t bn) { return ((tiles(bm, bn) + cus - 1) / cus) * bm * bn; };
     const int64_t c_sq = cost(256, 256), c_wide = cost(256, 320) * 24 / 25, c_tall = cost(320, 256) * 24 / 25, c_half = cost(128, 256) * 6 / 5;
     if (c_half < c_sq && c_half < c_wide && c_half < c_tall) return launch_gemm<2, 2, 2, 4, 3, false>(p, stream);
-    if (c_wide <= c_sq && c_wide <= c_tall) return launch_gemm<2, 5, 4, 2, 2, false>(p, stream);
-    if (c_tall <= c_sq) return launch_gemm<5, 2, 2, 4, 2, false>(p, stream);
-    return launch_gemm<4, 2, 2, 4, 2, false>(p, stream);                             // 256x256 tile, 8 waves
+    // Starting points in K of their own (us without and with): 16384 x 10240 x 2560 335 -> 313, 16384 x 10448 x 2560 364 -> 343,
+    // 8192 x 2048 x 4096 56.6 -> 53.6, 16384 x 4096 x 8192 394 -> 387, 12000 x 1536 x 3072 51.0 -> 49.1.  A short K is over before they drift
+    // together, and two rounds of tiles share less that way than in step: 12000 x 8192 x 2048 165 -> 170, 3000 x 10240 x 2560 63.5 -> 65.2.
+    const bool turn = p.k % kBK == 0 && (p.k >= 3072 || (p.k >= 2560 && tiles(256, 256) > 2 * cus));
+    auto go = [&](auto turn_c) {
+        constexpr bool kTurn = decltype(turn_c)::value;
+        if (c_wide <= c_sq && c_wide <= c_tall) return launch_gemm<2, 5, 4, 2, 2, false, kTurn>(p, stream);
+        if (c_tall <= c_sq) return launch_gemm<5, 2, 2, 4, 2, false, kTurn>(p, stream);
+        return launch_gemm<4, 2, 2, 4, 2, false, kTurn>(p, stream);                          // 256x256 tile, 8 waves
+    };
+    return turn ? go(std::true_type{}) : go(std::false_type{});
 }
 
 }  // namespace

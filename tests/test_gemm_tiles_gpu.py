@@ -46,6 +46,16 @@ def test_int8_weights_of_few_outputs(dev, M, N, K, order):
     test_int8_weights(dev, M, N, K, order)
 
 
+# workgroups that start at points of their own in K: few columns, a row block each (9 k tiles, the third turn of 7 passes their end);
+# tiles of 256 x 256, 256 x 320 and 320 x 256, an XCD each (20, 24 and 25 k tiles); beside them K with part of a tile, which starts
+# at its beginning
+@pytest.mark.parametrize("M,N,K", [(11000, 130, 1152), (11000, 192, 1024), (11000, 130, 1168), (4090, 4080, 3200), (4200, 10300, 2560), (4800, 5100, 3072),
+                                   (5100, 4800, 3072), (4200, 4300, 3216)])
+@pytest.mark.parametrize("order,dtype", [(0, torch.int8), (1, torch.int8), (0, torch.float16), (0, torch.bfloat16)])
+def test_starting_points_in_k(dev, M, N, K, order, dtype):
+    test_large_tiles_over_a_long_k(dev, M, N, K, order, dtype)
+
+
 # K over the waves of a workgroup: fewer 128-byte units of K than waves, one each, one more, the ring of two units round several
 # times, all with and without a remainder of K; then every other tile, at the K where the dispatch takes it
 @pytest.mark.parametrize("M,N,K", [(m, n, k) for m, n in [(9, 200), (20, 1000), (70, 1900)] for k in (16, 128, 1008, 1024, 1040, 2048, 2064, 3200, 4112)] +
