@@ -237,7 +237,7 @@ int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
         for (int r = 4; r <= 256; r *= 2) {
             const int64_t waves = ch_blocks * (((p.seqlen + r - 1) / r + 3) / 4 * 4) * p.batch;
             const int64_t cost = (waves + simds - 1) / simds * (145 * r + 350) + 100 * r;
-            if (best < 0 || cost < best) { best = cost; run = r; }
+            if (best < 0 || cost < best || (p.seqlen + 4LL * run - 1) / (4 * run) > 65535) { best = cost; run = r; }
         }
     }
     const int64_t run_blocks = (p.seqlen + 4 * run - 1) / (4 * run);
