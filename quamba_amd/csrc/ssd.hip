@@ -1043,11 +1043,19 @@ extern "C" int qa_ssd_chunk_scan_fwd(const QaSsdParams* p, void* stream_) {
     auto launch = [&](auto n_c, auto q_c) {
         constexpr int N = decltype(n_c)::value, Q = decltype(q_c)::value, kScanThreads = 64 * scan_waves_of(Q);
         constexpr size_t kStateLds = sizeof(StateSmem<N, Q>), kScanLds = sizeof(ScanSmem<N, Q>);
-        // as many scan workgroups as the chip holds at once (sixteen waves of up to 128 registers to a CU), each with its share of a
-        // group's heads
+        // Heads a scan workgroup walks: what takes the fewest of them one after the other in the places the chip has at once (sixteen
+        // waves of up to 128 registers to a CU), a workgroup's start counted as a fifth of a head.  (A share of the heads for each
+        // place, 10 and 6 of 16 in 640 workgroups on 512 places, took 8 x 1100 steps of 128 heads 169 us, 131 in
+        // shares of two; 3000 steps of 128 heads 58.6 in shares of three, 47.4 of four; 3 x 1000 steps 54 and 46.)
         const int hpg = heads64 / p->ngroups, units = static_cast<int>(bch / p->nheads) * p->ngroups;
         const int64_t places = static_cast<int64_t>(compute_units()) * (1024 / kScanThreads);
-        const int heads_each = static_cast<int>(std::min<int64_t>((static_cast<int64_t>(units) * hpg + places - 1) / places, hpg));
+        int heads_each = 1;
+        int64_t least = -1;
+        for (int parts = 1; parts <= hpg; ++parts) {
+            const int each = (hpg + parts - 1) / parts;
+            const int64_t cost = (static_cast<int64_t>(units) * ((hpg + each - 1) / each) + places - 1) / places * (5 * each + 1);
+            if (least < 0 || cost < least) { least = cost; heads_each = each; }
+        }
         const bool chain = sums_ws && heads_each == 1 && nc <= kChainChunks;
         auto scan_kernel = chain ? ssd_chunk_scan_kernel<N, Q, kScanChain> : heads_each == 1 ? ssd_chunk_scan_kernel<N, Q, kScanOne> : ssd_chunk_scan_kernel<N, Q, kScanWalk>;
         // With a workgroup per chunk and head these make the step sizes, too, in place of a launch in front: once per head instead of once
