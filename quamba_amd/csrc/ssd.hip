@@ -556,16 +556,15 @@ __global__ __launch_bounds__(256) void ssd_pass_kernel(QaSsdParams p, const floa
 // heads of one (batch, chunk, group) in turn.  A wave owns whole 16-row m-tiles with all 64 channels, a long and a short
 // causal range each (with sixteen tiles: 15 - w and w).
 // C B^T never exists in memory: the chunk's B codes sit in LDS, a lane holds 32 codes of its row of C, and
-// v_mfma_i32_16x16x64_i8 forms (C B^T)^T in 16 x 16 blocks - exact integers, times s_C s_B in fp32, the value
-// the reference's bmm kernel stores.  A block comes out with a lane per row m and four consecutive steps k, which
-// is how the next product wants its first operand: two blocks (steps 4 q .. 4 q + 3 and 16 + 4 q .. 16 + 4 q + 3
+// v_mfma_i32_16x16x64_i8 forms (C B^T)^T in 16 x 16 blocks - exact integers.  A block comes out with a lane per row m and
+// four consecutive steps k, which is how the next product wants its first operand: two blocks (steps 4 q .. 4 q + 3 and 16 + 4 q .. 16 + 4 q + 3
 // of a 32-step piece, q = lane / 16) are the eight values of a lane, and the x operand is read from LDS in the
 // same order (the order of the summation index is free as long as both operands agree).  The same codes of C,
 // dequantised to fp16, are the first operand of term 1; a lane's codes are states 64 i + 16 q .. + 15, and the
 // entering state is read in that order.  Below the diagonal the decay factors into exp(dA_m - R) (one exp per
-// lane and piece) and exp(R - dA_k) dt_k (a table per workgroup) with R = dA at the last step of the piece, so
-// that both exponents are <= 0; on the piece that holds the diagonal it is computed per element, in the
-// reference's order.  While a head's last tile is computed, what the next head needs from memory is on its way to registers.
+// lane and piece, times s_C s_B) and exp(R - dA_k) dt_k (a table per workgroup) with R = dA at the last step of the
+// piece, so that both exponents are <= 0; on the piece that holds the diagonal it is computed per element, in the
+// reference's order: s_C s_B times the integer, the value the reference's bmm kernel stores, times exp, times dt_k.  While a head's last tile is computed, what the next head needs from memory is on its way to registers.
 // Moving a head's bytes (the entering state and x in, y out) and computing it take about as long as each other: 89 us of each for
 // 4 x 4096 steps of 80 heads with nothing else in the kernel, and as a workgroup per head, two to a CU, they ran half one
 // after the other.  Walking heads overlaps them and reads the codes of B and C once for all: 158 -> 135 us, 16 x 1024 of
@@ -588,9 +587,9 @@ struct ScanSmem {
         __attribute__((aligned(16))) _Float16 prev[kP][N];
     };
     __attribute__((aligned(16))) int8_t bq[Q][N];   // B codes; 16-byte piece c of row k at position c ^ (k & BSWZ)
-    __attribute__((aligned(16))) float dt[Q];   // s_C s_B dt_k
+    __attribute__((aligned(16))) float dt[Q];
     __attribute__((aligned(16))) float dA[Q];
-    __attribute__((aligned(16))) float gk[Q];   // exp(dA[end of the 32-step piece] - dA_k) s_C s_B dt_k
+    __attribute__((aligned(16))) float gk[Q];   // exp(dA[end of the 32-step piece] - dA_k) dt_k
     __attribute__((aligned(16))) float xs[kP];  // x scale per channel
     __attribute__((aligned(16))) float xD[kP];  // x scale times skip weight per channel
     __attribute__((aligned(16))) float gate[256];   // SiLU(z_scale code) of the gate's 256 codes, indexed by the code's byte
@@ -791,10 +790,9 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
             sm.xD[tid] = r_xs * (D_scale * r_D);
         }
         if (tid < Q) {
-            const float scaled = cb_scale * r_dt;
-            sm.dt[tid] = scaled;
+            sm.dt[tid] = r_dt;
             sm.dA[tid] = r_dA;
-            sm.gk[tid] = fexp(__shfl(r_dA, lane | 31) - r_dA) * scaled;
+            sm.gk[tid] = fexp(__shfl(r_dA, lane | 31) - r_dA) * r_dt;
         }
 #pragma unroll
         for (int i = 0; i < PB; ++i) {
@@ -899,7 +897,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                 const v4i cb[2] = {cb_of(ks, 0), cb_of(ks, 1)};
                 const float4 g0 = *reinterpret_cast<const float4*>(&sm.gk[ka]), g1 = *reinterpret_cast<const float4*>(&sm.gk[ka + 16]);
                 const float gk[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-                const float e_m = fexp(dA_m - sm.dA[32 * ks + 31]);
+                const float e_m = cb_scale * fexp(dA_m - sm.dA[32 * ks + 31]);       // the scale of C B^T rides with the row's decay
 #pragma unroll
                 for (int e = 0; e < 8; ++e) wv[e] = static_cast<float>(cb[e / 4][e % 4]) * (e_m * gk[e]);
                 times_x(ks, wv);
@@ -911,7 +909,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                 const float4 a4 = *reinterpret_cast<const float4*>(&sm.dA[ka]), d4 = *reinterpret_cast<const float4*>(&sm.dt[ka]);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float cv = ka + e <= m_row ? static_cast<float>(cb[e]) : 0.0f;
+                    const float cv = ka + e <= m_row ? cb_scale * static_cast<float>(cb[e]) : 0.0f;
                     wv[4 * blk + e] = (cv * fexp(fminf(dA_m - lane_of(a4, e), 0.0f))) * lane_of(d4, e);
                 }
             };
