@@ -556,21 +556,21 @@ __global__ __launch_bounds__(256) void ssd_pass_kernel(QaSsdParams p, const floa
 // heads of one (batch, chunk, group) in turn.  A wave owns whole 16-row m-tiles with all 64 channels, a long and a short
 // causal range each (with sixteen tiles: 15 - w and w).
 // C B^T never exists in memory: the chunk's B codes sit in LDS, a lane holds 32 codes of its row of C, and
-// v_mfma_i32_16x16x64_i8 forms (C B^T)^T in 16 x 16 blocks - exact integers.  A block comes out with a lane per row m and
-// four consecutive steps k, which is how the next product wants its first operand: two blocks (steps 4 q .. 4 q + 3 and 16 + 4 q .. 16 + 4 q + 3
-// of a 32-step piece, q = lane / 16) are the eight values of a lane, and the x operand is read from LDS in the
-// same order (the order of the summation index is free as long as both operands agree).  The same codes of C,
-// dequantised to fp16, are the first operand of term 1; a lane's codes are states 64 i + 16 q .. + 15, and the
-// entering state is read in that order.  Below the diagonal the decay factors into exp(dA_m - R) (one exp per
-// lane and piece, times s_C s_B) and exp(R - dA_k) dt_k (a table per workgroup) with R = dA at the last step of the
-// piece, so that both exponents are <= 0; on the piece that holds the diagonal it is computed per element, in the
-// reference's order: s_C s_B times the integer, the value the reference's bmm kernel stores, times exp, times dt_k.  While a head's last tile is computed, what the next head needs from memory is on its way to registers.
-// Moving a head's bytes (the entering state and x in, y out) and computing it take about as long as each other: 89 us of each for
-// 4 x 4096 steps of 80 heads with nothing else in the kernel, and as a workgroup per head, two to a CU, they ran half one
-// after the other.  Walking heads overlaps them and reads the codes of B and C once for all: 158 -> 135 us, 16 x 1024 of
-// 128 257 -> 212, 1 x 1531 of 80 (a head each, so only the shorter code) 21.4 -> 18.9.  The walk has to stay inside 128 registers:
-// with the next head requested ahead of the first tile, or the reads of LDS gathered in front of the products, some values
-// spill, and waiting for a spilled one is waiting for the requests: 144 to 177 us.
+// v_mfma_i32_16x16x64_i8 forms (C B^T)^T in 16 x 16 blocks - exact integers.  A block comes out with a lane per row m and four
+// consecutive steps k, which is how the next product wants its first operand: two blocks (steps 4 q .. 4 q + 3 and 16 + 4 q
+// .. 16 + 4 q + 3 of a 32-step piece, q = lane / 16) are the eight values of a lane, and the x operand is read from LDS in
+// the same order (the order of the summation index is free as long as both operands agree).  The same codes of C, dequantised
+// to fp16, are the first operand of term 1; a lane's codes are states 64 i + 16 q .. + 15, and the entering state is read in
+// that order.  Below the diagonal the decay factors into exp(dA_m - R) (one exp per lane and piece, times s_C s_B) and exp(R -
+// dA_k) dt_k (a table per workgroup) with R = dA at the last step of the piece, so that both exponents are <= 0; on the piece
+// that holds the diagonal it is computed per element, in the reference's order: s_C s_B times the integer, the value the
+// reference's bmm kernel stores, times exp, times dt_k.  While a head's last tile is computed, what the next head needs from
+// memory is on its way to registers.  Moving a head's bytes (the entering state and x in, y out) and computing it take about
+// as long as each other: 89 us of each for 4 x 4096 steps of 80 heads with nothing else in the kernel, and as a workgroup per
+// head, two to a CU, they ran half one after the other.  Walking heads overlaps them and reads the codes of B and C once for
+// all: 158 -> 135 us, 16 x 1024 of 128 257 -> 212, 1 x 1531 of 80 (a head each, so only the shorter code) 21.4 -> 18.9.  The
+// walk has to stay inside 128 registers: with the next head requested ahead of the first tile, or the reads of LDS gathered in
+// front of the products, some values spill, and waiting for a spilled one is waiting for the requests: 144 to 177 us.
 // Two workgroups fit a CU's LDS with 128 states and chunks of 256 steps because the entering state and x take the same place:
 // term 1 of both tiles runs first, x is staged from its registers after it.
 // ---------------------------------------------------------------------------------------------
@@ -591,7 +591,7 @@ struct ScanSmem {
     __attribute__((aligned(16))) float dA[Q];
     __attribute__((aligned(16))) float gk[Q];   // exp(dA[end of the 32-step piece] - dA_k) dt_k
     __attribute__((aligned(16))) float xs[kP];  // x scale per channel
-    __attribute__((aligned(16))) float xD[kP];  // x scale times skip weight per channel
+    __attribute__((aligned(16))) float Dv[kP];  // skip weight per channel
     __attribute__((aligned(16))) float gate[256];   // SiLU(z_scale code) of the gate's 256 codes, indexed by the code's byte
 };
 
@@ -787,7 +787,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
         __half* out = static_cast<__half*>(p.out) + row0 + static_cast<int64_t>(h) * kP;
         if (tid < kP) {
             sm.xs[tid] = r_xs;
-            sm.xD[tid] = r_xs * (D_scale * r_D);
+            sm.Dv[tid] = D_scale * r_D;
         }
         if (tid < Q) {
             sm.dt[tid] = r_dt;
@@ -922,7 +922,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
             }
             times_x(nks - 1, wv);
             // Epilogue: acc[s][j][r] is row m0 + 4 (lane / 16) + r, channel 4 (lane % 16) + j
-            const float4 xD4 = *reinterpret_cast<const float4*>(&sm.xD[4 * l16]);
+            const float4 xs4 = *reinterpret_cast<const float4*>(&sm.xs[4 * l16]), Dv4 = *reinterpret_cast<const float4*>(&sm.Dv[4 * l16]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = m0 + 4 * lq + r;
@@ -930,7 +930,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                     float y[4] = {acc[s][0][r], acc[s][1][r], acc[s][2][r], acc[s][3][r]};
                     if (p.D) {
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) y[j] = __builtin_fmaf(sbyte_of(xq[r], j), lane_of(xD4, j), y[j]);
+                        for (int j = 0; j < 4; ++j) y[j] = __builtin_fmaf(lane_of(xs4, j) * sbyte_of(xq[r], j), lane_of(Dv4, j), y[j]);
                     }
                     if (p.z) {
 #pragma unroll
