@@ -506,7 +506,7 @@ extern "C" int qa_mamba1_step(const QaMamba1Params* p, void* stream) {
     const QaSsmUpdateParams u = update_of(*p, b);
     const QaLinearParams& dt = p->dt_proj;
     int st = QA_ERR_UNSUPPORTED;
-    if (dt.bits == 8) {
+    if (dt.bits == 8 && !(rows == 1 && dt.row_rule == QA_ROW_HALF_AWAY)) {                // (codes rounded half to even)
         const SsmDtProj proj = {static_cast<const int8_t*>(dt.weight), b.x_dbl, p->x_proj.n, dt.row_scale, dt.col_scale, dt.k / 16, dt.col_numel,
                                 rows == 1 && dt.row_rule == QA_ROW_ALPHA, dt.alpha};
         st = mamba1_step(u, proj, static_cast<hipStream_t>(stream));

@@ -1,10 +1,13 @@
 """The library call that enqueues a whole layer against the same layer run module by module: token counts around the
 edges of the scan's tiles and segments, both state types, states of three and four codes, one row (the single-row
 rules of the projections) and many; and what the call leaves to the modules."""
+import ctypes
+
 import pytest
 import torch
 
-from quamba_amd import W4A8QMamba, W4A8QMamba2, W8A8QMamba, W8A8QMamba2, _layer_call
+from quamba_amd import W4A8QMamba, W4A8QMamba2, W8A8QMamba, W8A8QMamba2, _layer_call, _lib
+from quamba_amd.linear import W8A8B8O8LinearParallel
 from tests import test_mixer_variants_gpu as variants
 from tests.test_mixer_variants_gpu import _mamba2, _ri
 
@@ -80,6 +83,33 @@ def test_step_of_a_wide_layer(dev, d_model):
         conv2, ssm2 = conv.clone(), ssm.clone()
         out = _layer_call.call(m, h, conv, ssm, True)
         _close(out[:, 0], m._step_modules(h, conv2, ssm2), (conv, conv2), (ssm, ssm2))
+
+
+def test_step_with_a_dt_proj_that_rounds_half_away(dev):
+    """One row's rule of the parallel linear, which a caller of the C ABI may name for any projection: half of the step sizes'
+    codes sit at a tie."""
+    m, g = _mamba1(W8A8QMamba, dev, seed=1)
+    lin, other = m.dt_proj, W8A8B8O8LinearParallel(m.dt_proj.in_features, m.dt_proj.out_features, device=dev)
+    for t in (lin, other):
+        t._set_weight(_ri(dev, torch.Generator(device=dev).manual_seed(2), t.out_features, t.in_features, lo=-1, hi=2))
+        t.a, t.b = torch.ones(1, 1, device=dev), torch.full((1, t.b.numel()), 0.5, device=dev)
+    h = _ri(dev, g, 1, 1, 256)
+    conv, ssm = _states(m, dev, g, 1, torch.float32, 4)
+    states = [(conv.clone(), ssm.clone()) for _ in range(3)]
+    p = _lib.QaMamba1Params.from_buffer_copy(_layer_call._native(m)[1])
+    p.batch = p.seqlen = p.state_is_fp32 = 1
+    p.dt_proj.row_rule = _lib.QA_ROW_HALF_AWAY
+    p.conv_state_batch_stride, p.conv_state_c_stride, p.conv_state_l_stride = conv.stride()
+    out = torch.empty(1, 1, p.out_proj.n, dtype=torch.float16, device=dev)
+    p.workspace_bytes = _lib.lib().qa_mamba1_workspace_bytes(ctypes.byref(p), 1)
+    work = torch.empty(p.workspace_bytes, dtype=torch.uint8, device=dev)
+    p.hidden, p.out, p.conv_state, p.ssm_state, p.workspace = (t.data_ptr() for t in (h, out, *states[0], work))
+    _lib.check(_lib.lib().qa_mamba1_step(ctypes.byref(p), _lib.current_stream(dev)), "mamba1_step")
+    even = m._step_modules(h, *states[1])
+    m.dt_proj = other
+    want = m._step_modules(h, *states[2])
+    _close(out[:, 0], want, *zip(states[0], states[2]))
+    assert not torch.equal(even, want) and float((states[1][1] - states[2][1]).abs().max()) > 1e-2 * float(ssm.abs().max())
 
 
 @pytest.mark.parametrize("cls,d_model,batch,width", [(W8A8QMamba, 768, 3, 4), (W8A8QMamba, 2560, 30, 4), (W8A8QMamba, 2560, 61, 4), (W8A8QMamba, 2560, 20, 3),
