@@ -16,7 +16,7 @@ def _t(a, dev):
     return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
 
 
-# 32 x 32 (K over the waves), 64 x 64, 128 x 64, 128 x 128, 128 x 256 in one round and in three, 256 x 256, 320-wide
+# K over the waves (the first two), 64 x 64, 128 x 64, 128 x 128, 128 x 256 in one round and in three, 256 x 256
 @pytest.mark.parametrize("M,N,K", [(130, 60, 272), (9, 2100, 2064), (300, 1000, 528), (900, 1200, 400), (1000, 2100, 384), (2100, 2100, 272),
                                    (4700, 4700, 144), (4000, 4000, 160), (4200, 4900, 128)])
 @pytest.mark.parametrize("order", [0, 1])
@@ -38,8 +38,8 @@ def test_int8_weights(dev, M, N, K, order):
     np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
-# K over the waves, 16 x 16 and 32 x 32 outputs: one k step and part of one, a ring of units that goes round, rows and columns
-# with remainders
+# few outputs, rows and columns with remainders: 64 x 64 tiles of one k step, part of one and two, and K over the waves with a ring of
+# units that goes round
 @pytest.mark.parametrize("M,N,K", [(9, 5, 16), (17, 33, 80), (16, 48, 6160), (100, 30, 12304), (256, 250, 144), (257, 250, 144)])
 @pytest.mark.parametrize("order", [0, 1])
 def test_int8_weights_of_few_outputs(dev, M, N, K, order):
@@ -47,8 +47,8 @@ def test_int8_weights_of_few_outputs(dev, M, N, K, order):
 
 
 # workgroups that start at points of their own in K: few columns, a row block each (9 k tiles, the third turn of 7 passes their end);
-# tiles of 256 x 256, 256 x 320 and 320 x 256, an XCD each (20, 24 and 25 k tiles); beside them K with part of a tile, which starts
-# at its beginning
+# tiles of 256 x 256, an XCD each (20 and 25 k tiles; the 320-wide ones are in test_kernel_choice_gpu.py); beside them 128 x 256 tiles
+# and K with part of a tile, which start at the beginning
 @pytest.mark.parametrize("M,N,K", [(11000, 130, 1152), (11000, 192, 1024), (11000, 130, 1168), (4090, 4080, 3200), (4200, 10300, 2560), (4800, 5100, 3072),
                                    (5100, 4800, 3072), (4200, 4300, 3216)])
 @pytest.mark.parametrize("order,dtype", [(0, torch.int8), (1, torch.int8), (0, torch.float16), (0, torch.bfloat16)])
@@ -56,8 +56,9 @@ def test_starting_points_in_k(dev, M, N, K, order, dtype):
     test_large_tiles_over_a_long_k(dev, M, N, K, order, dtype)
 
 
-# K over the waves of a workgroup: fewer 128-byte units of K than waves, one each, one more, the ring of two units round several
-# times, all with and without a remainder of K; then every other tile, at the K where the dispatch takes it
+# K over the waves of a workgroup: as many 128-byte units of K as waves, one more, the ring of two units round several times, all
+# with and without a remainder of K (a K of one unit is a 64 x 64 tile's, and so is 200 x 2510); then other tiles, at the K where the
+# dispatch takes them (every one, and units for a part of the waves only, in test_kernel_choice_gpu.py)
 @pytest.mark.parametrize("M,N,K", [(m, n, k) for m, n in [(9, 200), (20, 1000), (70, 1900)] for k in (16, 128, 1008, 1024, 1040, 2048, 2064, 3200, 4112)] +
                          [(16, 4201, 2192), (3, 12210, 2176), (64, 6001, 2192), (200, 2510, 2176), (61, 18500, 2064)])
 @pytest.mark.parametrize("order,dtype", [(0, torch.int8), (1, torch.int8), (0, torch.float16), (0, torch.bfloat16)])
@@ -97,7 +98,7 @@ def test_k_split_over_the_waves_with_4_bits(dev, M, N, K, grouped, dtype):
     assert torch.equal(got, want)
 
 
-# K over the waves, 64 x 64, 64 x 128, 128 x 128, 192 x 128, expanded once
+# K over the waves in 16 x 16 to 32 x 48, 64 x 128, 128 x 128, 192 x 128, expanded once
 @pytest.mark.parametrize("M,N,K,workspace", [(70, 200, 2176, False), (100, 1000, 384, False), (130, 2050, 1664, False), (250, 2500, 1152, False),
                                              (600, 2100, 256, False), (300, 4200, 1664, False), (70, 9000, 128, False), (700, 3100, 1152, False),
                                              (900, 6100, 128, False), (950, 6100, 896, False), (4000, 3300, 1664, False), (4000, 3300, 1664, True)])
@@ -147,7 +148,7 @@ def test_large_tiles_over_a_long_k(dev, M, N, K, order, dtype):
 
 @pytest.mark.parametrize("M,N,K", [(9, 37, 1040), (64, 300, 640), (65, 300, 640), (1500, 2500, 1712)])
 def test_the_single_row_rules_with_many_rows(dev, M, N, K):
-    """32 x 32 with K over the waves and 128 x 128 with two stages: the host's scalar, and rounding half away from zero."""
+    """16 x 16 with K over the waves and 128 x 128 with two stages: the host's scalar, and rounding half away from zero."""
     g = torch.Generator(device=dev).manual_seed(K)
     a, w = (torch.randint(-128, 128, s, dtype=torch.int8, device=dev, generator=g) for s in ((M, K), (N, K)))
     acc = (a.double() @ w.double().t()).float()

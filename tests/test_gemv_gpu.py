@@ -1,6 +1,6 @@
 """Products with up to eight activation rows against the oracle: one, two and four waves per four weight rows, K and N that
-leave remainders in the lane pieces and the row groups, every row count the kernel is compiled for (from three rows on mostly
-the kernel that splits K)."""
+leave remainders in the lane pieces and the row groups, every row count the kernel is compiled for (seven and eight rows, and three
+and four of many weights, go to the kernel that splits K)."""
 import numpy as np
 import pytest
 import torch

@@ -117,9 +117,10 @@ def test_step_with_a_dt_proj_that_rounds_half_away(dev):
                                                      (W8A8QMamba2, 2560, 17, 3), (W8A8QMamba, 3072, 2, 4),
                                                      (W8A8QMamba, 1024, 4, 4), (W4A8QMamba, 1536, 6, 4), (W4A8QMamba2, 2048, 40, 4), (W4A8QMamba2, 4096, 63, 4)])
 def test_step_of_many_sequences(dev, cls, d_model, batch, width):
-    """in_proj and the conv in one launch for more than two rows: each tile of the product, with one and two passes over its
-    sums, the conv's state by channel and by step (three and four codes), rows and columns with remainders; in the first family
-    dt_proj in the state update's launch, ranks of 48 to 192, one to four entries a wave."""
+    """in_proj and the conv in one launch for more than two rows: tiles of the product (each of them in
+    test_kernel_choice_gpu.py), with one and two passes over its sums, the conv's state by channel and by step (three and four codes),
+    rows and columns with remainders; in the first family dt_proj in the state update's launch, ranks of 48 to 192, one to four
+    entries a wave."""
     dtype = torch.float32 if batch % 2 == 0 else torch.int8
     second = cls in (W8A8QMamba2, W4A8QMamba2)
     sized = lambda d, *a, **k: cls(d_model, *a, **k)

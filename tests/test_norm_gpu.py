@@ -99,6 +99,7 @@ def test_state_dict_and_errors(dev):
 
 # (rows, dim, group_size): the Mamba2-8b form, one group per wave, a whole wave's span per group, decode rows
 FUSED = [(300, 8192, 1024), (70, 8192, 512), (150, 4096, 2048), (131, 2048, 512), (9, 2048, 1024), (1, 8192, 1024),
+         (130, 2048, 2048), (37, 4096, 512), (131, 4096, 1024), (133, 8192, 2048),
          # more rows than workgroups in flight: a workgroup then walks several rows
          (2100, 8192, 1024)]
 

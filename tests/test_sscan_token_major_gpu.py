@@ -49,8 +49,9 @@ def _token_major(d, s, state_dtype, with_z, workspace_bytes, lanes=None):
 
 @pytest.mark.parametrize("batch,dim,seqlen,dtype,with_z,ws", [
     (1, 64, 1, torch.int8, True, 0), (2, 36, 31, torch.float32, True, 0), (3, 1036, 33, torch.int8, False, 0),      # few channels
-    (40, 1024, 40, torch.float32, True, 0), (40, 1024, 65, torch.int8, False, 0),                                   # two kinds of workgroup
-    (48, 1024, 37, torch.float32, True, 0), (48, 1028, 64, torch.int8, False, 0),                                   # four lanes
+    (32, 1280, 40, torch.float32, True, 0), (32, 1280, 65, torch.int8, False, 0),                                   # two kinds of workgroup
+    (40, 1024, 40, torch.float32, True, 0), (40, 1024, 65, torch.int8, False, 0),                                   # four lanes
+    (48, 1024, 37, torch.float32, True, 0), (48, 1028, 64, torch.int8, False, 0),
     (1, 512, 256, torch.float32, True, 1 << 22), (2, 1540, 515, torch.int8, True, 1 << 22), (1, 96, 2049, torch.float32, False, 1 << 22)])
 def test_token_major(dev, batch, dim, seqlen, dtype, with_z, ws):
     d, s = _inputs(dev, batch, dim, seqlen, seed=dim + seqlen)

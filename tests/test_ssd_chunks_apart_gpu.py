@@ -34,7 +34,7 @@ def test_one_entry_at_a_time(dev, B, L, N, G, Q, final_dtype):
 
 
 # the most chunks whose sums the scan chains up itself (8), and one more (the pass between the two); last chunks of 128 and 1 steps
-@pytest.mark.parametrize("B,L,N,G,Q", [(5, 1024, 128, 1, 128), (5, 1025, 128, 2, 128), (5, 1025, 64, 1, 128)])
+@pytest.mark.parametrize("B,L,N,G,Q", [(5, 1024, 128, 1, 128), (5, 1025, 128, 2, 128), (5, 1025, 64, 1, 128), (5, 2050, 64, 1, 256)])
 @pytest.mark.parametrize("final_dtype", [torch.float32, torch.int8])
 def test_one_entry_at_a_time_eight_and_nine_chunks(dev, B, L, N, G, Q, final_dtype):
     test_one_entry_at_a_time(dev, B, L, N, G, Q, final_dtype)
