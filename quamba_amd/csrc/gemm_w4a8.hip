@@ -657,7 +657,7 @@ extern "C" int qa_gemm_w4a8(const QaGemmW4A8Params* p, void* stream_) {
         g.a = p->a; g.w = p->w_packed; g.s_group = p->group_size == 128 ? static_cast<const __half*>(p->s_group) : nullptr;
         g.row_scale = p->s_token; g.col_scale = p->s_channel; g.d = p->d;
         if (gemv_is_faster(4, p->m, p->n, p->k) && g.s_group && p->n % 4 == 0 && (reinterpret_cast<uintptr_t>(p->s_group) & 7u) == 0) return gemv_launch(g, nullptr, stream);
-        const SplitChoice split = split_addressable_w4(p->n, p->k) ? split_choice(4, p->m, p->n, p->k, cus) : SplitChoice{-1, 0.0f};
+        const SplitChoice split = split_addressable_w4(p->n, p->k) ? split_choice(4, p->m, p->n, p->k, cus) : SplitChoice{-1, 0.0f, 0.0f};
         const int way = cheapest_way(*p, cus, split, expandable);
         if (way == kWaySplit) return split_launch_w4(g, split.shape, nullptr, stream);
         if (way == kWay64x64) return p->out_type == QA_OUT_I8 ? launch_tile<QA_OUT_I8>(*p, stream) : launch_tile<QA_OUT_F16>(*p, stream);

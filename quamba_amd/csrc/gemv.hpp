@@ -83,10 +83,10 @@ constexpr SplitShape kSplitShapes[] = {
 };
 struct SplitChoice {
     int shape;
-    float us;
+    float us, rounds;
 };
 inline SplitChoice split_choice(int bits, int m, int n, int k, int cus) {
-    SplitChoice best = {-1, 1e30f};
+    SplitChoice best = {-1, 1e30f, 0.0f};
     for (int i = 0; i < static_cast<int>(sizeof(kSplitShapes) / sizeof(kSplitShapes[0])); ++i) {
         const SplitShape& s = kSplitShapes[i];
         if (s.fixed[bits == 4] < 0.0f) continue;
@@ -102,7 +102,7 @@ inline SplitChoice split_choice(int bits, int m, int n, int k, int cus) {
         if (bits == 4 && rounds > (s.rows == 64 ? 1.0f : 4.0f)) crowd = 1.3f;
         if (bits == 8 && m > n) crowd = rounds > 1.0f ? 1.6f : 1.2f;
         const float us = 2.9f + rounds * crowd * (s.fixed[bits == 4] + s.per_unit[bits == 4] * units);
-        if (tiles <= 0x7fffffff && us < best.us) best = {i, us};
+        if (tiles <= 0x7fffffff && us < best.us) best = {i, us, rounds};
     }
     return best;
 }

@@ -159,6 +159,12 @@ def test_in_proj_with_the_conv_behind_it(dev, cls, d_model, batch, shape):
     _step(dev, cls, d_model, batch, torch.int8 if batch % 2 else torch.float32, f"gemm_split_kernel<{shape}>")
 
 
+# a product in three rounds of workgroups would wait for the conv in each of them: a launch of its own
+@pytest.mark.parametrize("cls,d_model,batch", [(W8A8QMamba, 2048, 65), (W8A8QMamba2, 2560, 33), (W4A8QMamba2, 4096, 65)])
+def test_the_conv_of_many_rows(dev, cls, d_model, batch):
+    _step(dev, cls, d_model, batch, torch.int8, "conv2_update4_kernel")
+
+
 # few rows: dot products with the conv behind them, a wave and two for four weight rows; the recurrence of one, two and more
 # sequences with states of both types; for one row the transform inside out_proj's launch, 12, 1 and 40 column blocks
 @pytest.mark.parametrize("cls,d_model,batch,dtype,names", [
