@@ -122,7 +122,7 @@ int project_conv(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows
     // (words in every operand and in the columns that are stored)
     if (!conv_words_ok(conv) || !(conv_state_in_words(conv) || conv_state_in_rows(conv)) || w.n % 4 != 0 || !aligned4(d)) return QA_ERR_UNSUPPORTED;
     const int cus = compute_units();
-    const SplitChoice split = split_choice(w.bits, rows, w.n, w.k, cus);
+    const SplitChoice split = split_choice(w.bits, rows, w.n, w.k, cus, true);
     const float tiles = w.bits == 8 ? tiles_us_w8(rows, w.n, w.k, cus) : tiles_us_w4(rows, w.n, w.k, cus);
     const SplitShape& shape = kSplitShapes[split.shape];
     const int quads = (shape.rows * shape.cols / 4 + 511) / 512;

@@ -96,7 +96,10 @@ FOUR_BITS = [((9, 201, 128), "split_kernel<4, 16, 16, 2"), ((16, 4201, 1152), "s
              ((70, 1900, 1280), "split_kernel<4, 32, 32, 1"), ((64, 6001, 2176), "split_kernel<4, 32, 48, 1"), ((30, 20001, 2176), "split_kernel<4, 32, 80, 1"),
              ((61, 10201, 2176), "split_kernel<4, 64, 48, 1"), ((64, 18500, 2048), "split_kernel<4, 64, 80, 1"), ((200, 4001, 640), "w4a8_kernel<{}"),
              ((900, 1536, 768), "w4a8_reg_kernel<2, 4, 256, {}"), ((900, 2561, 768), "w4a8_reg_kernel<4, 4, 128, {}"),
-             ((777, 6144, 1536), "w4a8_reg_kernel<6, 4, 128, {}")]
+             ((777, 6144, 1536), "w4a8_reg_kernel<6, 4, 128, {}"),
+             # some rounds of split tiles, and far more rows than columns: tiles that stream K, or fewer rows a split tile
+             ((200, 3071, 768), "w4a8_kernel<{}"), ((1531, 768, 1536), "w4a8_reg_kernel<2, 4, 256, {}"), ((6000, 128, 3072), "w4a8_kernel<{}"),
+             ((4096, 160, 4096), "split_kernel<4, 32, 80, 1")]
 
 
 @pytest.mark.parametrize("size,shape", FOUR_BITS)
