@@ -234,8 +234,11 @@ int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
         // (64 rows and more columns than 256 times 64: what is wanted is the weights at the memory's rate, and 128 x 128 tiles, which
         // do not fetch the rows they lack, ask for them better: 64 x 18560 x 4096 17.9 us by 64 x 80, 15.4 in tiles, 48 x 17600 x 2048
         // 11.1 and 9.7, 33 x 16400 x 8192 24.7 and 25.7)
+        // (a short K: what the tiles' estimate leaves out, their first trip to memory, is then most of it: 9 x 3072 x 96 4.6 us and 4.0 by
+        // 16 x 16, 565 x 405 x 400 4.9 and 4.1 by 16 x 48, 65 x 3352 x 768 5.0 and 4.2 by 32 x 48; 512 x 1024 x 2048 5.7, 6.0 by 32 x 32)
+        const float alone = p.k <= 1024 ? 0.6f : 0.0f;
         const bool streams = p.m <= 64 && kSplitShapes[split.shape].rows == 64;
-        if (split.us < tiles_us_w8(p.m, p.n, p.k, cus) && !streams) return split_launch_w8(as_gemv(p), split.shape, nullptr, stream);
+        if (split.us < tiles_us_w8(p.m, p.n, p.k, cus) + alone && !streams) return split_launch_w8(as_gemv(p), split.shape, nullptr, stream);
     }
     if (tiles(64, 64) <= cus) return launch_gemm<1, 1, 2, 2, 4, false>(p, stream);
     if (tiles(128, 64) <= cus) return launch_gemm<1, 1, 4, 2, 4, false>(p, stream);

@@ -16,7 +16,7 @@ def _t(a, dev):
     return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
 
 
-# K over the waves (the first two), 64 x 64, 128 x 64, 128 x 128, 128 x 256 in one round and in three, 256 x 256
+# K over the waves (the first three), 128 x 64, 128 x 128, 128 x 256 in one round and in three, 256 x 256
 @pytest.mark.parametrize("M,N,K", [(130, 60, 272), (9, 2100, 2064), (300, 1000, 528), (900, 1200, 400), (1000, 2100, 384), (2100, 2100, 272),
                                    (4700, 4700, 144), (4000, 4000, 160), (4200, 4900, 128)])
 @pytest.mark.parametrize("order", [0, 1])
@@ -38,8 +38,8 @@ def test_int8_weights(dev, M, N, K, order):
     np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
-# few outputs, rows and columns with remainders: 64 x 64 tiles of one k step, part of one and two, and K over the waves with a ring of
-# units that goes round
+# few outputs, rows and columns with remainders: K over the waves, of one unit, part of one and two, and with a ring of units that goes
+# round
 @pytest.mark.parametrize("M,N,K", [(9, 5, 16), (17, 33, 80), (16, 48, 6160), (100, 30, 12304), (256, 250, 144), (257, 250, 144)])
 @pytest.mark.parametrize("order", [0, 1])
 def test_int8_weights_of_few_outputs(dev, M, N, K, order):
@@ -57,8 +57,8 @@ def test_starting_points_in_k(dev, M, N, K, order, dtype):
 
 
 # K over the waves of a workgroup: as many 128-byte units of K as waves, one more, the ring of two units round several times, all
-# with and without a remainder of K (a K of one unit is a 64 x 64 tile's, and so is 200 x 2510); then other tiles, at the K where the
-# dispatch takes them (every one, and units for a part of the waves only, in test_kernel_choice_gpu.py)
+# with and without a remainder of K; then other tiles, at the K where the dispatch takes them (200 x 2510 is in 64 x 64 tiles without
+# it, 61 x 18500 in 128 x 128; every one, and units for a part of the waves only, in test_kernel_choice_gpu.py)
 @pytest.mark.parametrize("M,N,K", [(m, n, k) for m, n in [(9, 200), (20, 1000), (70, 1900)] for k in (16, 128, 1008, 1024, 1040, 2048, 2064, 3200, 4112)] +
                          [(16, 4201, 2192), (3, 12210, 2176), (64, 6001, 2192), (200, 2510, 2176), (61, 18500, 2064)])
 @pytest.mark.parametrize("order,dtype", [(0, torch.int8), (1, torch.int8), (0, torch.float16), (0, torch.bfloat16)])

@@ -16,11 +16,12 @@ OUT = {torch.int8: _lib.QA_OUT_I8, torch.float16: _lib.QA_OUT_F16, torch.bfloat1
 
 # (M, N, K) -> what the kernel's name starts with, its output type, order of the scales and starting points in K left out.
 # K of one and of some 128-byte units, units for a part of the waves only, with and without a remainder
-SPLIT_INT8 = [((9, 2001, 400), "16, 16, 2"), ((70, 200, 528), "16, 16, 2"), ((16, 4201, 2192), "16, 32, 1"), ((5, 12210, 2176), "16, 48, 1"),
-              ((40, 4001, 400), "32, 32, 1"), ((70, 1900, 1040), "32, 32, 1"), ((64, 6001, 2192), "32, 48, 1"), ((20, 20001, 2176), "32, 80, 1"),
+SPLIT_INT8 = [((9, 5, 16), "16, 16, 2"), ((9, 3071, 96), "16, 16, 2"), ((300, 1000, 528), "32, 48, 1"), ((9, 2001, 400), "16, 16, 2"), ((70, 200, 528), "16, 16, 2"),
+              ((16, 4201, 2192), "16, 32, 1"), ((5, 12210, 2176), "16, 48, 1"), ((40, 4001, 400), "32, 32, 1"), ((70, 1900, 1040), "32, 32, 1"), ((64, 6001, 2192), "32, 48, 1"), ((20, 20001, 2176), "32, 80, 1"),
               ((17, 18003, 2064), "32, 80, 1"), ((71, 9001, 5136), "64, 80, 1")]
-TILES_INT8 = [((9, 5, 16), "1, 1, 2, 2, 4", False), ((300, 1000, 528), "1, 1, 2, 2, 4", False), ((900, 1200, 400), "1, 1, 4, 2, 4", False),
-              ((1500, 2500, 656), "2, 1, 2, 4, 4", False), ((61, 18500, 2064), "2, 1, 2, 4, 4", False), ((11000, 130, 1152), "2, 1, 2, 4, 4", True), ((1500, 5000, 528), "2, 2, 2, 4, 3", False),
+TILES_INT8 = [((300, 3000, 16), "1, 1, 2, 2, 4", False), ((600, 1000, 528), "1, 1, 2, 2, 4", False), ((900, 1200, 400), "1, 1, 4, 2, 4", False),
+              ((1500, 2500, 656), "2, 1, 2, 4, 4", False), ((61, 18500, 2064), "2, 1, 2, 4, 4", False), ((11000, 130, 1152), "2, 1, 2, 4, 4", True),
+              ((1500, 5000, 528), "2, 2, 2, 4, 3", False),
               ((4090, 5100, 528), "2, 5, 4, 2, 2", False), ((4090, 5100, 3200), "2, 5, 4, 2, 2", True), ((5100, 4090, 528), "5, 2, 2, 4, 2", False),
               ((5100, 4090, 3200), "5, 2, 2, 4, 2", True), ((4090, 4090, 528), "4, 2, 2, 4, 2", False), ((4090, 4080, 3200), "4, 2, 2, 4, 2", True)]
 GEMV_INT8 = [((m, n, k), f"{m + (m == 3)}, {waves}") for m in (1, 2, 3, 4) for n, k, waves in ((201, 1040, 1), (4002, 1552, 4), (5003, 2064, 2))]
@@ -29,7 +30,7 @@ GEMV_INT8 = [((m, n, k), f"{m + (m == 3)}, {waves}") for m in (1, 2, 3, 4) for n
 @pytest.mark.parametrize("size,shape", SPLIT_INT8)
 @pytest.mark.parametrize("order,dtype", [(0, torch.int8), (1, torch.int8), (0, torch.float16), (0, torch.bfloat16)])
 def test_int8_split_over_k(dev, size, shape, order, dtype):
-    _, names = launched.kernels(lambda: tiles.test_large_tiles_over_a_long_k(dev, *size, order, dtype))
+    _, names = launched.kernels(lambda: _int8(dev, *size, order, dtype))
     launched.expect(names, f"gemm_split_kernel<8, {shape}, {OUT[dtype]}, 0>")
 
 
