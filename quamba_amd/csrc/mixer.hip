@@ -97,11 +97,12 @@ constexpr int64_t kConvSteps = 65535LL * 4 * 256;       // of a sequence: the gr
 
 // in_proj of a decode step with the conv's step behind it in one launch (QA_ERR_UNSUPPORTED: two launches).  Behind a product
 // that splits K the conv takes 0.3 us and 1.1 per four outputs of a thread, on the few waves that hold the sums, in each round of
-// workgroups; a launch of its own takes 4.0, with grouped scales, whose table is walked first, 5.5 - and the product may then be
+// workgroups; 0.8 with 4-bit weights in tiles of up to 32 x 32, of which a CU has two at a time, one at its conv and one at its
+// product.  A launch of its own takes 4.0, with grouped scales, whose table is walked first, 5.5 - and the product may then be
 // another, faster one (us, apart -> together: int8 16 x 10240 x 2560 11.3 -> 8.6, 64 x 10240 x 2560 11.2 -> 10.8, 128 x 10240 x 2560
-// 14.2 -> 15.9; 4 bits 24 x 10240 x 2560 9.9 -> 8.1, 40 x 8480 x 2048 12.4 -> 10.9, 64 x 18560 x 4096 33 -> 31; in three rounds, for
-// which the conv was once counted once, int8 65 x 8192 x 2048 10.0 -> 12.3, 33 x 10576 x 2560 11.5 -> 13.2, 4 bits 65 x 18560 x 4096
-// 30.5 -> 37.4).
+// 14.2 -> 15.9; 4 bits 24 x 10240 x 2560 9.9 -> 8.1, 40 x 8480 x 2048 12.4 -> 10.9, 64 x 18560 x 4096 33 -> 31; in three and four rounds
+// int8 65 x 8192 x 2048 10.0 -> 12.3, 33 x 10576 x 2560 11.5 -> 13.2, 4 bits 65 x 18560 x 4096 30.5 -> 37.4, but 65 x 8192 x 2048
+// 13.5 -> 11.8, 65 x 10576 x 2560 17.7 -> 16.1).
 int project_conv(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows, int8_t* d, int ch0, const QaConv2Params& conv, void* stream) {
     const GemvConv f = {ch0, conv};
     if (!gemv_conv_ok(f)) return QA_ERR_UNSUPPORTED;
@@ -126,7 +127,8 @@ int project_conv(const QaLinearParams& w, const int8_t* a, int64_t lda, int rows
     const float tiles = w.bits == 8 ? tiles_us_w8(rows, w.n, w.k, cus) : tiles_us_w4(rows, w.n, w.k, cus);
     const SplitShape& shape = kSplitShapes[split.shape];
     const int quads = (shape.rows * shape.cols / 4 + 511) / 512;
-    if (split.us + split.rounds * (0.3f + 1.1f * static_cast<float>(quads)) > std::min(split.us, tiles) + (conv.x_head_group_range ? 5.5f : 4.0f)) return QA_ERR_UNSUPPORTED;
+    const float of_conv = w.bits == 4 && shape.rows * shape.cols <= 32 * 32 ? 0.8f : 0.3f + 1.1f * static_cast<float>(quads);
+    if (split.us + split.rounds * of_conv > std::min(split.us, tiles) + (conv.x_head_group_range ? 5.5f : 4.0f)) return QA_ERR_UNSUPPORTED;
     return w.bits == 8 ? split_launch_w8(g, split.shape, &f, static_cast<hipStream_t>(stream)) : split_launch_w4(g, split.shape, &f, static_cast<hipStream_t>(stream));
 }
 

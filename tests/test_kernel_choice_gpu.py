@@ -149,7 +149,7 @@ STEPS = [(W8A8QMamba, 256, 7, "8, 16, 16, 2, 0, 1"), (W8A8QMamba, 512, 61, "8, 1
          (W8A8QMamba, 1536, 67, "8, 32, 80, 1, 0, 1"),
          (W4A8QMamba, 256, 7, "4, 16, 16, 2, 0, 1"), (W4A8QMamba, 256, 66, "4, 16, 32, 1, 0, 1"), (W4A8QMamba, 2560, 5, "4, 16, 48, 1, 0, 1"),
          (W4A8QMamba, 512, 67, "4, 32, 32, 1, 0, 1"), (W4A8QMamba, 768, 83, "4, 32, 48, 1, 0, 1"), (W4A8QMamba, 1536, 67, "4, 64, 48, 1, 0, 1"),
-         (W4A8QMamba, 2560, 99, "4, 64, 80, 1, 0, 1"),
+         (W4A8QMamba, 2560, 99, "4, 64, 80, 1, 0, 1"), (W4A8QMamba, 2048, 65, "4, 32, 32, 1, 0, 1"),
          (W8A8QMamba2, 256, 7, "8, 16, 16, 2, 0, 2"), (W8A8QMamba2, 512, 47, "8, 16, 32, 1, 0, 2"), (W8A8QMamba2, 2048, 5, "8, 16, 48, 1, 0, 2"),
          (W8A8QMamba2, 256, 99, "8, 32, 32, 1, 0, 2"), (W8A8QMamba2, 768, 67, "8, 32, 48, 1, 0, 2"), (W8A8QMamba2, 1536, 66, "8, 32, 80, 1, 0, 2"),
          (W8A8QMamba2, 2048, 97, "8, 64, 80, 1, 0, 2"),
