@@ -266,17 +266,20 @@ int validate(const QaConv2Params* p, bool update) {
 
 namespace qa {
 int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
-    // Steps per wave: 4 to 256, whichever takes the busiest SIMD's waves the shortest: in ns about 145 a step and 350 for a
-    // wave's set-up (taps, scales, the three inputs ahead), and 100 a step of the last wave with nobody beside it.  Measured
+    // Steps per wave: 4 to 256, whichever takes the busiest SIMD's waves the shortest: in ns about 145 a step and 250 for a
+    // wave's set-up (taps, scales, the three inputs ahead), and 160 a step of the last wave with nobody beside it.  Measured
     // with runs of 4, 8, 16, 32, 64 steps, us: 1 x 512 x 1536 channels 5.5, 6.7, 8.2, 11.1, 17.4; 1 x 777 x 3072 5.9, 6.5, 8.1, 11.4, 18.2;
-    // 1 x 1531 x 5376 14.6, 12.6, 13.1, 14.4, 20.7; 4 x 4096 x 5376 87.7, 64.4, 57.0, 56.5, 60.8; 16 x 1024 x 10240 164, 118, 99, 95, 95.
+    // 1 x 1531 x 5376 14.6, 12.6, 13.1, 14.4, 20.7; 4 x 1299 x 1920 11.2, 11.2, 12.2, 14.5, 18.8; 4 x 4096 x 5376 87.7, 64.4, 57.0, 56.5, 60.8;
+    // 16 x 1024 x 10240 164, 118, 99, 95, 95.  Two and three taps, which come byte by byte: 350 and 100.  Over 148 sizes of each the choice
+    // is 0.2 % behind the best run and 0.3 with fewer taps (0.9 with their figures for four taps as well).
     int run = 4;
     {
         const int64_t ch_blocks = (p.dim + 255) / 256, simds = 4LL * compute_units();
+        const int set_up = p.width == 4 ? 250 : 350, alone = p.width == 4 ? 160 : 100;
         int64_t best = -1;
         for (int r = 4; r <= 256; r *= 2) {
             const int64_t waves = ch_blocks * (((p.seqlen + r - 1) / r + 3) / 4 * 4) * p.batch;
-            const int64_t cost = (waves + simds - 1) / simds * (145 * r + 350) + 100 * r;
+            const int64_t cost = (waves + simds - 1) / simds * (145 * r + set_up) + alone * r;
             if (best < 0 || cost < best || (p.seqlen + 4LL * run - 1) / (4 * run) > 65535) { best = cost; run = r; }
         }
     }
