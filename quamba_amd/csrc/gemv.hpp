@@ -32,8 +32,8 @@ struct GemvParams {
 };
 
 // The same as the kernels take it.  What a launch costs the host grows with its arguments - 2.8 us up to 64 bytes, 3.4 at 128, 3.7
-// at 256, 3.9 at 512 - and a decode step of one or two sequences is as long as its launches.  (Products of up to 64 rows:
-// operands below 2^31 bytes.)
+// at 256, 3.9 at 512 - and a decode step of one or two sequences is as long as its launches.  (Row pitches fit an int: qa_gemm_w8a8,
+// qa_gemm_w4a8 and a layer call's checks refuse operands of 0x70000000 bytes and more.)
 struct GemvArgs {
     const int8_t* a;
     const void* w;
@@ -127,7 +127,9 @@ float tiles_us_w4(int m, int n, int k, int cus);
 // block of sixteen here, but a launch of small size is the faster one there: one and two rows, and three and four while the
 // weights are few (in a layer, us with three and four rows, gemv against split: int8 8192 x 2048 with the conv 5.2 against 6.8, 2048 x
 // 4096 3.6 / 4.6, 10240 x 2560 8.0 / 7.7; 4 bits 6144 x 1536 with the conv 5.7 / 6.1, 10240 x 2560 10.3 / 7.5, 8416 x 2048 11.4 / 8.0, 192 x
-// 5120 3.2 / 4.4; at five to eight rows, where it takes twice the registers, int8 10240 x 2560 9.1 / 6.3).
+// 5120 3.2 / 4.4).  Five to eight rows, where a row more takes twice the registers, are the faster ones here with any weights (alone, weights
+// from beyond the L2s: int8 1536 x 48 and 2048 x 4096 the same 4.2, 8192 x 2048 6.4 / 4.8, 10240 x 2560 9.2 / 6.2; 4 bits 192 x 5120 4.2 / 4.3,
+// 3072 x 768 5.0 / 4.2, 2048 x 4096 5.8 / 4.2, 18560 x 4096 18.4 / 11.1).
 inline bool gemv_is_faster(int bits, int m, int n, int k) { return m <= 2 || (m <= kGemvRows && static_cast<int64_t>(n) * k < (bits == 8 ? 20000000 : 10000000)); }
 
 // One activation row that is made on the spot: sat8(round_half_away(H y * had_scale)) of a row y of k fp16 values
