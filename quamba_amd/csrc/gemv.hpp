@@ -95,7 +95,8 @@ inline SplitChoice split_choice(int bits, int m, int n, int k, int cus, bool con
         // 4 bits: workgroups that share a CU expand their codes at the same time, which tells from two of the large tiles and from five of the
         // others on: 777 x 2560 x 5120 33.4 us by 64 x 48, 28.0 expanded once; 777 x 1536 x 3072 17.3 by 64 x 48, 18.3 by 32 x 32, 16.9 in
         // 64 x 128 tiles; 100 x 18560 x 4096 37.5 by 64 x 80, 25.4 in 128 x 128 tiles.  With far more rows than columns hardly anyone
-        // shares the rows: 4096 x 160 x 4096 21.1 by 64 x 48, 14.8 in 64 x 64 tiles, 6000 x 128 x 3072 14.1 by 32 x 32, 11.9 in tiles.
+        // shares the rows: 4096 x 160 x 4096 and 4096 x 192 x 4096 21.1 and 21.5 by 64 x 48, 14.8 and 15.0 in 64 x 64 tiles, 6000 x 128 x 3072
+        // 14.1 by 32 x 32, 11.9 in tiles.
         // 8 bits: with more rows than columns the workgroups each fetch rows of their own from memory, most of all when a CU has
         // several: 2400 x 192 x 5120 14.8 us in two rounds of 32 x 32, 12.5 by 32 x 80, 11.0 in 64 x 64 tiles; 2400 x 160 x 4096 11.4 in
         // two rounds, 8.7 in tiles, 3000 x 128 x 3072 9.5 and 7.5 - but 1800 x 192 x 5120 10.0 by 32 x 48, 11.0 in tiles.
@@ -105,7 +106,7 @@ inline SplitChoice split_choice(int bits, int m, int n, int k, int cus, bool con
         // rounds, 11.8 in two), and a conv behind the product is priced by the round as it is.
         float crowd = 1.0f;
         if (bits == 4 && rounds > (s.rows == 64 ? 1.0f : 4.0f)) crowd = 1.3f;
-        if (bits == 4 && m / 4 > n) crowd = s.rows == 64 ? 1.6f : 1.3f;
+        if (bits == 4 && m / 4 > n) crowd = s.rows == 64 ? 1.8f : 1.3f;
         if (bits == 8 && m > n) crowd = rounds > 1.0f ? 1.6f : 1.2f;
         const float more = conv || k > 2048 ? 0.0f : 0.4f * (rounds - 1.0f);
         const float us = 2.9f + more + rounds * crowd * (s.fixed[bits == 4] + s.per_unit[bits == 4] * units);
