@@ -16,7 +16,8 @@
 // 4.8, 64 x 2560 x 5120 7.8 -> 6.6, 200 x 2560 x 5120 11.8 -> 10.2; 4 bits 24 x 192 x 5120 7.4 -> 4.4, 24 x 2560 x 5120 8.1 -> 5.9,
 // 64 x 4096 x 8192 12.3 -> 9.3, 24 x 10240 x 2560 9.7 -> 6.4, 64 x 18560 x 4096 18.6 -> 16.6.  What is left of a small one is the
 // launch (2.9); the large ones wait for their units, of which a CU holds 100 KB at a time (int8 64 x 10240 x 2560: 64 x 64
-// tiles that stream K past one ring take 7.2, 64 x 48 of these 9.4).
+// tiles that stream K past one ring take 7.2, 64 x 48 of these 9.4).  With 4-bit weights the fragment reads conflict in LDS, 1.6 to 2.2
+// cycles per active one (int8 32 x 32 none, 32 x 80 0.7).
 //
 // With a conv behind the product (GemvConv) a thread that has the new inputs of four channels makes their conv step as well:
 // the state arrives during the product, and a launch and a round trip through memory are saved.

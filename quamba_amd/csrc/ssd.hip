@@ -568,7 +568,7 @@ __global__ __launch_bounds__(256) void ssd_pass_kernel(QaSsdParams p, const floa
 // memory is on its way to registers.  Moving a head's bytes (the entering state and x in, y out) and computing it take about
 // as long as each other: 89 us of each for 4 x 4096 steps of 80 heads with nothing else in the kernel, and as a workgroup per
 // head, two to a CU, they ran half one after the other.  Walking heads overlaps them and reads the codes of B and C once for
-// all: 158 -> 135 us, 16 x 1024 of 128 257 -> 212, 1 x 1531 of 80 (a head each, so only the shorter code) 21.4 -> 18.9.  The
+// all: 158 -> 127 us, 16 x 1024 of 128 257 -> 213, 1 x 1531 of 80 (a head each, so only the shorter code) 21.4 -> 19.7.  The
 // walk has to stay inside 128 registers: with the next head requested ahead of the first tile, or the reads of LDS gathered in
 // front of the products, some values spill, and waiting for a spilled one is waiting for the requests: 144 to 177 us.
 // Two workgroups fit a CU's LDS with 128 states and chunks of 256 steps because the entering state and x take the same place:
