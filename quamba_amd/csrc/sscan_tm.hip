@@ -538,7 +538,9 @@ TmPlan plan_of(const QaSScanParams& p) {
     } else if (2 * waves4 <= 3 * simds) {
         // Few channels: eight lanes and, as the costs of the two launches have it, segments of 64 steps and more (the second
         // launch, its state loads and the chain of end states cost about 5 us: 1 x 4096 x 1536 channels takes 58 us in
-        // sixteen segments and 250 in one; 3 x 1021 x 5120, which has two waves per SIMD as it is, 88 in one and 106 in two)
+        // sixteen segments and 250 in one; 3 x 1021 x 5120, which has two waves per SIMD as it is, 88 in one and 106 in two).  Up to here
+        // eight lanes are the faster ones, from here on four: 8 x 512 x 3072, one and a half waves of four lanes per SIMD, 63 us against 72;
+        // 13 x 512 x 2048 78 against 71.
         const int64_t wave_rows8 = (p.dim + 31) / 32 * 4, wave_rows16 = (p.dim + 15) / 16 * 4;
         auto per_simd = [&](int64_t waves) { return (waves + simds - 1) / simds; };
         int64_t best = static_cast<int64_t>(p.seqlen) * step_cost(8, true, per_simd(wave_rows8 * p.batch));
