@@ -19,17 +19,18 @@
 // 3063 (nearly all of it writing the codes and reading them back); the scan with it takes 384 and 108 us, and took 384 and
 // 107 with the codes read.
 //
-// Lanes.  NSPLIT lanes share a channel, 16 / NSPLIT states each: four when there are waves enough, eight and sixteen when
-// there are few - a wave's time is then set by its own latencies, and more, shorter waves hide more of them (64 steps of
-// 1536 channels: 10.1 us with four lanes, 7.6 with eight, 6.1 with sixteen).
+// Lanes.  NSPLIT lanes share a channel, 16 / NSPLIT states each: four when there are waves enough, eight when there are fewer -
+// a wave's time is then set by its own latencies, and more, shorter waves hide more of them (64 steps of 1536 channels: 10.1 us
+// with four lanes, 7.6 with eight).  With fewer still the time is cut over the waves of a workgroup (sscan_waves.hip).
 //
-// Segments.  With fewer waves than that a sequence is cut into segments that are scanned side by side: one pass for every
-// segment's end state from a zero state and the sum of its step sizes (OUT false: no C, no outputs), one that starts every
-// segment from the state its predecessors chain up to.
+// Segments.  Few channels of a long sequence leave most of the chip idle even so: the sequence is cut into segments that are
+// scanned side by side, one pass for every segment's end state from a zero state and the sum of its step sizes (OUT false: no
+// C, no outputs), one that starts every segment from the state its predecessors chain up to.
 #include "conv_common.hpp"
 #include "gemm_core.hpp"
 #include "mixer_common.hpp"
 #include "sscan_common.hpp"
+#include "sscan_waves.hpp"
 
 #include <algorithm>
 
@@ -42,7 +43,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 
 template <int NSPLIT>
 struct TmCfg {
-    static constexpr int T = NSPLIT == 16 ? 64 : 32;       // steps per tile
+    static constexpr int T = 32;                           // steps per tile
     static constexpr int NPL = 16 / NSPLIT;                // states per lane
     static constexpr int kCh = kThreads / NSPLIT;          // channels per workgroup
     static constexpr int kWaveCh = 64 / NSPLIT;            // channels per wave
@@ -75,7 +76,7 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
     using Cfg = TmCfg<NSPLIT>;
     constexpr int T = Cfg::T, NPL = Cfg::NPL, kCh = Cfg::kCh, kSteps = Cfg::kSteps;
     constexpr bool kOuter = NSPLIT == 4;                   // B x (step size x input) on the matrix cores
-    static_assert(SPREAD ? NSPLIT <= 8 : !kOuter, "lanes as 16 x 16 products leave them");
+    static_assert(NSPLIT <= 8 && (SPREAD || !kOuter), "lanes as 16 x 16 products leave them");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int kWaveCh = Cfg::kWaveCh;
     const int c_local = SPREAD ? wave * kWaveCh + lane % kWaveCh : tid / NSPLIT;
@@ -94,8 +95,8 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
     // the one in which 16 x 16 products leave the matrix cores: lane l holds rows 4 (l / 16) .. + 3 (channels) of column
     // l % 16 (steps).
     const int g = lane >> 4, j = lane & 15;
-    const int quad = NSPLIT == 4 ? g : NSPLIT == 8 ? (g & 1) : 0;
-    const int step0 = NSPLIT == 4 ? 2 * j : NSPLIT == 8 ? j + 16 * (g >> 1) : lane;
+    const int quad = NSPLIT == 4 ? g : g & 1;
+    const int step0 = NSPLIT == 4 ? 2 * j : j + 16 * (g >> 1);
     const int lc4 = wave * Cfg::kWaveCh + 4 * quad;
     const int ch4 = min(c0 + lc4, p.dim - 4);              // channels past the last read the last four; nothing of theirs is stored
 
@@ -226,8 +227,7 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
                 for (int e = 0; e < 4; ++e) {
                     int sum;
                     if constexpr (NSPLIT == 4) sum = acc[i][e];
-                    else if constexpr (NSPLIT == 8) sum = g < 2 ? acc[0][e] : acc[1][e];
-                    else sum = g < 2 ? (g == 0 ? acc[0][e] : acc[1][e]) : (g == 2 ? acc[2][e] : acc[3][e]);
+                    else sum = g < 2 ? acc[0][e] : acc[1][e];
                     float v = dt_col[e] * (dt_row * static_cast<float>(sum));
                     v = __builtin_amdgcn_fmed3f(__builtin_rintf(v), -128.0f, 127.0f);          // the int8 code
                     dv[i][e] = __builtin_fmaf(s_dt, v, db4[e]);
@@ -403,7 +403,6 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
                 const float w23 = (odd ? acc[3] : acc[2]) + quad_xor<1>(odd ? acc[2] : acc[3]);
                 own_sum = (hi ? w23 : w01) + quad_xor<2>(hi ? w01 : w23);
                 own_sum += row_from_up<4>(own_sum);
-                if constexpr (NSPLIT == 16) own_sum += row_from_up<8>(own_sum);
             }
             float out_v = own_sum + D_u * code_byte_to_float(o.code, 0);
             if constexpr (HAS_Z) out_v *= gate;
@@ -469,7 +468,6 @@ __device__ __forceinline__ void scan_tm_body(const QaSScanParams& p, const Sscan
 #pragma unroll
             for (int m = 1; m < 16; m <<= 1) dt_sum4[e] += __shfl_xor(dt_sum4[e], m);
             if constexpr (kQuads <= 2) dt_sum4[e] += __shfl_xor(dt_sum4[e], 32);
-            if constexpr (kQuads == 1) dt_sum4[e] += __shfl_xor(dt_sum4[e], 16);
             if (j == 0 && g == quad && c0 + lc4 < p.dim) p.dt_sum_out[static_cast<int64_t>(y) * p.dim + c0 + lc4 + e] = dt_sum4[e];
         }
         if (c_ok) {
@@ -511,19 +509,18 @@ __global__ __launch_bounds__(kThreads, 3) void scan_tm_mixed_kernel(QaSScanParam
 // How a launch is laid out: lanes per channel (0: two kinds of workgroup, `blocks_a` of the first) and segments.
 struct TmPlan {
     int lanes, blocks_a, segments, segment_len;
+    int waves;                 // of a workgroup that cuts the time over them (sscan_waves.hip); 0: not so
 };
 
-// Nanoseconds per step of a launch with so many waves on its busiest SIMD, as measured (a wave alone is bound by its own
-// latencies; from about three on the vector units are): eight lanes per channel, the same without outputs, sixteen lanes
-// (while there is one wave per SIMD at most, where the shorter wave is the faster one).
-int step_cost(int lanes, bool out, int64_t waves) {
+// Nanoseconds per step of a launch of eight lanes per channel with so many waves on its busiest SIMD, as measured (a wave alone is
+// bound by its own latencies; from about three on the vector units are), and the same without outputs.
+int step_cost(bool out, int64_t waves) {
     static constexpr int kOut[4] = {63, 85, 117, 152}, kState[4] = {45, 60, 78, 100};
-    if (lanes == 16) return waves <= 1 ? 43 : 1 << 20;
     return static_cast<int>(waves <= 4 ? (out ? kOut : kState)[waves - 1] : waves * (out ? 38 : 25));
 }
 
 TmPlan plan_of(const QaSScanParams& p) {
-    TmPlan r = {4, 0, 1, p.seqlen};
+    TmPlan r = {4, 0, 1, p.seqlen, 0};
     const int cus = compute_units();
     const int64_t simds = 4LL * cus, rows = static_cast<int64_t>(p.batch) * p.dim;
     const int64_t waves4 = rows / 16, q = waves4 / simds, rest = waves4 % simds;
@@ -531,34 +528,43 @@ TmPlan plan_of(const QaSScanParams& p) {
         r.segment_len = ((p.seqlen + segments - 1) / segments + 31) / 32 * 32;
         r.segments = (p.seqlen + r.segment_len - 1) / r.segment_len;
     };
+    const ScanWavesPlan over_waves = scan_waves_plan(p, cus);
     if (p.mapping != 0) {
         r.lanes = (p.mapping >> 20) & 0xff;
         r.blocks_a = r.lanes == 0 ? p.mapping & 0xfffff : 0;
-        if (r.lanes == 8 && p.segments > 1) cut(p.segments);
-    } else if (2 * waves4 <= 3 * simds) {
-        // Few channels: eight lanes and, as the costs of the two launches have it, segments of 64 steps and more (the second
-        // launch, its state loads and the chain of end states cost about 5 us: 1 x 4096 x 1536 channels takes 58 us in
-        // sixteen segments and 250 in one; 3 x 1021 x 5120, which has two waves per SIMD as it is, 88 in one and 106 in two).  Up to here
-        // eight lanes are the faster ones, from here on four: 8 x 512 x 3072, one and a half waves of four lanes per SIMD, 63 us against 72;
-        // 13 x 512 x 2048 78 against 71.
-        const int64_t wave_rows8 = (p.dim + 31) / 32 * 4, wave_rows16 = (p.dim + 15) / 16 * 4;
-        auto per_simd = [&](int64_t waves) { return (waves + simds - 1) / simds; };
-        int64_t best = static_cast<int64_t>(p.seqlen) * step_cost(8, true, per_simd(wave_rows8 * p.batch));
-        r.lanes = 8;
-        const int64_t sixteen = static_cast<int64_t>(p.seqlen) * step_cost(16, true, per_simd(wave_rows16 * p.batch));
-        if (p.segments == 0 && sixteen < best) {
-            best = sixteen;
-            r.lanes = 16;
+        if (r.lanes == kScanWavesMapping) {
+            r.lanes = over_waves.lanes;
+            r.waves = over_waves.waves;
+        } else if (r.lanes >= kScanWavesNamed && r.lanes < kScanWavesNamed + 64) {
+            r.waves = r.lanes % 32 + 1;
+            r.lanes = r.lanes < kScanWavesNamed + 32 ? 4 : 8;
         }
+        if (r.lanes == 8 && r.waves == 0 && p.segments > 1) cut(p.segments);
+    } else if (2 * waves4 <= 3 * simds) {
+        // Up to one and a half waves of four lanes per SIMD eight lanes are the faster ones (8 x 512 x 3072 channels 63 us against
+        // 72; 13 x 512 x 2048 78 against 71), and with fewer the time over the waves of a workgroup, while all workgroups are on the
+        // chip at once (rule and measurements: scan_waves_plan).  Few channels of a long sequence are cut into segments of 64 steps
+        // and more, which take a second launch, their state loads and a chain of end states: about 6.5 us, and 1.3 times the steps'
+        // own cost in both launches (512 channels x 2048 steps 21.6 us, and 30.9 over the waves; 512 x 777 17.5 and 16.6, 1536 x
+        // 4096 68 and 64).
+        const int64_t wave_rows8 = (p.dim + 31) / 32 * 4;
+        auto per_simd = [&](int64_t waves) { return (waves + simds - 1) / simds; };
+        int64_t best = static_cast<int64_t>(p.seqlen) * step_cost(true, per_simd(wave_rows8 * p.batch));
+        r.lanes = 8;
         TmPlan chosen = r;
+        if (p.segments == 0 && over_waves.ns < kScanWavesNever) {
+            best = over_waves.ns;
+            chosen.lanes = over_waves.lanes;
+            chosen.waves = over_waves.waves;
+        }
         for (int n = 2; n <= 32 && 64 * n <= p.seqlen; ++n) {
             cut(n);
             const int64_t w = wave_rows8 * p.batch;
-            const int64_t cost = 5000 + r.segment_len * static_cast<int64_t>(step_cost(8, true, per_simd(w * r.segments)) + step_cost(8, false, per_simd(w * (r.segments - 1))));
+            const int64_t steps = r.segment_len * static_cast<int64_t>(step_cost(true, per_simd(w * r.segments)) + step_cost(false, per_simd(w * (r.segments - 1))));
+            const int64_t cost = 6500 + steps * 13 / 10;
             if (r.segments > 1 && (p.segments == 0 ? cost < best : n == p.segments)) {
                 best = cost;
                 chosen = r;
-                chosen.lanes = 8;
             }
         }
         r = chosen;
@@ -581,7 +587,8 @@ int launch(const QaSScanParams& p_in, const SscanDtProj& dtp, hipStream_t stream
     TmPlan plan = plan_of(p);
     const int vec_out = p.out_d_stride == 1 && aligned16(p.out) && p.out_batch_stride % 8 == 0 && p.out_l_stride % 8 == 0;
     if (plan.segments > 1 && (!p.workspace || p.workspace_bytes < segment_bytes(p, plan))) {
-        p.mapping = 0x40000000 | (plan.lanes << 20);       // one segment
+        const ScanWavesPlan over_waves = scan_waves_plan(p, compute_units());
+        p.mapping = 0x40000000 | (over_waves.ns < kScanWavesNever ? kScanWavesMapping : plan.lanes) << 20;       // one segment
         p.segments = 0;
         plan = plan_of(p);
     }
@@ -596,6 +603,7 @@ int launch(const QaSScanParams& p_in, const SscanDtProj& dtp, hipStream_t stream
         p.carry_state = p.dt_sum_out + static_cast<int64_t>(entries) * p.dim;
         hipLaunchKernelGGL((scan_tm_kernel<8, false, false, DTK>), grid(32, entries), dim3(kThreads), 0, stream, p, dtp, vec_out);
     }
+    if (plan.waves > 0) return sscan_waves_fwd(p, DTK != 0 ? &dtp : nullptr, plan.lanes, plan.waves, stream);
     const int entries = p.batch * plan.segments;
     switch (plan.lanes) {
         case 0:
@@ -603,7 +611,6 @@ int launch(const QaSScanParams& p_in, const SscanDtProj& dtp, hipStream_t stream
             break;
         case 4: hipLaunchKernelGGL((scan_tm_kernel<4, HAS_Z, true, DTK>), grid(64, entries), dim3(kThreads), 0, stream, p, dtp, vec_out); break;
         case 8: hipLaunchKernelGGL((scan_tm_kernel<8, HAS_Z, true, DTK>), grid(32, entries), dim3(kThreads), 0, stream, p, dtp, vec_out); break;
-        case 16: hipLaunchKernelGGL((scan_tm_kernel<16, HAS_Z, true, DTK>), grid(16, entries), dim3(kThreads), 0, stream, p, dtp, vec_out); break;
         default: return QA_ERR_UNSUPPORTED;
     }
     return check_launch();

@@ -205,11 +205,13 @@ def _step(dev, cls, d_model, batch, dtype, *names, per_channel=False):
     launched.expect(ran, *names)
 
 
-# the scan of a prompt with dt_proj inside it, ranks of 64, 80, 160 and 192: four lanes a channel, both kinds of workgroup, segments,
-# eight lanes
+# the scan of a prompt with dt_proj inside it, ranks of 16, 48, 64, 80, 96 and 160: four lanes a channel, both kinds of workgroup,
+# segments, eight lanes, the time over the waves of a workgroup
 @pytest.mark.parametrize("d_model,batch,seqlen,names", [
     (1024, 16, 33, ["scan_tm_kernel<4, true, true, 1>"]), (1280, 16, 35, ["scan_tm_mixed_kernel<true, 2>"]), (2560, 8, 37, ["scan_tm_mixed_kernel<true, 3>"]),
-    (2560, 1, 700, ["scan_tm_kernel<8, false, false, 3>", "scan_tm_kernel<8, true, true, 3>"]), (3072, 1, 515, ["scan_tm_kernel<8, true, true, 3>"])])
+    (256, 1, 1500, ["scan_tm_kernel<8, false, false, 1>", "scan_tm_kernel<8, true, true, 1>"]), (2560, 3, 515, ["scan_tm_kernel<8, true, true, 3>"]),
+    (1536, 1, 37, ["scan_waves_kernel<4, 12, true, 2>"]), (2560, 1, 700, ["scan_waves_kernel<8, 12, true, 3>"]), (768, 1, 515, ["scan_waves_kernel<8, 12, true, 1>"]),
+    (768, 1, 500, ["scan_waves_kernel<8, 16, true, 1>"])])
 def test_scan_of_a_layer(dev, d_model, batch, seqlen, names):
     m, g = _layer(W8A8QMamba, dev, d_model, seqlen)
     h = variants._ri(dev, g, batch, seqlen, d_model)

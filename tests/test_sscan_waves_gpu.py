@@ -1,0 +1,31 @@
+"""The scan that cuts the time over the waves of a workgroup, with named lanes and waves: one wave, the most there can be, lengths
+of a step, around a wave's steps, around a block of all waves and of several blocks, channel counts that are no multiple of a
+workgroup's.  Against the seqlen-major scan (which test_sscan_gpu.py holds to the oracle), with the bars of
+test_sscan_token_major_gpu.py."""
+import pytest
+import torch
+
+from quamba_amd import ops
+from tests.test_sscan_token_major_gpu import _inputs, _token_major
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lanes,waves", [(4, 1), (4, 5), (4, 12), (8, 1), (8, 4), (8, 16)])
+@pytest.mark.parametrize("batch,dim,dtype,with_z", [(1, 4, torch.float32, True), (2, 148, torch.int8, True), (1, 300, torch.float32, False)])
+def test_waves(dev, lanes, waves, batch, dim, dtype, with_z):
+    steps = 16 if lanes == 4 else 32
+    block = steps * waves
+    for seqlen in sorted({1, steps - 1, steps + 1, block - 1, block, block + 1, 2 * block + steps, 3 * block + 3}):
+        d, s = _inputs(dev, batch, dim, seqlen, seed=dim + seqlen)
+        rows = lambda a: a.transpose(1, 2).contiguous()
+        B, Cm = rows(d["bc"][:, :, 8:24])[:, None], rows(d["bc"][:, :, 24:40])[:, None]
+        want, st = ops.sscan_fwd(rows(d["u"]), s["u"], rows(d["dt"]), s["dt"], d["A"], s["A"], B, s["B"], Cm, s["C"], s["st"], d["D"], s["D"],
+                                 rows(d["z"]) if with_z else None, s["z"] if with_z else None, d["db"], s["db"], True, state_dtype=dtype)
+        out, state = _token_major(d, s, dtype, with_z, 0, (64 if lanes == 4 else 96) + waves - 1)
+        assert bool(((out.float() - want.float()).abs() <= 1e-3 + 2e-3 * want.float().abs()).all()), seqlen
+        a, b = state.float(), st[:, :, 0].float()
+        if dtype == torch.int8:
+            assert float((a - b).abs().max()) <= 1
+        else:
+            assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max())
