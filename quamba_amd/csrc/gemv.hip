@@ -1,11 +1,11 @@
 // Up to four activation rows against a weight matrix: a stream over the weights.
 //
 // A wave owns four rows of the weight and the whole of K: a lane takes 16 bytes of each row out of every 1024 (int8: 16
-// codes; 4 bits: 32 codes), so a load of the wave is 1 KB in one piece, and the loads of up to five such pieces of all
-// four rows go out before the first is used.  The matrix cores have nothing to give here - a tile of 16 activation rows
-// would be three quarters or more empty - and their fragments would have to pass through LDS; the products are 4-way int8
-// dot products in the lane that loaded the codes, and LDS is not used at all.  The lanes' partial sums meet through lane
-// swaps (two stages, four values at a time) and row permutes.
+// codes; 4 bits: 32 codes), so a load of the wave is 1 KB in one piece, and the loads of up to four such pieces of all
+// four rows go out before the first is used; a piece is multiplied as it arrives.  The matrix cores have nothing to give
+// here - a tile of 16 activation rows would be three quarters or more empty - and their fragments would have to pass through
+// LDS; the products are 4-way int8 dot products in the lane that loaded the codes, and LDS is not used at all.  The lanes'
+// partial sums meet through lane swaps (two stages, four values at a time) and row permutes.
 //
 // Bound by the memory round trips of a short kernel, not by bandwidth: 1 x 10240 x 2560 with 4-bit weights (13 MB)
 // 10.2 us as a 32-column matrix-core tile per workgroup.
@@ -47,59 +47,85 @@ __device__ __forceinline__ int row_sum(int v) {
     return v;
 }
 
-typedef const __attribute__((address_space(4))) float* const_floats;
-typedef const __attribute__((address_space(4))) int32_t* const_ints;
-template <typename P, typename T>
-__device__ __forceinline__ P scalar_ptr(const T* p) { return reinterpret_cast<P>(reinterpret_cast<uintptr_t>(p)); }
+// The conv behind a product: one output scale and a state of a word per channel (Mamba1's layer), or anything.
+enum ConvKind { kNoConv, kConvOneScale, kConvTables };
 
-// out_scale_of (conv2_common.hpp) for the four channels ch .. ch + 3 of one head, the same in every lane: scalar loads,
-// which do not queue behind the weights, all of a level's at once.
-__device__ __forceinline__ void uniform_out_scales(const QaConv2Params& p, const Part& part, int ch, float (&s)[4]) {
-    if (!p.x_out_scales) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] = p.x_out_scale;
-        return;
+// What a conv step takes of the conv's operands, requested behind the weights by every wave in one straight run: a branch
+// around loads leaves the compiler unsure how many are in flight, and it waits for all of them, the weights among them, where the
+// ways meet.  (Waves without conv channels read the operands of some that are.)
+//
+// The output scale of four channels, neighbours in one part and one head (out_scale_of in conv2_common.hpp): every lane requests its
+// share of the tables of the channels' group at once, and the search in them is a few ballots when the sums are there.  As three scalar
+// loads one after the other, each the index of the next, it held up the products of the weights that came first (in a layer, one row, us:
+// int8 10448 x 2560 8.2 -> 6.5, 3352 x 768 4.6 -> 4.1; 4 bits 18560 x 4096 13.5 -> 12.9, 6280 x 1536 5.7 -> 5.0; two rows 10448 x 2560
+// 9.7 -> 8.6).
+struct ConvOperands {
+    uint32_t taps, held;   // the last three codes of the lane's channel, the oldest in byte 0
+    uint8_t codes[3];      // the same as they are loaded where the state is no word
+    int8_t bias;
+    float scale;           // in_table: of head group lane / 8, dim group lane % 8; else of the lane's own channel
+    int head_end, dim_end; // in_table: where head group `lane` ends, and that dim group
+    bool in_table;
+};
+// ch: the wave's first channel; mine: the lane's; st: the state of that
+template <ConvKind CONV>
+__device__ __forceinline__ ConvOperands request_conv(const QaConv2Params& p, const Part& part, int ch, int mine, const int8_t* st, int lane) {
+    ConvOperands r;
+    r.taps = *reinterpret_cast<const uint32_t*>(p.weight + mine * 4);
+    r.bias = *(p.bias ? p.bias + mine : p.weight);
+    if constexpr (CONV == kConvOneScale) {
+        r.held = *reinterpret_cast<const uint32_t*>(st);
+        return r;
     }
-    const bool grouped = p.x_head_group_range != nullptr && p.x_dim_group_range != nullptr;
-    const const_floats scales = scalar_ptr<const_floats>(part.index == 0 ? p.x_out_scales : part.index == 1 ? p.B_out_scales : p.C_out_scales);
-    int at[4];
-    if (part.index != 0 || !grouped) {
+    const int drop = p.conv_state_len - 3;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) at[e] = grouped ? (ch + e - part.offset) / p.d_state : 0;
-    } else {
-        const int group_size = p.x_dim / p.n_groups, g = ch / group_size, head = (ch % group_size) / p.x_headdim, d = ch % p.x_headdim;
-        const const_ints hr = scalar_ptr<const_ints>(p.x_head_group_range) + g * p.nhead_groups;
-        int ends[kGemvConvGroups], hg = 0;
+    for (int i = 0; i < 3; ++i) r.codes[i] = static_cast<uint8_t>(st[(drop + i) * p.conv_state_l_stride]);
+    const bool grouped = p.x_out_scales && p.x_head_group_range != nullptr && p.x_dim_group_range != nullptr;
+    r.in_table = grouped && part.index == 0;
+    int g = 0, own = 0;
+    if (r.in_table && p.n_groups > 1) g = ch / (p.x_dim / p.n_groups);
+    if (grouped && part.index != 0) own = (mine - part.offset) / p.d_state;
+    const int row = r.in_table ? (g * p.nhead_groups + min(lane >> 3, p.nhead_groups - 1)) * p.ndim_groups + min(lane & 7, p.ndim_groups - 1) : own;
+    const float* const any = reinterpret_cast<const float*>(p.weight);         // (something to read)
+    const float* scales = part.index == 0 ? p.x_out_scales : part.index == 1 ? p.B_out_scales : p.C_out_scales;
+    r.scale = (p.x_out_scales ? scales : any)[row];
+    r.head_end = (r.in_table ? p.x_head_group_range : reinterpret_cast<const int32_t*>(any))[r.in_table ? g * p.nhead_groups + min(lane, p.nhead_groups - 1) : 0];
+    r.dim_end = (r.in_table ? p.x_dim_group_range : reinterpret_cast<const int32_t*>(any))[r.in_table ? row : 0];
+    return r;
+}
+// the output scale of channel ch + which, ch the wave's first (all lanes of the wave active)
+__device__ __forceinline__ float found_out_scale(const QaConv2Params& p, const ConvOperands& r, int ch, int which, int lane) {
+    static_assert(kGemvConvGroups == 8, "eight lanes a head group");
+    if (!p.x_out_scales) return p.x_out_scale;
+    if (!r.in_table) return r.scale;
+    const int head = ch % (p.x_dim / p.n_groups) / p.x_headdim, d = ch % p.x_headdim;
+    const int hg = __popcll(__builtin_amdgcn_ballot_w64(lane < p.nhead_groups - 1 && head >= r.head_end));
+    float found = 0.0f;
 #pragma unroll
-        for (int j = 0; j < kGemvConvGroups; ++j) ends[j] = hr[min(j, p.nhead_groups - 1)];
-#pragma unroll
-        for (int j = 0; j < kGemvConvGroups - 1; ++j) hg += j < p.nhead_groups - 1 && head >= ends[j] ? 1 : 0;
-        const int row = (g * p.nhead_groups + hg) * p.ndim_groups;
-        const const_ints dr = scalar_ptr<const_ints>(p.x_dim_group_range) + row;
-#pragma unroll
-        for (int j = 0; j < kGemvConvGroups; ++j) ends[j] = dr[min(j, p.ndim_groups - 1)];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            int dg = 0;
-#pragma unroll
-            for (int j = 0; j < kGemvConvGroups - 1; ++j) dg += j < p.ndim_groups - 1 && d + e >= ends[j] ? 1 : 0;
-            at[e] = row + dg;
-        }
+    for (int e = 0; e < kRows; ++e) {
+        const uint64_t beyond = __builtin_amdgcn_ballot_w64((lane & 7) < p.ndim_groups - 1 && d + e >= r.dim_end);
+        const int at = 8 * hg + __popcll((beyond >> (8 * hg)) & 0xff);
+        const float s = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.scale), at));
+        found = which == e ? s : found;
     }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] = scales[at[e]];
+    return found;
 }
 
 // BATCH: pieces of K (1 KB of each weight row) whose loads are in flight together.  KS: waves of the workgroup that share
 // four rows, a contiguous part of K each.
-template <int BITS, int M, int KS, int BATCH, int OUT, bool CONV>
-__global__ __launch_bounds__(256) void gemv_kernel(GemvArgs p, std::conditional_t<CONV, GemvConv, NoGemvConv> f) {
+template <int BITS, int M, int KS, int BATCH, int OUT, ConvKind CONV, class Conv>
+__device__ __forceinline__ void gemv_body(const GemvArgs& p, const Conv& f) {
     constexpr int V = kRows * M, PER = V / 4;                    // values of the wave, and per lane after two folds
     constexpr int kLaneCodes = BITS == 8 ? 16 : 32, kPieceCodes = 64 * kLaneCodes, AQ = kLaneCodes / 16;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), part_k = wave % KS;
-    const int n0 = (blockIdx.x * (static_cast<int>(blockDim.x) / (64 * KS)) + wave / KS) * kRows;
+    int n0 = (blockIdx.x * (static_cast<int>(blockDim.x) / (64 * KS)) + wave / KS) * kRows;
     if (KS == 1 && n0 >= p.n) return;
+    if constexpr (CONV != kNoConv) {
+        // the conv's columns go first: their waves have a step more to make when the sums are there
+        const int last = (p.n + kRows - 1) / kRows * kRows;
+        if (n0 < last) n0 += n0 + f.ch0 < last ? f.ch0 : f.ch0 - last;
+    }
     // this wave's part of K
     const int share = (p.k / kLaneCodes + KS - 1) / KS * kLaneCodes;
     const int k_first = part_k * share, k_end = min(k_first + share, p.k);
@@ -110,105 +136,104 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvArgs p, std::conditional_
     const int pieces = (k_end - k_first + kPieceCodes - 1) / kPieceCodes;
     v4u fw[BATCH][kRows], fa[BATCH][M][AQ];
     uint2 fs[BATCH];
-    auto load = [&](int c0) {
+    auto load = [&](int c, int b) __attribute__((always_inline)) {
+        // (lanes past the end read the row's start; their activations are zeroed below)
+        const int k0 = k_first + c * kPieceCodes + lane * kLaneCodes, kk = k0 < k_end ? k0 : 0;
 #pragma unroll
-        for (int b = 0; b < BATCH; ++b) {
-            // (pieces and lanes past the end read the row's start; their activations are zeroed below)
-            const int k0 = k_first + (c0 + b) * kPieceCodes + lane * kLaneCodes, kk = k0 < k_end ? k0 : 0;
+        for (int r = 0; r < kRows; ++r) fw[b][r] = *reinterpret_cast<const v4u*>(w_row[r] + kk * BITS / 8);
+        if constexpr (BITS == 4) fs[b] = *reinterpret_cast<const uint2*>(p.s_group + static_cast<int64_t>(kk / 128) * p.n + min(n0, p.n - 4));
 #pragma unroll
-            for (int r = 0; r < kRows; ++r) fw[b][r] = *reinterpret_cast<const v4u*>(w_row[r] + kk * BITS / 8);
-            if constexpr (BITS == 4) fs[b] = *reinterpret_cast<const uint2*>(p.s_group + static_cast<int64_t>(kk / 128) * p.n + min(n0, p.n - 4));
+        for (int m = 0; m < M; ++m) {
+            const int8_t* a = p.a + min(m, p.m - 1) * p.lda + kk;
 #pragma unroll
-            for (int m = 0; m < M; ++m) {
-                const int8_t* a = p.a + min(m, p.m - 1) * p.lda + kk;
-#pragma unroll
-                for (int q = 0; q < AQ; ++q) fa[b][m][q] = *reinterpret_cast<const v4u*>(a + 16 * q);
-            }
-            if (c0 + b + 1 >= pieces) break;
+            for (int q = 0; q < AQ; ++q) fa[b][m][q] = *reinterpret_cast<const v4u*>(a + 16 * q);
         }
     };
-    load(0);
-    __builtin_amdgcn_sched_barrier(0);
+    int acc[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[v] = 0;
+    auto multiply = [&](int c, int b) __attribute__((always_inline)) {
+        const bool in = k_first + c * kPieceCodes + lane * kLaneCodes < k_end;
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int q = 0; q < AQ; ++q) fa[b][m][q] = in ? fa[b][m][q] : v4u{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            if constexpr (BITS == 8) {
+#pragma unroll
+                for (int m = 0; m < M; ++m)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        acc[m * kRows + r] = __builtin_amdgcn_sdot4(static_cast<int>(fw[b][r][q]), static_cast<int>(fa[b][m][0][q]), acc[m * kRows + r], false);
+            } else {
+                const uint32_t pair = r & 2 ? fs[b].y : fs[b].x;
+                const uint32_t one = r & 1 ? pair >> 16 : pair & 0xffffu;
+                const __half2 s2 = bits_h2(one | (one << 16));
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint2 e = expand_grouped(fw[b][r][q], s2);
+#pragma unroll
+                    for (int m = 0; m < M; ++m) {
+                        int& s = acc[m * kRows + r];
+                        s = __builtin_amdgcn_sdot4(static_cast<int>(e.x), static_cast<int>(fa[b][m][q / 2][2 * (q & 1)]), s, false);
+                        s = __builtin_amdgcn_sdot4(static_cast<int>(e.y), static_cast<int>(fa[b][m][q / 2][2 * (q & 1) + 1]), s, false);
+                    }
+                }
+            }
+        }
+    };
 
     // the value this lane finishes: row `lane / 16` of four, `lane % 16` < PER
     const int quarter = lane >> 4, slot = lane & 15;
     const int value = (quarter >> 1) * (V / 2) + (quarter & 1) * PER + min(slot, PER - 1);
     const int my_m = min(value / kRows, p.m - 1), my_n = min(n0 + value % kRows, p.n - 1);
     const bool mine = slot < PER && value / kRows < p.m && n0 + value % kRows < p.n;
-    const float s_row = p.rule == kGemvAlpha ? p.alpha : p.row_scale[p.one_row_scale ? 0 : my_m];
-    const float s_col = p.rule == kGemvAlpha ? 1.0f : p.col_scale[p.one_col_scale ? 0 : my_n];
-
-    // operands of the conv step of this lane's column
-    bool conv_col = false;
-    int ch = 0;
-    int8_t* st = nullptr;
-    uint32_t taps = 0, held[3] = {};                             // the state's codes, as loaded
-    int bias_q = 0;
-    float c_out_scale = 1.0f;
-    Part part = {};
-    bool st_word = false;
+    float s_row = 0.0f, s_col = 0.0f;
     // (the four columns of a wave are all conv channels, of one part and one head, or none is)
-    if constexpr (CONV) if (n0 >= f.ch0 && n0 < f.ch0 + f.conv.dim) {
-        const QaConv2Params& c = f.conv;
-        conv_col = true;
-        ch = my_n - f.ch0;
-        part = part_of(c, n0 - f.ch0);
-        taps = *reinterpret_cast<const uint32_t*>(c.weight + ch * 4);
-        bias_q = *(c.bias ? c.bias + ch : c.weight);
-        st = c.conv_state + my_m * c.conv_state_batch_stride + ch * c.conv_state_c_stride;
-        st_word = c.conv_state_len == 4 && c.conv_state_l_stride == 1 && (reinterpret_cast<uintptr_t>(c.conv_state) & 3u) == 0 &&
-                  c.conv_state_batch_stride % 4 == 0 && c.conv_state_c_stride % 4 == 0;
-        if (st_word) {
-            held[0] = *reinterpret_cast<const uint32_t*>(st);
-        } else {
-            const int drop = c.conv_state_len - 3;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) held[i] = static_cast<uint8_t>(st[(drop + i) * c.conv_state_l_stride]);
+    bool conv_col = false;
+    int ch0 = 0, ch = 0;                                         // the wave's first channel, the lane's
+    Part part = {};
+    ConvOperands conv;
+    int8_t* st = nullptr;
+    // the scales and the conv's operands, behind the weights
+    auto request_rest = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        const float* const any = reinterpret_cast<const float*>(p.a);          // (the rule without scales reads something)
+        s_row = p.rule == kGemvAlpha ? p.alpha : p.row_scale[p.one_row_scale ? 0 : my_m];
+        s_col = p.rule == kGemvAlpha ? *any : p.col_scale[p.one_col_scale ? 0 : my_n];
+        if constexpr (CONV != kNoConv) {
+            const QaConv2Params& c = f.conv;
+            conv_col = n0 >= f.ch0 && n0 < f.ch0 + c.dim;
+            ch0 = conv_col ? n0 - f.ch0 : 0;
+            ch = conv_col ? my_n - f.ch0 : value % kRows;
+            part = part_of(c, ch0);
+            st = c.conv_state + my_m * c.conv_state_batch_stride + ch * c.conv_state_c_stride;
+            conv = request_conv<CONV>(c, part, ch0, ch, st, lane);
         }
-        float scales[kRows];
-        uniform_out_scales(c, part, n0 - f.ch0, scales);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // all loads of a batch, then its products in their order: one straight run for each number of pieces
+    auto batch = [&](auto p_c, int c0, bool first) __attribute__((always_inline)) {
+        constexpr int P = decltype(p_c)::value;
 #pragma unroll
-        for (int r = 0; r < kRows; ++r) c_out_scale = value % kRows == r ? scales[r] : c_out_scale;
-    }
-
-    int acc[V];
+        for (int b = 0; b < P; ++b) load(c0 + b, b);
+        if (first) request_rest();
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int v = 0; v < V; ++v) acc[v] = 0;
-    for (int c0 = 0; c0 < pieces; c0 += BATCH) {
-        if (c0) load(c0);
-#pragma unroll
-        for (int b = 0; b < BATCH; ++b) {
-            if (c0 + b >= pieces) break;
-            const bool in = k_first + (c0 + b) * kPieceCodes + lane * kLaneCodes < k_end;
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-#pragma unroll
-                for (int q = 0; q < AQ; ++q) fa[b][m][q] = in ? fa[b][m][q] : v4u{0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int r = 0; r < kRows; ++r) {
-                if constexpr (BITS == 8) {
-#pragma unroll
-                    for (int m = 0; m < M; ++m)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q)
-                            acc[m * kRows + r] = __builtin_amdgcn_sdot4(static_cast<int>(fw[b][r][q]), static_cast<int>(fa[b][m][0][q]), acc[m * kRows + r], false);
-                } else {
-                    const uint32_t pair = r & 2 ? fs[b].y : fs[b].x;
-                    const uint32_t one = r & 1 ? pair >> 16 : pair & 0xffffu;
-                    const __half2 s2 = bits_h2(one | (one << 16));
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const uint2 e = expand_grouped(fw[b][r][q], s2);
-#pragma unroll
-                        for (int m = 0; m < M; ++m) {
-                            int& s = acc[m * kRows + r];
-                            s = __builtin_amdgcn_sdot4(static_cast<int>(e.x), static_cast<int>(fa[b][m][q / 2][2 * (q & 1)]), s, false);
-                            s = __builtin_amdgcn_sdot4(static_cast<int>(e.y), static_cast<int>(fa[b][m][q / 2][2 * (q & 1) + 1]), s, false);
-                        }
-                    }
-                }
-            }
+        for (int b = 0; b < P; ++b) multiply(c0 + b, b);
+    };
+    bool done = false;
+    static_for<1, BATCH>([&](auto p_c) {
+        if (!done && pieces == decltype(p_c)::value) {
+            batch(p_c, 0, true);
+            done = true;
         }
+    });
+    if (!done) {
+        batch(std::integral_constant<int, BATCH>{}, 0, true);
+        // (pieces past the last one are lanes past the end)
+        for (int c0 = BATCH; c0 < pieces; c0 += BATCH) batch(std::integral_constant<int, BATCH>{}, c0, false);
     }
 
     int half[V / 2], sum = 0;
@@ -227,6 +252,9 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvArgs p, std::conditional_
 #pragma unroll
         for (int i = 1; i < KS; ++i) sum += parts[wave + i][lane];
     }
+    float c_out_scale = 1.0f;
+    if constexpr (CONV == kConvOneScale) c_out_scale = f.conv.x_out_scale;
+    if constexpr (CONV == kConvTables) if (conv_col) c_out_scale = found_out_scale(f.conv, conv, ch0, value % kRows, lane);
     if (!mine) return;
     const float accf = static_cast<float>(sum);
     float y = p.rule == kGemvHalfAway ? (s_col * s_row) * accf : p.rule == kGemvColOuter ? s_col * (s_row * accf)
@@ -234,19 +262,19 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvArgs p, std::conditional_
     asm volatile("" : "+v"(y));                                  // the fp32 product is rounded on its own
     if constexpr (OUT == QA_OUT_I8) {
         const int8_t q = static_cast<int8_t>(quant8(y, p.half_away ? QA_ROUND_HALF_AWAY : QA_ROUND_RNE));
-        if constexpr (CONV) if (conv_col) {
+        if constexpr (CONV != kNoConv) if (conv_col) {
             const QaConv2Params& c = f.conv;
-            const uint32_t kept = st_word ? held[0] >> 8 : held[0] | (held[1] << 8) | (held[2] << 16);
+            const uint32_t kept = CONV == kConvOneScale ? conv.held >> 8 : conv.codes[0] | (conv.codes[1] << 8) | (conv.codes[2] << 16);
             const uint32_t win = kept | (static_cast<uint32_t>(static_cast<uint8_t>(q)) << 24);
-            if (st_word) {
+            if constexpr (CONV == kConvOneScale) {
                 *reinterpret_cast<uint32_t*>(st) = win;
             } else {
                 for (int i = 0; i < c.conv_state_len; ++i) st[i * c.conv_state_l_stride] = static_cast<int8_t>(win >> (8 * (i + 4 - c.conv_state_len)));
             }
-            float v = c.bias ? part.s_bias * static_cast<float>(bias_q) : 0.0f;
+            float v = c.bias ? part.s_bias * static_cast<float>(conv.bias) : 0.0f;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                v = __builtin_fmaf(part.s_in * static_cast<float>(static_cast<int8_t>(taps >> (8 * i))), static_cast<float>(static_cast<int8_t>(win >> (8 * i))), v);
+                v = __builtin_fmaf(part.s_in * static_cast<float>(static_cast<int8_t>(conv.taps >> (8 * i))), static_cast<float>(static_cast<int8_t>(win >> (8 * i))), v);
             int64_t ls, cs;
             const ConvQuantRegs kq(c_out_scale);
             out_ptr(c, part, my_m, ch, &ls, &cs)[0] = static_cast<int8_t>(conv_quant(v, c_out_scale, 1.0f / c_out_scale, c.silu_activation,
@@ -259,6 +287,15 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvArgs p, std::conditional_
     }
 }
 
+template <int BITS, int M, int KS, int BATCH, int OUT, bool CONV>
+__global__ __launch_bounds__(256) void gemv_kernel(GemvArgs p, std::conditional_t<CONV, GemvConv, NoGemvConv> f) {
+    gemv_body<BITS, M, KS, BATCH, OUT, CONV ? kConvOneScale : kNoConv>(p, f);
+}
+template <int BITS, int M, int KS, int BATCH>
+__global__ __launch_bounds__(256) void gemv_conv_tables_kernel(GemvArgs p, GemvConv f) {
+    gemv_body<BITS, M, KS, BATCH, QA_OUT_I8, kConvTables>(p, f);
+}
+
 template <int BITS, int M, int KS, int BATCH>
 int launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
     const int64_t groups = (static_cast<int64_t>(p.n) + kRows - 1) / kRows;
@@ -266,7 +303,8 @@ int launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>((groups * KS + per_block - 1) / per_block)), block(64 * per_block);
     const GemvArgs args(p);
     const NoGemvConv none = {};
-    if (conv) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, true>), grid, block, 0, stream, args, *conv);
+    if (conv && !conv->conv.x_out_scales && conv_state_in_words(conv->conv)) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, true>), grid, block, 0, stream, args, *conv);
+    else if (conv) hipLaunchKernelGGL((gemv_conv_tables_kernel<BITS, M, KS, BATCH>), grid, block, 0, stream, args, *conv);
     else if (p.out_type == QA_OUT_I8) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, false>), grid, block, 0, stream, args, none);
     else if (p.out_type == QA_OUT_F16) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_F16, false>), grid, block, 0, stream, args, none);
     else hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_BF16, false>), grid, block, 0, stream, args, none);

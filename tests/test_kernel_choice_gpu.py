@@ -24,7 +24,7 @@ TILES_INT8 = [((300, 3000, 16), "1, 1, 2, 2, 4", False), ((600, 1000, 528), "1, 
               ((1500, 5000, 528), "2, 2, 2, 4, 3", False),
               ((4090, 5100, 528), "2, 5, 4, 2, 2", False), ((4090, 5100, 3200), "2, 5, 4, 2, 2", True), ((5100, 4090, 528), "5, 2, 2, 4, 2", False),
               ((5100, 4090, 3200), "5, 2, 2, 4, 2", True), ((4090, 4090, 528), "4, 2, 2, 4, 2", False), ((4090, 4080, 3200), "4, 2, 2, 4, 2", True)]
-GEMV_INT8 = [((m, n, k), f"{m + (m == 3)}, {waves}") for m in (1, 2, 3, 4) for n, k, waves in ((201, 1040, 1), (4002, 1552, 4), (5003, 2064, 2))]
+GEMV_INT8 = [((m, n, k), f"{m + (m == 3)}, {waves}") for m in (1, 2, 3, 4) for n, k, waves in ((201, 1040, 1), (4002, 1552, 4), (5003, 2064, 2), (201, 8336, 4))]
 
 
 @pytest.mark.parametrize("size,shape", SPLIT_INT8)
@@ -118,7 +118,7 @@ def test_four_bits_expanded_once(dev, dtype):
 
 
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
-@pytest.mark.parametrize("N,K,waves", [(204, 1152, 1), (4004, 1664, 4), (4100, 2176, 2)])
+@pytest.mark.parametrize("N,K,waves", [(204, 1152, 1), (4004, 1664, 4), (4100, 2176, 2), (204, 8320, 4)])
 @pytest.mark.parametrize("dtype", [torch.int8, torch.float16])
 def test_four_bits_dot_products(dev, M, N, K, waves, dtype):
     _, names = launched.kernels(lambda: _four_bits(dev, M, N, K, True, dtype))
@@ -179,7 +179,11 @@ def test_the_conv_of_many_rows(dev, cls, d_model, batch):
     (W4A8QMamba, 2048, 1, torch.int8, ["gemv_kernel<4, 1, 2, 1, 0, true>", "mamba1_step_kernel<1, false>", "gemv_rotated_kernel<4, 1>"]),
     (W4A8QMamba, 2048, 2, torch.int8, ["gemv_kernel<4, 2, 2, 1, 0, true>"]),
     (W4A8QMamba, 2560, 1, torch.int8, ["gemv_rotated_kernel<4, 40>"]),
-    (W8A8QMamba, 1536, 1, torch.int8, ["gemv_rotated_kernel<8, 12>"])])
+    (W8A8QMamba, 1536, 1, torch.int8, ["gemv_rotated_kernel<8, 12>"]),
+    # the conv's output scales from tables; a state by step
+    (W8A8QMamba2, 768, 1, torch.int8, ["gemv_conv_tables_kernel<8, 1, 1, 4>"]), (W8A8QMamba2, 2048, 2, torch.float32, ["gemv_conv_tables_kernel<8, 2, 2, 2>"]),
+    (W8A8QMamba2, 256, 3, torch.int8, ["gemv_conv_tables_kernel<8, 4, 1, 3>"]), (W4A8QMamba2, 4096, 1, torch.int8, ["gemv_conv_tables_kernel<4, 1, 1, 2>"]),
+    (W4A8QMamba2, 2048, 2, torch.float32, ["gemv_conv_tables_kernel<4, 2, 2, 1>"]), (W4A8QMamba2, 768, 4, torch.int8, ["gemv_conv_tables_kernel<4, 4, 1, 2>"])])
 def test_step_of_few_rows(dev, cls, d_model, batch, dtype, names):
     _step(dev, cls, d_model, batch, dtype, *names)
 
