@@ -843,7 +843,9 @@ int choose_mapping16(const QaSScanParams& p) {
 // run of loads, arithmetic and stores without loops or branches on the parameter block.
 // CONV_STATE: with CONV and FAST, the codes per row of the conv state (4: a word per row; 3: rows back to back).
 // A_ONE: A_log has one value for all states of a row (Mamba2: one per head), and the decay is evaluated once.
-template <int LPR, bool VEC, bool FP32, bool CONV, bool FAST = false, int CONV_STATE = 4, bool A_ONE = false>
+// STREAM: the state goes past the caches (kStreamBytes).
+typedef float v4f __attribute__((ext_vector_type(4)));
+template <int LPR, bool VEC, bool FP32, bool CONV, bool FAST = false, int CONV_STATE = 4, bool A_ONE = false, bool STREAM = false>
 __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, const QaConvParams* cp) {
     static_assert(!CONV || LPR == 1, "the conv step needs one lane per row");
     static_assert(!FAST || (LPR == 1 && VEC), "the fixed shape has one lane per row and whole pieces");
@@ -960,7 +962,10 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
                 const float4 v = wave_state_in[k * 64 + lane];
                 staged[k][0] = v.x; staged[k][1] = v.y; staged[k][2] = v.z; staged[k][3] = v.w;
             } else if constexpr (FP32) {
-                const float4 v = *reinterpret_cast<const float4*>(static_cast<const float*>(p.state) + st_base + n0);
+                const v4f* from = reinterpret_cast<const v4f*>(static_cast<const float*>(p.state) + st_base + n0);
+                v4f v;
+                if constexpr (STREAM) v = __builtin_nontemporal_load(from);
+                else v = *from;
                 hv[k][0] = v.x; hv[k][1] = v.y; hv[k][2] = v.z; hv[k][3] = v.w;
             } else {
                 *reinterpret_cast<int32_t*>(s8[k]) = *reinterpret_cast<const int32_t*>(static_cast<const int8_t*>(p.state) + st_base + n0);
@@ -1058,8 +1063,10 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
             turn[wv][4 * lane + (k ^ (lane / 4 % 4))] = make_float4(hv[k][0], hv[k][1], hv[k][2], hv[k][3]);
         } else if constexpr (VEC) {
             if constexpr (FP32) {
-                *reinterpret_cast<float4*>(static_cast<float*>(p.state) + st_base + n0) =
-                    make_float4(hv[k][0], hv[k][1], hv[k][2], hv[k][3]);
+                v4f* to = reinterpret_cast<v4f*>(static_cast<float*>(p.state) + st_base + n0);
+                const v4f v = {hv[k][0], hv[k][1], hv[k][2], hv[k][3]};
+                if constexpr (STREAM) __builtin_nontemporal_store(v, to);
+                else *to = v;
             } else {
                 float inv[4];
 #pragma unroll
@@ -1102,10 +1109,17 @@ __device__ __forceinline__ void ssm_update_body(const QaSsmUpdateParams& p, cons
     }
 }
 
-template <int LPR, bool VEC, bool FP32, bool FAST = false, bool A_ONE = false>
+template <int LPR, bool VEC, bool FP32, bool FAST = false, bool A_ONE = false, bool STREAM = false>
 __global__ __launch_bounds__(256) void ssm_update_kernel(QaSsmUpdateParams p) {
-    ssm_update_body<LPR, VEC, FP32, false, FAST, 4, A_ONE>(p, nullptr);
+    ssm_update_body<LPR, VEC, FP32, false, FAST, 4, A_ONE, STREAM>(p, nullptr);
 }
+
+// States from this size on do not stay in the last-level cache (256 MiB) until the next token anyway: kept there they only push
+// out the weights, and what they leave dirty is written back while the next product reads them.  Loads and stores past the
+// caches, a whole Mamba2 step, us: 64 sequences x 128 heads x 64 x 128 (268 MB) with 4-bit weights 132 -> 122 (in_proj 33 -> 24,
+// out_proj 14.4 -> 10.7, the update itself 83 -> 86), int8 143 -> 126; 128 sequences 259 -> 220; 128 x 80 heads (336 MB) 159 -> 135, 96 x
+// 80 (252 MB) 113.5 -> 107.5.  Smaller states are found there again: 48 x 128 (201 MB) 96 -> 100, 32 x 80 (84 MB) 50 -> 52.
+constexpr int64_t kStreamBytes = 224LL << 20;
 
 // conv step + state update of one token in one launch (d_state <= 16, one head)
 template <bool VEC, bool FP32, bool FAST, int CONV_STATE = 4>
@@ -1289,6 +1303,12 @@ int launch_update(const QaSsmUpdateParams& p, hipStream_t stream, const QaConvPa
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, p); };
     if constexpr (LPR == 4 || LPR == 8) {
         if (launch_heads_i8<LPR>(p, stream)) return check_launch();
+    }
+    if constexpr (LPR == 4 || LPR == 8) {
+        if (vec && p.state_is_fp32 && p.A_dstate_stride == 0 && 4LL * p.batch * p.nheads * p.dim * p.dstate >= kStreamBytes) {
+            go(ssm_update_kernel<LPR, true, true, false, true, true>);
+            return check_launch();
+        }
     }
     if (vec && LPR > 1 && p.A_dstate_stride == 0) {
         p.state_is_fp32 ? go(ssm_update_kernel<LPR, true, true, false, true>) : go(ssm_update_kernel<LPR, true, false, false, true>);
