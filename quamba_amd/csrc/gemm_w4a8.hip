@@ -611,8 +611,9 @@ int cheapest_way(const QaGemmW4A8Params& p, int cus, const SplitChoice& split, b
     if (split.shape >= 0) best.offer(kWaySplit, split.us);
     if (expandable) {
         // (the int8 x int8 kernel's own estimate up to a round of its 128 x 256 tiles, see there, with weights that come from the
-        // pass before: 777 x 2560 x 5120 takes 6.6 + 21.4 us; beyond, 3600 x 4096 x 1024 5.6 + 17.8, 26.0 in 128 x 128 tiles, 8800 x 3072
-        // x 768 5.5 + 26.3 and 33.9)
+        // pass before: 777 x 2560 x 5120 takes 6.6 + 21.4 us; a round of 192 x 128 there against one here 2000 x 2560 x 5120 36.4 and 39.1,
+        // 2500 x 2048 x 4096 29.1 and 32.1, 3300 x 1536 x 3072 23.5 and 25.4; beyond, 3600 x 4096 x 1024 5.6 + 17.8, 26.0 in 128 x 128 tiles,
+        // 8800 x 3072 x 768 5.5 + 26.3 and 33.9)
         const double rounds = static_cast<double>((tiles_of(p, 256, 256) + cus - 1) / cus);
         const double w8 = tiles_of(p, 128, 256) <= cus ? tiles_us_w8(p.m, p.n, p.k, cus) + 0.6 : 2.4 + 1.55 * rounds * (p.k / 128);
         best.offer(kWayExpandOnce, 5.1 + static_cast<double>(p.n) * p.k / 3.1e6 + w8);

@@ -219,7 +219,7 @@ GemvParams as_gemv(const QaGemmW8A8Params& p) {
 
 // Tile of a launch: the smallest whose tiles fit the part in one round.  With at most one tile per CU a launch takes a
 // tile's own time - about 2.5 us and, per 128 bytes of K, 0.20 us (64 x 64), 0.31 (128 x 64), 0.48 (128 x 128, four stages),
-// 0.68 (128 x 256), 1.15 (256 x 256) - so smaller tiles win until a second round starts; below that K split over the waves
+// 0.58 (192 x 128), 0.68 (128 x 256), 1.15 (256 x 256) - so smaller tiles win until a second round starts; below that K split over the waves
 // (gemm_split.hpp) where its cost is the smaller one.  Measured at M 16 .. 16384 with ten of the projections' N and K: this choice is the fastest or
 // within 8 % of it.  Against 128 x 128 tiles up to 192 tiles of 256 x 256 (rows x outputs x K, us): 512 x 1536 x 3072 14.6 ->
 // 7.7, 777 x 10240 x 2560 45 -> 38, 6144 x 1536 x 3072 47 -> 35.
@@ -247,6 +247,10 @@ int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
         if (p.n <= kNarrow && p.k >= 1024 && p.k % kBK == 0) return launch_gemm<2, 1, 2, 4, 4, false, true>(p, stream);
         return launch_gemm<2, 1, 2, 4, 4, false>(p, stream);
     }
+    // (between the two a tile's time goes with its area, and a round of 192 x 128 is three quarters of one of 128 x 256: 1536 x 4096 x 1024
+    // 10.3 -> 8.9 us, 777 x 6144 x 1536 15.9 -> 11.6, 768 x 8192 x 2048 19.7 -> 14.5, 2304 x 2560 x 5120 30 - 40 -> 27 - 34 with operands in the
+    // last-level cache and from memory)
+    if (tiles(192, 128) <= cus) return launch_gemm<3, 1, 2, 4, 3, false>(p, stream);
     if (tiles(128, 256) <= cus) return launch_gemm<2, 2, 2, 4, 3, false>(p, stream);
     // More than a round: what counts is rounds times the tile's work, 128 x 256 at six fifths of its share and the 320-wide
     // ones at 24/25: they move a tenth less per product through the caches, which at the power limit is time (against
@@ -271,7 +275,7 @@ int dispatch_tiles(const QaGemmW8A8Params& p, hipStream_t stream) {
 
 float tiles_us_w8(int m, int n, int k, int cus) {
     auto fits = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn) <= cus; };
-    return 2.5f + static_cast<float>((k + gemm::kBK - 1) / gemm::kBK) * (fits(64, 64) ? 0.20f : fits(128, 64) ? 0.31f : fits(128, 128) ? 0.48f : fits(128, 256) ? 0.68f : 1.15f);
+    return 2.5f + static_cast<float>((k + gemm::kBK - 1) / gemm::kBK) * (fits(64, 64) ? 0.20f : fits(128, 64) ? 0.31f : fits(128, 128) ? 0.48f : fits(192, 128) ? 0.58f : fits(128, 256) ? 0.68f : 1.15f);
 }
 
 }  // namespace qa

@@ -21,7 +21,7 @@ SPLIT_INT8 = [((9, 5, 16), "16, 16, 2"), ((9, 3071, 96), "16, 16, 2"), ((300, 10
               ((17, 18003, 2064), "32, 80, 1"), ((71, 9001, 5136), "64, 80, 1")]
 TILES_INT8 = [((300, 3000, 16), "1, 1, 2, 2, 4", False), ((600, 1000, 528), "1, 1, 2, 2, 4", False), ((900, 1200, 400), "1, 1, 4, 2, 4", False),
               ((1500, 2500, 656), "2, 1, 2, 4, 4", False), ((61, 18500, 2064), "2, 1, 2, 4, 4", False), ((11000, 130, 1152), "2, 1, 2, 4, 4", True),
-              ((1500, 5000, 528), "2, 2, 2, 4, 3", False),
+              ((1100, 5000, 528), "3, 1, 2, 4, 3", False), ((770, 6001, 16), "3, 1, 2, 4, 3", False), ((1500, 5000, 528), "2, 2, 2, 4, 3", False),
               ((4090, 5100, 528), "2, 5, 4, 2, 2", False), ((4090, 5100, 3200), "2, 5, 4, 2, 2", True), ((5100, 4090, 528), "5, 2, 2, 4, 2", False),
               ((5100, 4090, 3200), "5, 2, 2, 4, 2", True), ((4090, 4090, 528), "4, 2, 2, 4, 2", False), ((4090, 4080, 3200), "4, 2, 2, 4, 2", True)]
 GEMV_INT8 = [((m, n, k), f"{m + (m == 3)}, {waves}") for m in (1, 2, 3, 4) for n, k, waves in ((201, 1040, 1), (4002, 1552, 4), (5003, 2064, 2), (201, 8336, 4))]
