@@ -8,15 +8,28 @@
 
 namespace qa {
 
+// The tree v += v of lane ^ 32, ^ 16, ... ^ 1, and the same of maxima, in registers: six exchanges through LDS are six trips of
+// a hundred cycles.  (From lane ^ 8 on the sums repeat every eight lanes: a turn by four is lane ^ 4.)
+template <int CTRL>
+__device__ __forceinline__ float of_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <class Op>
+__device__ __forceinline__ float wave_tree(float v, Op op) {
+    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
+    v = op(v, of_lane<0x128>(v));
+    v = op(v, of_lane<0x124>(v));
+    v = op(v, of_lane<0x4e>(v));
+    return op(v, of_lane<0xb1>(v));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
-    return v;
+    return wave_tree(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m));
-    return v;
+    return wave_tree(v, [](float a, float b) { return fmaxf(a, b); });
 }
 __device__ __forceinline__ float silu_of(float z) { return z * (1.0f / (1.0f + expf(-z))); }
 
