@@ -18,63 +18,115 @@
 #include "conv2_common.hpp"
 #include "mixer_common.hpp"
 
+#include <type_traits>
+
 namespace qa {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kBatchLoads = 8;    // loads in flight per lane
+
+// What a lane takes of the channels' operands is requested in one straight run behind the inputs: where ways with and without
+// loads meet the compiler waits for every load in flight, the inputs among them, and the look-up of an output scale - the
+// head's group, the channel's group in it, their scale - was three trips to memory one after the other.  Now a wave requests the whole
+// table and looks it up across its lanes.  Bound by vector issue (some 55 instructions for four outputs, of which the exponential and the
+// reciprocal are a third) and, in short runs, by that set-up.  In a layer, us before and after: one scale 1 x 512 x 1536
+// channels 5.2 -> 4.6, 1 x 777 x 3072 6.0 -> 5.2, 3 x 1021 x 5120 15.6 -> 13.8, 8 x 2048 x 5120 51 -> 48; tables 1 x 500 x 5376 7.4 -> 6.6, 3 x 1000 x
+// 2304 12.3 -> 9.8, 1 x 1531 x 5376 12.5 -> 11.6, 4 x 4096 x 5376 51 -> 48.  (One copy of the exact route in a loop over a lane's outputs
+// instead of four, a third of the code: 48.4 -> 53.6.)
+enum ScaleKind { kOneScale, kTables, kWalk };
 
 // grid: x = blocks of 256 channels, y = blocks of 4 runs of `run` steps (one run per wave), z = batch
-template <bool SILU>
-__global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, int run, int packed) {
+// PACKED: four taps a channel, back to back: the lane's taps are one 16-byte piece, its biases one word.  SCALES kOneScale: one
+// output scale for all (the Mamba1 conv); kTables: up to 8 x 8 of an ssd group, whose channels are whole waves; kWalk: anything.
+// BATCH: loads in flight per lane.
+template <bool SILU, bool PACKED, ScaleKind SCALES, int BATCH>
+__global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, int run) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));   // the same in every lane: the step
                                                                                           // counters below stay in scalar registers
-    const int ch0 = (blockIdx.x * 64 + lane) * 4;
+    const int wave_ch = blockIdx.x * 256, ch0 = wave_ch + lane * 4;
     const int b = blockIdx.z;
     const int t0 = (blockIdx.y * 4 + wave) * run;
-    if (ch0 >= p.dim || t0 >= p.seqlen) return;
+    if (t0 >= p.seqlen || (SCALES != kTables && ch0 >= p.dim)) return;
     const int t_end = min(t0 + run, p.seqlen);
+    // (the tables are looked up by the whole wave: lanes past the last channel take that one's operands and store nothing)
+    const int ch = SCALES == kTables ? min(ch0, p.dim - 4) : ch0;
 
-    // The inputs are requested first: the walk over the group ranges below (dependent loads, four channels) then runs
-    // under their round trip instead of in front of it.
-    const int8_t* src = p.xBC + b * p.xBC_batch_stride + ch0;
+    // uniform row addresses and one offset per lane: the address arithmetic stays in scalar registers
+    const int8_t* const src = p.xBC + b * p.xBC_batch_stride;
+    const uint32_t at_ch = static_cast<uint32_t>(ch);
+    auto input = [&](int t) {
+        int64_t row = t * p.xBC_l_stride;
+        asm("" : "+s"(row));                                  // (the compiler would add the lane's offset first, and multiply in vector registers)
+        return *reinterpret_cast<const uint32_t*>(src + row + at_ch);
+    };
     uint32_t hist[3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const int t = t0 - 3 + i;
-        hist[i] = *reinterpret_cast<const uint32_t*>(src + max(t, 0) * p.xBC_l_stride);
-    }
+    for (int i = 0; i < 3; ++i) hist[i] = input(max(t0 - 3 + i, 0));
     // the loads of the next batch of steps are in flight while the current batch is worked on
-    uint32_t d[kBatchLoads], dn[kBatchLoads];
-    auto fetch = [&](int tb, uint32_t (&dst)[kBatchLoads]) {
+    uint32_t d[BATCH], dn[BATCH];
+    auto fetch = [&](int tb, uint32_t (&dst)[BATCH]) {
 #pragma unroll
-        for (int i = 0; i < kBatchLoads; ++i) {
-            const int t = min(tb + i, p.seqlen - 1);              // in range for every lane; steps past the end are never used
-            dst[i] = *reinterpret_cast<const uint32_t*>(src + t * p.xBC_l_stride);
-        }
+        for (int i = 0; i < BATCH; ++i) dst[i] = input(min(tb + i, p.seqlen - 1));      // in range for every lane; steps past the end are never used
     };
     fetch(t0, dn);
 
-    const Part part = part_of(p, ch0);          // the four channels of a lane never straddle two parts
-    uint32_t taps[4];
-    float bias_f[4], s_out[4], inv_s_out[4];
-    bool exact_only[4];
-    if (packed) {
-        // four taps a channel, back to back: the lane's taps are one 16-byte piece, its biases one word
-        const uint4 w = *reinterpret_cast<const uint4*>(p.weight + ch0 * 4);
+    const Part part = part_of(p, ch);          // the four channels of a lane never straddle two parts
+    uint32_t taps[4], bias4 = 0u;
+    if constexpr (PACKED) {
+        const uint4 w = *reinterpret_cast<const uint4*>(p.weight + ch * 4);
+        bias4 = *reinterpret_cast<const uint32_t*>(p.bias ? p.bias + ch : p.weight);
         taps[0] = w.x; taps[1] = w.y; taps[2] = w.z; taps[3] = w.w;
-        const uint32_t b4 = p.bias ? *reinterpret_cast<const uint32_t*>(p.bias + ch0) : 0u;
+    }
+    float s_out[4], inv_s_out[4], table = 0.0f, own = 0.0f;
+    int head_end = 0, dim_end = 0;
+    if constexpr (SCALES == kTables) {
+        // lane 8 h + d: head group h, group d of its channels; the table is that of the wave's first channel
+        const int g = p.n_groups > 1 && wave_ch < p.x_dim ? wave_ch / (p.x_dim / p.n_groups) : 0;
+        const int entry = (g * p.nhead_groups + min(lane >> 3, p.nhead_groups - 1)) * p.ndim_groups + min(lane & 7, p.ndim_groups - 1);
+        table = p.x_out_scales[entry];
+        dim_end = p.x_dim_group_range[entry];
+        head_end = p.x_head_group_range[g * p.nhead_groups + min(lane & 7, p.nhead_groups - 1)];
+        const float* const group = part.index == 0 ? p.x_out_scales : part.index == 1 ? p.B_out_scales : p.C_out_scales;
+        own = group[part.index == 0 || p.n_groups == 1 ? 0 : (ch - part.offset) / p.d_state];
+    }
+    if constexpr (SCALES != kWalk) __builtin_amdgcn_sched_barrier(0);
+    float bias_f[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) bias_f[e] = part.s_bias * static_cast<float>(static_cast<int8_t>(b4 >> (8 * e)));
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            taps[e] = pack_taps(p.weight + (ch0 + e) * p.weight_c_stride, p.weight_width_stride, p.width);
-            bias_f[e] = p.bias ? part.s_bias * static_cast<float>(p.bias[ch0 + e]) : 0.0f;
+    for (int e = 0; e < 4; ++e) {
+        if constexpr (PACKED) {
+            bias_f[e] = p.bias ? part.s_bias * static_cast<float>(static_cast<int8_t>(bias4 >> (8 * e))) : 0.0f;
+        } else {
+            taps[e] = pack_taps(p.weight + (ch + e) * p.weight_c_stride, p.weight_width_stride, p.width);
+            bias_f[e] = p.bias ? part.s_bias * static_cast<float>(p.bias[ch + e]) : 0.0f;
         }
     }
-    out_scales4_of(p, part, ch0, s_out);
+    if constexpr (SCALES == kOneScale) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s_out[e] = p.x_out_scale;
+    } else if constexpr (SCALES == kTables) {
+        // (a wave begins a head or lies in one: 256 channels are whole heads of 4 .. 256, a power of two)
+        const int shift = __builtin_ctz(p.x_headdim), in_group = p.n_groups > 1 ? wave_ch % (p.x_dim / p.n_groups) : wave_ch;
+        const int head = (in_group + lane * 4) >> shift, first = (lane * 4) & (p.x_headdim - 1);
+        int hg = 0, dg[4] = {};
+#pragma unroll
+        for (int j = 0; j < 7; ++j) hg += static_cast<int>(j < p.nhead_groups - 1) & static_cast<int>(head >= __builtin_amdgcn_readlane(head_end, j));
+#pragma unroll
+        for (int j = 0; j < 7; ++j) {
+            const int end = __builtin_amdgcn_ds_bpermute(4 * (8 * hg + j), dim_end);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dg[e] += static_cast<int>(j < p.ndim_groups - 1) & static_cast<int>(first + e >= end);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float s = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (8 * hg + dg[e]), __float_as_int(table)));
+            s_out[e] = part.index == 0 ? s : own;
+        }
+        if (ch0 >= p.dim) return;
+    } else {
+        out_scales4_of(p, part, ch, s_out);
+    }
+    bool exact_only[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         inv_s_out[e] = 1.0f / s_out[e];
@@ -84,6 +136,7 @@ __global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, in
     int64_t out_ls, out_cs;
     int8_t* out = out_ptr(p, part, b, ch0, &out_ls, &out_cs);
 
+    const int dot_magic = dot4_magic();
     // byte j of win[e] holds x[t-3+j] of channel ch0+e
     uint32_t win[4] = {0u, 0u, 0u, 0u};
     auto push = [&](uint32_t d) {
@@ -96,17 +149,17 @@ __global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, in
     for (int i = 0; i < 3; ++i) push(t0 - 3 + i >= 0 ? hist[i] : 0u);
     int8_t* out_at = out + t0 * out_ls;             // walks on by one step's stride (the stride differs from lane to lane: a
                                                     // product per step would be a 64-bit multiplication in vector registers)
-    for (int tb = t0; tb < t_end; tb += kBatchLoads) {
+    for (int tb = t0; tb < t_end; tb += BATCH) {
 #pragma unroll
-        for (int i = 0; i < kBatchLoads; ++i) d[i] = dn[i];
-        if (tb + kBatchLoads < t_end) fetch(tb + kBatchLoads, dn);
+        for (int i = 0; i < BATCH; ++i) d[i] = dn[i];
+        if (tb + BATCH < t_end) fetch(tb + BATCH, dn);
 #pragma unroll
-        for (int i = 0; i < kBatchLoads; ++i) {
+        for (int i = 0; i < BATCH; ++i) {
             if (tb + i >= t_end) break;
             push(d[i]);
             float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(part.s_in, static_cast<float>(dot4(win[e], taps[e])), bias_f[e]);
+            for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(part.s_in, dot4_float(win[e], taps[e], dot_magic), bias_f[e]);
             *reinterpret_cast<uint32_t*>(out_at) = conv_quant4(v, s_out, inv_s_out, SILU, exact_only, kq);
             out_at += out_ls;
         }
@@ -117,7 +170,7 @@ __global__ __launch_bounds__(kThreads) void conv2_fwd_kernel(QaConv2Params p, in
         const bool words = p.conv_state_c_stride == 1 && (reinterpret_cast<uintptr_t>(st) & 3u) == 0 && p.conv_state_l_stride % 4 == 0;
         for (int i = 0; i < p.conv_state_len; ++i) {
             const int t = p.seqlen - p.conv_state_len + i;
-            const uint32_t v = t >= 0 ? *reinterpret_cast<const uint32_t*>(src + t * p.xBC_l_stride) : 0u;
+            const uint32_t v = t >= 0 ? input(t) : 0u;
             if (words) {
                 *reinterpret_cast<uint32_t*>(st + i * p.conv_state_l_stride) = v;
             } else {
@@ -266,18 +319,24 @@ int validate(const QaConv2Params* p, bool update) {
 
 namespace qa {
 int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
-    // Steps per wave: 4 to 256, whichever takes the busiest SIMD's waves the shortest: in ns about 145 a step and 250 for a
-    // wave's set-up (taps, scales, the three inputs ahead), and 160 a step of the last wave with nobody beside it.  Measured
-    // with runs of 4, 8, 16, 32, 64 steps, us: 1 x 512 x 1536 channels 5.5, 6.7, 8.2, 11.1, 17.4; 1 x 777 x 3072 5.9, 6.5, 8.1, 11.4, 18.2;
-    // 1 x 1531 x 5376 14.6, 12.6, 13.1, 14.4, 20.7; 4 x 1299 x 1920 11.2, 11.2, 12.2, 14.5, 18.8; 4 x 4096 x 5376 87.7, 64.4, 57.0, 56.5, 60.8;
-    // 16 x 1024 x 10240 164, 118, 99, 95, 95.  Two and three taps, which come byte by byte: 350 and 100.  Over 148 sizes of each the choice
-    // is 0.2 % behind the best run and 0.3 with fewer taps (0.9 with their figures for four taps as well).
+    const bool packed = p.width == 4 && p.weight_width_stride == 1 && p.weight_c_stride == 4 && aligned16(p.weight) && aligned4(p.bias);
+    const bool one_scale = packed && !p.x_out_scales;
+    const bool tables = packed && p.x_out_scales && p.x_head_group_range && p.x_dim_group_range && p.nhead_groups <= 8 && p.ndim_groups <= 8 && p.x_headdim % 4 == 0 &&
+                        256 % p.x_headdim == 0 && p.d_state % 4 == 0 && (p.n_groups == 1 || p.x_dim / p.n_groups % 256 == 0) && p.x_dim > 0 && p.B_out_scales && p.C_out_scales;
+    // Steps per wave: 4 to 256, whichever takes the busiest SIMD's waves the shortest: in ns about 145 a step and for a wave's
+    // set-up (taps, scales, the three inputs ahead) 100 with one output scale and 400 with tables, and 160 a step of the last wave with
+    // nobody beside it.  Measured in a layer with runs of 4, 6, 8, 12, 16, 24, 32 steps, us: one scale 1 x 512 x 1536 channels 4.6, 4.6, 5.4, 5.8,
+    // 6.9, 8.1, 10.0; 3 x 1021 x 5120 13.4, 14.0, 14.9, 16.0, 15.6, 16.3, 16.0; 4 x 1500 x 2048 11.8, 12.1, 11.7, 12.4, 12.4, 12.7, 14.7; tables 1 x 1531 x
+    // 5376 11.8, 12.0, 11.6, 12.2, 11.6, 13.9, 14.6; 3 x 1000 x 2304 10.0, 9.8, 10.4, 10.8, 10.5, 12.5, 12.5; 4 x 4096 x 5376 62, 54, 52, 51, 49, 50, 50.  The
+    // choice is at most 4 % behind the best run.  Anything else: 250, and two and three taps, which come byte by byte, 350 and 100 a step (over
+    // 148 sizes of each the choice is 0.2 % behind the best power of two and 0.3 with fewer taps).
     int run = 4;
     {
         const int64_t ch_blocks = (p.dim + 255) / 256, simds = 4LL * compute_units();
-        const int set_up = p.width == 4 ? 250 : 350, alone = p.width == 4 ? 160 : 100;
+        const int set_up = one_scale ? 100 : tables ? 400 : p.width == 4 ? 250 : 350, alone = p.width == 4 ? 160 : 100;
         int64_t best = -1;
-        for (int r = 4; r <= 256; r *= 2) {
+        for (int r : {4, 6, 8, 12, 16, 24, 32, 48, 64, 128, 256}) {
+            if (!one_scale && !tables && (r & (r - 1))) continue;
             const int64_t waves = ch_blocks * (((p.seqlen + r - 1) / r + 3) / 4 * 4) * p.batch;
             const int64_t cost = (waves + simds - 1) / simds * (145 * r + set_up) + alone * r;
             if (best < 0 || cost < best || (p.seqlen + 4LL * run - 1) / (4 * run) > 65535) { best = cost; run = r; }
@@ -286,9 +345,22 @@ int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
     const int64_t run_blocks = (p.seqlen + 4 * run - 1) / (4 * run);
     if (run_blocks > 65535) return QA_ERR_SHAPE;
     dim3 grid((p.dim + 255) / 256, static_cast<unsigned>(run_blocks), p.batch);
-    const int packed = p.width == 4 && p.weight_width_stride == 1 && p.weight_c_stride == 4 && aligned16(p.weight) && aligned4(p.bias);
-    if (p.silu_activation) hipLaunchKernelGGL(conv2_fwd_kernel<true>, grid, dim3(kThreads), 0, stream, p, run, packed);
-    else hipLaunchKernelGGL(conv2_fwd_kernel<false>, grid, dim3(kThreads), 0, stream, p, run, packed);
+    auto with = [&](auto silu_c) {
+        constexpr bool kSilu = decltype(silu_c)::value;
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, p, run); };
+        auto by_run = [&](auto scales_c) {
+            constexpr ScaleKind kScales = decltype(scales_c)::value;
+            if (run == 4) go(conv2_fwd_kernel<kSilu, true, kScales, 4>);
+            else if (run == 6) go(conv2_fwd_kernel<kSilu, true, kScales, 6>);
+            else go(conv2_fwd_kernel<kSilu, true, kScales, 8>);
+        };
+        if (one_scale) by_run(std::integral_constant<ScaleKind, kOneScale>{});
+        else if (tables) by_run(std::integral_constant<ScaleKind, kTables>{});
+        else if (packed) go(conv2_fwd_kernel<kSilu, true, kWalk, 8>);
+        else go(conv2_fwd_kernel<kSilu, false, kWalk, 8>);
+    };
+    if (p.silu_activation) with(std::true_type{});
+    else with(std::false_type{});
     return check_launch();
 }
 }  // namespace qa
