@@ -553,9 +553,17 @@ TmPlan plan_of(const QaSScanParams& p) {
         r.lanes = 8;
         TmPlan chosen = r;
         if (p.segments == 0 && over_waves.ns < kScanWavesNever) {
-            best = over_waves.ns;
-            chosen.lanes = over_waves.lanes;
-            chosen.waves = over_waves.waves;
+            // one pass of eight lanes, in tiles of 32 steps, with one, two or three waves to a SIMD (within 5 % of it in 200 sizes of 16 ... 220
+            // steps): the shorter one for a tile or less (2 x 31 x 3072 5.6 us and 7.2, 1 x 31 x 5120 6.2 and 7.5) and behind a tile's
+            // beginning where the workgroups of the other are two or three to a CU (2 x 150 x 3072 13.4 and 14.4, 8 x 80 x 1536 12.7 and 14.4)
+            static constexpr int kStart[3] = {3450, 4150, 4800}, kTile[3] = {1950, 2850, 4400};
+            const int64_t w = std::min<int64_t>(per_simd(wave_rows8 * p.batch), 3) - 1;
+            best = kStart[w] + static_cast<int64_t>((p.seqlen + 31) / 32) * kTile[w];
+            if (over_waves.ns < best) {
+                best = over_waves.ns;
+                chosen.lanes = over_waves.lanes;
+                chosen.waves = over_waves.waves;
+            }
         }
         for (int n = 2; n <= 32 && 64 * n <= p.seqlen; ++n) {
             cut(n);

@@ -415,20 +415,20 @@ int sscan_waves_fwd(const QaSScanParams& p, const SscanDtProj* dt, int lanes, in
 // up; 956 launches of 1 ... 8 prompts of 16 ... 4096 steps x 512 ... 5120 channels lie within 6 % of this (rms), and the choice is the
 // fastest launch or within 3 % of it in all of them.  While workgroups are no more than a SIMD has room for (three waves of these
 // registers, four of sixteen-wave workgroups) nothing waits for a place; beyond, the one pass of sscan_tm.hip is the shorter one
-// (3 x 1021 x 5120 106 us against 102, 8 x 512 x 2048 56 and 52), as it is for a handful of steps on more than one workgroup
-// per CU (1 x 16 x 5120 6.8 and 5.8).
+// (3 x 1021 x 5120 106 us against 102, 8 x 512 x 2048 56 and 52), as it is for some short prompts (plan_of there).
 ScanWavesPlan scan_waves_plan(const QaSScanParams& p, int cus) {
     const auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
     ScanWavesPlan best = {4, 1, kScanWavesNever};
-    const bool short_one = p.seqlen <= WavesCfg<4>::T && up(p.dim, WavesCfg<4>::kCh) * p.batch > cus;
     for (const int lanes : {4, 8}) {
         const int64_t steps = lanes == 4 ? WavesCfg<4>::T : WavesCfg<8>::T, channels = lanes == 4 ? WavesCfg<4>::kCh : WavesCfg<8>::kCh;
         const int64_t per_cu = up(up(p.dim, channels) * p.batch, cus), pieces = up(p.seqlen, steps);
         for (int w = 1; w <= std::min<int64_t>(max_waves(lanes), pieces); ++w) {
             const int64_t per_simd = per_cu * up(w, 4), blocks = up(pieces, w);
             // (workgroups of other sizes share SIMDs unevenly)
-            if (short_one || per_simd > (w <= 12 ? 3 : 4) || (per_cu > 1 && w % 4 != 0 && blocks > 1)) continue;
-            const int64_t ns = 3590 + blocks * (lanes == 4 ? 1020 + 1030 * per_simd + 50 * w : 1550 + 1300 * per_simd + 40 * w);
+            if (per_simd > (w <= 12 ? 3 : 4) || (per_cu > 1 && w % 4 != 0 && blocks > 1)) continue;
+            // (three workgroups on a CU begin out of step with each other)
+            const int64_t crowd = lanes == 4 && per_cu > 2 ? 1300 + 700 * std::min<int64_t>(blocks - 1, 2) : 0;
+            const int64_t ns = 3590 + crowd + blocks * (lanes == 4 ? 1020 + 1030 * per_simd + 50 * w : 1550 + 1300 * per_simd + 40 * w);
             if (ns < best.ns) best = {lanes, w, ns};
         }
     }
