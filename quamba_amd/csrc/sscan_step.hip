@@ -59,7 +59,17 @@ __global__ __launch_bounds__(kThreads) void mamba1_step_kernel(StepArgs p) {
     StepSmem<NB>& sm = smem[wave];
     float(*const bc)[2][16] = bc_all[wave];
 
-    // the projection's operands first: everything else is needed behind them
+    // the states first, most of the bytes, then the projection's operands, behind which everything else is needed (the states last: a step of
+    // 32 x 3072 fp32 0.3 us longer in a layer's 23.7, of 64 x 4096 0.6 in 29.9, of 16 x 3072 int8 0.3 in 22.4)
+    const int64_t at = static_cast<int64_t>(c) * 16 + 4 * slice;
+    float4 st32[FP32 ? NB : 1];
+    uint32_t st8[FP32 ? 1 : NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int64_t e = entry(b) * p.state_batch_stride + at;
+        if constexpr (FP32) st32[b] = *reinterpret_cast<const float4*>(static_cast<const float*>(p.state) + e);
+        else st8[b] = *reinterpret_cast<const uint32_t*>(static_cast<const int8_t*>(p.state) + e);
+    }
     v4u rw[3], rx;
     const v4u* w = reinterpret_cast<const v4u*>(p.w + static_cast<int64_t>(c0) * (16 * p.pieces));
 #pragma unroll
@@ -77,15 +87,6 @@ __global__ __launch_bounds__(kThreads) void mamba1_step_kernel(StepArgs p) {
     const uint32_t A_codes = *reinterpret_cast<const uint32_t*>(p.A_log + static_cast<int64_t>(c) * p.A_dim_stride + 4 * slice);
     const float dt_row = p.use_alpha ? p.alpha : *p.row_scale;
     const float dt_col = p.use_alpha ? 1.0f : p.col_scale[p.one_col_scale ? 0 : c0 + (lane & 15)];
-    const int64_t at = static_cast<int64_t>(c) * 16 + 4 * slice;
-    float4 st32[FP32 ? NB : 1];
-    uint32_t st8[FP32 ? 1 : NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const int64_t e = entry(b) * p.state_batch_stride + at;
-        if constexpr (FP32) st32[b] = *reinterpret_cast<const float4*>(static_cast<const float*>(p.state) + e);
-        else st8[b] = *reinterpret_cast<const uint32_t*>(static_cast<const int8_t*>(p.state) + e);
-    }
     const float x_scale = *p.x_scale, dt_scale = *p.dt_scale, A_scale = *p.A_log_scale, B_scale = *p.B_scale, C_scale = *p.C_scale;
     const float bias_scale = p.dt_bias ? *p.dt_bias_scale : 0.0f, D_scale = p.D ? *p.D_scale : 0.0f, z_scale = p.z ? *p.z_scale : 0.0f;
     const float s_state = FP32 ? 0.0f : *p.state_scale;
