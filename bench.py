@@ -641,7 +641,7 @@ def valu_calibration(dev, ops_list=None, launches=4):
 # so (`stale`) instead of passing them off as current.
 SCAN_MIX = {"four_lane": {"plain": 96, "transcendental": 18}, "eight_lane": {"plain": 57, "transcendental": 9}}
 SCAN_MIX_SOURCES = ("sscan.hip", "sscan_common.hpp")
-SCAN_MIX_FINGERPRINT = "c65ca4fd126144d0"
+SCAN_MIX_FINGERPRINT = "ea59dd4b0bcca656"
 
 
 def source_fingerprint(names, root=os.path.join(ROOT, "quamba_amd", "csrc")):
