@@ -195,8 +195,9 @@ __device__ __forceinline__ XShare<CH> load_x_share(const int8_t* from) {
     }
     return r;
 }
-template <int XP, int CH>
-__device__ __forceinline__ void stage_x_share(_Float16 (*xt)[XP], const XShare<CH> (&xr)[4], const float* xs, int c0, int kb) {
+// `put(row, v)`: the four steps of a row of that tile
+template <int CH, class Put>
+__device__ __forceinline__ void stage_x_share(const XShare<CH> (&xr)[4], const float* xs, int c0, Put&& put) {
 #pragma unroll
     for (int d = 0; d < CH / 4; ++d) {
         const float4 s4 = *reinterpret_cast<const float4*>(xs + c0 + 4 * d);
@@ -209,7 +210,7 @@ __device__ __forceinline__ void stage_x_share(_Float16 (*xt)[XP], const XShare<C
             v[1] = rounded(__builtin_fmaf(ubyte_of(w1, cc), sc, nsc));
             v[2] = rounded(__builtin_fmaf(ubyte_of(w2, cc), sc, nsc));
             v[3] = rounded(__builtin_fmaf(ubyte_of(w3, cc), sc, nsc));
-            *reinterpret_cast<v4h*>(&xt[cc * 16 + c0 / 4 + d][kb * 4]) = v;              // row slot(c0 + 4 d + cc)
+            put(cc * 16 + c0 / 4 + d, v);                                                // row slot(c0 + 4 d + cc)
         }
     }
 }
@@ -235,21 +236,31 @@ __device__ __forceinline__ void unit_head_part(int linear, int units, int hpg, i
 // (64 x N of headdim x dstate, fp32) in registers; the fp32 chunk states never travel
 // through memory.  A wave owns 16 columns n and all rows p.  Its B operand, f16((s_B q_B[k,n]) w_k) with the
 // per-head weight w_k = exp(dA_last - dA_k) dt_k, is built in registers from the transposed int8 B tile in LDS
-// (rows n of 4-byte-aligned pitch with an odd number of dwords: conflict-free for the transposing dword stores
-// and for the operand reads); its A operand is the transposed x tile.  The tiles of chunk c+1 are fetched into
+// (8-byte reads); its A operand is the transposed x tile; both tiles are laid out so that neither the transposing stores nor the operand
+// reads meet on a bank.  The tiles of chunk c+1 are fetched into
 // registers while chunk c is multiplied.  The state entering chunk c >= 1 is stored as fp16, rows in slot order.
 // Bound by vector issue (converting x and B to fp16 operands) and by the LDS reads of the x tile, which every wave makes: with
-// one workgroup for all N columns x is staged once: as a workgroup per 64 columns 16 x 1024 steps of 128 heads took 146 us, now
-// 129.  (Four waves of 32 columns instead of eight of 16 read x half as often and take 138: too few waves for the latencies
+// one workgroup for all N columns x is staged once: as a workgroup per 64 columns 16 x 1024 steps of 128 heads took 146 us, so
+// 129; with the tiles padded by a piece a row (half of the LDS's busy cycles were conflicts) 129 -> 124, 4 x 4096 steps of 80 heads 104 -> 97, 1531
+// steps 14.7 -> 13.4.  (Four waves of 32 columns instead of eight of 16 read x half as often and take 138: too few waves for the latencies
 // of a chunk.  With s_B in the weight, q_B (s_B w_k), a product less per value: 128, but at fp16 ties another value than the
 // reference's; the general kernels round the same one.)
 // ---------------------------------------------------------------------------------------------
 template <int N, int Q>
 struct StateSmem {
-    static constexpr int XP = Q + 8;        // halves per row of the transposed x tile
-    static constexpr int BP = Q + 4;        // bytes per row of the transposed B tile
-    __attribute__((aligned(16))) _Float16 xt[kP][XP];
-    __attribute__((aligned(16))) int8_t b8[N][BP];
+    // A 16-byte read takes lanes 0 .. 3, 12 .. 15 and 20 .. 27 together, the other half of those 32 next: rows 0 .. 3 and 12 .. 15 of one piece
+    // with rows 4 .. 11 of its neighbour.  Rows of x have no pad; their pieces are exchanged by the row, which keeps both halves apart
+    // (and the transposing stores).  Rows of B are shifted by eight words and by four more past the eighth.
+    static constexpr int BP = Q + 32;       // bytes per row of the transposed B tile
+    __attribute__((aligned(16))) _Float16 xt[kP * Q];
+    __attribute__((aligned(16))) int8_t b8[N * BP + N / 8 * 16];
+    static __device__ __forceinline__ int turn(int row) { return Q == 64 ? (row >> 1) & 7 : row & 15; }
+    static __device__ __forceinline__ int x_at(int row, int piece) { return row * Q + ((piece ^ turn(row)) << 3); }
+    // piece 4 ks + lq of a row from piece lq: exchanged within sixteen (eight) pieces, past those further on
+    static constexpr int kPieces = Q == 64 ? 8 : 16;
+    static constexpr int x_turned(int ks) { return 4 * ks % kPieces * 8; }
+    static constexpr int x_past(int ks) { return 4 * ks / kPieces * kPieces * 8; }
+    static __device__ __forceinline__ int b_at(int row, int k) { return row * BP + (row >> 3) * 16 + k; }
     __attribute__((aligned(16))) float w[Q];
     __attribute__((aligned(16))) float xs[kP];    // x scale per channel
     int32_t srow[kP];                             // the channel's row of the grouped state scales
@@ -333,7 +344,7 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
                 if (4 * bkb + r >= valid_loaded) br[r] = make_uint4(0u, 0u, 0u, 0u);
             }
         }
-        if (mine_x) stage_x_share<S::XP, CH>(sm.xt, xr, sm.xs, xc, xkb);
+        if (mine_x) stage_x_share<CH>(xr, sm.xs, xc, [&](int row, const v4h& v) { *reinterpret_cast<v4h*>(&sm.xt[S::x_at(row, xkb >> 1) + 4 * (xkb & 1)]) = v; });
         if (mine_b) {
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
@@ -344,10 +355,10 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
                 const uint32_t lo23 = __builtin_amdgcn_perm(r3, r2, 0x05010400u);
                 const uint32_t hi23 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
                 const int n4 = bc + 4 * d;
-                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 0][bkb * 4]) = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 1][bkb * 4]) = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 2][bkb * 4]) = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-                *reinterpret_cast<uint32_t*>(&sm.b8[n4 + 3][bkb * 4]) = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+                *reinterpret_cast<uint32_t*>(&sm.b8[S::b_at(n4 + 0, bkb * 4)]) = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+                *reinterpret_cast<uint32_t*>(&sm.b8[S::b_at(n4 + 1, bkb * 4)]) = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+                *reinterpret_cast<uint32_t*>(&sm.b8[S::b_at(n4 + 2, bkb * 4)]) = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+                *reinterpret_cast<uint32_t*>(&sm.b8[S::b_at(n4 + 3, bkb * 4)]) = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
             }
         }
         if (steps_made && tid < Q) sm.w[tid] = fexp(r_last - r_dA) * r_dt;   // weight of step k in the chunk's state
@@ -440,15 +451,17 @@ __global__ __launch_bounds__(4 * N, N == 128 ? 4 : 3) void ssd_state_kernel(QaSs
         v4f accs[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) accs[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        int x_first = S::x_at(l16, lq);
+        asm("" : "+v"(x_first));                                   // (four addresses kept over the chunks are four registers spilled)
 #pragma unroll
         for (int ks = 0; ks < Q / 32; ++ks) {
             const int k0 = 32 * ks + 8 * lq;
-            const uint32_t b0 = *reinterpret_cast<const uint32_t*>(&sm.b8[16 * wave + l16][k0]);
-            const uint32_t b1 = *reinterpret_cast<const uint32_t*>(&sm.b8[16 * wave + l16][k0 + 4]);
+            const uint2 b01 = *reinterpret_cast<const uint2*>(&sm.b8[S::b_at(16 * wave + l16, k0)]);
+            const uint32_t b0 = b01.x, b1 = b01.y;
             const float4 w0 = *reinterpret_cast<const float4*>(&sm.w[k0]), w1 = *reinterpret_cast<const float4*>(&sm.w[k0 + 4]);
             v8h fx[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) fx[j] = *reinterpret_cast<const v8h*>(&sm.xt[j * 16 + l16][k0]);
+            for (int j = 0; j < 4; ++j) fx[j] = *reinterpret_cast<const v8h*>(&sm.xt[(x_first ^ S::x_turned(ks)) + S::x_past(ks) + j * 16 * Q]);
             const float wk[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
             v8h bw;
 #pragma unroll
@@ -843,7 +856,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                     if (4 * kb + r >= lim) xr[r] = XShare<CH>{};
                 }
             }
-            stage_x_share<S::XP, CH>(sm.xt, xr, sm.xs, xc, kb);
+            stage_x_share<CH>(xr, sm.xs, xc, [&](int row, const v4h& v) { *reinterpret_cast<v4h*>(&sm.xt[row][kb * 4]) = v; });
         }
         __syncthreads();
 
