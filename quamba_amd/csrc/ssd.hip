@@ -195,6 +195,18 @@ __device__ __forceinline__ XShare<CH> load_x_share(const int8_t* from) {
     }
     return r;
 }
+// Where the transposed x tile of both kernels has its 16-byte pieces: rows without a pad, the pieces exchanged by the row, so that the
+// rows of an operand read (and of the transposing stores) fall into different banks.
+template <int Q>
+struct XPlaces {
+    static __device__ __forceinline__ int turn(int row) { return Q == 64 ? (row >> 1) & 7 : row & 15; }
+    static __device__ __forceinline__ int x_at(int row, int piece) { return row * Q + ((piece ^ turn(row)) << 3); }
+    // piece 4 ks + lq of a row from piece lq < 4: exchanged within sixteen (eight) pieces, past those further on
+    static constexpr int kPieces = Q == 64 ? 8 : 16;
+    static constexpr int x_turned(int ks) { return 4 * ks % kPieces * 8; }
+    static constexpr int x_past(int ks) { return 4 * ks / kPieces * kPieces * 8; }
+};
+
 // `put(row, v)`: the four steps of a row of that tile
 template <int CH, class Put>
 __device__ __forceinline__ void stage_x_share(const XShare<CH> (&xr)[4], const float* xs, int c0, Put&& put) {
@@ -247,19 +259,13 @@ __device__ __forceinline__ void unit_head_part(int linear, int units, int hpg, i
 // reference's; the general kernels round the same one.)
 // ---------------------------------------------------------------------------------------------
 template <int N, int Q>
-struct StateSmem {
+struct StateSmem : XPlaces<Q> {
     // A 16-byte read takes lanes 0 .. 3, 12 .. 15 and 20 .. 27 together, the other half of those 32 next: rows 0 .. 3 and 12 .. 15 of one piece
     // with rows 4 .. 11 of its neighbour.  Rows of x have no pad; their pieces are exchanged by the row, which keeps both halves apart
     // (and the transposing stores).  Rows of B are shifted by eight words and by four more past the eighth.
     static constexpr int BP = Q + 32;       // bytes per row of the transposed B tile
     __attribute__((aligned(16))) _Float16 xt[kP * Q];
     __attribute__((aligned(16))) int8_t b8[N * BP + N / 8 * 16];
-    static __device__ __forceinline__ int turn(int row) { return Q == 64 ? (row >> 1) & 7 : row & 15; }
-    static __device__ __forceinline__ int x_at(int row, int piece) { return row * Q + ((piece ^ turn(row)) << 3); }
-    // piece 4 ks + lq of a row from piece lq: exchanged within sixteen (eight) pieces, past those further on
-    static constexpr int kPieces = Q == 64 ? 8 : 16;
-    static constexpr int x_turned(int ks) { return 4 * ks % kPieces * 8; }
-    static constexpr int x_past(int ks) { return 4 * ks / kPieces * kPieces * 8; }
     static __device__ __forceinline__ int b_at(int row, int k) { return row * BP + (row >> 3) * 16 + k; }
     __attribute__((aligned(16))) float w[Q];
     __attribute__((aligned(16))) float xs[kP];    // x scale per channel
@@ -588,15 +594,14 @@ __global__ __launch_bounds__(256) void ssd_pass_kernel(QaSsdParams p, const floa
 // term 1 of both tiles runs first, x is staged from its registers after it.
 // ---------------------------------------------------------------------------------------------
 template <int N, int Q>
-struct ScanSmem {
-    static constexpr int XP = Q + 8;        // halves per row of the transposed x tile
+struct ScanSmem : XPlaces<Q> {
     static constexpr int NCH = N / 8;       // 16-byte pieces per row of the entering state
     static constexpr int SWZ = (NCH < 16 ? NCH : 16) - 1;
     static constexpr int BSWZ = (N / 16 < 8 ? N / 16 : 8) - 1;
     // of the head at hand; the entering state first, then x.  The state's rows have no padding: piece c of row r sits
     // at position c ^ (r & SWZ), so that the sixteen rows of an operand read fall into different banks
     union {
-        __attribute__((aligned(16))) _Float16 xt[kP][XP];
+        __attribute__((aligned(16))) _Float16 xt[kP * Q];
         __attribute__((aligned(16))) _Float16 prev[kP][N];
     };
     __attribute__((aligned(16))) int8_t bq[Q][N];   // B codes; 16-byte piece c of row k at position c ^ (k & BSWZ)
@@ -679,9 +684,14 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
     // merges the two sets of destination registers by copies right behind the loads, i.e. waits for them there.
     float r_dt = 0.0f, r_dA = 0.0f, r_xs = 0.0f, r_D = 0.0f;
     v4i r_prev[PB];
+    // A lane's two groups of steps of a 32-step piece, 4 q and 16 + 4 q, share 16 bytes of the x tile: one read instead of two of 8 bytes,
+    // and neighbouring threads store the two halves of a place.  (Against rows with a pad: 16 x 1024 steps of 128 heads 217 -> 209 us, 4 x
+    // 4096 of 80 135 -> 134; the layers of 1531, 2 x 700 and 300 steps 1 %.  With the exchange but two reads of 8 bytes, which no longer
+    // share an address: 228 and 144.)
+    auto steps_of = [](int t) { return (t & ~7) | (t & 1) << 2 | (t & 6) >> 1; };
     XShare<CH> xr[4];                                             // steps 4 kb .. 4 kb + 3, channels xc .. xc + 7
     auto fetch_head = [&](int h, int tid) {
-        const int xc = tid % (kP / CH) * CH, kb = tid / (kP / CH);
+        const int xc = tid % (kP / CH) * CH, kb = steps_of(tid / (kP / CH));
         const int hp = h / split, ch0 = (h % split) * kP;
         if (Q == kThreads || tid < Q) {
             const int64_t row = ((static_cast<int64_t>(b) * p.nheads + hp) * nc + c) * Q;
@@ -848,7 +858,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
         }
         __syncthreads();                                               // everyone is done with the entering state
         if (kShares == kThreads || tid < kShares) {
-            const int xc = tid % (kP / CH) * CH, kb = tid / (kP / CH);
+            const int xc = tid % (kP / CH) * CH, kb = steps_of(tid / (kP / CH));
             if (lim < Q) {
                 // ragged last chunk: steps past the end of the sequence count as zero
 #pragma unroll
@@ -856,7 +866,7 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                     if (4 * kb + r >= lim) xr[r] = XShare<CH>{};
                 }
             }
-            stage_x_share<CH>(xr, sm.xs, xc, [&](int row, const v4h& v) { *reinterpret_cast<v4h*>(&sm.xt[row][kb * 4]) = v; });
+            stage_x_share<CH>(xr, sm.xs, xc, [&](int row, const v4h& v) { *reinterpret_cast<v4h*>(&sm.xt[S::x_at(row, (kb >> 1 & ~3) + (kb & 3)) + (kb & 4)]) = v; });
         }
         __syncthreads();
 
@@ -892,15 +902,15 @@ __global__ __launch_bounds__(64 * scan_waves_of(Q), 4) void ssd_chunk_scan_kerne
                 return cb;
             };
             // the weights of steps 32 ks + 4 q .. + 3 and 32 ks + 16 + 4 q .. + 3 times x
+            const int x_first = S::x_at(l16, lq);
             auto times_x = [&](int ks, const float (&wv)[8]) {
                 v8h fl;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) fl[e] = rounded(wv[e]);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const v4h x0 = *reinterpret_cast<const v4h*>(&sm.xt[j * 16 + l16][32 * ks + 4 * lq]);
-                    const v4h x1 = *reinterpret_cast<const v4h*>(&sm.xt[j * 16 + l16][32 * ks + 4 * lq + 16]);
-                    acc[s][j] = mfma16(fl, v8h{x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, acc[s][j]);
+                    const v8h fx = *reinterpret_cast<const v8h*>(&sm.xt[(x_first ^ S::x_turned(ks)) + S::x_past(ks) + j * 16 * Q]);
+                    acc[s][j] = mfma16(fl, fx, acc[s][j]);
                 }
             };
             float wv[8];
