@@ -387,10 +387,13 @@ template <int NSPLIT, bool HAS_Z, int DTK>
 int launch_one(const QaSScanParams& p, const SscanDtProj& dtp, int waves, hipStream_t stream) {
     using Cfg = WavesCfg<NSPLIT>;
     const int vec_out = p.out_d_stride == 1 && (reinterpret_cast<uintptr_t>(p.out) & 7u) == 0 && p.out_batch_stride % 4 == 0 && p.out_l_stride % 4 == 0;
-    const auto kernel = waves <= max_waves(4) ? scan_waves_kernel<NSPLIT, max_waves(4), HAS_Z, DTK> : scan_waves_kernel<NSPLIT, max_waves(NSPLIT), HAS_Z, DTK>;
+    constexpr int kFew = max_waves(4), kMost = max_waves(NSPLIT);
+    const auto kernel = waves <= kFew ? scan_waves_kernel<NSPLIT, kFew, HAS_Z, DTK> : scan_waves_kernel<NSPLIT, kMost, HAS_Z, DTK>;
     const int bytes = lds_bytes<NSPLIT>(waves, DTK);
-    static_assert(lds_bytes<NSPLIT>(max_waves(NSPLIT), DTK) <= 160 * 1024, "LDS of a CU");
-    if (bytes > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return check_launch();
+    // more LDS than a kernel gets by default: the limit is the kernel's, the same for launches of any number of waves (other threads make theirs)
+    const int limit = lds_bytes<NSPLIT>(waves <= kFew ? kFew : kMost, DTK);
+    static_assert(lds_bytes<NSPLIT>(kMost, DTK) <= 160 * 1024, "LDS of a CU");
+    if (bytes > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, limit) != hipSuccess) return check_launch();
     hipLaunchKernelGGL(kernel, dim3((p.dim + Cfg::kCh - 1) / Cfg::kCh, static_cast<unsigned>(p.batch)), dim3(64 * waves), bytes, stream, p, dtp, vec_out);
     return check_launch();
 }
