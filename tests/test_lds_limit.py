@@ -54,7 +54,7 @@ else:
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="no C++ compiler")
-@pytest.mark.parametrize("calls", ["scan"])
+@pytest.mark.parametrize("calls", ["scan", "hadamard"])
 def test_a_kernel_has_one_limit(tmp_path, calls):
     (tmp_path / "stand_ins.cpp").write_text(STAND_INS)
     built = str(tmp_path / "stand_ins.so")
