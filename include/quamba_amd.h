@@ -253,7 +253,8 @@ typedef struct QaSScanParams {
      * u_l_stride ... apart) and B, C states contiguous (B_dstate_stride == C_dstate_stride == 1, steps B_l_stride ...
      * apart), as the row-major projections leave them; all of them 4-byte aligned with strides of whole words.
      * dstate 16, one group, dim a multiple of 4, none of the carry fields above; mapping also takes 16 (the time cut over the waves of a workgroup, by the
-     * library's rule), 64 + w - 1 and 96 + w - 1 (the same with four and eight lanes a channel and w waves, up to 12 and 16).
+     * library's rule, or one pass of eight lanes), 64 + w - 1 and 96 + w - 1 (the time over w waves, up to 12 and 16, with four
+     * and eight lanes a channel; step sizes that are not negative).
      * `workspace` (or null): scratch for scanning few sequences as segments side by side; segments: 0, or how many
      * (tests); segment_len: set by the library. */
     int32_t token_major, segments, segment_len, reserved0;

@@ -175,6 +175,7 @@ struct Mamba1Buffers {
 QaSScanParams scan_sizes(const QaMamba1Params& p) {
     QaSScanParams s = {};
     s.batch = p.batch; s.dim = p.d_inner; s.seqlen = p.seqlen; s.dstate = p.d_state; s.n_groups = 1;
+    s.delta_softplus = p.delta_softplus;                                       // (the workspace goes with it, sscan_tm.hip)
     return s;
 }
 
@@ -245,7 +246,6 @@ SscanDtProj scan_dt_of(const QaMamba1Params& p, const Mamba1Buffers& b) {
 QaSScanParams scan_of(const QaMamba1Params& p, const Mamba1Buffers& b) {
     QaSScanParams s = scan_sizes(p);
     const int64_t dbl = p.x_proj.n, len = p.seqlen, d = p.d_inner;
-    s.delta_softplus = p.delta_softplus;
     s.token_major = 1;
     s.u_batch_stride = len * d; s.u_l_stride = d; s.u_d_stride = 1;
     s.delta_batch_stride = len * d; s.delta_l_stride = d; s.delta_d_stride = 1;

@@ -528,11 +528,11 @@ TmPlan plan_of(const QaSScanParams& p) {
         r.segment_len = ((p.seqlen + segments - 1) / segments + 31) / 32 * 32;
         r.segments = (p.seqlen + r.segment_len - 1) / r.segment_len;
     };
-    const ScanWavesPlan over_waves = scan_waves_plan(p, cus);
     if (p.mapping != 0) {
         r.lanes = (p.mapping >> 20) & 0xff;
         r.blocks_a = r.lanes == 0 ? p.mapping & 0xfffff : 0;
         if (r.lanes == kScanWavesMapping) {
+            const ScanWavesPlan over_waves = scan_waves_plan(p, cus);
             r.lanes = over_waves.lanes;
             r.waves = over_waves.waves;
         } else if (r.lanes >= kScanWavesNamed && r.lanes < kScanWavesNamed + 64) {
@@ -552,6 +552,7 @@ TmPlan plan_of(const QaSScanParams& p) {
         int64_t best = static_cast<int64_t>(p.seqlen) * step_cost(true, per_simd(wave_rows8 * p.batch));
         r.lanes = 8;
         TmPlan chosen = r;
+        const ScanWavesPlan over_waves = scan_waves_plan(p, cus);
         if (p.segments == 0 && over_waves.ns < kScanWavesNever) {
             // one pass of eight lanes, in tiles of 32 steps, with one, two or three waves to a SIMD (within 5 % of it in 200 sizes of 16 ... 220
             // steps): the shorter one for a tile or less (2 x 31 x 3072 5.6 us and 7.2, 1 x 31 x 5120 6.2 and 7.5) and behind a tile's
@@ -595,8 +596,7 @@ int launch(const QaSScanParams& p_in, const SscanDtProj& dtp, hipStream_t stream
     TmPlan plan = plan_of(p);
     const int vec_out = p.out_d_stride == 1 && aligned16(p.out) && p.out_batch_stride % 8 == 0 && p.out_l_stride % 8 == 0;
     if (plan.segments > 1 && (!p.workspace || p.workspace_bytes < segment_bytes(p, plan))) {
-        const ScanWavesPlan over_waves = scan_waves_plan(p, compute_units());
-        p.mapping = 0x40000000 | (over_waves.ns < kScanWavesNever ? kScanWavesMapping : plan.lanes) << 20;       // one segment
+        p.mapping = 0x40000000 | kScanWavesMapping << 20;       // one segment
         p.segments = 0;
         plan = plan_of(p);
     }

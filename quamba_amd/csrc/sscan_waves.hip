@@ -421,7 +421,10 @@ int sscan_waves_fwd(const QaSScanParams& p, const SscanDtProj* dt, int lanes, in
 // (3 x 1021 x 5120 106 us against 102, 8 x 512 x 2048 56 and 52), as it is for some short prompts (plan_of there).
 ScanWavesPlan scan_waves_plan(const QaSScanParams& p, int cus) {
     const auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-    ScanWavesPlan best = {4, 1, kScanWavesNever};
+    ScanWavesPlan best = {8, 0, kScanWavesNever};
+    // (Without softplus step sizes may be negative, and the decay of all of a wave's steps beyond fp32 - a factor that nothing else would
+    // make of them while the state is still zero: the product is no number then.)
+    if (!p.delta_softplus) return best;
     for (const int lanes : {4, 8}) {
         const int64_t steps = lanes == 4 ? WavesCfg<4>::T : WavesCfg<8>::T, channels = lanes == 4 ? WavesCfg<4>::kCh : WavesCfg<8>::kCh;
         const int64_t per_cu = up(up(p.dim, channels) * p.batch, cus), pieces = up(p.seqlen, steps);

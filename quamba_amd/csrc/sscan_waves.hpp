@@ -9,8 +9,8 @@ constexpr int kScanWavesMax = 16;          // waves of a workgroup
 // channel (32 more: eight) and one wave (w more: w + 1)
 constexpr int kScanWavesMapping = 16, kScanWavesNamed = 64;
 
-// Lanes per channel and waves per workgroup for these sizes, and the estimated time (kScanWavesNever: these sizes are better left
-// to another kernel).
+// Lanes per channel and waves per workgroup for these sizes, and the estimated time (kScanWavesNever: better left to another
+// kernel, one pass of eight lanes).
 constexpr int64_t kScanWavesNever = 1LL << 62;
 struct ScanWavesPlan {
     int lanes, waves;

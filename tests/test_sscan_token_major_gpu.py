@@ -20,13 +20,13 @@ def _inputs(dev, batch, dim, seqlen, seed):
     return d, s
 
 
-def _token_major(d, s, state_dtype, with_z, workspace_bytes, lanes=None):
+def _token_major(d, s, state_dtype, with_z, workspace_bytes, lanes=None, softplus=1):
     batch, L, dim = d["u"].shape
     out = torch.empty((batch, L, dim), dtype=torch.float16, device=d["u"].device)
     state = torch.empty((batch, dim, 16), dtype=state_dtype, device=out.device)
     ws = torch.empty(max(workspace_bytes, 1), dtype=torch.uint8, device=out.device)
     p = _lib.QaSScanParams()
-    p.batch, p.dim, p.seqlen, p.dstate, p.n_groups, p.delta_softplus, p.token_major = batch, dim, L, 16, 1, 1, 1
+    p.batch, p.dim, p.seqlen, p.dstate, p.n_groups, p.delta_softplus, p.token_major = batch, dim, L, 16, 1, softplus, 1
     p.u_batch_stride = p.delta_batch_stride = p.z_batch_stride = p.out_batch_stride = L * dim
     p.u_l_stride = p.delta_l_stride = p.z_l_stride = p.out_l_stride = dim
     p.u_d_stride = p.delta_d_stride = p.z_d_stride = p.out_d_stride = 1

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from quamba_amd import ops
+from tests import launched
 from tests.test_sscan_token_major_gpu import _inputs, _token_major
 
 pytestmark = pytest.mark.gpu
@@ -29,3 +30,22 @@ def test_waves(dev, lanes, waves, batch, dim, dtype, with_z):
             assert float((a - b).abs().max()) <= 1
         else:
             assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("dim,seqlen", [(1536, 300), (512, 90), (5120, 40)])
+@pytest.mark.parametrize("sizes", [range(-127, -60), range(-127, 128)])
+def test_step_sizes_below_zero(dev, dim, seqlen, sizes):
+    """Without softplus decays may grow without bounds, and a state that is zero until the last step stays zero: the grown product of many
+    decays must not meet it.  (Growth of exp(1.3 x 11) a step, 88 is the largest exponent of fp32.)"""
+    d, s = _inputs(dev, 1, dim, seqlen, seed=dim)
+    g = torch.Generator(device=dev).manual_seed(seqlen)
+    d["u"][:, :-1] = 0
+    d["dt"] = torch.randint(sizes.start, sizes.stop, d["dt"].shape, dtype=torch.int8, device=dev, generator=g)
+    d["A"].fill_(120)
+    s["dt"], s["db"] = s["dt"] / 3, s["db"] / 100
+    (out, state), names = launched.kernels(lambda: _token_major(d, s, torch.float32, True, 0, softplus=0))
+    step = s["dt"] * d["dt"][:, -1].double() + s["db"] * d["db"].double()
+    want = (step * s["u"] * d["u"][:, -1].double())[..., None] * s["B"] * d["bc"][:, -1, None, 8:24].double()
+    assert float((state - want).abs().max()) <= 1e-5 * float(want.abs().max())
+    assert not bool(out[:, :-1].any()) and bool(out.isfinite().all())
+    launched.expect(names, "scan_tm_kernel<8, true, true, 0>")
