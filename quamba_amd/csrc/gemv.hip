@@ -47,8 +47,11 @@ __device__ __forceinline__ int row_sum(int v) {
     return v;
 }
 
-// The conv behind a product: one output scale and a state of a word per channel (Mamba1's layer), or anything.
-enum ConvKind { kNoConv, kConvOneScale, kConvTables };
+// The conv behind a product: one output scale and a state of a word per channel (Mamba1's layer), output scales from tables and such
+// a state, or anything.  A word may stand anywhere on four bytes: read code by code (channels 4 and 8 bytes apart, one row, us) int8
+// 10240 x 2560 5.8 -> 6.25, 4 bits 6.1 -> 6.7, with tables int8 10576 x 2560 6.3 -> 6.5, 4 bits two rows 6320 x 1536 4.6 -> 4.9.
+enum ConvKind { kNoConv, kConvOneScale, kConvTablesWords, kConvTables };
+constexpr bool words_held(ConvKind c) { return c == kConvOneScale || c == kConvTablesWords; }
 
 // What a conv step takes of the conv's operands, requested behind the weights by every wave in one straight run: a branch
 // around loads leaves the compiler unsure how many are in flight, and it waits for all of them, the weights among them, where the
@@ -73,13 +76,14 @@ __device__ __forceinline__ ConvOperands request_conv(const QaConv2Params& p, con
     ConvOperands r;
     r.taps = *reinterpret_cast<const uint32_t*>(p.weight + mine * 4);
     r.bias = *(p.bias ? p.bias + mine : p.weight);
-    if constexpr (CONV == kConvOneScale) {
+    if constexpr (words_held(CONV)) {
         r.held = *reinterpret_cast<const uint32_t*>(st);
-        return r;
-    }
-    const int drop = p.conv_state_len - 3;
+    } else {
+        const int drop = p.conv_state_len - 3;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) r.codes[i] = static_cast<uint8_t>(st[(drop + i) * p.conv_state_l_stride]);
+        for (int i = 0; i < 3; ++i) r.codes[i] = static_cast<uint8_t>(st[(drop + i) * p.conv_state_l_stride]);
+    }
+    if constexpr (CONV == kConvOneScale) return r;
     const bool grouped = p.x_out_scales && p.x_head_group_range != nullptr && p.x_dim_group_range != nullptr;
     r.in_table = grouped && part.index == 0;
     int g = 0, own = 0;
@@ -254,7 +258,7 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& p, const Conv& f) {
     }
     float c_out_scale = 1.0f;
     if constexpr (CONV == kConvOneScale) c_out_scale = f.conv.x_out_scale;
-    if constexpr (CONV == kConvTables) if (conv_col) c_out_scale = found_out_scale(f.conv, conv, ch0, value % kRows, lane);
+    else if constexpr (CONV != kNoConv) if (conv_col) c_out_scale = found_out_scale(f.conv, conv, ch0, value % kRows, lane);
     if (!mine) return;
     const float accf = static_cast<float>(sum);
     float y = p.rule == kGemvHalfAway ? (s_col * s_row) * accf : p.rule == kGemvColOuter ? s_col * (s_row * accf)
@@ -264,9 +268,9 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& p, const Conv& f) {
         const int8_t q = static_cast<int8_t>(quant8(y, p.half_away ? QA_ROUND_HALF_AWAY : QA_ROUND_RNE));
         if constexpr (CONV != kNoConv) if (conv_col) {
             const QaConv2Params& c = f.conv;
-            const uint32_t kept = CONV == kConvOneScale ? conv.held >> 8 : conv.codes[0] | (conv.codes[1] << 8) | (conv.codes[2] << 16);
+            const uint32_t kept = words_held(CONV) ? conv.held >> 8 : conv.codes[0] | (conv.codes[1] << 8) | (conv.codes[2] << 16);
             const uint32_t win = kept | (static_cast<uint32_t>(static_cast<uint8_t>(q)) << 24);
-            if constexpr (CONV == kConvOneScale) {
+            if constexpr (words_held(CONV)) {
                 *reinterpret_cast<uint32_t*>(st) = win;
             } else {
                 for (int i = 0; i < c.conv_state_len; ++i) st[i * c.conv_state_l_stride] = static_cast<int8_t>(win >> (8 * (i + 4 - c.conv_state_len)));
@@ -292,6 +296,10 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvArgs p, std::conditional_
     gemv_body<BITS, M, KS, BATCH, OUT, CONV ? kConvOneScale : kNoConv>(p, f);
 }
 template <int BITS, int M, int KS, int BATCH>
+__global__ __launch_bounds__(256) void gemv_conv_words_kernel(GemvArgs p, GemvConv f) {
+    gemv_body<BITS, M, KS, BATCH, QA_OUT_I8, kConvTablesWords>(p, f);
+}
+template <int BITS, int M, int KS, int BATCH>
 __global__ __launch_bounds__(256) void gemv_conv_tables_kernel(GemvArgs p, GemvConv f) {
     gemv_body<BITS, M, KS, BATCH, QA_OUT_I8, kConvTables>(p, f);
 }
@@ -303,7 +311,9 @@ int launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>((groups * KS + per_block - 1) / per_block)), block(64 * per_block);
     const GemvArgs args(p);
     const NoGemvConv none = {};
-    if (conv && !conv->conv.x_out_scales && conv_state_in_words(conv->conv)) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, true>), grid, block, 0, stream, args, *conv);
+    const bool words = conv && gemv_state_in_words(conv->conv);
+    if (words && !conv->conv.x_out_scales) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, true>), grid, block, 0, stream, args, *conv);
+    else if (words) hipLaunchKernelGGL((gemv_conv_words_kernel<BITS, M, KS, BATCH>), grid, block, 0, stream, args, *conv);
     else if (conv) hipLaunchKernelGGL((gemv_conv_tables_kernel<BITS, M, KS, BATCH>), grid, block, 0, stream, args, *conv);
     else if (p.out_type == QA_OUT_I8) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_I8, false>), grid, block, 0, stream, args, none);
     else if (p.out_type == QA_OUT_F16) hipLaunchKernelGGL((gemv_kernel<BITS, M, KS, BATCH, QA_OUT_F16, false>), grid, block, 0, stream, args, none);

@@ -65,6 +65,10 @@ inline bool gemv_conv_ok(const GemvConv& f) {
            c.x_dim % 4 == 0 && c.x_headdim % 4 == 0 && (c.x_dim == c.dim || (c.d_state * c.n_groups) % 4 == 0) &&
            c.nhead_groups <= kGemvConvGroups && c.ndim_groups <= kGemvConvGroups;
 }
+// a state of four codes that is one word, whatever lies between the channels' words
+inline bool gemv_state_in_words(const QaConv2Params& c) {
+    return c.conv_state_len == 4 && c.conv_state_l_stride == 1 && c.conv_state_c_stride % 4 == 0 && c.conv_state_batch_stride % 4 == 0 && aligned4(c.conv_state);
+}
 
 int gemv_launch(const GemvParams& p, const GemvConv* conv, hipStream_t stream);
 

@@ -195,7 +195,22 @@ def test_in_proj_without_group_scales(dev, cls, d_model, batch, shape):
     _step(dev, cls, d_model, batch, torch.float32, f"gemm_split_kernel<{shape}>", per_channel=True)
 
 
-def _step(dev, cls, d_model, batch, dtype, *names, per_channel=False):
+# a conv state whose codes of a channel are one word, in buffers that are not the package's own: channels eight bytes apart behind a
+# base of four, the second family's by channel
+@pytest.mark.parametrize("apart", [4, 8])
+@pytest.mark.parametrize("cls,d_model,batch,name", [
+    (W8A8QMamba, 768, 1, "gemv_kernel<8, 1, 1, 4, 0, true>"), (W8A8QMamba, 2048, 2, "gemv_kernel<8, 2, 2, 2, 0, true>"), (W4A8QMamba, 768, 2, "gemv_kernel<4, 2, 1, 2, 0, true>"),
+    (W8A8QMamba2, 768, 1, "gemv_conv_words_kernel<8, 1, 1, 4>"), (W8A8QMamba2, 256, 3, "gemv_conv_words_kernel<8, 4, 1, 3>"),
+    (W4A8QMamba2, 2048, 2, "gemv_conv_words_kernel<4, 2, 2, 1>"), (W4A8QMamba2, 4096, 1, "gemv_conv_words_kernel<4, 1, 1, 2>")])
+def test_step_with_a_state_of_words(dev, cls, d_model, batch, name, apart):
+    def view(conv):
+        buf = torch.zeros(4 + batch * conv.shape[1] * apart, dtype=torch.int8, device=dev)
+        v = buf[4:].view(batch, conv.shape[1], apart)[..., :4]
+        return v.copy_(conv)
+    _step(dev, cls, d_model, batch, torch.int8, name, conv_view=view)
+
+
+def _step(dev, cls, d_model, batch, dtype, *names, per_channel=False, conv_view=lambda conv: conv):
     m, g = _layer(cls, dev, d_model, batch)
     if per_channel:
         m.in_proj.s_group = torch.empty((0, m.in_proj.size_n), dtype=torch.float16, device=dev)
@@ -203,6 +218,7 @@ def _step(dev, cls, d_model, batch, dtype, *names, per_channel=False):
     h = variants._ri(dev, g, batch, 1, d_model)
     conv, ssm = layers._states(m, dev, g, batch, dtype, 4)
     conv2, ssm2 = conv.clone(), ssm.clone()
+    conv = conv_view(conv)
     out, ran = launched.kernels(lambda: _layer_call.call(m, h, conv, ssm, True))
     assert out is not None
     layers._close(out[:, 0], m._step_modules(h, conv2, ssm2), (conv, conv2), (ssm, ssm2))
