@@ -231,7 +231,9 @@ def _step(dev, cls, d_model, batch, dtype, *names, per_channel=False, conv_view=
     (1024, 16, 33, ["scan_tm_kernel<4, true, true, 1>"]), (1280, 16, 35, ["scan_tm_mixed_kernel<true, 2>"]), (2560, 8, 37, ["scan_tm_mixed_kernel<true, 3>"]),
     (256, 1, 1500, ["scan_tm_kernel<8, false, false, 1>", "scan_tm_kernel<8, true, true, 1>"]), (2560, 3, 515, ["scan_tm_kernel<8, true, true, 3>"]),
     (1536, 1, 37, ["scan_waves_kernel<4, 12, true, 2>"]), (2560, 1, 700, ["scan_waves_kernel<8, 12, true, 3>"]), (768, 1, 515, ["scan_waves_kernel<8, 12, true, 1>"]),
-    (768, 1, 500, ["scan_waves_kernel<8, 16, true, 1>"])])
+    (768, 1, 500, ["scan_waves_kernel<8, 16, true, 1>"]), (768, 1, 1024, ["scan_waves_kernel<8, 16, true, 1>"]), (2560, 1, 48, ["scan_waves_kernel<4, 12, true, 3>"]),
+    (2560, 1, 300, ["scan_waves_kernel<4, 12, true, 3>"]), (1536, 2, 67, ["scan_waves_kernel<8, 12, true, 2>"]), (1536, 2, 400, ["scan_waves_kernel<8, 12, true, 2>"]),
+    (3072, 1, 515, ["scan_waves_kernel<8, 12, true, 3>"]), (256, 2, 1300, ["scan_tm_kernel<8, false, false, 1>", "scan_tm_kernel<8, true, true, 1>"])])
 def test_scan_of_a_layer(dev, d_model, batch, seqlen, names):
     m, g = _layer(W8A8QMamba, dev, d_model, seqlen)
     h = variants._ri(dev, g, batch, seqlen, d_model)

@@ -160,7 +160,7 @@ def test_norm_of_whole_rows_of_4096(dev, batch, seqlen, norm_first):
 
 @pytest.mark.parametrize("d_model,batch,seqlen", [(768, 1, 65), (768, 16, 33), (1536, 1, 515), (1536, 12, 70), (2560, 16, 31), (3072, 3, 100)])
 def test_forward_of_a_wide_layer(dev, d_model, batch, seqlen):
-    """dt_proj inside the scan: ranks of 48, 96, 160 and 192, sixteen, eight and four lanes per channel, both at once."""
+    """dt_proj inside the scan: ranks of 48, 96, 160 and 192, the time over waves, eight and four lanes per channel, both at once."""
     m, g = _mamba1(W8A8QMamba, dev, seed=seqlen, d_model=d_model)
     h = _ri(dev, g, batch, seqlen, d_model)
     conv, ssm = _states(m, dev, g, batch, torch.float32, 4)

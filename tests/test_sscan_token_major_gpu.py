@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from quamba_amd import _lib, ops
+from tests import launched
 
 pytestmark = pytest.mark.gpu
 
@@ -20,7 +21,7 @@ def _inputs(dev, batch, dim, seqlen, seed):
     return d, s
 
 
-def _token_major(d, s, state_dtype, with_z, workspace_bytes, lanes=None, softplus=1):
+def _token_major(d, s, state_dtype, with_z, workspace_bytes, lanes=None, softplus=1, segments=0):
     batch, L, dim = d["u"].shape
     out = torch.empty((batch, L, dim), dtype=torch.float16, device=d["u"].device)
     state = torch.empty((batch, dim, 16), dtype=state_dtype, device=out.device)
@@ -42,7 +43,7 @@ def _token_major(d, s, state_dtype, with_z, workspace_bytes, lanes=None, softplu
     p.out = out.data_ptr()
     setattr(p, "last_state_i8" if state_dtype == torch.int8 else "last_state_f32", state.data_ptr())
     p.workspace, p.workspace_bytes = ws.data_ptr(), workspace_bytes
-    p.mapping = 0 if lanes is None else 0x40000000 | lanes << 20
+    p.mapping, p.segments = 0 if lanes is None else 0x40000000 | lanes << 20, segments
     _lib.check(_lib.lib().qa_sscan_fwd(C.byref(p), _lib.current_stream(out.device)), "sscan_fwd")
     return out, state
 
@@ -54,13 +55,30 @@ def _token_major(d, s, state_dtype, with_z, workspace_bytes, lanes=None, softplu
     (48, 1024, 37, torch.float32, True, 0), (48, 1028, 64, torch.int8, False, 0),
     (1, 512, 256, torch.float32, True, 1 << 22), (2, 1540, 515, torch.int8, True, 1 << 22), (1, 96, 2049, torch.float32, False, 1 << 22)])
 def test_token_major(dev, batch, dim, seqlen, dtype, with_z, ws):
+    # (lanes 16: the library's own choice of waves)
+    _against_seqlen_major(dev, batch, dim, seqlen, dtype, with_z, [dict(lanes=n) for n in ((None,) if ws else (None, 4, 8, 16))], ws)
+
+
+# cut into segments by name, whatever the library's rule would choose: two, a ragged last one, as many as there are tiles
+@pytest.mark.parametrize("batch,dim,seqlen,dtype,with_z", [(1, 512, 256, torch.float32, True), (2, 1540, 515, torch.int8, True), (1, 96, 2049, torch.float32, False),
+                                                           (2, 512, 1300, torch.float32, True), (5, 36, 97, torch.int8, False), (1, 5120, 700, torch.float32, True)])
+def test_segments(dev, batch, dim, seqlen, dtype, with_z):
+    ways = [dict(lanes=8, segments=n) for n in sorted({2, 3, 7, (seqlen + 31) // 32})]
+    names = _against_seqlen_major(dev, batch, dim, seqlen, dtype, with_z, ways, 1 << 28)
+    for ran in names:
+        launched.expect(ran, "scan_tm_kernel<8, false, false, 0>", f"scan_tm_kernel<8, {'true' if with_z else 'false'}, true, 0>")
+
+
+def _against_seqlen_major(dev, batch, dim, seqlen, dtype, with_z, ways, ws):
     d, s = _inputs(dev, batch, dim, seqlen, seed=dim + seqlen)
     rows = lambda a: a.transpose(1, 2).contiguous()
     B, Cm = rows(d["bc"][:, :, 8:24])[:, None], rows(d["bc"][:, :, 24:40])[:, None]
     want, st = ops.sscan_fwd(rows(d["u"]), s["u"], rows(d["dt"]), s["dt"], d["A"], s["A"], B, s["B"], Cm, s["C"], s["st"], d["D"], s["D"],
                              rows(d["z"]) if with_z else None, s["z"] if with_z else None, d["db"], s["db"], True, state_dtype=dtype)
-    for lanes in (None,) if ws else (None, 4, 8, 16):
-        out, state = _token_major(d, s, dtype, with_z, ws, lanes)
+    names = []
+    for way in ways:
+        (out, state), ran = launched.kernels(lambda: _token_major(d, s, dtype, with_z, ws, **way))
+        names.append(ran)
         diff = (out.float() - want.float()).abs()
         assert bool((diff <= 1e-3 + 2e-3 * want.float().abs()).all())
         a, b = state.float(), st[:, :, 0].float()
@@ -68,3 +86,4 @@ def test_token_major(dev, batch, dim, seqlen, dtype, with_z, ws):
             assert float((a - b).abs().max()) <= 1
         else:
             assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max())
+    return names

@@ -1,16 +1,18 @@
 """The update of fp32 states beyond the last-level cache, which goes past it, against the same entries some at a time, which do not:
-states and outputs to the bit."""
+states and outputs to the bit, and the kernel by its name on both sides of the border."""
 import pytest
 import torch
 
 from quamba_amd import ops
+from tests import launched
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B,H,P,N", [(57, 128, 64, 128), (241, 61, 64, 64)])
-def test_streamed(dev, B, H, P, N):
-    assert B * H * P * N * 4 >= 224 << 20 > 20 * H * P * N * 4
+@pytest.mark.parametrize("B,H,P,N,lanes", [(57, 128, 64, 128, 8), (241, 61, 64, 64, 4), (55, 128, 64, 128, 8), (234, 61, 64, 64, 4)])
+def test_streamed(dev, B, H, P, N, lanes):
+    streamed = B * H * P * N * 4 >= 224 << 20
+    assert abs(B * H * P * N * 4 / (224 << 20) - 1) < 0.03 and 20 * H * P * N * 4 < 224 << 20
     gen = torch.Generator(device=dev).manual_seed(B)
     ri = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device=dev, generator=gen)
     f = lambda *v: torch.tensor(v, device=dev)
@@ -24,9 +26,12 @@ def test_streamed(dev, B, H, P, N):
                                 Bq[b], f(0.02), Cq[b], f(0.02), D.view(H, 1).expand(H, P), f(0.02), z[b], f(0.03), bias.view(H, 1).expand(H, P), None, True)
 
     many = state.clone()
-    y = run(many, slice(None))
+    y, names = launched.kernels(lambda: run(many, slice(None)))
+    kernel = f"ssm_update_kernel<{lanes}, true, true, false, true, "
+    launched.expect(names, kernel + ("true>" if streamed else "false>"))
     assert not torch.equal(many, state)
     for b in range(0, B, 20):
         some = state[b:b + 20].clone()
-        ys = run(some, slice(b, b + 20))
+        ys, names = launched.kernels(lambda: run(some, slice(b, b + 20)))
+        launched.expect(names, kernel + "false>")
         assert torch.equal(some, many[b:b + 20]) and torch.equal(ys, y[b:b + 20])
