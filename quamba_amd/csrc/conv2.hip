@@ -29,10 +29,13 @@ constexpr int kThreads = 256;
 // loads meet the compiler waits for every load in flight, the inputs among them, and the look-up of an output scale - the
 // head's group, the channel's group in it, their scale - was three trips to memory one after the other.  Now a wave requests the whole
 // table and looks it up across its lanes.  Bound by vector issue (some 55 instructions for four outputs, of which the exponential and the
-// reciprocal are a third) and, in short runs, by that set-up.  In a layer, us before and after: one scale 1 x 512 x 1536
-// channels 5.2 -> 4.6, 1 x 777 x 3072 6.0 -> 5.2, 3 x 1021 x 5120 15.6 -> 13.8, 8 x 2048 x 5120 51 -> 48; tables 1 x 500 x 5376 7.4 -> 6.6, 3 x 1000 x
-// 2304 12.3 -> 9.8, 1 x 1531 x 5376 12.5 -> 11.6, 4 x 4096 x 5376 51 -> 48.  (One copy of the exact route in a loop over a lane's outputs
-// instead of four, a third of the code: 48.4 -> 53.6.)
+// reciprocal are a third) and, in short runs, by that set-up.  In a layer, kernel times in turn on one card, us before and after: one
+// scale 1 x 512 x 1536 channels 5.2 -> 4.6, 1 x 777 x 3072 5.9 -> 4.9, 3 x 1021 x 5120 15.4 -> 13.2, 8 x 2048 x 5120 55.6 -> 50.5; tables 1 x 500 x 5376
+// 7.3 -> 6.3, 3 x 1000 x 2304 12.0 -> 9.7, 1 x 1531 x 5376 11.8 -> 11.0, 4 x 4096 x 5376 60.7 -> 57.7, 16 x 1024 x 10240 105 -> 98.  Of this the sums as
+// floats (dot4_float) are 52.7 -> 50.5 at 8 x 2048 x 5120, 103 -> 98 at 16 x 1024 x 10240, 6.5 -> 6.3 at 1 x 500 x 5376 and nothing at 3 x 1021; runs of 6, 12,
+// 24 and 48 steps 9.9 -> 9.7 at 3 x 1000 x 2304, 6.4 -> 6.3 at 1 x 500 x 5376, 20.1 -> 19.7 at 1 x 12000 x 1792, elsewhere nothing; the rest is the
+// straight run.  (One copy of the exact route in a loop over a lane's outputs instead of four, a third of the code: 48.4 -> 53.6 at 8 x 2048
+// x 5120 on another card.)
 enum ScaleKind { kOneScale, kTables, kWalk };
 
 // grid: x = blocks of 256 channels, y = blocks of 4 runs of `run` steps (one run per wave), z = batch
@@ -327,7 +330,7 @@ int conv_channel_last_fwd(const QaConv2Params& p, hipStream_t stream) {
     // set-up (taps, scales, the three inputs ahead) 100 with one output scale and 400 with tables, and 160 a step of the last wave with
     // nobody beside it.  Measured in a layer with runs of 4, 6, 8, 12, 16, 24, 32 steps, us: one scale 1 x 512 x 1536 channels 4.6, 4.6, 5.4, 5.8,
     // 6.9, 8.1, 10.0; 3 x 1021 x 5120 13.4, 14.0, 14.9, 16.0, 15.6, 16.3, 16.0; 4 x 1500 x 2048 11.8, 12.1, 11.7, 12.4, 12.4, 12.7, 14.7; tables 1 x 1531 x
-    // 5376 11.8, 12.0, 11.6, 12.2, 11.6, 13.9, 14.6; 3 x 1000 x 2304 10.0, 9.8, 10.4, 10.8, 10.5, 12.5, 12.5; 4 x 4096 x 5376 62, 54, 52, 51, 49, 50, 50.  The
+    // 5376 11.8, 12.0, 11.6, 12.2, 11.6, 13.9, 14.6; 3 x 1000 x 2304 10.0, 9.8, 10.4, 10.8, 10.5, 12.5, 12.5; 4 x 4096 x 5376 (a faster card than that of the figures at the top) 62, 54, 52, 51, 49, 50, 50.  The
     // choice is at most 4 % behind the best run.  Anything else: 250, and two and three taps, which come byte by byte, 350 and 100 a step (over
     // 148 sizes of each the choice is 0.2 % behind the best power of two and 0.3 with fewer taps).
     int run = 4;

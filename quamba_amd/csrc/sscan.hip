@@ -1114,11 +1114,18 @@ __global__ __launch_bounds__(256) void ssm_update_kernel(QaSsmUpdateParams p) {
     ssm_update_body<LPR, VEC, FP32, false, FAST, 4, A_ONE, STREAM>(p, nullptr);
 }
 
-// States from this size on do not stay in the last-level cache (256 MiB) until the next token anyway: kept there they only push
-// out the weights, and what they leave dirty is written back while the next product reads them.  Loads and stores past the
-// caches, a whole Mamba2 step, us: 64 sequences x 128 heads x 64 x 128 (268 MB) with 4-bit weights 132 -> 122 (in_proj 33 -> 24,
-// out_proj 14.4 -> 10.7, the update itself 83 -> 86), int8 143 -> 126; 128 sequences 259 -> 220; 128 x 80 heads (336 MB) 159 -> 135, 96 x
-// 80 (252 MB) 113.5 -> 107.5.  Smaller states are found there again: 48 x 128 (201 MB) 96 -> 100, 32 x 80 (84 MB) 50 -> 52.
+// States from this size on go past the caches: they only push the weights out of the last-level cache (256 MiB), and what they leave
+// dirty there is written back while the next product reads its weights.  A whole Mamba2 step (sequences x heads of 64 x 128), us, kept in
+// the caches -> past them.
+// One layer called again and again, which finds there what it left: 64 x 128 (268 MB), 4-bit weights 134.7 -> 122.9 (in_proj 33 -> 24, out_proj
+// 14.4 -> 10.7, the update itself 82 -> 87), int8 143 -> 126; 96 x 80 (252 MB) int8 114.1 -> 108.3, 4 bits 109.9 -> 111.9; 112 x 64 (235 MB) 4 bits
+// 96.3 -> 101.9, int8 98.9 -> 101.3; below the border 100 x 64 (210 MB) 89.1 -> 93.6, 48 x 128 (201 MB) 4 bits 96.4 -> 99.3, int8 108.9 -> 104.1, 32 x 80
+// (84 MB) 50.7 -> 52.3.
+// Six layers one after the other, which find nothing: 64 x 128 143 -> 128, 96 x 80 129 -> 114, 112 x 64 116 -> 103; below the border 100 x 64 106 -> 95, 32 x 128
+// 86 -> 79, 32 x 80 62.5 -> 54.8, 4 x 128 (17 MB) 38.3 -> 35.1, 32 x 24 (25 MB) 24.0 -> 24.8.
+// The border stands where a lone layer's states and weights stop fitting in the cache (it gains from 230 to 270 MiB of both on, by the
+// weights; up to there few weights lose by 2 to 6 %); layers one after the other would gain far below it as well.  A state that a prompt
+// has just left costs the step behind it the same either way (64 x 128 126 and 128, 96 x 80 114 and 116).
 constexpr int64_t kStreamBytes = 224LL << 20;
 
 // conv step + state update of one token in one launch (d_state <= 16, one head)

@@ -59,8 +59,12 @@ __global__ __launch_bounds__(kThreads) void mamba1_step_kernel(StepArgs p) {
     StepSmem<NB>& sm = smem[wave];
     float(*const bc)[2][16] = bc_all[wave];
 
-    // the states first, most of the bytes, then the projection's operands, behind which everything else is needed (the states last: a step of
-    // 32 x 3072 fp32 0.3 us longer in a layer's 23.7, of 64 x 4096 0.6 in 29.9, of 16 x 3072 int8 0.3 in 22.4)
+    // The states first - of many sequences most of the bytes, of few what comes from furthest away, the weights having passed through
+    // the caches since - then the projection's operands, behind which everything else is needed.  With the states last a layer's step is
+    // longer: 32 x 3072 fp32 by 0.3 of 23.7 us, 64 x 4096 by 0.6 of 29.9; one to eight sequences in a chain of 24 layers, int8 by 0.1 to 1.0
+    // of 13 to 30 us (1 x 5120 21.2 -> 21.3, 3 x 1536 16.9 -> 17.2, 8 x 3072 23.9 -> 24.4), fp32 by -0.1 to 0.25 (1 x 1536 12.9 -> 13.1, 5 x 3072 23.8 as
+    // well).  Of one layer called again and again, whose states the caches hold, 5 and 8 sequences of 1536 and 2048 channels in fp32 are 0.0 to
+    // 0.2 of 16.2 us shorter that way.
     const int64_t at = static_cast<int64_t>(c) * 16 + 4 * slice;
     float4 st32[FP32 ? NB : 1];
     uint32_t st8[FP32 ? 1 : NB];

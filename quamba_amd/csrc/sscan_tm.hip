@@ -25,7 +25,9 @@
 //
 // Segments.  Few channels of a long sequence leave most of the chip idle even so: the sequence is cut into segments that are
 // scanned side by side, one pass for every segment's end state from a zero state and the sum of its step sizes (OUT false: no
-// C, no outputs), one that starts every segment from the state its predecessors chain up to.
+// C, no outputs), one that starts every segment from the state its predecessors chain up to.  By the rule below (256 CUs) that is from
+// 832 steps on with up to 1280 channels of one sequence or 1152 of two; wider layers are scanned over waves.  Step sizes that may be
+// negative are not (scan_waves_plan), and take segments by the same costs in layers of up to 5120 channels (one sequence, from 576 steps on).
 #include "conv_common.hpp"
 #include "gemm_core.hpp"
 #include "mixer_common.hpp"
